@@ -326,6 +326,27 @@ bool mfma_applicable(const vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     return a.k <= 256;
 }
 
+// The width to pad every column block to so that the matrix-core kernels take the shape (squared L2
+// and Euclidean; 0: they take it as it is, or padding does not pay).  Below 8 floats the padded block
+// costs what a block of 8 costs, about 290 vector instructions per 32 rows and 256 centroids, where the
+// vector-ALU kernel needs 3 sub_dim + 3 per row and centroid: 3-10 times as many, and 50 times as
+// long where there is no kernel for the width (10 floats, 60,007 rows x 10 blocks, k = 200: 3.94 ms
+// per pass).  Under 32 centroids half of a tile of the matrix kernels is padding: those stay.
+int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd) {
+    if (ctx->assign_path == 1 || ctx->no_alloc || (metric != VQ_SQEUCLIDEAN && metric != VQ_EUCLIDEAN)) return 0;
+    if (a.k < 32 || a.k > vq::kMaxK || a.m > 65535) return 0;
+    if (mfma_applicable<vq::M_SQ, true>(ctx, a, sd) || mfma_wide_applicable<vq::M_SQ, true>(ctx, a, sd)) return 0;
+    const int sdp = (sd + 7) / 8 * 8;
+    // the limits of those kernels
+    if ((int64_t)a.m * sdp > (1 << 20) || sdp > (1 << 16) || a.n * a.m >= (1LL << 32)) return 0;
+    return sdp;
+}
+
+void launch_pad(vq_ctx *ctx, const float *x, int64_t n, int64_t ld, int m, int sd, int sdp, float *y) {
+    hipLaunchKernelGGL(vq::k_pad_blocks, dim3(cdiv(n * m * (sdp / 4), 1024)), dim3(256), 0, ctx->stream, x, n, ld, m, sd,
+                       sdp, y);
+}
+
 template <bool LBG>
 int32_t launch_assign(vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bool tables_ready = false,
                       hipEvent_t *started = nullptr, hipEvent_t *done = nullptr) {
@@ -600,7 +621,27 @@ int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, i
         *dist_written = true;
     }
     ProfSpan sp(ctx, VQ_PROF_ENCODE);
-    return launch_assign<false>(ctx, metric, a, sd);
+    const int sdp = pend ? 0 : pad_width(ctx, metric, a, sd);
+    if (!sdp) return launch_assign<false>(ctx, metric, a, sd);
+    // padded a slice of rows at a time: the copy is read back from the memory-side cache (256 MB)
+    // and the workspace stays small whatever n is
+    const int64_t row_bytes = (int64_t)sizeof(float) * m * sdp;
+    const int64_t slice = std::min<int64_t>(n, std::max<int64_t>(4096, (96 << 20) / row_bytes / 4096 * 4096));
+    VQ_TRY(ensure(ctx, ctx->pad_x, (size_t)(slice * row_bytes)));
+    VQ_TRY(ensure(ctx, ctx->pad_cb, sizeof(float) * (size_t)m * k * sdp));
+    launch_pad(ctx, d_codebooks, (int64_t)m * k, sd, 1, sd, sdp, (float *)ctx->pad_cb.p);
+    a.x = (const float *)ctx->pad_x.p;
+    a.ld = (int64_t)m * sdp;
+    a.cb = (const float *)ctx->pad_cb.p;
+    if (d_dist && dist_written && sdp == 8) *dist_written = true;
+    for (int64_t r0 = 0; r0 < n; r0 += slice) {
+        a.n = std::min(slice, n - r0);
+        a.codes = d_codes + r0 * m;
+        a.dist = d_dist && sdp == 8 ? d_dist + r0 * m : nullptr;
+        launch_pad(ctx, d_x + r0 * ld, a.n, ld, m, sd, sdp, (float *)ctx->pad_x.p);
+        VQ_TRY(launch_assign<false>(ctx, metric, a, sdp));
+    }
+    return VQ_OK;
 }
 
 }  // namespace vqh
@@ -650,7 +691,7 @@ int32_t vq_ctx_destroy(vq_ctx *ctx) {
     if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     DevBuf *bufs[] = {&ctx->flags, &ctx->tables, &ctx->hist, &ctx->perm, &ctx->leaf_desc,
                       &ctx->leaf_sum, &ctx->codes, &ctx->idx, &ctx->reseed, &ctx->cnorm,
-                      &ctx->seg, &ctx->part_sum, &ctx->mfma_tab, &ctx->mfma_list, &ctx->mfma_stat, &ctx->tsvq_sq, &ctx->tsvq_split, &ctx->tsvq_level, &ctx->tsvq_means, &ctx->tsvq_scan, &ctx->tsvq_km, &ctx->tsvq_bsum, &ctx->tsvq_segmaps, &ctx->tsvq_gsum, &ctx->tsvq_guess, &ctx->tsvq_maps, &ctx->tmp_a, &ctx->tmp_b, &ctx->tmp_c, &ctx->tmp_d, &ctx->tmp_e, &ctx->tmp_f,
+                      &ctx->seg, &ctx->part_sum, &ctx->pad_x, &ctx->pad_cb, &ctx->mfma_tab, &ctx->mfma_list, &ctx->mfma_stat, &ctx->tsvq_sq, &ctx->tsvq_split, &ctx->tsvq_level, &ctx->tsvq_means, &ctx->tsvq_scan, &ctx->tsvq_km, &ctx->tsvq_bsum, &ctx->tsvq_segmaps, &ctx->tsvq_gsum, &ctx->tsvq_guess, &ctx->tsvq_maps, &ctx->tmp_a, &ctx->tmp_b, &ctx->tmp_c, &ctx->tmp_d, &ctx->tmp_e, &ctx->tmp_f,
                       &ctx->big_chunk, &ctx->big_win, &ctx->big_wind, &ctx->big_best, &ctx->big_fresh, &ctx->big_codes, &ctx->big_keys,
                       &ctx->big_sorted, &ctx->big_sort_tmp, &ctx->big_tables, &ctx->big_flags};
     for (DevBuf *b : bufs)
@@ -1057,6 +1098,14 @@ int32_t vq_copy_f32(vq_ctx *ctx, float *d_dst, const float *d_src, int64_t count
     return VQ_OK;
 }
 
+}  // extern "C"
+
+template <typename Last>
+static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
+                           int32_t max_iters, const uint32_t *h_init_idx, const uint32_t *h_reseed_stream,
+                           int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used,
+                           const float *pend_cb, const uint8_t *pend_codes, const Last &last);
+
 // pend_cb / pend_codes: a residual update x[i] -= pend_cb[pend_codes[i]] that the fit applies to the
 // rows in place as its first assignment pass reads them (the caller has checked that this shape's
 // first pass is the kernel that can: lbg_pending_fusable).
@@ -1083,6 +1132,45 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
     if (k > vq::kMaxK)
         return vqh::lbg_fit_big(ctx, d_x, n, ld, m, sd, k, max_iters, h_init_idx, h_reseed_stream, n_reseed,
                                 d_codebooks, h_iters_run, h_reseeds_used);
+    vq::AssignArgs shape;
+    shape.x = d_x;
+    shape.n = n;
+    shape.ld = ld;
+    shape.m = m;
+    shape.k = k;
+    shape.cb = d_codebooks;
+    const int sdp = max_iters > 0 ? pad_width(ctx, VQ_SQEUCLIDEAN, shape, sd) : 0;
+    if (sdp && (int64_t)k * cdiv(n, vq::kPartRows) * sdp <= (1LL << 31)) {
+        // the rows padded once for all passes of the fit (a shape too large for a second copy of its
+        // rows trains on the rows as they are)
+        const size_t bytes = sizeof(float) * (size_t)n * m * sdp;
+        const int32_t rc = ensure(ctx, ctx->pad_x, bytes);
+        if (rc == VQ_OK) {
+            VQ_TRY(ensure(ctx, ctx->pad_cb, sizeof(float) * (size_t)m * k * sdp));
+            float *px = (float *)ctx->pad_x.p, *pcb = (float *)ctx->pad_cb.p;
+            launch_pad(ctx, d_x, n, ld, m, sd, sdp, px);
+            const int32_t fit = lbg_fit_run(ctx, px, n, (int64_t)m * sdp, m, sdp, k, max_iters, h_init_idx,
+                                            h_reseed_stream, n_reseed, pcb, h_iters_run, h_reseeds_used, nullptr, nullptr,
+                                            [&] {
+                                                hipLaunchKernelGGL(vq::k_unpad_rows, dim3(cdiv((int64_t)m * k * sd, 256)),
+                                                                   dim3(256), 0, ctx->stream, (const float *)pcb,
+                                                                   (int64_t)m * k, sd, sdp, d_codebooks);
+                                            });
+            return fit;
+        }
+        if (rc != VQ_ERR_OOM) return rc;
+    }
+    return lbg_fit_run(ctx, d_x, n, ld, m, sd, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, d_codebooks,
+                       h_iters_run, h_reseeds_used, pend_cb, pend_codes, [] {});
+}
+
+// The LBG loop for up to 256 centroids, on validated arguments.  last: enqueues what follows the
+// last update, before the loop's results are read back.
+template <typename Last>
+static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
+                           int32_t max_iters, const uint32_t *h_init_idx, const uint32_t *h_reseed_stream,
+                           int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used,
+                           const float *pend_cb, const uint8_t *pend_codes, const Last &last) {
     hipStream_t st = ctx->stream;
 
     const int nparts = (int)((n + vq::kPartRows - 1) / vq::kPartRows);
@@ -1245,6 +1333,7 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
         VQ_HIP(ctx, hipEventRecord(end, st));
         ctx->prof_open.push_back({VQ_PROF_LBG_UPDATE, prev_done, end, false, true});
     }
+    last();
     std::vector<int> host(7 * (size_t)m + 1);
     VQ_HIP(ctx, hipMemcpyAsync(host.data(), f, sizeof(int) * host.size(), hipMemcpyDeviceToHost, st));
     VQ_HIP(ctx, hipStreamSynchronize(st));
@@ -1256,6 +1345,8 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
                     "re-seed stream exhausted: pass n_reseed = k*max_iters");
     return VQ_OK;
 }
+
+extern "C" {
 
 int32_t vq_lbg_fit(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd,
                    int32_t k, int32_t max_iters, const uint32_t *h_init_idx,
