@@ -1,0 +1,48 @@
+"""The one-launch update of small LBG fits (two launches per iteration) against the CPU oracle, bit for
+bit: centroids, iterations run, re-seed rows used."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests import data
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import vq_amd
+    c = vq_amd.Context(0)
+    yield c
+    c.close()
+
+
+# n, m, sub_dim, k, iterations, kind
+CASES = [(16, 4, 8, 16, 3, "normal"),          # one row per cluster
+         (8191, 4, 8, 256, 3, "normal"), (8193, 4, 8, 250, 3, "normal"),  # a step of codes, and one row more
+         (70_001, 4, 8, 256, 2, "skewed"),     # clusters above 1024 members in several parts, the list worked off twice
+         (30_000, 1, 8, 100, 3, "skewed"), (20_000, 3, 4, 64, 3, "skewed"),
+         (9000, 2, 12, 40, 4, "same"),         # one cluster, every other one re-seeded
+         (2000, 5, 8, 7, 30, "blobs"),         # early stop
+         (3000, 2, 32, 20, 3, "normal"), (5000, 1, 36, 64, 3, "normal"), (4097, 1, 100, 33, 3, "normal"),
+         (12_000, 1, 256, 256, 2, "skewed"), (6000, 2, 64, 32, 3, "skewed"), (300, 1, 1000, 5, 2, "normal")]
+
+
+@pytest.mark.parametrize("n,m,sd,k,iters,kind", CASES)
+def test_small_fit(ctx, n, m, sd, k, iters, kind):
+    rng = np.random.default_rng(n + sd)
+    dim = m * sd
+    x = rng.standard_normal((n, dim)).astype(F)
+    if kind == "skewed":
+        x[rng.random(n) < 0.7] = x[0]  # most rows in one cluster
+    elif kind == "same":
+        x[:] = x[0]
+    elif kind == "blobs":
+        x = (10.0 * rng.integers(0, k, (n, 1)) + 0.01 * x).astype(F)
+    init, reseed = data.index_streams(n, m, k, iters, seed=n)
+    dcb = ctx.empty((m, k, sd), F)
+    it, used = ctx.lbg_fit(ctx.to_device(x), n, dim, m, sd, k, iters, init, reseed, dcb)
+    ref = O.pq_fit(x, m, k, iters, init, reseed)
+    assert np.array_equal(dcb.download().view(np.uint32), ref["codebooks"].view(np.uint32))
+    assert np.array_equal(it, ref["iters"]) and np.array_equal(used, ref["reseeds"])

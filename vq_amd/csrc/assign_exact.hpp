@@ -27,6 +27,7 @@ struct AssignArgs {
     uint8_t *codes;       // LBG mode: [m][n] in place (old -> new); encode mode: [n][m]
     int *changed;         // LBG mode: changed[s] set to 1 when any code of block s differs
     const int *done;      // LBG mode: blocks with done[s] != 0 are skipped
+    const int *before = nullptr;  // LBG mode, instead of done: the changed flags of the pass before (0: skipped)
     float *dist = nullptr;  // encode mode, k_assign_mfma_bf only: [n][m] distance of the chosen centroid, or null
     // A residual update that the pass applies before it scores the rows (single wide column block,
     // k_assign_mfma_wide_bf only): x[i] = src[i] - pend_cb[pend_codes[i]], where src is the rows
@@ -37,6 +38,11 @@ struct AssignArgs {
     const float *pend_src = nullptr;
     int64_t pend_src_ld = 0;
 };
+
+// LBG mode: column block s has converged (src/utils.rs:104-106).
+__device__ __forceinline__ bool block_done(const AssignArgs &a, int s) {
+    return a.before ? a.before[s] == 0 : a.done[s] != 0;
+}
 
 // Called by the lanes of a wave that changed a code.  Every store to one address is serialised
 // in its L2 channel and a million rows may change in a pass, so one lane of the wave stores, and
@@ -200,7 +206,7 @@ __global__ void __launch_bounds__(256) k_assign_static(AssignArgs a) {
     if constexpr (LBG) {
         any = false;
 #pragma unroll
-        for (int g = 0; g < G; ++g) any |= (a.done[s0 + g] == 0);
+        for (int g = 0; g < G; ++g) any |= !block_done(a, s0 + g);
         if (!any) return;  // uniform over the workgroup
     }
     // codebooks of blocks s0..s0+G-1 are contiguous: G*k*SD floats
@@ -252,7 +258,7 @@ __global__ void __launch_bounds__(256) k_assign_static(AssignArgs a) {
     for (int g = 0; g < G; ++g) {
         const int s = s0 + g;
         if constexpr (LBG) {
-            if (a.done[s]) continue;  // uniform
+            if (block_done(a, s)) continue;  // uniform
         }
         int best = argmin_lds<SD, METRIC>(x[g], lds + (size_t)g * k * SD, lds_cn + g * k, k);
         if constexpr (LBG) {
@@ -281,7 +287,7 @@ template <int METRIC, bool LBG>
 __global__ void __launch_bounds__(256) k_assign_dyn(AssignArgs a, int sd) {
     const int s = blockIdx.y;
     if constexpr (LBG) {
-        if (a.done[s]) return;
+        if (block_done(a, s)) return;
     }
     const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (row >= a.n) return;
@@ -952,7 +958,7 @@ __global__ void __launch_bounds__(256) k_assign_wide_exact(AssignArgs a, int sd,
     float *lds_x = lds_wide + (size_t)wave * kWideRows * sd;
     const int64_t total = LISTED ? (int64_t)*list_count : a.n;
     if constexpr (LBG && !LISTED) {
-        if (a.done[blockIdx.y]) return;
+        if (block_done(a, blockIdx.y)) return;
     }
     if constexpr (LISTED && VEC && (METRIC == M_SQ || METRIC == M_EUCLID)) {
         // a handful of pairs: one per workgroup, one centroid per thread

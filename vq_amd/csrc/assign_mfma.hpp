@@ -141,6 +141,7 @@ struct MfmaBfTables {
     const float *mu;       // [m][8]  the block's centre: mean of its centroids
     uint32_t *stat;        // [kStatSlots * kStatStride]  pairs decided by the exact path (measurement)
     int nb;                // blocks of 32 centroids, padded to an even number
+    uint32_t *stat_next = nullptr;  // (OWN) the counters of the pass after this one, to be cleared
 };
 
 // float -> bf16 bits, round to nearest even (NaN stays NaN).
@@ -244,13 +245,73 @@ __device__ __forceinline__ void mfma_bf_prep_block(float (&c)[8], int s, int j, 
 
 static __global__ void __launch_bounds__(256) k_mfma_bf_prep(const float *__restrict__ cb, int m, int k, int nb,
                                                              u32x4 *__restrict__ atab, float *__restrict__ maxc2,
-                                                             float *__restrict__ mu, uint32_t *__restrict__ stat) {
+                                                             float *__restrict__ mu, uint32_t *__restrict__ stat,
+                                                             uint32_t *__restrict__ stat_next) {
     const int s = blockIdx.x, j = threadIdx.x;
-    if (s == 0 && j < kStatSlots) stat[j * kStatStride] = 0u;
+    if (s == 0 && j < kStatSlots) stat[j * kStatStride] = stat_next[j * kStatStride] = 0u;
     float c[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) c[t] = (j < k) ? cb[((size_t)s * k + j) * 8 + t] : 0.0f;
     mfma_bf_prep_block(c, s, j, k, nb, atab, maxc2, mu);
+}
+
+// The tables of mfma_bf_prep_block made by one wave for itself (the same operands up to the order in
+// which the centre's sum is added, which any centre allows): lane (r, h) makes its own operands of
+// the centroids 32 b + r, dimensions [4h, 4h + 4), from the wave's copy of the centroids in LDS.
+__device__ __forceinline__ void own_operands(const float *cl, int k, int nb, int r, int h, u32x4 (&A1)[8],
+                                             u32x4 (&A2)[8], float (&muh)[4], float &mc2) {
+    float cv[8][4];
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        const int j = 32 * b + r;
+        const float4 v = *reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * 8 + 4 * h);
+        cv[b][0] = v.x, cv[b][1] = v.y, cv[b][2] = v.z, cv[b][3] = v.w;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sum[u] += j < k ? cv[b][u] * 0.00390625f : 0.0f;  // no overflow for k <= 256
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1) sum[u] += __shfl_xor(sum[u], off);  // over the lanes of this half
+        muh[u] = sum[u] * (256.0f / (float)k);
+    }
+    float mx = 0.0f;
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        if (b >= nb) {  // uniform; never multiplied
+            A1[b] = A1[0];
+            A2[b] = A2[0];
+            continue;
+        }
+        const bool live = 32 * b + r < k;
+        float p = 0.0f, a[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float c = live ? cv[b][u] - muh[u] : 0.0f;
+            p = __builtin_fmaf(c, c, p);
+            a[u] = -2.0f * c;
+        }
+        int pa, pb;
+        swap_halves(__float_as_int(p), pa, pb);
+        float c2 = __int_as_float(pa) + __int_as_float(pb);
+        mx = (mx == mx && c2 == c2) ? fmaxf(mx, c2) : __builtin_nanf("");
+        c2 = live ? c2 : kPadScore;
+        const uint32_t h01 = bf16_pack2(a[0], a[1]), h23 = bf16_pack2(a[2], a[3]);
+        const uint32_t l01 = bf16_pack2(a[0] - __uint_as_float(h01 << 16), a[1] - __uint_as_float(h01 & 0xffff0000u));
+        const uint32_t l23 = bf16_pack2(a[2] - __uint_as_float(h23 << 16), a[3] - __uint_as_float(h23 & 0xffff0000u));
+        const uint32_t c2a = bf16_rne_bits(c2);
+        const float c2r = c2 - bf16_bits_to_float(c2a);
+        const uint32_t c2b = bf16_rne_bits(c2r), c2c = bf16_rne_bits(c2r - bf16_bits_to_float(c2b));
+        A1[b] = u32x4{h01, h23, h01, h23};
+        A2[b] = u32x4{l01, l23, 0x3f803f80u, h == 0 ? (c2a | (c2b << 16)) : c2c};
+    }
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) {
+        const float o = __shfl_xor(mx, off);
+        mx = (mx == mx && o == o) ? fmaxf(mx, o) : __builtin_nanf("");
+    }
+    mc2 = mx;
 }
 
 // ---- the exact path of k_assign_mfma_bf ---------------------------------------------------------
@@ -352,7 +413,10 @@ __device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, fl
 // SG = 4: the four waves of a workgroup take the four column blocks of one 128-byte line of the
 // same rows.  SG = 1 (m not a multiple of 4): the four waves take consecutive runs of one block.
 // FULL: 8 blocks of 32 centroids (k above 224), scored without a branch between them.
-template <int METRIC, bool LBG, int SG, bool FULL>
+// OWN: every wave makes the operands, the centre and the bound of its block from the centroids it
+// holds in LDS, about 500 vector instructions, instead of reading the tables that k_mfma_bf_prep has
+// made: for grids of one round of workgroups, where that launch (6.5 us) is in the way.
+template <int METRIC, bool LBG, int SG, bool FULL, bool OWN = false>
 __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfTables tb, int run_tiles, int64_t nruns,
                                                             int64_t run_stride) {
     constexpr int SD = 8;
@@ -373,7 +437,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
     const int s = SG == 4 ? g * 4 + wave : g;
     if (run_first >= nruns) return;
     if constexpr (LBG) {
-        if (__builtin_amdgcn_readfirstlane(a.done[s]) != 0) return;  // the block has converged
+        if (__builtin_amdgcn_readfirstlane((int)block_done(a, s))) return;  // the block has converged
     }
 
     // the block's centroids: this wave's copy in LDS (no other wave reads it: no barrier)
@@ -389,9 +453,17 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
             if (i < nv) dst[i] = v;
         }
     }
-    // the A operands of every block of 32 centroids
+    // the A operands of every block of 32 centroids, the centre's dimensions [4h, 4h + 4), the bound
     u32x4 A1[8], A2[8];
-    {
+    float muh[4];
+    float mc2;
+    if constexpr (OWN) {
+        if (blockIdx.x == 0)
+            for (int i = threadIdx.x; i < kStatSlots; i += 256) tb.stat_next[i * kStatStride] = 0u;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        own_operands(cl, k, nb, r, h, A1, A2, muh, mc2);
+    } else {
         const u32x4 *ap = tb.atab + (size_t)s * nb * 128 + lane;
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
@@ -399,11 +471,10 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
             A1[b] = ap[(size_t)bc * 128];
             A2[b] = ap[(size_t)bc * 128 + 64];
         }
-    }
-    float muh[4];  // the centre's dimensions [4h, 4h + 4)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) muh[u] = tb.mu[(size_t)s * 8 + 4 * h + u];
-    const float mc2 = tb.maxc2[s];
+        for (int u = 0; u < 4; ++u) muh[u] = tb.mu[(size_t)s * 8 + 4 * h + u];
+        mc2 = tb.maxc2[s];
+    }
     const uint32_t keep = opaque_vgpr(0xFFFFFF00u);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -871,7 +942,7 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
     __shared__ uint32_t wg_count, wg_base, wg_pcount, wg_pbase;
     const int s = blockIdx.y;
     if constexpr (LBG) {
-        if (a.done[s]) return;
+        if (block_done(a, s)) return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 31, h = lane >> 5;

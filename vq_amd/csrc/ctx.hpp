@@ -32,6 +32,8 @@ struct vq_ctx {
     DevBuf tsvq_means;           // TSVQ build: the means of all nodes, read back once at the end
     DevBuf tsvq_scan;            // TSVQ build: workspace of the partition's prefix scan
     DevBuf tsvq_km;              // TSVQ build with 2-means splits: centroids, part sums, flags, draws of a level
+    void *lbg_pin = nullptr;     // LBG: page-locked index streams and results of a fit
+    size_t lbg_pin_cap = 0;
     void *tsvq_pin = nullptr;    // TSVQ build: page-locked staging of a level's tables and decisions
     size_t tsvq_pin_cap = 0;
     // vq_h2d from pageable memory: page-locked staging buffers and the events of their uploads
@@ -43,8 +45,10 @@ struct vq_ctx {
     int tsvq_var_path = 0;       // 0 = composed integer maps, 1 = one chain of adds per column
     DevBuf pad_x, pad_cb;        // rows and codebooks whose column blocks are padded to a multiple of 8 floats
     DevBuf mfma_tab, mfma_list, mfma_stat;  // tables, re-check list and counters of the matrix-core assignment
+    int mfma_stat_cur = 0;       // which of the two sets of counters in mfma_stat the last pass used
     int recheck_src = 0;         // where the last pass counted its undecided pairs: 1 mfma_stat, 2 mfma_list, 3 the fixed scratch
     int assign_path = 0;         // 0 = matrix cores where a kernel exists, 1 = vector ALU only
+    bool lbg_small_lds_set = false;  // dynamic-LDS limit granted to k_lbg_update_small
     int compute_units = 0;       // of the context's GPU (0: not asked for yet)
     int decode_lds_set[4] = {0, 0, 0, 0};  // dynamic-LDS limit already granted to the four resident decode kernels
     int tsvq_descend_path = 0;   // 0 = one inner product per node where it decides (cosine, L2), 1 = two distances per node always
@@ -118,6 +122,21 @@ inline int32_t ensure(vq_ctx *ctx, DevBuf &b, size_t bytes) {
     size_t want = bytes + bytes / 8 + 256;
     VQ_HIP(ctx, hipMalloc(&b.p, want));
     b.cap = want;
+    return VQ_OK;
+}
+
+// Page-locked host memory of the context, grow-only (the device reads and writes it in place).
+inline int32_t ensure_pinned(vq_ctx *ctx, void *&p, size_t &cap, size_t bytes) {
+    if (bytes <= cap) return VQ_OK;
+    if (p) {
+        VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        VQ_HIP(ctx, hipHostFree(p));
+        p = nullptr;
+        cap = 0;
+    }
+    const size_t want = bytes + bytes / 8 + 4096;
+    VQ_HIP(ctx, hipHostMalloc(&p, want, hipHostMallocDefault));
+    cap = want;
     return VQ_OK;
 }
 

@@ -634,6 +634,361 @@ static __global__ void __launch_bounds__(256) k_lbg_finalize(LbgState st, const 
     *out = sum / __uint2float_rn(cnt);
 }
 
+// ---- the whole update of a small fit in one launch ------------------------------------------------
+// Below some ten thousand rows every kernel of the path above is a handful of waves and the update is
+// a chain of launches and memory round trips: 75 us per iteration at 10,000 x 128, m = 16, k = 256 (the
+// streaming kernel's 12 workgroups 47 of them), 11 us here; 29 us at 50,000 rows.  Here a workgroup owns C clusters of one column block:
+// it reads all codes of the block, lists the rows of its own clusters in row order, sorts a window of
+// the list by cluster (a stable counting sort by ballots), brings the window's sub-vectors into LDS
+// (every load of up to 8192 floats in flight together), and one lane per (cluster, component) adds
+// them in list order, eight LDS reads ahead.  The orders of summation are those above: row order up
+// to 1024 members, part sums in part order above.
+// STAGED: sub_dim a multiple of 4 up to 512, a thread per component.  Else (wider blocks) a wave takes
+// one cluster and 64 components at a time and reads the rows themselves, 16 rows in flight.
+constexpr int kSmallList = 8192;    // listed rows held before the list is worked off: at least 16 per thread
+constexpr int kSmallThreads = 512;  // one workgroup per compute unit: eight waves
+constexpr int kSmallWindow = 4 * kSmallThreads;  // listed rows sorted at a time
+constexpr int kSmallClusters = 16;  // most clusters per workgroup: four bits of a list entry
+constexpr int kSmallWaves = kSmallThreads / 64;
+constexpr int kSmallStage = 32 * kSmallThreads;  // floats staged at a time: eight 16-byte loads per thread in flight
+
+// Workgroup number -> index such that each XCD (workgroups are dealt to the 8 XCDs in turn) gets a
+// contiguous range: the workgroups that read the same codes and the same lines share an L2.
+__device__ __forceinline__ unsigned xcd_contiguous(unsigned id, unsigned total) {
+    const unsigned per = total / 8u, rest = total % 8u, xcd = id % 8u;
+    return xcd * per + (xcd < rest ? xcd : rest) + id / 8u;
+}
+
+// The loop control of src/utils.rs:57,104-106 needs no launch of its own: every iteration has its own
+// flags.  changed[it][s], it >= 1: a code of block s changed in iteration it - 1 (changed[0] is all
+// ones); a block whose flag is 0 has converged, and its later flags then stay 0.  empties[it][s]: empty
+// clusters re-seeded in iteration it, whose sum over the iterations before is the block's place in
+// its re-seed stream.
+struct LbgSmall {
+    int *changed;    // [max_iters + 1][m]
+    int *empties;    // [max_iters][m]
+    int *err;        // 1   set to 1 when a re-seed stream runs out
+    uint8_t *codes;  // [m][n]
+};
+
+// codes = 0 (src/utils.rs:55), the flags, and the initial centroids x[idx[s][j]] (src/utils.rs:54; with
+// pend_cb, one column block: the row as the pending residual update will leave it).
+static __global__ void __launch_bounds__(256) k_lbg_small_init(LbgSmall st, const float *__restrict__ x, int64_t n,
+                                                               int64_t ld, int m, int k, int sd, int max_iters,
+                                                               const uint32_t *__restrict__ idx, float *__restrict__ cb,
+                                                               const float *__restrict__ pend_cb,
+                                                               const uint8_t *__restrict__ pend_codes) {
+    const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
+    for (int64_t i = i0; i < (int64_t)m * k * sd; i += stride) {
+        const int t = (int)(i % sd);
+        const int64_t sj = i / sd;
+        const uint32_t row = idx[sj];
+        const float v = x[(int64_t)row * ld + (sj / k) * sd + t];
+        cb[i] = pend_cb ? v - pend_cb[(size_t)pend_codes[row] * sd + t] : v;
+    }
+    for (int64_t i = i0; i < ((int64_t)m * n + 3) / 4; i += stride) reinterpret_cast<uint32_t *>(st.codes)[i] = 0u;
+    for (int64_t i = i0; i < (int64_t)(2 * max_iters + 1) * m + 1; i += stride) st.changed[i] = i < m ? 1 : 0;
+}
+
+// The flags to page-locked host memory.
+static __global__ void __launch_bounds__(256) k_lbg_small_report(const int *__restrict__ flags, int count, int *out) {
+    for (int i = threadIdx.x; i < count; i += 256) out[i] = flags[i];
+}
+
+template <bool STAGED>
+static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSmall st, int it, int m,
+                                                                           const float *__restrict__ x, int64_t n,
+                                                                           int64_t ld, int sd, int k, int C, int groups,
+                                                                           const uint32_t *__restrict__ reseed,
+                                                                           int n_reseed, float *__restrict__ cb) {
+    const unsigned id = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int s = (int)(id / (unsigned)groups), j0 = (int)(id % (unsigned)groups) * C;
+    if (st.changed[it * m + s] == 0) return;  // converged before this iteration
+    const int jn = k - j0 < C ? k - j0 : C;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    __shared__ uint32_t list[kSmallList];          // row | cluster << 28
+    __shared__ uint32_t sorted[kSmallWindow];      // the window's rows, cluster by cluster
+    __shared__ uint32_t hist[kSmallWindow / 64][kSmallClusters];
+    __shared__ uint32_t cl_off[kSmallClusters + 1];  // first position of a cluster in the sorted window
+    __shared__ uint32_t cl_cnt[kSmallClusters];      // members
+    __shared__ uint32_t cl_part[kSmallClusters];     // (not STAGED) part of the last member added
+    __shared__ uint32_t wave_tot[2][kSmallWaves];
+    extern __shared__ float dyn[];  // STAGED: the sub-vectors; else three sums per (cluster, component)
+    const uint8_t *codes = st.codes + (size_t)s * n;
+    const float *xs = x + (int64_t)s * sd;
+    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    if (tid < kSmallClusters) {
+        cl_cnt[tid] = 0u;
+        cl_part[tid] = 0u;
+    }
+    if constexpr (!STAGED)
+        for (int i = tid; i < 3 * C * sd; i += kSmallThreads) dyn[i] = 0.0f;
+    float *sseq = dyn, *stot = dyn + C * sd, *spart = dyn + 2 * C * sd;
+    // STAGED: the sums of this thread's (cluster, component): in row order; and by parts
+    float seq = 0.0f, total = 0.0f, part = 0.0f;
+    uint32_t cur_part = 0;
+    const int my_c = STAGED ? tid / sd : 0, my_t = STAGED ? tid % sd : 0;
+    const bool summing = STAGED && my_c < jn;
+    bool track = false, drained = false;  // uniform; track: the part sums are needed as well
+    uint32_t cnt = 0;                     // entries of list, uniform
+
+    // one member's value into (row-order sum; closed parts, open part)
+    auto add_tracked = [](float v, uint32_t row, float &a, float &tt, float &pp, uint32_t &open) {
+        const uint32_t p = row / (uint32_t)kPartRows;
+        const bool close = p != open;
+        const float closed = tt + pp;
+        tt = close ? closed : tt;
+        pp = close ? 0.0f : pp;
+        open = p;
+        a = a + v;
+        pp = pp + v;
+    };
+    auto drain = [&]() {
+        for (uint32_t w0 = 0; w0 < cnt; w0 += kSmallWindow) {
+            const uint32_t wn = cnt - w0 < (uint32_t)kSmallWindow ? cnt - w0 : (uint32_t)kSmallWindow;
+            // ranks inside chunks of 64 entries, chunk kSmallWaves * u + wave by this wave
+            uint32_t ent[4], rank[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t i = 64u * (kSmallWaves * u + wave) + lane;
+                const bool valid = i < wn;
+                ent[u] = valid ? list[w0 + i] : 0u;
+                const uint32_t c = ent[u] >> 28;
+                uint64_t same = __ballot(valid);
+#pragma unroll
+                for (int bit = 0; bit < 4; ++bit) {
+                    const bool set = (c >> bit) & 1u;
+                    const uint64_t bal = __ballot(set);
+                    same &= set ? bal : ~bal;
+                }
+                rank[u] = (uint32_t)__popcll(same & lt);
+                if (lane < kSmallClusters) hist[kSmallWaves * u + wave][lane] = 0u;
+                __builtin_amdgcn_wave_barrier();  // one wave's LDS operations are performed in order
+                if (valid && rank[u] == 0) hist[kSmallWaves * u + wave][c] = (uint32_t)__popcll(same);
+            }
+            __syncthreads();
+            if (tid < kSmallClusters) {  // exclusive prefixes over the chunks, then over the clusters
+                uint32_t h[kSmallWindow / 64], run = 0;
+#pragma unroll
+                for (int q = 0; q < kSmallWindow / 64; ++q) h[q] = hist[q][tid];
+#pragma unroll
+                for (int q = 0; q < kSmallWindow / 64; ++q) {
+                    hist[q][tid] = run;
+                    run += h[q];
+                }
+                uint32_t inc = run;
+#pragma unroll
+                for (int off = 1; off < kSmallClusters; off <<= 1) {
+                    const uint32_t o = __shfl_up(inc, off);
+                    if (tid >= off) inc += o;
+                }
+                cl_off[tid + 1] = inc;
+                if (tid == 0) cl_off[0] = 0u;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t i = 64u * (kSmallWaves * u + wave) + lane, c = ent[u] >> 28;
+                if (i < wn) sorted[cl_off[c] + hist[kSmallWaves * u + wave][c] + rank[u]] = ent[u] & 0x0fffffffu;
+            }
+            __syncthreads();
+            if constexpr (STAGED) {
+                const uint32_t per = (uint32_t)sd / 4u, most = (uint32_t)kSmallStage / (uint32_t)sd;
+                typedef float piece4 __attribute__((ext_vector_type(4), aligned(4)));
+                for (uint32_t p0 = 0; p0 < wn; p0 += most) {
+                    const uint32_t pn = wn - p0 < most ? wn - p0 : most;
+                    constexpr int E = kSmallStage / 4 / kSmallThreads;
+                    piece4 v[E];
+#pragma unroll
+                    for (int e = 0; e < E; ++e) {
+                        const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * e, ic = i < pn * per ? i : 0u;
+                        v[e] = *reinterpret_cast<const piece4 *>(xs + (int64_t)sorted[p0 + ic / per] * ld + 4u * (ic % per));
+                    }
+#pragma unroll
+                    for (int e = 0; e < E; ++e) {
+                        const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * e;
+                        if (i < pn * per)
+                            *reinterpret_cast<float4 *>(dyn + 4u * i) = make_float4(v[e][0], v[e][1], v[e][2], v[e][3]);
+                    }
+                    __syncthreads();
+                    if (summing) {
+                        const uint32_t c_lo = cl_off[my_c], c_hi = cl_off[my_c + 1];
+                        uint32_t i = c_lo > p0 ? c_lo - p0 : 0u;
+                        const uint32_t end = c_hi > p0 ? c_hi - p0 : 0u, hi = end < pn ? end : pn;
+                        const float *d = dyn + my_t;
+                        if (track) {
+                            for (; i + 8 <= hi; i += 8) {
+                                float t[8];
+                                uint32_t row[8];
+#pragma unroll
+                                for (int u = 0; u < 8; ++u) {
+                                    t[u] = d[(i + u) * (uint32_t)sd];
+                                    row[u] = sorted[p0 + i + u];
+                                }
+#pragma unroll
+                                for (int u = 0; u < 8; ++u) add_tracked(t[u], row[u], seq, total, part, cur_part);
+                            }
+                            for (; i < hi; ++i) add_tracked(d[i * (uint32_t)sd], sorted[p0 + i], seq, total, part, cur_part);
+                        } else {
+                            for (; i + 8 <= hi; i += 8) {
+                                float t[8];
+#pragma unroll
+                                for (int u = 0; u < 8; ++u) t[u] = d[(i + u) * (uint32_t)sd];
+#pragma unroll
+                                for (int u = 0; u < 8; ++u) seq = seq + t[u];
+                            }
+                            for (; i < hi; ++i) seq = seq + d[i * (uint32_t)sd];
+                        }
+                    }
+                    __syncthreads();
+                }
+            } else {
+                const int slices = (sd + 63) / 64;
+                for (int task = wave; task < jn * slices; task += kSmallWaves) {
+                    const int c = task / slices, t = (task % slices) * 64 + lane, tc = t < sd ? t : sd - 1;
+                    const float *col = xs + tc;
+                    const uint32_t lo = cl_off[c], hi = cl_off[c + 1];
+                    if (lo >= hi) continue;
+                    float a = sseq[c * sd + tc], tt = stot[c * sd + tc], pp = spart[c * sd + tc];
+                    uint32_t open = cl_part[c];
+                    constexpr int B = 16;
+                    for (uint32_t i = lo; i < hi; i += B) {
+                        float v[B];
+                        uint32_t r[B];
+#pragma unroll
+                        for (int u = 0; u < B; ++u) r[u] = sorted[i + u < hi ? i + u : hi - 1];
+#pragma unroll
+                        for (int u = 0; u < B; ++u) v[u] = col[(int64_t)r[u] * ld];
+#pragma unroll
+                        for (int u = 0; u < B; ++u)
+                            if (i + u < hi) {
+                                if (track) add_tracked(v[u], r[u], a, tt, pp, open);
+                                else a = a + v[u];
+                            }
+                    }
+                    if (t < sd) {
+                        sseq[c * sd + t] = a;
+                        stot[c * sd + t] = tt;
+                        spart[c * sd + t] = pp;
+                    }
+                }
+                __syncthreads();
+                if (tid < jn && cl_off[tid] < cl_off[tid + 1])
+                    cl_part[tid] = sorted[cl_off[tid + 1] - 1] / (uint32_t)kPartRows;
+                __syncthreads();
+            }
+        }
+        cnt = 0;
+        drained = true;
+    };
+
+    // 16 consecutive codes per thread and step, the next step's in flight
+    typedef uint32_t codes16 __attribute__((ext_vector_type(4), aligned(1)));
+    auto fetch = [&](int64_t r0, uint32_t &have) {
+        codes16 v = {0u, 0u, 0u, 0u};
+        have = r0 >= n ? 0u : (n - r0 < 16 ? (1u << (uint32_t)(n - r0)) - 1u : 0xffffu);
+        if (have == 0xffffu) {
+            v = *reinterpret_cast<const codes16 *>(codes + r0);
+        } else if (have) {
+            for (int u = 0; u < (int)(n - r0); ++u) v[u >> 2] |= (uint32_t)codes[r0 + u] << (8 * (u & 3));
+        }
+        return v;
+    };
+    uint32_t have_next;
+    codes16 next = fetch(16 * tid, have_next);
+    constexpr int kStep = 16 * kSmallThreads;  // rows
+    const int nsteps = (int)((n + kStep - 1) / kStep);
+    for (int p = 0; p < nsteps; ++p) {
+        const uint32_t row0 = (uint32_t)p * (uint32_t)kStep + 16u * tid;
+        const codes16 v = next;
+        const uint32_t have = have_next;
+        next = fetch((int64_t)row0 + kStep, have_next);
+        uint32_t mine = 0;  // bit u: row row0 + u belongs to one of the workgroup's clusters
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const uint32_t c = (v[u >> 2] >> (8 * (u & 3))) & 0xffu;
+            mine |= (c - (uint32_t)j0 < (uint32_t)jn ? 1u : 0u) << u;
+        }
+        mine &= have;
+        const uint32_t m1 = __popc(mine);
+        uint32_t inc = m1;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_up(inc, off);
+            if (lane >= off) inc += o;
+        }
+        if (lane == 63) wave_tot[p & 1][wave] = inc;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < kSmallWaves; ++w) {
+            const uint32_t t = wave_tot[p & 1][w];
+            before += w < wave ? t : 0u;
+            all += t;
+        }
+        if (cnt + all > (uint32_t)kSmallList) {  // the sizes of the clusters are not known yet: keep both sums
+            track = true;
+            drain();
+        }
+        uint32_t at = cnt + before + inc - m1;
+        for (uint32_t mm = mine; mm; mm &= mm - 1) {
+            const uint32_t u = (uint32_t)__ffs(mm) - 1u;
+            const uint32_t w = u < 8u ? (u < 4u ? v[0] : v[1]) : (u < 12u ? v[2] : v[3]);
+            const uint32_t c = ((w >> (8u * (u & 3u))) & 0xffu) - (uint32_t)j0;
+            list[at++] = (row0 + u) | (c << 28);
+            atomicAdd(&cl_cnt[c], 1u);
+        }
+        cnt += all;
+    }
+    __syncthreads();
+    if (!drained) {
+        for (int c = 0; c < jn; ++c) track = track || cl_cnt[c] > (uint32_t)kSeqMax;
+    }
+    drain();
+    float *out = cb + ((size_t)s * k + j0) * sd;
+    if constexpr (STAGED) {
+        if (summing) {
+            const uint32_t cm = cl_cnt[my_c];
+            if (cm) out[my_c * sd + my_t] = (cm <= (uint32_t)kSeqMax ? seq : total + part) / __uint2float_rn(cm);
+        }
+    } else {
+        for (int i = tid; i < jn * sd; i += kSmallThreads) {
+            const uint32_t cm = cl_cnt[i / sd];
+            if (cm) out[i] = (cm <= (uint32_t)kSeqMax ? sseq[i] : stot[i] + spart[i]) / __uint2float_rn(cm);
+        }
+    }
+    // Empty clusters take the next rows of the block's re-seed stream in cluster order
+    // (src/utils.rs:98-101): the workgroup goes over the codes once more for the clusters that have
+    // members (`list` is free by now).
+    bool open = false;
+    for (int c = 0; c < jn; ++c) open = open || cl_cnt[c] == 0u;
+    if (!open) return;
+    for (int j = tid; j < kMaxK; j += kSmallThreads) list[j] = 0u;
+    __syncthreads();
+    for (int64_t i = tid; i < n; i += kSmallThreads) list[codes[i]] = 1u;
+    __syncthreads();
+    if (tid == 0) {
+        int used = 0, mine = 0;
+        for (int i = 0; i < it; ++i) used += st.empties[i * m + s];
+        for (int j = 0; j < j0; ++j) used += list[j] == 0u;
+        for (int c = 0; c < jn; ++c) {
+            cl_off[c] = (uint32_t)(used + mine);  // place in the stream
+            mine += cl_cnt[c] == 0u;
+        }
+        atomicAdd(st.empties + it * m + s, mine);
+    }
+    __syncthreads();
+    for (int i = tid; i < jn * sd; i += kSmallThreads) {
+        const int c = i / sd, t = i % sd;
+        if (cl_cnt[c]) continue;
+        const int pos = (int)cl_off[c];
+        if (pos >= n_reseed)
+            st.err[0] = 1;  // the centroid stays
+        else
+            out[i] = xs[(int64_t)reseed[(size_t)s * n_reseed + pos] * ld + t];
+    }
+}
+
 // ---- streaming sums of the large clusters (sub_dim 8, 4 column blocks per 128-byte line) ------
 // One workgroup per (part, group of 4 column blocks); wave w of the group owns column block
 // 4g + w, so the four waves together consume whole 128-byte lines of the rows.  A wave walks
@@ -842,9 +1197,10 @@ static __global__ void k_lbg_advance(LbgState st, int m) {
 static __global__ void __launch_bounds__(256) k_lbg_finalize_prep8(
     LbgState st, const float *__restrict__ x, int64_t ld, int k, const uint32_t *__restrict__ reseed, int n_reseed,
     float *__restrict__ cb, const float *__restrict__ big_sum, int nb, u32x4 *__restrict__ atab,
-    float *__restrict__ maxc2, float *__restrict__ mu, uint32_t *__restrict__ stat) {
+    float *__restrict__ maxc2, float *__restrict__ mu, uint32_t *__restrict__ stat,
+                                                             uint32_t *__restrict__ stat_next) {
     const int s = blockIdx.x, j = threadIdx.x;
-    if (s == 0 && j < kStatSlots) stat[j * kStatStride] = 0u;
+    if (s == 0 && j < kStatSlots) stat[j * kStatStride] = stat_next[j * kStatStride] = 0u;
     if (st.done[s]) return;  // the same in the whole workgroup; a finished block is skipped by the assignment
     float c[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (j < k) {

@@ -26,6 +26,12 @@
 #ifndef VQ_MFMA_WGS
 #define VQ_MFMA_WGS 3072 // workgroups of the matrix-core assignment: four rounds of three per compute unit
 #endif
+#ifndef VQ_MFMA_ROUND
+#define VQ_MFMA_ROUND 768  // workgroups of one round: three per compute unit
+#endif
+#ifndef VQ_MFMA_OWN
+#define VQ_MFMA_OWN 8    // most tiles per workgroup of a one-round grid
+#endif
 #include "lbg_update.hpp"
 #include "calibrate.hpp"
 
@@ -135,7 +141,7 @@ int32_t launch_assign_m(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
 struct MfmaTabPtrs {
     vq::u32x4 *atab;
     float *maxc2, *mu;
-    uint32_t *stat;
+    uint32_t *stat, *stat_next;  // the counters of this pass; of the next one
     int nb;
 };
 int32_t mfma_tab_ptrs(vq_ctx *ctx, int m, int k, MfmaTabPtrs &t) {
@@ -146,16 +152,21 @@ int32_t mfma_tab_ptrs(vq_ctx *ctx, int m, int k, MfmaTabPtrs &t) {
         t.atab = (vq::u32x4 *)ctx->static_scratch;
         t.maxc2 = (float *)(ctx->static_scratch + kNoAllocAuxOff);
         t.mu = t.maxc2 + m;
-        t.stat = (uint32_t *)(ctx->static_scratch + kNoAllocStatOff);
+        t.stat = t.stat_next = (uint32_t *)(ctx->static_scratch + kNoAllocStatOff);
         return VQ_OK;
     }
     VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + 9 * (size_t)m) + 64));
-    VQ_TRY(ensure(ctx, ctx->mfma_stat, sizeof(uint32_t) * vq::kStatSlots * vq::kStatStride));
+    const size_t n_stat = (size_t)vq::kStatSlots * vq::kStatStride;
+    if (!ctx->mfma_stat.p) {
+        VQ_TRY(ensure(ctx, ctx->mfma_stat, sizeof(uint32_t) * 2 * n_stat));
+        VQ_HIP(ctx, hipMemsetAsync(ctx->mfma_stat.p, 0, sizeof(uint32_t) * 2 * n_stat, ctx->stream));
+    }
     float *atab = (float *)ctx->mfma_tab.p;
     t.atab = (vq::u32x4 *)atab;
     t.maxc2 = atab + n_atab;
     t.mu = t.maxc2 + m;
-    t.stat = (uint32_t *)ctx->mfma_stat.p;
+    t.stat = (uint32_t *)ctx->mfma_stat.p + ctx->mfma_stat_cur * n_stat;
+    t.stat_next = (uint32_t *)ctx->mfma_stat.p + (ctx->mfma_stat_cur ^ 1) * n_stat;
     return VQ_OK;
 }
 
@@ -168,26 +179,23 @@ int32_t mfma_tab_ptrs(vq_ctx *ctx, int m, int k, MfmaTabPtrs &t) {
 template <int METRIC, bool LBG>
 int32_t launch_mfma(vq_ctx *ctx, const vq::AssignArgs &a, bool tables_ready, hipEvent_t *started = nullptr,
                     hipEvent_t *done = nullptr) {
-    MfmaTabPtrs t;
-    VQ_TRY(mfma_tab_ptrs(ctx, a.m, a.k, t));
-    const int nb = t.nb;
-    if (!tables_ready)
-        hipLaunchKernelGGL(vq::k_mfma_bf_prep, dim3(a.m), dim3(256), 0, ctx->stream, a.cb, a.m, a.k, nb, t.atab,
-                           t.maxc2, t.mu, t.stat);
-    vq::MfmaBfTables tb{(const vq::u32x4 *)t.atab, t.maxc2, t.mu, t.stat, nb};
     // a workgroup = 4 column blocks of 8 floats (one 128-byte line per row) against one run of row
     // tiles, or, where m is not a multiple of 4, one column block against four runs
+    const int nb = 2 * ((a.k + 63) / 64);
     const bool grouped = a.m % 4 == 0, full = nb == 8;
-    const void *kern =
-        grouped ? (full ? (const void *)vq::k_assign_mfma_bf<METRIC, LBG, 4, true> : (const void *)vq::k_assign_mfma_bf<METRIC, LBG, 4, false>)
-                : (full ? (const void *)vq::k_assign_mfma_bf<METRIC, LBG, 1, true> : (const void *)vq::k_assign_mfma_bf<METRIC, LBG, 1, false>);
     // A wave loads the operands of its column block once (16 KB + 8 KB) and amortises them over
     // its run: 8 tiles of 32 rows where that still leaves several rounds of workgroups per compute unit.
     const int64_t tiles = cdiv(a.n, 32);
-    const int64_t groups = grouped ? a.m / 4 : a.m;
+    const int64_t groups = grouped ? a.m / 4 : a.m, per_run = grouped ? 1 : 4;
     int run_tiles = VQ_MFMA_RUN;
-    while (run_tiles > 1 && cdiv(tiles, (grouped ? 1 : 4) * run_tiles) * groups < 8192) run_tiles >>= 1;
-    int64_t runs = cdiv(tiles, (grouped ? 1 : 4) * (int64_t)run_tiles);
+    while (run_tiles > 1 && cdiv(tiles, per_run * run_tiles) * groups < 8192) run_tiles >>= 1;
+    // Up to VQ_MFMA_OWN tiles for each workgroup of a single round: what counts then is the time of one
+    // workgroup, and every wave makes its operands itself (OWN) instead of waiting for the launch that
+    // makes the tables (10,000 x 128, m = 16: 14.5 us after a launch of 6.5 us -> 15.0 us).
+    const int64_t share = cdiv(tiles * groups, per_run * VQ_MFMA_ROUND);
+    const bool own = !tables_ready && !ctx->no_alloc && share <= VQ_MFMA_OWN;
+    if (own) run_tiles = (int)share;
+    const int64_t runs = cdiv(tiles, per_run * (int64_t)run_tiles);
     // a workgroup walks over several runs with the operands it has loaded once; the grid is a few
     // rounds of the three workgroups a compute unit holds (768: the slowest workgroup sets the
     // time; one workgroup per run: the operands are loaded 15,000 times), a multiple of 8 per group
@@ -195,6 +203,23 @@ int32_t launch_mfma(vq_ctx *ctx, const vq::AssignArgs &a, bool tables_ready, hip
     run_stride = std::min<int64_t>(run_stride, cdiv(runs, 8) * 8);
     const int64_t blocks = run_stride * groups;
     if (blocks >= (1LL << 31)) return fail(ctx, VQ_ERR_UNSUPPORTED, "n * m too large for one launch");
+    if (own) ctx->mfma_stat_cur ^= 1;  // cleared by the pass before
+    MfmaTabPtrs t;
+    VQ_TRY(mfma_tab_ptrs(ctx, a.m, a.k, t));
+    if (!tables_ready && !own)
+        hipLaunchKernelGGL(vq::k_mfma_bf_prep, dim3(a.m), dim3(256), 0, ctx->stream, a.cb, a.m, a.k, nb, t.atab,
+                           t.maxc2, t.mu, t.stat, t.stat_next);
+    vq::MfmaBfTables tb{(const vq::u32x4 *)t.atab, t.maxc2, t.mu, t.stat, nb, t.stat_next};
+    auto pick = [&](auto SGc, auto FULLc) {
+        constexpr int SGv = decltype(SGc)::value;
+        constexpr bool FULLv = decltype(FULLc)::value;
+        return own ? (const void *)vq::k_assign_mfma_bf<METRIC, LBG, SGv, FULLv, true>
+                   : (const void *)vq::k_assign_mfma_bf<METRIC, LBG, SGv, FULLv, false>;
+    };
+    using Four = std::integral_constant<int, 4>;
+    using One = std::integral_constant<int, 1>;
+    const void *kern = grouped ? (full ? pick(Four{}, std::true_type{}) : pick(Four{}, std::false_type{}))
+                               : (full ? pick(One{}, std::true_type{}) : pick(One{}, std::false_type{}));
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     if (ctx->prof_on) {
         ev_a = prof_event(ctx);
@@ -204,7 +229,8 @@ int32_t launch_mfma(vq_ctx *ctx, const vq::AssignArgs &a, bool tables_ready, hip
         ev_b = ctx->ev_fork;
     }
     vq::AssignArgs aa = a;
-    void *args[] = {&aa, &tb, &run_tiles, &runs, &run_stride};
+    int64_t runs_arg = runs;
+    void *args[] = {&aa, &tb, &run_tiles, &runs_arg, &run_stride};
     if (ev_a || ev_b)
         VQ_HIP(ctx, hipExtLaunchKernel(kern, dim3((unsigned)blocks), dim3(256), args, 0, ctx->stream, ev_a, ev_b, 0u));
     else
@@ -697,6 +723,7 @@ int32_t vq_ctx_destroy(vq_ctx *ctx) {
     for (DevBuf *b : bufs)
         if (b->p) (void)hipFree(b->p);
     if (ctx->tsvq_pin) (void)hipHostFree(ctx->tsvq_pin);
+    if (ctx->lbg_pin) (void)hipHostFree(ctx->lbg_pin);
     for (int i = 0; i < vq_ctx::kStageBuffers; ++i) {
         if (ctx->h2d_stage[i]) (void)hipHostFree(ctx->h2d_stage[i]);
         if (ctx->h2d_event[i]) (void)hipEventDestroy(ctx->h2d_event[i]);
@@ -1047,7 +1074,9 @@ int32_t vq_ctx_last_recheck_split(vq_ctx *ctx, uint32_t *h_count, uint32_t *h_tw
     *h_two = 0;
     if (ctx->recheck_src == 1 || ctx->recheck_src == 3) {
         uint32_t h[vq::kStatSlots * vq::kStatStride];
-        const void *src = ctx->recheck_src == 1 ? ctx->mfma_stat.p : ctx->static_scratch + kNoAllocStatOff;
+        const void *src = ctx->recheck_src == 1
+                              ? (const void *)((uint32_t *)ctx->mfma_stat.p + ctx->mfma_stat_cur * vq::kStatSlots * vq::kStatStride)
+                              : ctx->static_scratch + kNoAllocStatOff;
         VQ_HIP(ctx, hipMemcpyAsync(h, src, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
         VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
         for (int i = 0; i < vq::kStatSlots; ++i) *h_count += h[i * vq::kStatStride];
@@ -1164,6 +1193,108 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
                        h_iters_run, h_reseeds_used, pend_cb, pend_codes, [] {});
 }
 
+// Clusters per workgroup of k_lbg_update_small: as many as one thread per (cluster, component) and
+// four bits per list entry allow, but at least a workgroup per compute unit.
+static int lbg_small_clusters(int m, int sd, int k) {
+    return (int)std::max<int64_t>(1, std::min<int64_t>({vq::kSmallClusters, (int64_t)k * m / 256,
+                                                        (sd <= vq::kSmallThreads ? vq::kSmallThreads : 4096) / sd}));
+}
+
+// Whether the update of a fit runs as k_lbg_update_small.  Its time follows the members of a cluster
+// (one chain of additions each) and the floats that a workgroup brings in, the other path's the number
+// of its launches.  The two take the same time near 700 members where the chain decides (blocks of
+// 8 floats, k = 116) and near 40,000-50,000 floats (130 members of 256, 250 of 128, four clusters of 250
+// members of 48), on uniform rows and on mixtures; above 32 components, where the rows are often
+// residuals with clusters of very different sizes (one workgroup works off the largest alone), the line
+// lies at half of that.  Ten iterations, m = 16, k = 256, blocks of 8: 2,000
+// rows 0.83 -> 0.22 ms, 10,000 1.07 -> 0.29 ms, 50,000 1.35 -> 0.74 ms.
+static bool lbg_small(int64_t n, int m, int sd, int k) {
+    if (sd % 4 != 0 || sd > 4096 || n > 131072) return false;
+    if (sd > vq::kSmallThreads) return n <= 128 * (int64_t)k;
+    return n <= 640 * (int64_t)k && n * lbg_small_clusters(m, sd, k) * sd <= (sd <= 32 ? 40960 : 20480) * (int64_t)k;
+}
+
+// The LBG loop of a small fit, two launches per iteration: the assignment and k_lbg_update_small.  The
+// index streams stay in page-locked host memory: the initial rows are read once, re-seed rows rarely.
+template <typename Last>
+static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
+                             int32_t max_iters, const uint32_t *h_init_idx, const uint32_t *h_reseed_stream,
+                             int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used,
+                             const float *pend_cb, const uint8_t *pend_codes, const Last &last) {
+    hipStream_t st = ctx->stream;
+    const size_t n_flags = (2 * (size_t)max_iters + 1) * m + 1, n_idx = (size_t)m * k, n_res = (size_t)m * n_reseed;
+    VQ_TRY(ensure(ctx, ctx->flags, sizeof(int) * n_flags));
+    VQ_TRY(ensure(ctx, ctx->codes, (size_t)m * n + 4));
+    VQ_TRY(ensure_pinned(ctx, ctx->lbg_pin, ctx->lbg_pin_cap, sizeof(uint32_t) * (n_idx + n_res + n_flags)));
+    uint32_t *idx = (uint32_t *)ctx->lbg_pin, *reseed = idx + n_idx;
+    int *report = (int *)(reseed + n_res);
+    memcpy(idx, h_init_idx, sizeof(uint32_t) * n_idx);
+    if (n_res) memcpy(reseed, h_reseed_stream, sizeof(uint32_t) * n_res);
+    vq::LbgSmall S;
+    S.changed = (int *)ctx->flags.p;
+    S.empties = S.changed + (size_t)(max_iters + 1) * m;
+    S.err = S.empties + (size_t)max_iters * m;
+    S.codes = (uint8_t *)ctx->codes.p;
+    const int64_t init_items = std::max<int64_t>((int64_t)m * k * sd, (int64_t)m * n / 4);
+    hipLaunchKernelGGL(vq::k_lbg_small_init, dim3(std::min<unsigned>(cdiv(init_items, 256), 1024u)), dim3(256), 0, st, S,
+                       d_x, n, ld, m, k, sd, max_iters, (const uint32_t *)idx, d_codebooks, pend_cb, pend_codes);
+    vq::AssignArgs a;
+    a.x = d_x;
+    a.n = n;
+    a.ld = ld;
+    a.m = m;
+    a.k = k;
+    a.cb = d_codebooks;
+    a.cnorm = nullptr;
+    a.codes = S.codes;
+    a.done = nullptr;
+    const bool staged = sd <= vq::kSmallThreads;
+    const int C = lbg_small_clusters(m, sd, k);
+    const int groups = (int)cdiv(k, C);
+    if (staged && !ctx->lbg_small_lds_set) {
+        VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_lbg_update_small<true>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(float) * vq::kSmallStage)));
+        ctx->lbg_small_lds_set = true;
+    }
+    for (int it = 0; it < max_iters; ++it) {
+        a.pend_cb = it == 0 ? pend_cb : nullptr;  // the first pass leaves the rows updated
+        a.pend_codes = it == 0 ? pend_codes : nullptr;
+        a.before = S.changed + (size_t)it * m;
+        a.changed = S.changed + (size_t)(it + 1) * m;
+        {
+            ProfSpan sp(ctx, VQ_PROF_LBG_ASSIGN);
+            VQ_TRY(launch_assign<true>(ctx, VQ_SQEUCLIDEAN, a, sd));
+        }
+        ProfSpan sp(ctx, VQ_PROF_LBG_UPDATE);
+        if (staged)
+            hipLaunchKernelGGL(vq::k_lbg_update_small<true>, dim3(groups * m), dim3(vq::kSmallThreads),
+                               sizeof(float) * vq::kSmallStage, st, S, it, m, d_x, n, ld, sd, k, C, groups,
+                               (const uint32_t *)reseed, n_reseed, d_codebooks);
+        else
+            hipLaunchKernelGGL(vq::k_lbg_update_small<false>, dim3(groups * m), dim3(vq::kSmallThreads),
+                               sizeof(float) * 3 * C * sd, st, S, it, m, d_x, n, ld, sd, k, C, groups,
+                               (const uint32_t *)reseed, n_reseed, d_codebooks);
+    }
+    last();
+    hipLaunchKernelGGL(vq::k_lbg_small_report, dim3(1), dim3(256), 0, st, (const int *)S.changed, (int)n_flags, report);
+    VQ_HIP(ctx, hipGetLastError());
+    VQ_HIP(ctx, hipStreamSynchronize(st));
+    prof_collect(ctx);
+    const int *changed = report, *empties = report + (size_t)(max_iters + 1) * m;
+    for (int s = 0; s < m; ++s) {
+        int iters = 0, used = 0;
+        for (int it = 0; it < max_iters && changed[(size_t)it * m + s]; ++it) {
+            ++iters;
+            used += empties[(size_t)it * m + s];
+        }
+        if (h_iters_run) h_iters_run[s] = iters;
+        if (h_reseeds_used) h_reseeds_used[s] = used;
+    }
+    if (report[n_flags - 1])
+        return fail(ctx, VQ_ERR_RESEED_EXHAUSTED, "re-seed stream exhausted: pass n_reseed = k*max_iters");
+    return VQ_OK;
+}
+
 // The LBG loop for up to 256 centroids, on validated arguments.  last: enqueues what follows the
 // last update, before the loop's results are read back.
 template <typename Last>
@@ -1171,6 +1302,9 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
                            int32_t max_iters, const uint32_t *h_init_idx, const uint32_t *h_reseed_stream,
                            int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used,
                            const float *pend_cb, const uint8_t *pend_codes, const Last &last) {
+    if (lbg_small(n, m, sd, k))
+        return lbg_fit_small(ctx, d_x, n, ld, m, sd, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, d_codebooks,
+                             h_iters_run, h_reseeds_used, pend_cb, pend_codes, last);
     hipStream_t st = ctx->stream;
 
     const int nparts = (int)((n + vq::kPartRows - 1) / vq::kPartRows);
@@ -1320,7 +1454,7 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
         if (fused_tail) {
             hipLaunchKernelGGL(vq::k_lbg_finalize_prep8, dim3(m), dim3(256), 0, st, S, d_x, ld, k,
                                (const uint32_t *)ctx->reseed.p, n_reseed, d_codebooks, (const float *)big_sum,
-                               tabs.nb, tabs.atab, tabs.maxc2, tabs.mu, tabs.stat);
+                               tabs.nb, tabs.atab, tabs.maxc2, tabs.mu, tabs.stat, tabs.stat_next);
         } else {
             hipLaunchKernelGGL(vq::k_lbg_finalize, dim3(cdiv((int64_t)k * sd, 256), m), dim3(256), 0, st, S,
                                d_x, ld, k, sd, (const uint32_t *)ctx->reseed.p, n_reseed, d_codebooks);
