@@ -127,10 +127,10 @@ int32_t vq_host_alloc(vq_ctx *ctx, size_t bytes, void **h_ptr);
 int32_t vq_host_free(vq_ctx *ctx, void *h_ptr);
 /* Synchronous copies (they synchronise the context's stream). Replaces the per-vector heap
  * layout `&[Vector<f32>]` (src/vector.rs:150-152): the host packs rows into one buffer.
- * vq_h2d of 64 MiB or more from pageable memory is staged by the library: up to eight host threads
- * copy 16 MiB chunks into page-locked buffers of the context while the copy engine uploads the chunk
- * before (about 50 GB/s instead of 18-29 for one plain copy; a page-locked source goes up directly);
- * vq_d2h into pageable memory does the same in the other direction. */
+ * vq_h2d of 1 MiB or more from pageable memory is staged by the library: the caller and up to seven
+ * host threads that the context keeps copy chunks into its page-locked buffers while the copy engine
+ * uploads the chunk before (about 50 GB/s instead of 18-29 for one plain copy; a page-locked source goes
+ * up directly); vq_d2h into pageable memory does the same in the other direction. */
 int32_t vq_h2d(vq_ctx *ctx, void *d_dst, const void *h_src, size_t bytes);
 int32_t vq_d2h(vq_ctx *ctx, void *h_dst, const void *d_src, size_t bytes);
 
@@ -140,6 +140,22 @@ int32_t vq_d2h(vq_ctx *ctx, void *h_dst, const void *d_src, size_t bytes);
  * Both pointers 16-byte aligned.  Asynchronous. */
 int32_t vq_copy_f32(vq_ctx *ctx, float *d_dst, const float *d_src, int64_t count);
 
+/* ---- host rows in, host results out ------------------------------------------------------- */
+
+/* The batch forms of the quantizers' `quantize` for callers whose rows lie in host memory (pageable or
+ * not): the rows go through the GPU chunk by chunk, upload, kernels and download of neighbouring chunks
+ * side by side, copied by the threads of the context; a few rows are read and their results written in
+ * place, in page-locked memory.  Rows are compact (n x dim floats).  Any output may be NULL.  Results
+ * as from the calls on device memory, bit for bit.  Synchronise.
+ *
+ * ProductQuantizer::quantize (src/pq.rs:146-187) with d_rotation NULL, OptimizedProductQuantizer::quantize
+ * (src/opq.rs:222-264) with the rotation, dim x dim.  h_codes: n*m codes, bytes up to 256 centroids,
+ * else uint16.  h_out: n*dim binary16. */
+int32_t vq_pq_quantize_host(vq_ctx *ctx, int32_t metric, const float *h_x, int64_t n, int32_t m, int32_t sub_dim, int32_t k,
+                            const float *d_codebooks, const float *d_rotation, void *h_codes, uint16_t *h_out);
+/* ResidualQuantizer::quantize (src/rvq.rs:171-215), h_codes n*stages. */
+int32_t vq_rvq_quantize_host(vq_ctx *ctx, int32_t metric, const float *h_x, int64_t n, int32_t dim, int32_t stages, int32_t k,
+                             const float *d_codebooks, float epsilon, void *h_codes, uint16_t *h_out);
 /* ---- timing (HIP events on the context's stream) --------------------------------------- */
 int32_t vq_timer_start(vq_ctx *ctx);
 /* Records the stop event, synchronises, returns elapsed milliseconds since vq_timer_start. */
@@ -377,6 +393,10 @@ int32_t vq_ctx_set_tsvq_descend_path(vq_ctx *ctx, int32_t path);
 /* d_out[i] = f16(centroid of leaf d_leaf[i]) (src/tsvq.rs:241-248), n x dim.  Asynchronous. */
 int32_t vq_tsvq_decode_f16(vq_ctx *ctx, const vq_tree *tree, const int32_t *d_leaf, int64_t n,
                            uint16_t *d_out);
+
+/* TSVQ::quantize (src/tsvq.rs:231-249) for host rows, as vq_pq_quantize_host.  h_leaf: n leaf indices. */
+int32_t vq_tsvq_quantize_host(vq_ctx *ctx, int32_t metric, const float *h_x, int64_t n, const vq_tree *tree, int32_t *h_leaf,
+                              uint16_t *h_out);
 
 #ifdef __cplusplus
 }

@@ -1,0 +1,91 @@
+"""A few rows in one launch (k_assign_few, k_rvq_few, k_tsvq_few) and batches of host rows through the
+host calls at every way they take (in place, one chunk, pipelined, with copying threads), against the CPU
+oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests import data
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+METRICS = [O.SQEUCLIDEAN, O.EUCLIDEAN, O.COSINE, O.MANHATTAN]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import vq_amd
+    c = vq_amd.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("metric", METRICS)
+@pytest.mark.parametrize("n,m,sd,k", [(1, 1, 1, 1), (1, 16, 8, 256), (3, 5, 7, 255), (2, 2, 130, 257), (9, 3, 12, 1000), (512, 1, 8, 40)])
+def test_assign_few(ctx, metric, n, m, sd, k):
+    rng = np.random.default_rng(n + sd + k)
+    x = np.round(rng.standard_normal((n, m * sd)) * 2).astype(F)  # ties
+    cb = np.round(rng.standard_normal((m, k, sd)) * 2).astype(F)
+    if k > 2:
+        cb[:, 1] = 0.0
+    if n > 2:
+        x[1] = 0.0
+        x[2, 0] = np.nan
+        cb[-1, 0, 0] = np.inf
+    want = O.pq_encode(metric, x, cb)
+    codes = ctx.empty((n, m), np.uint16)
+    ctx.assign_u16(metric, ctx.to_device(x), n, m * sd, m, sd, k, ctx.to_device(cb), codes)
+    assert np.array_equal(codes.download(), want.astype(np.uint16))
+    if k <= 256:
+        codes8 = ctx.empty((n * m + 3,), np.uint8)
+        ctx.assign(metric, ctx.to_device(x), n, m * sd, m, sd, k, ctx.to_device(cb), codes8)
+        assert np.array_equal(codes8.download()[:n * m].reshape(n, m), want.astype(np.uint8))
+
+
+@pytest.mark.parametrize("metric", METRICS)
+@pytest.mark.parametrize("n,dim,stages,k,eps", [(1, 6, 3, 1, 0.0), (5, 33, 4, 20, 3.0), (512, 16, 2, 256, 0.0), (7, 300, 5, 60, 14.0)])
+def test_rvq_few(ctx, metric, n, dim, stages, k, eps):
+    rng = np.random.default_rng(dim)
+    x, cb = rng.standard_normal((n, dim)).astype(F), (0.5 * rng.standard_normal((stages, k, dim))).astype(F)
+    codes, rec = ctx.empty((n, stages), np.uint8), ctx.empty((n, dim), np.uint16)
+    ctx.rvq_encode(metric, ctx.to_device(x), n, dim, dim, stages, k, ctx.to_device(cb), eps, codes, None, rec)
+    want, want_rec = O.rvq_quantize(metric, x, cb, eps)
+    assert np.array_equal(codes.download(), want.astype(np.uint8)) and np.array_equal(rec.download(), want_rec)
+
+
+@pytest.mark.parametrize("metric", METRICS)
+@pytest.mark.parametrize("n,dim,depth", [(1, 3, 2), (40, 70, 6), (512, 128, 9)])
+def test_tsvq_few(ctx, metric, n, dim, depth):
+    rng = np.random.default_rng(dim + depth)
+    x = rng.standard_normal((max(n, 300), dim)).astype(F)
+    tree = ctx.tsvq_build(ctx.to_device(x), len(x), dim, dim, depth)
+    t = tree.download()
+    q = x[:n].copy()
+    q[0] = 0.0
+    leaf = ctx.empty(n, np.int32)
+    ctx.tsvq_descend(metric, ctx.to_device(q), n, dim, tree, leaf)
+    assert np.array_equal(leaf.download(), O.tsvq_descend(metric, q, t))
+
+
+@pytest.mark.parametrize("n", [1, 5, 100, 2048, 2049, 8192, 33_001, 140_003])
+def test_host_batches(n):
+    from vq_amd import api
+    rng = np.random.default_rng(n)
+    x = rng.random((max(n, 600), 128), dtype=F)
+    E = api.Distance.Euclidean
+    st = data.index_streams(600, 16, 64, 2, seed=1)
+    pq = api.ProductQuantizer.fit(x[:600], 16, 64, 2, E, 0, streams=st)
+    cb = pq.codebooks()
+    at = np.unique(np.concatenate([np.arange(min(n, 600)), rng.integers(0, n, 1500), np.arange(max(0, n - 600), n)]))
+    want = O.pq_encode(O.EUCLIDEAN, x[at], cb).astype(np.uint8)
+    assert np.array_equal(pq.encode(x[:n])[at], want)
+    assert np.array_equal(pq.quantize_batch(x[:n])[at].view(np.uint16), O.pq_decode_f16(want, cb))
+    rv = api.ResidualQuantizer.fit(x[:600], 2, 64, 2, 0.0, E, 0, streams=data.index_streams(600, 2, 64, 2, seed=2))
+    codes, rec = O.rvq_quantize(O.EUCLIDEAN, x[at], rv.codebooks(), 0.0)
+    assert np.array_equal(rv.encode(x[:n])[at], codes.astype(np.uint8))
+    assert np.array_equal(rv.quantize_batch(x[:n])[at].view(np.uint16), rec)
+    ts = api.TSVQ.new(x[:600], 5, E)
+    t = ts.tree()
+    leaves = ts.leaves(x[:n])
+    assert np.array_equal(leaves[at], O.tsvq_descend(O.EUCLIDEAN, x[at], dict(t, n_nodes=len(t["left"]))))
+    assert np.array_equal(ts.quantize_batch(x[:n])[at].view(np.uint16), O.f32_to_f16_bits(t["centroids"][leaves[at]]).reshape(len(at), 128))

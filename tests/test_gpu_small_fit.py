@@ -26,7 +26,7 @@ CASES = [(16, 4, 8, 16, 3, "normal"),          # one row per cluster
          (9000, 2, 12, 40, 4, "same"),         # one cluster, every other one re-seeded
          (2000, 5, 8, 7, 30, "blobs"),         # early stop
          (3000, 2, 32, 20, 3, "normal"), (5000, 1, 36, 64, 3, "normal"), (4097, 1, 100, 33, 3, "normal"),
-         (12_000, 1, 256, 256, 2, "skewed"), (6000, 2, 64, 32, 3, "skewed"), (300, 1, 1000, 5, 2, "normal")]
+         (12_000, 1, 256, 256, 2, "skewed"), (20_001, 2, 40, 64, 3, "skewed"), (10_000, 1, 48, 16, 3, "same"), (6000, 2, 64, 32, 3, "skewed"), (300, 1, 1000, 5, 2, "normal")]
 
 
 @pytest.mark.parametrize("n,m,sd,k,iters,kind", CASES)

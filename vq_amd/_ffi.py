@@ -74,6 +74,9 @@ SYMBOLS = {
     "vq_tree_download": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "vq_tsvq_descend": (_i32, [_vp, _i32, _vp, _i64, _i64, _vp, _vp]),
     "vq_tsvq_decode_f16": (_i32, [_vp, _vp, _vp, _i64, _vp]),
+    "vq_pq_quantize_host": (_i32, [_vp, _i32, _vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp]),
+    "vq_rvq_quantize_host": (_i32, [_vp, _i32, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _vp]),
+    "vq_tsvq_quantize_host": (_i32, [_vp, _i32, _vp, _i64, _vp, _vp, _vp]),
 }
 
 

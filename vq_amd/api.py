@@ -20,6 +20,9 @@ if not os.path.exists(HOST_LIB_PATH):
 _h = C.CDLL(HOST_LIB_PATH)
 _h.vqh_last_error.restype = C.c_char_p
 _vp, _i64, _i32, _u64 = C.c_void_p, C.c_int64, C.c_int32, C.c_uint64
+# the calls made per vector: argument types known, so plain integers (addresses, sizes) go through
+_h.vqh_quantize.argtypes = [_vp, _vp, _i64, _vp, _vp]
+_h.vqh_quantize_batch.argtypes = [_vp, _vp, _i64, _i64, _vp]
 
 
 class Distance:
@@ -92,24 +95,24 @@ class _Quantizer:
     def quantize(self, vector):
         """quantize(&self, &Vector<f32>) -> Vector<f16>"""
         v = np.ascontiguousarray(vector, np.float32).reshape(-1)
-        out = np.zeros(max(self.dim, v.size), np.uint16)
+        out = np.empty(max(self.dim, v.size), np.float16)
         got = _i64(0)
-        _check(_h.vqh_quantize(_vp(self._o), _p(v), _i64(v.size), _p(out), C.byref(got)))
-        return out[:got.value].view(np.float16)
+        _check(_h.vqh_quantize(self._o, v.ctypes.data, v.size, out.ctypes.data, C.byref(got)))
+        return out[:got.value]
 
     def quantize_batch(self, data):
         x = _rows(data)
-        out = np.zeros(x.shape, np.uint16)
-        _check(_h.vqh_quantize_batch(_vp(self._o), _p(x), _i64(x.shape[0]), _i64(x.shape[1]), _p(out)))
-        return out.view(np.float16)
+        out = np.empty(x.shape, np.float16)
+        _check(_h.vqh_quantize_batch(self._o, x.ctypes.data, x.shape[0], x.shape[1], out.ctypes.data))
+        return out
 
     def _encode(self, x, width):
         """n x width codes: bytes up to 256 centroids, uint16 above."""
         if self.k > 256:
-            codes = np.zeros((x.shape[0], width), np.uint16)
+            codes = np.empty((x.shape[0], width), np.uint16)
             _check(_h.vqh_encode16(_vp(self._o), _p(x), _i64(x.shape[0]), _i64(x.shape[1]), _p(codes)))
         else:
-            codes = np.zeros((x.shape[0], width), np.uint8)
+            codes = np.empty((x.shape[0], width), np.uint8)
             _check(_h.vqh_encode(_vp(self._o), _p(x), _i64(x.shape[0]), _i64(x.shape[1]), _p(codes)))
         return codes
 
@@ -163,7 +166,7 @@ class OptimizedProductQuantizer(_Quantizer):
     def quantize_batch(self, data):
         if self.k == 0:  # the reference returns an empty vector per row (src/opq.rs:122,244-263)
             x = _rows(data)
-            _check(_h.vqh_quantize_batch(_vp(self._o), _p(x), _i64(x.shape[0]), _i64(x.shape[1]), None))
+            _check(_h.vqh_quantize_batch(self._o, x.ctypes.data, x.shape[0], x.shape[1], None))
             return np.zeros((x.shape[0], 0), np.float16)
         return super().quantize_batch(data)
 
@@ -234,7 +237,7 @@ class TSVQ(_Quantizer):
 
     def leaves(self, data):
         x = _rows(data)
-        out = np.zeros(x.shape[0], np.int32)
+        out = np.empty(x.shape[0], np.int32)
         _check(_h.vqh_leaves(_vp(self._o), _p(x), _i64(x.shape[0]), _i64(x.shape[1]), _p(out)))
         return out
 

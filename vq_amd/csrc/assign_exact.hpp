@@ -9,6 +9,7 @@
 // Mapping: one lane = one row.  The lane keeps its sub-vectors in registers; the centroid
 // operand is identical for all lanes of a wave and is read from LDS as a broadcast.
 #pragma once
+#include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -29,6 +30,7 @@ struct AssignArgs {
     const int *done;      // LBG mode: blocks with done[s] != 0 are skipped
     const int *before = nullptr;  // LBG mode, instead of done: the changed flags of the pass before (0: skipped)
     float *dist = nullptr;  // encode mode, k_assign_mfma_bf only: [n][m] distance of the chosen centroid, or null
+    uint16_t *out16 = nullptr;  // encode mode, k_assign_mfma_bf only: [n][8 m] chosen centroids as binary16, or null
     // A residual update that the pass applies before it scores the rows (single wide column block,
     // k_assign_mfma_wide_bf only): x[i] = src[i] - pend_cb[pend_codes[i]], where src is the rows
     // themselves (an update in place) or, pend_src != null, other rows of stride pend_src_ld that
@@ -980,6 +982,166 @@ __global__ void __launch_bounds__(256) k_assign_wide_exact(AssignArgs a, int sd,
         }
     }
     wide_exact_groups<METRIC, LBG, LISTED, VEC, kWideRows>(a, sd, list, total, lds_x, lane, wave, block, exact_blocks);
+}
+
+}  // namespace vq
+
+// ---------------------------------------------------------------------------------------------
+// A few rows: one workgroup per (row, column block), thread j takes the centroids j, j + 256, ... one
+// after the other, each distance one sequential chain in the reference's order, and the smallest
+// (distance, index) of the workgroup wins.  Any metric, width and number of centroids, no tables and
+// no second launch: what a call of a few rows costs is launches and memory round trips (one row of
+// 128 floats, m = 16, k = 256: 4.6 us, where a wave of the matrix-core kernel takes 8.2 us to bring in
+// a column block).  Euclidean compares the roots, as the reference does.
+// out16 (nullable): the chosen centroids as binary16, round to nearest even.
+
+namespace vq {
+
+// The index of the first of the k centroids at cs nearest to the sub-vector in lds_x (16-byte aligned,
+// written before the workgroup's last barrier), by 256 threads; the same value in every thread.
+template <int METRIC>
+__device__ __forceinline__ int few_argmin(const float *lds_x, const float *__restrict__ cs, int sd, int k) {
+    __shared__ float red_d[4];
+    __shared__ int red_i[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const float inf = __builtin_inff();
+    float na = 0.0f;
+    if constexpr (METRIC == M_COS) {
+        float sa = 0.0f;
+        for (int t = 0; t < sd; ++t) {
+            const float p = lds_x[t] * lds_x[t];
+            sa = sa + p;
+        }
+        na = sqrtf(sa);
+    }
+    float bd = inf;
+    int bi = 0x7fffffff;
+    bool first_nan = false;  // centroid 0's distance is NaN: never displaced
+    const bool vec = sd % 4 == 0 && (reinterpret_cast<uintptr_t>(cs) & 15) == 0;
+    for (int j = tid; j < k; j += 256) {
+        const float *c = cs + (size_t)j * sd;
+        float acc = 0.0f, sb = 0.0f;
+        auto step = [&](float xv, float cv) {
+            wide_step<METRIC>(acc, xv, cv);
+            if constexpr (METRIC == M_COS) {
+                const float p = cv * cv;
+                sb = sb + p;
+            }
+        };
+        int t = 0;
+        if (vec) {
+#pragma unroll 8
+            for (; t + 4 <= sd; t += 4) {
+                const float4 cv = *reinterpret_cast<const float4 *>(c + t);
+                const float4 xv = *reinterpret_cast<const float4 *>(lds_x + t);
+                step(xv.x, cv.x);
+                step(xv.y, cv.y);
+                step(xv.z, cv.z);
+                step(xv.w, cv.w);
+            }
+        }
+#pragma unroll 8
+        for (; t < sd; ++t) step(lds_x[t], c[t]);
+        float d = acc;
+        if constexpr (METRIC == M_EUCLID) d = sqrtf(d);
+        if constexpr (METRIC == M_COS) {
+            const float nb = sqrtf(sb), den = na * nb, q = acc / den;
+            d = 1.0f - q;
+            d = (na == 0.0f || nb == 0.0f) ? 1.0f : d;
+        }
+        if (j == 0) first_nan = !(d == d);
+        // (all +inf: the lowest index; a NaN loses against everything)
+        if (d < bd || (d == inf && bi == 0x7fffffff)) {
+            bd = d;
+            bi = j;
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const float od = __shfl_xor(bd, off);
+        const int oi = __shfl_xor(bi, off);
+        const bool take = od < bd || (od == bd && oi < bi);
+        bd = take ? od : bd;
+        bi = take ? oi : bi;
+    }
+    if (lane == 0) {
+        red_d[wave] = bd;
+        red_i[wave] = tid == 0 && first_nan ? -1 : bi;
+    }
+    __syncthreads();
+    bi = red_i[0];
+    bd = red_d[0];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+        const bool take = bi >= 0 && (red_d[w] < bd || (red_d[w] == bd && red_i[w] < bi));
+        bd = take ? red_d[w] : bd;
+        bi = take ? red_i[w] : bi;
+    }
+    return bi < 0 || bi == 0x7fffffff ? 0 : bi;
+}
+
+template <int METRIC, typename CodeT>
+static __global__ void __launch_bounds__(256) k_assign_few(const float *__restrict__ x, int64_t ld, int m, int sd, int k,
+                                                           const float *__restrict__ cb, CodeT *__restrict__ codes,
+                                                           uint16_t *__restrict__ out16) {
+    extern __shared__ __attribute__((aligned(16))) float lds_few[];  // the row's sub-vector
+    const int s = blockIdx.x, tid = threadIdx.x;
+    const int64_t row = blockIdx.y;
+    const float *xr = x + row * ld + (int64_t)s * sd;
+    const float *cs = cb + (size_t)s * k * sd;
+    for (int t = tid; t < sd; t += 256) lds_few[t] = xr[t];
+    __syncthreads();
+    const int best = few_argmin<METRIC>(lds_few, cs, sd, k);
+    if (tid == 0) codes[row * m + s] = (CodeT)best;
+    if (out16)
+        for (int t = tid; t < sd; t += 256)
+            out16[row * ((int64_t)m * sd) + (int64_t)s * sd + t] = __half_as_ushort(__float2half_rn(cs[(size_t)best * sd + t]));
+}
+
+// ResidualQuantizer::quantize (src/rvq.rs:171-215) for a few rows: one workgroup per row takes it through
+// every stage in one launch, the residual and the sum in LDS.
+template <int METRIC, typename CodeT>
+static __global__ void __launch_bounds__(256) k_rvq_few(const float *__restrict__ x, int64_t ld, int dim, int stages, int k,
+                                                        const float *__restrict__ books, float epsilon,
+                                                        CodeT *__restrict__ codes, uint8_t *__restrict__ stages_used,
+                                                        uint16_t *__restrict__ out16) {
+    extern __shared__ __attribute__((aligned(16))) float lds_few[];  // the residual, then the sum
+    __shared__ int stop;
+    const int tid = threadIdx.x;
+    const int64_t row = blockIdx.x;
+    float *res = lds_few, *sum = lds_few + ((dim + 3) & ~3);
+    for (int t = tid; t < dim; t += 256) {
+        res[t] = x[row * ld + t];
+        sum[t] = 0.0f;
+    }
+    if (tid == 0) stop = 0;
+    __syncthreads();
+    int used = 0;
+    for (; used < stages && stop == 0; ++used) {
+        const float *cs = books + (size_t)used * k * dim;
+        const int best = k < 2 ? 0 : few_argmin<METRIC>(res, cs, dim, k);
+        __syncthreads();  // (the residual has been read; `stop` too)
+        for (int t = tid; t < dim; t += 256) {
+            const float c = cs[(size_t)best * dim + t];
+            sum[t] = sum[t] + c;
+            res[t] = res[t] - c;
+        }
+        if (tid == 0) codes[row * stages + used] = (CodeT)best;
+        __syncthreads();
+        if (epsilon > 0.0f && tid == 0) {  // a norm is never below a non-positive threshold
+            float acc = 0.0f;
+            for (int t = 0; t < dim; ++t) {
+                const float q = res[t] * res[t];
+                acc = acc + q;
+            }
+            if (sqrtf(acc) < epsilon) stop = 1;
+        }
+        if (epsilon > 0.0f) __syncthreads();
+    }
+    for (int st = used + tid; st < stages; st += 256) codes[row * stages + st] = (CodeT)0;
+    if (tid == 0 && stages_used) stages_used[row] = (uint8_t)used;
+    if (out16)
+        for (int t = tid; t < dim; t += 256) out16[row * dim + t] = __half_as_ushort(__float2half_rn(sum[t]));
 }
 
 }  // namespace vq

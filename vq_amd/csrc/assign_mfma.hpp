@@ -17,6 +17,7 @@
 // per chunk of 8 dimensions; the undecided pairs are listed for the exact kernel of assign_exact.hpp.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <hip/hip_fp16.h>
 #include <stdint.h>
 
 #include "assign_exact.hpp"
@@ -680,6 +681,14 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
                 const size_t out0 = (size_t)row0 * m + s;  // uniform
                 a.codes[out0 + rr * (uint32_t)m] = (uint8_t)code;
                 if (a.dist) a.dist[out0 + rr * (uint32_t)m] = dist;  // for the caller that merges chunks of a larger codebook
+                if (a.out16) {  // the reconstruction, round to nearest even
+                    const float4 c0 = *reinterpret_cast<const float4 *>(cl + code * SD), c1 = *reinterpret_cast<const float4 *>(cl + code * SD + 4);
+                    auto two = [](float lo, float hi) {
+                        return (uint32_t)__half_as_ushort(__float2half_rn(lo)) | ((uint32_t)__half_as_ushort(__float2half_rn(hi)) << 16);
+                    };
+                    reinterpret_cast<u32x4 *>(a.out16)[out0 + rr * (uint32_t)m] =
+                        u32x4{two(c0.x, c0.y), two(c0.z, c0.w), two(c1.x, c1.y), two(c1.z, c1.w)};
+                }
             }
         }
     }

@@ -16,6 +16,10 @@ struct DevBuf {
     size_t cap = 0;
 };
 
+namespace vqh {
+class CopyCrew;  // host_batch.hpp
+}
+
 struct vq_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -36,10 +40,15 @@ struct vq_ctx {
     size_t lbg_pin_cap = 0;
     void *tsvq_pin = nullptr;    // TSVQ build: page-locked staging of a level's tables and decisions
     size_t tsvq_pin_cap = 0;
-    // vq_h2d from pageable memory: page-locked staging buffers and the events of their uploads
-    static constexpr int kStageBuffers = 3;
-    void *h2d_stage[kStageBuffers] = {nullptr, nullptr, nullptr};
-    hipEvent_t h2d_event[kStageBuffers] = {nullptr, nullptr, nullptr};
+    // host rows on their way through the GPU (host_batch.hpp): page-locked and device slots of the chunks
+    // in flight, the streams and events that order them, the threads that copy
+    static constexpr int kPipe = 4;
+    void *pipe_pin = nullptr;
+    size_t pipe_pin_cap = 0;
+    DevBuf pipe_dev, pipe_rot;
+    hipStream_t up = nullptr, down = nullptr;
+    hipEvent_t pipe_up[kPipe] = {}, pipe_run[kPipe] = {}, pipe_down[kPipe] = {};
+    vqh::CopyCrew *crew = nullptr;
     DevBuf tsvq_gsum, tsvq_guess, tsvq_maps;  // per group of 32 squares: sum, binade guess, integer maps
     DevBuf tsvq_bsum, tsvq_segmaps;           // per block of groups: f64 sum; per run of groups: composed map
     int tsvq_var_path = 0;       // 0 = composed integer maps, 1 = one chain of adds per column
@@ -196,6 +205,8 @@ int32_t check_common(vq_ctx *ctx, const void *x, int64_t n, int64_t ld, int32_t 
 // Launchers defined in vq_api.hip, used by the RVQ / OPQ entry points.
 // d_dist (optional, n x m floats): receives the chosen centroids' distances where the kernel that runs
 // computes them anyway; *dist_written says whether it did.
+// d_out16 (optional, n x m * sd binary16 values, 16-byte aligned): receives the chosen centroids themselves
+// where the kernel that runs has them at hand; *out_written says whether it did.
 // pend (optional; one column block, and only where assign_pending_fusable says so): a residual
 // update that the pass applies to the rows before it scores them, d_x[i] = src[i] - cb[codes[i]]
 // with src = the rows of d_x themselves (src null: d_x is updated in place) or other rows of stride
@@ -208,16 +219,30 @@ struct PendingUpdate {
 };
 int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m,
                      int32_t sd, int32_t k, const float *d_codebooks, uint8_t *d_codes, float *d_dist = nullptr,
-                     bool *dist_written = nullptr, const PendingUpdate *pend = nullptr);
+                     bool *dist_written = nullptr, const PendingUpdate *pend = nullptr, uint16_t *d_out16 = nullptr,
+                     bool *out_written = nullptr);
+// Up to this many (row, column block) pairs an assignment runs as one workgroup per pair, one launch
+// (k_assign_few): two rounds of workgroups; the matrix-core kernels take two to four launches.
+constexpr int64_t kFewPairs = 512;
+template <typename CodeT>
+int32_t assign_few(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
+                   const float *d_codebooks, CodeT *d_codes, uint16_t *d_out16);
+inline bool assign_few_applicable(const vq_ctx *ctx, int64_t n, int32_t m, int32_t sd) {
+    return ctx->assign_path == 0 && n * m <= kFewPairs && sd <= 8192;
+}
 // Whether the assignment of these rows (one column block of sd floats) runs on the pass that can
 // take a pending update along.
 bool assign_pending_fusable(const vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t sd,
                             int32_t k, const float *d_codebook);
 
+// Defined in vq_api_host.hip: ends the copying threads.
+void drop_crew(vq_ctx *ctx);
+
 // Defined in vq_api_bigk.hip: the same for any k up to 65536 with 16-bit codes, and the LBG above
 // 256 centroids (arguments as vq_lbg_fit, already validated).
 int32_t assign_codes_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m,
-                         int32_t sd, int32_t k, const float *d_codebooks, uint16_t *d_codes);
+                         int32_t sd, int32_t k, const float *d_codebooks, uint16_t *d_codes,
+                         uint16_t *d_out16 = nullptr, bool *out_written = nullptr);
 int32_t lbg_fit_big(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
                     int32_t max_iters, const uint32_t *h_init_idx, const uint32_t *h_reseed_stream,
                     int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used);

@@ -643,6 +643,7 @@ static __global__ void __launch_bounds__(256) k_lbg_finalize(LbgState st, const 
 // (every load of up to 8192 floats in flight together), and one lane per (cluster, component) adds
 // them in list order, eight LDS reads ahead.  The orders of summation are those above: row order up
 // to 1024 members, part sums in part order above.
+// DEFER: clusters above 1024 members are counted and left to k_lbg_large.
 // STAGED: sub_dim a multiple of 4 up to 512, a thread per component.  Else (wider blocks) a wave takes
 // one cluster and 64 components at a time and reads the rows themselves, 16 rows in flight.
 constexpr int kSmallList = 8192;    // listed rows held before the list is worked off: at least 16 per thread
@@ -669,12 +670,17 @@ struct LbgSmall {
     int *empties;    // [max_iters][m]
     int *err;        // 1   set to 1 when a re-seed stream runs out
     uint8_t *codes;  // [m][n]
+    // wide blocks: the clusters above 1024 members, left to k_lbg_large
+    int *n_large;        // [max_iters]
+    uint2 *large;        // [most of an iteration]  {s * 256 + cluster, members}
+    int *arrived;        // [most of an iteration]  parts summed
+    float *large_sum;    // [most of an iteration][nparts][sd]
 };
 
 // codes = 0 (src/utils.rs:55), the flags, and the initial centroids x[idx[s][j]] (src/utils.rs:54; with
 // pend_cb, one column block: the row as the pending residual update will leave it).
 static __global__ void __launch_bounds__(256) k_lbg_small_init(LbgSmall st, const float *__restrict__ x, int64_t n,
-                                                               int64_t ld, int m, int k, int sd, int max_iters,
+                                                               int64_t ld, int m, int k, int sd, int max_iters, int most_large,
                                                                const uint32_t *__restrict__ idx, float *__restrict__ cb,
                                                                const float *__restrict__ pend_cb,
                                                                const uint8_t *__restrict__ pend_codes) {
@@ -687,7 +693,9 @@ static __global__ void __launch_bounds__(256) k_lbg_small_init(LbgSmall st, cons
         cb[i] = pend_cb ? v - pend_cb[(size_t)pend_codes[row] * sd + t] : v;
     }
     for (int64_t i = i0; i < ((int64_t)m * n + 3) / 4; i += stride) reinterpret_cast<uint32_t *>(st.codes)[i] = 0u;
-    for (int64_t i = i0; i < (int64_t)(2 * max_iters + 1) * m + 1; i += stride) st.changed[i] = i < m ? 1 : 0;
+    // (changed, empties, err, n_large, arrived lie one behind the other)
+    for (int64_t i = i0; i < (int64_t)(2 * max_iters + 1) * m + 1 + max_iters + most_large; i += stride)
+        st.changed[i] = i < m ? 1 : 0;
 }
 
 // The flags to page-locked host memory.
@@ -695,7 +703,7 @@ static __global__ void __launch_bounds__(256) k_lbg_small_report(const int *__re
     for (int i = threadIdx.x; i < count; i += 256) out[i] = flags[i];
 }
 
-template <bool STAGED>
+template <bool STAGED, bool DEFER = false>
 static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSmall st, int it, int m,
                                                                            const float *__restrict__ x, int64_t n,
                                                                            int64_t ld, int sd, int k, int C, int groups,
@@ -795,15 +803,19 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
             if constexpr (STAGED) {
                 const uint32_t per = (uint32_t)sd / 4u, most = (uint32_t)kSmallStage / (uint32_t)sd;
                 typedef float piece4 __attribute__((ext_vector_type(4), aligned(4)));
-                for (uint32_t p0 = 0; p0 < wn; p0 += most) {
+                constexpr int E = kSmallStage / 4 / kSmallThreads;
+                piece4 v[E];
+                auto gather = [&](uint32_t p0) {  // past the window's end: its first row again, not stored
                     const uint32_t pn = wn - p0 < most ? wn - p0 : most;
-                    constexpr int E = kSmallStage / 4 / kSmallThreads;
-                    piece4 v[E];
 #pragma unroll
                     for (int e = 0; e < E; ++e) {
                         const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * e, ic = i < pn * per ? i : 0u;
                         v[e] = *reinterpret_cast<const piece4 *>(xs + (int64_t)sorted[p0 + ic / per] * ld + 4u * (ic % per));
                     }
+                };
+                gather(0);
+                for (uint32_t p0 = 0; p0 < wn; p0 += most) {
+                    const uint32_t pn = wn - p0 < most ? wn - p0 : most;
 #pragma unroll
                     for (int e = 0; e < E; ++e) {
                         const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * e;
@@ -811,6 +823,7 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
                             *reinterpret_cast<float4 *>(dyn + 4u * i) = make_float4(v[e][0], v[e][1], v[e][2], v[e][3]);
                     }
                     __syncthreads();
+                    if (p0 + most < wn) gather(p0 + most);  // in flight while this stage is added
                     if (summing) {
                         const uint32_t c_lo = cl_off[my_c], c_hi = cl_off[my_c + 1];
                         uint32_t i = c_lo > p0 ? c_lo - p0 : 0u;
@@ -819,14 +832,20 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
                         if (track) {
                             for (; i + 8 <= hi; i += 8) {
                                 float t[8];
-                                uint32_t row[8];
 #pragma unroll
-                                for (int u = 0; u < 8; ++u) {
-                                    t[u] = d[(i + u) * (uint32_t)sd];
-                                    row[u] = sorted[p0 + i + u];
+                                for (int u = 0; u < 8; ++u) t[u] = d[(i + u) * (uint32_t)sd];
+                                // (rows ascend: the last one in the open part means all eight)
+                                if (sorted[p0 + i + 7] / (uint32_t)kPartRows == cur_part) {
+#pragma unroll
+                                    for (int u = 0; u < 8; ++u) {
+                                        seq = seq + t[u];
+                                        part = part + t[u];
+                                    }
+                                } else {
+#pragma unroll
+                                    for (int u = 0; u < 8; ++u)
+                                        add_tracked(t[u], sorted[p0 + i + u], seq, total, part, cur_part);
                                 }
-#pragma unroll
-                                for (int u = 0; u < 8; ++u) add_tracked(t[u], row[u], seq, total, part, cur_part);
                             }
                             for (; i < hi; ++i) add_tracked(d[i * (uint32_t)sd], sorted[p0 + i], seq, total, part, cur_part);
                         } else {
@@ -894,22 +913,48 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
         }
         return v;
     };
-    uint32_t have_next;
-    codes16 next = fetch(16 * tid, have_next);
     constexpr int kStep = 16 * kSmallThreads;  // rows
     const int nsteps = (int)((n + kStep - 1) / kStep);
-    for (int p = 0; p < nsteps; ++p) {
-        const uint32_t row0 = (uint32_t)p * (uint32_t)kStep + 16u * tid;
-        const codes16 v = next;
-        const uint32_t have = have_next;
-        next = fetch((int64_t)row0 + kStep, have_next);
-        uint32_t mine = 0;  // bit u: row row0 + u belongs to one of the workgroup's clusters
+    // bit u: row row0 + u belongs to one of the workgroup's clusters
+    auto own_rows = [&](const codes16 &v) {
+        uint32_t mine = 0;
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
             const uint32_t c = (v[u >> 2] >> (8 * (u & 3))) & 0xffu;
             mine |= (c - (uint32_t)j0 < (uint32_t)jn ? 1u : 0u) << u;
         }
-        mine &= have;
+        return mine;
+    };
+    auto cluster_of = [&](const codes16 &v, uint32_t u) {
+        const uint32_t w = u < 8u ? (u < 4u ? v[0] : v[1]) : (u < 12u ? v[2] : v[3]);
+        return ((w >> (8u * (u & 3u))) & 0xffu) - (uint32_t)j0;
+    };
+    uint32_t have_next;
+    codes16 next = fetch(16 * tid, have_next);
+    uint32_t large = 0;  // (DEFER) bit c: cluster j0 + c is not summed here, uniform
+    if constexpr (DEFER) {
+        __syncthreads();
+        for (int p = 0; p < nsteps; ++p) {
+            const codes16 v = next;
+            uint32_t mine = own_rows(v) & have_next;
+            next = fetch((int64_t)(p + 1 < nsteps ? p + 1 : 0) * kStep + 16 * tid, have_next);  // (then the first step again)
+            for (; mine; mine &= mine - 1) atomicAdd(&cl_cnt[cluster_of(v, (uint32_t)__ffs(mine) - 1u)], 1u);
+        }
+        __syncthreads();
+        for (int c = 0; c < jn; ++c) large |= (cl_cnt[c] > (uint32_t)kSeqMax ? 1u : 0u) << c;
+        large = __builtin_amdgcn_readfirstlane(large);
+        if (tid < jn && ((large >> tid) & 1u))
+            st.large[atomicAdd(st.n_large + it, 1)] = make_uint2((uint32_t)(s * kMaxK + j0 + tid), cl_cnt[tid]);
+    }
+    for (int p = 0; p < nsteps; ++p) {
+        const uint32_t row0 = (uint32_t)p * (uint32_t)kStep + 16u * tid;
+        const codes16 v = next;
+        const uint32_t have = have_next;
+        next = fetch((int64_t)row0 + kStep, have_next);
+        uint32_t mine = own_rows(v) & have;
+        if (DEFER && large)
+            for (uint32_t mm = mine; mm; mm &= mm - 1)
+                if ((large >> cluster_of(v, (uint32_t)__ffs(mm) - 1u)) & 1u) mine &= ~(mm & (0u - mm));
         const uint32_t m1 = __popc(mine);
         uint32_t inc = m1;
 #pragma unroll
@@ -927,21 +972,20 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
             all += t;
         }
         if (cnt + all > (uint32_t)kSmallList) {  // the sizes of the clusters are not known yet: keep both sums
-            track = true;
+            track = !DEFER;
             drain();
         }
         uint32_t at = cnt + before + inc - m1;
         for (uint32_t mm = mine; mm; mm &= mm - 1) {
             const uint32_t u = (uint32_t)__ffs(mm) - 1u;
-            const uint32_t w = u < 8u ? (u < 4u ? v[0] : v[1]) : (u < 12u ? v[2] : v[3]);
-            const uint32_t c = ((w >> (8u * (u & 3u))) & 0xffu) - (uint32_t)j0;
+            const uint32_t c = cluster_of(v, u);
             list[at++] = (row0 + u) | (c << 28);
-            atomicAdd(&cl_cnt[c], 1u);
+            if constexpr (!DEFER) atomicAdd(&cl_cnt[c], 1u);
         }
         cnt += all;
     }
     __syncthreads();
-    if (!drained) {
+    if (!DEFER && !drained) {
         for (int c = 0; c < jn; ++c) track = track || cl_cnt[c] > (uint32_t)kSeqMax;
     }
     drain();
@@ -949,7 +993,8 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
     if constexpr (STAGED) {
         if (summing) {
             const uint32_t cm = cl_cnt[my_c];
-            if (cm) out[my_c * sd + my_t] = (cm <= (uint32_t)kSeqMax ? seq : total + part) / __uint2float_rn(cm);
+            if (cm && !((large >> my_c) & 1u))
+                out[my_c * sd + my_t] = (cm <= (uint32_t)kSeqMax ? seq : total + part) / __uint2float_rn(cm);
         }
     } else {
         for (int i = tid; i < jn * sd; i += kSmallThreads) {
@@ -986,6 +1031,109 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
             st.err[0] = 1;  // the centroid stays
         else
             out[i] = xs[(int64_t)reseed[(size_t)s * n_reseed + pos] * ld + t];
+    }
+}
+
+// The clusters above 1024 members of a small fit over wide blocks (rows that are residuals gather in a
+// few of them): workgroup (part p, y) takes the listed clusters y, y + gridDim.y, ... and adds the
+// members in part p in row order, staged through LDS as above; the workgroup that brings a cluster's
+// last part adds the part sums in part order and divides.  One workgroup that adds such a cluster alone
+// is bound by what it has in flight, 64 KB per memory round trip: 6,000 rows of 128 took 200 us.
+static __global__ void __launch_bounds__(kSmallThreads) k_lbg_large(LbgSmall st, int it, const float *__restrict__ x,
+                                                                    int64_t n, int64_t ld, int sd, int k,
+                                                                    float *__restrict__ cb) {
+    const int count = st.n_large[it];
+    if ((int)blockIdx.y >= count) return;
+    const int p = blockIdx.x, nparts = gridDim.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    __shared__ uint16_t list[kPartRows];
+    __shared__ uint32_t wave_tot[kSmallWaves];
+    __shared__ int last;
+    extern __shared__ float dyn[];
+    const int64_t lo = (int64_t)p * kPartRows;
+    const int rows = n - lo < kPartRows ? (int)(n - lo) : kPartRows;
+    typedef float piece4 __attribute__((ext_vector_type(4), aligned(4)));
+    for (int e = blockIdx.y; e < count; e += gridDim.y) {
+        const uint2 ent = st.large[e];
+        const int s = (int)(ent.x / kMaxK);
+        const uint32_t j = ent.x % kMaxK;
+        const uint8_t *codes = st.codes + (size_t)s * n + lo;
+        uint32_t mine = 0;  // of the thread's eight consecutive rows
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = 8 * tid + u;
+            mine |= (i < rows && codes[i < rows ? i : 0] == j ? 1u : 0u) << u;
+        }
+        uint32_t inc = __popc(mine);
+        const uint32_t own = inc;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_up(inc, off);
+            if (lane >= off) inc += o;
+        }
+        if (lane == 63) wave_tot[wave] = inc;
+        __syncthreads();
+        uint32_t at = inc - own, cnt = 0;
+#pragma unroll
+        for (int w = 0; w < kSmallWaves; ++w) {
+            at += w < wave ? wave_tot[w] : 0u;
+            cnt += wave_tot[w];
+        }
+        for (; mine; mine &= mine - 1) list[at++] = (uint16_t)(8 * tid + __ffs(mine) - 1);
+        __syncthreads();
+        const float *xs = x + lo * ld + (int64_t)s * sd;
+        const uint32_t per = (uint32_t)sd / 4u, most = (uint32_t)kSmallStage / (uint32_t)sd;
+        constexpr int E = kSmallStage / 4 / kSmallThreads;
+        piece4 v[E];
+        auto gather = [&](uint32_t p0) {
+            const uint32_t pn = cnt - p0 < most ? cnt - p0 : most;
+#pragma unroll
+            for (int u = 0; u < E; ++u) {
+                const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * u, ic = i < pn * per ? i : 0u;
+                v[u] = *reinterpret_cast<const piece4 *>(xs + (int64_t)list[p0 + ic / per] * ld + 4u * (ic % per));
+            }
+        };
+        float sum = 0.0f;
+        if (cnt) gather(0);
+        for (uint32_t p0 = 0; p0 < cnt; p0 += most) {
+            const uint32_t pn = cnt - p0 < most ? cnt - p0 : most;
+#pragma unroll
+            for (int u = 0; u < E; ++u) {
+                const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * u;
+                if (i < pn * per) *reinterpret_cast<float4 *>(dyn + 4u * i) = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
+            }
+            __syncthreads();
+            if (p0 + most < cnt) gather(p0 + most);
+            if (tid < sd) {
+                uint32_t i = 0;
+                for (; i + 8 <= pn; i += 8) {
+                    float t[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) t[u] = dyn[(i + u) * (uint32_t)sd + tid];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) sum = sum + t[u];
+                }
+                for (; i < pn; ++i) sum = sum + dyn[i * (uint32_t)sd + tid];
+            }
+            __syncthreads();
+        }
+        float *sums = st.large_sum + (size_t)e * nparts * sd;
+        if (tid < sd) sums[(size_t)p * sd + tid] = sum;
+        __threadfence();
+        __syncthreads();
+        if (tid == 0) last = atomicAdd(st.arrived + e, 1) == nparts - 1;
+        __syncthreads();
+        if (last) {
+            __threadfence();
+            if (tid < sd) {
+                float total = 0.0f;
+                for (int q = 0; q < nparts; ++q)
+                    total = total + __hip_atomic_load(sums + (size_t)q * sd + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                cb[((size_t)s * k + j) * sd + tid] = total / __uint2float_rn(ent.y);
+            }
+            if (tid == 0) st.arrived[e] = 0;  // for the next iteration
+        }
+        __syncthreads();
     }
 }
 

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "assign_exact.hpp"
+
 namespace vq {
 
 // res[i] -= codebook[code[i]]   (src/rvq.rs:127).  One lane per element.

@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "assign_exact.hpp"
+
 namespace vq {
 
 // One lane per (leaf, component): sequential sum over perm[lo, hi).
@@ -1613,6 +1615,65 @@ __global__ void __launch_bounds__(512) k_tsvq_descend_w(const float *__restrict_
         }
         if (row0 + lane < n) leaf[row0 + lane] = node;
     }  // batches
+}
+
+// TSVQNode::quantize_with_distance (src/tsvq.rs:162-181) for a few rows: one wave per row, which brings
+// both children's centroids of a node into LDS with whole-line loads; lane 0 adds up the left distance
+// and lane 1 the right one, each in the reference's order.  out16 (nullable): the leaf's centroid.
+// (A lane of k_tsvq_descend reads its centroids alone, and k_tsvq_descend_w stages 134 KB first.)
+template <int METRIC>
+__global__ void __launch_bounds__(64) k_tsvq_few(const float *__restrict__ x, int64_t ld, int dim,
+                                                 const float *__restrict__ cen, const float *__restrict__ cnorm,
+                                                 const int *__restrict__ left, const int *__restrict__ right,
+                                                 int *__restrict__ leaf, uint16_t *__restrict__ out16) {
+    extern __shared__ float lds_few[];  // the row, the left centroid, the right one: rows of dim + 1
+    const int lane = threadIdx.x;
+    const int64_t row = blockIdx.x;
+    const int stride = dim + 1;
+    float *xs = lds_few, *cs = lds_few + stride;
+    for (int t = lane; t < dim; t += 64) xs[t] = x[row * ld + t];
+    __syncthreads();
+    float na = 0.0f;
+    if constexpr (METRIC == M_COS) {
+        float sa = 0.0f;
+        for (int t = 0; t < dim; ++t) {
+            const float p = xs[t] * xs[t];
+            sa = sa + p;
+        }
+        na = sqrtf(sa);
+    }
+    int node = 0;
+    for (;;) {
+        const int l = left[node], r = right[node];
+        if (l < 0 && r < 0) break;
+        if (l < 0 || r < 0) {
+            node = l >= 0 ? l : r;
+            continue;
+        }
+#pragma unroll 2
+        for (int t = lane; t < dim; t += 64) {
+            cs[t] = cen[(size_t)l * dim + t];
+            cs[stride + t] = cen[(size_t)r * dim + t];
+        }
+        const float nc = METRIC == M_COS ? cnorm[lane == 0 ? l : r] : 0.0f;
+        __syncthreads();
+        const float *c = cs + (lane & 1) * stride;  // (the other lanes repeat these two sums)
+        float acc = 0.0f;
+#pragma unroll 8
+        for (int t = 0; t < dim; ++t) wide_step<METRIC>(acc, xs[t], c[t]);
+        float d = acc;
+        if constexpr (METRIC == M_COS) {
+            const float q = acc / (na * nc);
+            d = (na == 0.0f || nc == 0.0f) ? 1.0f : 1.0f - q;
+        }
+        if constexpr (METRIC == M_EUCLID) d = sqrtf(d);
+        const float dl = __shfl(d, 0), dr = __shfl(d, 1);
+        node = dl <= dr ? l : r;
+        __syncthreads();
+    }
+    if (lane == 0) leaf[row] = node;
+    if (out16)
+        for (int t = lane; t < dim; t += 64) out16[row * dim + t] = __half_as_ushort(__float2half_rn(cen[(size_t)node * dim + t]));
 }
 
 // out[i][t] = f16(centroid[leaf[i]][t])   (src/tsvq.rs:242-248)

@@ -27,7 +27,9 @@ void launch_merge(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int m, i
 namespace vqh {
 
 int32_t assign_codes_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m,
-                         int32_t sd, int32_t k, const float *d_codebooks, uint16_t *d_codes) {
+                         int32_t sd, int32_t k, const float *d_codebooks, uint16_t *d_codes, uint16_t *d_out16,
+                         bool *out_written) {
+    if (out_written) *out_written = false;
     VQ_TRY(check_common(ctx, d_x, n, ld, m, sd, k, 65536));
     if (!d_codebooks || !d_codes) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter: null pointer");
     if (reinterpret_cast<uintptr_t>(d_codes) & 1)
@@ -36,6 +38,10 @@ int32_t assign_codes_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t 
     if (metric < VQ_SQEUCLIDEAN || metric > VQ_MANHATTAN)
         return fail(ctx, VQ_ERR_UNSUPPORTED, "metric %d has no kernel", metric);
     VQ_HIP(ctx, hipSetDevice(ctx->device));
+    if (assign_few_applicable(ctx, n, m, sd)) {
+        if (out_written) *out_written = d_out16 != nullptr;
+        return assign_few<uint16_t>(ctx, metric, d_x, n, ld, m, sd, k, d_codebooks, d_codes, d_out16);
+    }
     const size_t pairs = (size_t)n * m;
     VQ_TRY(ensure(ctx, ctx->big_win, (pairs + 3) & ~(size_t)3));
     uint8_t *win = (uint8_t *)ctx->big_win.p;

@@ -57,6 +57,22 @@ int32_t rvq_encode(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int
         return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
     VQ_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
+    if (stages > 0 && assign_few_applicable(ctx, n, 1, dim)) {
+        const size_t lds = sizeof(float) * 2 * ((size_t)dim + 3);
+#define FEW(M)                                                                                                      \
+    hipLaunchKernelGGL((vq::k_rvq_few<M, CodeT>), dim3((unsigned)n), dim3(256), lds, st, d_x, ld, dim, stages, k,      \
+                       d_codebooks, epsilon, d_codes, d_stages_used, d_recon_f16)
+        switch (metric) {
+        case VQ_SQEUCLIDEAN: FEW(vq::M_SQ); break;
+        case VQ_EUCLIDEAN: FEW(vq::M_EUCLID); break;
+        case VQ_COSINE: FEW(vq::M_COS); break;
+        case VQ_MANHATTAN: FEW(vq::M_L1); break;
+        default: return fail(ctx, VQ_ERR_UNSUPPORTED, "metric %d has no kernel", metric);
+        }
+#undef FEW
+        VQ_HIP(ctx, hipGetLastError());
+        return VQ_OK;
+    }
     const bool vec4 = dim % 4 == 0 && (reinterpret_cast<uintptr_t>(d_codebooks) & 15) == 0;
     // The first stage reads the caller's rows where they lie and writes the first residual; the last
     // stage leaves the residual alone.  One stage then needs no residual buffer at all.

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "ctx.hpp"
+#include "host_batch.hpp"
 #include "assign_exact.hpp"
 #include "tsvq.hpp"
 #include "tsvq_kmeans.hpp"
@@ -676,6 +677,24 @@ int32_t vq_ctx_set_tsvq_descend_path(vq_ctx *ctx, int32_t path) {
     return VQ_OK;
 }
 
+static int32_t descend_few(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, const vq_tree *tree,
+                           int32_t *d_leaf, uint16_t *d_out) {
+    const size_t lds = sizeof(float) * 3 * ((size_t)tree->dim + 1);
+#define FEW(M)                                                                                                    \
+    hipLaunchKernelGGL(vq::k_tsvq_few<M>, dim3((unsigned)n), dim3(64), lds, ctx->stream, d_x, ld, tree->dim,         \
+                       tree->d_centroids, tree->d_cnorm, tree->d_left, tree->d_right, d_leaf, d_out)
+    switch (metric) {
+    case VQ_SQEUCLIDEAN: FEW(vq::M_SQ); break;
+    case VQ_EUCLIDEAN: FEW(vq::M_EUCLID); break;
+    case VQ_COSINE: FEW(vq::M_COS); break;
+    case VQ_MANHATTAN: FEW(vq::M_L1); break;
+    default: return fail(ctx, VQ_ERR_UNSUPPORTED, "metric %d has no kernel", metric);
+    }
+#undef FEW
+    VQ_HIP(ctx, hipGetLastError());
+    return VQ_OK;
+}
+
 int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld,
                         const vq_tree *tree, int32_t *d_leaf) {
     if (!ctx || !tree) return VQ_ERR_INVALID_ARG;
@@ -684,6 +703,7 @@ int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n
     if (ld < tree->dim)
         return fail(ctx, VQ_ERR_DIM_MISMATCH, "Dimension mismatch: expected %d, got %lld", tree->dim, (long long)ld);
     VQ_HIP(ctx, hipSetDevice(ctx->device));
+    if (n <= kFewPairs && tree->dim <= 4096) return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
     // rows in registers: dim a multiple of 32 up to 128, 16-byte aligned rows
     if (tree->dim % 32 == 0 && tree->dim <= 128 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0) {
         // one workgroup per compute unit (the staged centroids fill its LDS), walking over the rows
@@ -752,6 +772,23 @@ int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n
 #undef DESC
     VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;
+}
+
+int32_t vq_tsvq_quantize_host(vq_ctx *ctx, int32_t metric, const float *h_x, int64_t n, const vq_tree *tree, int32_t *h_leaf,
+                              uint16_t *h_out) {
+    if (!ctx) return VQ_ERR_INVALID_ARG;
+    if (n == 0) return VQ_OK;
+    if (!h_x || n < 0 || !tree) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
+    const int32_t dim = tree->dim;
+    const HostOut outs[2] = {{h_out, 2 * (size_t)dim}, {h_leaf, sizeof(int32_t)}};
+    return host_batch(ctx, h_x, n, sizeof(float) * (size_t)dim, outs, 4u << 20, true,
+                      [&](const float *d_x, int64_t rows, void *d_out, void *d_leaf) -> int32_t {
+                          uint16_t *out = h_out ? (uint16_t *)d_out : nullptr;
+                          if (rows <= kFewPairs && dim <= 4096)
+                              return descend_few(ctx, metric, d_x, rows, dim, tree, (int32_t *)d_leaf, out);
+                          VQ_TRY(vq_tsvq_descend(ctx, metric, d_x, rows, dim, tree, (int32_t *)d_leaf));
+                          return out ? vq_tsvq_decode_f16(ctx, tree, (const int32_t *)d_leaf, rows, out) : VQ_OK;
+                      });
 }
 
 int32_t vq_tsvq_decode_f16(vq_ctx *ctx, const vq_tree *tree, const int32_t *d_leaf, int64_t n, uint16_t *d_out) {

@@ -22,16 +22,22 @@
 // (k distinct rows, uniform re-seed rows, deterministic in the seed), different numbers.
 // A host that owns the real generator passes explicit IndexStreams instead.
 #pragma once
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <memory>
 #include <stdexcept>
 #include <string>
-#include <unordered_set>
 #include <vector>
 
 #include "../../include/vq_hip.h"
+
+// The calls that take host rows through the GPU in one go.  Weak: a host built against this header also
+// runs on a library without them (device buffers and one call per step then).
+#pragma weak vq_pq_quantize_host
+#pragma weak vq_rvq_quantize_host
+#pragma weak vq_tsvq_quantize_host
 
 namespace vq {
 
@@ -125,13 +131,27 @@ struct IndexStreams {
         z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
         return z ^ (z >> 31);
     }
-    static uint64_t below(uint64_t &s, uint64_t bound) {  // unbiased, by rejection
-        uint64_t lim = UINT64_MAX - UINT64_MAX % bound;
+    // unbiased, by rejection of draws from the last, incomplete multiple of bound on
+    static uint64_t below(uint64_t &s, uint64_t bound) {
         uint64_t r;
         do r = splitmix(s);
-        while (r >= lim);
+        while (r > UINT64_MAX - bound && r >= UINT64_MAX - UINT64_MAX % bound);
         return r % bound;
     }
+    // The same for many draws below one bound, the remainder by a multiplication with its reciprocal
+    // (streams of a fit with m = 16, k = 256, 10 iterations: 0.40 -> 0.16 ms with the set below).
+    struct Below {
+        uint64_t bound, lim, recip;
+        explicit Below(uint64_t b) : bound(b), lim(UINT64_MAX - UINT64_MAX % b), recip(UINT64_MAX / b) {}
+        uint64_t operator()(uint64_t &s) const {
+            uint64_t r;
+            do r = splitmix(s);
+            while (r >= lim);
+            uint64_t rem = r - (uint64_t)(((unsigned __int128)r * recip) >> 64) * bound;  // the quotient is at most 2 short
+            while (rem >= bound) rem -= bound;
+            return rem;
+        }
+    };
     // Problem i is seeded with seed + i (src/pq.rs:119, src/opq.rs:140, src/rvq.rs:107): first k
     // distinct rows (Floyd's algorithm, insertion order), then k*max_iters re-seed draws.
     static IndexStreams from_seed(uint64_t seed, size_t problems, size_t n, size_t k, size_t max_iters) {
@@ -139,18 +159,28 @@ struct IndexStreams {
         st.n_reseed = (int32_t)(k * max_iters);
         st.init.resize(problems * k);
         st.reseed.resize(problems * (size_t)st.n_reseed);
+        // the rows drawn so far: an open-addressed set of twice their number, row + 1 (0: free)
+        size_t slots = 4;
+        while (slots < 4 * k) slots *= 2;
+        std::vector<uint64_t> seen(slots);
+        const Below row(n);
         for (size_t i = 0; i < problems; ++i) {
             uint64_t s = seed + i;
-            std::unordered_set<uint32_t> seen;
+            std::fill(seen.begin(), seen.end(), 0);
+            auto insert = [&](uint64_t v) {
+                size_t at = (size_t)((v * 0x9e3779b97f4a7c15ull) >> 20) & (slots - 1);
+                while (seen[at] && seen[at] != v + 1) at = (at + 1) & (slots - 1);
+                const bool fresh = seen[at] == 0;
+                seen[at] = v + 1;
+                return fresh;
+            };
             size_t w = 0;
             for (size_t j = n - k; j < n; ++j) {
-                uint32_t t = (uint32_t)below(s, j + 1);
-                uint32_t pick = seen.insert(t).second ? t : (uint32_t)j;
-                if (pick == (uint32_t)j) seen.insert(pick);
-                st.init[i * k + w++] = pick;
+                uint64_t pick = below(s, j + 1);
+                if (!insert(pick)) insert(pick = j);
+                st.init[i * k + w++] = (uint32_t)pick;
             }
-            for (int32_t r = 0; r < st.n_reseed; ++r)
-                st.reseed[i * (size_t)st.n_reseed + r] = (uint32_t)below(s, n);
+            for (int32_t r = 0; r < st.n_reseed; ++r) st.reseed[i * (size_t)st.n_reseed + r] = (uint32_t)row(s);
         }
         return st;
     }
@@ -321,6 +351,15 @@ inline std::vector<Vector<f16>> unpack_f16(const std::vector<uint16_t> &flat, si
     return out;
 }
 
+// quantize(&self, &Vector<f32>): one row through the quantizer's batch call.
+template <class Q>
+Vector<f16> quantize_one(const Q &q, const Vector<float> &vector) {
+    static_assert(sizeof(f16) == sizeof(uint16_t), "f16 is its bit pattern");
+    Vector<f16> out(std::vector<f16>(vector.len()));
+    q.quantize_into(Rows::view(vector.data.data(), 1, vector.len()), reinterpret_cast<uint16_t *>(out.data.data()));
+    return out;
+}
+
 // ---- lbg_quantize (src/utils.rs:32-109) --------------------------------------------------------
 inline std::vector<Vector<float>> lbg_quantize(const Rows &data, size_t k,
                                                size_t max_iters, uint64_t seed,
@@ -387,7 +426,7 @@ public:
     // src/pq.rs:146-187
     Vector<f16> quantize(const Vector<float> &vector) const {
         if (vector.len() != sub_dim_ * m_) throw VqError::DimensionMismatch(sub_dim_ * m_, vector.len());
-        return quantize_batch(std::vector<Vector<float>>{vector})[0];
+        return quantize_one(*this, vector);
     }
 
     std::vector<Vector<f16>> quantize_batch(const Rows &vectors) const {
@@ -396,10 +435,22 @@ public:
 
     // the same reconstructions as one row-major n x dim array of f16 bit patterns
     std::vector<uint16_t> quantize_batch_flat(const Rows &vectors) const {
+        std::vector<uint16_t> out(vectors.size() * sub_dim_ * m_);
+        quantize_into(vectors, out.data());
+        return out;
+    }
+
+    // ... into the caller's array
+    void quantize_into(const Rows &vectors, uint16_t *out) const {
         size_t dim = sub_dim_ * m_, n = vectors.size();
-        if (n == 0) return {};
+        if (n == 0) return;
         vectors.expect_dim(dim);
         const float *flat = vectors.data();
+        if (vq_pq_quantize_host) {
+            dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), flat, (int64_t)n, (int32_t)m_,
+                                            (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(), nullptr, nullptr, out));
+            return;
+        }
         DeviceBuffer<float> dx(dev_, n * dim);
         dx.upload(flat, dx.size());
         DeviceCodes dcodes(dev_, n * m_, k_);
@@ -407,13 +458,30 @@ public:
         dev_->check(abi_assign(dev_->ctx(), distance_.abi_metric(), dx.get(), n, dim, m_, sub_dim_, k_,
                                codebooks_.get(), dcodes));
         dev_->check(abi_decode_f16(dev_->ctx(), dcodes, n, m_, sub_dim_, k_, codebooks_.get(), dout.get()));
-        return dout.to_host();
+        dout.download(out, n * dim);
     }
 
     // The integer codes the reference keeps only as `best_index` (src/pq.rs:166-174): n x m bytes
     // (k <= 256), or 16 bits each for any k.
-    std::vector<uint8_t> encode(const Rows &vectors) const { return encode_device(vectors).to_host8(); }
+    std::vector<uint8_t> encode(const Rows &vectors) const {
+        std::vector<uint8_t> codes(vectors.size() * m_);
+        encode_into(vectors, codes.data());
+        return codes;
+    }
     std::vector<uint16_t> encode16(const Rows &vectors) const { return encode_device(vectors).to_host16(); }
+    // n x m bytes (k <= 256) into the caller's array
+    void encode_into(const Rows &vectors, uint8_t *codes) const {
+        const size_t n = vectors.size();
+        if (n == 0) return;
+        vectors.expect_dim(sub_dim_ * m_);
+        if (k_ <= 256 && vq_pq_quantize_host) {
+            dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)n, (int32_t)m_,
+                                            (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(), nullptr, codes, nullptr));
+            return;
+        }
+        const std::vector<uint8_t> c = encode_device(vectors).to_host8();
+        std::copy(c.begin(), c.end(), codes);
+    }
 
     std::vector<float> codebooks() const { return codebooks_.to_host(); }  // m*k*sub_dim
     size_t m() const { return m_; }
@@ -511,7 +579,7 @@ public:
     Vector<f16> quantize(const Vector<float> &vector) const {
         if (vector.len() != dim_) throw VqError::DimensionMismatch(dim_, vector.len());
         if (!trained_) return Vector<f16>();  // the loop over no codebooks pushes nothing (opq.rs:244-263)
-        return quantize_batch(std::vector<Vector<float>>{vector})[0];
+        return quantize_one(*this, vector);
     }
 
     std::vector<Vector<f16>> quantize_batch(const Rows &vectors) const {
@@ -524,21 +592,51 @@ public:
 
     // n x dim f16 bit patterns; empty (n rows of length 0) when fit ran no outer iteration
     std::vector<uint16_t> quantize_batch_flat(const Rows &vectors) const {
-        size_t n = vectors.size();
-        if (n == 0) return {};
         if (!trained_) {
             vectors.expect_dim(dim_);
             return {};
         }
+        std::vector<uint16_t> out(vectors.size() * dim_);
+        quantize_into(vectors, out.data());
+        return out;
+    }
+
+    // ... into the caller's array (nothing is written when fit ran no outer iteration)
+    void quantize_into(const Rows &vectors, uint16_t *out) const {
+        size_t n = vectors.size();
+        if (n == 0) return;
+        vectors.expect_dim(dim_);
+        if (!trained_) return;
+        if (vq_pq_quantize_host) {
+            dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)n, (int32_t)m_,
+                                            (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(), d_rotation_.get(), nullptr,
+                                            out));
+            return;
+        }
         DeviceCodes dcodes = encode_device(vectors);
         DeviceBuffer<uint16_t> dout(dev_, n * dim_);
         dev_->check(abi_decode_f16(dev_->ctx(), dcodes, n, m_, sub_dim_, k_, codebooks_.get(), dout.get()));
-        return dout.to_host();
+        dout.download(out, n * dim_);
     }
 
     std::vector<uint8_t> encode(const Rows &vectors) const {
         if (vectors.empty() || !trained_) return {};
-        return encode_device(vectors).to_host8();
+        std::vector<uint8_t> codes(vectors.size() * m_);
+        encode_into(vectors, codes.data());
+        return codes;
+    }
+    // n x m bytes (k <= 256) into the caller's array
+    void encode_into(const Rows &vectors, uint8_t *codes) const {
+        if (vectors.empty() || !trained_) return;
+        vectors.expect_dim(dim_);
+        if (k_ <= 256 && vq_pq_quantize_host) {
+            dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)vectors.size(),
+                                            (int32_t)m_, (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(),
+                                            d_rotation_.get(), codes, nullptr));
+            return;
+        }
+        const std::vector<uint8_t> c = encode_device(vectors).to_host8();
+        std::copy(c.begin(), c.end(), codes);
     }
     std::vector<uint16_t> encode16(const Rows &vectors) const {  // any k
         if (vectors.empty() || !trained_) return {};
@@ -658,7 +756,7 @@ public:
     // src/rvq.rs:171-215
     Vector<f16> quantize(const Vector<float> &vector) const {
         if (vector.len() != dim_) throw VqError::DimensionMismatch(dim_, vector.len());
-        return quantize_batch(std::vector<Vector<float>>{vector})[0];
+        return quantize_one(*this, vector);
     }
 
     std::vector<Vector<f16>> quantize_batch(const Rows &vectors, std::vector<uint8_t> *codes = nullptr) const {
@@ -668,15 +766,38 @@ public:
     // codes: n x stages bytes (k <= 256 only); codes16: the same 16 bits wide, any k
     std::vector<uint16_t> quantize_batch_flat(const Rows &vectors, std::vector<uint8_t> *codes = nullptr,
                                               std::vector<uint16_t> *codes16 = nullptr) const {
-        size_t n = vectors.size();
+        const size_t n = vectors.size();
         if (n == 0) return {};
+        std::vector<uint16_t> out(n * dim_);
+        if (codes && k_ > 256) throw VqError::InvalidParameter("codes above 256 centroids are 16 bits wide");
+        if (k_ > 256) {
+            if (codes16) codes16->resize(n * stages_);
+            quantize_into(vectors, out.data(), codes16 ? codes16->data() : nullptr);
+            return out;
+        }
+        std::vector<uint8_t> c8(codes || codes16 ? n * stages_ : 0);
+        quantize_into(vectors, out.data(), codes || codes16 ? c8.data() : nullptr);
+        if (codes16) codes16->assign(c8.begin(), c8.end());
+        if (codes) *codes = std::move(c8);
+        return out;
+    }
+
+    // The same into the caller's arrays (either may be null); codes: bytes up to 256 centroids, else 16 bits.
+    void quantize_into(const Rows &vectors, uint16_t *out, void *codes = nullptr) const {
+        const size_t n = vectors.size();
+        if (n == 0) return;
         vectors.expect_dim(dim_);
         const float *flat = vectors.data();
+        const int32_t k = (int32_t)std::max<size_t>(k_, 1);
+        if (vq_rvq_quantize_host) {
+            dev_->check(vq_rvq_quantize_host(dev_->ctx(), distance_.abi_metric(), flat, (int64_t)n, (int32_t)dim_,
+                                             (int32_t)stages_, k, codebooks_.get(), epsilon_, codes, out));
+            return;
+        }
         DeviceBuffer<float> dx(dev_, n * dim_);
         dx.upload(flat, dx.size());
         DeviceCodes dcodes(dev_, std::max<size_t>(n * stages_, 1), k_);
         DeviceBuffer<uint16_t> dout(dev_, n * dim_);
-        const int32_t k = (int32_t)std::max<size_t>(k_, 1);
         dev_->check(dcodes.wide()
                         ? vq_rvq_encode_u16(dev_->ctx(), distance_.abi_metric(), dx.get(), (int64_t)n, (int64_t)dim_,
                                             (int32_t)dim_, (int32_t)stages_, k, codebooks_.get(), epsilon_,
@@ -684,12 +805,15 @@ public:
                         : vq_rvq_encode(dev_->ctx(), distance_.abi_metric(), dx.get(), (int64_t)n, (int64_t)dim_,
                                         (int32_t)dim_, (int32_t)stages_, k, codebooks_.get(), epsilon_, dcodes.p8(),
                                         nullptr, dout.get()));
-        if (codes) *codes = dcodes.to_host8();
-        if (codes16) *codes16 = dcodes.to_host16();
-        return dout.to_host();
+        if (codes && stages_) {
+            const void *c = dcodes.wide() ? (const void *)dcodes.p16() : (const void *)dcodes.p8();
+            dev_->check(vq_d2h(dev_->ctx(), codes, c, n * stages_ * (dcodes.wide() ? 2 : 1)));
+        }
+        if (out) dout.download(out, n * dim_);
     }
 
     size_t stages() const { return stages_; }
+    size_t k() const { return k_; }
     std::vector<float> codebooks() const {  // stages*k*dim
         std::vector<float> all = codebooks_.to_host();
         all.resize(stages_ * k_ * dim_);
@@ -771,7 +895,7 @@ public:
     // src/tsvq.rs:231-249
     Vector<f16> quantize(const Vector<float> &vector) const {
         if (vector.len() != dim_) throw VqError::DimensionMismatch(dim_, vector.len());
-        return quantize_batch(std::vector<Vector<float>>{vector})[0];
+        return quantize_one(*this, vector);
     }
 
     std::vector<Vector<f16>> quantize_batch(const Rows &vectors, std::vector<int32_t> *leaves = nullptr) const {
@@ -779,19 +903,32 @@ public:
     }
 
     std::vector<uint16_t> quantize_batch_flat(const Rows &vectors, std::vector<int32_t> *leaves = nullptr) const {
+        std::vector<uint16_t> out(vectors.size() * dim_);
+        if (leaves && !vectors.empty()) leaves->resize(vectors.size());
+        quantize_into(vectors, out.data(), leaves ? leaves->data() : nullptr);
+        return out;
+    }
+
+    // The same into the caller's arrays (either may be null).
+    void quantize_into(const Rows &vectors, uint16_t *out, int32_t *leaves = nullptr) const {
         size_t n = vectors.size();
-        if (n == 0) return {};
+        if (n == 0) return;
         vectors.expect_dim(dim_);
         const float *flat = vectors.data();
+        if (vq_tsvq_quantize_host) {
+            dev_->check(vq_tsvq_quantize_host(dev_->ctx(), distance.abi_metric(), flat, (int64_t)n, tree_.get(), leaves, out));
+            return;
+        }
         DeviceBuffer<float> dx(dev_, n * dim_);
         dx.upload(flat, dx.size());
         DeviceBuffer<int32_t> dleaf(dev_, n);
         DeviceBuffer<uint16_t> dout(dev_, n * dim_);
         dev_->check(vq_tsvq_descend(dev_->ctx(), distance.abi_metric(), dx.get(), (int64_t)n, (int64_t)dim_,
                                     tree_.get(), dleaf.get()));
+        if (leaves) dleaf.download(leaves, n);
+        if (!out) return;
         dev_->check(vq_tsvq_decode_f16(dev_->ctx(), tree_.get(), dleaf.get(), (int64_t)n, dout.get()));
-        if (leaves) *leaves = dleaf.to_host();
-        return dout.to_host();
+        dout.download(out, n * dim_);
     }
 
     int32_t n_nodes() const {

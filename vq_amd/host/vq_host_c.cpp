@@ -48,9 +48,6 @@ int guarded(F &&f) {
     }
 }
 
-void flatten(const std::vector<uint16_t> &q, uint16_t *out) {
-    if (!q.empty()) std::memcpy(out, q.data(), q.size() * sizeof(uint16_t));
-}
 }  // namespace
 
 extern "C" {
@@ -172,10 +169,10 @@ int vqh_quantize_batch(void *obj, const float *x, int64_t n, int64_t dim, uint16
         Obj *o = (Obj *)obj;
         auto rows = rows_of(x, n, dim);
         switch (o->kind) {
-        case 1: flatten(o->pq->quantize_batch_flat(rows), out); break;
-        case 2: flatten(o->opq->quantize_batch_flat(rows), out); break;
-        case 3: flatten(o->rvq->quantize_batch_flat(rows), out); break;
-        default: flatten(o->tsvq->quantize_batch_flat(rows), out); break;
+        case 1: o->pq->quantize_into(rows, out); break;
+        case 2: o->opq->quantize_into(rows, out); break;
+        case 3: o->rvq->quantize_into(rows, out); break;
+        default: o->tsvq->quantize_into(rows, out); break;
         }
     });
 }
@@ -207,14 +204,15 @@ int vqh_encode(void *obj, const float *x, int64_t n, int64_t dim, uint8_t *codes
     return guarded([&] {
         Obj *o = (Obj *)obj;
         auto rows = rows_of(x, n, dim);
-        std::vector<uint8_t> c;
         switch (o->kind) {
-        case 1: c = o->pq->encode(rows); break;
-        case 2: c = o->opq->encode(rows); break;
-        case 3: o->rvq->quantize_batch_flat(rows, &c); break;
+        case 1: o->pq->encode_into(rows, codes); break;
+        case 2: o->opq->encode_into(rows, codes); break;
+        case 3:
+            if (o->rvq->k() > 256) throw vq::VqError::InvalidParameter("codes above 256 centroids are 16 bits wide");
+            o->rvq->quantize_into(rows, nullptr, codes);
+            break;
         default: throw vq::VqError::InvalidParameter("TSVQ has leaves, not codes");
         }
-        std::memcpy(codes, c.data(), c.size());
     });
 }
 
@@ -238,9 +236,7 @@ int vqh_leaves(void *obj, const float *x, int64_t n, int64_t dim, int32_t *leave
     return guarded([&] {
         Obj *o = (Obj *)obj;
         if (o->kind != 4) throw vq::VqError::InvalidParameter("not a TSVQ");
-        std::vector<int32_t> l;
-        o->tsvq->quantize_batch_flat(rows_of(x, n, dim), &l);
-        std::memcpy(leaves, l.data(), l.size() * sizeof(int32_t));
+        o->tsvq->quantize_into(rows_of(x, n, dim), nullptr, leaves);
     });
 }
 
