@@ -908,17 +908,28 @@ __device__ __forceinline__ void wide_pair_blocks(const AssignArgs &a, int sd, co
         const int j = (int)((ent.y >> (8 * (lane & 1))) & 0xFFu);
         const float4 *xp = reinterpret_cast<const float4 *>(a.x + row * a.ld + (int64_t)s * sd);
         const float4 *cp = reinterpret_cast<const float4 *>(a.cb + ((size_t)s * a.k + j) * sd);
-        float acc = 0.0f;
+        float acc = 0.0f, sa = 0.0f;
+        auto step = [&](float x, float c) {
+            wide_step<METRIC>(acc, x, c);
+            if constexpr (METRIC == M_COS) {
+                const float p = x * x;
+                sa = sa + p;
+            }
+        };
 #pragma unroll 4
         for (int t = 0; t < sd / 4; ++t) {
             const float4 xv = xp[t], cv = cp[t];
-            wide_step<METRIC>(acc, xv.x, cv.x);
-            wide_step<METRIC>(acc, xv.y, cv.y);
-            wide_step<METRIC>(acc, xv.z, cv.z);
-            wide_step<METRIC>(acc, xv.w, cv.w);
+            step(xv.x, cv.x);
+            step(xv.y, cv.y);
+            step(xv.z, cv.z);
+            step(xv.w, cv.w);
         }
         float d = acc;
         if constexpr (METRIC == M_EUCLID) d = sqrtf(d);
+        if constexpr (METRIC == M_COS) {
+            const float na = sqrtf(sa), nb = a.cnorm[(size_t)s * a.k + j], den = na * nb, q = acc / den;
+            d = (na == 0.0f || nb == 0.0f) ? 1.0f : 1.0f - q;
+        }
         d = (d == d) ? d : inf;
         const float od = __shfl_xor(d, 1);
         const int oj = __shfl_xor(j, 1);
@@ -949,7 +960,7 @@ __global__ void __launch_bounds__(256) k_assign_wide_exact(AssignArgs a, int sd,
     // follow-ups of the matrix-core pass are independent and run side by side in one launch (the
     // pairs first: workgroups start in index order, and behind a long list of rows they would wait).
     unsigned block = blockIdx.x;
-    if constexpr (LISTED && (METRIC == M_SQ || METRIC == M_EUCLID)) {
+    if constexpr (LISTED && METRIC != M_L1) {
         const unsigned pair_blocks = gridDim.x - exact_blocks;
         if (block < pair_blocks) {
             wide_pair_blocks<METRIC, LBG>(a, sd, pairs, *pair_count, block, pair_blocks);

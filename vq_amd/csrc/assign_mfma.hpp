@@ -161,6 +161,60 @@ __device__ __forceinline__ uint32_t bf16_pack2(float a, float b) {
     return __builtin_bit_cast(uint32_t, h);
 }
 
+// ---- cosine -----------------------------------------------------------------------------------
+// d = 1 - x.c / (|x| |c|) falls as x.c/|c| grows, so with the centroids divided by their norms the scores
+// s[j] = P - 2 x.(c_j / |c_j|), P >= 2 |x| the same in every score of a row (it keeps them from turning
+// negative), order the candidates: no centre, no ||c||^2.  u = 2^-24, sd the block's width.
+//   score: 3 * 2^-16 * 2 |x| from the operand split, 2^-22 * 2 |x| from the division by the norm,
+//     the fp32 accumulation of partial sums below 4.2 |x|;
+//   reference (src/distances.rs:141-151): the sums, the product of the norms, the quotient and the
+//     difference from 1 leave d within (sd + 6) u of its value at the computed norms, 2 |x| (sd + 6) u here.
+// Width 8: (9.2e-5 + 7.5e-6 + 4.8e-7 + 1.7e-6) |x| per candidate, below 2.1e-4 |x| for two; the test
+// uses 2^-12 |x| (2.44e-4), plus 2^-14 |second| for the packed bits.  Rows and centroids whose norm is
+// outside [1e-15, 1e15] and not zero, where the reference's products may over- or underflow, and rows
+// of norm zero go to the exact argmin (a centroid of norm zero has d = 1, its score P: in order).
+__device__ __forceinline__ float seq_norm8(const float (&c)[8]) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const float p = c[t] * c[t];
+        acc = acc + p;
+    }
+    return sqrtf(acc);
+}
+// c divided by its norm; 0, or NaN if the block must not be scored with this centroid in it.
+__device__ __forceinline__ float cos_normalise(float (&c)[8]) {
+    const float nb = seq_norm8(c);
+    const bool zero = nb == 0.0f;
+    const float inv = zero ? 0.0f : 1.0f / nb;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) c[t] *= inv;
+    return zero || (nb >= 1e-15f && nb <= 1e15f) ? 0.0f : __builtin_nanf("");
+}
+// Distances as sort keys: smaller distance, smaller unsigned key.  Squared and plain Euclidean
+// distances are non-negative, a cosine distance may be a little below zero.
+template <int METRIC> __device__ __forceinline__ uint32_t dist_key(float d) {
+    const uint32_t b = __float_as_uint(d);
+    if constexpr (METRIC == M_COS) return b ^ ((uint32_t)((int)b >> 31) | 0x80000000u);
+    return b;
+}
+template <int METRIC> __device__ __forceinline__ float key_dist(uint32_t k) {
+    if constexpr (METRIC == M_COS) return __uint_as_float(k ^ ((k & 0x80000000u) ? 0x80000000u : 0xffffffffu));
+    return __uint_as_float(k);
+}
+// The distance of a row's eight floats to centroid c, in the reference's order; na, nb: the two norms.
+template <int METRIC>
+__device__ __forceinline__ float dist8(const float (&x)[8], const float (&c)[8], float na, float nb) {
+    if constexpr (METRIC == M_COS) {
+        const float dot = d_dot<8>(x, c);
+        const float den = na * nb, q = dot / den;
+        return (na == 0.0f || nb == 0.0f) ? 1.0f : 1.0f - q;
+    } else {
+        const float d = d_sq<8>(x, c);
+        return METRIC == M_EUCLID ? sqrtf(d) : d;
+    }
+}
+
 // Tables for k_assign_mfma_bf.  One workgroup per column block s, one thread per padded centroid
 // (k <= 256).  Rows and centroids are scored relative to mu[s] = mean of the block's centroids
 // (distances do not change under a common shift, the bound on the score error, which is
@@ -168,6 +222,9 @@ __device__ __forceinline__ uint32_t bf16_pack2(float a, float b) {
 // block (NaN if any is NaN).  mfma_bf_prep_block is the work of one workgroup, given centroid j
 // of the block in thread j's registers (zeros from k on); k_mfma_bf_prep reads the centroids from
 // the codebook, the LBG loop's last update kernel has just computed them.
+// COS: the operands are those of the centroids divided by their norms, the centre and ||c||^2 are zero
+// and maxc2[s] only says whether the block can be scored (see own_operands).
+template <bool COS = false>
 __device__ __forceinline__ void mfma_bf_prep_block(float (&c)[8], int s, int j, int k, int nb,
                                                    u32x4 *__restrict__ atab, float *__restrict__ maxc2,
                                                    float *__restrict__ mu) {
@@ -175,9 +232,11 @@ __device__ __forceinline__ void mfma_bf_prep_block(float (&c)[8], int s, int j, 
     __shared__ float sh_mu[4][8];
     // centre: sum of c / 256 (no overflow for k <= 256), then * 256 / k
     float centre[8];
+    float cos_bad = 0.0f;
+    if constexpr (COS) cos_bad = cos_normalise(c);
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-        float v = c[t] * 0.00390625f;
+        float v = COS ? 0.0f : c[t] * 0.00390625f;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
         if ((j & 63) == 0) sh_mu[j >> 6][t] = v;
@@ -197,9 +256,9 @@ __device__ __forceinline__ void mfma_bf_prep_block(float (&c)[8], int s, int j, 
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
                 c[t] -= centre[t];
-                c2 = __builtin_fmaf(c[t], c[t], c2);
+                c2 = COS ? 0.0f : __builtin_fmaf(c[t], c[t], c2);
             }
-            mx = c2;
+            mx = COS ? cos_bad : c2;
         }
         uint32_t hb[8], lb[8];
 #pragma unroll
@@ -244,6 +303,7 @@ __device__ __forceinline__ void mfma_bf_prep_block(float (&c)[8], int s, int j, 
     }
 }
 
+template <bool COS = false>
 static __global__ void __launch_bounds__(256) k_mfma_bf_prep(const float *__restrict__ cb, int m, int k, int nb,
                                                              u32x4 *__restrict__ atab, float *__restrict__ maxc2,
                                                              float *__restrict__ mu, uint32_t *__restrict__ stat,
@@ -253,14 +313,16 @@ static __global__ void __launch_bounds__(256) k_mfma_bf_prep(const float *__rest
     float c[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) c[t] = (j < k) ? cb[((size_t)s * k + j) * 8 + t] : 0.0f;
-    mfma_bf_prep_block(c, s, j, k, nb, atab, maxc2, mu);
+    mfma_bf_prep_block<COS>(c, s, j, k, nb, atab, maxc2, mu);
 }
 
 // The tables of mfma_bf_prep_block made by one wave for itself (the same operands up to the order in
 // which the centre's sum is added, which any centre allows): lane (r, h) makes its own operands of
 // the centroids 32 b + r, dimensions [4h, 4h + 4), from the wave's copy of the centroids in LDS.
-__device__ __forceinline__ void own_operands(const float *cl, int k, int nb, int r, int h, u32x4 (&A1)[8],
-                                             u32x4 (&A2)[8], float (&muh)[4], float &mc2) {
+// COS: of the centroids divided by their norms (norms: one per centroid, in LDS).
+template <bool COS>
+__device__ __forceinline__ void own_operands(const float *cl, const float *norms, int k, int nb, int r, int h,
+                                             u32x4 (&A1)[8], u32x4 (&A2)[8], float (&muh)[4], float &mc2) {
     float cv[8][4];
     float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -269,7 +331,7 @@ __device__ __forceinline__ void own_operands(const float *cl, int k, int nb, int
         const float4 v = *reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * 8 + 4 * h);
         cv[b][0] = v.x, cv[b][1] = v.y, cv[b][2] = v.z, cv[b][3] = v.w;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) sum[u] += j < k ? cv[b][u] * 0.00390625f : 0.0f;  // no overflow for k <= 256
+        for (int u = 0; u < 4; ++u) sum[u] += j < k && !COS ? cv[b][u] * 0.00390625f : 0.0f;  // no overflow for k <= 256
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -286,18 +348,25 @@ __device__ __forceinline__ void own_operands(const float *cl, int k, int nb, int
             continue;
         }
         const bool live = 32 * b + r < k;
-        float p = 0.0f, a[4];
+        float p = 0.0f, a[4], scale = -2.0f, c2;
+        if constexpr (COS) {
+            const float nc = live ? norms[32 * b + r] : 0.0f;
+            scale = nc == 0.0f ? 0.0f : -2.0f * (1.0f / nc);
+            c2 = nc == 0.0f || (nc >= 1e-15f && nc <= 1e15f) ? 0.0f : __builtin_nanf("");
+        }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const float c = live ? cv[b][u] - muh[u] : 0.0f;
             p = __builtin_fmaf(c, c, p);
-            a[u] = -2.0f * c;
+            a[u] = scale * c;
         }
-        int pa, pb;
-        swap_halves(__float_as_int(p), pa, pb);
-        float c2 = __int_as_float(pa) + __int_as_float(pb);
+        if constexpr (!COS) {
+            int pa, pb;
+            swap_halves(__float_as_int(p), pa, pb);
+            c2 = __int_as_float(pa) + __int_as_float(pb);
+        }
         mx = (mx == mx && c2 == c2) ? fmaxf(mx, c2) : __builtin_nanf("");
-        c2 = live ? c2 : kPadScore;
+        c2 = live ? (COS ? 0.0f : c2) : kPadScore;
         const uint32_t h01 = bf16_pack2(a[0], a[1]), h23 = bf16_pack2(a[2], a[3]);
         const uint32_t l01 = bf16_pack2(a[0] - __uint_as_float(h01 << 16), a[1] - __uint_as_float(h01 & 0xffff0000u));
         const uint32_t l23 = bf16_pack2(a[2] - __uint_as_float(h23 << 16), a[3] - __uint_as_float(h23 & 0xffff0000u));
@@ -327,7 +396,7 @@ __device__ __forceinline__ void own_operands(const float *cl, int k, int nb, int
 template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
 }
-// (d, i) <- the lexicographically smaller of (d, i) and (od, oi); d holds non-negative float bits
+// (d, i) <- the lexicographically smaller of (d, i) and (od, oi); d holds dist_key values
 __device__ __forceinline__ void lexmin(uint32_t &d, uint32_t &i, uint32_t od, uint32_t oi) {
     const bool take = od < d || (od == d && oi < i);
     d = take ? od : d;
@@ -340,7 +409,8 @@ __device__ __forceinline__ void lexmin(uint32_t &d, uint32_t &i, uint32_t od, ui
 // `code` and `dist`).
 template <int METRIC>
 __device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, float &dist, const float *cl,
-                                           const float *__restrict__ xblk, int64_t ld, int k, int lane) {
+                                           const float *norms, const float *__restrict__ xblk, int64_t ld, int k,
+                                           int lane) {
     const float inf = __builtin_inff();
     while (todo) {
         int src[8];
@@ -361,14 +431,14 @@ __device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, fl
                 xs[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(val), 8 * i + d));
             float bd = inf, dfirst = 0.0f;
             uint32_t bi = 0x7fffffffu;
+            const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int j = lane + 64 * q;
                 const float4 *cp = reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * 8);
                 const float4 c0 = cp[0], c1 = cp[1];
                 const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-                float d = d_sq<8>(xs, c);
-                if constexpr (METRIC == M_EUCLID) d = sqrtf(d);
+                float d = dist8<METRIC>(xs, c, na, METRIC == M_COS ? norms[j < k ? j : 0] : 0.0f);
                 if (q == 0) dfirst = d;
                 d = (d == d) ? d : inf;
                 if (j < k && (d < bd || bi == 0x7fffffffu)) {
@@ -376,7 +446,7 @@ __device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, fl
                     bi = (uint32_t)j;
                 }
             }
-            uint32_t kd = __float_as_uint(bd), ki = bi;
+            uint32_t kd = dist_key<METRIC>(bd), ki = bi;
             lexmin(kd, ki, dpp_u32<0xB1>(kd), dpp_u32<0xB1>(ki));
             lexmin(kd, ki, dpp_u32<0x4E>(kd), dpp_u32<0x4E>(ki));
             lexmin(kd, ki, dpp_u32<0x141>(kd), dpp_u32<0x141>(ki));
@@ -393,7 +463,7 @@ __device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, fl
             for (int u = 1; u < 8; ++u) who = (i == u) ? src[u] : who;
             if (lane == who) {
                 code = best;
-                dist = (d0 == d0) ? __uint_as_float(rd) : d0;  // the chosen centroid's distance as computed
+                dist = (d0 == d0) ? key_dist<METRIC>(rd) : d0;  // the chosen centroid's distance as computed
             }
         }
     }
@@ -422,6 +492,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
                                                             int64_t run_stride) {
     constexpr int SD = 8;
     __shared__ __attribute__((aligned(16))) float lds_cb[4][256 * SD];
+    __shared__ float lds_norm[METRIC == M_COS ? 4 : 1][METRIC == M_COS ? 256 : 1];  // the centroids' norms
     // the wave's number through readfirstlane: what follows from it (column block, first row, base
     // addresses) is then uniform for the compiler and lives in scalar registers
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -454,6 +525,19 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
             if (i < nv) dst[i] = v;
         }
     }
+    float *norms = lds_norm[METRIC == M_COS ? wave : 0];
+    if constexpr (METRIC == M_COS) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int j = lane + 64 * q;
+            const float4 *cp = reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * SD);
+            const float4 c0 = cp[0], c1 = cp[1];
+            const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+            norms[j] = seq_norm8(c);
+        }
+    }
     // the A operands of every block of 32 centroids, the centre's dimensions [4h, 4h + 4), the bound
     u32x4 A1[8], A2[8];
     float muh[4];
@@ -463,7 +547,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
             for (int i = threadIdx.x; i < kStatSlots; i += 256) tb.stat_next[i * kStatStride] = 0u;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        own_operands(cl, k, nb, r, h, A1, A2, muh, mc2);
+        own_operands<METRIC == M_COS>(cl, norms, k, nb, r, h, A1, A2, muh, mc2);
     } else {
         const u32x4 *ap = tb.atab + (size_t)s * nb * 128 + lane;
 #pragma unroll
@@ -541,12 +625,17 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
             // this half's share of ||x||^2 as one bf16 number rounded up (p >= 0; the same in every score
             // of the row, so its rounding cancels in their differences, and rounding up keeps the
             // scores from turning negative), then ones for the parts of ||c||^2
-            const uint32_t p0 = (__float_as_uint(p) + 0xFFFFu) >> 16;
-            b1 = u32x4{h01, h23, l01, l23};
-            b2 = u32x4{h01, h23, p0, 0x3f803f80u};
+            // (cosine: x2 becomes |x|, and the lower half brings P = 2.01 |x| in)
             int pa, pb;
             swap_halves(__float_as_int(p), pa, pb);
             x2 = __int_as_float(pa) + __int_as_float(pb);  // lower half's share + upper half's, in both
+            if constexpr (METRIC == M_COS) {
+                x2 = __builtin_amdgcn_sqrtf(x2);
+                p = h == 0 ? 2.01f * x2 : 0.0f;
+            }
+            const uint32_t p0 = (__float_as_uint(p) + 0xFFFFu) >> 16;
+            b1 = u32x4{h01, h23, l01, l23};
+            b2 = u32x4{h01, h23, p0, 0x3f803f80u};
         }
         int m1 = 0x7f800000, m2 = 0x7f800000;  // +inf
         // One block of 32 centroids.  The tag leaves out the lane half (bit 2), so it is the same in
@@ -623,12 +712,12 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
         const float s1 = __int_as_float(imin(f1, g1));
         const float s2 = __int_as_float(imin(imax(f1, g1), imin(f2, g2)));
         const bool mine = h == 0 && t < lane_tiles;  // the lane's row of this tile exists
-        const float bound = x2 + mc2;
-        const float margin = 6.103515625e-05f * fabsf(s2) + 1.220703125e-04f * bound;
+        const float bound = x2 + mc2;  // (cosine: |x|, or NaN)
+        const float margin = 6.103515625e-05f * fabsf(s2) + (METRIC == M_COS ? 2.44140625e-04f : 1.220703125e-04f) * bound;
         bool sure = (s2 - s1) > margin;  // false for NaN / inf-inf
         // below 1e-31 the bf16 parts of ||c - mu||^2 may be subnormal, which the matrix cores may
         // flush: up to 3 * 2^-126 lost, more than the margin allows for at such a bound
-        sure = sure && (bound < 1e29f) && (bound > 1e-31f) && (s1 < 1e29f);
+        sure = sure && (bound < (METRIC == M_COS ? 1e15f : 1e29f)) && (bound > (METRIC == M_COS ? 1e-15f : 1e-31f)) && (s1 < 1e29f);
         const int first = (int)(__float_as_uint(s1) & 0xFFu);  // first centroid of the best run
         const unsigned long long todo = __ballot(mine && !sure);
         int code;
@@ -650,24 +739,22 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
             }
             const float ca[8] = {ca0.x, ca0.y, ca0.z, ca0.w, ca1.x, ca1.y, ca1.z, ca1.w};
             const float cc[8] = {cb0.x, cb0.y, cb0.z, cb0.w, cb1.x, cb1.y, cb1.z, cb1.w};
-            float da = d_sq<8>(xs, ca), db = d_sq<8>(xs, cc);
-            if constexpr (METRIC == M_EUCLID) {
-                da = sqrtf(da);
-                db = sqrtf(db);
-            }
+            const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
+            const float da = dist8<METRIC>(xs, ca, na, METRIC == M_COS ? norms[ja] : 0.0f);
+            const float db = dist8<METRIC>(xs, cc, na, METRIC == M_COS ? norms[jb] : 0.0f);
             const bool second = (j0 + 1 < k) && (db < da);  // strict: the first of equals
-            uint32_t kd = __float_as_uint(second ? db : da);
+            uint32_t kd = dist_key<METRIC>(second ? db : da);
             const uint32_t ki = (uint32_t)(second ? j0 + 1 : j0);
-            kd = j0 < k ? kd : 0x7f800000u;  // a padding centroid
+            kd = j0 < k ? kd : 0xffffffffu;  // a padding centroid
             int dlo, dhi, ilo, ihi;
             swap_halves((int)kd, dlo, dhi);
             swap_halves((int)ki, ilo, ihi);
             code = (uint32_t)dhi < (uint32_t)dlo ? ihi : ilo;  // the lower half holds the lower indices
-            dist = __uint_as_float((uint32_t)dhi < (uint32_t)dlo ? (uint32_t)dhi : (uint32_t)dlo);
+            dist = key_dist<METRIC>((uint32_t)dhi < (uint32_t)dlo ? (uint32_t)dhi : (uint32_t)dlo);
         }
         if (todo) {  // the same in every lane: the reference-order argmin of the undecided rows
             n_exact += (uint32_t)__popcll(todo);
-            code = exact_rows8<METRIC>(todo, code, dist, cl, a.x + (row0 + 32 * (int64_t)t) * a.ld + (int64_t)s * SD, a.ld,
+            code = exact_rows8<METRIC>(todo, code, dist, cl, norms, a.x + (row0 + 32 * (int64_t)t) * a.ld + (int64_t)s * SD, a.ld,
                                            k, lane);
         }
         if (mine) {
@@ -842,6 +929,9 @@ static __global__ void __launch_bounds__(256) k_block_centres(const float *__res
     }
 }
 
+// COS: the operands of the centroids divided by their norms (cnorm), no centre, no ||c||^2; blockmax is 0,
+// or NaN where a norm is outside the range that the scores can decide (see cos_normalise).
+template <bool COS = false>
 static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *__restrict__ cb,
                                                                   const float *__restrict__ mu,
                                                                   const float2 *__restrict__ norms,
@@ -849,7 +939,8 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
                                                                   int sd, u32x4 *__restrict__ atab,
                                                                   float *__restrict__ c2perm,
                                                                   float *__restrict__ blockmax,
-                                                                  uint32_t *__restrict__ list_count) {
+                                                                  uint32_t *__restrict__ list_count,
+                                                                  const float *__restrict__ cnorm = nullptr) {
     const int s = blockIdx.x, b = blockIdx.y;
     const int i = threadIdx.x & 31, g = threadIdx.x >> 5;
     const int j = b * 32 + i;
@@ -857,12 +948,14 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
     __shared__ float part[8][32];
     // the same decision in every workgroup of the column block (same values, same order)
     float mm = 0.0f, cc = 0.0f;
-    for (int y = 0; y < (sd + 31) / 32; ++y) {
+    for (int y = 0; y < (COS ? 0 : (sd + 31) / 32); ++y) {
         const float2 v = norms[(size_t)s * ((sd + 31) / 32) + y];
         mm += v.x;
         cc += v.y;
     }
-    const bool on = mm > 0.25f * cc && mm < 1e30f && sd <= kWideCentreMax;  // false for NaN
+    const float nc = COS ? cnorm[(size_t)s * k + (j < k ? j : 0)] : 1.0f;
+    const float scale = nc == 0.0f ? 0.0f : -2.0f * (1.0f / nc);
+    const bool on = !COS && mm > 0.25f * cc && mm < 1e30f && sd <= kWideCentreMax;  // false for NaN
     if (b == 0 && threadIdx.x == 0) shifted[s] = on ? 1 : 0;
     const float *c = cb + ((size_t)s * k + (j < k ? j : 0)) * sd;
     float p = 0.0f;
@@ -893,7 +986,7 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
                 for (int e = 0; e < 2; ++e) {
                     const float x = in ? cv[2 * w + e] : 0.0f;
                     p = __builtin_fmaf(x, x, p);
-                    const float a = (j < k) ? -2.0f * x : 0.0f;
+                    const float a = (j < k) ? (COS ? scale : -2.0f) * x : 0.0f;
                     hb[e] = bf16_rne_bits(a);
                     lb[e] = bf16_rne_bits(a - bf16_bits_to_float(hb[e]));
                 }
@@ -910,7 +1003,9 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
         float c2 = 0.0f;
 #pragma unroll
         for (int q = 0; q < 8; ++q) c2 = c2 + part[q][i];
+        if constexpr (COS) c2 = nc == 0.0f || (nc >= 1e-15f && nc <= 1e15f) ? 0.0f : __builtin_nanf("");
         float mx = c2;
+        if constexpr (COS) c2 = 0.0f;
         if (j >= k) {
             c2 = kPadScore;
             mx = 0.0f;
@@ -940,7 +1035,9 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // per element, as the separate pass would; in place, or from the rows of a.pend_src into a.x — and
 // then scores them as any other rows, which it now reads from the cache levels it has just written
 // through.  No other workgroup reads or writes these rows.
-template <bool LBG, int NB, bool PEND = false>
+// COS: cosine distance (see cos_normalise): the scores are P - 2 x.c/|c| with P = 2.01 |x|, the bound is in
+// units of |x|.
+template <bool LBG, int NB, bool PEND = false, bool COS = false>
 __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, MfmaWideBfTables tb) {
     constexpr int NBMAX = 8;
     __shared__ u32x4 lds_a[2][NBMAX * 128];  // 2 stages x 16 dimensions x 256 centroids x {high, low}: 2 x 16 KB
@@ -1135,6 +1232,8 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
         lds_barrier();
     }
     x2 += __shfl_xor(x2, 32);  // both halves' shares of ||x - mu||^2
+    const float nx = COS ? __builtin_amdgcn_sqrtf(x2) : 0.0f;
+    if constexpr (COS) x2 = 2.01f * nx;
     // the three smallest scores of the row, the index in the low 8 bits (one v_and_or per score; the
     // tag leaves out the lane half, bit 2, so it is the same in every lane: a scalar operand)
     int m1 = 0x7f800000, m2 = 0x7f800000, m3 = 0x7f800000;
@@ -1165,8 +1264,8 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
         }
         const float s1 = __int_as_float(m1), s2 = __int_as_float(m2), s3 = __int_as_float(m3);
         if (valid) {
-            const float bound = x2 + mc2;
-            const bool finite = (bound < 1e29f) && (s1 < 1e29f);  // false for NaN
+            const float bound = (COS ? nx : x2) + mc2;
+            const bool finite = (bound < (COS ? 1e15f : 1e29f)) && (!COS || bound > 1e-15f) && (s1 < 1e29f);  // false for NaN
             const float slack = tb.kappa * bound;
             // the smallest exact distance is the best-scored centroid's when the second score is
             // further away than the error bound ...

@@ -208,8 +208,8 @@ int32_t launch_mfma(vq_ctx *ctx, const vq::AssignArgs &a, bool tables_ready, hip
     MfmaTabPtrs t;
     VQ_TRY(mfma_tab_ptrs(ctx, a.m, a.k, t));
     if (!tables_ready && !own)
-        hipLaunchKernelGGL(vq::k_mfma_bf_prep, dim3(a.m), dim3(256), 0, ctx->stream, a.cb, a.m, a.k, nb, t.atab,
-                           t.maxc2, t.mu, t.stat, t.stat_next);
+        hipLaunchKernelGGL(vq::k_mfma_bf_prep<METRIC == vq::M_COS>, dim3(a.m), dim3(256), 0, ctx->stream, a.cb, a.m, a.k,
+                           nb, t.atab, t.maxc2, t.mu, t.stat, t.stat_next);
     vq::MfmaBfTables tb{(const vq::u32x4 *)t.atab, t.maxc2, t.mu, t.stat, nb, t.stat_next};
     auto pick = [&](auto SGc, auto FULLc) {
         constexpr int SGv = decltype(SGc)::value;
@@ -295,18 +295,26 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     uint2 *pairs = (uint2 *)(list + ((n_pairs + 1) & ~(size_t)1));  // 8-byte aligned
     float2 *norms = (float2 *)(mu + (size_t)a.m * sd);  // sd is a multiple of 8: 8-byte aligned
     int *shifted = (int *)(norms + (size_t)a.m * nsl);
-    hipLaunchKernelGGL(vq::k_block_centres, dim3(a.m, nsl), dim3(256), 0, ctx->stream, a.cb, a.k, sd, mu, norms);
-    hipLaunchKernelGGL(vq::k_mfma_wide_bf_prep, dim3(a.m, nb), dim3(256), 0, ctx->stream, a.cb, mu, norms, shifted,
-                       a.m, a.k, nb, sd,
-                       (vq::u32x4 *)atab, c2perm, maxc2, count);
+    constexpr bool COS = METRIC == vq::M_COS;
+    if (!COS)
+        hipLaunchKernelGGL(vq::k_block_centres, dim3(a.m, nsl), dim3(256), 0, ctx->stream, a.cb, a.k, sd, mu, norms);
+    hipLaunchKernelGGL(vq::k_mfma_wide_bf_prep<COS>, dim3(a.m, nb), dim3(256), 0, ctx->stream, a.cb, mu, norms, shifted,
+                       a.m, a.k, nb, sd, (vq::u32x4 *)atab, c2perm, maxc2, count, a.cnorm);
     // two candidates, each: operand split 3 * 2^-16, fp32 accumulation (34 per 8 dimensions + 16)
     // * 2^-24 (an upper bound), rounding of the differences from the centre 2^-22
-    const float kappa = 2.0f * (3.0f * 1.52587890625e-05f + (34.0f * nkc + 16.0f + 4.0f) * 5.9604644775390625e-08f);
+    // cosine, in units of |x|: the split of an operand twice as long, 2^-22 for the division by the norm,
+    // partial sums up to 4.2 |x|, the reference's own rounding 2 (sub_dim + 6) * 2^-24
+    const float u24 = 5.9604644775390625e-08f, split = 3.0f * 1.52587890625e-05f;
+    const float kappa = 2.0f * (COS ? 2.0f * split + (8.0f + 4.2f * (34.0f * nkc + 16.0f) + 2.0f * (sd + 6.0f)) * u24
+                                    : split + (34.0f * nkc + 16.0f + 4.0f) * u24);
     vq::MfmaWideBfTables tb{(const vq::u32x4 *)atab, c2perm, maxc2, mu, shifted, list, count, pairs, nb, sd, kappa};
     {
         ProfSpan sp(ctx, VQ_PROF_ASSIGN_KERNEL);
 #define WIDE(NB)                                                                                             \
-    if (a.pend_cb)                                                                                           \
+    if (COS)                                                                                                 \
+        hipLaunchKernelGGL((vq::k_assign_mfma_wide_bf<false, NB, false, true>), dim3(cdiv(a.n, 128), (unsigned)a.m), \
+                           dim3(256), 0, ctx->stream, a, tb);                                                \
+    else if (a.pend_cb)                                                                                           \
         hipLaunchKernelGGL((vq::k_assign_mfma_wide_bf<LBG, NB, true>), dim3(cdiv(a.n, 128), (unsigned)a.m),    \
                            dim3(256), 0, ctx->stream, a, tb);                                                \
     else                                                                                                     \
@@ -334,7 +342,7 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
 template <int METRIC, bool LBG>
 bool mfma_wide_applicable(const vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     if (ctx->assign_path == 1 || ctx->no_alloc) return false;  // its lists grow with n: not for a fixed scratch
-    if (METRIC != vq::M_SQ && METRIC != vq::M_EUCLID) return false;
+    if (METRIC != vq::M_SQ && METRIC != vq::M_EUCLID && !(METRIC == vq::M_COS && !LBG)) return false;
     if (sd < 16 || sd % 8 != 0 || a.k > 256 || a.m > 65535) return false;
     // float4 row and centroid loads; the rows of a workgroup and the operand table within 32-bit byte offsets
     if (a.ld % 4 != 0 || ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.cb)) & 15) != 0)
@@ -346,26 +354,37 @@ bool mfma_wide_applicable(const vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
 template <int METRIC, bool LBG>
 bool mfma_applicable(const vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     if (ctx->assign_path == 1) return false;
-    if (METRIC != vq::M_SQ && METRIC != vq::M_EUCLID) return false;
+    if (METRIC != vq::M_SQ && METRIC != vq::M_EUCLID && !(METRIC == vq::M_COS && !LBG)) return false;
     if (sd != 8 || (reinterpret_cast<uintptr_t>(a.cb) & 15) != 0) return false;  // float4 centroid loads
     // the kernel addresses the rows of a wave's run (at most 288 of them) with 32-bit offsets
     if (a.ld > (1 << 20) || a.m > (1 << 16)) return false;
     return a.k <= 256;
 }
 
-// The width to pad every column block to so that the matrix-core kernels take the shape (squared L2
-// and Euclidean; 0: they take it as it is, or padding does not pay).  Below 8 floats the padded block
-// costs what a block of 8 costs, about 290 vector instructions per 32 rows and 256 centroids, where the
-// vector-ALU kernel needs 3 sub_dim + 3 per row and centroid: 3-10 times as many, and 50 times as
-// long where there is no kernel for the width (10 floats, 60,007 rows x 10 blocks, k = 200: 3.94 ms
-// per pass).  Under 32 centroids half of a tile of the matrix kernels is padding: those stay.
-int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd) {
-    if (ctx->assign_path == 1 || ctx->no_alloc || (metric != VQ_SQEUCLIDEAN && metric != VQ_EUCLIDEAN)) return 0;
-    if (a.k < 32 || a.k > vq::kMaxK || a.m > 65535) return 0;
+// The width to pad every column block to so that the matrix-core kernels take the shape (squared L2,
+// Euclidean, cosine; 0: they take it as it is, or padding does not pay).  fit: for the passes of a fit,
+// which pads its rows once and whose update then streams blocks of 8 as well.
+// Widths without a register kernel always gain (10 floats, 60,007 rows x 10 blocks, k = 200: 3.94 ms per
+// pass on k_assign_dyn).  k_assign_static does 3 sd + 1 vector instructions per row and centroid (cosine:
+// about 2 sd + 26), the padded kernels about 600 per row and block and half the bytes more to read; the
+// lines below are where the two took the same time at 20,000-600,000 rows, 12 and 25 blocks.  One float
+// per block leaves most rows to the exact path of the matrix-core kernels: never.
+int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bool fit) {
+    if (ctx->assign_path == 1 || ctx->no_alloc || metric < VQ_SQEUCLIDEAN || metric > VQ_COSINE) return 0;
+    if (sd == 1 || a.k < 32 || a.k > vq::kMaxK || a.m > 65535) return 0;
     if (mfma_applicable<vq::M_SQ, true>(ctx, a, sd) || mfma_wide_applicable<vq::M_SQ, true>(ctx, a, sd)) return 0;
     const int sdp = (sd + 7) / 8 * 8;
     // the limits of those kernels
     if ((int64_t)a.m * sdp > (1 << 20) || sdp > (1 << 16) || a.n * a.m >= (1LL << 32)) return 0;
+    const bool has_static = (sd <= 6 || sd == 12 || sd == 16 || sd == 32) && ((size_t)a.k * (sd + 1)) * sizeof(float) <= 64 * 1024;
+    if (has_static) {
+        const int cost = a.k * (metric == VQ_COSINE ? 2 * sd + 26 : 3 * sd + 1);
+        if (metric == VQ_COSINE ? cost < (sd < 8 ? 1500 : 3500)
+            : sd > 8            ? cost < (fit ? 4700 : 3500)
+            : fit               ? a.k < 40
+                                : sd == 2 || cost < 1600 || (a.m % 4 != 0 && (cost - 1600) * (double)(a.n * a.m) < 5e8))
+            return 0;
+    }
     return sdp;
 }
 
@@ -383,6 +402,12 @@ int32_t launch_assign(vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, 
         return launch_mfma<vq::M_SQ, LBG>(ctx, a, tables_ready, started, done);
     if (metric == VQ_EUCLIDEAN && mfma_applicable<vq::M_EUCLID, LBG>(ctx, a, sd))
         return launch_mfma<vq::M_EUCLID, LBG>(ctx, a, tables_ready, started, done);
+    if constexpr (!LBG)
+        if (metric == VQ_COSINE && mfma_applicable<vq::M_COS, false>(ctx, a, sd))
+            return launch_mfma<vq::M_COS, false>(ctx, a, tables_ready, started, done);
+    if constexpr (!LBG)
+        if (metric == VQ_COSINE && mfma_wide_applicable<vq::M_COS, false>(ctx, a, sd))
+            return launch_mfma_wide<vq::M_COS, false>(ctx, a, sd);
     if (metric == VQ_SQEUCLIDEAN && mfma_wide_applicable<vq::M_SQ, LBG>(ctx, a, sd))
         return launch_mfma_wide<vq::M_SQ, LBG>(ctx, a, sd);
     if (metric == VQ_EUCLIDEAN && mfma_wide_applicable<vq::M_EUCLID, LBG>(ctx, a, sd))
@@ -660,7 +685,20 @@ int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, i
         a.pend_src = pend->src;
         a.pend_src_ld = pend->src_ld;
     }
-    if (metric == VQ_COSINE) {
+    // the 8-float matrix-core kernel has the chosen centroid's exact distance at hand
+    const bool mfma8 = metric != VQ_MANHATTAN && mfma_applicable<vq::M_SQ, false>(ctx, a, sd);
+    if (d_dist && dist_written && mfma8) {
+        a.dist = d_dist;
+        *dist_written = true;
+    }
+    // ... and the chosen centroid in LDS
+    if (d_out16 && out_written && (reinterpret_cast<uintptr_t>(d_out16) & 15) == 0 && mfma8) {
+        a.out16 = d_out16;
+        *out_written = true;
+    }
+    ProfSpan sp(ctx, VQ_PROF_ENCODE);
+    const int sdp = pend ? 0 : pad_width(ctx, metric, a, sd, false);
+    if (metric == VQ_COSINE && !mfma8 && sdp != 8) {  // the 8-float kernel makes the norms itself
         float *cnorm = (float *)(ctx->static_scratch + kNoAllocNormOff);
         if (!ctx->no_alloc) {
             VQ_TRY(ensure(ctx, ctx->cnorm, sizeof(float) * (size_t)m * k));
@@ -670,22 +708,6 @@ int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, i
                            ctx->stream, d_codebooks, (int64_t)m * k, sd, cnorm);
         a.cnorm = cnorm;
     }
-    // the 8-float matrix-core kernel has the chosen centroid's exact distance at hand
-    if (d_dist && dist_written &&
-        ((metric == VQ_SQEUCLIDEAN && mfma_applicable<vq::M_SQ, false>(ctx, a, sd)) ||
-         (metric == VQ_EUCLIDEAN && mfma_applicable<vq::M_EUCLID, false>(ctx, a, sd)))) {
-        a.dist = d_dist;
-        *dist_written = true;
-    }
-    // ... and the chosen centroid in LDS
-    if (d_out16 && out_written && (reinterpret_cast<uintptr_t>(d_out16) & 15) == 0 &&
-        ((metric == VQ_SQEUCLIDEAN && mfma_applicable<vq::M_SQ, false>(ctx, a, sd)) ||
-         (metric == VQ_EUCLIDEAN && mfma_applicable<vq::M_EUCLID, false>(ctx, a, sd)))) {
-        a.out16 = d_out16;
-        *out_written = true;
-    }
-    ProfSpan sp(ctx, VQ_PROF_ENCODE);
-    const int sdp = pend ? 0 : pad_width(ctx, metric, a, sd);
     if (!sdp) return launch_assign<false>(ctx, metric, a, sd);
     // padded a slice of rows at a time: the copy is read back from the memory-side cache (256 MB)
     // and the workspace stays small whatever n is
@@ -1087,7 +1109,7 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
     shape.m = m;
     shape.k = k;
     shape.cb = d_codebooks;
-    const int sdp = max_iters > 0 ? pad_width(ctx, VQ_SQEUCLIDEAN, shape, sd) : 0;
+    const int sdp = max_iters > 0 ? pad_width(ctx, VQ_SQEUCLIDEAN, shape, sd, true) : 0;
     if (sdp && (int64_t)k * cdiv(n, vq::kPartRows) * sdp <= (1LL << 31)) {
         // the rows padded once for all passes of the fit (a shape too large for a second copy of its
         // rows trains on the rows as they are)
