@@ -20,8 +20,8 @@ def ctx():
 
 # n, m, sub_dim, k, extra columns of the row buffer
 CASES = [(33, 1, 1, 32, 0), (300, 5, 2, 40, 0), (1025, 4, 3, 256, 0), (4097, 8, 4, 64, 3), (129, 4, 7, 33, 1),
-         (2000, 3, 9, 200, 0), (6007, 10, 10, 200, 0), (700, 2, 15, 32, 5), (513, 1, 25, 256, 0), (400, 1, 100, 50, 0),
-         (1500, 2, 16, 96, 1), (260, 1, 300, 256, 0)]
+         (2000, 3, 9, 200, 0), (6007, 10, 10, 200, 0), (700, 2, 15, 32, 5), (513, 1, 25, 256, 0), (400, 1, 100, 50, 0), (66_001, 5, 8, 33, 0),
+         (1500, 2, 16, 96, 1), (260, 1, 300, 256, 0), (70_000, 6, 3, 40, 0)]
 
 
 @pytest.mark.parametrize("n,m,sd,k,extra", CASES)

@@ -1137,7 +1137,7 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_large(LbgSmall st,
     }
 }
 
-// ---- streaming sums of the large clusters (sub_dim 8, 4 column blocks per 128-byte line) ------
+// ---- streaming sums of the large clusters (sub_dim 8, 4 column blocks per 128 bytes) -----------
 // One workgroup per (part, group of 4 column blocks); wave w of the group owns column block
 // 4g + w, so the four waves together consume whole 128-byte lines of the rows.  A wave walks
 // its part 64 rows at a time; a lane holds the 32-byte sub-vector of its row.  The rows of a
@@ -1149,13 +1149,16 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_large(LbgSmall st,
 // chunk (the barrier waits for nothing else: the prefetches stay in flight): each of them reads
 // a different 32-byte quarter of the same lines, and waves that drift apart by the length of
 // their prefetch queues find those lines gone from the compute unit's cache.
+// (m not a multiple of 4: the waves of the last group without a column block only keep the barriers.)
 static __global__ void __launch_bounds__(256) k_lbg_stream8(LbgState st, const float *__restrict__ x, int64_t n,
-                                                            int64_t ld) {
+                                                            int64_t ld, int m) {
     const int g = blockIdx.y, b = blockIdx.x;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int s = 4 * g + w;
     __shared__ float4 acc_lo[4][kMaxK], acc_hi[4][kMaxK];  // components 0-3 and 4-7 of every cluster
-    if (st.done[4 * g] && st.done[4 * g + 1] && st.done[4 * g + 2] && st.done[4 * g + 3]) return;
+    bool work = false;
+    for (int u = 0; u < 4; ++u) work = work || (4 * g + u < m && !st.done[4 * g + u]);
+    if (!work) return;
     float4 *alo = acc_lo[w], *ahi = acc_hi[w];
     for (int i = lane; i < kMaxK; i += 64) {
         alo[i] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1168,7 +1171,7 @@ static __global__ void __launch_bounds__(256) k_lbg_stream8(LbgState st, const f
     const int rows = (int)(hi - lo);
     const int nchunks = (rows + 63) / 64, rows_last = rows - 64 * (nchunks - 1);
     const int nsteps = (nchunks + PF - 1) / PF * PF;  // chunk steps of the loop below, one barrier each
-    if (st.done[s]) {  // this wave's column block has stopped: it only keeps the others' barriers company
+    if (s >= m || st.done[s]) {  // this wave's column block has stopped: it only keeps the others' barriers company
         for (int c = 0; c < nsteps; ++c) __builtin_amdgcn_s_barrier();
         return;
     }

@@ -1271,8 +1271,10 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
 
     const int nparts = (int)((n + vq::kPartRows - 1) / vq::kPartRows);
     const int nseg = (nparts + vq::kScanSeg - 1) / vq::kScanSeg;
-    // streaming sums of the large clusters: 32-byte sub-vectors, 4 per 128-byte line, aligned rows
-    const bool stream = sd == 8 && m % 4 == 0 && ld % 4 == 0 && ld <= (1 << 20) &&
+    // streaming sums of the large clusters: 32-byte sub-vectors, 4 to a workgroup, aligned rows (a last
+    // group with idle waves pays from some 60,000 rows on: 25 blocks, k = 16: 20,000 rows 117 us per
+    // iteration without, 150 with; 200,000 rows 283 and 223)
+    const bool stream = sd == 8 && (m % 4 == 0 || nparts >= 16) && ld % 4 == 0 && ld <= (1 << 20) &&
                         (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;  // (32-bit lane offsets inside a chunk)
     const int64_t leaf_cap64 = stream ? (int64_t)k : (int64_t)k * nparts;
     if (leaf_cap64 * sd > (1LL << 31)) return fail(ctx, VQ_ERR_UNSUPPORTED, "n * k * sub_dim too large");
@@ -1382,7 +1384,7 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
                 done = ctx->ev_fork;
             }
             VQ_HIP(ctx, hipStreamWaitEvent(gs, done, 0));
-            hipLaunchKernelGGL(vq::k_lbg_stream8, dim3(nparts, m / 4), dim3(256), 0, st, S, d_x, n, ld);
+            hipLaunchKernelGGL(vq::k_lbg_stream8, dim3(nparts, cdiv(m, 4)), dim3(256), 0, st, S, d_x, n, ld, m);
         }
         hipLaunchKernelGGL(vq::k_lbg_hist, dim3(nparts, m), dim3(64), 0, gs, S, n);
         hipLaunchKernelGGL(vq::k_lbg_scan_seg, dim3(nseg, m), dim3(256), 0, gs, S);
@@ -1396,7 +1398,9 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
             // leaves are the few clusters of up to 1024 members beside the streaming kernel
             hipLaunchKernelGGL(vq::k_lbg_leafsum_wg, dim3(leaf_cap, m), dim3(256), 0, gs, S, d_x, n, ld, sd,
                                shift);
-        } else if (sd <= 32 && (1 << shift) == sd) {
+        } else if (sd <= 32 && (1 << shift) == sd && (int64_t)leaf_cap * sd * m < (1 << 20)) {
+            // few leaves: a wave each; from a million (leaf, component) pairs on a lane each fills the GPU
+            // (600,000 rows in 12 blocks of 16, k = 256, 16 rows per leaf: 1.1 against 0.25 ms)
             hipLaunchKernelGGL(vq::k_lbg_leafsum_wave, dim3(cdiv(leaf_cap, 4), m), dim3(256), 0, gs, S, d_x, n,
                                ld, sd, shift);
         } else {
