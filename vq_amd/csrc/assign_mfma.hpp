@@ -855,15 +855,24 @@ namespace vq {
 // added to the scores before the selection.  The A operands of 16 dimensions (16 KB for 256
 // centroids) are staged in LDS once per workgroup, double-buffered; the next A operands are
 // fetched one stage ahead, the row two.
-// Error of a score: 3 * 2^-16 (split, as above) + (34 * sd/8 + 16) * 2^-24 (fp32 accumulation, an
-// upper bound: at most 17 additions per instruction, 1.5 instructions per 8 dimensions, and the
-// final sum) + 2^-22 (rounding of x - mu and c - mu), per unit of ||x - mu||^2 + ||c - mu||^2;
-// twice that for two candidates.
+// What decides (x and c relative to the centre, t = kWideT): a score is off by no more than
+//   A ||c||^2 + (S + A) 2 ||x|| ||c||,  S = 3 * 2^-16 (split, as above),  A = (27 sd/8 + 28) * 2^-24
+// (fp32 accumulation, an upper bound: at most 17 additions per instruction, 1.5 instructions per 8
+// dimensions, the sum of ||c||^2, the rounding of x - mu and c - mu), and 2 ||x|| ||c|| <= t ||x||^2 +
+// ||c||^2 / t.  The share of the row is the same for every centroid; the share of the centroid, pen[j],
+// is taken off its score before the selection.  A centroid whose lowered score is clear of the best one
+// by both rows' shares, 2 pen[best], the tag (2^-14 of the score) and the reference's own rounding
+// (2 (sd + 16) * 2^-24 of the distance) has lost.  A bound from the LARGEST ||c|| of the block listed 7-20 %
+// of the rows of a late residual stage (up to 7 % of them for all centroids, 0.65 ms per pass at
+// 1M x 256, 194 us on average, now 15-25; the fit of 8 stages 80 -> 65 ms): there most rows choose between a few centroids of small norm beside many of large norm.
+// t is a compromise: the undecided share is flat between 0.25 and 0.7 (it doubles outside).
+constexpr float kWideT = 0.35f;
 constexpr int kWideCentreMax = 2048;  // widest column block whose centre is staged in LDS
 
 struct MfmaWideBfTables {
     const u32x4 *atab;     // [m][ceil(sd/16)][nb][2][64]  ah, then al, of the lane's eight dimensions
-    const float *c2perm;   // [m][nb][2][16]
+    const float *c2perm;   // [m][nb][2][16]  ||c - mu||^2 less the centroid's share of the error bound
+    const float *pen;      // [m][nb * 32]  that share
     const float *blockmax; // [m][nb]  largest ||c - mu||^2 per block of 32 centroids (NaN if any is NaN)
     const float *mu;       // [m][sd]  centre of every column block: mean of its centroids
     const int *shifted;    // [m]  0: the centre is not used
@@ -872,7 +881,10 @@ struct MfmaWideBfTables {
     uint2 *pairs;          // undecided pairs with only two candidates: {row * m + s, c1 | c2 << 8}
     int nb;
     int sd;
-    float kappa;           // error-bound coefficient on (||x||^2 + max ||c||^2)
+    float kappa;           // COS: error-bound coefficient on ||x||
+    float row_share;       // else: the rows' share of the bound of two candidates, per unit of ||x - mu||^2,
+    float lift;            // what is added to the scores so that they are positive, likewise,
+    float rel;             // and the tag and the reference's rounding, per unit of the score
 };
 
 // One workgroup per (column block s, block b of 32 centroids): thread (i, g) = (tid % 32, tid / 32)
@@ -940,6 +952,7 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
                                                                   float *__restrict__ c2perm,
                                                                   float *__restrict__ blockmax,
                                                                   uint32_t *__restrict__ list_count,
+                                                                  float *__restrict__ pen, float pen_c2,
                                                                   const float *__restrict__ cnorm = nullptr) {
     const int s = blockIdx.x, b = blockIdx.y;
     const int i = threadIdx.x & 31, g = threadIdx.x >> 5;
@@ -1005,11 +1018,13 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
         for (int q = 0; q < 8; ++q) c2 = c2 + part[q][i];
         if constexpr (COS) c2 = nc == 0.0f || (nc >= 1e-15f && nc <= 1e15f) ? 0.0f : __builtin_nanf("");
         float mx = c2;
-        if constexpr (COS) c2 = 0.0f;
+        const float share = COS ? 0.0f : pen_c2 * c2;
+        c2 = COS ? 0.0f : c2 - share;
         if (j >= k) {
             c2 = kPadScore;
             mx = 0.0f;
         }
+        pen[((size_t)s * nb + b) * 32 + i] = share;
         const int hh = (i / 4) % 2, v = (i / 8) * 4 + i % 4;
         c2perm[(((size_t)s * nb + b) * 2 + hh) * 16 + v] = c2;
 #pragma unroll
@@ -1042,6 +1057,7 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
     constexpr int NBMAX = 8;
     __shared__ u32x4 lds_a[2][NBMAX * 128];  // 2 stages x 16 dimensions x 256 centroids x {high, low}: 2 x 16 KB
     __shared__ float lds_c2[NBMAX * 32];
+    __shared__ float lds_pen[COS ? 1 : NBMAX * 32];
     __shared__ float lds_mu[kWideCentreMax];
     __shared__ uint32_t wg_list[128];
     __shared__ uint2 wg_pairs[128];
@@ -1057,6 +1073,8 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
     const u32x4 *ag = tb.atab + (size_t)s * npair * nb * 128;
     const int pair16 = nb * 128;  // 16-byte pieces per 16 dimensions
     for (int i = threadIdx.x; i < nb * 32; i += 256) lds_c2[i] = tb.c2perm[(size_t)s * nb * 32 + i];
+    if constexpr (!COS)
+        for (int i = threadIdx.x; i < nb * 32; i += 256) lds_pen[i] = tb.pen[(size_t)s * nb * 32 + i];
     for (int i = threadIdx.x; i < pair16; i += 256) lds_a[0][i] = ag[i];
     if (threadIdx.x == 0) {
         wg_count = 0;
@@ -1103,8 +1121,9 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
     const uint32_t xlane = valid ? 4u * (uint32_t)(wave * 32 + r) * (uint32_t)a.ld : 0u;
     auto row_piece = [&](int d) { return *reinterpret_cast<const float4 *>(xwg + (xlane + 4u * (uint32_t)d)); };
     const bool shifted = tb.shifted[s] != 0;  // uniform
-    // the accumulators start at ||c - mu||^2; ||x - mu||^2, the same in every score of a row, is
-    // summed on the side and added before the selection
+    // the accumulators start at ||c - mu||^2 less the centroid's share of the bound; ||x - mu||^2, the same
+    // in every score of a row, is summed on the side and added, a little enlarged, before the selection
+    // (a score is then positive, and its bits order as an integer)
     floatx16 acc[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -1233,7 +1252,7 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
     }
     x2 += __shfl_xor(x2, 32);  // both halves' shares of ||x - mu||^2
     const float nx = COS ? __builtin_amdgcn_sqrtf(x2) : 0.0f;
-    if constexpr (COS) x2 = 2.01f * nx;
+    const float lifted = COS ? 2.01f * nx : tb.lift * x2;
     // the three smallest scores of the row, the index in the low 8 bits (one v_and_or per score; the
     // tag leaves out the lane half, bit 2, so it is the same in every lane: a scalar operand)
     int m1 = 0x7f800000, m2 = 0x7f800000, m3 = 0x7f800000;
@@ -1245,7 +1264,7 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
             int key[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                key[u] = pack_tag(acc[b][v + u] + x2, keep, (uint32_t)(32 * b + 8 * (v / 4) + u));
+                key[u] = pack_tag(acc[b][v + u] + lifted, keep, (uint32_t)(32 * b + 8 * (v / 4) + u));
             top3_push4(m1, m2, m3, key[0], key[1], key[2], key[3]);
         }
     }
@@ -1266,12 +1285,14 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
         if (valid) {
             const float bound = (COS ? nx : x2) + mc2;
             const bool finite = (bound < (COS ? 1e15f : 1e29f)) && (!COS || bound > 1e-15f) && (s1 < 1e29f);  // false for NaN
-            const float slack = tb.kappa * bound;
+            // (1e-32: what products below the smallest normal number can lose)
+            const float slack = COS ? tb.kappa * bound : tb.row_share * x2 + 2.1f * lds_pen[COS ? 0 : i1] + 1e-32f;
+            const float rel = COS ? 6.103515625e-05f : tb.rel;
             // the smallest exact distance is the best-scored centroid's when the second score is
             // further away than the error bound ...
-            const bool sure = finite && (s2 - s1) > 6.103515625e-05f * fabsf(s2) + slack;
+            const bool sure = finite && (s2 - s1) > rel * fabsf(s2) + slack;
             // ... and one of the two best-scored centroids' when the third score is
-            const bool two = finite && (s2 < 1e29f) && (s3 - s1) > 6.103515625e-05f * fabsf(s3) + slack;
+            const bool two = finite && (s2 < 1e29f) && (s3 - s1) > rel * fabsf(s3) + slack;
             if (sure) {
                 const uint8_t code = (uint8_t)i1;
                 if constexpr (LBG) {

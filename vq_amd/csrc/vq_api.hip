@@ -282,13 +282,14 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     const int nb = (a.k + 31) / 32, nkc = sd / 8, nsl = (sd + 31) / 32;
     // A operands: 2 x 64 lanes x 16 bytes per (s, 16 dimensions, block of 32 centroids)
     const size_t n_atab = (size_t)a.m * ((sd + 15) / 16) * nb * 128 * 4, n_c2 = (size_t)a.m * nb * 32;  // floats
-    VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + n_c2 + (size_t)a.m * nb + (size_t)a.m * sd + a.m + 2 * (size_t)a.m * nsl + 8) + 64));
+    VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + 2 * n_c2 + (size_t)a.m * nb + (size_t)a.m * sd + a.m + 2 * (size_t)a.m * nsl + 8) + 64));
     // header (two counts), the list for the all-centroid check, the list for the two-candidate check
     const size_t n_pairs = (size_t)a.n * a.m;
     VQ_TRY(ensure(ctx, ctx->mfma_list, sizeof(uint32_t) * (4 + ((n_pairs + 1) & ~(size_t)1) + 2 * n_pairs)));
     float *atab = (float *)ctx->mfma_tab.p;
     float *c2perm = atab + n_atab;
-    float *maxc2 = c2perm + n_c2;  // per block of 32 centroids
+    float *pen = c2perm + n_c2;
+    float *maxc2 = pen + n_c2;  // per block of 32 centroids
     float *mu = maxc2 + (((size_t)a.m * nb + 3) & ~(size_t)3);  // 16-byte aligned: read as float4
     uint32_t *count = (uint32_t *)ctx->mfma_list.p;
     uint32_t *list = count + 4;
@@ -298,16 +299,19 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     constexpr bool COS = METRIC == vq::M_COS;
     if (!COS)
         hipLaunchKernelGGL(vq::k_block_centres, dim3(a.m, nsl), dim3(256), 0, ctx->stream, a.cb, a.k, sd, mu, norms);
+    // squared L2, Euclidean: see kWideT.  2.1 instead of 2: the roundings of x2, pen and the bound itself
+    // cosine, in units of |x|, two candidates: the split of an operand twice as long, 2^-22 for the division by
+    // the norm, fp32 accumulation (34 per 8 dimensions + 16) * 2^-24 of partial sums up to 4.2 |x|, the
+    // reference's own rounding 2 (sub_dim + 6) * 2^-24
+    const float u24 = 5.9604644775390625e-08f, split = 3.0f * 1.52587890625e-05f, t = vq::kWideT;
+    const float kappa = 2.0f * (2.0f * split + (8.0f + 4.2f * (34.0f * nkc + 16.0f) + 2.0f * (sd + 6.0f)) * u24);
+    const float acc_err = (27.0f * nkc + 28.0f) * u24;
+    const float pen_c2 = acc_err + (split + acc_err) / t;
+    const float lift = 1.001f + 8.0f * pen_c2, rel = 6.103515625e-05f + 2.0f * (sd + 16.0f) * u24;
     hipLaunchKernelGGL(vq::k_mfma_wide_bf_prep<COS>, dim3(a.m, nb), dim3(256), 0, ctx->stream, a.cb, mu, norms, shifted,
-                       a.m, a.k, nb, sd, (vq::u32x4 *)atab, c2perm, maxc2, count, a.cnorm);
-    // two candidates, each: operand split 3 * 2^-16, fp32 accumulation (34 per 8 dimensions + 16)
-    // * 2^-24 (an upper bound), rounding of the differences from the centre 2^-22
-    // cosine, in units of |x|: the split of an operand twice as long, 2^-22 for the division by the norm,
-    // partial sums up to 4.2 |x|, the reference's own rounding 2 (sub_dim + 6) * 2^-24
-    const float u24 = 5.9604644775390625e-08f, split = 3.0f * 1.52587890625e-05f;
-    const float kappa = 2.0f * (COS ? 2.0f * split + (8.0f + 4.2f * (34.0f * nkc + 16.0f) + 2.0f * (sd + 6.0f)) * u24
-                                    : split + (34.0f * nkc + 16.0f + 4.0f) * u24);
-    vq::MfmaWideBfTables tb{(const vq::u32x4 *)atab, c2perm, maxc2, mu, shifted, list, count, pairs, nb, sd, kappa};
+                       a.m, a.k, nb, sd, (vq::u32x4 *)atab, c2perm, maxc2, count, pen, pen_c2, a.cnorm);
+    vq::MfmaWideBfTables tb{(const vq::u32x4 *)atab, c2perm, pen, maxc2, mu, shifted, list, count, pairs, nb, sd,
+                            kappa, 2.1f * (split + acc_err) * t, lift, rel};
     {
         ProfSpan sp(ctx, VQ_PROF_ASSIGN_KERNEL);
 #define WIDE(NB)                                                                                             \
