@@ -33,6 +33,10 @@ def _case(kind, n, m, sd, k):
     elif kind == "spread":  # norms of rows and centroids over twelve decades
         x *= (10.0 ** rng.uniform(-6, 6, (n, 1, 1))).astype(F)
         cb *= (10.0 ** rng.uniform(-6, 6, (m, k, 1))).astype(F)
+    elif kind == "overflow":  # beside centroids of norm one, rows past the range of binary16 and far below it
+        x *= (10.0 ** rng.uniform(-9, 6, (n, 1, 1))).astype(F)
+        x[:, :, 1::3] *= F(1e-6)
+        cb[:, :, 2::3] *= F(1e-7)
     elif kind == "tiny":
         x, cb = x * F(1e-18), cb * F(1e-18)
         cb[:, 0] *= F(1e15)
@@ -46,10 +50,11 @@ def _case(kind, n, m, sd, k):
     return np.ascontiguousarray(x.reshape(n, m * sd)), cb
 
 
-@pytest.mark.parametrize("kind", ["normal", "collapsed", "near_ties", "grid", "spread", "tiny", "offset", "edges"])
+@pytest.mark.parametrize("kind", ["normal", "collapsed", "near_ties", "grid", "spread", "overflow", "tiny", "offset", "edges"])
 @pytest.mark.parametrize("metric", [O.SQEUCLIDEAN, O.EUCLIDEAN])
 @pytest.mark.parametrize("n,m,sd,k", [(1300, 3, 16, 256), (700, 2, 24, 33), (900, 1, 64, 200), (300, 2, 104, 256),
-                                      (1000, 1, 128, 100), (2049, 1, 256, 256), (130, 1, 264, 31), (200, 1, 1000, 256)])
+                                      (1000, 1, 128, 100), (2049, 1, 256, 256), (130, 1, 264, 31), (333, 1, 264, 61),
+                                      (200, 2, 72, 225), (200, 1, 1000, 256)])
 def test_wide_codes(ctx, n, m, sd, k, metric, kind):
     x, cb = _case(kind, n, m, sd, k)
     codes = ctx.empty((n, m), np.uint8)

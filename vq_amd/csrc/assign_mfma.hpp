@@ -867,15 +867,33 @@ namespace vq {
 // 1M x 256, 194 us on average, now 15-25; the fit of 8 stages 80 -> 65 ms): there most rows choose between a few centroids of small norm beside many of large norm.
 // t is a compromise: the undecided share is flat between 0.25 and 0.7 (it doubles outside).
 constexpr float kWideT = 0.35f;
+
+// HALF: one product of binary16 operands instead of three of bf16 parts.  Rows and centroids are scaled by
+// a power of two that brings the centroids' root mean square norm to 32 ... 64; what the rounding of a row
+// (dx = ||x - xh||, summed as it happens) and of a centroid (dc) can do is 2 dx ||c|| + 2 ||x|| dc, split
+// between the row and the centroid as above, with kWideRho the usual dx / ||x||:
+//   2 dx ||c|| <= dx^2 t / rho + ||c||^2 rho / t,   2 ||x|| dc <= ||x||^2 rho t + dc^2 / (rho t).
+// Three times as many rows are undecided (1-4 % of a residual stage instead of 0.3-1.5 %), a third of the matrix
+// instructions and half of the staged operands are left.  A value beyond the range of binary16 makes dx
+// infinite, and the row is listed; elements below its normal range count as if they were flushed.
+// The line lies where the matrix instructions outweigh the undecided rows (three parts -> one product,
+// encode of 400,000 rows): k = 256: sd = 32 311 -> 328 us (8 blocks), 48 199 -> 193, 64 239 -> 207 (4 blocks),
+// 128 110 -> 88, 256 203 -> 153 (1 block); k = 64: sd = 64 70 -> 74 (2 blocks), 128 65 -> 64; k = 32: sd = 256
+// 125 -> 117.
+constexpr float kWideRho = 2.0e-4f;
+inline bool wide_half(int sd, int nb) { return sd >= 64 && sd * nb >= 512; }
+using f16x8 = _Float16 __attribute__((ext_vector_type(8)));
 constexpr int kWideCentreMax = 2048;  // widest column block whose centre is staged in LDS
 
 struct MfmaWideBfTables {
     const u32x4 *atab;     // [m][ceil(sd/16)][nb][2][64]  ah, then al, of the lane's eight dimensions
+                           // (HALF: [m][ceil(sd/16)][nb][64])
     const float *c2perm;   // [m][nb][2][16]  ||c - mu||^2 less the centroid's share of the error bound
     const float *pen;      // [m][nb * 32]  that share
     const float *blockmax; // [m][nb]  largest ||c - mu||^2 per block of 32 centroids (NaN if any is NaN)
     const float *mu;       // [m][sd]  centre of every column block: mean of its centroids
     const int *shifted;    // [m]  0: the centre is not used
+    const float *sigma;    // [m]  HALF: the scale
     uint32_t *list;        // undecided pairs (row * m + s) for the exact kernel over all centroids
     uint32_t *list_count;  // [0] entries of list, [1] entries of pairs
     uint2 *pairs;          // undecided pairs with only two candidates: {row * m + s, c1 | c2 << 8}
@@ -883,6 +901,7 @@ struct MfmaWideBfTables {
     int sd;
     float kappa;           // COS: error-bound coefficient on ||x||
     float row_share;       // else: the rows' share of the bound of two candidates, per unit of ||x - mu||^2,
+    float dx_share;        // HALF: and per unit of dx^2,
     float lift;            // what is added to the scores so that they are positive, likewise,
     float rel;             // and the tag and the reference's rounding, per unit of the score
 };
@@ -943,7 +962,7 @@ static __global__ void __launch_bounds__(256) k_block_centres(const float *__res
 
 // COS: the operands of the centroids divided by their norms (cnorm), no centre, no ||c||^2; blockmax is 0,
 // or NaN where a norm is outside the range that the scores can decide (see cos_normalise).
-template <bool COS = false>
+template <bool COS = false, bool HALF = false>
 static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *__restrict__ cb,
                                                                   const float *__restrict__ mu,
                                                                   const float2 *__restrict__ norms,
@@ -953,12 +972,14 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
                                                                   float *__restrict__ blockmax,
                                                                   uint32_t *__restrict__ list_count,
                                                                   float *__restrict__ pen, float pen_c2,
+                                                                  float *__restrict__ sigma, float pen_dc,
                                                                   const float *__restrict__ cnorm = nullptr) {
     const int s = blockIdx.x, b = blockIdx.y;
     const int i = threadIdx.x & 31, g = threadIdx.x >> 5;
     const int j = b * 32 + i;
     const int npair = (sd + 15) / 16;
     __shared__ float part[8][32];
+    __shared__ float part_dc[8][32];
     // the same decision in every workgroup of the column block (same values, same order)
     float mm = 0.0f, cc = 0.0f;
     for (int y = 0; y < (COS ? 0 : (sd + 31) / 32); ++y) {
@@ -969,14 +990,23 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
     const float nc = COS ? cnorm[(size_t)s * k + (j < k ? j : 0)] : 1.0f;
     const float scale = nc == 0.0f ? 0.0f : -2.0f * (1.0f / nc);
     const bool on = !COS && mm > 0.25f * cc && mm < 1e30f && sd <= kWideCentreMax;  // false for NaN
-    if (b == 0 && threadIdx.x == 0) shifted[s] = on ? 1 : 0;
+    float sg = 1.0f;
+    if constexpr (HALF) {
+        // (1e-6: where mean ||c||^2 and ||mu||^2 cancel, any scale will do)
+        const float r2 = on ? fmaxf(cc - mm, 1e-6f * cc) : cc;
+        if (r2 > 1e-36f && r2 < 1e36f) sg = ldexpf(1.0f, 5 - (ilogbf(r2) >> 1));
+    }
+    if (b == 0 && threadIdx.x == 0) {
+        shifted[s] = on ? 1 : 0;
+        if constexpr (HALF) sigma[s] = sg;
+    }
     const float *c = cb + ((size_t)s * k + (j < k ? j : 0)) * sd;
-    float p = 0.0f;
+    float p = 0.0f, dcs = 0.0f;
     for (int pr = g; pr < npair; pr += 8) {
         // lane i + 32 h holds the dimensions 16 pr + 8 h .. + 7 (zeros past the block's width): 16
         // bytes of high parts, then, 64 entries on, 16 bytes of low parts, each the operand of a
         // matrix instruction as it lies in LDS
-        u32x4 *dst = atab + (((size_t)s * npair + pr) * nb + b) * 128;
+        u32x4 *dst = atab + (((size_t)s * npair + pr) * nb + b) * (HALF ? 64 : 128);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int d0 = 16 * pr + 8 * h;
@@ -991,6 +1021,21 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
             }
             float cv[8] = {v0.x - u0.x, v0.y - u0.y, v0.z - u0.z, v0.w - u0.w,
                            v1.x - u1.x, v1.y - u1.y, v1.z - u1.z, v1.w - u1.w};
+            if constexpr (HALF) {
+                f16x8 hv;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x = in ? cv[e] * sg : 0.0f;
+                    p = __builtin_fmaf(x, x, p);
+                    const float a = (j < k) ? -2.0f * x : 0.0f;
+                    hv[e] = (_Float16)a;
+                    if (fabsf((float)hv[e]) < 6.103515625e-05f) hv[e] = (_Float16)0.0f;
+                    const float d = a - (float)hv[e];
+                    dcs = __builtin_fmaf(d, d, dcs);
+                }
+                dst[32 * h + i] = __builtin_bit_cast(u32x4, hv);
+                continue;
+            }
             uint32_t hw[4], lw[4];  // packed pairs of the high and low parts
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
@@ -1011,14 +1056,21 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
         }
     }
     part[g][i] = p;
+    if constexpr (HALF) part_dc[g][i] = dcs;
     __syncthreads();
     if (g == 0) {
         float c2 = 0.0f;
 #pragma unroll
         for (int q = 0; q < 8; ++q) c2 = c2 + part[q][i];
+        dcs = 0.0f;
+        if constexpr (HALF) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) dcs = dcs + part_dc[q][i];
+            dcs *= 0.25f;  // (the operand is -2 c)
+        }
         if constexpr (COS) c2 = nc == 0.0f || (nc >= 1e-15f && nc <= 1e15f) ? 0.0f : __builtin_nanf("");
         float mx = c2;
-        const float share = COS ? 0.0f : pen_c2 * c2;
+        const float share = COS ? 0.0f : pen_c2 * c2 + (HALF ? pen_dc * dcs : 0.0f);
         c2 = COS ? 0.0f : c2 - share;
         if (j >= k) {
             c2 = kPadScore;
@@ -1052,7 +1104,7 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // through.  No other workgroup reads or writes these rows.
 // COS: cosine distance (see cos_normalise): the scores are P - 2 x.c/|c| with P = 2.01 |x|, the bound is in
 // units of |x|.
-template <bool LBG, int NB, bool PEND = false, bool COS = false>
+template <bool LBG, int NB, bool PEND = false, bool COS = false, bool HALF = false>
 __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, MfmaWideBfTables tb) {
     constexpr int NBMAX = 8;
     __shared__ u32x4 lds_a[2][NBMAX * 128];  // 2 stages x 16 dimensions x 256 centroids x {high, low}: 2 x 16 KB
@@ -1070,18 +1122,20 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
     const int r = lane & 31, h = lane >> 5;
     constexpr int nb = NB;
     const int sd = tb.sd, npair = (sd + 15) / 16;
-    const u32x4 *ag = tb.atab + (size_t)s * npair * nb * 128;
-    const int pair16 = nb * 128;  // 16-byte pieces per 16 dimensions
+    const u32x4 *ag = tb.atab + (size_t)s * npair * nb * (HALF ? 64 : 128);
+    const int pair16 = nb * 128;  // 16-byte pieces per 16 dimensions (HALF: per 32)
+    const int total16 = npair * nb * (HALF ? 64 : 128);
+    const float sg = HALF ? tb.sigma[s] : 1.0f;
     for (int i = threadIdx.x; i < nb * 32; i += 256) lds_c2[i] = tb.c2perm[(size_t)s * nb * 32 + i];
     if constexpr (!COS)
         for (int i = threadIdx.x; i < nb * 32; i += 256) lds_pen[i] = tb.pen[(size_t)s * nb * 32 + i];
-    for (int i = threadIdx.x; i < pair16; i += 256) lds_a[0][i] = ag[i];
+    for (int i = threadIdx.x; i < pair16; i += 256) lds_a[0][i] = ag[i < total16 ? i : total16 - 1];
     if (threadIdx.x == 0) {
         wg_count = 0;
         wg_pcount = 0;
     }
     if (tb.shifted[s] != 0)
-        for (int i = threadIdx.x; i < sd; i += 256) lds_mu[i] = tb.mu[(size_t)s * sd + i];
+        for (int i = threadIdx.x; i < sd; i += 256) lds_mu[i] = HALF ? -(tb.mu[(size_t)s * sd + i] * sg) : tb.mu[(size_t)s * sd + i];
     if constexpr (PEND) {
         const int64_t row0 = (int64_t)blockIdx.x * 128;
         const int nrows = a.n - row0 < 128 ? (int)(a.n - row0) : 128;
@@ -1134,12 +1188,109 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
     // every outstanding load at each use instead of counting them.
     // This half's 8 of the 16 dimensions of a stage: 16 pr + 8 h .. + 7.
     auto piece = [&](int pr) { return 16 * pr + 8 * h < sd ? 16 * pr + 8 * h : 0; };
+    float x2 = 0.0f, dx2 = 0.0f;
+    if constexpr (HALF) {
+        // A stage is 32 dimensions in two steps of 16: whole 128-byte lines of a row per stage, one barrier
+        // per 2 NB matrix instructions; a last step past the width is left out.
+        const int nst = (npair + 1) / 2;
+        auto fetch = [&](int st, float4(&p)[4]) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int d = piece(2 * st + q);
+                p[2 * q] = row_piece(d);
+                p[2 * q + 1] = row_piece(d + 4);
+            }
+        };
+        auto halves = [&](int st, const float4(&p)[4], f16x8(&b)[2]) {
+            const bool last = st == nst - 1 && (sd & 31) != 0;  // uniform
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                float xv[8] = {p[2 * q].x, p[2 * q].y, p[2 * q].z, p[2 * q].w,
+                               p[2 * q + 1].x, p[2 * q + 1].y, p[2 * q + 1].z, p[2 * q + 1].w};
+                if (shifted) {  // x sigma - mu sigma in one rounding
+                    const float *mp = lds_mu + piece(2 * st + q);
+                    const float4 m0 = *reinterpret_cast<const float4 *>(mp), m1 = *reinterpret_cast<const float4 *>(mp + 4);
+                    const float mv[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) xv[u] = __builtin_fmaf(xv[u], sg, mv[u]);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) xv[u] *= sg;
+                }
+                if (last) {
+                    if (16 * (2 * st + q) + 8 * h >= sd) {
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) xv[u] = 0.0f;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    b[q][u] = (_Float16)xv[u];
+                    const float d = __builtin_fmaf((float)b[q][u], -1.0f, xv[u]);
+                    x2 = __builtin_fmaf(xv[u], xv[u], x2);
+                    dx2 = __builtin_fmaf(d, d, dx2);
+                }
+            }
+        };
+        float4 xn[4], xf[4];
+        f16x8 b[2], bn[2];
+        fetch(0, xn);
+        fetch(1 < nst ? 1 : 0, xf);
+        halves(0, xn, b);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) xn[q] = xf[q];
+        fetch(2 < nst ? 2 : nst - 1, xf);
+        for (int st = 0; st < nst; ++st) {
+            const int cur = st & 1;
+            const bool more = st + 1 < nst;
+            u32x4 pre[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t i = (uint32_t)((st + 1) * pair16) + threadIdx.x + 256u * (uint32_t)q;
+                const uint32_t ic = i < (uint32_t)total16 ? i : (uint32_t)total16 - 1u;
+                pre[q] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(ag) + 16u * ic);
+            }
+            auto step = [&](int q, const f16x8 &bq) {
+#pragma unroll
+                for (int b0 = 0; b0 < NB; b0 += 4) {
+                    u32x4 ah[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (b0 + c < NB) ah[c] = lds_a[cur][(q * NB + b0 + c) * 64 + lane];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (b0 + c < NB)
+                            acc[b0 + c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, ah[c]), bq,
+                                                                                acc[b0 + c], 0, 0, 0);
+                }
+            };
+            step(0, b[0]);
+            if (more) {
+                // the next stage's row operands, behind the first matrix instructions of this stage
+                halves(st + 1, xn, bn);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) xn[q] = xf[q];
+                fetch(st + 3 < nst ? st + 3 : nst - 1, xf);
+            }
+            if (2 * st + 1 < npair) step(1, b[1]);
+            b[0] = bn[0];
+            b[1] = bn[1];
+            if (more) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int i = threadIdx.x + 256 * q;
+                    if (i < pair16) lds_a[cur ^ 1][i] = pre[q];
+                }
+            }
+            lds_barrier();
+        }
+        dx2 += __shfl_xor(dx2, 32);
+    } else {
     float4 xn0 = row_piece(piece(0));  // the next piece of the row
     float4 xn1 = row_piece(piece(0) + 4);
     const int second = npair > 1 ? 1 : 0;
     float4 xf0 = row_piece(piece(second));  // and the one after it
     float4 xf1 = row_piece(piece(second) + 4);
-    float x2 = 0.0f;
     // The row operands of a stage: this half's 8 dimensions relative to the centre, their share of
     // ||x - mu||^2, and their high and low bf16 parts.
     auto split = [&](int st, const float4 &p0, const float4 &p1, u32x4 &bh, u32x4 &bl) {
@@ -1180,7 +1331,6 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
     // The row operands of stage st + 1 are made while the matrix instructions of stage st run: a
     // matrix instruction holds back the vector instructions of the other waves of its SIMD, but
     // independent vector instructions of its own wave issue in its shadow.
-    const int total16 = npair * pair16;
     u32x4 bh, bl;
     split(0, xn0, xn1, bh, bl);
     xn0 = xf0;
@@ -1250,9 +1400,10 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
         }
         lds_barrier();
     }
+    }
     x2 += __shfl_xor(x2, 32);  // both halves' shares of ||x - mu||^2
     const float nx = COS ? __builtin_amdgcn_sqrtf(x2) : 0.0f;
-    const float lifted = COS ? 2.01f * nx : tb.lift * x2;
+    const float lifted = COS ? 2.01f * nx : HALF ? tb.lift * x2 + 1.0f : tb.lift * x2;
     // the three smallest scores of the row, the index in the low 8 bits (one v_and_or per score; the
     // tag leaves out the lane half, bit 2, so it is the same in every lane: a scalar operand)
     int m1 = 0x7f800000, m2 = 0x7f800000, m3 = 0x7f800000;
@@ -1286,7 +1437,8 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
             const float bound = (COS ? nx : x2) + mc2;
             const bool finite = (bound < (COS ? 1e15f : 1e29f)) && (!COS || bound > 1e-15f) && (s1 < 1e29f);  // false for NaN
             // (1e-32: what products below the smallest normal number can lose)
-            const float slack = COS ? tb.kappa * bound : tb.row_share * x2 + 2.1f * lds_pen[COS ? 0 : i1] + 1e-32f;
+            const float slack = COS ? tb.kappa * bound : tb.row_share * x2 + (HALF ? tb.dx_share * (dx2 + (float)sd * 0x1p-28f) : 0.0f) +
+                                          2.1f * lds_pen[COS ? 0 : i1] + 1e-32f;
             const float rel = COS ? 6.103515625e-05f : tb.rel;
             // the smallest exact distance is the best-scored centroid's when the second score is
             // further away than the error bound ...

@@ -282,7 +282,7 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     const int nb = (a.k + 31) / 32, nkc = sd / 8, nsl = (sd + 31) / 32;
     // A operands: 2 x 64 lanes x 16 bytes per (s, 16 dimensions, block of 32 centroids)
     const size_t n_atab = (size_t)a.m * ((sd + 15) / 16) * nb * 128 * 4, n_c2 = (size_t)a.m * nb * 32;  // floats
-    VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + 2 * n_c2 + (size_t)a.m * nb + (size_t)a.m * sd + a.m + 2 * (size_t)a.m * nsl + 8) + 64));
+    VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + 2 * n_c2 + (size_t)a.m * nb + (size_t)a.m * sd + 2 * a.m + 2 * (size_t)a.m * nsl + 8) + 64));
     // header (two counts), the list for the all-centroid check, the list for the two-candidate check
     const size_t n_pairs = (size_t)a.n * a.m;
     VQ_TRY(ensure(ctx, ctx->mfma_list, sizeof(uint32_t) * (4 + ((n_pairs + 1) & ~(size_t)1) + 2 * n_pairs)));
@@ -296,6 +296,7 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     uint2 *pairs = (uint2 *)(list + ((n_pairs + 1) & ~(size_t)1));  // 8-byte aligned
     float2 *norms = (float2 *)(mu + (size_t)a.m * sd);  // sd is a multiple of 8: 8-byte aligned
     int *shifted = (int *)(norms + (size_t)a.m * nsl);
+    float *sigma = (float *)(shifted + a.m);
     constexpr bool COS = METRIC == vq::M_COS;
     if (!COS)
         hipLaunchKernelGGL(vq::k_block_centres, dim3(a.m, nsl), dim3(256), 0, ctx->stream, a.cb, a.k, sd, mu, norms);
@@ -305,18 +306,37 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     // reference's own rounding 2 (sub_dim + 6) * 2^-24
     const float u24 = 5.9604644775390625e-08f, split = 3.0f * 1.52587890625e-05f, t = vq::kWideT;
     const float kappa = 2.0f * (2.0f * split + (8.0f + 4.2f * (34.0f * nkc + 16.0f) + 2.0f * (sd + 6.0f)) * u24);
-    const float acc_err = (27.0f * nkc + 28.0f) * u24;
-    const float pen_c2 = acc_err + (split + acc_err) / t;
-    const float lift = 1.001f + 8.0f * pen_c2, rel = 6.103515625e-05f + 2.0f * (sd + 16.0f) * u24;
-    hipLaunchKernelGGL(vq::k_mfma_wide_bf_prep<COS>, dim3(a.m, nb), dim3(256), 0, ctx->stream, a.cb, mu, norms, shifted,
-                       a.m, a.k, nb, sd, (vq::u32x4 *)atab, c2perm, maxc2, count, pen, pen_c2, a.cnorm);
-    vq::MfmaWideBfTables tb{(const vq::u32x4 *)atab, c2perm, pen, maxc2, mu, shifted, list, count, pairs, nb, sd,
-                            kappa, 2.1f * (split + acc_err) * t, lift, rel};
+    const bool half = !COS && vq::wide_half(sd, nb);
+    const float rho = vq::kWideRho;
+    // HALF: 17 additions per instruction, one instruction per 16 dimensions begun, and a rounding per dimension
+    const float acc_err = (half ? 10.0f * nkc + 26.0f : 27.0f * nkc + 28.0f) * u24;
+    const float cross = half ? acc_err + rho : split + acc_err;
+    const float pen_c2 = acc_err + cross / t, pen_dc = 1.0f / (rho * t);
+    // (HALF: dc is at most 2^-11 ||c||)
+    const float lift = 1.001f + 8.0f * (pen_c2 + (half ? 2.4e-7f * pen_dc : 0.0f));
+    const float rel = 6.103515625e-05f + 2.0f * (sd + 16.0f) * u24;
+    const void *prep = half ? (const void *)vq::k_mfma_wide_bf_prep<false, true> : (const void *)vq::k_mfma_wide_bf_prep<COS, false>;
+    {
+        vq::u32x4 *atab4 = (vq::u32x4 *)atab;
+        int m = a.m, k = a.k, nbv = nb, sdv = sd;
+        float pc = pen_c2, pd = pen_dc;
+        const float *cb = a.cb, *cnorm = a.cnorm;
+        void *args[] = {&cb, &mu, &norms, &shifted, &m, &k, &nbv, &sdv, &atab4, &c2perm, &maxc2, &count, &pen, &pc, &sigma, &pd, &cnorm};
+        VQ_HIP(ctx, hipLaunchKernel(prep, dim3(a.m, nb), dim3(256), args, 0, ctx->stream));
+    }
+    vq::MfmaWideBfTables tb{(const vq::u32x4 *)atab, c2perm, pen, maxc2, mu, shifted, sigma, list, count, pairs, nb, sd,
+                            kappa, 2.1f * cross * t, 2.1f * t / rho, lift, rel};
     {
         ProfSpan sp(ctx, VQ_PROF_ASSIGN_KERNEL);
 #define WIDE(NB)                                                                                             \
     if (COS)                                                                                                 \
         hipLaunchKernelGGL((vq::k_assign_mfma_wide_bf<false, NB, false, true>), dim3(cdiv(a.n, 128), (unsigned)a.m), \
+                           dim3(256), 0, ctx->stream, a, tb);                                                \
+    else if (half && a.pend_cb)                                                                              \
+        hipLaunchKernelGGL((vq::k_assign_mfma_wide_bf<LBG, NB, true, false, true>), dim3(cdiv(a.n, 128), (unsigned)a.m), \
+                           dim3(256), 0, ctx->stream, a, tb);                                                \
+    else if (half)                                                                                           \
+        hipLaunchKernelGGL((vq::k_assign_mfma_wide_bf<LBG, NB, false, false, true>), dim3(cdiv(a.n, 128), (unsigned)a.m), \
                            dim3(256), 0, ctx->stream, a, tb);                                                \
     else if (a.pend_cb)                                                                                           \
         hipLaunchKernelGGL((vq::k_assign_mfma_wide_bf<LBG, NB, true>), dim3(cdiv(a.n, 128), (unsigned)a.m),    \
