@@ -114,6 +114,62 @@ static __global__ void __launch_bounds__(64) k_row_norms(const float *__restrict
     if (row0 + lane < n) norms[row0 + lane] = sqrtf(acc);
 }
 
+// A stage of an encode with the early stop, in one pass over the residual: k_residual_sub4, the sequential
+// norm of k_row_norms and the test `||residual|| < epsilon` (src/rvq.rs:200-207).  One wave = 64 rows, 32
+// columns at a time: a lane loads 16 bytes of eight rows and of their centroids, all in flight together,
+// stores the differences and leaves them in a padded LDS tile, and each lane then walks its own row.
+// HBM-bound: 200,000 x 128 read and written in 36 us; three launches and a second read of the
+// residual took 34 + 22 + 5 us.  (32 columns: 8 KB of LDS per wave; with 64 a compute unit holds 9 waves.)
+template <typename CodeT>
+static __global__ void __launch_bounds__(64) k_rvq_stage_step4(float *res, int64_t n, int dim,
+                                                               const float *__restrict__ cb,
+                                                               const CodeT *__restrict__ stage_codes,
+                                                               CodeT *__restrict__ codes_out, int stages, int stage,
+                                                               uint8_t *__restrict__ active, uint8_t *__restrict__ used,
+                                                               const float *src, int64_t src_ld, float epsilon) {
+    __shared__ float tile[64][33];
+    const int lane = threadIdx.x;
+    const int64_t row0 = (int64_t)blockIdx.x * 64, own = row0 + lane;
+    const int left = n - row0 < 64 ? (int)(n - row0) : 64;
+    const bool on = own < n && active[own] != 0;
+    const int code = on ? (int)stage_codes[own] : 0;
+    if (own < n) codes_out[own * stages + stage] = (CodeT)code;
+    if (on) used[own] = (uint8_t)(stage + 1);
+    const uint64_t live = __ballot(on);
+    if (live == 0) return;
+    const int sub = lane >> 3, piece = 4 * (lane & 7);
+    float acc = 0.0f;
+    for (int c0 = 0; c0 < dim; c0 += 32) {
+        const int w = dim - c0 < 32 ? dim - c0 : 32;
+        const bool in = piece < w;
+        const int col = c0 + (in ? piece : 0);
+        float4 v[8], c[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {  // unconditional, clamped: nothing of the surplus is stored or summed
+            const int r = 8 * i + sub, rc = r < left ? r : 0;
+            v[i] = *reinterpret_cast<const float4 *>(src + (row0 + rc) * src_ld + col);
+            c[i] = *reinterpret_cast<const float4 *>(cb + (size_t)__shfl(code, r) * dim + col);
+        }
+        __syncthreads();  // the lanes have read the previous tile
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int r = 8 * i + sub;
+            const float4 d = make_float4(v[i].x - c[i].x, v[i].y - c[i].y, v[i].z - c[i].z, v[i].w - c[i].w);
+            if (in && ((live >> r) & 1)) *reinterpret_cast<float4 *>(res + (row0 + r) * (int64_t)dim + col) = d;
+            tile[r][piece] = d.x;
+            tile[r][piece + 1] = d.y;
+            tile[r][piece + 2] = d.z;
+            tile[r][piece + 3] = d.w;
+        }
+        __syncthreads();
+        for (int t = 0; t < w; ++t) {
+            const float q = tile[lane][t] * tile[lane][t];
+            acc = acc + q;
+        }
+    }
+    if (on && sqrtf(acc) < epsilon) active[own] = 0;
+}
+
 // Fixed-shape two-level sum of n floats in f64: every workgroup sums a contiguous slice with a
 // fixed intra-group tree; a second launch of one workgroup sums the partials the same way.
 static __global__ void __launch_bounds__(256) k_sum_f64(const float *__restrict__ in_f32,

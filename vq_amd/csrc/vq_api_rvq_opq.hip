@@ -128,6 +128,11 @@ int32_t rvq_encode(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int
             pend_from_x = from_x;
             continue;
         }
+        if (vec4 && epsilon > 0.0f) {
+            hipLaunchKernelGGL(vq::k_rvq_stage_step4<CodeT>, dim3(cdiv(n, 64)), dim3(64), 0, st, res, n, dim, cb,
+                               (const CodeT *)cur, d_codes, stages, s, active, used, rows, rows_ld, epsilon);
+            continue;
+        }
         if (vec4)
             hipLaunchKernelGGL(vq::k_residual_sub4<CodeT>, dim3(cdiv(n * (dim / 4), 1024)), dim3(256), 0, st, res, n,
                                (int64_t)dim, dim / 4, cb, (const CodeT *)cur, (const uint8_t *)active, d_codes,
