@@ -62,3 +62,44 @@ def test_wide_codes(ctx, n, m, sd, k, metric, kind):
         ctx.assign(metric, ctx.to_device(x), n, m * sd, m, sd, k, ctx.to_device(cb), codes)
         want = O.pq_encode(metric, x, cb).astype(np.uint8)
     assert np.array_equal(codes.download(), want)
+
+
+@pytest.mark.parametrize("n,m,sd,k,kind", [(131_075, 1, 256, 256, "collapsed"), (140_001, 1, 304, 256, "grid"),
+                                           (65_540, 2, 104, 200, "near_ties"), (14_600, 9, 72, 256, "edges"),
+                                           (140_000, 1, 264, 33, "spread"), (45_000, 3, 64, 256, "overflow")])
+def test_resident_codes(ctx, n, m, sd, k, kind):
+    """Large calls: the operands resident in LDS, several tiles per wave; also a fit's pass (codes in planes,
+    compared through the centroids)."""
+    x, cb = _case(kind, n, m, sd, k)
+    codes = ctx.empty((n, m), np.uint8)
+    dx, dcb = ctx.to_device(x), ctx.to_device(cb)
+    with np.errstate(all="ignore"):
+        ctx.assign(O.EUCLIDEAN, dx, n, m * sd, m, sd, k, dcb, codes)
+        got = codes.download()
+        pick = np.unique(np.concatenate([np.arange(300), np.random.default_rng(1).integers(0, n, 3000), np.arange(n - 300, n)]))
+        assert np.array_equal(got[pick], O.pq_encode(O.EUCLIDEAN, x[pick], cb).astype(np.uint8))
+        # every row against the all-vector kernels
+        ctx.set_assign_path(1)
+        try:
+            ctx.assign(O.EUCLIDEAN, dx, n, m * sd, m, sd, k, dcb, codes)
+        finally:
+            ctx.set_assign_path(0)
+        assert np.array_equal(got, codes.download())
+
+
+def test_resident_fit(ctx):
+    n, m, sd, k, iters = 70_003, 2, 64, 256, 3
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((n, m * sd)).astype(F)
+    init = np.stack([rng.permutation(n)[:k] for _ in range(m)]).astype(np.uint32)
+    reseed = rng.integers(0, n, (m, k * iters), dtype=np.uint32)
+    dx, out = ctx.to_device(x), []
+    for path in (0, 1):
+        cb = ctx.empty((m, k, sd), np.float32)
+        ctx.set_assign_path(path)
+        try:
+            ctx.lbg_fit(dx, n, m * sd, m, sd, k, iters, init, reseed, cb)
+        finally:
+            ctx.set_assign_path(0)
+        out.append(cb.download())
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))

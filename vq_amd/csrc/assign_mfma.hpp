@@ -872,7 +872,7 @@ constexpr float kWideT = 0.35f;
 // a power of two that brings the centroids' root mean square norm to 32 ... 64; what the rounding of a row
 // (dx = ||x - xh||, summed as it happens) and of a centroid (dc) can do is 2 dx ||c|| + 2 ||x|| dc, split
 // between the row and the centroid as above, with kWideRho the usual dx / ||x||:
-//   2 dx ||c|| <= dx^2 t / rho + ||c||^2 rho / t,   2 ||x|| dc <= ||x||^2 rho t + dc^2 / (rho t).
+//   (x c - xh ch = (x - xh) ch + x (c - ch));  2 dx ||c|| <= dx^2 t / rho + ||c||^2 rho / t,   2 ||x|| dc <= ||x||^2 rho t + dc^2 / (rho t).
 // Three times as many rows are undecided (1-4 % of a residual stage instead of 0.3-1.5 %), a third of the matrix
 // instructions and half of the staged operands are left.  A value beyond the range of binary16 makes dx
 // infinite, and the row is listed; elements below its normal range count as if they were flushed.
@@ -880,7 +880,10 @@ constexpr float kWideT = 0.35f;
 // encode of 400,000 rows): k = 256: sd = 32 311 -> 328 us (8 blocks), 48 199 -> 193, 64 239 -> 207 (4 blocks),
 // 128 110 -> 88, 256 203 -> 153 (1 block); k = 64: sd = 64 70 -> 74 (2 blocks), 128 65 -> 64; k = 32: sd = 256
 // 125 -> 117.
-constexpr float kWideRho = 2.0e-4f;
+// t: where most centroids are as long as the rows (a random codebook) 0.35 leaves 6.3 % of the rows undecided and
+// 0.6 4.5 %, where they are short (a late residual stage) 2 and 3 %.
+constexpr float kWideRho = 2.0e-4f, kWideHalfT = 0.6f;
+constexpr float kWideTwo = 2.1f, kWideHalfTwo = 2.01f;  // both shares twice, and the roundings of x2, pen and the bound itself
 inline bool wide_half(int sd, int nb) { return sd >= 64 && sd * nb >= 512; }
 using f16x8 = _Float16 __attribute__((ext_vector_type(8)));
 constexpr int kWideCentreMax = 2048;  // widest column block whose centre is staged in LDS
@@ -1093,6 +1096,44 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
 // (__syncthreads would wait for the prefetches as well).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// HALF: the row operands of 32 dimensions, a lane's 8 of each 16 (from d0 and d0 + 16; zeros past the
+// width: the surplus loads repeat the row's first pieces, and a factor of zero takes them out).  mu: -mu sigma,
+// zeros up to a multiple of 32.
+__device__ __forceinline__ void wide_round(const float4 (&p)[4], int d0, int sd, bool shifted, const float *mu, float sg,
+                                           f16x8 (&b)[2], float &x2, float &dx2) {
+    using h2 = _Float16 __attribute__((ext_vector_type(2)));
+    using f2 = float __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const float sq = d0 + 16 * q < sd ? sg : 0.0f;
+        float xv[8] = {p[2 * q].x, p[2 * q].y, p[2 * q].z, p[2 * q].w,
+                       p[2 * q + 1].x, p[2 * q + 1].y, p[2 * q + 1].z, p[2 * q + 1].w};
+        if (shifted) {  // x sigma - mu sigma in one rounding
+            const float4 m0 = *reinterpret_cast<const float4 *>(mu + d0 + 16 * q);
+            const float4 m1 = *reinterpret_cast<const float4 *>(mu + d0 + 16 * q + 4);
+            const float mv[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+#pragma unroll
+            for (int u = 0; u < 8; ++u) xv[u] = __builtin_fmaf(xv[u], sq, mv[u]);
+        } else {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) xv[u] *= sq;
+        }
+        uint32_t w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            w[u] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{xv[2 * u], xv[2 * u + 1]}), h2));
+            float dl, dh;  // x - xh: one instruction each that reads a half of the pair
+            asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(dl) : "v"(w[u]), "v"(xv[2 * u]));
+            asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(dh) : "v"(w[u]), "v"(xv[2 * u + 1]));
+            x2 = __builtin_fmaf(xv[2 * u], xv[2 * u], x2);
+            x2 = __builtin_fmaf(xv[2 * u + 1], xv[2 * u + 1], x2);
+            dx2 = __builtin_fmaf(dl, dl, dx2);
+            dx2 = __builtin_fmaf(dh, dh, dx2);
+        }
+        b[q] = __builtin_bit_cast(f16x8, u32x4{w[0], w[1], w[2], w[3]});
+    }
+}
+
 // grid (ceil(n/128), m); 256 threads = 4 waves, one tile of 32 rows each against every centroid.
 // NB = tiles of 32 centroids (tb.nb), a template parameter so that the chains of matrix
 // instructions are straight-line code.
@@ -1135,7 +1176,10 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
         wg_pcount = 0;
     }
     if (tb.shifted[s] != 0)
-        for (int i = threadIdx.x; i < sd; i += 256) lds_mu[i] = HALF ? -(tb.mu[(size_t)s * sd + i] * sg) : tb.mu[(size_t)s * sd + i];
+        for (int i = threadIdx.x; i < (HALF ? (sd + 31) & ~31 : sd); i += 256) {
+            const float c = tb.mu[(size_t)s * sd + (i < sd ? i : 0)];
+            lds_mu[i] = !HALF ? c : i < sd ? -(c * sg) : 0.0f;
+        }
     if constexpr (PEND) {
         const int64_t row0 = (int64_t)blockIdx.x * 128;
         const int nrows = a.n - row0 < 128 ? (int)(a.n - row0) : 128;
@@ -1202,35 +1246,7 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
             }
         };
         auto halves = [&](int st, const float4(&p)[4], f16x8(&b)[2]) {
-            const bool last = st == nst - 1 && (sd & 31) != 0;  // uniform
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                float xv[8] = {p[2 * q].x, p[2 * q].y, p[2 * q].z, p[2 * q].w,
-                               p[2 * q + 1].x, p[2 * q + 1].y, p[2 * q + 1].z, p[2 * q + 1].w};
-                if (shifted) {  // x sigma - mu sigma in one rounding
-                    const float *mp = lds_mu + piece(2 * st + q);
-                    const float4 m0 = *reinterpret_cast<const float4 *>(mp), m1 = *reinterpret_cast<const float4 *>(mp + 4);
-                    const float mv[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) xv[u] = __builtin_fmaf(xv[u], sg, mv[u]);
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) xv[u] *= sg;
-                }
-                if (last) {
-                    if (16 * (2 * st + q) + 8 * h >= sd) {
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) xv[u] = 0.0f;
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    b[q][u] = (_Float16)xv[u];
-                    const float d = __builtin_fmaf((float)b[q][u], -1.0f, xv[u]);
-                    x2 = __builtin_fmaf(xv[u], xv[u], x2);
-                    dx2 = __builtin_fmaf(d, d, dx2);
-                }
-            }
+            wide_round(p, 32 * st + 8 * h, sd, shifted, lds_mu, sg, b, x2, dx2);
         };
         float4 xn[4], xf[4];
         f16x8 b[2], bn[2];
@@ -1438,7 +1454,7 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
             const bool finite = (bound < (COS ? 1e15f : 1e29f)) && (!COS || bound > 1e-15f) && (s1 < 1e29f);  // false for NaN
             // (1e-32: what products below the smallest normal number can lose)
             const float slack = COS ? tb.kappa * bound : tb.row_share * x2 + (HALF ? tb.dx_share * (dx2 + (float)sd * 0x1p-28f) : 0.0f) +
-                                          2.1f * lds_pen[COS ? 0 : i1] + 1e-32f;
+                                          (HALF ? kWideHalfTwo : kWideTwo) * lds_pen[COS ? 0 : i1] + 1e-32f;
             const float rel = COS ? 6.103515625e-05f : tb.rel;
             // the smallest exact distance is the best-scored centroid's when the second score is
             // further away than the error bound ...
@@ -1473,6 +1489,213 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < cnt; i += 256) tb.list[wg_base + i] = wg_list[i];
     for (uint32_t i = threadIdx.x; i < pcnt; i += 256) tb.pairs[wg_pbase + i] = wg_pairs[i];
+}
+
+
+// The same scores and decisions (HALF) where the operands of a whole column block fit LDS: one workgroup of
+// eight waves per compute unit keeps them (128 KB at 256 x 256) and walks over tiles of 32 rows, each wave on
+// its own.  No barrier and no operand fetch in the loop, so nothing but the rows is in flight and the
+// prefetch, three stages of 32 dimensions ahead and on across the tiles, is never drained (loads return in
+// order: in the staged kernel the wait for the next operands is one for the rows fetched before them too).
+// HBM-bound: 1,000,000 x 256, k = 256: 238 us = 4.3 TB/s, where the staged kernel takes 330 (vector ALU and
+// matrix cores busy for half of its cycles, the rest waits).  From two tiles per wave on: 60,000 rows of 256
+// take 38 us staged, 39.5 resident (256 workgroups fill 128 KB of LDS for one tile per wave); 60,000 x 4 of 64
+// 47 and 40; 20,000 x 7 of 72 38.5 and 37.5.
+constexpr int kWideResThreads = 512;
+constexpr int64_t kWideResMinRows = 256 * 8 * 32 * 2;  // rows x column blocks
+inline size_t wide_res_lds(int sd, int nb) {
+    const size_t npair = (sd + 15) / 16;
+    return npair * nb * 1024 + 2 * (size_t)nb * 128 + ((sd + 31) / 32) * 128 + 8 * 64 * (sizeof(uint2) + sizeof(uint32_t));
+}
+
+template <bool LBG, int NB>
+__global__ void __launch_bounds__(kWideResThreads, 2) k_assign_mfma_wide_res(AssignArgs a, MfmaWideBfTables tb) {
+    extern __shared__ u32x4 res_a[];  // [npair][NB][64], ||c||^2, pen, mu, the waves' lists
+    const int s = blockIdx.y;
+    if constexpr (LBG) {
+        if (block_done(a, s)) return;
+    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 31, h = lane >> 5;
+    const int sd = tb.sd, npair = (sd + 15) / 16, nst = (npair + 1) / 2, total16 = npair * NB * 64;
+    float *lds_c2 = reinterpret_cast<float *>(res_a + total16), *lds_pen = lds_c2 + NB * 32, *lds_mu = lds_pen + NB * 32;
+    uint2 *my_pairs = reinterpret_cast<uint2 *>(lds_mu + ((sd + 31) & ~31)) + wave * 64;
+    uint32_t *my_list = reinterpret_cast<uint32_t *>(reinterpret_cast<uint2 *>(lds_mu + ((sd + 31) & ~31)) + 8 * 64) + wave * 64;
+    const float sg = tb.sigma[s];
+    const bool shifted = tb.shifted[s] != 0;  // uniform
+    const u32x4 *ag = tb.atab + (size_t)s * total16;
+    for (int i = threadIdx.x; i < total16; i += kWideResThreads) res_a[i] = ag[i];
+    for (int i = threadIdx.x; i < NB * 32; i += kWideResThreads) {
+        lds_c2[i] = tb.c2perm[(size_t)s * NB * 32 + i];
+        lds_pen[i] = tb.pen[(size_t)s * NB * 32 + i];
+    }
+    for (int i = threadIdx.x; i < ((sd + 31) & ~31); i += kWideResThreads)
+        lds_mu[i] = shifted && i < sd ? -(tb.mu[(size_t)s * sd + i] * sg) : 0.0f;
+    float mc2 = 0.0f;  // largest ||c||^2 of the column block; a NaN stays
+    for (int b = 0; b < NB; ++b) {
+        const float o = tb.blockmax[(size_t)s * NB + b];
+        mc2 = (mc2 == mc2 && o == o) ? fmaxf(mc2, o) : __builtin_nanf("");
+    }
+    __syncthreads();
+
+    const int64_t ntiles = (a.n + 31) / 32, step_tiles = (int64_t)gridDim.x * 8;
+    int64_t tile = (int64_t)blockIdx.x * 8 + wave;
+    if (tile >= ntiles) return;  // (no barrier follows)
+    const char *xs = reinterpret_cast<const char *>(a.x + (int64_t)s * sd);
+    const int64_t tile_bytes = 128 * a.ld;
+    auto lane_base = [&](int64_t t) { return t * 32 + r < a.n ? 4u * (uint32_t)r * (uint32_t)a.ld : 0u; };
+    auto piece = [&](int pr) { return 16 * pr + 8 * h < sd ? 16 * pr + 8 * h : 0; };
+    // where the prefetch is: it runs on into the wave's next tile (and stays on the last one)
+    int64_t ptile = tile;
+    int pst = 0;
+    const char *pbase = xs + ptile * tile_bytes;
+    uint32_t plane = lane_base(ptile);
+    auto fetch = [&](float4(&p)[4]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const uint32_t o = plane + 4u * (uint32_t)piece(2 * pst + q);
+            p[2 * q] = *reinterpret_cast<const float4 *>(pbase + o);
+            p[2 * q + 1] = *reinterpret_cast<const float4 *>(pbase + (o + 16u));
+        }
+        if (++pst == nst) {
+            pst = 0;
+            if (ptile + step_tiles < ntiles) ptile += step_tiles;
+            pbase = xs + ptile * tile_bytes;
+            plane = lane_base(ptile);
+        }
+    };
+    float4 x0[4], x1[4], x3[4];
+    f16x8 b[2], bn[2];
+    float x2 = 0.0f, dx2 = 0.0f;
+    fetch(x0);
+    fetch(x1);
+    fetch(x3);
+    auto next_rows = [&](int st) {  // the operands of a stage; everything behind it moves up
+        wide_round(x0, 32 * st + 8 * h, sd, shifted, lds_mu, sg, bn, x2, dx2);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            x0[q] = x1[q];
+            x1[q] = x3[q];
+        }
+        fetch(x3);
+    };
+    next_rows(0);
+    const uint32_t keep = opaque_vgpr(0xFFFFFF00u);
+    uint32_t npairs = 0, nlist = 0;  // uniform
+    auto flush_pairs = [&]() {
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(tb.list_count + 1, npairs);
+        base = __builtin_amdgcn_readfirstlane(base);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if ((uint32_t)lane < npairs) tb.pairs[base + lane] = my_pairs[lane];
+        __builtin_amdgcn_wave_barrier();
+        npairs = 0;
+    };
+    auto flush_list = [&]() {
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(tb.list_count, nlist);
+        base = __builtin_amdgcn_readfirstlane(base);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if ((uint32_t)lane < nlist) tb.list[base + lane] = my_list[lane];
+        __builtin_amdgcn_wave_barrier();
+        nlist = 0;
+    };
+    for (; tile < ntiles; tile += step_tiles) {
+        const int64_t row = tile * 32 + r;
+        const bool valid = row < a.n;
+        uint8_t old = 0;
+        if constexpr (LBG) old = a.codes[(size_t)s * a.n + (valid ? row : a.n - 1)];
+        floatx16 acc[NB];
+#pragma unroll
+        for (int c = 0; c < NB; ++c)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[c][v] = lds_c2[(c * 2 + h) * 16 + v];
+        float row2 = 0.0f, rowd2 = 0.0f;
+        for (int st = 0; st < nst; ++st) {
+            b[0] = bn[0];
+            b[1] = bn[1];
+            auto step = [&](int pr, const f16x8 &bq) {
+#pragma unroll
+                for (int b0 = 0; b0 < NB; b0 += 4) {
+                    u32x4 ah[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (b0 + c < NB) ah[c] = res_a[(pr * NB + b0 + c) * 64 + lane];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (b0 + c < NB)
+                            acc[b0 + c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, ah[c]), bq,
+                                                                                acc[b0 + c], 0, 0, 0);
+                }
+            };
+            step(2 * st, b[0]);
+            // the next stage's row operands (the next tile's first, behind the last stage), in the shadow of
+            // the matrix instructions
+            const bool last = st + 1 == nst;
+            if (last) {
+                row2 = x2;
+                rowd2 = dx2;
+                x2 = 0.0f;
+                dx2 = 0.0f;
+            }
+            next_rows(last ? 0 : st + 1);
+            if (2 * st + 1 < npair) step(2 * st + 1, b[1]);
+        }
+        row2 += __shfl_xor(row2, 32);
+        rowd2 += __shfl_xor(rowd2, 32);
+        const float lifted = tb.lift * row2 + 1.0f;
+        int m1 = 0x7f800000, m2 = 0x7f800000, m3 = 0x7f800000;
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
+#pragma unroll
+            for (int v = 0; v < 16; v += 4) {
+                int key[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    key[u] = pack_tag(acc[c][v + u] + lifted, keep, (uint32_t)(32 * c + 8 * (v / 4) + u));
+                top3_push4(m1, m2, m3, key[0], key[1], key[2], key[3]);
+            }
+        }
+        m1 |= 4 * h;
+        m2 |= 4 * h;
+        const int o1 = __shfl_xor(m1, 32), o2 = __shfl_xor(m2, 32), o3 = __shfl_xor(m3, 32);
+        top3_push4(m1, m2, m3, o1, o2, o3, 0x7f800000);
+        const uint32_t i1 = (uint32_t)m1 & 0xFFu, i2 = (uint32_t)m2 & 0xFFu;
+        const float s1 = __int_as_float(m1), s2 = __int_as_float(m2), s3 = __int_as_float(m3);
+        const float bound = row2 + mc2;
+        const bool finite = (bound < 1e29f) && (s1 < 1e29f);  // false for NaN
+        const float slack = tb.row_share * row2 + tb.dx_share * (rowd2 + (float)sd * 0x1p-28f) +
+                            kWideHalfTwo * lds_pen[i1] + 1e-32f;
+        const bool sure = finite && (s2 - s1) > tb.rel * fabsf(s2) + slack;
+        const bool two = finite && (s2 < 1e29f) && (s3 - s1) > tb.rel * fabsf(s3) + slack;
+        const bool mine = valid && h == 0;
+        if (mine && sure) {
+            if constexpr (LBG) {
+                if (old != (uint8_t)i1) {
+                    a.codes[(size_t)s * a.n + row] = (uint8_t)i1;
+                    mark_changed(a.changed + s);
+                }
+            } else {
+                a.codes[row * a.m + s] = (uint8_t)i1;
+            }
+        }
+        const uint64_t pm = __ballot(mine && !sure && two), lm = __ballot(mine && !sure && !two);
+        const uint64_t below = ((uint64_t)1 << lane) - 1;
+        if (pm) {  // uniform
+            if (npairs > 32) flush_pairs();
+            if ((pm >> lane) & 1) my_pairs[npairs + __popcll(pm & below)] = make_uint2((uint32_t)(row * a.m + s), i1 | (i2 << 8));
+            npairs += (uint32_t)__popcll(pm);
+        }
+        if (lm) {
+            if (nlist > 32) flush_list();
+            if ((lm >> lane) & 1) my_list[nlist + __popcll(lm & below)] = (uint32_t)(row * a.m + s);
+            nlist += (uint32_t)__popcll(lm);
+        }
+    }
+    if (npairs) flush_pairs();
+    if (nlist) flush_list();
 }
 
 }  // namespace vq

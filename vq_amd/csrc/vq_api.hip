@@ -300,19 +300,20 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     constexpr bool COS = METRIC == vq::M_COS;
     if (!COS)
         hipLaunchKernelGGL(vq::k_block_centres, dim3(a.m, nsl), dim3(256), 0, ctx->stream, a.cb, a.k, sd, mu, norms);
-    // squared L2, Euclidean: see kWideT.  2.1 instead of 2: the roundings of x2, pen and the bound itself
+    // squared L2, Euclidean: see kWideT and kWideRho
     // cosine, in units of |x|, two candidates: the split of an operand twice as long, 2^-22 for the division by
     // the norm, fp32 accumulation (34 per 8 dimensions + 16) * 2^-24 of partial sums up to 4.2 |x|, the
     // reference's own rounding 2 (sub_dim + 6) * 2^-24
-    const float u24 = 5.9604644775390625e-08f, split = 3.0f * 1.52587890625e-05f, t = vq::kWideT;
+    const float u24 = 5.9604644775390625e-08f, split = 3.0f * 1.52587890625e-05f;
     const float kappa = 2.0f * (2.0f * split + (8.0f + 4.2f * (34.0f * nkc + 16.0f) + 2.0f * (sd + 6.0f)) * u24);
     const bool half = !COS && vq::wide_half(sd, nb);
-    const float rho = vq::kWideRho;
-    // HALF: 17 additions per instruction, one instruction per 16 dimensions begun, and a rounding per dimension
+    const float rho = vq::kWideRho, t = half ? vq::kWideHalfT : vq::kWideT;
+    const float twice = half ? vq::kWideHalfTwo : vq::kWideTwo;
+    // half: 17 additions per instruction, one instruction per 16 dimensions begun, and a rounding per dimension
     const float acc_err = (half ? 10.0f * nkc + 26.0f : 27.0f * nkc + 28.0f) * u24;
     const float cross = half ? acc_err + rho : split + acc_err;
     const float pen_c2 = acc_err + cross / t, pen_dc = 1.0f / (rho * t);
-    // (HALF: dc is at most 2^-11 ||c||)
+    // (half: dc is at most 2^-11 ||c||)
     const float lift = 1.001f + 8.0f * (pen_c2 + (half ? 2.4e-7f * pen_dc : 0.0f));
     const float rel = 6.103515625e-05f + 2.0f * (sd + 16.0f) * u24;
     const void *prep = half ? (const void *)vq::k_mfma_wide_bf_prep<false, true> : (const void *)vq::k_mfma_wide_bf_prep<COS, false>;
@@ -325,7 +326,11 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
         VQ_HIP(ctx, hipLaunchKernel(prep, dim3(a.m, nb), dim3(256), args, 0, ctx->stream));
     }
     vq::MfmaWideBfTables tb{(const vq::u32x4 *)atab, c2perm, pen, maxc2, mu, shifted, sigma, list, count, pairs, nb, sd,
-                            kappa, 2.1f * cross * t, 2.1f * t / rho, lift, rel};
+                            kappa, twice * cross * t, twice * t / rho, lift, rel};
+    const size_t res_lds = vq::wide_res_lds(sd, nb);
+    const bool resident = half && !a.pend_cb && res_lds <= 160 * 1024 && a.n * a.m >= vq::kWideResMinRows &&
+                          a.ld < ((int64_t)1 << 24);  // (32 rows below 2^31 bytes)
+    const int64_t res_groups = std::max<int64_t>(1, 256 / a.m);
     {
         ProfSpan sp(ctx, VQ_PROF_ASSIGN_KERNEL);
 #define WIDE(NB)                                                                                             \
@@ -335,7 +340,13 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     else if (half && a.pend_cb)                                                                              \
         hipLaunchKernelGGL((vq::k_assign_mfma_wide_bf<LBG, NB, true, false, true>), dim3(cdiv(a.n, 128), (unsigned)a.m), \
                            dim3(256), 0, ctx->stream, a, tb);                                                \
-    else if (half)                                                                                           \
+    else if (resident) {                                                                                     \
+        const void *kern = (const void *)vq::k_assign_mfma_wide_res<LBG, NB>;                                \
+        if (res_lds > 48 * 1024)                                                                             \
+            VQ_HIP(ctx, hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)res_lds)); \
+        hipLaunchKernelGGL((vq::k_assign_mfma_wide_res<LBG, NB>), dim3((unsigned)res_groups, (unsigned)a.m), \
+                           dim3(vq::kWideResThreads), res_lds, ctx->stream, a, tb);                          \
+    } else if (half)                                                                                         \
         hipLaunchKernelGGL((vq::k_assign_mfma_wide_bf<LBG, NB, false, false, true>), dim3(cdiv(a.n, 128), (unsigned)a.m), \
                            dim3(256), 0, ctx->stream, a, tb);                                                \
     else if (a.pend_cb)                                                                                           \
