@@ -1090,6 +1090,145 @@ static __global__ void k_seg_median(const SegSelect *__restrict__ sel, const uin
     median[i] = (cnt % 2u == 0u) ? sum / 2.0f : a;
 }
 
+// Split dimension, median and stable partition of one node by one workgroup, for levels whose nodes all fit
+// LDS: k_seg_argmax_last ... k_seg_partition are fourteen launches with the host's launch times between
+// them (100-150 us per level of 100,000 rows), whatever the nodes' sizes; this is one of 45 us (8 nodes of 12,500
+// rows) to 9 us (512 nodes).
+// lds: the keys of the node's rows, 2 x 256 counters, the waves' partial sums.  Any number of whole waves.
+constexpr uint32_t kSplitWgMax = 16384;  // rows: 64 KB of keys
+inline size_t split_wg_lds(uint32_t longest) { return sizeof(uint32_t) * ((size_t)longest + 512 + 64); }
+
+static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__restrict__ perm,
+                                                              const uint2 *__restrict__ seg_range,
+                                                              const float *__restrict__ var, int dim,
+                                                              const float *__restrict__ x, int64_t ld,
+                                                              int *__restrict__ split_dim, float *__restrict__ median,
+                                                              uint32_t *__restrict__ nleft, uint32_t *__restrict__ perm_out) {
+    extern __shared__ uint32_t lds_split[];
+    uint32_t *hist = lds_split, *part = hist + 512, *key = part + 64;
+    const int g = blockIdx.x, tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
+    const uint2 r = seg_range[g];
+    const uint32_t cnt = r.y - r.x;
+    // The reference's scan keeps an index for which !(v[t] < best so far): the last of the largest values, and a
+    // NaN or what follows one is always taken.  A run of values acts on what came before as its own result
+    // does, unless it holds a NaN: then it decides alone; so runs compose in order, one per lane.
+    if (wave == 0) {
+        const float *v = var + (size_t)g * dim;
+        const int per = (dim + 63) / 64, t0 = lane * per, t1 = t0 + per < dim ? t0 + per : dim;
+        int best = t0;
+        float vb = t0 < dim ? v[t0] : 0.0f;
+        bool any = t0 < dim, alone = any && !(vb == vb);
+        for (int t = t0 + 1; t < t1; ++t) {
+            const float w = v[t];
+            alone = alone || !(w == w);
+            if (!(w < vb)) {
+                best = t;
+                vb = w;
+            }
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {  // lane l holds the runs l .. l + 2 off - 1
+            const int ob = __shfl_down(best, off);
+            const float ov = __shfl_down(vb, off);
+            const bool oa = __shfl_down((int)alone, off) != 0, on = __shfl_down((int)any, off) != 0;
+            if (lane + off < 64 && on && (oa || !(ov < vb))) {
+                best = ob;
+                vb = ov;
+            }
+            alone = alone || oa;
+        }
+        if (lane == 0) {
+            part[0] = (uint32_t)best;
+            split_dim[g] = best;
+        }
+    }
+    for (int i = tid; i < 512; i += nt) hist[i] = 0u;
+    __syncthreads();
+    const int col = (int)part[0];
+    for (uint32_t p = tid; p < cnt; p += nt) key[p] = float_order_key(x[(int64_t)perm[r.x + p] * ld + col]);
+    __syncthreads();
+    // both middle ranks, a byte per pass; waves 0 and 1 pick
+    uint32_t pre0 = 0u, pre1 = 0u, rank0 = (cnt % 2 == 0) ? cnt / 2 - 1 : cnt / 2, rank1 = cnt / 2;
+    for (int pass = 0; pass < 4; ++pass) {
+        const int shift = 24 - 8 * pass;
+        const uint32_t high = pass == 0 ? 0u : (0xFFFFFFFFu << (shift + 8));
+        const bool same = pre0 == pre1;  // uniform: one histogram serves both
+        for (uint32_t p = tid; p < cnt; p += nt) {
+            const uint32_t k = key[p], byte = (k >> shift) & 255u;
+            if ((k & high) == pre0) atomicAdd(&hist[byte], 1u);
+            if (!same && (k & high) == pre1) atomicAdd(&hist[256 + byte], 1u);
+        }
+        __syncthreads();
+        for (int w = wave; w < 2; w += nw) {
+            const uint32_t *h = hist + (same ? 0 : 256 * w) + 4 * lane;
+            const uint32_t c0 = h[0], c1 = h[1], c2 = h[2], tot = c0 + c1 + c2 + h[3], rank = w ? rank1 : rank0;
+            uint32_t inc = tot;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t v = __shfl_up(inc, off);
+                if (lane >= off) inc += v;
+            }
+            uint32_t left = rank - (inc - tot);
+            if (rank >= inc - tot && rank < inc) {  // one lane: every rank is below cnt
+                uint32_t byte = 4u * (uint32_t)lane;
+                if (left >= c0) {
+                    left -= c0;
+                    ++byte;
+                    if (left >= c1) {
+                        left -= c1;
+                        ++byte;
+                        if (left >= c2) {
+                            left -= c2;
+                            ++byte;
+                        }
+                    }
+                }
+                part[2 * w] = byte << shift;
+                part[2 * w + 1] = left;
+            }
+        }
+        __syncthreads();
+        pre0 |= part[0];
+        rank0 = part[1];
+        pre1 |= part[2];
+        rank1 = part[3];
+        for (int i = tid; i < 512; i += nt) hist[i] = 0u;
+        __syncthreads();
+    }
+    const float ma = float_from_order_key(pre0), mb = float_from_order_key(pre1), sum = ma + mb;
+    const float med = (cnt % 2u == 0u) ? sum / 2.0f : ma;
+    // left count, then the rows in order: each wave's share of a stretch of nt rows by its ballot
+    uint32_t mine = 0;
+    for (uint32_t p = tid; p < cnt; p += nt) mine += float_from_order_key(key[p]) <= med ? 1u : 0u;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off);
+    if (lane == 0) part[wave] = mine;
+    __syncthreads();
+    uint32_t total = 0;
+    for (int w = 0; w < nw; ++w) total += part[w];
+    if (tid == 0) {
+        median[g] = med;
+        nleft[g] = total;
+    }
+    uint32_t before = 0;  // left rows of the stretches so far
+    for (uint32_t base = 0; base < cnt; base += nt) {
+        const uint32_t p = base + tid;
+        const bool in = p < cnt, left = in && float_from_order_key(key[p]) <= med;
+        const uint64_t m = __ballot(left);
+        __syncthreads();  // (part has been read)
+        if (lane == 0) part[wave] = (uint32_t)__popcll(m);
+        __syncthreads();
+        uint32_t mybefore = before + (uint32_t)__popcll(m & (((uint64_t)1 << lane) - 1));
+        for (int w = 0; w < nw; ++w) {
+            const uint32_t c = part[w];
+            if (w < wave) mybefore += c;
+            before += c;
+        }
+        if (in) perm_out[left ? r.x + mybefore : r.x + total + (p - mybefore)] = perm[r.x + p];
+    }
+}
+
+
 // out[i][t] = means[idx[i]][t]: the means of the nodes that split, side by side
 static __global__ void __launch_bounds__(256) k_gather_means(const float *__restrict__ means,
                                                              const int *__restrict__ idx, int ns, int dim,

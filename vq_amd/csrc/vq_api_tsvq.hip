@@ -144,6 +144,11 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     VQ_TRY(ensure(ctx, ctx->tmp_f, sizeof(uint32_t) * (size_t)n));
     // two-step variance (squares on the whole GPU, then the chains): dim a multiple of 8, and room
     // for a level's squares with every node starting on its own group of 32 positions
+    // levels whose longest node is no longer than this: a workgroup per node (k_seg_variance_wg, 11 ns per row of
+    // 128 and node, one launch) instead of the composed maps (four launches, 115 us at one node of 100,000 rows,
+    // 62 at 16 nodes, 275 at 512, where the walks over many short columns cost most): 16 nodes of 6,250 rows
+    // 78 and 62 us, 32 of 3,125 44 and 71, 512 of 195 22 and 275
+    constexpr uint32_t kVarWgRows = 4096;
     constexpr int kChainSegs = 2048;  // levels with more nodes than this take the other kernels
     const bool var_chain = dim % 8 == 0;
     // per group of 32 squares (composed-maps path): approximate sum, binade guess, integer maps;
@@ -340,6 +345,9 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
         int *d_sdim = (int *)d_down;
         float *d_median = (float *)d_down + ns;
         uint32_t *d_nleft = (uint32_t *)d_down + 2 * (size_t)ns;
+        uint32_t longest = 0;
+        for (int i = 0; i < ns; ++i) longest = std::max(longest, range[i].y - range[i].x);
+        const bool split_wg = !km && longest <= vq::kSplitWgMax;
         if (km) {
             // ---- 2-means split: lbg_quantize with k = 2 on every splitting node's rows ----------
             km_first.assign((size_t)ns + 1, 0u);
@@ -456,9 +464,8 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
         hipLaunchKernelGGL(vq::k_gather_means, dim3(cdiv((int64_t)ns * dim, 256)), dim3(256), 0, st,
                            (const float *)d_means, (const int *)d_split, ns, dim, (float *)d_smeans);
         // per-dimension sums of squared deviations (src/tsvq.rs:88-99)
-        if (var_chain && ns <= kChainSegs) {
-            uint32_t longest = 0;
-            for (int i = 0; i < ns; ++i) longest = std::max(longest, range[i].y - range[i].x);
+        const bool var_wg = dim % 4 == 0 && dim <= 1024 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;
+        if (var_chain && ns <= kChainSegs && !(var_wg && ctx->tsvq_var_path == 0 && longest <= kVarWgRows)) {
             hipLaunchKernelGGL(vq::k_seg_sqdev32, dim3((unsigned)cdiv((int64_t)longest, 64), (unsigned)ns), dim3(256),
                                0, st, perm, (const uint2 *)d_range, (const float *)d_smeans, (int64_t)0, d_x, ld, dim,
                                var_maps ? (float *)nullptr : d_sq, var_maps ? (float *)ctx->tsvq_gsum.p : (float *)nullptr);
@@ -508,7 +515,7 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                 hipLaunchKernelGGL(vq::k_seg_chain32, dim3((unsigned)ns, (unsigned)cdiv(dim, 32)), dim3(256), 0, st,
                                    (const float *)d_sq, (const uint2 *)d_range, dim, (float *)d_var);
             }
-        } else if (dim % 4 == 0 && dim <= 1024 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0) {
+        } else if (var_wg) {
 #define VARIANCE_WG(D)                                                                                     \
     hipLaunchKernelGGL((vq::k_seg_variance_wg<D>), dim3(ns), dim3(1024), 0, st, perm, (const uint2 *)d_range, \
                        (const float *)d_smeans, (int64_t)0, d_x, ld, dim, (float *)d_var)
@@ -525,6 +532,15 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                                (const uint2 *)d_range, ns, (const float *)d_smeans, (int64_t)0, d_x, ld, dim,
                                (float *)d_var);
         SP_HIP(hipGetLastError());
+        if (split_wg) {  // (a leaf's rows are not moved: nothing reads them again)
+            const size_t lds = vq::split_wg_lds(longest);
+            if (lds > 48 * 1024)
+                SP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_seg_split_wg),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            hipLaunchKernelGGL(vq::k_seg_split_wg, dim3((unsigned)ns), dim3(longest > 1024 ? 1024u : 256u), lds, st, perm,
+                               (const uint2 *)d_range, (const float *)d_var, dim, d_x, ld, d_sdim, d_median, d_nleft, perm2);
+            SP_HIP(hipGetLastError());
+        } else {
         // split dimension on the device (src/tsvq.rs:102-106); read back with the left counts below
         hipLaunchKernelGGL(vq::k_seg_argmax_last, dim3(cdiv((int64_t)ns * 512, 256)), dim3(256), 0, st,
                            (const float *)d_var, ns, dim, (int *)d_sdim, (const uint2 *)d_range, (vq::SegSelect *)d_sel,
@@ -544,7 +560,9 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
         // stable partition by `<= median` (src/tsvq.rs:120-123)
         hipLaunchKernelGGL(vq::k_seg_flags, dim3(cdiv(n, 256)), dim3(256), 0, st, vals, n, (const uint2 *)d_range,
                            ns, (const float *)d_median, flags);
+        }
         }  // median split
+        if (!split_wg) {
         size_t need = 0;
         SP_HIP(rocprim::exclusive_scan(nullptr, need, flags, scan, 0u, (size_t)n, rocprim::plus<uint32_t>(), st));
         {
@@ -558,6 +576,7 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
         hipLaunchKernelGGL(vq::k_seg_partition, dim3(cdiv(n, 256)), dim3(256), 0, st, perm, n,
                            (const uint2 *)d_range, ns, flags, scan, perm2, (uint32_t *)d_nleft);
         SP_HIP(hipGetLastError());
+        }
         char *h_down = (char *)ctx->tsvq_pin + up_bytes;
         SP_HIP(hipMemcpyAsync(h_down, d_down, down_bytes, hipMemcpyDeviceToHost, st));
         SP_HIP(hipStreamSynchronize(st));
