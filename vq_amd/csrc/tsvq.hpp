@@ -50,6 +50,57 @@ static __global__ void __launch_bounds__(256) k_seg_leafsum(const uint32_t *__re
     leaf_sum[leaf * sd + t] = acc;
 }
 
+// The same sums where there are too few of them to fill the chip with a lane each: a workgroup takes 32
+// components of a leaf, all of its threads bring the rows in, 128 at a time through LDS, and one half wave
+// adds them in order while the next tile is on its way (the row numbers a tile ahead of the rows).
+// 128 leaves of 782 rows of 128 (100,000 rows): 31 -> 13 us, a level of the tree each.
+static __global__ void __launch_bounds__(256) k_seg_leafsum_wg(const uint32_t *__restrict__ perm,
+                                                               const uint2 *__restrict__ desc,
+                                                               const float *__restrict__ x, int64_t ld, int sd,
+                                                               float *__restrict__ leaf_sum) {
+    __shared__ float tile[2][128][32];
+    const int64_t leaf = blockIdx.x;
+    const int c = threadIdx.x & 31, sub = threadIdx.x >> 5, t = blockIdx.y * 32 + c;
+    const uint2 d = desc[leaf];
+    const float *xc = x + (t < sd ? t : 0);
+    float acc = 0.0f;
+    if (d.y > d.x) {
+        const uint32_t last = d.y - 1;
+        uint32_t id[16];
+        float v[16];
+        auto ids = [&](uint32_t p) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) id[u] = perm[p + 8 * u + sub <= last ? p + 8 * u + sub : last];
+        };
+        auto rows = [&]() {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = xc[(int64_t)id[u] * ld];
+        };
+        ids(d.x);
+        rows();
+        ids(d.x + 128);
+        int buf = 0;
+        for (uint32_t p = d.x; p < d.y; p += 128, buf ^= 1) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) tile[buf][8 * u + sub][c] = v[u];
+            rows();  // (past the leaf: its last row again, not added)
+            ids(p + 256);
+            __syncthreads();
+            if (threadIdx.x < 32) {
+                const uint32_t left = d.y - p;
+                if (left >= 128) {
+#pragma unroll 32
+                    for (int r = 0; r < 128; ++r) acc = acc + tile[buf][r][c];
+                } else {
+#pragma unroll 8
+                    for (uint32_t r = 0; r < left; ++r) acc = acc + tile[buf][r][c];
+                }
+            }
+        }
+    }
+    if (threadIdx.x < 32 && t < sd) leaf_sum[leaf * sd + t] = acc;
+}
+
 // One lane per (segment, component): combine 2^depth leaves left + right, divide by the count.
 // seg_info[g] = {first leaf, depth, count, unused}
 static __global__ void __launch_bounds__(256) k_seg_mean(float *__restrict__ leaf_sum,

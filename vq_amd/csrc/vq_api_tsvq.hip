@@ -149,6 +149,7 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     // 62 at 16 nodes, 275 at 512, where the walks over many short columns cost most): 16 nodes of 6,250 rows
     // 78 and 62 us, 32 of 3,125 44 and 71, 512 of 195 22 and 275
     constexpr uint32_t kVarWgRows = 4096;
+    constexpr int64_t kLeafWgSums = 65536;  // a lane per sum fills half of the chip: both take the same time there
     constexpr int kChainSegs = 2048;  // levels with more nodes than this take the other kernels
     const bool var_chain = dim % 8 == 0;
     // per group of 32 squares (composed-maps path): approximate sum, binade guess, integer maps;
@@ -296,8 +297,12 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
             LV_HIP(hipMalloc(&d_means, sizeof(float) * (size_t)nseg * dim));
         level_means.push_back({d_means, first_node, nseg});
         LV_HIP(hipMemcpyAsync(ctx->tsvq_level.p, ctx->tsvq_pin, up_bytes, hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(vq::k_seg_leafsum, dim3(cdiv((int64_t)nleaves * dim, 256)), dim3(256), 0, st, perm,
-                           (const uint2 *)d_desc, (int64_t)nleaves, d_x, ld, dim, (float *)d_lsum);
+        if ((int64_t)nleaves * dim <= kLeafWgSums)
+            hipLaunchKernelGGL(vq::k_seg_leafsum_wg, dim3((unsigned)nleaves, cdiv(dim, 32)), dim3(256), 0, st, perm,
+                               (const uint2 *)d_desc, d_x, ld, dim, (float *)d_lsum);
+        else
+            hipLaunchKernelGGL(vq::k_seg_leafsum, dim3(cdiv((int64_t)nleaves * dim, 256)), dim3(256), 0, st, perm,
+                               (const uint2 *)d_desc, (int64_t)nleaves, d_x, ld, dim, (float *)d_lsum);
         int max_dep = 0;
         for (int g = 0; g < nseg; ++g) max_dep = std::max(max_dep, (int)info[g].y);
         if (max_dep >= 5 && (1 << max_dep) <= vq::kMeanWgLeaves && nseg <= 64)  // few segments of many leaves
