@@ -1169,11 +1169,14 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
                        h_iters_run, h_reseeds_used, pend_cb, pend_codes, [] {});
 }
 
-// Clusters per workgroup of k_lbg_update_small: as many as one thread per (cluster, component) and
-// four bits per list entry allow, but at least a workgroup per compute unit.
+// Clusters per workgroup of k_lbg_update_small: the fewest with which the workgroups (106 KB of LDS each) are one
+// round of the 256 compute units, as far as one thread per (cluster, component) and four bits per list entry
+// allow.  (m = 10, k = 200, 60,007 rows: 7 clusters are 290 workgroups and 64 us, 8 are 250 and 42 us.)
 static int lbg_small_clusters(int m, int sd, int k) {
-    return (int)std::max<int64_t>(1, std::min<int64_t>({vq::kSmallClusters, (int64_t)k * m / 256,
-                                                        (sd <= vq::kSmallThreads ? vq::kSmallThreads : 4096) / sd}));
+    const int most = std::max(1, std::min(vq::kSmallClusters, (sd <= vq::kSmallThreads ? vq::kSmallThreads : 4096) / sd));
+    int c = 1;
+    while (c < most && (int64_t)m * ((k + c - 1) / c) > 256) ++c;
+    return c;
 }
 
 // Whether the update of a fit runs as k_lbg_update_small.  Its time follows the members of a cluster
