@@ -16,10 +16,11 @@ using namespace vqh;
 namespace {
 
 template <int METRIC>
-void launch_merge(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int m, int sd, int kc, const float *chunk,
-                  const uint8_t *win, const float *win_d, int base, float *best, uint16_t *out) {
+void launch_merge(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int m, int sd, int k, const float *chunks,
+                  int base, int count, const uint8_t *win, const float *win_d, int64_t stride, unsigned have_d,
+                  float *best, uint16_t *out) {
     hipLaunchKernelGGL(vq::k_chunk_merge<METRIC>, dim3(cdiv(n * m, 256)), dim3(256), 0, ctx->stream, d_x, n, ld, m, sd,
-                       kc, chunk, win, win_d, base, best, out);
+                       k, chunks, base, count, win, win_d, stride, have_d, best, out);
 }
 
 }  // namespace
@@ -43,7 +44,11 @@ int32_t assign_codes_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t 
         return assign_few<uint16_t>(ctx, metric, d_x, n, ld, m, sd, k, d_codebooks, d_codes, d_out16);
     }
     const size_t pairs = (size_t)n * m;
-    VQ_TRY(ensure(ctx, ctx->big_win, (pairs + 3) & ~(size_t)3));
+    // chunks merged by one launch: their winners lie side by side (20 bytes per pair for four)
+    const int chunks = (int)cdiv(k, vq::kChunk);
+    const int together = pairs <= ((size_t)256 << 20) ? std::min(chunks, vq::kMergeChunks) : 1;
+    const size_t stride = (pairs + 255) & ~(size_t)255;
+    VQ_TRY(ensure(ctx, ctx->big_win, stride * together));
     uint8_t *win = (uint8_t *)ctx->big_win.p;
     if (k <= vq::kChunk) {  // one chunk: its winner is the answer
         VQ_TRY(assign_codes(ctx, metric, d_x, n, ld, m, sd, k, d_codebooks, win));
@@ -52,27 +57,34 @@ int32_t assign_codes_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t 
         VQ_HIP(ctx, hipGetLastError());
         return VQ_OK;
     }
-    VQ_TRY(ensure(ctx, ctx->big_chunk, sizeof(float) * (size_t)m * vq::kChunk * sd));
-    VQ_TRY(ensure(ctx, ctx->big_best, sizeof(float) * pairs));
-    VQ_TRY(ensure(ctx, ctx->big_wind, sizeof(float) * pairs));
-    float *chunk = (float *)ctx->big_chunk.p;
+    VQ_TRY(ensure(ctx, ctx->big_chunk, sizeof(float) * (size_t)m * k * sd));
+    if (chunks > together) VQ_TRY(ensure(ctx, ctx->big_best, sizeof(float) * pairs));
+    VQ_TRY(ensure(ctx, ctx->big_wind, sizeof(float) * stride * together));
+    float *tables = (float *)ctx->big_chunk.p;
     float *best = (float *)ctx->big_best.p;
     float *wind = (float *)ctx->big_wind.p;
-    for (int base = 0; base < k; base += vq::kChunk) {
-        const int kc = std::min(vq::kChunk, k - base);
-        hipLaunchKernelGGL(vq::k_chunk_tables, dim3(cdiv((int64_t)m * kc * sd, 256)), dim3(256), 0, ctx->stream,
-                           d_codebooks, m, k, sd, base, kc, chunk);
-        VQ_HIP(ctx, hipGetLastError());
-        // the winners' distances come with the codes where the assignment kernel computes them anyway
-        bool have_d = false;
-        VQ_TRY(assign_codes(ctx, metric, d_x, n, ld, m, sd, kc, chunk, win, wind, &have_d));
-        const float *wd = have_d ? wind : nullptr;
-        switch (metric) {
-        case VQ_SQEUCLIDEAN: launch_merge<vq::M_SQ>(ctx, d_x, n, ld, m, sd, kc, chunk, win, wd, base, best, d_codes); break;
-        case VQ_EUCLIDEAN: launch_merge<vq::M_EUCLID>(ctx, d_x, n, ld, m, sd, kc, chunk, win, wd, base, best, d_codes); break;
-        case VQ_COSINE: launch_merge<vq::M_COS>(ctx, d_x, n, ld, m, sd, kc, chunk, win, wd, base, best, d_codes); break;
-        default: launch_merge<vq::M_L1>(ctx, d_x, n, ld, m, sd, kc, chunk, win, wd, base, best, d_codes); break;
+    hipLaunchKernelGGL(vq::k_chunk_tables, dim3(cdiv((int64_t)m * k * sd, 256)), dim3(256), 0, ctx->stream, d_codebooks,
+                       m, k, sd, tables);
+    VQ_HIP(ctx, hipGetLastError());
+    for (int c0 = 0; c0 < chunks; c0 += together) {
+        const int count = std::min(together, chunks - c0), base = c0 * vq::kChunk;
+        unsigned have = 0;
+        for (int c = 0; c < count; ++c) {
+            const int b0 = base + c * vq::kChunk, kc = std::min(vq::kChunk, k - b0);
+            // the winners' distances come with the codes where the assignment kernel computes them anyway
+            bool have_d = false;
+            VQ_TRY(assign_codes(ctx, metric, d_x, n, ld, m, sd, kc, tables + (size_t)b0 * m * sd, win + c * stride,
+                                wind + c * stride, &have_d));
+            if (have_d) have |= 1u << c;
         }
+#define MERGE(M) launch_merge<M>(ctx, d_x, n, ld, m, sd, k, tables, base, count, win, wind, (int64_t)stride, have, best, d_codes)
+        switch (metric) {
+        case VQ_SQEUCLIDEAN: MERGE(vq::M_SQ); break;
+        case VQ_EUCLIDEAN: MERGE(vq::M_EUCLID); break;
+        case VQ_COSINE: MERGE(vq::M_COS); break;
+        default: MERGE(vq::M_L1); break;
+        }
+#undef MERGE
         VQ_HIP(ctx, hipGetLastError());
     }
     return VQ_OK;
