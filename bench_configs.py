@@ -296,15 +296,16 @@ def run_c4(ctx, log, parity=True):
     flop = 2.0 * k * dim * n
     tf = flop / (avg * 1e-3) / 1e12 if avg else 0.0
     out["dominant_kernel"] = {
-        "name": "k_assign_mfma_wide_bf (bf16-split scores of 32 rows x 256 centroids per wave, three matrix "
-                "instructions per 16 dimensions; 8 x 10 LBG passes + 7 residual passes)",
-        "bound": "mfma", "avg_launch_ms": round(avg, 4), "launches": cnt,
+        "name": "k_assign_mfma_wide_res (binary16 scores of 32 rows x 256 centroids per wave, one matrix instruction "
+                "per 16 dimensions, operands resident in LDS; 8 x 10 LBG passes + 7 residual passes, the first pass "
+                "of stages 2-8 by k_assign_mfma_wide_bf)",
+        "bound": "hbm", "avg_launch_ms": round(avg, 4), "launches": cnt,
         "algorithmic_work": "2*k*D = 131,072 flop per row and pass",
         # the distance sums priced as fp32 matrix work (what the accounting of the path asks for) ...
         "achieved": round(tf, 1), "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s", "frac": round(tf / PEAK_FP32_MFMA_TFLOPS, 4),
-        # ... and as what is issued on the bf16 units they run on (three bf16 products per fp32 one)
-        "issued_bf16_TFLOPs": round(3.0 * tf, 1), "issued_frac_of_bf16_peak": round(3.0 * tf / PEAK_BF16_MFMA_TFLOPS, 4),
-        "note": "frac above 1: the fp32-grade scores come from the bf16 matrix units, which the second pair of fields prices"}
+        # ... and as what is issued on the 16-bit units they run on (one product per fp32 one)
+        "issued_f16_TFLOPs": round(tf, 1), "issued_frac_of_f16_peak": round(tf / PEAK_BF16_MFMA_TFLOPS, 4),
+        "note": "frac above 1: the scores come from the 16-bit matrix units, which the second pair of fields prices"}
     dall = ctx.empty((n, stages), np.uint8)
     drec = ctx.empty((n, dim), np.uint16)
     enc = lambda: ctx.rvq_encode(vq_amd.EUCLIDEAN, dx, n, dim, dim, stages, k, dcb, 0.0, dall, None, drec)
