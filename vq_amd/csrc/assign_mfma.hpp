@@ -1302,120 +1302,120 @@ __global__ void __launch_bounds__(256, 2) k_assign_mfma_wide_bf(AssignArgs a, Mf
         }
         dx2 += __shfl_xor(dx2, 32);
     } else {
-    float4 xn0 = row_piece(piece(0));  // the next piece of the row
-    float4 xn1 = row_piece(piece(0) + 4);
-    const int second = npair > 1 ? 1 : 0;
-    float4 xf0 = row_piece(piece(second));  // and the one after it
-    float4 xf1 = row_piece(piece(second) + 4);
-    // The row operands of a stage: this half's 8 dimensions relative to the centre, their share of
-    // ||x - mu||^2, and their high and low bf16 parts.
-    auto split = [&](int st, const float4 &p0, const float4 &p1, u32x4 &bh, u32x4 &bl) {
-        float xv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-        if (shifted) {
-            const float4 m0 = *reinterpret_cast<const float4 *>(lds_mu + piece(st));
-            const float4 m1 = *reinterpret_cast<const float4 *>(lds_mu + piece(st) + 4);
-            xv[0] -= m0.x;
-            xv[1] -= m0.y;
-            xv[2] -= m0.z;
-            xv[3] -= m0.w;
-            xv[4] -= m1.x;
-            xv[5] -= m1.y;
-            xv[6] -= m1.z;
-            xv[7] -= m1.w;
-        }
-        if (st == npair - 1 && (sd & 8) != 0) {  // uniform: a width that is an odd multiple of 8 ends in the lower half
-            if (h != 0) {
-#pragma unroll
-                for (int u = 0; u < 8; ++u) xv[u] = 0.0f;
+        float4 xn0 = row_piece(piece(0));  // the next piece of the row
+        float4 xn1 = row_piece(piece(0) + 4);
+        const int second = npair > 1 ? 1 : 0;
+        float4 xf0 = row_piece(piece(second));  // and the one after it
+        float4 xf1 = row_piece(piece(second) + 4);
+        // The row operands of a stage: this half's 8 dimensions relative to the centre, their share of
+        // ||x - mu||^2, and their high and low bf16 parts.
+        auto split = [&](int st, const float4 &p0, const float4 &p1, u32x4 &bh, u32x4 &bl) {
+            float xv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+            if (shifted) {
+                const float4 m0 = *reinterpret_cast<const float4 *>(lds_mu + piece(st));
+                const float4 m1 = *reinterpret_cast<const float4 *>(lds_mu + piece(st) + 4);
+                xv[0] -= m0.x;
+                xv[1] -= m0.y;
+                xv[2] -= m0.z;
+                xv[3] -= m0.w;
+                xv[4] -= m1.x;
+                xv[5] -= m1.y;
+                xv[6] -= m1.z;
+                xv[7] -= m1.w;
             }
-        }
-        uint32_t hp[4], lp[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            x2 = __builtin_fmaf(xv[2 * u], xv[2 * u], x2);
-            x2 = __builtin_fmaf(xv[2 * u + 1], xv[2 * u + 1], x2);
-            hp[u] = bf16_pack2(xv[2 * u], xv[2 * u + 1]);
-            lp[u] = bf16_pack2(xv[2 * u] - __uint_as_float(hp[u] << 16), xv[2 * u + 1] - __uint_as_float(hp[u] & 0xffff0000u));
-        }
-        bh = u32x4{hp[0], hp[1], hp[2], hp[3]};
-        bl = u32x4{lp[0], lp[1], lp[2], lp[3]};
-    };
-    // A stage is 16 dimensions: with the high and low parts of the centroid operand (ah, al) and of
-    // the row operand (xh, xl), three matrix instructions per tile of 32 centroids,
-    //   ah . xh + al . xh + ah . xl,
-    // every contraction slot of each in use; one barrier per 3 NB matrix instructions of a wave.
-    // The row operands of stage st + 1 are made while the matrix instructions of stage st run: a
-    // matrix instruction holds back the vector instructions of the other waves of its SIMD, but
-    // independent vector instructions of its own wave issue in its shadow.
-    u32x4 bh, bl;
-    split(0, xn0, xn1, bh, bl);
-    xn0 = xf0;
-    xn1 = xf1;
-    {
-        const int nx = 2 < npair ? 2 : npair - 1;
-        xf0 = row_piece(piece(nx));
-        xf1 = row_piece(piece(nx) + 4);
-    }
-    for (int st = 0; st < npair; ++st) {
-        const int cur = st & 1;
-        const bool more = st + 1 < npair;
-        // the A operands of the next stage: into registers now, into LDS at the end of this stage
-        u32x4 pre[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t i = (uint32_t)((st + 1) * pair16) + threadIdx.x + 256u * (uint32_t)q;
-            const uint32_t ic = i < (uint32_t)total16 ? i : (uint32_t)total16 - 1u;
-            pre[q] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(ag) + 16u * ic);
-        }
-        // The stage's centroid operands are read from LDS four tiles (one group) at a time.
-        constexpr int NG = (NB + 3) / 4;  // groups of four centroid tiles
-        u32x4 nbh = bh, nbl = bl;
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            u32x4 ah[4], al[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int b = 4 * g + c < nb ? 4 * g + c : nb - 1;  // past the last block: read it, not multiplied
-                ah[c] = lds_a[cur][b * 128 + lane];
-                al[c] = lds_a[cur][b * 128 + 64 + lane];
+            if (st == npair - 1 && (sd & 8) != 0) {  // uniform: a width that is an odd multiple of 8 ends in the lower half
+                if (h != 0) {
+    #pragma unroll
+                    for (int u = 0; u < 8; ++u) xv[u] = 0.0f;
+                }
             }
-            // the three dependent instructions of a tile are three others apart
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (4 * g + c < nb)
-                    acc[4 * g + c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        __builtin_bit_cast(bf16x8, ah[c]), __builtin_bit_cast(bf16x8, bh), acc[4 * g + c], 0, 0, 0);
-            if (g == 0 && more) {
-                // next stage's row operands, behind the first matrix instructions of this stage
-                split(st + 1, xn0, xn1, nbh, nbl);
-                const int nx = st + 3 < npair ? st + 3 : npair - 1;
-                xn0 = xf0;
-                xn1 = xf1;
-                xf0 = row_piece(piece(nx));
-                xf1 = row_piece(piece(nx) + 4);
+            uint32_t hp[4], lp[4];
+    #pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                x2 = __builtin_fmaf(xv[2 * u], xv[2 * u], x2);
+                x2 = __builtin_fmaf(xv[2 * u + 1], xv[2 * u + 1], x2);
+                hp[u] = bf16_pack2(xv[2 * u], xv[2 * u + 1]);
+                lp[u] = bf16_pack2(xv[2 * u] - __uint_as_float(hp[u] << 16), xv[2 * u + 1] - __uint_as_float(hp[u] & 0xffff0000u));
             }
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (4 * g + c < nb)
-                    acc[4 * g + c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        __builtin_bit_cast(bf16x8, al[c]), __builtin_bit_cast(bf16x8, bh), acc[4 * g + c], 0, 0, 0);
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (4 * g + c < nb)
-                    acc[4 * g + c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        __builtin_bit_cast(bf16x8, ah[c]), __builtin_bit_cast(bf16x8, bl), acc[4 * g + c], 0, 0, 0);
+            bh = u32x4{hp[0], hp[1], hp[2], hp[3]};
+            bl = u32x4{lp[0], lp[1], lp[2], lp[3]};
+        };
+        // A stage is 16 dimensions: with the high and low parts of the centroid operand (ah, al) and of
+        // the row operand (xh, xl), three matrix instructions per tile of 32 centroids,
+        //   ah . xh + al . xh + ah . xl,
+        // every contraction slot of each in use; one barrier per 3 NB matrix instructions of a wave.
+        // The row operands of stage st + 1 are made while the matrix instructions of stage st run: a
+        // matrix instruction holds back the vector instructions of the other waves of its SIMD, but
+        // independent vector instructions of its own wave issue in its shadow.
+        u32x4 bh, bl;
+        split(0, xn0, xn1, bh, bl);
+        xn0 = xf0;
+        xn1 = xf1;
+        {
+            const int nx = 2 < npair ? 2 : npair - 1;
+            xf0 = row_piece(piece(nx));
+            xf1 = row_piece(piece(nx) + 4);
         }
-        bh = nbh;
-        bl = nbl;
-        if (more) {
-#pragma unroll
+        for (int st = 0; st < npair; ++st) {
+            const int cur = st & 1;
+            const bool more = st + 1 < npair;
+            // the A operands of the next stage: into registers now, into LDS at the end of this stage
+            u32x4 pre[4];
+    #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int i = threadIdx.x + 256 * q;
-                if (i < pair16) lds_a[cur ^ 1][i] = pre[q];
+                const uint32_t i = (uint32_t)((st + 1) * pair16) + threadIdx.x + 256u * (uint32_t)q;
+                const uint32_t ic = i < (uint32_t)total16 ? i : (uint32_t)total16 - 1u;
+                pre[q] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(ag) + 16u * ic);
             }
+            // The stage's centroid operands are read from LDS four tiles (one group) at a time.
+            constexpr int NG = (NB + 3) / 4;  // groups of four centroid tiles
+            u32x4 nbh = bh, nbl = bl;
+    #pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                u32x4 ah[4], al[4];
+    #pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int b = 4 * g + c < nb ? 4 * g + c : nb - 1;  // past the last block: read it, not multiplied
+                    ah[c] = lds_a[cur][b * 128 + lane];
+                    al[c] = lds_a[cur][b * 128 + 64 + lane];
+                }
+                // the three dependent instructions of a tile are three others apart
+    #pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (4 * g + c < nb)
+                        acc[4 * g + c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            __builtin_bit_cast(bf16x8, ah[c]), __builtin_bit_cast(bf16x8, bh), acc[4 * g + c], 0, 0, 0);
+                if (g == 0 && more) {
+                    // next stage's row operands, behind the first matrix instructions of this stage
+                    split(st + 1, xn0, xn1, nbh, nbl);
+                    const int nx = st + 3 < npair ? st + 3 : npair - 1;
+                    xn0 = xf0;
+                    xn1 = xf1;
+                    xf0 = row_piece(piece(nx));
+                    xf1 = row_piece(piece(nx) + 4);
+                }
+    #pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (4 * g + c < nb)
+                        acc[4 * g + c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            __builtin_bit_cast(bf16x8, al[c]), __builtin_bit_cast(bf16x8, bh), acc[4 * g + c], 0, 0, 0);
+    #pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (4 * g + c < nb)
+                        acc[4 * g + c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            __builtin_bit_cast(bf16x8, ah[c]), __builtin_bit_cast(bf16x8, bl), acc[4 * g + c], 0, 0, 0);
+            }
+            bh = nbh;
+            bl = nbl;
+            if (more) {
+    #pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int i = threadIdx.x + 256 * q;
+                    if (i < pair16) lds_a[cur ^ 1][i] = pre[q];
+                }
+            }
+            lds_barrier();
         }
-        lds_barrier();
-    }
     }
     x2 += __shfl_xor(x2, 32);  // both halves' shares of ||x - mu||^2
     const float nx = COS ? __builtin_amdgcn_sqrtf(x2) : 0.0f;
