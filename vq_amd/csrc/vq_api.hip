@@ -298,7 +298,8 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     int *shifted = (int *)(norms + (size_t)a.m * nsl);
     float *sigma = (float *)(shifted + a.m);
     constexpr bool COS = METRIC == vq::M_COS;
-    if (!COS)
+    const bool own_centre = !COS && vq::wide_own_centre(a.k, sd);
+    if (!COS && !own_centre)
         hipLaunchKernelGGL(vq::k_block_centres, dim3(a.m, nsl), dim3(256), 0, ctx->stream, a.cb, a.k, sd, mu, norms);
     // squared L2, Euclidean: see kWideT and kWideRho
     // cosine, in units of |x|, two candidates: the split of an operand twice as long, 2^-22 for the division by
@@ -316,7 +317,10 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     // (half: dc is at most 2^-11 ||c||)
     const float lift = 1.001f + 8.0f * (pen_c2 + (half ? 2.4e-7f * pen_dc : 0.0f));
     const float rel = 6.103515625e-05f + 2.0f * (sd + 16.0f) * u24;
-    const void *prep = half ? (const void *)vq::k_mfma_wide_bf_prep<false, true> : (const void *)vq::k_mfma_wide_bf_prep<COS, false>;
+    const void *prep = half ? own_centre ? (const void *)vq::k_mfma_wide_bf_prep<false, true, true>
+                                         : (const void *)vq::k_mfma_wide_bf_prep<false, true>
+                            : own_centre ? (const void *)vq::k_mfma_wide_bf_prep<false, false, true>
+                                         : (const void *)vq::k_mfma_wide_bf_prep<COS, false>;
     {
         vq::u32x4 *atab4 = (vq::u32x4 *)atab;
         int m = a.m, k = a.k, nbv = nb, sdv = sd;
