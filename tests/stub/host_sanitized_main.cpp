@@ -148,6 +148,15 @@ int main() {
         vqh_free(obj);
         CHECK(vqh_pq_fit(flat.data(), (int64_t)n, (int64_t)dim, 3, 0, 2, 1, 0.0, 0, nullptr, nullptr, 0, &obj) != 0);
         CHECK(std::string(vqh_last_error()) == "Invalid parameter: k must be greater than 0");
+        // an OPQ without codebooks (no outer iteration) writes zeros, whatever the caller's arrays held
+        CHECK(vqh_opq_fit(flat.data(), (int64_t)n, (int64_t)dim, 3, 4, 2, 0, 1, 0.0, 0, nullptr, nullptr, 0, &obj) == 0);
+        std::fill(codes.begin(), codes.end(), 0xAB);
+        CHECK(vqh_encode(obj, flat.data(), (int64_t)n, (int64_t)dim, codes.data()) == 0);
+        CHECK(codes == std::vector<uint8_t>(n * 3, 0));
+        std::vector<uint16_t> codes16(n * 3, 0xABAB);
+        CHECK(vqh_encode16(obj, flat.data(), (int64_t)n, (int64_t)dim, codes16.data()) == 0);
+        CHECK(codes16 == std::vector<uint16_t>(n * 3, 0));
+        vqh_free(obj);
         void *tr = nullptr;
         CHECK(vqh_tsvq_new(flat.data(), (int64_t)n, (int64_t)dim, 2, 2, 0.0, &tr) == 0);
         std::vector<int32_t> leaves(n);

@@ -625,8 +625,9 @@ public:
         encode_into(vectors, codes.data());
         return codes;
     }
-    // n x m bytes (k <= 256) into the caller's array
+    // n x m bytes (k <= 256) into the caller's array; zeros when fit ran no outer iteration
     void encode_into(const Rows &vectors, uint8_t *codes) const {
+        if (!trained_) std::fill_n(codes, vectors.size() * m_, uint8_t{0});
         if (vectors.empty() || !trained_) return;
         vectors.expect_dim(dim_);
         if (k_ <= 256 && vq_pq_quantize_host) {

@@ -216,7 +216,7 @@ int vqh_encode(void *obj, const float *x, int64_t n, int64_t dim, uint8_t *codes
     });
 }
 
-// the same 16 bits wide: any k up to 65536
+// the same 16 bits wide: any k up to 65536 (zeros, too, from an OPQ whose fit ran no outer iteration)
 int vqh_encode16(void *obj, const float *x, int64_t n, int64_t dim, uint16_t *codes) {
     return guarded([&] {
         Obj *o = (Obj *)obj;
@@ -224,7 +224,10 @@ int vqh_encode16(void *obj, const float *x, int64_t n, int64_t dim, uint16_t *co
         std::vector<uint16_t> c;
         switch (o->kind) {
         case 1: c = o->pq->encode16(rows); break;
-        case 2: c = o->opq->encode16(rows); break;
+        case 2:
+            c = o->opq->encode16(rows);
+            c.resize(rows.size() * o->opq->m());
+            break;
         case 3: o->rvq->quantize_batch_flat(rows, nullptr, &c); break;
         default: throw vq::VqError::InvalidParameter("TSVQ has leaves, not codes");
         }
