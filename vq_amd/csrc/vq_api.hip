@@ -11,13 +11,10 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
-#include <atomic>
 #include <mutex>
-#include <thread>
 #include <vector>
 
 #include "ctx.hpp"
-#include "host_batch.hpp"
 #include "assign_exact.hpp"
 #include "assign_mfma.hpp"
 
@@ -885,32 +882,6 @@ int32_t vq_host_free(vq_ctx *ctx, void *h_ptr) {
     if (!h_ptr) return VQ_OK;
     VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
     VQ_HIP(ctx, hipHostFree(h_ptr));
-    return VQ_OK;
-}
-
-// Copies of pageable memory from here on go through the staging buffers and threads of the context: the
-// runtime's own path copies on one thread (5 MB up: 0.25 -> 0.15 ms; 512 MB: 17-29 -> 9.6 ms).
-static constexpr size_t kStagedCopy = 1u << 20;
-static bool pageable(const void *h) {
-    hipPointerAttribute_t attr;
-    const bool locked = hipPointerGetAttributes(&attr, h) == hipSuccess && attr.type == hipMemoryTypeHost;
-    (void)hipGetLastError();  // an unregistered host pointer is reported as an error: that is the pageable case
-    return !locked;
-}
-
-int32_t vq_h2d(vq_ctx *ctx, void *d_dst, const void *h_src, size_t bytes) {
-    if (!ctx || (bytes && (!d_dst || !h_src))) return VQ_ERR_INVALID_ARG;
-    if (bytes >= kStagedCopy && pageable(h_src)) return staged_copy(ctx, d_dst, const_cast<void *>(h_src), bytes, true);
-    VQ_HIP(ctx, hipMemcpyAsync(d_dst, h_src, bytes, hipMemcpyHostToDevice, ctx->stream));
-    VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return VQ_OK;
-}
-
-int32_t vq_d2h(vq_ctx *ctx, void *h_dst, const void *d_src, size_t bytes) {
-    if (!ctx || (bytes && (!h_dst || !d_src))) return VQ_ERR_INVALID_ARG;
-    if (bytes >= kStagedCopy && pageable(h_dst)) return staged_copy(ctx, const_cast<void *>(d_src), h_dst, bytes, false);
-    VQ_HIP(ctx, hipMemcpyAsync(h_dst, d_src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return VQ_OK;
 }
 

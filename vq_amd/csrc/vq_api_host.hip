@@ -1,4 +1,4 @@
-// libvqhip — batches of host rows (declared in include/vq_hip.h).
+// libvqhip — copies between host and device memory, batches of host rows (declared in include/vq_hip.h).
 #include <hip/hip_runtime.h>
 
 #include "ctx.hpp"
@@ -59,6 +59,7 @@ int32_t staged_copy(vq_ctx *ctx, void *d, void *h, size_t bytes, bool upload) {
     constexpr int NB = vq_ctx::kPipe;
     // chunks short enough that the first and the last, which nothing overlaps, cost little
     const size_t chunk = std::min<size_t>(4u << 20, std::max<size_t>(512u << 10, up256(bytes / 8)));
+    VQ_HIP(ctx, hipSetDevice(ctx->device));  // the pipeline's streams and events are made on the current device
     VQ_TRY(ensure_pipe(ctx));
     VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));  // the data is there, the staging memory is idle
     VQ_TRY(ensure_pinned(ctx, ctx->pipe_pin, ctx->pipe_pin_cap, NB * chunk));
@@ -254,7 +255,33 @@ int32_t host_batch(vq_ctx *ctx, const float *h_x, int64_t n, size_t row_in, cons
 
 using namespace vqh;
 
+// Copies of pageable memory from here on go through the staging buffers and threads of the context: the
+// runtime's own path copies on one thread (5 MB up: 0.25 -> 0.15 ms; 512 MB: 17-29 -> 9.6 ms).
+static constexpr size_t kStagedCopy = 1u << 20;
+static bool pageable(const void *h) {
+    hipPointerAttribute_t attr;
+    const bool locked = hipPointerGetAttributes(&attr, h) == hipSuccess && attr.type == hipMemoryTypeHost;
+    (void)hipGetLastError();  // an unregistered host pointer is reported as an error: that is the pageable case
+    return !locked;
+}
+
 extern "C" {
+
+int32_t vq_h2d(vq_ctx *ctx, void *d_dst, const void *h_src, size_t bytes) {
+    if (!ctx || (bytes && (!d_dst || !h_src))) return VQ_ERR_INVALID_ARG;
+    if (bytes >= kStagedCopy && pageable(h_src)) return staged_copy(ctx, d_dst, const_cast<void *>(h_src), bytes, true);
+    VQ_HIP(ctx, hipMemcpyAsync(d_dst, h_src, bytes, hipMemcpyHostToDevice, ctx->stream));
+    VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return VQ_OK;
+}
+
+int32_t vq_d2h(vq_ctx *ctx, void *h_dst, const void *d_src, size_t bytes) {
+    if (!ctx || (bytes && (!h_dst || !d_src))) return VQ_ERR_INVALID_ARG;
+    if (bytes >= kStagedCopy && pageable(h_dst)) return staged_copy(ctx, const_cast<void *>(d_src), h_dst, bytes, false);
+    VQ_HIP(ctx, hipMemcpyAsync(h_dst, d_src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return VQ_OK;
+}
 
 int32_t vq_pq_quantize_host(vq_ctx *ctx, int32_t metric, const float *h_x, int64_t n, int32_t m, int32_t sub_dim, int32_t k,
                             const float *d_codebooks, const float *d_rotation, void *h_codes, uint16_t *h_out) {
