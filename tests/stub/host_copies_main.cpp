@@ -152,6 +152,13 @@ int main() {
     for (size_t bytes : {(size_t)(1u << 20) - 1, (size_t)(1u << 20), (size_t)(1u << 20) + 1, (size_t)(4u << 20) + 4096,
                          (size_t)5000003, (size_t)(70u << 20) + 13})
         copy_there_and_back(first, bytes);
+    // a large copy is few transfers: the copy engine stands still between two of them
+    {
+        std::vector<uint8_t> h(130u << 20, 7), d(h.size());
+        const int n0 = cpu_hip::copies;
+        CHECK(vq_h2d(first, d.data(), h.data(), h.size()) == VQ_OK && d == h);
+        CHECK(cpu_hip::copies - n0 <= 9);
+    }
     // page-locked memory goes to the copy engine as it is
     void *pin = nullptr;
     CHECK(hipHostMalloc(&pin, 2u << 20, hipHostMallocDefault) == hipSuccess);
