@@ -127,10 +127,11 @@ int32_t vq_host_alloc(vq_ctx *ctx, size_t bytes, void **h_ptr);
 int32_t vq_host_free(vq_ctx *ctx, void *h_ptr);
 /* Synchronous copies (they synchronise the context's stream). Replaces the per-vector heap
  * layout `&[Vector<f32>]` (src/vector.rs:150-152): the host packs rows into one buffer.
- * vq_h2d of 1 MiB or more from pageable memory is staged by the library: the caller and up to seven
- * host threads that the context keeps copy chunks into its page-locked buffers while the copy engine
- * uploads the chunk before (about 50 GB/s instead of 18-29 for one plain copy; a page-locked source goes
- * up directly); vq_d2h into pageable memory does the same in the other direction. */
+ * vq_h2d of 16 MiB or more from pageable memory is staged by the library: the caller, from 64 MiB on with
+ * up to seven host threads that the context keeps, copies chunks into its page-locked buffers while the
+ * copy engine uploads the chunk before (512 MB at 53 GB/s instead of 18-29 for one plain copy; a
+ * page-locked source goes up directly); vq_d2h of 4 MiB or more into pageable memory does the same in the
+ * other direction. */
 int32_t vq_h2d(vq_ctx *ctx, void *d_dst, const void *h_src, size_t bytes);
 int32_t vq_d2h(vq_ctx *ctx, void *h_dst, const void *d_src, size_t bytes);
 

@@ -139,19 +139,29 @@ int main() {
     // a context whose device is not the calling thread's current one: the first staged copy makes the
     // streams and events of its pipeline, and they have to be its own device's
     (void)hipSetDevice(0);
-    copy_there_and_back(second, (3u << 20) + 5);
+    copy_there_and_back(second, (17u << 20) + 5);
     CHECK(second->up && second->up->device == 1 && second->down->device == 1 && second->pipe_up[0]->device == 1);
     (void)hipSetDevice(0);
     batch(second, 30000, 16, 8, 200, false, true, true);
     std::thread other([&] {  // a thread's current device is 0 at its start
-        copy_there_and_back(second, (2u << 20) + 77);
+        copy_there_and_back(second, (18u << 20) + 77);
     });
     other.join();
 
     // around the limits of the staged copies and the chunks; above 64 MB with the copying threads
-    for (size_t bytes : {(size_t)(1u << 20) - 1, (size_t)(1u << 20), (size_t)(1u << 20) + 1, (size_t)(4u << 20) + 4096,
-                         (size_t)5000003, (size_t)(70u << 20) + 13})
+    for (size_t bytes : {(size_t)(4u << 20) - 1, (size_t)(4u << 20), (size_t)(4u << 20) + 1, (size_t)5000003,
+                         (size_t)(16u << 20) - 1, (size_t)(16u << 20), (size_t)(16u << 20) + 4097, (size_t)(70u << 20) + 13})
         copy_there_and_back(first, bytes);
+    // uploads below 16 MiB and downloads below 4 MiB are the runtime's: one transfer
+    for (int mb : {1, 3, 5, 15, 16, 20}) {
+        std::vector<uint8_t> h((size_t)mb << 20, 9), d(h.size());
+        int n0 = cpu_hip::copies;
+        CHECK(vq_h2d(first, d.data(), h.data(), h.size()) == VQ_OK && d == h);
+        CHECK((cpu_hip::copies - n0 == 1) == (mb < 16));
+        n0 = cpu_hip::copies;
+        CHECK(vq_d2h(first, h.data(), d.data(), h.size()) == VQ_OK);
+        CHECK((cpu_hip::copies - n0 == 1) == (mb < 4));
+    }
     // a large copy is few transfers: the copy engine stands still between two of them
     {
         std::vector<uint8_t> h(130u << 20, 7), d(h.size());
@@ -161,11 +171,11 @@ int main() {
     }
     // page-locked memory goes to the copy engine as it is
     void *pin = nullptr;
-    CHECK(hipHostMalloc(&pin, 2u << 20, hipHostMallocDefault) == hipSuccess);
-    std::vector<uint8_t> dev(2u << 20);
-    std::memset(pin, 0x5A, 2u << 20);
+    CHECK(hipHostMalloc(&pin, 20u << 20, hipHostMallocDefault) == hipSuccess);
+    std::vector<uint8_t> dev(20u << 20);
+    std::memset(pin, 0x5A, dev.size());
     const int before = cpu_hip::copies;
-    CHECK(vq_h2d(first, dev.data(), pin, dev.size()) == VQ_OK && dev == std::vector<uint8_t>(2u << 20, 0x5A));
+    CHECK(vq_h2d(first, dev.data(), pin, dev.size()) == VQ_OK && dev == std::vector<uint8_t>(dev.size(), 0x5A));
     CHECK(cpu_hip::copies == before + 1);
     (void)hipHostFree(pin);
 
@@ -196,7 +206,7 @@ int main() {
 
     // a copy or a computation that fails half way: an error, nothing left running, the context as before
     for (int at : {1, 3, 7}) {
-        const std::vector<uint8_t> h = pattern(9u << 20, 1);
+        const std::vector<uint8_t> h = pattern(20u << 20, 1);
         std::vector<uint8_t> d(h.size());
         cpu_hip::copies = 0;
         cpu_hip::fail_copy_at = at;
@@ -212,7 +222,7 @@ int main() {
         CHECK(vq_pq_quantize_host(first, VQ_EUCLIDEAN, x.data(), 58000, 16, 8, 256, &book, nullptr, c.data(), nullptr) ==
               VQ_ERR_UNSUPPORTED);
         fail_run_at = 0;
-        copy_there_and_back(first, 6u << 20);
+        copy_there_and_back(first, 17u << 20);
         batch(first, 20000, 16, 8, 256, false, true, true);
     }
 

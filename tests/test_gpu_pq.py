@@ -473,7 +473,7 @@ def test_failures_forced_from_the_host_come_back_as_status_codes(ctx):
 
 @pytest.mark.parametrize("nbytes", [(64 << 20) - 4, 64 << 20, (64 << 20) + 4, (150 << 20) + 12345 * 4])
 def test_large_upload_from_pageable_memory_is_exact(ctx, nbytes):
-    """vq_h2d stages a pageable source of 64 MiB or more through page-locked chunks with several host
+    """vq_h2d stages a large pageable source through page-locked chunks, from 64 MB on with several host
     threads: every byte must arrive, whatever the size relative to the chunks and the threads' slices."""
     n = nbytes // 4
     x = np.random.default_rng(nbytes % 997).integers(0, 2 ** 31, n, dtype=np.int64).astype(np.uint32).view(F)

@@ -257,9 +257,12 @@ int32_t host_batch(vq_ctx *ctx, const float *h_x, int64_t n, size_t row_in, cons
 
 using namespace vqh;
 
-// Copies of pageable memory from here on go through the staging buffers and threads of the context: the
-// runtime's own path copies on one thread (5 MB up: 0.25 -> 0.15 ms; 512 MB: 17-29 -> 9.6 ms).
-static constexpr size_t kStagedCopy = 1u << 20;
+// Copies of pageable memory from here on go through the staging buffers of the context, below them through
+// the runtime's own path.  Up, rows that the caller has just written (an array not touched for long in
+// brackets): 5 MB 0.16 ms by the runtime, 0.24 staged, 12 MB 0.34 and 0.38 (0.43 and 0.40), 20 MB 0.55 and
+// 0.56 (0.75 and 0.61), 100 MB 3.5 and 2.5; down: 3 MB 0.17 and 0.18, 5 MB 0.28 and 0.25, 12 MB 0.67 and
+// 0.39, 100 MB 5.9 and 2.3.
+static constexpr size_t kStagedUp = 16u << 20, kStagedDown = 4u << 20;
 static bool pageable(const void *h) {
     hipPointerAttribute_t attr;
     const bool locked = hipPointerGetAttributes(&attr, h) == hipSuccess && attr.type == hipMemoryTypeHost;
@@ -271,7 +274,7 @@ extern "C" {
 
 int32_t vq_h2d(vq_ctx *ctx, void *d_dst, const void *h_src, size_t bytes) {
     if (!ctx || (bytes && (!d_dst || !h_src))) return VQ_ERR_INVALID_ARG;
-    if (bytes >= kStagedCopy && pageable(h_src)) return staged_copy(ctx, d_dst, const_cast<void *>(h_src), bytes, true);
+    if (bytes >= kStagedUp && pageable(h_src)) return staged_copy(ctx, d_dst, const_cast<void *>(h_src), bytes, true);
     VQ_HIP(ctx, hipMemcpyAsync(d_dst, h_src, bytes, hipMemcpyHostToDevice, ctx->stream));
     VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return VQ_OK;
@@ -279,7 +282,7 @@ int32_t vq_h2d(vq_ctx *ctx, void *d_dst, const void *h_src, size_t bytes) {
 
 int32_t vq_d2h(vq_ctx *ctx, void *h_dst, const void *d_src, size_t bytes) {
     if (!ctx || (bytes && (!h_dst || !d_src))) return VQ_ERR_INVALID_ARG;
-    if (bytes >= kStagedCopy && pageable(h_dst)) return staged_copy(ctx, const_cast<void *>(d_src), h_dst, bytes, false);
+    if (bytes >= kStagedDown && pageable(h_dst)) return staged_copy(ctx, const_cast<void *>(d_src), h_dst, bytes, false);
     VQ_HIP(ctx, hipMemcpyAsync(h_dst, d_src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return VQ_OK;
