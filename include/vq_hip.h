@@ -75,6 +75,12 @@ void *vq_ctx_stream(vq_ctx *ctx);
  * Both give bit-identical codes; the switch exists for measurement and tests. */
 int32_t vq_ctx_set_assign_path(vq_ctx *ctx, int32_t path);
 
+/* Which kernels take an encode or a descent of a few rows (up to 512 (row, column block) pairs):
+ *   0 (default)  one workgroup per pair or row in one launch, where that is the faster way
+ *   1            the kernels of longer calls
+ * Both give the reference's results bit for bit; the switch exists for measurement and tests. */
+int32_t vq_ctx_set_few_path(vq_ctx *ctx, int32_t path);
+
 /* How vq_tsvq_build sums a node's squared deviations per dimension in row order (src/tsvq.rs:88-99)
  * when dim is a multiple of 8:
  *   0 (default)  groups of 32 squares as integer maps on the running sum, composed by a scan, with

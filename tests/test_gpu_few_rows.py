@@ -6,6 +6,7 @@ import pytest
 
 from oracle import oracle as O
 from tests import data
+from tests.test_gpu_wide_bound import _case
 
 pytestmark = pytest.mark.gpu
 F = np.float32
@@ -40,6 +41,33 @@ def test_assign_few(ctx, metric, n, m, sd, k):
         codes8 = ctx.empty((n * m + 3,), np.uint8)
         ctx.assign(metric, ctx.to_device(x), n, m * sd, m, sd, k, ctx.to_device(cb), codes8)
         assert np.array_equal(codes8.download()[:n * m].reshape(n, m), want.astype(np.uint8))
+
+
+@pytest.mark.parametrize("kind", ["collapsed", "near_ties", "grid", "spread", "overflow", "tiny", "offset", "edges"])
+@pytest.mark.parametrize("n,m,sd,k", [(130, 1, 264, 31), (64, 2, 33, 60), (60, 8, 8, 256), (500, 1, 128, 100), (24, 2, 16, 500)])
+def test_few_path_against_the_kernels_of_longer_calls(ctx, n, m, sd, k, kind):
+    """Values at the ends of the range, near ties, non-finite rows and centroids: the one-launch kernels give the
+    codes that the kernels of longer calls give, under the four metrics and in a residual encode."""
+    x, cb = _case(kind, n, m, sd, k)
+    dx, dcb = ctx.to_device(x), ctx.to_device(cb)
+    for metric in METRICS:
+        got = []
+        for path in (0, 1):
+            ctx.set_few_path(path)
+            try:
+                codes = ctx.empty((n, m), np.uint16)
+                ctx.assign_u16(metric, dx, n, m * sd, m, sd, k, dcb, codes)
+                got.append([codes.download()])
+                if m > 1 and k <= 256:  # the column blocks' codebooks as the stages of one block
+                    rows = ctx.to_device(np.ascontiguousarray(x[:, :sd]))
+                    rcodes, used, rec = ctx.empty((n, m), np.uint8), ctx.empty(n, np.uint8), ctx.empty((n, sd), np.uint16)
+                    ctx.rvq_encode(metric, rows, n, sd, sd, m, k, dcb, 0.5, rcodes, used, rec)
+                    # (a NaN has many bit patterns)
+                    f = rec.download()
+                    got[-1] += [rcodes.download(), used.download(), np.where((f & 0x7FFF) > 0x7C00, 0x7E00, f)]
+            finally:
+                ctx.set_few_path(0)
+        assert all(np.array_equal(a, b) for a, b in zip(*got)), (metric, kind)
 
 
 @pytest.mark.parametrize("metric", METRICS)

@@ -21,6 +21,7 @@ KINDS = ["normal", "uniform", "grid", "offset", "mixture", "dupcb", "tiny", "hug
 def ctx():
     import vq_amd
     c = vq_amd.Context(0)
+    c.set_few_path(1)  # short calls, too, by the kernels named here (test_gpu_few_rows.py has the others)
     yield c
     c.close()
 

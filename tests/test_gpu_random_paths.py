@@ -20,6 +20,7 @@ N_CASES = int(os.environ.get("VQ_PARITY_CASES", "40"))
 def ctx():
     import vq_amd
     c = vq_amd.Context(0)
+    c.set_few_path(1)  # short calls, too, by the kernels named here (test_gpu_few_rows.py has the others)
     yield c
     c.close()
 

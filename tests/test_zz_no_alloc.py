@@ -16,6 +16,7 @@ F = np.float32
 def ctx():
     import vq_amd
     c = vq_amd.Context(0)
+    c.set_few_path(1)  # short calls, too, by the kernels that use the scratch (test_gpu_few_rows.py has the others)
     yield c
     c.close()
 

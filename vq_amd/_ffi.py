@@ -27,6 +27,7 @@ SYMBOLS = {
     "vq_ctx_sync": (_i32, [_vp]),
     "vq_ctx_stream": (_vp, [_vp]),
     "vq_ctx_set_assign_path": (_i32, [_vp, _i32]),
+    "vq_ctx_set_few_path": (_i32, [_vp, _i32]),
     "vq_ctx_set_tsvq_variance_path": (_i32, [_vp, _i32]),
     "vq_calibrate": (_i32, [_vp, _i32, C.POINTER(C.c_double)]),
     "vq_ctx_set_procrustes_path": (_i32, [_vp, _i32]),
@@ -242,6 +243,10 @@ class Context:
     def set_assign_path(self, path):
         """0 = matrix cores + exact re-check (default), 1 = vector ALU only."""
         self._check(_lib.vq_ctx_set_assign_path(self._h, path))
+
+    def set_few_path(self, path):
+        """0 = a few rows in one launch (default), 1 = by the kernels of longer calls."""
+        self._check(_lib.vq_ctx_set_few_path(self._h, path))
 
     def calibrate(self, what):
         """Measured peak: 0 copy GB/s (read + write); 1-5 wave64 instructions per second of

@@ -57,6 +57,7 @@ struct vq_ctx {
     int mfma_stat_cur = 0;       // which of the two sets of counters in mfma_stat the last pass used
     int recheck_src = 0;         // where the last pass counted its undecided pairs: 1 mfma_stat, 2 mfma_list, 3 the fixed scratch
     int assign_path = 0;         // 0 = matrix cores where a kernel exists, 1 = vector ALU only
+    int few_path = 0;            // 0 = a few rows in one launch, 1 = by the kernels of longer calls
     bool lbg_small_lds_set = false;  // dynamic-LDS limit granted to k_lbg_update_small
     int compute_units = 0;       // of the context's GPU (0: not asked for yet)
     int decode_lds_set[4] = {0, 0, 0, 0};  // dynamic-LDS limit already granted to the four resident decode kernels
@@ -228,7 +229,7 @@ template <typename CodeT>
 int32_t assign_few(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
                    const float *d_codebooks, CodeT *d_codes, uint16_t *d_out16);
 inline bool assign_few_applicable(const vq_ctx *ctx, int64_t n, int32_t m, int32_t sd) {
-    return ctx->assign_path == 0 && n * m <= kFewPairs && sd <= 8192;
+    return ctx->assign_path == 0 && ctx->few_path == 0 && n * m <= kFewPairs && sd <= 8192;
 }
 // Whether the assignment of these rows (one column block of sd floats) runs on the pass that can
 // take a pending update along.

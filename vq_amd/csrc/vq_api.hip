@@ -1011,6 +1011,12 @@ int32_t vq_ctx_set_assign_path(vq_ctx *ctx, int32_t path) {
     return VQ_OK;
 }
 
+int32_t vq_ctx_set_few_path(vq_ctx *ctx, int32_t path) {
+    if (!ctx || (path != 0 && path != 1)) return VQ_ERR_INVALID_ARG;
+    ctx->few_path = path;
+    return VQ_OK;
+}
+
 int32_t vq_ctx_last_recheck_count(vq_ctx *ctx, uint32_t *h_count) {
     if (!ctx || !h_count) return VQ_ERR_INVALID_ARG;
     uint32_t all = 0, two = 0;

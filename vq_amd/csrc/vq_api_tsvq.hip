@@ -701,6 +701,11 @@ int32_t vq_ctx_set_tsvq_descend_path(vq_ctx *ctx, int32_t path) {
     return VQ_OK;
 }
 
+// Whether a descent of n rows runs as k_tsvq_few.
+static bool few_applicable(const vq_ctx *ctx, int64_t n, int32_t dim) {
+    return ctx->few_path == 0 && n <= kFewPairs && dim <= 4096;
+}
+
 static int32_t descend_few(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, const vq_tree *tree,
                            int32_t *d_leaf, uint16_t *d_out) {
     const size_t lds = sizeof(float) * 3 * ((size_t)tree->dim + 1);
@@ -727,7 +732,7 @@ int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n
     if (ld < tree->dim)
         return fail(ctx, VQ_ERR_DIM_MISMATCH, "Dimension mismatch: expected %d, got %lld", tree->dim, (long long)ld);
     VQ_HIP(ctx, hipSetDevice(ctx->device));
-    if (n <= kFewPairs && tree->dim <= 4096) return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
+    if (few_applicable(ctx, n, tree->dim)) return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
     // rows in registers: dim a multiple of 32 up to 128, 16-byte aligned rows
     if (tree->dim % 32 == 0 && tree->dim <= 128 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0) {
         // one workgroup per compute unit (the staged centroids fill its LDS), walking over the rows
@@ -808,7 +813,7 @@ int32_t vq_tsvq_quantize_host(vq_ctx *ctx, int32_t metric, const float *h_x, int
     return host_batch(ctx, h_x, n, sizeof(float) * (size_t)dim, outs, 4u << 20, true,
                       [&](const float *d_x, int64_t rows, void *d_out, void *d_leaf) -> int32_t {
                           uint16_t *out = h_out ? (uint16_t *)d_out : nullptr;
-                          if (rows <= kFewPairs && dim <= 4096)
+                          if (few_applicable(ctx, rows, dim))
                               return descend_few(ctx, metric, d_x, rows, dim, tree, (int32_t *)d_leaf, out);
                           VQ_TRY(vq_tsvq_descend(ctx, metric, d_x, rows, dim, tree, (int32_t *)d_leaf));
                           return out ? vq_tsvq_decode_f16(ctx, tree, (const int32_t *)d_leaf, rows, out) : VQ_OK;
