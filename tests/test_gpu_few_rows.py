@@ -95,6 +95,22 @@ def test_tsvq_few(ctx, metric, n, dim, depth):
     assert np.array_equal(leaf.download(), O.tsvq_descend(metric, q, t))
 
 
+@pytest.mark.parametrize("metric", METRICS)
+@pytest.mark.parametrize("dim,depth", [(32, 8), (128, 9)])
+def test_tsvq_rows_on_both_sides_of_the_lines(ctx, metric, dim, depth):
+    """Row widths that fit registers: which kernel takes a few rows depends on their number and the tree's size."""
+    rng = np.random.default_rng(dim)
+    x = np.round(rng.standard_normal((3000, dim)) * 2).astype(F)  # ties
+    dx = ctx.to_device(x)
+    tree = ctx.tsvq_build(dx, len(x), dim, dim, depth)
+    assert (tree.n_nodes <= 511) == (depth == 8)
+    want = O.tsvq_descend(metric, x[:513], tree.download())
+    for n in (1, 64, 65, 256, 257, 384, 385, 512, 513):
+        leaf = ctx.empty(n, np.int32)
+        ctx.tsvq_descend(metric, dx, n, dim, tree, leaf)
+        assert np.array_equal(leaf.download(), want[:n]), n
+
+
 @pytest.mark.parametrize("n", [1, 5, 100, 2048, 2049, 8192, 33_001, 140_003])
 def test_host_batches(n):
     from vq_amd import api

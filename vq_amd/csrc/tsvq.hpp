@@ -1810,7 +1810,8 @@ __global__ void __launch_bounds__(512) k_tsvq_descend_w(const float *__restrict_
 // TSVQNode::quantize_with_distance (src/tsvq.rs:162-181) for a few rows: one wave per row, which brings
 // both children's centroids of a node into LDS with whole-line loads; lane 0 adds up the left distance
 // and lane 1 the right one, each in the reference's order.  out16 (nullable): the leaf's centroid.
-// (A lane of k_tsvq_descend reads its centroids alone, and k_tsvq_descend_w stages 134 KB first.)
+// (A lane of k_tsvq_descend reads its centroids alone; where the kernels that hold rows in registers are
+// faster, regs_rows says up to how many rows.)
 template <int METRIC>
 __global__ void __launch_bounds__(64) k_tsvq_few(const float *__restrict__ x, int64_t ld, int dim,
                                                  const float *__restrict__ cen, const float *__restrict__ cnorm,

@@ -706,6 +706,16 @@ static bool few_applicable(const vq_ctx *ctx, int64_t n, int32_t dim) {
     return ctx->few_path == 0 && n <= kFewPairs && dim <= 4096;
 }
 
+// Up to how many rows the kernels that hold rows in registers (regs; inner: by one inner product per node) are
+// faster than k_tsvq_few.  They walk a level in half the time, but the rows of a wave read the levels that are not
+// in LDS (beyond 255 inner nodes) one after the other.  128 floats, Euclidean: 511 nodes 64 rows 11.1 us against
+// 19.4, 384 17.0 and 20.2, 512 19.2 and 20.9 (31 nodes: 14.1 and 11.4); 8191 nodes 64 rows 20.7 and 27.9, 128
+// 27.3 and 28.0, 256 41.7 and 28.1; Manhattan, 32 floats, 511 nodes: 64 rows 6.8 and 8.5, 384 8.9 and 8.5.
+// k_tsvq_descend, one lane per row with its centroids read by that lane alone, is slower at every number of rows.
+static int64_t regs_rows(bool regs, bool inner, int32_t n_nodes) {
+    return !regs ? 0 : !inner ? 64 : n_nodes <= 511 ? 384 : n_nodes <= 1023 ? 256 : 160;
+}
+
 static int32_t descend_few(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, const vq_tree *tree,
                            int32_t *d_leaf, uint16_t *d_out) {
     const size_t lds = sizeof(float) * 3 * ((size_t)tree->dim + 1);
@@ -732,16 +742,19 @@ int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n
     if (ld < tree->dim)
         return fail(ctx, VQ_ERR_DIM_MISMATCH, "Dimension mismatch: expected %d, got %lld", tree->dim, (long long)ld);
     VQ_HIP(ctx, hipSetDevice(ctx->device));
-    if (few_applicable(ctx, n, tree->dim)) return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
     // rows in registers: dim a multiple of 32 up to 128, 16-byte aligned rows
-    if (tree->dim % 32 == 0 && tree->dim <= 128 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0) {
+    const bool regs = tree->dim % 32 == 0 && tree->dim <= 128 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;
+    // cosine and (squared) Euclidean: a step decided by one inner product with the node's vector,
+    // the two sums of the reference only where that cannot decide
+    const bool inner = ctx->tsvq_descend_path == 0 && metric >= VQ_SQEUCLIDEAN && metric <= VQ_COSINE;
+    if (n > regs_rows(regs, inner, tree->n_nodes) && few_applicable(ctx, n, tree->dim))
+        return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
+    if (regs) {
         // one workgroup per compute unit (the staged centroids fill its LDS), walking over the rows
         int cus = 0;
         VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
         dim3 g(std::min<unsigned>(cdiv(n, 512), (unsigned)std::max(cus, 1))), b(512);
-        // cosine and (squared) Euclidean: a step decided by one inner product with the node's vector,
-        // the two sums of the reference only where that cannot decide
-        if (ctx->tsvq_descend_path == 0 && metric != VQ_MANHATTAN && metric >= VQ_SQEUCLIDEAN && metric <= VQ_COSINE) {
+        if (inner) {
             const bool cosine = metric == VQ_COSINE;
             const float *wt = cosine ? tree->d_wcos : tree->d_wl2, *sc = cosine ? tree->d_sccos : tree->d_scl2;
 #define DESC_W(M, D)                                                                                   \
