@@ -218,7 +218,8 @@ int32_t vq_lbg_fit(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t
 
 /* d_codes[i*m + s] = first index j minimising metric(x_i[block s], codebook[s][j]), strict '<'.
  * Replaces the inline loops at src/pq.rs:166-174, src/opq.rs:155-163,250-258,
- * src/rvq.rs:116-124,189-197 (m = 1 there).  Asynchronous. */
+ * src/rvq.rs:116-124,189-197 (m = 1 there).  sub_dim up to 1280, here and in the training
+ * (VQ_ERR_UNSUPPORTED above).  Asynchronous. */
 int32_t vq_assign(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m,
                   int32_t sub_dim, int32_t k, const float *d_codebooks, uint8_t *d_codes);
 

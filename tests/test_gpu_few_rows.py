@@ -43,6 +43,27 @@ def test_assign_few(ctx, metric, n, m, sd, k):
         assert np.array_equal(codes8.download()[:n * m].reshape(n, m), want.astype(np.uint8))
 
 
+def test_the_widest_block_is_the_same_for_few_rows_and_many(ctx):
+    import vq_amd
+    rng = np.random.default_rng(3)
+    for sd in (1280, 1281):
+        x, cb = rng.standard_normal((600, sd)).astype(F), rng.standard_normal((1, 5, sd)).astype(F)
+        dx, dcb = ctx.to_device(x), ctx.to_device(cb)
+        for n in (1, 512, 600):
+            codes, wide, stages = ctx.empty((n,), np.uint8), ctx.empty((n,), np.uint16), ctx.empty((n, 1), np.uint8)
+            calls = [lambda: ctx.assign(O.MANHATTAN, dx, n, sd, 1, sd, 5, dcb, codes),
+                     lambda: ctx.assign_u16(O.MANHATTAN, dx, n, sd, 1, sd, 5, dcb, wide),
+                     lambda: ctx.rvq_encode(O.MANHATTAN, dx, n, sd, sd, 1, 5, dcb, 0.0, stages)]
+            for call, out in zip(calls, (codes, wide, stages)):
+                if sd == 1280:
+                    call()
+                    assert np.array_equal(out.download().reshape(n, 1), O.pq_encode(O.MANHATTAN, x[:n], cb))
+                else:
+                    with pytest.raises(vq_amd.VqError) as e:
+                        call()
+                    assert e.value.code == vq_amd._ffi.ERR_UNSUPPORTED
+
+
 @pytest.mark.parametrize("kind", ["collapsed", "near_ties", "grid", "spread", "overflow", "tiny", "offset", "edges"])
 @pytest.mark.parametrize("n,m,sd,k", [(130, 1, 264, 31), (64, 2, 33, 60), (60, 8, 8, 256), (500, 1, 128, 100), (24, 2, 16, 500)])
 def test_few_path_against_the_kernels_of_longer_calls(ctx, n, m, sd, k, kind):

@@ -252,6 +252,7 @@ int32_t launch_wide_exact(vq_ctx *ctx, const vq::AssignArgs &a, int sd, const ui
     if (listed) lds = std::max(lds, sizeof(float) * ((size_t)sd + vq::kPairWgLdsFloats));
     // ... or eight rows of a single column block per workgroup
     if (listed && a.m == 1) lds = std::max(lds, sizeof(float) * ((size_t)vq::kRowsWg * sd + vq::kRowsWgLdsFloats));
+    static_assert(sizeof(float) * 4 * vq::kWideRows * kFewWidth == 160 * 1024, "k_assign_few takes the same widths");
     if (lds > 160 * 1024) return fail(ctx, VQ_ERR_UNSUPPORTED, "sub_dim %d too large", sd);
     auto pick = [&](auto L, auto V) {
         constexpr bool LISTED = decltype(L)::value, VEC = decltype(V)::value;
