@@ -15,6 +15,8 @@ using namespace vqh;
 
 namespace {
 
+constexpr int64_t kSlicePairs = 16 << 20;  // pairs assigned chunk by chunk at a time
+
 template <int METRIC>
 void launch_merge(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int m, int sd, int k, const float *chunks,
                   int base, int count, const uint8_t *win, const float *win_d, int64_t stride, unsigned have_d,
@@ -43,49 +45,60 @@ int32_t assign_codes_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t 
         if (out_written) *out_written = d_out16 != nullptr;
         return assign_few<uint16_t>(ctx, metric, d_x, n, ld, m, sd, k, d_codebooks, d_codes, d_out16);
     }
-    const size_t pairs = (size_t)n * m;
-    // chunks merged by one launch: their winners lie side by side (20 bytes per pair for four)
-    const int chunks = (int)cdiv(k, vq::kChunk);
-    const int together = pairs <= ((size_t)256 << 20) ? std::min(chunks, vq::kMergeChunks) : 1;
-    const size_t stride = (pairs + 255) & ~(size_t)255;
-    VQ_TRY(ensure(ctx, ctx->big_win, stride * together));
-    uint8_t *win = (uint8_t *)ctx->big_win.p;
     if (k <= vq::kChunk) {  // one chunk: its winner is the answer
+        const size_t pairs = (size_t)n * m;
+        VQ_TRY(ensure(ctx, ctx->big_win, pairs));
+        uint8_t *win = (uint8_t *)ctx->big_win.p;
         VQ_TRY(assign_codes(ctx, metric, d_x, n, ld, m, sd, k, d_codebooks, win));
         hipLaunchKernelGGL(vq::k_widen_codes, dim3(cdiv((int64_t)pairs, 256)), dim3(256), 0, ctx->stream,
                            (const uint8_t *)win, (int64_t)pairs, d_codes);
         VQ_HIP(ctx, hipGetLastError());
         return VQ_OK;
     }
+    // The rows in slices of up to kSlicePairs (row, block) pairs: the chunks that one launch merges have their
+    // winners and distances side by side, 24 bytes per pair for four and the running minimum, and the
+    // workspace stays at 400 MB whatever n is (slices of half the size: 1,000,000 x 16 pairs, k = 1024 1.68 ->
+    // 1.71 ms, k = 2048 3.28 -> 3.34; 1,000,000 x 32 blocks of 2, k = 600: 4.22 -> 3.96).
+    const int chunks = (int)cdiv(k, vq::kChunk), together = std::min(chunks, vq::kMergeChunks);
+    const int64_t slice = std::min<int64_t>(n, std::max<int64_t>(1, kSlicePairs / m));
+    const size_t pairs = (size_t)slice * m, stride = (pairs + 255) & ~(size_t)255;
     VQ_TRY(ensure(ctx, ctx->big_chunk, sizeof(float) * (size_t)m * k * sd));
+    VQ_TRY(ensure(ctx, ctx->big_win, stride * together));
     if (chunks > together) VQ_TRY(ensure(ctx, ctx->big_best, sizeof(float) * pairs));
     VQ_TRY(ensure(ctx, ctx->big_wind, sizeof(float) * stride * together));
+    uint8_t *win = (uint8_t *)ctx->big_win.p;
     float *tables = (float *)ctx->big_chunk.p;
     float *best = (float *)ctx->big_best.p;
     float *wind = (float *)ctx->big_wind.p;
     hipLaunchKernelGGL(vq::k_chunk_tables, dim3(cdiv((int64_t)m * k * sd, 256)), dim3(256), 0, ctx->stream, d_codebooks,
                        m, k, sd, tables);
     VQ_HIP(ctx, hipGetLastError());
-    for (int c0 = 0; c0 < chunks; c0 += together) {
-        const int count = std::min(together, chunks - c0), base = c0 * vq::kChunk;
-        unsigned have = 0;
-        for (int c = 0; c < count; ++c) {
-            const int b0 = base + c * vq::kChunk, kc = std::min(vq::kChunk, k - b0);
-            // the winners' distances come with the codes where the assignment kernel computes them anyway
-            bool have_d = false;
-            VQ_TRY(assign_codes(ctx, metric, d_x, n, ld, m, sd, kc, tables + (size_t)b0 * m * sd, win + c * stride,
-                                wind + c * stride, &have_d));
-            if (have_d) have |= 1u << c;
-        }
-#define MERGE(M) launch_merge<M>(ctx, d_x, n, ld, m, sd, k, tables, base, count, win, wind, (int64_t)stride, have, best, d_codes)
-        switch (metric) {
-        case VQ_SQEUCLIDEAN: MERGE(vq::M_SQ); break;
-        case VQ_EUCLIDEAN: MERGE(vq::M_EUCLID); break;
-        case VQ_COSINE: MERGE(vq::M_COS); break;
-        default: MERGE(vq::M_L1); break;
-        }
+    for (int64_t r0 = 0; r0 < n; r0 += slice) {
+        const int64_t rows = std::min(slice, n - r0);
+        const float *x = d_x + r0 * ld;
+        uint16_t *codes = d_codes + r0 * m;
+        for (int c0 = 0; c0 < chunks; c0 += together) {
+            const int count = std::min(together, chunks - c0), base = c0 * vq::kChunk;
+            unsigned have = 0;
+            for (int c = 0; c < count; ++c) {
+                const int b0 = base + c * vq::kChunk, kc = std::min(vq::kChunk, k - b0);
+                // the winners' distances come with the codes where the assignment kernel computes them anyway
+                bool have_d = false;
+                VQ_TRY(assign_codes(ctx, metric, x, rows, ld, m, sd, kc, tables + (size_t)b0 * m * sd, win + c * stride,
+                                    wind + c * stride, &have_d));
+                if (have_d) have |= 1u << c;
+            }
+#define MERGE(M) \
+    launch_merge<M>(ctx, x, rows, ld, m, sd, k, tables, base, count, win, wind, (int64_t)stride, have, best, codes)
+            switch (metric) {
+            case VQ_SQEUCLIDEAN: MERGE(vq::M_SQ); break;
+            case VQ_EUCLIDEAN: MERGE(vq::M_EUCLID); break;
+            case VQ_COSINE: MERGE(vq::M_COS); break;
+            default: MERGE(vq::M_L1); break;
+            }
 #undef MERGE
-        VQ_HIP(ctx, hipGetLastError());
+            VQ_HIP(ctx, hipGetLastError());
+        }
     }
     return VQ_OK;
 }
