@@ -1,5 +1,5 @@
-"""What the context keeps after a call: the workspace of an assignment above 256 centroids does not grow with
-the number of rows."""
+"""What the context keeps after a call: a fit of padded column blocks gives its copy of the rows back, and
+the workspace of an assignment above 256 centroids does not grow with the number of rows."""
 import ctypes
 import time
 
@@ -36,6 +36,26 @@ def _held_at_most(before, limit):
             return True
         time.sleep(0.05)
     return False
+
+
+def test_padded_rows_of_a_fit_are_given_back(ctx):
+    n, m, sd, k, iters = 1_200_000, 64, 2, 64, 2  # 2.5 GB of padded copy for 614 MB of rows
+    rng = np.random.default_rng(1)
+    x = rng.random((n, m * sd), dtype=F)
+    init = np.stack([rng.permutation(n)[:k] for _ in range(m)]).astype(np.uint32)
+    reseed = rng.integers(0, n, (m, k * iters), dtype=np.uint32)
+    dx, out = ctx.to_device(x), []
+    for path in (0, 1):  # by the padded copy; by the kernels that take the rows as they are
+        cb = ctx.empty((m, k, sd), F)
+        ctx.set_assign_path(path)
+        before = _free()
+        ctx.lbg_fit(dx, n, m * sd, m, sd, k, iters, init, reseed, cb)
+        ctx.sync()
+        if path == 0:
+            # member lists, codes, part sums: 11 bytes per (row, block) pair at most
+            assert _held_at_most(before, 11 * n * m + 64 * MB)
+        out.append(cb.download())
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
 
 
 def test_rows_in_slices_above_256_centroids(ctx):

@@ -135,6 +135,16 @@ inline int32_t ensure(vq_ctx *ctx, DevBuf &b, size_t bytes) {
     return VQ_OK;
 }
 
+// Gives a workspace buffer back once nothing on the context's streams uses it.
+inline int32_t release(vq_ctx *ctx, DevBuf &b) {
+    if (!b.p) return VQ_OK;
+    VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (ctx->side) VQ_HIP(ctx, hipStreamSynchronize(ctx->side));
+    VQ_HIP(ctx, hipFree(b.p));
+    b = DevBuf();
+    return VQ_OK;
+}
+
 // Page-locked host memory of the context, grow-only (the device reads and writes it in place).
 inline int32_t ensure_pinned(vq_ctx *ctx, void *&p, size_t &cap, size_t bytes) {
     if (bytes <= cap) return VQ_OK;

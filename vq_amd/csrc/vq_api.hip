@@ -425,6 +425,9 @@ int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bo
     return sdp;
 }
 
+constexpr int64_t kPadSlice = 96 << 20;  // bytes of padded rows that an encode makes at a time
+constexpr size_t kPadKeep = 2u << 30;    // bytes that the context keeps of a fit's padded copy of its rows
+
 void launch_pad(vq_ctx *ctx, const float *x, int64_t n, int64_t ld, int m, int sd, int sdp, float *y) {
     hipLaunchKernelGGL(vq::k_pad_blocks, dim3(cdiv(n * m * (sdp / 4), 1024)), dim3(256), 0, ctx->stream, x, n, ld, m, sd,
                        sdp, y);
@@ -749,7 +752,7 @@ int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, i
     // padded a slice of rows at a time: the copy is read back from the memory-side cache (256 MB)
     // and the workspace stays small whatever n is
     const int64_t row_bytes = (int64_t)sizeof(float) * m * sdp;
-    const int64_t slice = std::min<int64_t>(n, std::max<int64_t>(4096, (96 << 20) / row_bytes / 4096 * 4096));
+    const int64_t slice = std::min<int64_t>(n, std::max<int64_t>(4096, kPadSlice / row_bytes / 4096 * 4096));
     VQ_TRY(ensure(ctx, ctx->pad_x, (size_t)(slice * row_bytes)));
     VQ_TRY(ensure(ctx, ctx->pad_cb, sizeof(float) * (size_t)m * k * sdp));
     launch_pad(ctx, d_codebooks, (int64_t)m * k, sd, 1, sd, sdp, (float *)ctx->pad_cb.p);
@@ -1128,22 +1131,25 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
     shape.cb = d_codebooks;
     const int sdp = max_iters > 0 ? pad_width(ctx, VQ_SQEUCLIDEAN, shape, sd, true) : 0;
     if (sdp && (int64_t)k * cdiv(n, vq::kPartRows) * sdp <= (1LL << 31)) {
-        // the rows padded once for all passes of the fit (a shape too large for a second copy of its
-        // rows trains on the rows as they are)
-        const size_t bytes = sizeof(float) * (size_t)n * m * sdp;
-        const int32_t rc = ensure(ctx, ctx->pad_x, bytes);
+        // the rows padded once for all passes of the fit (where the second copy of the rows and the fit's
+        // workspace do not fit together, it trains on the rows as they are: the same results)
+        int32_t rc = ensure(ctx, ctx->pad_x, sizeof(float) * (size_t)n * m * sdp);
+        if (rc == VQ_OK) rc = ensure(ctx, ctx->pad_cb, sizeof(float) * (size_t)m * k * sdp);
         if (rc == VQ_OK) {
-            VQ_TRY(ensure(ctx, ctx->pad_cb, sizeof(float) * (size_t)m * k * sdp));
             float *px = (float *)ctx->pad_x.p, *pcb = (float *)ctx->pad_cb.p;
             launch_pad(ctx, d_x, n, ld, m, sd, sdp, px);
-            const int32_t fit = lbg_fit_run(ctx, px, n, (int64_t)m * sdp, m, sdp, k, max_iters, h_init_idx,
-                                            h_reseed_stream, n_reseed, pcb, h_iters_run, h_reseeds_used, nullptr, nullptr,
-                                            [&] {
-                                                hipLaunchKernelGGL(vq::k_unpad_rows, dim3(cdiv((int64_t)m * k * sd, 256)),
-                                                                   dim3(256), 0, ctx->stream, (const float *)pcb,
-                                                                   (int64_t)m * k, sd, sdp, d_codebooks);
-                                            });
-            return fit;
+            rc = lbg_fit_run(ctx, px, n, (int64_t)m * sdp, m, sdp, k, max_iters, h_init_idx, h_reseed_stream, n_reseed,
+                             pcb, h_iters_run, h_reseeds_used, nullptr, nullptr, [&] {
+                                 hipLaunchKernelGGL(vq::k_unpad_rows, dim3(cdiv((int64_t)m * k * sd, 256)), dim3(256), 0,
+                                                    ctx->stream, (const float *)pcb, (int64_t)m * k, sd, sdp,
+                                                    d_codebooks);
+                             });
+        }
+        // a large copy is not held for later calls (taking 2.3 GB again costs a fit of 1,500,000 x 96 in
+        // blocks of 2 0.8 ms of 18)
+        if (rc == VQ_ERR_OOM || ctx->pad_x.cap > kPadKeep) {
+            const int32_t gone = release(ctx, ctx->pad_x);
+            if (rc == VQ_OK) rc = gone;
         }
         if (rc != VQ_ERR_OOM) return rc;
     }
