@@ -223,6 +223,37 @@ int32_t vq_procrustes_rotation(vq_ctx *, const double *A, int32_t dim, double *R
     return VQ_OK;
 }
 
+// host rows in, host results out: by the calls above on copies of exactly the size that the arrays have
+int32_t vq_pq_quantize_host(vq_ctx *c, int32_t metric, const float *x, int64_t n, int32_t m, int32_t sd, int32_t k,
+                            const float *cb, const float *R, void *codes, uint16_t *out) {
+    const int64_t dim = (int64_t)m * sd;
+    std::vector<float> rows(x, x + n * dim), turned(rows);
+    if (R) vq_rotate(c, rows.data(), n, dim, (int32_t)dim, R, turned.data());
+    const auto run = [&](auto *own) {
+        assign_any(turned.data(), n, dim, m, sd, k, cb, own, (int)sizeof(*own));
+        if (out) decode_any(own, n, m, sd, k, cb, out);
+        if (codes) std::memcpy(codes, own, sizeof(*own) * (size_t)(n * m));
+    };
+    if (k > 256)
+        run(std::vector<uint16_t>((size_t)(n * m)).data());
+    else
+        run(std::vector<uint8_t>((size_t)(n * m)).data());
+    (void)metric;
+    return VQ_OK;
+}
+int32_t vq_rvq_quantize_host(vq_ctx *, int32_t, const float *x, int64_t n, int32_t dim, int32_t stages, int32_t k,
+                             const float *cb, float, void *codes, uint16_t *out) {
+    const auto run = [&](auto *own) {
+        rvq_any(x, n, (int64_t)dim, dim, stages, k, cb, own, nullptr, out);
+        if (codes && stages) std::memcpy(codes, own, sizeof(*own) * (size_t)(n * stages));
+    };
+    if (k > 256)
+        run(std::vector<uint16_t>((size_t)(n * stages)).data());
+    else
+        run(std::vector<uint8_t>((size_t)(n * stages)).data());
+    return VQ_OK;
+}
+
 // a tree of depth min(max_depth, 1): the mean of all rows, and two children equal to the first and last row
 int32_t vq_tsvq_build(vq_ctx *, const float *x, int64_t n, int64_t ld, int32_t dim, int32_t max_depth, vq_tree **out) {
     vq_tree *t = new vq_tree();
@@ -283,6 +314,14 @@ int32_t vq_tsvq_decode_f16(vq_ctx *, const vq_tree *t, const int32_t *leaf, int6
         if (leaf[i] < 0 || leaf[i] >= t->n_nodes) std::abort();
         for (int d = 0; d < t->dim; ++d) out[i * t->dim + d] = (uint16_t)(leaf[i] + d);
     }
+    return VQ_OK;
+}
+int32_t vq_tsvq_quantize_host(vq_ctx *c, int32_t metric, const float *x, int64_t n, const vq_tree *t, int32_t *leaf,
+                              uint16_t *out) {
+    std::vector<int32_t> own((size_t)n);
+    vq_tsvq_descend(c, metric, x, n, t->dim, t, own.data());
+    if (out) vq_tsvq_decode_f16(c, t, own.data(), n, out);
+    if (leaf) std::memcpy(leaf, own.data(), sizeof(int32_t) * (size_t)n);
     return VQ_OK;
 }
 

@@ -3,7 +3,8 @@ vq_host_c.cpp) under -fsanitize=address,undefined WITHOUT a GPU: a C++ driver
 (tests/stub/host_sanitized_main.cpp) linked against a stand-in for libvqhip
 (tests/stub/vqhip_stub.cpp) whose "device" memory is host memory of exactly the size asked for.
 Packing of per-row vectors, validation and panic texts, index streams, the call sequences and
-buffer sizes of the four quantizers and the C flattening are host code; the kernels are not."""
+buffer sizes of the four quantizers and the C flattening are host code; the kernels are not.  (The library's
+own host code behind the calls that take host rows: test_host_copies.py.)"""
 import os
 import subprocess
 

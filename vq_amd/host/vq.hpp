@@ -33,12 +33,6 @@
 
 #include "../../include/vq_hip.h"
 
-// The calls that take host rows through the GPU in one go.  Weak: a host built against this header also
-// runs on a library without them (device buffers and one call per step then).
-#pragma weak vq_pq_quantize_host
-#pragma weak vq_rvq_quantize_host
-#pragma weak vq_tsvq_quantize_host
-
 namespace vq {
 
 // ---- errors (src/exceptions.rs) ----------------------------------------------------------------
@@ -263,10 +257,6 @@ public:
     DeviceBuffer<uint8_t> &narrow() { return b8_; }
     uint8_t *p8() const { return b8_.get(); }
     uint16_t *p16() const { return b16_.get(); }
-    std::vector<uint8_t> to_host8() const {
-        if (wide_) throw VqError::InvalidParameter("codes above 256 centroids are 16 bits wide");
-        return b8_.to_host();
-    }
     std::vector<uint16_t> to_host16() const {
         if (wide_) return b16_.to_host();
         const std::vector<uint8_t> v = b8_.to_host();
@@ -285,11 +275,6 @@ inline int32_t abi_assign(vq_ctx *c, int32_t metric, const float *x, size_t n, s
                                         cb, codes.p16())
                         : vq_assign(c, metric, x, (int64_t)n, (int64_t)ld, (int32_t)m, (int32_t)sd, (int32_t)k, cb,
                                     codes.p8());
-}
-inline int32_t abi_decode_f16(vq_ctx *c, const DeviceCodes &codes, size_t n, size_t m, size_t sd, size_t k,
-                              const float *cb, uint16_t *out) {
-    return codes.wide() ? vq_decode_f16_u16(c, codes.p16(), (int64_t)n, (int32_t)m, (int32_t)sd, (int32_t)k, cb, out)
-                        : vq_decode_f16(c, codes.p8(), (int64_t)n, (int32_t)m, (int32_t)sd, (int32_t)k, cb, out);
 }
 inline int32_t abi_decode_f32(vq_ctx *c, const DeviceCodes &codes, size_t n, size_t m, size_t sd, size_t k,
                               const float *cb, float *out) {
@@ -442,23 +427,11 @@ public:
 
     // ... into the caller's array
     void quantize_into(const Rows &vectors, uint16_t *out) const {
-        size_t dim = sub_dim_ * m_, n = vectors.size();
+        const size_t n = vectors.size();
         if (n == 0) return;
-        vectors.expect_dim(dim);
-        const float *flat = vectors.data();
-        if (vq_pq_quantize_host) {
-            dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), flat, (int64_t)n, (int32_t)m_,
-                                            (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(), nullptr, nullptr, out));
-            return;
-        }
-        DeviceBuffer<float> dx(dev_, n * dim);
-        dx.upload(flat, dx.size());
-        DeviceCodes dcodes(dev_, n * m_, k_);
-        DeviceBuffer<uint16_t> dout(dev_, n * dim);
-        dev_->check(abi_assign(dev_->ctx(), distance_.abi_metric(), dx.get(), n, dim, m_, sub_dim_, k_,
-                               codebooks_.get(), dcodes));
-        dev_->check(abi_decode_f16(dev_->ctx(), dcodes, n, m_, sub_dim_, k_, codebooks_.get(), dout.get()));
-        dout.download(out, n * dim);
+        vectors.expect_dim(sub_dim_ * m_);
+        dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)n, (int32_t)m_,
+                                        (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(), nullptr, nullptr, out));
     }
 
     // The integer codes the reference keeps only as `best_index` (src/pq.rs:166-174): n x m bytes
@@ -474,13 +447,10 @@ public:
         const size_t n = vectors.size();
         if (n == 0) return;
         vectors.expect_dim(sub_dim_ * m_);
-        if (k_ <= 256 && vq_pq_quantize_host) {
-            dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)n, (int32_t)m_,
-                                            (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(), nullptr, codes, nullptr));
-            return;
-        }
-        const std::vector<uint8_t> c = encode_device(vectors).to_host8();
-        std::copy(c.begin(), c.end(), codes);
+        const int32_t metric = distance_.abi_metric();
+        if (k_ > 256) throw VqError::InvalidParameter("codes above 256 centroids are 16 bits wide");
+        dev_->check(vq_pq_quantize_host(dev_->ctx(), metric, vectors.data(), (int64_t)n, (int32_t)m_, (int32_t)sub_dim_,
+                                        (int32_t)k_, codebooks_.get(), nullptr, codes, nullptr));
     }
 
     std::vector<float> codebooks() const { return codebooks_.to_host(); }  // m*k*sub_dim
@@ -607,16 +577,9 @@ public:
         if (n == 0) return;
         vectors.expect_dim(dim_);
         if (!trained_) return;
-        if (vq_pq_quantize_host) {
-            dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)n, (int32_t)m_,
-                                            (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(), d_rotation_.get(), nullptr,
-                                            out));
-            return;
-        }
-        DeviceCodes dcodes = encode_device(vectors);
-        DeviceBuffer<uint16_t> dout(dev_, n * dim_);
-        dev_->check(abi_decode_f16(dev_->ctx(), dcodes, n, m_, sub_dim_, k_, codebooks_.get(), dout.get()));
-        dout.download(out, n * dim_);
+        dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)n, (int32_t)m_,
+                                        (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(), d_rotation_.get(), nullptr,
+                                        out));
     }
 
     std::vector<uint8_t> encode(const Rows &vectors) const {
@@ -630,14 +593,10 @@ public:
         if (!trained_) std::fill_n(codes, vectors.size() * m_, uint8_t{0});
         if (vectors.empty() || !trained_) return;
         vectors.expect_dim(dim_);
-        if (k_ <= 256 && vq_pq_quantize_host) {
-            dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)vectors.size(),
-                                            (int32_t)m_, (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(),
-                                            d_rotation_.get(), codes, nullptr));
-            return;
-        }
-        const std::vector<uint8_t> c = encode_device(vectors).to_host8();
-        std::copy(c.begin(), c.end(), codes);
+        if (k_ > 256) throw VqError::InvalidParameter("codes above 256 centroids are 16 bits wide");
+        dev_->check(vq_pq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)vectors.size(),
+                                        (int32_t)m_, (int32_t)sub_dim_, (int32_t)k_, codebooks_.get(),
+                                        d_rotation_.get(), codes, nullptr));
     }
     std::vector<uint16_t> encode16(const Rows &vectors) const {  // any k
         if (vectors.empty() || !trained_) return {};
@@ -788,29 +747,9 @@ public:
         const size_t n = vectors.size();
         if (n == 0) return;
         vectors.expect_dim(dim_);
-        const float *flat = vectors.data();
         const int32_t k = (int32_t)std::max<size_t>(k_, 1);
-        if (vq_rvq_quantize_host) {
-            dev_->check(vq_rvq_quantize_host(dev_->ctx(), distance_.abi_metric(), flat, (int64_t)n, (int32_t)dim_,
-                                             (int32_t)stages_, k, codebooks_.get(), epsilon_, codes, out));
-            return;
-        }
-        DeviceBuffer<float> dx(dev_, n * dim_);
-        dx.upload(flat, dx.size());
-        DeviceCodes dcodes(dev_, std::max<size_t>(n * stages_, 1), k_);
-        DeviceBuffer<uint16_t> dout(dev_, n * dim_);
-        dev_->check(dcodes.wide()
-                        ? vq_rvq_encode_u16(dev_->ctx(), distance_.abi_metric(), dx.get(), (int64_t)n, (int64_t)dim_,
-                                            (int32_t)dim_, (int32_t)stages_, k, codebooks_.get(), epsilon_,
-                                            dcodes.p16(), nullptr, dout.get())
-                        : vq_rvq_encode(dev_->ctx(), distance_.abi_metric(), dx.get(), (int64_t)n, (int64_t)dim_,
-                                        (int32_t)dim_, (int32_t)stages_, k, codebooks_.get(), epsilon_, dcodes.p8(),
-                                        nullptr, dout.get()));
-        if (codes && stages_) {
-            const void *c = dcodes.wide() ? (const void *)dcodes.p16() : (const void *)dcodes.p8();
-            dev_->check(vq_d2h(dev_->ctx(), codes, c, n * stages_ * (dcodes.wide() ? 2 : 1)));
-        }
-        if (out) dout.download(out, n * dim_);
+        dev_->check(vq_rvq_quantize_host(dev_->ctx(), distance_.abi_metric(), vectors.data(), (int64_t)n, (int32_t)dim_,
+                                         (int32_t)stages_, k, codebooks_.get(), epsilon_, codes, out));
     }
 
     size_t stages() const { return stages_; }
@@ -915,21 +854,8 @@ public:
         size_t n = vectors.size();
         if (n == 0) return;
         vectors.expect_dim(dim_);
-        const float *flat = vectors.data();
-        if (vq_tsvq_quantize_host) {
-            dev_->check(vq_tsvq_quantize_host(dev_->ctx(), distance.abi_metric(), flat, (int64_t)n, tree_.get(), leaves, out));
-            return;
-        }
-        DeviceBuffer<float> dx(dev_, n * dim_);
-        dx.upload(flat, dx.size());
-        DeviceBuffer<int32_t> dleaf(dev_, n);
-        DeviceBuffer<uint16_t> dout(dev_, n * dim_);
-        dev_->check(vq_tsvq_descend(dev_->ctx(), distance.abi_metric(), dx.get(), (int64_t)n, (int64_t)dim_,
-                                    tree_.get(), dleaf.get()));
-        if (leaves) dleaf.download(leaves, n);
-        if (!out) return;
-        dev_->check(vq_tsvq_decode_f16(dev_->ctx(), tree_.get(), dleaf.get(), (int64_t)n, dout.get()));
-        dout.download(out, n * dim_);
+        dev_->check(vq_tsvq_quantize_host(dev_->ctx(), distance.abi_metric(), vectors.data(), (int64_t)n, tree_.get(),
+                                          leaves, out));
     }
 
     int32_t n_nodes() const {
