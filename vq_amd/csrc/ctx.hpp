@@ -41,7 +41,9 @@ struct vq_ctx {
     void *tsvq_pin = nullptr;    // TSVQ build: page-locked staging of a level's tables and decisions
     size_t tsvq_pin_cap = 0;
     // host rows on their way through the GPU (host_batch.hpp): page-locked and device slots of the chunks
-    // in flight, the streams and events that order them, the threads that copy
+    // in flight, the streams and events that order them, the threads that copy.  Held until the context is
+    // closed; four chunks and their results, so bounded: 64 MiB for copies, 25 MB for product quantizers and
+    // trees, 100 MB for residual quantizers (rows longer than a chunk: four rows)
     static constexpr int kPipe = 4;
     void *pipe_pin = nullptr;
     size_t pipe_pin_cap = 0;
@@ -235,9 +237,10 @@ int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, i
 // Up to this many (row, column block) pairs an assignment runs as one workgroup per pair, one launch
 // (k_assign_few): two rounds of workgroups; the matrix-core kernels take two to four launches.  The faster way
 // at every width, k and metric up to there, and the longer the codebook the more, although each workgroup
-// reads all of it.  32 rows of 16 blocks of 8 floats, k = 256, Euclidean: 4.1 us against 6.3; 512 rows of one block of
-// 128 floats, k = 256 10 and 20, 1024 floats, k = 256 59 and 78 (256 pairs: 32 and 79), k = 1024 227 and 1220; Manhattan, 1024 floats,
-// k = 256: 59 and 217; a residual encode of 512 x 1024, four stages: 232 and 426.
+// reads all of it.  32 rows of 16 blocks of 8 floats, k = 256, Euclidean: 4.1 us against 6.3;
+// 512 rows of one block of 128 floats, k = 256 10 and 20, 1024 floats, k = 256 59 and 78 (256 rows: 32 and 79),
+// k = 1024 227 and 1220; Manhattan, 1024 floats, k = 256: 59 and 217; a residual encode of 512 x 1024, four
+// stages: 232 and 426.
 constexpr int64_t kFewPairs = 512;
 constexpr int32_t kFewWidth = 1280;  // the widest block that the kernels of longer calls take, whatever the number of rows
 template <typename CodeT>

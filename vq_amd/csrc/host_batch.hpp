@@ -109,8 +109,10 @@ struct Chunks {
 
 // How many threads help the caller with `bytes`.  None below 64 MB: lines that other processors have read
 // or written have to be taken back from their caches when the caller's thread next touches them, which
-// cost it more (5 MB of rows written again after an upload by eight threads: 1.2 -> 3.1-4.6 ms) than the
-// help saved (50,000 x 128 rows quantized: 1.4 -> 0.9 ms).  Larger arrays do not stay in caches.
+// costs it about what the help saves (50,000 x 128 rows quantized: 1.62 -> 0.94 ms, the caller's next write of
+// its rows 0.60 -> 1.19 ms; 10,000: 0.32 -> 0.36 and 0.07 -> 0.31).  Help with the results alone does not pay
+// either (50,000 rows: 1.62 ms, with three threads 1.49, with seven 1.69; 80,000: 2.6, 3.1, 2.6).  Larger arrays
+// do not stay in caches.
 inline int crew_for(size_t bytes) {
     const unsigned hw = std::thread::hardware_concurrency();
     return bytes < (64u << 20) ? 0 : (int)std::min<unsigned>(7u, hw > 2 ? hw / 2 - 1 : 0u);

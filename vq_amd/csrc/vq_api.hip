@@ -189,7 +189,10 @@ int32_t launch_mfma(vq_ctx *ctx, const vq::AssignArgs &a, bool tables_ready, hip
     while (run_tiles > 1 && cdiv(tiles, per_run * run_tiles) * groups < 8192) run_tiles >>= 1;
     // Up to VQ_MFMA_OWN tiles for each workgroup of a single round: what counts then is the time of one
     // workgroup, and every wave makes its operands itself (OWN) instead of waiting for the launch that
-    // makes the tables (10,000 x 128, m = 16: 14.5 us after a launch of 6.5 us -> 15.0 us).
+    // makes the tables (10,000 x 128, m = 16, k = 256: 18.0 us in two launches -> 13.1; 40,000: 34 -> 26).
+    // Above that line as below it one round is the faster way for a while: 50,000 rows (9 tiles) 38 us as it
+    // runs and 30 by one round, 100,000 (17) 56 and 48, 200,000 (33) 88 and 83, 400,000 (66) 152 and 150; m =
+    // 10, a column block per workgroup: 100,000 (11) 42 and 34, but 200,000 (21) 64 and 69, 400,000 104 and 125.
     const int64_t share = cdiv(tiles * groups, per_run * VQ_MFMA_ROUND);
     const bool own = !tables_ready && !ctx->no_alloc && share <= VQ_MFMA_OWN;
     if (own) run_tiles = (int)share;
@@ -332,6 +335,10 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     const size_t res_lds = vq::wide_res_lds(sd, nb);
     const bool resident = half && !a.pend_cb && res_lds <= 160 * 1024 && a.n * a.m >= vq::kWideResMinRows &&
                           a.ld < ((int64_t)1 << 24);  // (32 rows below 2^31 bytes)
+    // a workgroup per compute unit, the same number for every column block: where 256 / m rounds down, some
+    // units have none, and the kernel is still the faster one (6,000 rows of 96 blocks of 64, 192 workgroups: 104
+    // -> 91 us staged -> resident, 127 blocks, 254: 132 -> 100, 4,000 rows of 200 blocks, 200: 140 -> 113; close to
+    // kWideResMinRows 1,500 x 96 49 -> 51)
     const int64_t res_groups = std::max<int64_t>(1, 256 / a.m);
     {
         ProfSpan sp(ctx, VQ_PROF_ASSIGN_KERNEL);
