@@ -387,84 +387,83 @@ __device__ __forceinline__ void own_operands(const float *cl, const float *norms
 // ---- the exact path of k_assign_mfma_bf ---------------------------------------------------------
 // Undecided rows of one (tile of 32 rows, column block) are decided by the whole wave in the
 // reference's order (src/utils.rs:63-70, src/pq.rs:166-174): lane l owns centroids l, l + 64,
-// l + 128, l + 192 (read from the wave's copy in LDS), computes their distances to the row in sequential f32 order, keeps the first smallest
-// (strict '<' over ascending indices), and the smallest (distance, index) pair over the lanes wins.
+// l + 128, l + 192 (read from the wave's copy in LDS) and computes their distances to the row in
+// sequential f32 order; the first of the smallest wins, as strict '<' over ascending indices gives.
 // A NaN distance is never chosen unless it is centroid 0's, which is never replaced.  Euclidean
-// compares the roots, as the reference does.  No LDS and, per batch of up to eight rows, one
-// memory round trip: lane L fetches float L % 8 of the batch's row L / 8, and the row's floats
-// reach every lane as scalars (v_readlane).
+// compares the roots, as the reference does: the root is monotone, so the smallest root is that of the
+// smallest square, and only a square within 2^-21 of it can share it; the others' roots are not taken.
+// The row's floats come from the lanes that hold the tile (v_readlane): no memory access at all.  Read from
+// memory again, eight rows to a round trip, and with every root taken: encode of 200,000 x 96 under cosine 93.5
+// us, 88.0 so; of 300,000 x 128, k = 1024, 554 and 535; a fit of 1M x 128 with its encode 5.01 and 4.97 ms.
 template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
 }
-// (d, i) <- the lexicographically smaller of (d, i) and (od, oi); d holds dist_key values
-__device__ __forceinline__ void lexmin(uint32_t &d, uint32_t &i, uint32_t od, uint32_t oi) {
-    const bool take = od < d || (od == d && oi < i);
-    d = take ? od : d;
-    i = take ? oi : i;
+__device__ __forceinline__ uint32_t umin_u32(uint32_t a, uint32_t b) { return a < b ? a : b; }
+// the smallest of all lanes' values, the same in every lane
+__device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
+    v = umin_u32(v, dpp_u32<0xB1>(v));
+    v = umin_u32(v, dpp_u32<0x4E>(v));
+    v = umin_u32(v, dpp_u32<0x141>(v));
+    v = umin_u32(v, dpp_u32<0x140>(v));
+    uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)v, 0);
+#pragma unroll
+    for (int row = 1; row < 4; ++row) r = umin_u32(r, (uint32_t)__builtin_amdgcn_readlane((int)v, 16 * row));
+    return r;
 }
 
 // cl: the column block's centroids in LDS (k x 8 floats, this wave's copy).
-// todo: ballot of the lanes (below 32) whose row is undecided; xblk = first row of the tile.
+// todo: ballot of the lanes (below 32) whose row is undecided; xr: the lane's row.
 // Returns the codes of those rows in their lanes, and their distances in dist (other lanes keep
 // `code` and `dist`).
 template <int METRIC>
 __device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, float &dist, const float *cl,
-                                           const float *norms, const float *__restrict__ xblk, int64_t ld, int k,
-                                           int lane) {
-    const float inf = __builtin_inff();
+                                           const float *norms, const float (&xr)[8], int k, int lane) {
+    constexpr uint32_t kInfKey = METRIC == M_COS ? 0xff800000u : 0x7f800000u;  // sort key of +inf
     while (todo) {
-        int src[8];
-        int cnt = 0;
-        int mine = __builtin_amdgcn_readfirstlane(__ffsll(todo) - 1);
+        const int src = __builtin_amdgcn_readfirstlane(__ffsll(todo) - 1);
+        todo &= todo - 1;
+        float xs[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            src[i] = todo ? __builtin_amdgcn_readfirstlane(__ffsll(todo) - 1) : src[0];
-            if (todo) ++cnt;
-            todo &= todo - 1;
-            if ((lane >> 3) == i) mine = src[i];
+        for (int d = 0; d < 8; ++d) xs[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xr[d]), src));
+        const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
+        // sort keys of the lane's four distances (Euclidean: of the squares); a NaN sorts behind +inf
+        uint32_t key[4];
+        float first = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int j = lane + 64 * q;
+            const float4 *cp = reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * 8);
+            const float4 c0 = cp[0], c1 = cp[1];
+            const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+            const float d = dist8<METRIC == M_COS ? M_COS : M_SQ>(xs, c, na, METRIC == M_COS ? norms[j < k ? j : 0] : 0.0f);
+            if (q == 0) first = d;
+            key[q] = j < k && d == d ? dist_key<METRIC>(d) : 0xffffffffu;
         }
-        const float val = xblk[(int64_t)mine * ld + (lane & 7)];
-        for (int i = 0; i < cnt; ++i) {
-            float xs[8];
+        const uint32_t best_key = wave_umin(umin_u32(umin_u32(key[0], key[1]), umin_u32(key[2], key[3])));
+        const float d0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(first), 0));
+        int best = 0;
+        float bd = METRIC == M_EUCLID ? sqrtf(d0) : d0;  // centroid 0 where nothing is below +inf
+        if (d0 == d0 && best_key < kInfKey) {  // uniform
+            unsigned long long at[4];
+            bd = key_dist<METRIC>(best_key);
+            if constexpr (METRIC == M_EUCLID) {
+                const uint32_t close = __float_as_uint(__builtin_fmaf(bd, 4.76837158203125e-07f, bd));
+                bd = sqrtf(bd);
 #pragma unroll
-            for (int d = 0; d < 8; ++d)
-                xs[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(val), 8 * i + d));
-            float bd = inf, dfirst = 0.0f;
-            uint32_t bi = 0x7fffffffu;
-            const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
+                for (int q = 0; q < 4; ++q) at[q] = __ballot(key[q] <= close);
+                if (__popcll(at[0]) + __popcll(at[1]) + __popcll(at[2]) + __popcll(at[3]) > 1) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int j = lane + 64 * q;
-                const float4 *cp = reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * 8);
-                const float4 c0 = cp[0], c1 = cp[1];
-                const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-                float d = dist8<METRIC>(xs, c, na, METRIC == M_COS ? norms[j < k ? j : 0] : 0.0f);
-                if (q == 0) dfirst = d;
-                d = (d == d) ? d : inf;
-                if (j < k && (d < bd || bi == 0x7fffffffu)) {
-                    bd = d;
-                    bi = (uint32_t)j;
+                    for (int q = 0; q < 4; ++q) at[q] = __ballot(key[q] <= close && sqrtf(__uint_as_float(key[q])) == bd);
                 }
-            }
-            uint32_t kd = dist_key<METRIC>(bd), ki = bi;
-            lexmin(kd, ki, dpp_u32<0xB1>(kd), dpp_u32<0xB1>(ki));
-            lexmin(kd, ki, dpp_u32<0x4E>(kd), dpp_u32<0x4E>(ki));
-            lexmin(kd, ki, dpp_u32<0x141>(kd), dpp_u32<0x141>(ki));
-            lexmin(kd, ki, dpp_u32<0x140>(kd), dpp_u32<0x140>(ki));
-            uint32_t rd = (uint32_t)__builtin_amdgcn_readlane((int)kd, 0), ri = (uint32_t)__builtin_amdgcn_readlane((int)ki, 0);
+            } else {
 #pragma unroll
-            for (int row = 1; row < 4; ++row)
-                lexmin(rd, ri, (uint32_t)__builtin_amdgcn_readlane((int)kd, 16 * row),
-                       (uint32_t)__builtin_amdgcn_readlane((int)ki, 16 * row));
-            const float d0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dfirst), 0));
-            const int best = (d0 == d0) ? (int)ri : 0;
-            int who = src[0];
-#pragma unroll
-            for (int u = 1; u < 8; ++u) who = (i == u) ? src[u] : who;
-            if (lane == who) {
-                code = best;
-                dist = (d0 == d0) ? key_dist<METRIC>(rd) : d0;  // the chosen centroid's distance as computed
+                for (int q = 0; q < 4; ++q) at[q] = __ballot(key[q] == best_key);
             }
+            best = at[0] ? __ffsll(at[0]) - 1 : at[1] ? __ffsll(at[1]) + 63 : at[2] ? __ffsll(at[2]) + 127 : __ffsll(at[3]) + 191;
+        }
+        if (lane == src) {
+            code = best;
+            dist = bd;  // the chosen centroid's distance as computed
         }
     }
     return code;
@@ -722,6 +721,14 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
         const unsigned long long todo = __ballot(mine && !sure);
         int code;
         float dist;  // of the chosen centroid, as the reference computes it
+        float xs[8];  // the lane's row
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            int lo, hi;
+            swap_halves(__float_as_int(xraw[u]), lo, hi);
+            xs[u] = __int_as_float(lo);
+            xs[4 + u] = __int_as_float(hi);
+        }
         {
             // the best run's four centroids, two per lane half, in the reference's order
             const int j0 = first + 2 * h;
@@ -729,14 +736,6 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
             const float4 *pa = reinterpret_cast<const float4 *>(cl + ja * SD);
             const float4 *pb = reinterpret_cast<const float4 *>(cl + jb * SD);
             const float4 ca0 = pa[0], ca1 = pa[1], cb0 = pb[0], cb1 = pb[1];
-            float xs[8];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                int lo, hi;
-                swap_halves(__float_as_int(xraw[u]), lo, hi);
-                xs[u] = __int_as_float(lo);
-                xs[4 + u] = __int_as_float(hi);
-            }
             const float ca[8] = {ca0.x, ca0.y, ca0.z, ca0.w, ca1.x, ca1.y, ca1.z, ca1.w};
             const float cc[8] = {cb0.x, cb0.y, cb0.z, cb0.w, cb1.x, cb1.y, cb1.z, cb1.w};
             const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
@@ -754,8 +753,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
         }
         if (todo) {  // the same in every lane: the reference-order argmin of the undecided rows
             n_exact += (uint32_t)__popcll(todo);
-            code = exact_rows8<METRIC>(todo, code, dist, cl, norms, a.x + (row0 + 32 * (int64_t)t) * a.ld + (int64_t)s * SD, a.ld,
-                                           k, lane);
+            code = exact_rows8<METRIC>(todo, code, dist, cl, norms, xs, k, lane);
         }
         if (mine) {
             const uint32_t rr = 32u * (uint32_t)t + (uint32_t)r;  // row within the run
