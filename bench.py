@@ -37,8 +37,8 @@ N_ROWS, DIM, M, K, ITERS = 1_000_000, 128, 16, 256, 10
 PEAK_FP32_MFMA_TFLOPS = 157.3  # MI355X published dense fp32 matrix peak
 PEAK_VALU_TLANESLOTS = 78.6    # 256 CUs x 128 lanes x 2.4 GHz (= the 157.3 TFLOP/s fp32 vector figure / 2)
 PEAK_HBM_GBS = 8000.0
-PEAK_BF16_MFMA_TFLOPS = 2500.0  # MI355X published dense bf16 matrix peak
-# rocprofv3 FETCH_SIZE / WRITE_SIZE of one LBG launch of k_assign_mfma_bf (KiB per dispatch), scaled by
+PEAK_F16_MFMA_TFLOPS = 2500.0  # MI355X published dense binary16 (and bf16) matrix peak
+# rocprofv3 FETCH_SIZE / WRITE_SIZE of one LBG launch of k_assign_mfma8 (KiB per dispatch), scaled by
 # the plain copy kernel (FETCH x 2.000, WRITE x 1.000): profiles/pq_fit_encode_1Mx128.md
 MEASURED_ASSIGN_TRAFFIC_BYTES = int((273044.0 * 2.000 + 12678.0 * 1.000) * 1024)
 
@@ -126,7 +126,7 @@ def main():
     ms_per_step = wall_ms / args.steps
     value = n / (ms_per_step * 1e-3)
 
-    # Dominant kernel: the assignment pass (k_assign_mfma_bf), timed alone by HIP events on the
+    # Dominant kernel: the assignment pass (k_assign_mfma8), timed alone by HIP events on the
     # library's stream (start and stop events of each launch's own dispatch).  What binds it is
     # instruction issue: the n x (m*k) scores come out of the matrix cores, every one of them has
     # to pass through the selection of the row's two smallest keys on the vector ALU, and on this
@@ -140,7 +140,7 @@ def main():
     # The kernel spends 17 instructions on 16 scores (v_min_i32 / v_min3_i32 over runs of four
     # centroids, one v_and_or_b32 tag per run, v_min3_i32 / v_med3_i32 for the two smallest keys),
     # each 4.2 clocks per wave64 on this chip, not 1; selection_floor_ms prices exactly those, and
-    # issue_floor_ms adds the two matrix instructions per 32 x 32 tile at the nominal clock.
+    # issue_floor_ms adds the matrix instruction per 32 x 32 tile at the nominal clock.
     flop_per_launch = 2.0 * K * DIM * n
     bytes_per_launch = (4.0 * DIM + 2.0 * M) * n
     slots_per_launch = 2.0 * M * K * n
@@ -150,7 +150,7 @@ def main():
     achieved_slots = slots_per_launch / sec / 1e12
     roofline = {
         "bound": "valu",
-        "kernel": "k_assign_mfma_bf (bf16-split matrix-core scores, top-2 selection over runs of four "
+        "kernel": "k_assign_mfma8 (matrix-core scores from one binary16 product, top-2 selection over runs of four "
                   "centroids on the vector ALU, exact pick inside the best run, in-wave exact re-check; "
                   "the 10 LBG passes and the encode pass)",
         "achieved": round(achieved_slots, 3),
@@ -169,8 +169,8 @@ def main():
         # secondary views of the same launch time; none of them is the bound
         "mfma_fp32_equiv_TFLOPs": round(achieved_tflops, 1),
         "mfma_fp32_equiv_frac_of_157.3": round(achieved_tflops / PEAK_FP32_MFMA_TFLOPS, 4),
-        "mfma_issued_bf16_TFLOPs": round(4.0 * achieved_tflops, 1),
-        "mfma_issued_frac_of_bf16_peak": round(4.0 * achieved_tflops / PEAK_BF16_MFMA_TFLOPS, 4),
+        "mfma_issued_f16_TFLOPs": round(2.0 * achieved_tflops, 1),
+        "mfma_issued_frac_of_f16_peak": round(2.0 * achieved_tflops / PEAK_F16_MFMA_TFLOPS, 4),
         "hbm_GBs_algorithmic": round(bytes_per_launch / sec / 1e9, 1),
         "hbm_frac": round(bytes_per_launch / sec / 1e9 / PEAK_HBM_GBS, 4),
         "assign_ms_incl_tables": round(assign_ms / max(assign_n, 1), 4),
@@ -179,13 +179,13 @@ def main():
     # (v_min_i32 / v_min3_i32, one class) for the four runs, 4 v_and_or_b32 (the runs' tags), and
     # 3 v_min3_i32 + 2 v_med3_i32 (top-2 update); one wave64 instruction handles 64 lanes.  The
     # selection floor is the time those instructions alone take with every SIMD full; the issue
-    # floor adds the matrix instructions (2 per 32 x 32 tile, 32 clocks each, 1024 SIMDs at 2.4 GHz).
+    # floor adds the matrix instructions (one per 32 x 32 tile, 32 clocks each, 1024 SIMDs at 2.4 GHz).
     rate = {name: ctx.calibrate(kind) for kind, name in
             ((1, "v_fma_f32"), (2, "v_min3_i32"), (3, "v_med3_i32"), (4, "v_and_or_b32"), (5, "v_add_u32"))}
     scores = float(n) * M * K
     floor_ms = scores / 64.0 * ((11.0 / 16.0) / rate["v_min3_i32"] + 0.25 / rate["v_and_or_b32"]
                                 + 0.125 / rate["v_med3_i32"]) * 1e3
-    mfma_ms = scores / 1024.0 * 2.0 * 32.0 / (1024.0 * 2.4e9) * 1e3
+    mfma_ms = scores / 1024.0 * 32.0 / (1024.0 * 2.4e9) * 1e3
     roofline["selection_floor_ms"] = round(floor_ms, 4)
     roofline["frac_of_selection_floor"] = round(floor_ms / avg_kern_ms, 4)
     roofline["issue_floor_ms"] = round(floor_ms + mfma_ms, 4)
@@ -197,7 +197,7 @@ def main():
     # Do matrix and vector instructions of a SIMD run side by side?  (ms: matrix alone, vector alone,
     # together.)  From different waves they take turns (together = sum), which is why issue_floor_ms
     # adds them; behind a matrix instruction of the SAME wave independent vector instructions issue
-    # in its shadow, all but about a quarter of its 32 clocks — the kernel places half a block's
+    # in its shadow, all but about a quarter of its 32 clocks — the kernel places a block's
     # selection behind each matrix instruction for that reason.
     ov = {}
     for mode, name in ((0, "different_waves_8_min3_per_mfma"), (1, "same_wave_7_min3_per_mfma"),

@@ -144,7 +144,7 @@ def run_c3(ctx, log, x=None, dx=None, parity=True):
                                                        vq_amd.EUCLIDEAN, bufs))
     slots = 2.0 * m * k * n
     out["dominant_kernel"] = {
-        "name": "k_assign_mfma_bf (the same kernel as the headline: 5 x (10 LBG passes + 1 reconstruction pass))",
+        "name": "k_assign_mfma8 (the same kernel as the headline: 5 x (10 LBG passes + 1 reconstruction pass))",
         "bound": "valu", "avg_launch_ms": round(avg, 4), "launches": cnt,
         "achieved": round(slots / (avg * 1e-3) / 1e12, 3) if avg else None, "peak": PEAK_VALU_TLANESLOTS,
         "unit": "T lane-slots/s", "frac": round(slots / (avg * 1e-3) / 1e12 / PEAK_VALU_TLANESLOTS, 4) if avg else None,

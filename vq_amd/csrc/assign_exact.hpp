@@ -29,8 +29,8 @@ struct AssignArgs {
     int *changed;         // LBG mode: changed[s] set to 1 when any code of block s differs
     const int *done;      // LBG mode: blocks with done[s] != 0 are skipped
     const int *before = nullptr;  // LBG mode, instead of done: the changed flags of the pass before (0: skipped)
-    float *dist = nullptr;  // encode mode, k_assign_mfma_bf only: [n][m] distance of the chosen centroid, or null
-    uint16_t *out16 = nullptr;  // encode mode, k_assign_mfma_bf only: [n][8 m] chosen centroids as binary16, or null
+    float *dist = nullptr;  // encode mode, k_assign_mfma8 only: [n][m] distance of the chosen centroid, or null
+    uint16_t *out16 = nullptr;  // encode mode, k_assign_mfma8 only: [n][8 m] chosen centroids as binary16, or null
     // A residual update that the pass applies before it scores the rows (single wide column block,
     // k_assign_mfma_wide_bf only): x[i] = src[i] - pend_cb[pend_codes[i]], where src is the rows
     // themselves (an update in place) or, pend_src != null, other rows of stride pend_src_ld that

@@ -12,9 +12,9 @@
 // run's smallest score, tagged with the run's first index) and picks inside the best run by exact
 // distances; the wide kernel keeps the three smallest scores, one tag per score.
 //
-// 8-float column blocks (k_assign_mfma_bf): bf16 matrix cores with split operands; the undecided
-// rows are resolved inside the same wave.  Wider blocks (k_assign_mfma_wide_bf): the same split
-// per chunk of 8 dimensions; the undecided pairs are listed for the exact kernel of assign_exact.hpp.
+// 8-float column blocks (k_assign_mfma8): one product of binary16 operands per score; the undecided
+// rows are resolved inside the same wave.  Wider blocks (k_assign_mfma_wide_bf): operands split into bf16
+// parts, or rounded to binary16; the undecided pairs are listed for the exact kernel of assign_exact.hpp.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
@@ -106,40 +106,52 @@ __device__ __forceinline__ void top2_push4(int &m1, int &m2, int k0, int k1, int
 }
 
 // ---------------------------------------------------------------------------------------------
-// 8-float column blocks on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16, 4x the fp32 rate).
+// 8-float column blocks on the binary16 matrix cores (v_mfma_f32_32x32x16_f16), one instruction per 32 rows x
+// 32 centroids.
 //
-// Every fp32 operand is split into two bf16 numbers, v = vh + vl + e with |e| <= 2^-16 |v|
-// (round-to-nearest-even twice).  With a = -2c, the lanes of half h = lane / 32 own dimensions
-// [4h, 4h + 4) of the block and the 8 contraction slots of that half hold
-//     instruction 1:  ah . xh  (4 slots)   ah . xl  (4 slots)
-//     instruction 2:  al . xh  (4 slots)   1 . (the half's share of ||x||^2, one slot; an empty
-//                                               slot; ||c||^2 in three bf16 parts over the two halves)
-// so a lane loads and splits only its own 16 bytes of the row and both halves do the same work:
-// the result is the score ||c||^2 + ||x||^2 - 2 x.c + delta with an error of at most
-// 3 * 2^-16 * sum|a_t||x_t| <= 3 * 2^-16 (||x||^2 + ||c||^2) from the dropped terms (a ex, x ea,
-// al xl) plus at most 2^-17.9 (||x||^2 + ||c||^2) from the fp32 accumulation of the 2 x 15
-// addends.  delta: the share of ||x||^2 rides as ONE bf16 number rounded up, 0 <= delta <
-// 2^-7 ||x||^2; the product 1 . share is exact and the same addend in every score of the row, so
-// delta cancels in the difference of two scores (it lengthens the partial sums, and with them the
-// accumulation bound, by under 1 %), and rounding up keeps scores of near-zero distances from
-// turning negative.  Two candidates compared: below 2^-13.2 (||x||^2 + max ||c||^2); the test
-// uses 2^-13, plus 2^-14 |second| for the packed bits and the reference's own rounding.  bf16
-// keeps the fp32 exponent range, so no scaling is needed; non-finite values fail the test.
-// x and c here are the row and the centroid minus the block's centre mu (rounded to fp32): the
-// rounding of the two differences moves a squared distance by at most 2^-22 (||x||^2 + ||c||^2),
-// far inside the slack between 2^-13.2 and 2^-13, and the bound itself shrinks with the norms.
+// Rows and centroids are taken relative to the block's centre and scaled by a power of two (mfma8_scale).
+// The lanes of half h = lane / 32 own dimensions [4h, 4h + 4); with a = -2c the 8 contraction slots of that
+// half hold
+//     ah . xh  (4 slots)   al . xh  (the half's first two dimensions)   1 . (the half's share of ||x||^2)
+//     (||c~||^2 in two parts, the higher in the lower half) . 1
+// where xh, ah are the values rounded to binary16 and al what that left of a.  So a lane loads and rounds
+// only its own 16 bytes of the row, and the scores are the squared distances between the ROUNDED row x~ and the
+// ROUNDED centroids c~ up to the accumulation (the share of ||x||^2, the same in every score of the row, only keeps
+// them positive; it is enlarged by kLift8 and rounded itself).
+// What that is worth: with ex = x - x~ and ec = c - c~ the distances of two centroids differ by
+//     d2^2 - d1^2 >= s2 - s1 - 2 |c~1 - c~2| |ex| - 2 sqrt(s1) |ec1| - 2 sqrt(s2) |ec2| - (second order)
+// and |c~1 - c~2| <= sqrt(s1) + sqrt(s2): the first candidate has won when
+//     s2 - s1 > 4 (sqrt(s2) + e) e,   e = |ex| + max |ec| <= sqrt(2 (|ex|^2 + max |ec|^2)),
+// an error in proportion to the DISTANCE, not to the norms.  |ex|^2 is summed as the row is rounded, max |ec|^2
+// made with the tables.  On top of it 2^-16 (||x||^2 + max ||c~||^2) for the accumulation of 16 products, the two
+// parts of ||c~||^2 (2^-22) and the rounding of x and c relative to the centre (2^-24), and 2^-14 |second| for the
+// packed bits and the reference's own rounding.  Non-finite values, and rows beyond the range of binary16, fail
+// the test.
+// Measured against two instructions of bf16 parts (ah.xh + ah.xl + al.xh; a margin of 2^-13 (||x||^2 + max
+// ||c||^2), 0.07-0.3 % of the pairs undecided where this leaves 0.2-1 %): half the matrix instructions and half
+// the operand registers, a fifth fewer vector instructions to make the row's operand.  1M x 128, m = 16, k = 256:
+// a pass of a fit 382 -> 295-315 us under the profiler; fit and encode 5.19 -> 4.61 ms; encode of 200,000 x 96
+// under cosine 95 -> 83 us (with the undecided rows read from registers, exact_rows8).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
+using f16x8 = _Float16 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr float kPad8 = 65504.0f;  // padding centroids: ||c~||^2 = 2 kPad8, longer than any that is scored
+constexpr float kLift8 = 1.004f;   // the row's share of ||x||^2 in binary16 is then above its rounded operand's
+constexpr float kFlush8 = 3.0e-8f; // eight elements below the normal range of binary16, squared
+constexpr float kCosScale = 4.0f;  // cosine: the length of rows and centroids
 
 constexpr int kStatSlots = 64;    // counters of undecided pairs, one 128-byte line apart
 constexpr int kStatStride = 32;
 
-struct MfmaBfTables {
-    const u32x4 *atab;     // [m][nb][2][64]  A operands of the two instructions, lane order
-    const float *maxc2;    // [m]  largest ||c - mu||^2 of the column block (NaN if any is NaN)
-    const float *mu;       // [m][8]  the block's centre: mean of its centroids
+constexpr int kMfma8Aux = 12;  // floats per column block beside the operands
+// aux[s]: [0, 8) minus the centre times the scale, [8] largest ||c~||^2 (NaN: no row of the block may be
+// decided by its scores), [9] largest dc^2, [10] the scale
+struct Mfma8Tables {
+    const u32x4 *atab;     // [m][nb][64]  A operands, lane order
+    const float *aux;      // [m][kMfma8Aux]
     uint32_t *stat;        // [kStatSlots * kStatStride]  pairs decided by the exact path (measurement)
     int nb;                // blocks of 32 centroids, padded to an even number
     uint32_t *stat_next = nullptr;  // (OWN) the counters of the pass after this one, to be cleared
@@ -162,17 +174,13 @@ __device__ __forceinline__ uint32_t bf16_pack2(float a, float b) {
 }
 
 // ---- cosine -----------------------------------------------------------------------------------
-// d = 1 - x.c / (|x| |c|) falls as x.c/|c| grows, so with the centroids divided by their norms the scores
-// s[j] = P - 2 x.(c_j / |c_j|), P >= 2 |x| the same in every score of a row (it keeps them from turning
-// negative), order the candidates: no centre, no ||c||^2.  u = 2^-24, sd the block's width.
-//   score: 3 * 2^-16 * 2 |x| from the operand split, 2^-22 * 2 |x| from the division by the norm,
-//     the fp32 accumulation of partial sums below 4.2 |x|;
-//   reference (src/distances.rs:141-151): the sums, the product of the norms, the quotient and the
-//     difference from 1 leave d within (sd + 6) u of its value at the computed norms, 2 |x| (sd + 6) u here.
-// Width 8: (9.2e-5 + 7.5e-6 + 4.8e-7 + 1.7e-6) |x| per candidate, below 2.1e-4 |x| for two; the test
-// uses 2^-12 |x| (2.44e-4), plus 2^-14 |second| for the packed bits.  Rows and centroids whose norm is
-// outside [1e-15, 1e15] and not zero, where the reference's products may over- or underflow, and rows
-// of norm zero go to the exact argmin (a centroid of norm zero has d = 1, its score P: in order).
+// d = 1 - x.c / (|x| |c|) is half the squared distance of x / |x| and c / |c|: rows and centroids are brought
+// to length kCosScale, about the origin, and scored like the others.  What this adds to the bound, in units of
+// kCosScale^2: the scaling of the row and of the centroid, below 2^-20; the reference (src/distances.rs:141-151),
+// whose sums, product of the norms, quotient and difference from 1 leave d within 14 * 2^-24, 2^-18.2 for two
+// candidates; the 2^-16 of both norms covers them.  Rows and centroids whose norm is outside [1e-15, 1e15]
+// and not zero, where the reference's products may over- or underflow, and rows of norm zero go to the exact
+// argmin (a centroid of norm zero has d = 1: its operand is zero and its ||c~||^2 kCosScale^2, in order).
 __device__ __forceinline__ float seq_norm8(const float (&c)[8]) {
     float acc = 0.0f;
 #pragma unroll
@@ -183,9 +191,9 @@ __device__ __forceinline__ float seq_norm8(const float (&c)[8]) {
     return sqrtf(acc);
 }
 // c divided by its norm; 0, or NaN if the block must not be scored with this centroid in it.
-__device__ __forceinline__ float cos_normalise(float (&c)[8]) {
+__device__ __forceinline__ float cos_normalise(float (&c)[8], bool &zero) {
     const float nb = seq_norm8(c);
-    const bool zero = nb == 0.0f;
+    zero = nb == 0.0f;
     const float inv = zero ? 0.0f : 1.0f / nb;
 #pragma unroll
     for (int t = 0; t < 8; ++t) c[t] *= inv;
@@ -215,176 +223,243 @@ __device__ __forceinline__ float dist8(const float (&x)[8], const float (&c)[8],
     }
 }
 
-// Tables for k_assign_mfma_bf.  One workgroup per column block s, one thread per padded centroid
-// (k <= 256).  Rows and centroids are scored relative to mu[s] = mean of the block's centroids
-// (distances do not change under a common shift, the bound on the score error, which is
-// proportional to ||x - mu||^2 + ||c - mu||^2, does); maxc2[s] = largest ||c - mu||^2 of the
-// block (NaN if any is NaN).  mfma_bf_prep_block is the work of one workgroup, given centroid j
-// of the block in thread j's registers (zeros from k on); k_mfma_bf_prep reads the centroids from
+// The scale of a column block: the power of two that brings the centroids' root mean square norm about the
+// centre to 4 ... 8 (r2: the mean square; NaN where the scores cannot decide).  A centroid is then no longer
+// than 128 (k <= 256), and a row's share of ||x||^2 fits binary16 up to 32 ... 64 times that norm.
+__device__ __forceinline__ float mfma8_scale(float r2) {
+    if (r2 == 0.0f) return 1.0f;  // all centroids are the same
+    return r2 > 1e-36f && r2 < 1e36f ? ldexpf(1.0f, 2 - (ilogbf(r2) >> 1)) : __builtin_nanf("");
+}
+// The A operand of one centroid and one lane half: a[t] = -2 c[t] of the half's four dimensions, scaled.
+// Elements below the normal range of binary16 count as zero, whatever the matrix cores make of them.
+// n2, d2: the half's shares of ||c~||^2 and of ||c - c~||^2.
+struct Half8 {
+    uint32_t h01, h23, l01;
+    float n2, d2;
+};
+__device__ __forceinline__ float f16_normal(float v) {
+    const float r = (float)(_Float16)v;
+    return fabsf(r) < 6.103515625e-05f ? 0.0f : r;
+}
+__device__ __forceinline__ uint32_t f16_pack2(float a, float b) {  // round to nearest even
+    using h2 = _Float16 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, h2{(_Float16)a, (_Float16)b});
+}
+__device__ __forceinline__ Half8 half8(const float (&a)[4]) {
+    float hi[4], lo[4] = {0.f, 0.f, 0.f, 0.f};
+    Half8 o;
+    o.n2 = o.d2 = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        hi[t] = f16_normal(a[t]);
+        if (t < 2) lo[t] = f16_normal(a[t] - hi[t]);
+        const float d = (a[t] - hi[t]) - lo[t], v = hi[t] + lo[t];
+        o.n2 = __builtin_fmaf(0.25f * v, v, o.n2);
+        o.d2 = __builtin_fmaf(0.25f * d, d, o.d2);
+    }
+    o.h01 = f16_pack2(hi[0], hi[1]);
+    o.h23 = f16_pack2(hi[2], hi[3]);
+    o.l01 = f16_pack2(lo[0], lo[1]);
+    return o;
+}
+// The last word: 1 against the row's share of ||x||^2, and the half's part of c2 = ||c~||^2 against 1.
+__device__ __forceinline__ uint32_t c2_word(float c2, int h, bool live) {
+    const float hi = live ? (float)(_Float16)c2 : kPad8, lo = live ? c2 - hi : kPad8;
+    return f16_pack2(1.0f, h == 0 ? hi : lo);
+}
+
+// Tables for k_assign_mfma8.  One workgroup per column block s, one thread per padded centroid
+// (k <= 256).  Rows and centroids are scored relative to the mean of the block's centroids
+// (distances do not change under a common shift, the rounding of the operands does).
+// mfma8_prep_block is the work of one workgroup, given centroid j
+// of the block in thread j's registers (zeros from k on); k_mfma8_prep reads the centroids from
 // the codebook, the LBG loop's last update kernel has just computed them.
-// COS: the operands are those of the centroids divided by their norms, the centre and ||c||^2 are zero
-// and maxc2[s] only says whether the block can be scored (see own_operands).
+// COS: the centroids divided by their norms, about the origin (see cos_normalise).
 template <bool COS = false>
-__device__ __forceinline__ void mfma_bf_prep_block(float (&c)[8], int s, int j, int k, int nb,
-                                                   u32x4 *__restrict__ atab, float *__restrict__ maxc2,
-                                                   float *__restrict__ mu) {
-    __shared__ float sh_max[4];
+__device__ __forceinline__ void mfma8_prep_block(float (&c)[8], int s, int j, int k, int nb,
+                                                   u32x4 *__restrict__ atab, float *__restrict__ aux) {
+    __shared__ float sh_red[3][4];
     __shared__ float sh_mu[4][8];
-    // centre: sum of c / 256 (no overflow for k <= 256), then * 256 / k
     float centre[8];
-    float cos_bad = 0.0f;
-    if constexpr (COS) cos_bad = cos_normalise(c);
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        float v = COS ? 0.0f : c[t] * 0.00390625f;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-        if ((j & 63) == 0) sh_mu[j >> 6][t] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        centre[t] = (((sh_mu[0][t] + sh_mu[1][t]) + sh_mu[2][t]) + sh_mu[3][t]) * (256.0f / (float)k);
-        if (j == 0) mu[s * 8 + t] = centre[t];
-    }
-    float mx = 0.0f;
-    if (j < nb * 32) {
-        const int b = j / 32, i = j % 32;
-        float c2 = kPadScore;  // padding centroids: finite, so that index bits can be packed in
-        if (j < k) {
-            c2 = 0.0f;
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                c[t] -= centre[t];
-                c2 = COS ? 0.0f : __builtin_fmaf(c[t], c[t], c2);
-            }
-            mx = COS ? cos_bad : c2;
-        }
-        uint32_t hb[8], lb[8];
+    float bad = 0.0f;
+    bool zero = false;
+    float *out = aux + (size_t)s * kMfma8Aux;
+    float sg = kCosScale;
+    if constexpr (COS) {
+        bad = cos_normalise(c, zero);
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
-            const float a = -2.0f * c[t];
-            hb[t] = bf16_rne_bits(a);
-            lb[t] = bf16_rne_bits(a - bf16_bits_to_float(hb[t]));
+            centre[t] = 0.0f;
+            if (j == 0) out[t] = 0.0f;
         }
-        // ||c - mu||^2 rides in the spare slots of the second instruction as three bf16 parts
-        // (exact: 3 x 8 bits), against ones in the row operand
-        const uint32_t c2a = bf16_rne_bits(c2);
-        const float c2r = c2 - bf16_bits_to_float(c2a);
-        const uint32_t c2b = bf16_rne_bits(c2r);
-        const uint32_t c2c = bf16_rne_bits(c2r - bf16_bits_to_float(c2b));
-        // lane i + 32 h: instruction 1 {ah[4h..4h+3], ah[4h..4h+3]}, instruction 2
-        // {al[4h..4h+3], 1, 1, c2 parts: (1st, 2nd) in the lower half, (3rd, 0) in the upper}
-        u32x4 *dst = atab + ((size_t)s * nb + b) * 128;
+    } else {
+        // centre: sum of c / 256 (no overflow for k <= 256), then * 256 / k
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t ah0 = hb[4 * h] | (hb[4 * h + 1] << 16), ah1 = hb[4 * h + 2] | (hb[4 * h + 3] << 16);
-            const uint32_t al0 = lb[4 * h] | (lb[4 * h + 1] << 16), al1 = lb[4 * h + 2] | (lb[4 * h + 3] << 16);
-            dst[32 * h + i] = u32x4{ah0, ah1, ah0, ah1};
-            dst[64 + 32 * h + i] = u32x4{al0, al1, 0x3f803f80u, h == 0 ? (c2a | (c2b << 16)) : c2c};
+        for (int t = 0; t < 8; ++t) {
+            float v = c[t] * 0.00390625f;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+            if ((j & 63) == 0) sh_mu[j >> 6][t] = v;
+        }
+        __syncthreads();
+        float p = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            centre[t] = (((sh_mu[0][t] + sh_mu[1][t]) + sh_mu[2][t]) + sh_mu[3][t]) * (256.0f / (float)k);
+            if (j < k) c[t] -= centre[t];
+            p = __builtin_fmaf(c[t] * 0.0625f, c[t] * 0.0625f, p);  // / 256
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) p += __shfl_xor(p, off);
+        if ((j & 63) == 0) sh_red[2][j >> 6] = p;
+        __syncthreads();
+        sg = mfma8_scale((((sh_red[2][0] + sh_red[2][1]) + sh_red[2][2]) + sh_red[2][3]) * (256.0f / (float)k));
+        if (j == 0) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) out[t] = -(centre[t] * sg);
         }
     }
-    // largest ||c||^2; a NaN poisons the bound on purpose
+    float mx = 0.0f, md = 0.0f;
+    if (j < nb * 32) {
+        const int b = j / 32, i = j % 32;
+        u32x4 *dst = atab + ((size_t)s * nb + b) * 64;
+        Half8 o[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float a[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) a[t] = j < k ? -2.0f * (c[4 * h + t] * sg) : 0.0f;
+            o[h] = half8(a);
+        }
+        // (a centroid of norm zero has the cosine distance 1: as far as any at a right angle)
+        const float c2 = COS && zero ? kCosScale * kCosScale : o[0].n2 + o[1].n2;
+        if (j < k) {
+            mx = c2 + bad + (sg - sg);  // NaN: the block is not scored
+            md = o[0].d2 + o[1].d2;
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) dst[32 * h + i] = u32x4{o[h].h01, o[h].h23, o[h].l01, c2_word(c2, h, j < k)};
+    }
+    // a NaN poisons the bound on purpose
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         const float o = __shfl_xor(mx, off);
         mx = (mx == mx && o == o) ? fmaxf(mx, o) : __builtin_nanf("");
+        md = fmaxf(md, __shfl_xor(md, off));
     }
-    if ((j & 63) == 0) sh_max[j >> 6] = mx;
+    if ((j & 63) == 0) {
+        sh_red[0][j >> 6] = mx;
+        sh_red[1][j >> 6] = md;
+    }
     __syncthreads();
     if (j == 0) {
-        float r = sh_max[0];
+        float r = sh_red[0][0], d = sh_red[1][0];
 #pragma unroll
         for (int w = 1; w < 4; ++w) {
-            const float o = sh_max[w];
+            const float o = sh_red[0][w];
             r = (r == r && o == o) ? fmaxf(r, o) : __builtin_nanf("");
+            d = fmaxf(d, sh_red[1][w]);
         }
-        maxc2[s] = r;
+        out[8] = r;
+        out[9] = d;
+        out[10] = sg;
     }
 }
 
 template <bool COS = false>
-static __global__ void __launch_bounds__(256) k_mfma_bf_prep(const float *__restrict__ cb, int m, int k, int nb,
-                                                             u32x4 *__restrict__ atab, float *__restrict__ maxc2,
-                                                             float *__restrict__ mu, uint32_t *__restrict__ stat,
+static __global__ void __launch_bounds__(256) k_mfma8_prep(const float *__restrict__ cb, int m, int k, int nb,
+                                                             u32x4 *__restrict__ atab, float *__restrict__ aux,
+                                                             uint32_t *__restrict__ stat,
                                                              uint32_t *__restrict__ stat_next) {
     const int s = blockIdx.x, j = threadIdx.x;
     if (s == 0 && j < kStatSlots) stat[j * kStatStride] = stat_next[j * kStatStride] = 0u;
     float c[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) c[t] = (j < k) ? cb[((size_t)s * k + j) * 8 + t] : 0.0f;
-    mfma_bf_prep_block<COS>(c, s, j, k, nb, atab, maxc2, mu);
+    mfma8_prep_block<COS>(c, s, j, k, nb, atab, aux);
 }
 
-// The tables of mfma_bf_prep_block made by one wave for itself (the same operands up to the order in
-// which the centre's sum is added, which any centre allows): lane (r, h) makes its own operands of
-// the centroids 32 b + r, dimensions [4h, 4h + 4), from the wave's copy of the centroids in LDS.
+// The tables of mfma8_prep_block made by one wave for itself (the same operands up to the order in
+// which the sums for the centre and the scale are added, which any centre and scale allow): lane (r, h) makes its
+// own operands of the centroids 32 b + r, dimensions [4h, 4h + 4), from the wave's copy of the centroids in LDS.
 // COS: of the centroids divided by their norms (norms: one per centroid, in LDS).
 template <bool COS>
 __device__ __forceinline__ void own_operands(const float *cl, const float *norms, int k, int nb, int r, int h,
-                                             u32x4 (&A1)[8], u32x4 (&A2)[8], float (&muh)[4], float &mc2) {
+                                             u32x4 (&A)[8], float (&muh)[4], float &mc2, float &mdc, float &sg) {
     float cv[8][4];
     float sum[4] = {0.f, 0.f, 0.f, 0.f};
+    float bad = 0.0f;
+    sg = kCosScale;
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
         const int j = 32 * b + r;
         const float4 v = *reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * 8 + 4 * h);
         cv[b][0] = v.x, cv[b][1] = v.y, cv[b][2] = v.z, cv[b][3] = v.w;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) sum[u] += j < k && !COS ? cv[b][u] * 0.00390625f : 0.0f;  // no overflow for k <= 256
+        for (int u = 0; u < 4; ++u) sum[u] += j < k ? cv[b][u] * 0.00390625f : 0.0f;  // no overflow for k <= 256
+    }
+    if constexpr (!COS) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+#pragma unroll
+            for (int off = 16; off > 0; off >>= 1) sum[u] += __shfl_xor(sum[u], off);  // over the lanes of this half
+            sum[u] *= 256.0f / (float)k;  // the centre
+        }
+        float p = 0.0f;
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float c = 32 * b + r < k ? (cv[b][u] - sum[u]) * 0.0625f : 0.0f;
+                p = __builtin_fmaf(c, c, p);
+            }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) p += __shfl_xor(p, off);
+        sg = mfma8_scale(p * (256.0f / (float)k));
+        bad = sg - sg;  // 0 or NaN
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-#pragma unroll
-        for (int off = 16; off > 0; off >>= 1) sum[u] += __shfl_xor(sum[u], off);  // over the lanes of this half
-        muh[u] = sum[u] * (256.0f / (float)k);
-    }
-    float mx = 0.0f;
+    for (int u = 0; u < 4; ++u) muh[u] = COS ? 0.0f : -(sum[u] * sg);
+    float mx = 0.0f, md = 0.0f;
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
         if (b >= nb) {  // uniform; never multiplied
-            A1[b] = A1[0];
-            A2[b] = A2[0];
+            A[b] = A[0];
             continue;
         }
         const bool live = 32 * b + r < k;
-        float p = 0.0f, a[4], scale = -2.0f, c2;
+        float scale = -2.0f * sg, c2, d2;
+        const float nc = COS && live ? norms[32 * b + r] : 0.0f;
         if constexpr (COS) {
-            const float nc = live ? norms[32 * b + r] : 0.0f;
             scale = nc == 0.0f ? 0.0f : -2.0f * (1.0f / nc);
-            c2 = nc == 0.0f || (nc >= 1e-15f && nc <= 1e15f) ? 0.0f : __builtin_nanf("");
+            bad = nc == 0.0f || (nc >= 1e-15f && nc <= 1e15f) ? 0.0f : __builtin_nanf("");
         }
+        float a[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const float c = live ? cv[b][u] - muh[u] : 0.0f;
-            p = __builtin_fmaf(c, c, p);
-            a[u] = scale * c;
-        }
-        if constexpr (!COS) {
-            int pa, pb;
-            swap_halves(__float_as_int(p), pa, pb);
-            c2 = __int_as_float(pa) + __int_as_float(pb);
-        }
-        mx = (mx == mx && c2 == c2) ? fmaxf(mx, c2) : __builtin_nanf("");
-        c2 = live ? (COS ? 0.0f : c2) : kPadScore;
-        const uint32_t h01 = bf16_pack2(a[0], a[1]), h23 = bf16_pack2(a[2], a[3]);
-        const uint32_t l01 = bf16_pack2(a[0] - __uint_as_float(h01 << 16), a[1] - __uint_as_float(h01 & 0xffff0000u));
-        const uint32_t l23 = bf16_pack2(a[2] - __uint_as_float(h23 << 16), a[3] - __uint_as_float(h23 & 0xffff0000u));
-        const uint32_t c2a = bf16_rne_bits(c2);
-        const float c2r = c2 - bf16_bits_to_float(c2a);
-        const uint32_t c2b = bf16_rne_bits(c2r), c2c = bf16_rne_bits(c2r - bf16_bits_to_float(c2b));
-        A1[b] = u32x4{h01, h23, h01, h23};
-        A2[b] = u32x4{l01, l23, 0x3f803f80u, h == 0 ? (c2a | (c2b << 16)) : c2c};
+        for (int u = 0; u < 4; ++u)
+            a[u] = !live ? 0.0f : COS ? (scale * cv[b][u]) * kCosScale : scale * (cv[b][u] - sum[u]);
+        const Half8 o = half8(a);
+        int pa, pb;
+        swap_halves(__float_as_int(o.n2), pa, pb);
+        c2 = COS && nc == 0.0f ? kCosScale * kCosScale : __int_as_float(pa) + __int_as_float(pb);
+        swap_halves(__float_as_int(o.d2), pa, pb);
+        d2 = __int_as_float(pa) + __int_as_float(pb);
+        const float cx = live ? c2 + bad : 0.0f;
+        mx = (mx == mx && cx == cx) ? fmaxf(mx, cx) : __builtin_nanf("");
+        md = fmaxf(md, live ? d2 : 0.0f);
+        A[b] = u32x4{o.h01, o.h23, o.l01, c2_word(c2, h, live)};
     }
 #pragma unroll
     for (int off = 16; off > 0; off >>= 1) {
         const float o = __shfl_xor(mx, off);
         mx = (mx == mx && o == o) ? fmaxf(mx, o) : __builtin_nanf("");
+        md = fmaxf(md, __shfl_xor(md, off));
     }
     mc2 = mx;
+    mdc = md;
 }
 
-// ---- the exact path of k_assign_mfma_bf ---------------------------------------------------------
+// ---- the exact path of k_assign_mfma8 ---------------------------------------------------------
 // Undecided rows of one (tile of 32 rows, column block) are decided by the whole wave in the
 // reference's order (src/utils.rs:63-70, src/pq.rs:166-174): lane l owns centroids l, l + 64,
 // l + 128, l + 192 (read from the wave's copy in LDS) and computes their distances to the row in
@@ -470,8 +545,7 @@ __device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, fl
 }
 
 // One wave = one column block of 8 floats against a run of tiles of 32 rows.  The wave keeps the
-// A operands of all the block's centroids in registers (8 blocks of 32 centroids x 2 instructions
-// x 4 registers) and a copy of the block's centroids in LDS, and streams the rows past them: the
+// A operands of all the block's centroids in registers (8 blocks of 32 centroids x 4 registers) and a copy of the block's centroids in LDS, and streams the rows past them: the
 // inner loop reads no memory.  A lane's 16 scores of a tile are four runs of four consecutive
 // centroids; the smallest score of a run, tagged with the run's first index, is the run's key, and
 // the smallest and second-smallest key of the row are kept (two minima and one v_and_or per run,
@@ -484,10 +558,10 @@ __device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, fl
 // same rows.  SG = 1 (m not a multiple of 4): the four waves take consecutive runs of one block.
 // FULL: 8 blocks of 32 centroids (k above 224), scored without a branch between them.
 // OWN: every wave makes the operands, the centre and the bound of its block from the centroids it
-// holds in LDS, about 500 vector instructions, instead of reading the tables that k_mfma_bf_prep has
+// holds in LDS, about 700 vector instructions, instead of reading the tables that k_mfma8_prep has
 // made: for grids of one round of workgroups, where that launch (6.5 us) is in the way.
 template <int METRIC, bool LBG, int SG, bool FULL, bool OWN = false>
-__global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfTables tb, int run_tiles, int64_t nruns,
+__global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tables tb, int run_tiles, int64_t nruns,
                                                             int64_t run_stride) {
     constexpr int SD = 8;
     __shared__ __attribute__((aligned(16))) float lds_cb[4][256 * SD];
@@ -538,26 +612,25 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
         }
     }
     // the A operands of every block of 32 centroids, the centre's dimensions [4h, 4h + 4), the bound
-    u32x4 A1[8], A2[8];
+    u32x4 A[8];
     float muh[4];
-    float mc2;
+    float mc2, mdc, sg;
     if constexpr (OWN) {
         if (blockIdx.x == 0)
             for (int i = threadIdx.x; i < kStatSlots; i += 256) tb.stat_next[i * kStatStride] = 0u;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        own_operands<METRIC == M_COS>(cl, norms, k, nb, r, h, A1, A2, muh, mc2);
+        own_operands<METRIC == M_COS>(cl, norms, k, nb, r, h, A, muh, mc2, mdc, sg);
     } else {
-        const u32x4 *ap = tb.atab + (size_t)s * nb * 128 + lane;
+        const u32x4 *ap = tb.atab + (size_t)s * nb * 64 + lane;
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const int bc = b < nb ? b : 0;
-            A1[b] = ap[(size_t)bc * 128];
-            A2[b] = ap[(size_t)bc * 128 + 64];
-        }
+        for (int b = 0; b < 8; ++b) A[b] = ap[(size_t)(b < nb ? b : 0) * 64];
+        const float *aux = tb.aux + (size_t)s * kMfma8Aux;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) muh[u] = tb.mu[(size_t)s * 8 + 4 * h + u];
-        mc2 = tb.maxc2[s];
+        for (int u = 0; u < 4; ++u) muh[u] = aux[4 * h + u];
+        mc2 = aux[8];
+        mdc = aux[9];
+        sg = aux[10];
     }
     const uint32_t keep = opaque_vgpr(0xFFFFFF00u);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -609,32 +682,46 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
         xb = fetch_x(t + 2);
         if constexpr (LBG) ob = fetch_c(t + 2);
         const float xraw[4] = {xc.x, xc.y, xc.z, xc.w};
-        u32x4 b1, b2;
-        float x2;
+        u32x4 xb16;
+        float x2, e2;  // ||x~||^2 and what its rounding lost, both halves
         {
-            float xv[4];  // relative to the block's centre
+            float xv[4];  // relative to the block's centre (cosine: of length kCosScale)
+            int pa, pb;
+            float p = 0.0f, d2 = 0.0f;
+            if constexpr (METRIC == M_COS) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) xv[u] = xraw[u] - muh[u];
-            float p = 0.0f;
+                for (int u = 0; u < 4; ++u) p = __builtin_fmaf(xraw[u], xraw[u], p);
+                swap_halves(__float_as_int(p), pa, pb);
+                x2 = __int_as_float(pa) + __int_as_float(pb);
+                const float f = kCosScale * __builtin_amdgcn_rsqf(x2);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) xv[u] = xraw[u] * f;
+                p = 0.0f;
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) xv[u] = __builtin_fmaf(xraw[u], sg, muh[u]);
+            }
 #pragma unroll
             for (int u = 0; u < 4; ++u) p = __builtin_fmaf(xv[u], xv[u], p);
-            const uint32_t h01 = bf16_pack2(xv[0], xv[1]), h23 = bf16_pack2(xv[2], xv[3]);
-            const uint32_t l01 = bf16_pack2(xv[0] - __uint_as_float(h01 << 16), xv[1] - __uint_as_float(h01 & 0xffff0000u));
-            const uint32_t l23 = bf16_pack2(xv[2] - __uint_as_float(h23 << 16), xv[3] - __uint_as_float(h23 & 0xffff0000u));
-            // this half's share of ||x||^2 as one bf16 number rounded up (p >= 0; the same in every score
-            // of the row, so its rounding cancels in their differences, and rounding up keeps the
-            // scores from turning negative), then ones for the parts of ||c||^2
-            // (cosine: x2 becomes |x|, and the lower half brings P = 2.01 |x| in)
-            int pa, pb;
-            swap_halves(__float_as_int(p), pa, pb);
-            x2 = __int_as_float(pa) + __int_as_float(pb);  // lower half's share + upper half's, in both
-            if constexpr (METRIC == M_COS) {
-                x2 = __builtin_amdgcn_sqrtf(x2);
-                p = h == 0 ? 2.01f * x2 : 0.0f;
+            using h2 = _Float16 __attribute__((ext_vector_type(2)));
+            uint32_t w[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                w[u] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{xv[2 * u], xv[2 * u + 1]}), h2));
+                float dl, dh;  // x~ - x: one instruction each that reads a half of the pair
+                asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(dl) : "v"(w[u]), "v"(xv[2 * u]));
+                asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(dh) : "v"(w[u]), "v"(xv[2 * u + 1]));
+                d2 = __builtin_fmaf(dl, dl, d2);
+                d2 = __builtin_fmaf(dh, dh, d2);
             }
-            const uint32_t p0 = (__float_as_uint(p) + 0xFFFFu) >> 16;
-            b1 = u32x4{h01, h23, l01, l23};
-            b2 = u32x4{h01, h23, p0, 0x3f803f80u};
+            if constexpr (METRIC != M_COS) {
+                swap_halves(__float_as_int(p), pa, pb);
+                x2 = __int_as_float(pa) + __int_as_float(pb);
+            }
+            swap_halves(__float_as_int(d2), pa, pb);
+            e2 = __int_as_float(pa) + __int_as_float(pb);
+            xb16 = u32x4{w[0], w[1], w[0],
+                         __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{p * kLift8, 1.0f}), h2))};
         }
         int m1 = 0x7f800000, m2 = 0x7f800000;  // +inf
         // One block of 32 centroids.  The tag leaves out the lane half (bit 2), so it is the same in
@@ -642,13 +729,10 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
         // The scores of block b + 1 are made while block b's go through the selection: a matrix
         // instruction holds back the vector instructions of OTHER waves of its SIMD for as long as it
         // runs, but independent vector instructions of its own wave issue in its shadow, so every
-        // matrix instruction is followed by half a block's selection from the same wave.
-#define VQ_MFMA_1(b, acc)                                                                                       \
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, A1[b]),                            \
-                                                  __builtin_bit_cast(bf16x8, b1), zero, 0, 0, 0);
-#define VQ_MFMA_2(b, acc)                                                                                       \
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, A2[b]),                            \
-                                                  __builtin_bit_cast(bf16x8, b2), acc, 0, 0, 0);
+        // matrix instruction is followed by a block's selection from the same wave.
+#define VQ_MFMA(b, acc)                                                                                         \
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, A[b]), __builtin_bit_cast(f16x8, xb16), \
+                                                 zero, 0, 0, 0);
 #define VQ_RUN_KEY(b, acc, p)                                                                                   \
     {                                                                                                           \
         const int gmin = imin(imin(imin(__float_as_int(acc[4 * p]), __float_as_int(acc[4 * p + 1])),            \
@@ -660,20 +744,15 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
 #define VQ_SCORE_BLOCK(b, cur, nb, nxt, more)                                                                   \
     {                                                                                                           \
         int key[4];                                                                                             \
-        if (more) { VQ_MFMA_1(nb, nxt) }                                                                        \
+        if (more) { VQ_MFMA(nb, nxt) }                                                                          \
         __builtin_amdgcn_sched_barrier(0);                                                                      \
-        VQ_RUN_KEY(b, cur, 0) VQ_RUN_KEY(b, cur, 1)                                                             \
-        __builtin_amdgcn_sched_barrier(0);                                                                      \
-        if (more) { VQ_MFMA_2(nb, nxt) }                                                                        \
-        __builtin_amdgcn_sched_barrier(0);                                                                      \
-        VQ_RUN_KEY(b, cur, 2) VQ_RUN_KEY(b, cur, 3)                                                             \
+        VQ_RUN_KEY(b, cur, 0) VQ_RUN_KEY(b, cur, 1) VQ_RUN_KEY(b, cur, 2) VQ_RUN_KEY(b, cur, 3)                  \
         top2_push4(m1, m2, key[0], key[1], key[2], key[3]);                                                     \
         __builtin_amdgcn_sched_barrier(0);                                                                      \
     }
         const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         floatx16 accA, accB;
-        VQ_MFMA_1(0, accA)
-        VQ_MFMA_2(0, accA)
+        VQ_MFMA(0, accA)
         if constexpr (FULL) {
             VQ_SCORE_BLOCK(0, accA, 1, accB, true) VQ_SCORE_BLOCK(1, accB, 2, accA, true)
             VQ_SCORE_BLOCK(2, accA, 3, accB, true) VQ_SCORE_BLOCK(3, accB, 4, accA, true)
@@ -698,8 +777,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
                 VQ_SCORE_BLOCK(1, accB, 0, accA, false)
             }
         }
-#undef VQ_MFMA_1
-#undef VQ_MFMA_2
+#undef VQ_MFMA
 #undef VQ_RUN_KEY
 #undef VQ_SCORE_BLOCK
         // the partner lane (other half) saw the other 16 centroids of every block
@@ -711,12 +789,13 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma_bf(AssignArgs a, MfmaBfT
         const float s1 = __int_as_float(imin(f1, g1));
         const float s2 = __int_as_float(imin(imax(f1, g1), imin(f2, g2)));
         const bool mine = h == 0 && t < lane_tiles;  // the lane's row of this tile exists
-        const float bound = x2 + mc2;  // (cosine: |x|, or NaN)
-        const float margin = 6.103515625e-05f * fabsf(s2) + (METRIC == M_COS ? 2.44140625e-04f : 1.220703125e-04f) * bound;
-        bool sure = (s2 - s1) > margin;  // false for NaN / inf-inf
-        // below 1e-31 the bf16 parts of ||c - mu||^2 may be subnormal, which the matrix cores may
-        // flush: up to 3 * 2^-126 lost, more than the margin allows for at such a bound
-        sure = sure && (bound < (METRIC == M_COS ? 1e15f : 1e29f)) && (bound > (METRIC == M_COS ? 1e-15f : 1e-31f)) && (s1 < 1e29f);
+        // (cosine: the operands' norms are kCosScale; x2 is the row's own)
+        const float bound = (METRIC == M_COS ? kCosScale * kCosScale : x2) + mc2;
+        const float E = (e2 + kFlush8) + mdc;
+        const float margin = __builtin_fmaf(4.001f, __builtin_amdgcn_sqrtf(2.0f * s2 * E), 8.0f * E) +
+                             __builtin_fmaf(6.103515625e-05f, s2, 1.52587890625e-05f * bound);
+        bool sure = (s2 - s1) > margin && s1 < 1.2e5f;  // false for NaN / inf-inf; 1.2e5: below every padding centroid
+        if constexpr (METRIC == M_COS) sure = sure && x2 > 1e-30f && x2 < 1e30f;
         const int first = (int)(__float_as_uint(s1) & 0xFFu);  // first centroid of the best run
         const unsigned long long todo = __ballot(mine && !sure);
         int code;
@@ -839,7 +918,7 @@ static __global__ void __launch_bounds__(256) k_unpad_rows(const float *__restri
 namespace vq {
 
 // ---------------------------------------------------------------------------------------------
-// Wide column blocks on the bf16 matrix cores: the operand split of k_assign_mfma_bf applied to
+// Wide column blocks on the bf16 matrix cores: the operand split of k_assign_mfma8 applied to
 // 16 dimensions at a time.  With the high and low bf16 parts of the centroid operand (ah, al) and
 // of the row operand (xh, xl), a tile of 32 rows x 32 centroids takes three instructions per 16
 // dimensions, ah.xh + al.xh + ah.xl, each with all 16 contraction slots in use (each lane half
@@ -883,7 +962,6 @@ constexpr float kWideT = 0.35f;
 constexpr float kWideRho = 2.0e-4f, kWideHalfT = 0.6f;
 constexpr float kWideTwo = 2.1f, kWideHalfTwo = 2.01f;  // both shares twice, and the roundings of x2, pen and the bound itself
 inline bool wide_half(int sd, int nb) { return sd >= 64 && sd * nb >= 512; }
-using f16x8 = _Float16 __attribute__((ext_vector_type(8)));
 constexpr int kWideCentreMax = 2048;  // widest column block whose centre is staged in LDS
 
 struct MfmaWideBfTables {
@@ -911,7 +989,7 @@ struct MfmaWideBfTables {
 // writes the chunks kc = g, g + 8, ... of centroid 32 b + i and sums their share of ||c||^2; the
 // eight shares are added in g order.  blockmax[s][b] = largest ||c||^2 of the block (NaN stays).
 // mu[s][t] = mean over the k <= 256 centroids of column block s (sum of c / 256, then * 256 / k:
-// no overflow).  Rows and centroids are scored relative to it, as in k_mfma_bf_prep, when that
+// no overflow).  Rows and centroids are scored relative to it, as in k_mfma8_prep, when that
 // shrinks the norms the error bound is proportional to: k_mfma_wide_bf_prep sets shifted[s] = 0
 // and ignores the centre if ||mu||^2 is no more than a quarter of the mean ||c||^2 (or the block
 // is wider than kWideCentreMax), and the assignment kernel then skips the subtraction.  Grid (m, ceil(sd / 32)); thread (i, g) =

@@ -1343,13 +1343,12 @@ static __global__ void k_lbg_advance(LbgState st, int m) {
 // (8-float blocks, streaming path, matrix-core assignment).  Thread j makes centroid j — the mean
 // of a small cluster from its leaf or of a large one from k_lbg_fold8's sum, the re-seed row of
 // an empty cluster (src/vector.rs:315-316, src/utils.rs:98-101) — thread 0 does the loop
-// control of src/utils.rs:57,104-106, and all of them the tables of k_assign_mfma_bf from the
+// control of src/utils.rs:57,104-106, and all of them the tables of k_assign_mfma8 from the
 // centroids they hold.  Needs x 16-byte aligned, ld % 4 == 0 (as the streaming kernel does).
 static __global__ void __launch_bounds__(256) k_lbg_finalize_prep8(
     LbgState st, const float *__restrict__ x, int64_t ld, int k, const uint32_t *__restrict__ reseed, int n_reseed,
     float *__restrict__ cb, const float *__restrict__ big_sum, int nb, u32x4 *__restrict__ atab,
-    float *__restrict__ maxc2, float *__restrict__ mu, uint32_t *__restrict__ stat,
-                                                             uint32_t *__restrict__ stat_next) {
+    float *__restrict__ aux, uint32_t *__restrict__ stat, uint32_t *__restrict__ stat_next) {
     const int s = blockIdx.x, j = threadIdx.x;
     if (s == 0 && j < kStatSlots) stat[j * kStatStride] = stat_next[j * kStatStride] = 0u;
     if (st.done[s]) return;  // the same in the whole workgroup; a finished block is skipped by the assignment
@@ -1395,7 +1394,7 @@ static __global__ void __launch_bounds__(256) k_lbg_finalize_prep8(
         if (!st.changed[s]) st.done[s] = 1;
         st.changed[s] = 0;
     }
-    mfma_bf_prep_block(c, s, j, k, nb, atab, maxc2, mu);
+    mfma8_prep_block(c, s, j, k, nb, atab, aux);
 }
 
 }  // namespace vq

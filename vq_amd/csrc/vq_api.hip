@@ -52,8 +52,8 @@ namespace {
 constexpr size_t kNoAllocTabBytes = 1u << 20;       // A operands: 64 bytes per (column block, padded centroid)
 constexpr int kNoAllocMaxCells = 16384;             // column blocks x centroids (padded to 64) the tables hold
 constexpr int kNoAllocMaxM = 1024;
-constexpr size_t kNoAllocAuxOff = kNoAllocTabBytes;                                   // maxc2 [m], mu [m][8]
-constexpr size_t kNoAllocStatOff = kNoAllocAuxOff + 9 * sizeof(float) * kNoAllocMaxM + 256;  // counters
+constexpr size_t kNoAllocAuxOff = kNoAllocTabBytes;                                   // aux [m][kMfma8Aux]
+constexpr size_t kNoAllocStatOff = kNoAllocAuxOff + vq::kMfma8Aux * sizeof(float) * kNoAllocMaxM + 256;  // counters
 constexpr size_t kNoAllocNormOff = kNoAllocStatOff + sizeof(uint32_t) * vq::kStatSlots * vq::kStatStride;
 constexpr size_t kNoAllocBytes = kNoAllocNormOff + sizeof(float) * kNoAllocMaxCells;  // centroid norms (cosine)
 static_assert(kNoAllocStatOff % 256 == 0 && kNoAllocNormOff % 256 == 0, "scratch areas stay 256-byte aligned");
@@ -135,25 +135,24 @@ int32_t launch_assign_m(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
 
 // 8-float column blocks: bf16-split scores on the matrix cores, undecided rows resolved in the
 // same kernel by the reference-order argmin (assign_mfma.hpp).
-// Where the tables of k_assign_mfma_bf live in the workspace.
+// Where the tables of k_assign_mfma8 live in the workspace.
 struct MfmaTabPtrs {
     vq::u32x4 *atab;
-    float *maxc2, *mu;
+    float *aux;
     uint32_t *stat, *stat_next;  // the counters of this pass; of the next one
     int nb;
 };
 int32_t mfma_tab_ptrs(vq_ctx *ctx, int m, int k, MfmaTabPtrs &t) {
     t.nb = 2 * ((k + 63) / 64);  // blocks of 32 centroids, an even number (the kernel scores them in pairs)
-    // A operands: 2 x 64 lanes x 16 bytes per (s, block of 32 centroids)
-    const size_t n_atab = (size_t)m * t.nb * 512;
+    // A operands: 64 lanes x 16 bytes per (s, block of 32 centroids)
+    const size_t n_atab = (size_t)m * t.nb * 256;
     if (ctx->no_alloc) {  // the fixed scratch array; vq_assign_noalloc has checked that the shape fits
         t.atab = (vq::u32x4 *)ctx->static_scratch;
-        t.maxc2 = (float *)(ctx->static_scratch + kNoAllocAuxOff);
-        t.mu = t.maxc2 + m;
+        t.aux = (float *)(ctx->static_scratch + kNoAllocAuxOff);
         t.stat = t.stat_next = (uint32_t *)(ctx->static_scratch + kNoAllocStatOff);
         return VQ_OK;
     }
-    VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + 9 * (size_t)m) + 64));
+    VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + vq::kMfma8Aux * (size_t)m) + 64));
     const size_t n_stat = (size_t)vq::kStatSlots * vq::kStatStride;
     if (!ctx->mfma_stat.p) {
         VQ_TRY(ensure(ctx, ctx->mfma_stat, sizeof(uint32_t) * 2 * n_stat));
@@ -161,8 +160,7 @@ int32_t mfma_tab_ptrs(vq_ctx *ctx, int m, int k, MfmaTabPtrs &t) {
     }
     float *atab = (float *)ctx->mfma_tab.p;
     t.atab = (vq::u32x4 *)atab;
-    t.maxc2 = atab + n_atab;
-    t.mu = t.maxc2 + m;
+    t.aux = atab + n_atab;
     t.stat = (uint32_t *)ctx->mfma_stat.p + ctx->mfma_stat_cur * n_stat;
     t.stat_next = (uint32_t *)ctx->mfma_stat.p + (ctx->mfma_stat_cur ^ 1) * n_stat;
     return VQ_OK;
@@ -208,14 +206,14 @@ int32_t launch_mfma(vq_ctx *ctx, const vq::AssignArgs &a, bool tables_ready, hip
     MfmaTabPtrs t;
     VQ_TRY(mfma_tab_ptrs(ctx, a.m, a.k, t));
     if (!tables_ready && !own)
-        hipLaunchKernelGGL(vq::k_mfma_bf_prep<METRIC == vq::M_COS>, dim3(a.m), dim3(256), 0, ctx->stream, a.cb, a.m, a.k,
-                           nb, t.atab, t.maxc2, t.mu, t.stat, t.stat_next);
-    vq::MfmaBfTables tb{(const vq::u32x4 *)t.atab, t.maxc2, t.mu, t.stat, nb, t.stat_next};
+        hipLaunchKernelGGL(vq::k_mfma8_prep<METRIC == vq::M_COS>, dim3(a.m), dim3(256), 0, ctx->stream, a.cb, a.m, a.k,
+                           nb, t.atab, t.aux, t.stat, t.stat_next);
+    vq::Mfma8Tables tb{(const vq::u32x4 *)t.atab, t.aux, t.stat, nb, t.stat_next};
     auto pick = [&](auto SGc, auto FULLc) {
         constexpr int SGv = decltype(SGc)::value;
         constexpr bool FULLv = decltype(FULLc)::value;
-        return own ? (const void *)vq::k_assign_mfma_bf<METRIC, LBG, SGv, FULLv, true>
-                   : (const void *)vq::k_assign_mfma_bf<METRIC, LBG, SGv, FULLv, false>;
+        return own ? (const void *)vq::k_assign_mfma8<METRIC, LBG, SGv, FULLv, true>
+                   : (const void *)vq::k_assign_mfma8<METRIC, LBG, SGv, FULLv, false>;
     };
     using Four = std::integral_constant<int, 4>;
     using One = std::integral_constant<int, 1>;
@@ -1453,7 +1451,7 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
         if (fused_tail) {
             hipLaunchKernelGGL(vq::k_lbg_finalize_prep8, dim3(m), dim3(256), 0, st, S, d_x, ld, k,
                                (const uint32_t *)ctx->reseed.p, n_reseed, d_codebooks, (const float *)big_sum,
-                               tabs.nb, tabs.atab, tabs.maxc2, tabs.mu, tabs.stat, tabs.stat_next);
+                               tabs.nb, tabs.atab, tabs.aux, tabs.stat, tabs.stat_next);
         } else {
             hipLaunchKernelGGL(vq::k_lbg_finalize, dim3(cdiv((int64_t)k * sd, 256), m), dim3(256), 0, st, S,
                                d_x, ld, k, sd, (const uint32_t *)ctx->reseed.p, n_reseed, d_codebooks);
