@@ -379,12 +379,122 @@ static __global__ void __launch_bounds__(256) k_mfma8_prep(const float *__restri
     mfma8_prep_block<COS>(c, s, j, k, nb, atab, aux);
 }
 
+// ---- the exact path of k_assign_mfma8 ---------------------------------------------------------
+// Undecided rows of one (tile of 32 rows, column block) are decided by the whole wave in the
+// reference's order (src/utils.rs:63-70, src/pq.rs:166-174): lane l owns centroids l, l + 64,
+// l + 128, l + 192 (read from the wave's copy in LDS) and computes their distances to the row in
+// sequential f32 order; the first of the smallest wins, as strict '<' over ascending indices gives.
+// A NaN distance is never chosen unless it is centroid 0's, which is never replaced.  Euclidean
+// compares the roots, as the reference does: the root is monotone, so the smallest root is that of the
+// smallest square, and only a square within 2^-21 of it can share it; the others' roots are not taken.
+// The row's floats come from the lanes that hold the tile (v_readlane): no memory access at all.  Read from
+// memory again, eight rows to a round trip, and with every root taken: encode of 200,000 x 96 under cosine 93.5
+// us, 88.0 so; of 300,000 x 128, k = 1024, 554 and 535; a fit of 1M x 128 with its encode 5.01 and 4.97 ms.
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
+}
+__device__ __forceinline__ uint32_t umin_u32(uint32_t a, uint32_t b) { return a < b ? a : b; }
+// the smallest of all lanes' values, the same in every lane
+__device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
+    v = umin_u32(v, dpp_u32<0xB1>(v));
+    v = umin_u32(v, dpp_u32<0x4E>(v));
+    v = umin_u32(v, dpp_u32<0x141>(v));
+    v = umin_u32(v, dpp_u32<0x140>(v));
+    uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)v, 0);
+#pragma unroll
+    for (int row = 1; row < 4; ++row) r = umin_u32(r, (uint32_t)__builtin_amdgcn_readlane((int)v, 16 * row));
+    return r;
+}
+
+// A wave's copy of its block's centroids in LDS: two planes, one per half of a centroid, of 16 bytes per
+// centroid.  The pick reads the four pieces of one run per lane, and the runs of the sixteen lanes of a read phase are
+// to lie in different banks (with 32 bytes per centroid 38 % of the kernel's cycles were bank conflicts): 16 bytes
+// stay free after every run, or, under cosine, where the norms need the room (40 KB per workgroup: four of
+// them in a compute unit, cosine 86 -> 83 us), the order inside a run depends on the run.  Unused centroids are far off.
+constexpr float kFar8 = 3e38f;
+template <int METRIC> struct Lds8 {
+    static constexpr bool SWZ = METRIC == M_COS;
+    static constexpr int run_bytes = SWZ ? 64 : 80, plane = 64 * run_bytes;
+    static __device__ __forceinline__ int run(int j, int h) {  // of the run's first centroid j
+        return h * plane + (j >> 2) * run_bytes + (SWZ ? ((j >> 4) & 3) * 16 : 0);
+    }
+    static __device__ __forceinline__ float4 piece(const char *cl, int at, int i) {
+        return *reinterpret_cast<const float4 *>(cl + (SWZ ? at ^ (i * 16) : at + i * 16));
+    }
+    static __device__ __forceinline__ float4 half(const char *cl, int j, int h) { return piece(cl, run(j & ~3, h), j & 3); }
+    static __device__ __forceinline__ void set(char *cl, int j, int h, float4 v) {
+        const int at = run(j & ~3, h), i = j & 3;
+        *reinterpret_cast<float4 *>(cl + (SWZ ? at ^ (i * 16) : at + i * 16)) = v;
+    }
+    static __device__ __forceinline__ void load(const char *cl, int j, float (&c)[8]) {
+        const float4 a = half(cl, j, 0), b = half(cl, j, 1);
+        c[0] = a.x, c[1] = a.y, c[2] = a.z, c[3] = a.w, c[4] = b.x, c[5] = b.y, c[6] = b.z, c[7] = b.w;
+    }
+};
+
+// cl: the column block's centroids in LDS (this wave's copy).
+// todo: ballot of the lanes (below 32) whose row is undecided; xr: the lane's row.
+// Returns the codes of those rows in their lanes, and their distances in dist (other lanes keep
+// `code` and `dist`).
+template <int METRIC>
+__device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, float &dist, const char *cl,
+                                           const float *norms, const float (&xr)[8], int k, int lane) {
+    constexpr uint32_t kInfKey = METRIC == M_COS ? 0xff800000u : 0x7f800000u;  // sort key of +inf
+    while (todo) {
+        const int src = __builtin_amdgcn_readfirstlane(__ffsll(todo) - 1);
+        todo &= todo - 1;
+        float xs[8];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) xs[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xr[d]), src));
+        const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
+        // sort keys of the lane's four distances (Euclidean: of the squares); a NaN sorts behind +inf
+        uint32_t key[4];
+        float first = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int j = lane + 64 * q;
+            float c[8];
+            Lds8<METRIC>::load(cl, j, c);
+            const float d = dist8<METRIC == M_COS ? M_COS : M_SQ>(xs, c, na, METRIC == M_COS ? norms[j] : 0.0f);
+            if (q == 0) first = d;
+            key[q] = j < k && d == d ? dist_key<METRIC>(d) : 0xffffffffu;
+        }
+        const uint32_t best_key = wave_umin(umin_u32(umin_u32(key[0], key[1]), umin_u32(key[2], key[3])));
+        const float d0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(first), 0));
+        int best = 0;
+        float bd = METRIC == M_EUCLID ? sqrtf(d0) : d0;  // centroid 0 where nothing is below +inf
+        if (d0 == d0 && best_key < kInfKey) {  // uniform
+            unsigned long long at[4];
+            bd = key_dist<METRIC>(best_key);
+            if constexpr (METRIC == M_EUCLID) {
+                const uint32_t close = __float_as_uint(__builtin_fmaf(bd, 4.76837158203125e-07f, bd));
+                bd = sqrtf(bd);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) at[q] = __ballot(key[q] <= close);
+                if (__popcll(at[0]) + __popcll(at[1]) + __popcll(at[2]) + __popcll(at[3]) > 1) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) at[q] = __ballot(key[q] <= close && sqrtf(__uint_as_float(key[q])) == bd);
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) at[q] = __ballot(key[q] == best_key);
+            }
+            best = at[0] ? __ffsll(at[0]) - 1 : at[1] ? __ffsll(at[1]) + 63 : at[2] ? __ffsll(at[2]) + 127 : __ffsll(at[3]) + 191;
+        }
+        if (lane == src) {
+            code = best;
+            dist = bd;  // the chosen centroid's distance as computed
+        }
+    }
+    return code;
+}
+
 // The tables of mfma8_prep_block made by one wave for itself (the same operands up to the order in
 // which the sums for the centre and the scale are added, which any centre and scale allow): lane (r, h) makes its
 // own operands of the centroids 32 b + r, dimensions [4h, 4h + 4), from the wave's copy of the centroids in LDS.
 // COS: of the centroids divided by their norms (norms: one per centroid, in LDS).
 template <bool COS>
-__device__ __forceinline__ void own_operands(const float *cl, const float *norms, int k, int nb, int r, int h,
+__device__ __forceinline__ void own_operands(const char *cl, const float *norms, int k, int nb, int r, int h,
                                              u32x4 (&A)[8], float (&muh)[4], float &mc2, float &mdc, float &sg) {
     float cv[8][4];
     float sum[4] = {0.f, 0.f, 0.f, 0.f};
@@ -393,7 +503,7 @@ __device__ __forceinline__ void own_operands(const float *cl, const float *norms
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
         const int j = 32 * b + r;
-        const float4 v = *reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * 8 + 4 * h);
+        const float4 v = Lds8<COS ? M_COS : M_SQ>::half(cl, j, h);
         cv[b][0] = v.x, cv[b][1] = v.y, cv[b][2] = v.z, cv[b][3] = v.w;
 #pragma unroll
         for (int u = 0; u < 4; ++u) sum[u] += j < k ? cv[b][u] * 0.00390625f : 0.0f;  // no overflow for k <= 256
@@ -459,91 +569,6 @@ __device__ __forceinline__ void own_operands(const float *cl, const float *norms
     mdc = md;
 }
 
-// ---- the exact path of k_assign_mfma8 ---------------------------------------------------------
-// Undecided rows of one (tile of 32 rows, column block) are decided by the whole wave in the
-// reference's order (src/utils.rs:63-70, src/pq.rs:166-174): lane l owns centroids l, l + 64,
-// l + 128, l + 192 (read from the wave's copy in LDS) and computes their distances to the row in
-// sequential f32 order; the first of the smallest wins, as strict '<' over ascending indices gives.
-// A NaN distance is never chosen unless it is centroid 0's, which is never replaced.  Euclidean
-// compares the roots, as the reference does: the root is monotone, so the smallest root is that of the
-// smallest square, and only a square within 2^-21 of it can share it; the others' roots are not taken.
-// The row's floats come from the lanes that hold the tile (v_readlane): no memory access at all.  Read from
-// memory again, eight rows to a round trip, and with every root taken: encode of 200,000 x 96 under cosine 93.5
-// us, 88.0 so; of 300,000 x 128, k = 1024, 554 and 535; a fit of 1M x 128 with its encode 5.01 and 4.97 ms.
-template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
-}
-__device__ __forceinline__ uint32_t umin_u32(uint32_t a, uint32_t b) { return a < b ? a : b; }
-// the smallest of all lanes' values, the same in every lane
-__device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
-    v = umin_u32(v, dpp_u32<0xB1>(v));
-    v = umin_u32(v, dpp_u32<0x4E>(v));
-    v = umin_u32(v, dpp_u32<0x141>(v));
-    v = umin_u32(v, dpp_u32<0x140>(v));
-    uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)v, 0);
-#pragma unroll
-    for (int row = 1; row < 4; ++row) r = umin_u32(r, (uint32_t)__builtin_amdgcn_readlane((int)v, 16 * row));
-    return r;
-}
-
-// cl: the column block's centroids in LDS (k x 8 floats, this wave's copy).
-// todo: ballot of the lanes (below 32) whose row is undecided; xr: the lane's row.
-// Returns the codes of those rows in their lanes, and their distances in dist (other lanes keep
-// `code` and `dist`).
-template <int METRIC>
-__device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, float &dist, const float *cl,
-                                           const float *norms, const float (&xr)[8], int k, int lane) {
-    constexpr uint32_t kInfKey = METRIC == M_COS ? 0xff800000u : 0x7f800000u;  // sort key of +inf
-    while (todo) {
-        const int src = __builtin_amdgcn_readfirstlane(__ffsll(todo) - 1);
-        todo &= todo - 1;
-        float xs[8];
-#pragma unroll
-        for (int d = 0; d < 8; ++d) xs[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xr[d]), src));
-        const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
-        // sort keys of the lane's four distances (Euclidean: of the squares); a NaN sorts behind +inf
-        uint32_t key[4];
-        float first = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int j = lane + 64 * q;
-            const float4 *cp = reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * 8);
-            const float4 c0 = cp[0], c1 = cp[1];
-            const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-            const float d = dist8<METRIC == M_COS ? M_COS : M_SQ>(xs, c, na, METRIC == M_COS ? norms[j < k ? j : 0] : 0.0f);
-            if (q == 0) first = d;
-            key[q] = j < k && d == d ? dist_key<METRIC>(d) : 0xffffffffu;
-        }
-        const uint32_t best_key = wave_umin(umin_u32(umin_u32(key[0], key[1]), umin_u32(key[2], key[3])));
-        const float d0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(first), 0));
-        int best = 0;
-        float bd = METRIC == M_EUCLID ? sqrtf(d0) : d0;  // centroid 0 where nothing is below +inf
-        if (d0 == d0 && best_key < kInfKey) {  // uniform
-            unsigned long long at[4];
-            bd = key_dist<METRIC>(best_key);
-            if constexpr (METRIC == M_EUCLID) {
-                const uint32_t close = __float_as_uint(__builtin_fmaf(bd, 4.76837158203125e-07f, bd));
-                bd = sqrtf(bd);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) at[q] = __ballot(key[q] <= close);
-                if (__popcll(at[0]) + __popcll(at[1]) + __popcll(at[2]) + __popcll(at[3]) > 1) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) at[q] = __ballot(key[q] <= close && sqrtf(__uint_as_float(key[q])) == bd);
-                }
-            } else {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) at[q] = __ballot(key[q] == best_key);
-            }
-            best = at[0] ? __ffsll(at[0]) - 1 : at[1] ? __ffsll(at[1]) + 63 : at[2] ? __ffsll(at[2]) + 127 : __ffsll(at[3]) + 191;
-        }
-        if (lane == src) {
-            code = best;
-            dist = bd;  // the chosen centroid's distance as computed
-        }
-    }
-    return code;
-}
-
 // One wave = one column block of 8 floats against a run of tiles of 32 rows.  The wave keeps the
 // A operands of all the block's centroids in registers (8 blocks of 32 centroids x 4 registers) and a copy of the block's centroids in LDS, and streams the rows past them: the
 // inner loop reads no memory.  A lane's 16 scores of a tile are four runs of four consecutive
@@ -552,8 +577,12 @@ __device__ __forceinline__ int exact_rows8(unsigned long long todo, int code, fl
 // five v_min3 / v_med3 per four runs: 17 vector instructions for 16 scores).  When the two best
 // keys are further apart than the error bound, every centroid outside the best run is provably
 // further from the row than the run's best one, and the reference's choice is the first smallest
-// exact distance among the run's four centroids, which the two lane halves compute from the LDS
-// copy, two centroids each.  Otherwise the row goes through the reference-order argmin.
+// exact distance among the run's four centroids.  Each lane half sums its four dimensions of all four with fused
+// multiply-adds; the smallest sum decides where it is clear of the second, else the run is gone through
+// in the reference's order.  (Two full chains of rounded products per half, and two roots under Euclidean,
+// took 46 to 75 vector instructions where this takes 36: a pass of a fit over 1M x 16 blocks 340 -> 320 us, fit and
+// encode of 1M x 128 4.61 -> 4.42 ms.)  Otherwise the row goes through the reference-order argmin.
+// Bound by vector-instruction issue: 275 per tile and column block, half of them the selection's, 2.1 GHz.
 // SG = 4: the four waves of a workgroup take the four column blocks of one 128-byte line of the
 // same rows.  SG = 1 (m not a multiple of 4): the four waves take consecutive runs of one block.
 // FULL: 8 blocks of 32 centroids (k above 224), scored without a branch between them.
@@ -564,8 +593,8 @@ template <int METRIC, bool LBG, int SG, bool FULL, bool OWN = false>
 __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tables tb, int run_tiles, int64_t nruns,
                                                             int64_t run_stride) {
     constexpr int SD = 8;
-    __shared__ __attribute__((aligned(16))) float lds_cb[4][256 * SD];
-    __shared__ float lds_norm[METRIC == M_COS ? 4 : 1][METRIC == M_COS ? 256 : 1];  // the centroids' norms
+    __shared__ __attribute__((aligned(16))) char lds_cb[4][2 * Lds8<METRIC>::plane];
+    __shared__ float lds_norm[METRIC == M_COS ? 4 : 1][METRIC == M_COS ? 512 : 1];  // the centroids' norms, then their reciprocals
     // the wave's number through readfirstlane: what follows from it (column block, first row, base
     // addresses) is then uniform for the compiler and lives in scalar registers
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -586,16 +615,15 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
     }
 
     // the block's centroids: this wave's copy in LDS (no other wave reads it: no barrier)
-    float *cl = lds_cb[wave];
+    char *cl = lds_cb[wave];
     {
         const float4 *src = reinterpret_cast<const float4 *>(a.cb + (size_t)s * k * SD);
-        float4 *dst = reinterpret_cast<float4 *>(cl);
         const int nv = 2 * k;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             const int i = lane + 64 * c;
             const float4 v = src[i < nv ? i : 0];
-            if (i < nv) dst[i] = v;
+            Lds8<METRIC>::set(cl, i >> 1, i & 1, i < nv ? v : make_float4(kFar8, kFar8, kFar8, kFar8));
         }
     }
     float *norms = lds_norm[METRIC == M_COS ? wave : 0];
@@ -605,10 +633,10 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int j = lane + 64 * q;
-            const float4 *cp = reinterpret_cast<const float4 *>(cl + (j < k ? j : 0) * SD);
-            const float4 c0 = cp[0], c1 = cp[1];
-            const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+            float c[8];
+            Lds8<METRIC>::load(cl, j, c);
             norms[j] = seq_norm8(c);
+            norms[256 + j] = norms[j] == 0.0f ? 0.0f : 1.0f / norms[j];
         }
     }
     // the A operands of every block of 32 centroids, the centre's dimensions [4h, 4h + 4), the bound
@@ -633,6 +661,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
         sg = aux[10];
     }
     const uint32_t keep = opaque_vgpr(0xFFFFFF00u);
+    const float acc8 = 4.57763671875e-05f * mc2;  // 2^-16 * 3: see the margin
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
 
@@ -683,7 +712,8 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
         if constexpr (LBG) ob = fetch_c(t + 2);
         const float xraw[4] = {xc.x, xc.y, xc.z, xc.w};
         u32x4 xb16;
-        float x2, e2;  // ||x~||^2 and what its rounding lost, both halves
+        float x2 = 0.0f, rx = 0.0f;  // cosine: ||x||^2 and 1 / ||x|| of the row as it is
+        float e2;                    // what the rounding lost, squared, both halves
         {
             float xv[4];  // relative to the block's centre (cosine: of length kCosScale)
             int pa, pb;
@@ -693,7 +723,8 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
                 for (int u = 0; u < 4; ++u) p = __builtin_fmaf(xraw[u], xraw[u], p);
                 swap_halves(__float_as_int(p), pa, pb);
                 x2 = __int_as_float(pa) + __int_as_float(pb);
-                const float f = kCosScale * __builtin_amdgcn_rsqf(x2);
+                rx = __builtin_amdgcn_rsqf(x2);
+                const float f = kCosScale * rx;
 #pragma unroll
                 for (int u = 0; u < 4; ++u) xv[u] = xraw[u] * f;
                 p = 0.0f;
@@ -713,10 +744,6 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
                 asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(dh) : "v"(w[u]), "v"(xv[2 * u + 1]));
                 d2 = __builtin_fmaf(dl, dl, d2);
                 d2 = __builtin_fmaf(dh, dh, d2);
-            }
-            if constexpr (METRIC != M_COS) {
-                swap_halves(__float_as_int(p), pa, pb);
-                x2 = __int_as_float(pa) + __int_as_float(pb);
             }
             swap_halves(__float_as_int(d2), pa, pb);
             e2 = __int_as_float(pa) + __int_as_float(pb);
@@ -789,50 +816,109 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
         const float s1 = __int_as_float(imin(f1, g1));
         const float s2 = __int_as_float(imin(imax(f1, g1), imin(f2, g2)));
         const bool mine = h == 0 && t < lane_tiles;  // the lane's row of this tile exists
-        // (cosine: the operands' norms are kCosScale; x2 is the row's own)
-        const float bound = (METRIC == M_COS ? kCosScale * kCosScale : x2) + mc2;
         const float E = (e2 + kFlush8) + mdc;
-        const float margin = __builtin_fmaf(4.001f, __builtin_amdgcn_sqrtf(2.0f * s2 * E), 8.0f * E) +
-                             __builtin_fmaf(6.103515625e-05f, s2, 1.52587890625e-05f * bound);
-        bool sure = (s2 - s1) > margin && s1 < 1.2e5f;  // false for NaN / inf-inf; 1.2e5: below every padding centroid
-        if constexpr (METRIC == M_COS) sure = sure && x2 > 1e-30f && x2 < 1e30f;
-        const int first = (int)(__float_as_uint(s1) & 0xFFu);  // first centroid of the best run
-        const unsigned long long todo = __ballot(mine && !sure);
+        // (||x||^2 <= 2 (s2 + ||c||^2) + ...: the accumulation's share without the row's norm)
+        const float margin = __builtin_fmaf(4.001f, __builtin_amdgcn_sqrtf(2.0f * s2 * E), __builtin_fmaf(8.0f, E, acc8)) +
+                             9.1552734375e-05f * s2;
+        // false for NaN / inf-inf; 1.2e5: below every padding centroid
+        const bool near = (s2 - s1) > margin && s1 < 1.2e5f && (METRIC != M_COS || (x2 > 1e-30f && x2 < 1e30f));
+        const int first = (int)(__float_as_uint(s1) & 0xFCu);  // first centroid of the best run
+        // The best of the run's four centroids.  Each lane half takes its four dimensions of all of them (fused
+        // multiply-adds), the halves' sums meet two centroids each; the smallest that is clear of the second by
+        // 2^-17, more than this sum and the reference's round, is the reference's choice.
         int code;
-        float dist;  // of the chosen centroid, as the reference computes it
-        float xs[8];  // the lane's row
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            int lo, hi;
-            swap_halves(__float_as_int(xraw[u]), lo, hi);
-            xs[u] = __int_as_float(lo);
-            xs[4 + u] = __int_as_float(hi);
-        }
+        bool clear;
         {
-            // the best run's four centroids, two per lane half, in the reference's order
+            const int run = Lds8<METRIC>::run(first, h);
+            float p[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float4 v = Lds8<METRIC>::piece(cl, run, i);
+                const float c[4] = {v.x, v.y, v.z, v.w};
+                if constexpr (METRIC == M_COS) {
+                    p[i] = xraw[0] * c[0];
+#pragma unroll
+                    for (int u = 1; u < 4; ++u) p[i] = __builtin_fmaf(xraw[u], c[u], p[i]);
+                } else {
+                    float d = xraw[0] - c[0];
+                    p[i] = d * d;
+#pragma unroll
+                    for (int u = 1; u < 4; ++u) {
+                        d = xraw[u] - c[u];
+                        p[i] = __builtin_fmaf(d, d, p[i]);
+                    }
+                }
+            }
+            // lower half: centroids first, first + 1; upper half: first + 2, first + 3
+            const auto r02 = __builtin_amdgcn_permlane32_swap(__float_as_int(p[0]), __float_as_int(p[2]), false, false);
+            const auto r13 = __builtin_amdgcn_permlane32_swap(__float_as_int(p[1]), __float_as_int(p[3]), false, false);
+            float da = __int_as_float((int)r02[0]) + __int_as_float((int)r02[1]);
+            float db = __int_as_float((int)r13[0]) + __int_as_float((int)r13[1]);
             const int j0 = first + 2 * h;
-            const int ja = j0 < k ? j0 : k - 1, jb = j0 + 1 < k ? j0 + 1 : k - 1;
-            const float4 *pa = reinterpret_cast<const float4 *>(cl + ja * SD);
-            const float4 *pb = reinterpret_cast<const float4 *>(cl + jb * SD);
-            const float4 ca0 = pa[0], ca1 = pa[1], cb0 = pb[0], cb1 = pb[1];
-            const float ca[8] = {ca0.x, ca0.y, ca0.z, ca0.w, ca1.x, ca1.y, ca1.z, ca1.w};
-            const float cc[8] = {cb0.x, cb0.y, cb0.z, cb0.w, cb1.x, cb1.y, cb1.z, cb1.w};
-            const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
-            const float da = dist8<METRIC>(xs, ca, na, METRIC == M_COS ? norms[ja] : 0.0f);
-            const float db = dist8<METRIC>(xs, cc, na, METRIC == M_COS ? norms[jb] : 0.0f);
-            const bool second = (j0 + 1 < k) && (db < da);  // strict: the first of equals
-            uint32_t kd = dist_key<METRIC>(second ? db : da);
-            const uint32_t ki = (uint32_t)(second ? j0 + 1 : j0);
-            kd = j0 < k ? kd : 0xffffffffu;  // a padding centroid
-            int dlo, dhi, ilo, ihi;
-            swap_halves((int)kd, dlo, dhi);
-            swap_halves((int)ki, ilo, ihi);
-            code = (uint32_t)dhi < (uint32_t)dlo ? ihi : ilo;  // the lower half holds the lower indices
-            dist = key_dist<METRIC>((uint32_t)dhi < (uint32_t)dlo ? (uint32_t)dhi : (uint32_t)dlo);
+            int ka, kb;  // sort keys: non-negative distances as they are
+            if constexpr (METRIC == M_COS) {
+                // 1 - cos (a centroid of norm zero: 1), lifted so that rounding leaves it positive
+                const float2 inv = *reinterpret_cast<const float2 *>(norms + 256 + j0);
+                da = __builtin_fmaf(-(da * rx), inv.x, 1.001f);
+                db = __builtin_fmaf(-(db * rx), inv.y, 1.001f);
+                ka = j0 < k ? __float_as_int(da) : 0x7f800000;
+                kb = j0 + 1 < k ? __float_as_int(db) : 0x7f800000;
+            } else {
+                ka = __float_as_int(da);
+                kb = __float_as_int(db);
+            }
+            int lo = imin(ka, kb), hi = imax(ka, kb), at = j0 + (kb < ka ? 1 : 0);
+            int l0, l1, h0, h1, a0, a1;
+            swap_halves(lo, l0, l1);
+            swap_halves(hi, h0, h1);
+            swap_halves(at, a0, a1);
+            code = l1 < l0 ? a1 : a0;  // (lower half: 0 its own, 1 the partner's)
+            const float best = __int_as_float(imin(l0, l1));
+            const float second = __int_as_float(imin3(imax(l0, l1), h0, h1));
+            // (1e-36: sums of squares in the subnormal range)
+            if constexpr (METRIC == M_COS)
+                clear = second - best > 7.62939453125e-06f;
+            else
+                clear = __builtin_fmaf(second, 0.99999237060546875f, -1e-36f) > best;
         }
-        if (todo) {  // the same in every lane: the reference-order argmin of the undecided rows
-            n_exact += (uint32_t)__popcll(todo);
-            code = exact_rows8<METRIC>(todo, code, dist, cl, norms, xs, k, lane);
+        const unsigned long long todo = __ballot(mine && !near), ties = __ballot(mine && near && !clear);
+        float dist = 0.0f;  // of the chosen centroid, as the reference computes it (where it is asked for)
+        bool want_dist = false;
+        if constexpr (!LBG) want_dist = a.dist != nullptr;
+        if ((todo | ties) != 0 || want_dist) {  // the same in every lane
+            float xs[8];  // the lane's row
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                int lo, hi;
+                swap_halves(__float_as_int(xraw[u]), lo, hi);
+                xs[u] = __int_as_float(lo);
+                xs[4 + u] = __int_as_float(hi);
+            }
+            const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
+            if (ties) {
+                // the run's four centroids in the reference's order: the first of the smallest
+                float bd = 0.0f;
+                int bj = first;
+                for (int i = 0; i < 4; ++i) {
+                    float c[8];
+                    Lds8<METRIC>::load(cl, first + i, c);
+                    const float d = dist8<METRIC>(xs, c, na, METRIC == M_COS ? norms[first + i] : 0.0f);
+                    if (i == 0 || (first + i < k && d < bd)) {
+                        bd = d;
+                        bj = first + i;
+                    }
+                }
+                code = clear ? code : bj;
+            }
+            if (want_dist) {
+                float c[8];
+                Lds8<METRIC>::load(cl, code, c);
+                dist = dist8<METRIC>(xs, c, na, METRIC == M_COS ? norms[code] : 0.0f);
+            }
+            if (todo) {  // the reference-order argmin of the undecided rows
+                n_exact += (uint32_t)__popcll(todo);
+                code = exact_rows8<METRIC>(todo, code, dist, cl, norms, xs, k, lane);
+            }
         }
         if (mine) {
             const uint32_t rr = 32u * (uint32_t)t + (uint32_t)r;  // row within the run
@@ -846,7 +932,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
                 a.codes[out0 + rr * (uint32_t)m] = (uint8_t)code;
                 if (a.dist) a.dist[out0 + rr * (uint32_t)m] = dist;  // for the caller that merges chunks of a larger codebook
                 if (a.out16) {  // the reconstruction, round to nearest even
-                    const float4 c0 = *reinterpret_cast<const float4 *>(cl + code * SD), c1 = *reinterpret_cast<const float4 *>(cl + code * SD + 4);
+                    const float4 c0 = Lds8<METRIC>::half(cl, code, 0), c1 = Lds8<METRIC>::half(cl, code, 1);
                     auto two = [](float lo, float hi) {
                         return (uint32_t)__half_as_ushort(__float2half_rn(lo)) | ((uint32_t)__half_as_ushort(__float2half_rn(hi)) << 16);
                     };

@@ -28,7 +28,7 @@
 #define VQ_MFMA_ROUND 768  // workgroups of one round: three per compute unit
 #endif
 #ifndef VQ_MFMA_OWN
-#define VQ_MFMA_OWN 8    // most tiles per workgroup of a one-round grid
+#define VQ_MFMA_OWN 8   // most tiles per workgroup of a one-round grid
 #endif
 #include "lbg_update.hpp"
 #include "calibrate.hpp"
