@@ -28,7 +28,7 @@
 #define VQ_MFMA_ROUND 768  // workgroups of one round: three per compute unit
 #endif
 #ifndef VQ_MFMA_OWN
-#define VQ_MFMA_OWN 8   // most tiles per workgroup of a one-round grid
+#define VQ_MFMA_OWN 16  // most tiles per workgroup of a one-round grid
 #endif
 #include "lbg_update.hpp"
 #include "calibrate.hpp"
@@ -187,10 +187,9 @@ int32_t launch_mfma(vq_ctx *ctx, const vq::AssignArgs &a, bool tables_ready, hip
     while (run_tiles > 1 && cdiv(tiles, per_run * run_tiles) * groups < 8192) run_tiles >>= 1;
     // Up to VQ_MFMA_OWN tiles for each workgroup of a single round: what counts then is the time of one
     // workgroup, and every wave makes its operands itself (OWN) instead of waiting for the launch that
-    // makes the tables (10,000 x 128, m = 16, k = 256: 18.0 us in two launches -> 13.1; 40,000: 34 -> 26).
-    // Above that line as below it one round is the faster way for a while: 50,000 rows (9 tiles) 38 us as it
-    // runs and 30 by one round, 100,000 (17) 56 and 48, 200,000 (33) 88 and 83, 400,000 (66) 152 and 150; m =
-    // 10, a column block per workgroup: 100,000 (11) 42 and 34, but 200,000 (21) 64 and 69, 400,000 104 and 125.
+    // makes the tables.  Four rounds with that launch -> one round, m = 16, k = 256: 1,000 rows 11.4 -> 8.3 us, 10,000
+    // 17 -> 14, 50,000 (9 tiles) 32.9 -> 29.4, 100,000 (17) 49.6 -> 49.3, 200,000 (33) 76 -> 82; k = 64, 50,000
+    // 24.1 -> 19.7; m = 10, a column block per workgroup: 100,000 (11) 35.5 -> 32.7, 200,000 (21) 56 -> 66.
     const int64_t share = cdiv(tiles * groups, per_run * VQ_MFMA_ROUND);
     const bool own = !tables_ready && !ctx->no_alloc && share <= VQ_MFMA_OWN;
     if (own) run_tiles = (int)share;
