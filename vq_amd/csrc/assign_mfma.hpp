@@ -226,9 +226,9 @@ __device__ __forceinline__ float dist8(const float (&x)[8], const float (&c)[8],
 // The scale of a column block: the power of two that brings the centroids' root mean square norm about the
 // centre to 4 ... 8 (r2: the mean square; NaN where the scores cannot decide).  A centroid is then no longer
 // than 128 (k <= 256), and a row's share of ||x||^2 fits binary16 up to 32 ... 64 times that norm.
-__device__ __forceinline__ float mfma8_scale(float r2) {
+__device__ __forceinline__ float mfma8_scale(float r2, int up = 2, float most = 1e36f) {
     if (r2 == 0.0f) return 1.0f;  // all centroids are the same
-    return r2 > 1e-36f && r2 < 1e36f ? ldexpf(1.0f, 2 - (ilogbf(r2) >> 1)) : __builtin_nanf("");
+    return r2 > 1e-36f && r2 < most ? ldexpf(1.0f, up - (ilogbf(r2) >> 1)) : __builtin_nanf("");
 }
 // The A operand of one centroid and one lane half: a[t] = -2 c[t] of the half's four dimensions, scaled.
 // Elements below the normal range of binary16 count as zero, whatever the matrix cores make of them.
@@ -569,6 +569,80 @@ __device__ __forceinline__ void own_operands(const char *cl, const float *norms,
     mdc = md;
 }
 
+// The row operand of a tile: the lane's four dimensions relative to the centre (cosine: of length kCosScale).
+struct Row8 {
+    u32x4 b16;
+    float e2;            // what the rounding lost, squared, both halves
+    float x2 = 0.0f, rx = 0.0f;  // cosine: ||x||^2 and 1 / ||x|| of the row as it is
+};
+template <int METRIC>
+__device__ __forceinline__ Row8 row8(const float (&xraw)[4], float sg, const float (&muh)[4]) {
+    Row8 o;
+    float xv[4];
+    int pa, pb;
+    float p = 0.0f, d2 = 0.0f;
+    if constexpr (METRIC == M_COS) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p = __builtin_fmaf(xraw[u], xraw[u], p);
+        swap_halves(__float_as_int(p), pa, pb);
+        o.x2 = __int_as_float(pa) + __int_as_float(pb);
+        o.rx = __builtin_amdgcn_rsqf(o.x2);
+        const float f = kCosScale * o.rx;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) xv[u] = xraw[u] * f;
+        p = 0.0f;
+    } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) xv[u] = __builtin_fmaf(xraw[u], sg, muh[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) p = __builtin_fmaf(xv[u], xv[u], p);
+    using h2 = _Float16 __attribute__((ext_vector_type(2)));
+    uint32_t w[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        w[u] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{xv[2 * u], xv[2 * u + 1]}), h2));
+        float dl, dh;  // x~ - x: one instruction each that reads a half of the pair
+        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(dl) : "v"(w[u]), "v"(xv[2 * u]));
+        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(dh) : "v"(w[u]), "v"(xv[2 * u + 1]));
+        d2 = __builtin_fmaf(dl, dl, d2);
+        d2 = __builtin_fmaf(dh, dh, d2);
+    }
+    swap_halves(__float_as_int(d2), pa, pb);
+    o.e2 = __int_as_float(pa) + __int_as_float(pb);
+    o.b16 = u32x4{w[0], w[1], w[0],
+                  __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{p * kLift8, 1.0f}), h2))};
+    return o;
+}
+// Whether the best of the two smallest keys has won (false for NaN / inf - inf); e2c: the centroids' share of
+// the rounding, acc8: 3 * 2^-16 max ||c~||^2 (||x||^2 <= 2 (s2 + ||c||^2) stands for the row's norm).
+template <int METRIC>
+__device__ __forceinline__ bool decided8(float s1, float s2, const Row8 &row, float e2c, float acc8) {
+    const float E = (row.e2 + kFlush8) + e2c;
+    const float margin = __builtin_fmaf(4.001f, __builtin_amdgcn_sqrtf(2.0f * s2 * E), __builtin_fmaf(8.0f, E, acc8)) +
+                         9.1552734375e-05f * s2;
+    // 1.2e5: below every padding centroid
+    return (s2 - s1) > margin && s1 < 1.2e5f && (METRIC != M_COS || (row.x2 > 1e-30f && row.x2 < 1e30f));
+}
+// A lane half's share of the distance to a centroid: its four dimensions, fused.  Cosine: of the inner product.
+template <int METRIC> __device__ __forceinline__ float share8(const float (&xraw)[4], float4 v) {
+    const float c[4] = {v.x, v.y, v.z, v.w};
+    if constexpr (METRIC == M_COS) {
+        float p = xraw[0] * c[0];
+#pragma unroll
+        for (int u = 1; u < 4; ++u) p = __builtin_fmaf(xraw[u], c[u], p);
+        return p;
+    } else {
+        float d = xraw[0] - c[0], p = d * d;
+#pragma unroll
+        for (int u = 1; u < 4; ++u) {
+            d = xraw[u] - c[u];
+            p = __builtin_fmaf(d, d, p);
+        }
+        return p;
+    }
+}
+
 // One wave = one column block of 8 floats against a run of tiles of 32 rows.  The wave keeps the
 // A operands of all the block's centroids in registers (8 blocks of 32 centroids x 4 registers) and a copy of the block's centroids in LDS, and streams the rows past them: the
 // inner loop reads no memory.  A lane's 16 scores of a tile are four runs of four consecutive
@@ -711,45 +785,8 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
         xb = fetch_x(t + 2);
         if constexpr (LBG) ob = fetch_c(t + 2);
         const float xraw[4] = {xc.x, xc.y, xc.z, xc.w};
-        u32x4 xb16;
-        float x2 = 0.0f, rx = 0.0f;  // cosine: ||x||^2 and 1 / ||x|| of the row as it is
-        float e2;                    // what the rounding lost, squared, both halves
-        {
-            float xv[4];  // relative to the block's centre (cosine: of length kCosScale)
-            int pa, pb;
-            float p = 0.0f, d2 = 0.0f;
-            if constexpr (METRIC == M_COS) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) p = __builtin_fmaf(xraw[u], xraw[u], p);
-                swap_halves(__float_as_int(p), pa, pb);
-                x2 = __int_as_float(pa) + __int_as_float(pb);
-                rx = __builtin_amdgcn_rsqf(x2);
-                const float f = kCosScale * rx;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) xv[u] = xraw[u] * f;
-                p = 0.0f;
-            } else {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) xv[u] = __builtin_fmaf(xraw[u], sg, muh[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) p = __builtin_fmaf(xv[u], xv[u], p);
-            using h2 = _Float16 __attribute__((ext_vector_type(2)));
-            uint32_t w[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                w[u] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{xv[2 * u], xv[2 * u + 1]}), h2));
-                float dl, dh;  // x~ - x: one instruction each that reads a half of the pair
-                asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(dl) : "v"(w[u]), "v"(xv[2 * u]));
-                asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(dh) : "v"(w[u]), "v"(xv[2 * u + 1]));
-                d2 = __builtin_fmaf(dl, dl, d2);
-                d2 = __builtin_fmaf(dh, dh, d2);
-            }
-            swap_halves(__float_as_int(d2), pa, pb);
-            e2 = __int_as_float(pa) + __int_as_float(pb);
-            xb16 = u32x4{w[0], w[1], w[0],
-                         __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{p * kLift8, 1.0f}), h2))};
-        }
+        const Row8 row = row8<METRIC>(xraw, sg, muh);
+        const u32x4 xb16 = row.b16;
         int m1 = 0x7f800000, m2 = 0x7f800000;  // +inf
         // One block of 32 centroids.  The tag leaves out the lane half (bit 2), so it is the same in
         // every lane and lives in scalar registers.
@@ -816,12 +853,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
         const float s1 = __int_as_float(imin(f1, g1));
         const float s2 = __int_as_float(imin(imax(f1, g1), imin(f2, g2)));
         const bool mine = h == 0 && t < lane_tiles;  // the lane's row of this tile exists
-        const float E = (e2 + kFlush8) + mdc;
-        // (||x||^2 <= 2 (s2 + ||c||^2) + ...: the accumulation's share without the row's norm)
-        const float margin = __builtin_fmaf(4.001f, __builtin_amdgcn_sqrtf(2.0f * s2 * E), __builtin_fmaf(8.0f, E, acc8)) +
-                             9.1552734375e-05f * s2;
-        // false for NaN / inf-inf; 1.2e5: below every padding centroid
-        const bool near = (s2 - s1) > margin && s1 < 1.2e5f && (METRIC != M_COS || (x2 > 1e-30f && x2 < 1e30f));
+        const bool near = decided8<METRIC>(s1, s2, row, mdc, acc8);
         const int first = (int)(__float_as_uint(s1) & 0xFCu);  // first centroid of the best run
         // The best of the run's four centroids.  Each lane half takes its four dimensions of all of them (fused
         // multiply-adds), the halves' sums meet two centroids each; the smallest that is clear of the second by
@@ -832,23 +864,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
             const int run = Lds8<METRIC>::run(first, h);
             float p[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float4 v = Lds8<METRIC>::piece(cl, run, i);
-                const float c[4] = {v.x, v.y, v.z, v.w};
-                if constexpr (METRIC == M_COS) {
-                    p[i] = xraw[0] * c[0];
-#pragma unroll
-                    for (int u = 1; u < 4; ++u) p[i] = __builtin_fmaf(xraw[u], c[u], p[i]);
-                } else {
-                    float d = xraw[0] - c[0];
-                    p[i] = d * d;
-#pragma unroll
-                    for (int u = 1; u < 4; ++u) {
-                        d = xraw[u] - c[u];
-                        p[i] = __builtin_fmaf(d, d, p[i]);
-                    }
-                }
-            }
+            for (int i = 0; i < 4; ++i) p[i] = share8<METRIC>(xraw, Lds8<METRIC>::piece(cl, run, i));
             // lower half: centroids first, first + 1; upper half: first + 2, first + 3
             const auto r02 = __builtin_amdgcn_permlane32_swap(__float_as_int(p[0]), __float_as_int(p[2]), false, false);
             const auto r13 = __builtin_amdgcn_permlane32_swap(__float_as_int(p[1]), __float_as_int(p[3]), false, false);
@@ -859,8 +875,8 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
             if constexpr (METRIC == M_COS) {
                 // 1 - cos (a centroid of norm zero: 1), lifted so that rounding leaves it positive
                 const float2 inv = *reinterpret_cast<const float2 *>(norms + 256 + j0);
-                da = __builtin_fmaf(-(da * rx), inv.x, 1.001f);
-                db = __builtin_fmaf(-(db * rx), inv.y, 1.001f);
+                da = __builtin_fmaf(-(da * row.rx), inv.x, 1.001f);
+                db = __builtin_fmaf(-(db * row.rx), inv.y, 1.001f);
                 ka = j0 < k ? __float_as_int(da) : 0x7f800000;
                 kb = j0 + 1 < k ? __float_as_int(db) : 0x7f800000;
             } else {

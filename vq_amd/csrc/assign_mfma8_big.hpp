@@ -1,0 +1,440 @@
+// Nearest-centroid assignment for 8-float column blocks with 257 to 2048 centroids: one pass over the rows for
+// the whole codebook, 16-bit codes.  The scores, their bound and the decision are those of k_assign_mfma8
+// (assign_mfma.hpp); what differs is where the operands lie and how a row's best centroids are kept.
+//
+// This translation unit must be compiled with -ffp-contract=off.
+#pragma once
+#include "assign_mfma.hpp"
+
+namespace vq {
+
+constexpr int kBig8Max = 2048;
+constexpr float kBig8Far = 1e18f;   // components of the padding centroids: squares stay finite, and farther off than
+                                    // any centroid of a block whose scale exists (kBig8Rms)
+constexpr float kBig8Rms = 1e30f;   // largest mean square norm about the centre that is scored
+
+struct Big8Args {
+    const float *x;
+    int64_t n, ld;
+    int m, k;
+    const float *cb;     // [m][k][8], 16-byte aligned
+    uint16_t *codes;     // [n][m]
+    int64_t stride;      // workgroups of a column block
+    uint32_t *stat, *stat_next;  // counters of undecided pairs: of this pass, and of the next (cleared)
+};
+
+// Centroids padded to whole pairs of blocks of 32; operands 32 bytes and the centroid itself 32 bytes each, under
+// cosine its norm and the reciprocal.
+inline int big8_padded(int k) { return (k + 63) / 64 * 64; }
+inline size_t big8_lds(bool cosine, int k) { return (size_t)big8_padded(k) * (64 + (cosine ? 8 : 0)); }
+
+// The workgroup's copy of its block's centroids: planes as in Lds8, runs of 64 bytes with the order inside a
+// run depending on the run, so that a phase of the pick's reads, sixteen runs at random, meets all banks.
+struct LdsBig8 {
+    char *cl;
+    int plane;
+    __device__ __forceinline__ int run(int j, int h) const { return h * plane + j * 16 + ((j >> 4) & 3) * 16; }
+    __device__ __forceinline__ float4 piece(int at, int i) const { return *reinterpret_cast<const float4 *>(cl + (at ^ (i * 16))); }
+    __device__ __forceinline__ float4 half(int j, int h) const { return piece(run(j & ~3, h), j & 3); }
+    __device__ __forceinline__ void set(int j, int h, float4 v) const {
+        *reinterpret_cast<float4 *>(cl + (run(j & ~3, h) ^ ((j & 3) * 16))) = v;
+    }
+    __device__ __forceinline__ void load(int j, float (&c)[8]) const {
+        const float4 a = half(j, 0), b = half(j, 1);
+        c[0] = a.x, c[1] = a.y, c[2] = a.z, c[3] = a.w, c[4] = b.x, c[5] = b.y, c[6] = b.z, c[7] = b.w;
+    }
+};
+
+// The undecided rows of a tile, one after the other: a lane takes the centroids lane, lane + 64, ... by fused
+// sums and keeps the two smallest.  One lane with one centroid within 2^-16 of the smallest has the answer;
+// otherwise the reference's distances decide, the first of the smallest (a NaN sorts behind +inf, centroid 0 wins
+// where it is NaN or nothing is below +inf).
+template <int METRIC>
+__device__ __forceinline__ int exact_rows_big8(unsigned long long todo, int code, const LdsBig8 &cl, const float *norms,
+                                               int kp, const float (&xr)[8], float rx, int k, int lane) {
+    constexpr uint32_t kInfKey = METRIC == M_COS ? 0xff800000u : 0x7f800000u;  // sort key of +inf
+    constexpr int M = METRIC == M_COS ? M_COS : M_SQ;  // Euclidean: squares first
+    const int at0 = cl.run(lane & ~3, 0) ^ ((lane & 3) * 16);  // of centroid lane; 64 centroids on is 1 KB on
+    while (todo) {
+        const int src = __builtin_amdgcn_readfirstlane(__ffsll(todo) - 1);
+        todo &= todo - 1;
+        float xs[8];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) xs[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xr[d]), src));
+        int best = -1;
+        {
+            const float rxs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rx), src));
+            const float lo4[4] = {xs[0], xs[1], xs[2], xs[3]}, hi4[4] = {xs[4], xs[5], xs[6], xs[7]};
+            uint32_t lo = 0xffffffffu, second = 0xffffffffu, first = 0;
+            int at = 0;
+            for (int q = 0; q < k; q += 64) {
+                const char *p = cl.cl + at0 + 16 * q;
+                float d = share8<METRIC>(lo4, *reinterpret_cast<const float4 *>(p)) +
+                          share8<METRIC>(hi4, *reinterpret_cast<const float4 *>(p + cl.plane));
+                if constexpr (METRIC == M_COS) d = __builtin_fmaf(-(d * rxs), norms[kp + q + lane], 1.001f);
+                const uint32_t key = __float_as_uint(d);
+                if (q == 0) first = key;
+                second = umin_u32(second, key < lo ? lo : key);
+                at = key < lo ? q + lane : at;
+                lo = umin_u32(lo, key);
+            }
+            const uint32_t least = wave_umin(lo);
+            const float b = __uint_as_float(least);
+            const uint32_t close = __float_as_uint(METRIC == M_COS ? b + 1.1444091796875e-05f : __builtin_fmaf(b, 1.0000152587890625f, 1e-36f));
+            const unsigned long long who = __ballot(lo <= close), also = __ballot(second <= close);
+            const int j = __builtin_amdgcn_readlane(at, __ffsll(who | 1ull << 63) - 1);
+            const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)first, 0);
+            // (below 1e34: no sum near overflow; centroid 0 is a number; not one of the padding)
+            if (least < 0x77f684dfu && d0 <= 0x7f800000u && __popcll(who) == 1 && !also && j < k) best = j;
+        }
+        if (best < 0) {  // uniform
+            const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
+            auto key_of = [&](int j) {
+                float c[8];
+                cl.load(j, c);
+                const float d = dist8<M>(xs, c, na, METRIC == M_COS ? norms[j] : 0.0f);
+                return j < k && d == d ? dist_key<M>(d) : 0xffffffffu;
+            };
+            uint32_t lo = 0xffffffffu;
+            for (int q = 0; q < k; q += 64) lo = umin_u32(lo, key_of(q + lane));
+            const uint32_t best_key = wave_umin(lo);
+            uint32_t close = best_key;  // keys up to here may be the smallest distance
+            float root = 0.0f;
+            if constexpr (METRIC == M_EUCLID) {
+                const float b = __uint_as_float(best_key);
+                close = __float_as_uint(__builtin_fmaf(b, 4.76837158203125e-07f, b));
+                root = sqrtf(b);
+            }
+            best = 0;
+            const bool nan0 = __builtin_amdgcn_readlane((int)key_of(lane), 0) == -1;  // centroid 0's
+            for (int q = 0; q < k && !nan0 && best_key < kInfKey; q += 64) {
+                const uint32_t key = key_of(q + lane);
+                const bool is = METRIC == M_EUCLID ? key <= close && sqrtf(__uint_as_float(key)) == root : key == close;
+                const unsigned long long f = __ballot(is);
+                if (f) {
+                    best = q + __ffsll(f) - 1;
+                    break;
+                }
+            }
+        }
+        code = lane == src ? best : code;
+    }
+    return code;
+}
+
+// One workgroup = one column block: its operands (1 KB per 32 centroids) and centroids lie in LDS, made by the
+// workgroup itself, and its waves walk over tiles of 32 rows on their own, no barrier after the set-up.  The
+// 32 scores that a lane has of 64 centroids go into four sets of eight, {32 b + 8 p + 4 h + 0..3} of two neighbouring
+// blocks b: 16 minima, four tags and five operations for the two smallest keys, 25 instructions where sets of
+// four take 34 (k_assign_mfma8, whose pick among four instead of eight centroids weighs as much there).
+// Even and odd pairs of blocks, and the two lane halves, each have two smallest keys of their own, so that the four
+// best sets are known with their tags and a row that only two sets can win is decided among their sixteen
+// centroids; the others, a tenth of the pairs that one bound leaves open, go through all k.
+// The matrix instructions of the next 64 centroids issue between the halves of this selection.
+// Against chunks of 256 centroids, each with its own pass over the rows, and a merge, 16 blocks, Euclidean: 300,000 rows,
+// k = 300 240 -> 140 us, 512 269 -> 170, 1024 515 -> 235; 200,000, k = 1500 568 -> 249; 150,000, k = 2048 613 -> 243;
+// 1,000, k = 257 20 -> 11, k = 2048 84 -> 30; 100,000 x 12 blocks of 7, k = 1024 269 -> 93.  Bound by vector-instruction
+// issue (26 per 64 centroids and tile) and the matrix instructions that only partly hide behind it.
+template <int METRIC>
+__global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    __shared__ float red[2][16][8];
+    constexpr bool COS = METRIC == M_COS;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int T = (int)blockDim.x, W = T >> 6;
+    const int r = lane & 31, h = lane >> 5;
+    const int m = a.m, k = a.k, kp = (k + 63) / 64 * 64, np = kp / 64;
+    // (blocks to XCDs as in k_assign_mfma8: the column blocks of the same rows on one XCD)
+    const unsigned per_chunk = 8u * (unsigned)m;
+    const unsigned chunk_id = blockIdx.x / per_chunk, rem = blockIdx.x % per_chunk;
+    const int s = (int)(rem / 8u);
+    const int64_t first_wg = (int64_t)chunk_id * 8 + (rem % 8u);
+    const int64_t ntiles = (a.n + 31) / 32;
+    if (first_wg * W >= ntiles) return;
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < kStatSlots; i += T) a.stat_next[i * kStatStride] = 0u;
+
+    u32x4 *at = reinterpret_cast<u32x4 *>(lds);  // [kp / 32][64]
+    const LdsBig8 cl{lds + kp * 32, kp * 16};
+    float *norms = reinterpret_cast<float *>(lds + kp * 64);
+    {
+        const float4 *src = reinterpret_cast<const float4 *>(a.cb + (size_t)s * k * 8);
+        for (int i = threadIdx.x; i < 2 * kp; i += T)
+            cl.set(i >> 1, i & 1, i < 2 * k ? src[i] : make_float4(kBig8Far, kBig8Far, kBig8Far, kBig8Far));
+    }
+    __syncthreads();
+    float mu[8], sg = kCosScale, bad = 0.0f;
+    if constexpr (COS) {
+        for (int j = threadIdx.x; j < kp; j += T) {
+            float c[8];
+            cl.load(j, c);
+            const float nc = seq_norm8(c);
+            norms[j] = nc;
+            norms[kp + j] = nc == 0.0f || j >= k ? 0.0f : 1.0f / nc;
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) mu[t] = 0.0f;
+    } else {
+        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (int j = threadIdx.x; j < k; j += T) {
+            float c[8];
+            cl.load(j, c);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] += c[t] * 0.00048828125f;  // / 2048: no overflow
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) v[t] += __shfl_xor(v[t], off);
+            if (lane == 0) red[0][wave][t] = v[t];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            mu[t] = 0.0f;
+            for (int w = 0; w < W; ++w) mu[t] += red[0][w][t];
+            mu[t] *= 2048.0f / (float)k;
+        }
+        float p = 0.0f;
+        for (int j = threadIdx.x; j < k; j += T) {
+            float c[8];
+            cl.load(j, c);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const float d = (c[t] - mu[t]) * 0.015625f;
+                p = __builtin_fmaf(d, d, p);  // / 4096
+            }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) p += __shfl_xor(p, off);
+        if (lane == 0) red[1][wave][0] = p;
+        __syncthreads();
+        float r2 = 0.0f;
+        for (int w = 0; w < W; ++w) r2 += red[1][w][0];
+        sg = mfma8_scale(r2 * (4096.0f / (float)k), 1, kBig8Rms);  // root mean square 2 ... 4: none longer than 181
+        bad = sg - sg;
+    }
+    float mc2 = 0.0f, mdc = 0.0f;
+    for (int j = threadIdx.x; j < kp; j += T) {
+        float c[8];
+        cl.load(j, c);
+        const bool live = j < k;
+        const float nc = COS && live ? norms[j] : 1.0f;
+        Half8 o[2];
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+            float v[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const float e = c[4 * hh + t];
+                v[t] = !live ? 0.0f : COS ? (nc == 0.0f ? 0.0f : -2.0f * (e * (1.0f / nc)) * kCosScale) : -2.0f * ((e - mu[4 * hh + t]) * sg);
+            }
+            o[hh] = half8(v);
+        }
+        const float c2 = COS && nc == 0.0f ? kCosScale * kCosScale : o[0].n2 + o[1].n2;
+        if (live) {
+            float x = c2 + bad;
+            if (COS && !(nc == 0.0f || (nc >= 1e-15f && nc <= 1e15f))) x = __builtin_nanf("");
+            mc2 = (mc2 == mc2 && x == x) ? fmaxf(mc2, x) : __builtin_nanf("");
+            mdc = fmaxf(mdc, o[0].d2 + o[1].d2);
+        }
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh)
+            at[(j / 32) * 64 + 32 * hh + j % 32] = u32x4{o[hh].h01, o[hh].h23, o[hh].l01, c2_word(c2, hh, live)};
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const float o = __shfl_xor(mc2, off);
+        mc2 = (mc2 == mc2 && o == o) ? fmaxf(mc2, o) : __builtin_nanf("");
+        mdc = fmaxf(mdc, __shfl_xor(mdc, off));
+    }
+    if (lane == 0) {
+        red[0][wave][0] = mc2;
+        red[0][wave][1] = mdc;
+    }
+    __syncthreads();  // (red[0] was read before the barrier that red[1] needed)
+    for (int w = 0; w < W; ++w) {
+        const float o = red[0][w][0];
+        mc2 = (mc2 == mc2 && o == o) ? fmaxf(mc2, o) : __builtin_nanf("");
+        mdc = fmaxf(mdc, red[0][w][1]);
+    }
+    float muh[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) muh[u] = COS ? 0.0f : -((h ? mu[4 + u] : mu[u]) * sg);
+    const uint32_t keep = opaque_vgpr(0xFFFFFF00u);
+    const float acc8 = 4.57763671875e-05f * mc2;  // 3 * 2^-16: see decided8
+
+    // tiles t, t + step, ...; rows two tiles ahead
+    const int64_t step = a.stride * W;
+    int64_t t = first_wg * W + wave;
+    const uint32_t loff = 4u * ((uint32_t)r * (uint32_t)a.ld + 4u * (uint32_t)h);
+    typedef float rowpiece __attribute__((ext_vector_type(4), aligned(4)));
+    auto fetch = [&](int64_t tile) {
+        const int64_t row0 = (tile < ntiles ? tile : ntiles - 1) * 32;  // uniform
+        const char *base = reinterpret_cast<const char *>(a.x + row0 * a.ld + (int64_t)s * 8);
+        const rowpiece v = *reinterpret_cast<const rowpiece *>(base + (r < a.n - row0 ? loff : 16u * (uint32_t)h));
+        return make_float4(v[0], v[1], v[2], v[3]);
+    };
+    uint32_t n_exact = 0;
+    float4 xa = fetch(t), xb = fetch(t + step);
+    for (; t < ntiles; t += step) {
+        const float xraw[4] = {xa.x, xa.y, xa.z, xa.w};
+        xa = xb;
+        xb = fetch(t + 2 * step);
+        const Row8 row = row8<METRIC>(xraw, sg, muh);
+        const u32x4 xb16 = row.b16;
+        const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        int m1 = 0x7f800000, m2 = 0x7f800000, o1 = 0x7f800000, o2 = 0x7f800000;  // +inf; even and odd pairs
+        floatx16 p0, p1, q0, q1;
+#define VQ_MFMA(av, acc)                                                                                              \
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, av), __builtin_bit_cast(f16x8, xb16), zero, 0, 0, 0);
+#define VQ_MIN8(c, d, p)                                                                                              \
+    imin(imin(imin(imin(imin(imin(imin(__float_as_int(c[4 * p]), __float_as_int(c[4 * p + 1])),                       \
+                                   __float_as_int(c[4 * p + 2])), __float_as_int(c[4 * p + 3])),                      \
+                        __float_as_int(d[4 * p])), __float_as_int(d[4 * p + 1])), __float_as_int(d[4 * p + 2])),      \
+         __float_as_int(d[4 * p + 3]))
+#define VQ_KEY(c, d, p, tag) key[p] = (int)(((uint32_t)VQ_MIN8(c, d, p) & keep) | (tag));
+        // selection of 64 centroids (scores in c, d) with the matrix instructions of the next 64 (into e, f)
+#define VQ_PAIR(c, d, e, f, first, second, T0, T1, T2, T3, next)                                                      \
+    {                                                                                                                 \
+        int key[4];                                                                                                   \
+        VQ_MFMA(n0, e)                                                                                                \
+        __builtin_amdgcn_sched_barrier(0);                                                                            \
+        VQ_KEY(c, d, 0, T0) VQ_KEY(c, d, 1, T1)                                                                       \
+        __builtin_amdgcn_sched_barrier(0);                                                                            \
+        VQ_MFMA(n1, f)                                                                                                \
+        n0 = ap[(next) * 128];                                                                                        \
+        n1 = ap[(next) * 128 + 64];                                                                                   \
+        __builtin_amdgcn_sched_barrier(0);                                                                            \
+        VQ_KEY(c, d, 2, T2) VQ_KEY(c, d, 3, T3)                                                                       \
+        top2_push4(first, second, key[0], key[1], key[2], key[3]);                                                    \
+        __builtin_amdgcn_sched_barrier(0);                                                                            \
+    }
+        // the tags of the sets, one scalar register each: tag = 8 * pair + 2 * set
+        uint32_t t0 = 0, t1 = 2, t2 = 4, t3 = 6, t4 = 8, t5 = 10, t6 = 12, t7 = 14;
+        auto opaque = [](uint32_t &v) { asm volatile("" : "+s"(v)); };  // (else each is made again from one of them)
+        const u32x4 *ap = at + lane;
+        u32x4 n0 = ap[0], n1 = ap[64];
+        VQ_MFMA(n0, p0)
+        VQ_MFMA(n1, p1)
+        n0 = ap[128];
+        n1 = ap[192];
+        for (int p = 0; p < np; p += 2) {
+            opaque(t0), opaque(t1), opaque(t2), opaque(t3), opaque(t4), opaque(t5), opaque(t6), opaque(t7);
+            VQ_PAIR(p0, p1, q0, q1, m1, m2, t0, t1, t2, t3, p + 2 < np ? p + 2 : 0)
+            if (p + 1 < np) VQ_PAIR(q0, q1, p0, p1, o1, o2, t4, t5, t6, t7, p + 3 < np ? p + 3 : 0)
+            t0 += 16, t1 += 16, t2 += 16, t3 += 16, t4 += 16, t5 += 16, t6 += 16, t7 += 16;
+        }
+#undef VQ_MFMA
+#undef VQ_MIN8
+#undef VQ_KEY
+#undef VQ_PAIR
+        m1 |= h;  // bit 0 of the tag: the lane half
+        o1 |= h;
+        int f0, f1, g0, g1, e0, e1;
+        swap_halves(m1, f0, f1);
+        swap_halves(o1, g0, g1);
+        swap_halves(imin(m2, o2), e0, e1);
+        const int lo_a = imin(f0, f1), hi_a = imax(f0, f1), lo_b = imin(g0, g1), hi_b = imax(g0, g1);
+        const int mid_a = imax(lo_a, lo_b), mid_b = imin(hi_a, hi_b);
+        const int set1 = imin(lo_a, lo_b), set2 = imin(mid_a, mid_b);        // the two best sets with a tag
+        const int others = imin(imax(mid_a, mid_b), imin(e0, e1));           // no other set is below
+        const float s1 = __int_as_float(set1), s2 = __int_as_float(imin(set2, others));
+        const int64_t row0 = t * 32;
+        const bool mine = h == 0 && r < a.n - row0;  // the lane's row exists
+        bool near = decided8<METRIC>(s1, s2, row, mdc, acc8);
+        // The best of a set's eight centroids, runs first and first + 32: each lane half sums its four dimensions of
+        // all of them, the lower half then holds the first run's distances, the upper half the second's, the place in
+        // the run in the two low bits.  at: the best; lo, hi: the two smallest keys (lower lanes).
+        auto first_of = [](int set) {
+            const uint32_t tag = (uint32_t)set & 0xFFu;
+            return (int)((tag >> 3) * 64 + ((tag >> 1) & 3u) * 8 + (tag & 1u) * 4);
+        };
+        auto pick = [&](int first, int &at, int &lo, int &hi) {
+            const int ra = cl.run(first, h), rb = cl.run(first + 32, h);
+            const int j0 = first + 32 * h;
+            float4 inv = make_float4(0.f, 0.f, 0.f, 0.f);
+            if constexpr (COS) inv = *reinterpret_cast<const float4 *>(norms + kp + j0);
+            const float iv[4] = {inv.x, inv.y, inv.z, inv.w};
+            int ky[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(share8<METRIC>(xraw, cl.piece(ra, i))),
+                                                                 __float_as_int(share8<METRIC>(xraw, cl.piece(rb, i))), false, false);
+                float d = __int_as_float((int)sw[0]) + __int_as_float((int)sw[1]);
+                if constexpr (COS) d = j0 + i < k ? __builtin_fmaf(-(d * row.rx), iv[i], 1.001f) : 1e30f;
+                ky[i] = (int)((__float_as_uint(d) & 0xFFFFFFFCu) | (uint32_t)i);
+            }
+            const int a3 = imin3(ky[0], ky[1], ky[2]), b3 = imed3a(ky[0], ky[1], ky[2]);
+            int l0, l1, h0, h1;
+            swap_halves(imin(a3, ky[3]), l0, l1);
+            swap_halves(imin(b3, imax(a3, ky[3])), h0, h1);
+            lo = imin(l0, l1);
+            hi = imin3(imax(l0, l1), h0, h1);
+            at = first + (l1 < l0 ? 32 : 0) + (lo & 3);  // (lower half: 0 its own, 1 the partner's)
+        };
+        // (2^-16: the sums' rounding and the reference's, the bits left out; 1e-36: subnormal sums of squares)
+        auto apart = [](int lo, int hi) {
+            const float best = __int_as_float(lo & ~3), second = __int_as_float(hi & ~3);
+            return COS ? second - best > 1.1444091796875e-05f : __builtin_fmaf(second, 0.9999847412109375f, -1e-36f) > best;
+        };
+        const int first = first_of(set1);
+        int code, lo, hi;
+        pick(first, code, lo, hi);
+        bool clear = apart(lo, hi);
+        int other = -1;  // the second set, where it may have the answer
+        unsigned long long todo = __ballot(mine && !near);
+        if (todo) {  // the same in every lane
+            if (!near && decided8<METRIC>(s1, __int_as_float(others), row, mdc, acc8)) other = first_of(set2);
+            const bool two = other >= 0;
+            if (__ballot(mine && two)) {
+                int code2, lo2, hi2;
+                pick(two ? other : first, code2, lo2, hi2);
+                if (two) {
+                    code = lo2 < lo ? code2 : code;
+                    hi = imin3(imax(lo, lo2), hi, hi2);
+                    lo = imin(lo, lo2);
+                    clear = apart(lo, hi);
+                    near = true;
+                }
+                todo = __ballot(mine && !near);
+            }
+        }
+        const unsigned long long ties = __ballot(mine && near && !clear);
+        if (todo | ties) {  // the same in every lane
+            float xs[8];  // the lane's row
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                int lo, hi;
+                swap_halves(__float_as_int(xraw[u]), lo, hi);
+                xs[u] = __int_as_float(lo);
+                xs[4 + u] = __int_as_float(hi);
+            }
+            if (ties) {  // the sets' centroids by the reference's distances: the first of the smallest
+                const float na = COS ? seq_norm8(xs) : 0.0f;
+                float bd = 0.0f;
+                int bj = -1;
+                for (int i = 0; i < (__ballot(other >= 0 && !clear) ? 16 : 8); ++i) {
+                    const int j = (i < 8 || other < 0 ? first : other) + (i & 3) + ((i >> 2) & 1) * 32;
+                    float c[8];
+                    cl.load(j, c);
+                    const float d = dist8<METRIC>(xs, c, na, COS ? norms[j] : 0.0f);
+                    if (j < k && (bj < 0 || d < bd || (d == bd && j < bj))) {
+                        bd = d;
+                        bj = j;
+                    }
+                }
+                code = clear ? code : bj;
+            }
+            if (todo) {
+                n_exact += (uint32_t)__popcll(todo);
+                code = exact_rows_big8<METRIC>(todo, code, cl, norms, kp, xs, row.rx, k, lane);
+            }
+        }
+        if (mine) a.codes[(size_t)(row0 + r) * m + s] = (uint16_t)code;
+    }
+    if (lane == 0 && n_exact)
+        atomicAdd(a.stat + ((first_wg * W + wave) & (kStatSlots - 1)) * kStatStride, n_exact);
+}
+
+}  // namespace vq

@@ -1,6 +1,7 @@
 // Codebooks of more than 256 centroids (16-bit codes).
 //
-// Assignment: the codebook of every column block is cut into chunks of 256 consecutive centroids.
+// Assignment (blocks of 8 floats up to 2048 centroids: assign_mfma8_big.hpp): the codebook of every column block is
+// cut into chunks of 256 consecutive centroids.
 // Each chunk goes through the 8-bit assignment kernels unchanged, which leave the chunk's own
 // winner (the lowest index of the smallest distance inside the chunk, src/utils.rs:62-70); a merge
 // kernel then evaluates that winner's distance in the reference's operation order and keeps it

@@ -254,6 +254,16 @@ inline bool assign_few_applicable(const vq_ctx *ctx, int64_t n, int32_t m, int32
 bool assign_pending_fusable(const vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t sd,
                             int32_t k, const float *d_codebook);
 
+// The width to which an encode pads the column blocks of such rows (0: not at all), and the copy itself:
+// n rows of m blocks of sd floats to m blocks of sdp floats, zeros after each block.
+int encode_pad_width(const vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd,
+                     int32_t k, const float *d_codebooks);
+void pad_blocks(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t sdp, float *d_y);
+// Turns to the other set of counters of undecided pairs: this pass's (cleared by the pass before), and the
+// next pass's, which this pass clears.
+int32_t next_counters(vq_ctx *ctx, uint32_t **now, uint32_t **next);
+constexpr int64_t kPadSlice = 96 << 20;  // bytes of padded rows that an encode makes at a time
+
 // Defined in vq_api_host.hip: ends the copying threads.
 void drop_crew(vq_ctx *ctx);
 

@@ -142,6 +142,17 @@ struct MfmaTabPtrs {
     uint32_t *stat, *stat_next;  // the counters of this pass; of the next one
     int nb;
 };
+// The counters of undecided pairs, of the present pass and of the next.
+int32_t counters(vq_ctx *ctx, uint32_t **now, uint32_t **next) {
+    const size_t n_stat = (size_t)vq::kStatSlots * vq::kStatStride;
+    if (!ctx->mfma_stat.p) {
+        VQ_TRY(ensure(ctx, ctx->mfma_stat, sizeof(uint32_t) * 2 * n_stat));
+        VQ_HIP(ctx, hipMemsetAsync(ctx->mfma_stat.p, 0, sizeof(uint32_t) * 2 * n_stat, ctx->stream));
+    }
+    *now = (uint32_t *)ctx->mfma_stat.p + ctx->mfma_stat_cur * n_stat;
+    *next = (uint32_t *)ctx->mfma_stat.p + (ctx->mfma_stat_cur ^ 1) * n_stat;
+    return VQ_OK;
+}
 int32_t mfma_tab_ptrs(vq_ctx *ctx, int m, int k, MfmaTabPtrs &t) {
     t.nb = 2 * ((k + 63) / 64);  // blocks of 32 centroids, an even number (the kernel scores them in pairs)
     // A operands: 64 lanes x 16 bytes per (s, block of 32 centroids)
@@ -153,16 +164,10 @@ int32_t mfma_tab_ptrs(vq_ctx *ctx, int m, int k, MfmaTabPtrs &t) {
         return VQ_OK;
     }
     VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + vq::kMfma8Aux * (size_t)m) + 64));
-    const size_t n_stat = (size_t)vq::kStatSlots * vq::kStatStride;
-    if (!ctx->mfma_stat.p) {
-        VQ_TRY(ensure(ctx, ctx->mfma_stat, sizeof(uint32_t) * 2 * n_stat));
-        VQ_HIP(ctx, hipMemsetAsync(ctx->mfma_stat.p, 0, sizeof(uint32_t) * 2 * n_stat, ctx->stream));
-    }
+    VQ_TRY(counters(ctx, &t.stat, &t.stat_next));
     float *atab = (float *)ctx->mfma_tab.p;
     t.atab = (vq::u32x4 *)atab;
     t.aux = atab + n_atab;
-    t.stat = (uint32_t *)ctx->mfma_stat.p + ctx->mfma_stat_cur * n_stat;
-    t.stat_next = (uint32_t *)ctx->mfma_stat.p + (ctx->mfma_stat_cur ^ 1) * n_stat;
     return VQ_OK;
 }
 
@@ -429,7 +434,6 @@ int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bo
     return sdp;
 }
 
-constexpr int64_t kPadSlice = 96 << 20;  // bytes of padded rows that an encode makes at a time
 constexpr size_t kPadKeep = 2u << 30;    // bytes that the context keeps of a fit's padded copy of its rows
 
 void launch_pad(vq_ctx *ctx, const float *x, int64_t n, int64_t ld, int m, int sd, int sdp, float *y) {
@@ -691,6 +695,28 @@ template int32_t assign_few<uint8_t>(vq_ctx *, int32_t, const float *, int64_t, 
                                      const float *, uint8_t *, uint16_t *);
 template int32_t assign_few<uint16_t>(vq_ctx *, int32_t, const float *, int64_t, int64_t, int32_t, int32_t, int32_t,
                                       const float *, uint16_t *, uint16_t *);
+
+int encode_pad_width(const vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd,
+                     int32_t k, const float *d_codebooks) {
+    vq::AssignArgs a{};
+    a.x = d_x;
+    a.n = n;
+    a.ld = ld;
+    a.m = m;
+    a.k = k;
+    a.cb = d_codebooks;
+    return pad_width(ctx, metric, a, sd, false);
+}
+
+void pad_blocks(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t sdp, float *d_y) {
+    launch_pad(ctx, d_x, n, ld, m, sd, sdp, d_y);
+}
+
+int32_t next_counters(vq_ctx *ctx, uint32_t **now, uint32_t **next) {
+    ctx->mfma_stat_cur ^= 1;
+    ctx->recheck_src = 1;
+    return counters(ctx, now, next);
+}
 
 int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m,
                   int32_t sd, int32_t k, const float *d_codebooks, uint8_t *d_codes, float *d_dist,
