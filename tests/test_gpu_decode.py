@@ -1,0 +1,49 @@
+"""Reconstruction from codes: the table in LDS whole or by groups of column blocks, and the gather through the
+vector cache, at sizes that end inside a run of rows, a workgroup's pieces or a group; exact against numpy."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import vq_amd
+    c = vq_amd.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("n,m,sd,k", [
+    (1, 1, 8, 2), (1025, 3, 8, 40), (70_001, 1, 8, 256), (5463, 12, 16, 256), (70_000, 1, 512, 20),  # whole table / gather
+    (110_001, 10, 8, 1024), (66_000, 17, 8, 2048), (33_001, 33, 24, 300), (263_000, 4, 16, 3000),   # groups, the last short
+    (130_000, 9, 16, 5000), (4097, 2, 64, 700), (999, 5, 12, 300)])                                 # a block too large: gather
+def test_decode(ctx, n, m, sd, k):
+    rng = np.random.default_rng(n + k)
+    cb = (rng.standard_normal((m, k, sd)) * 100).astype(F)
+    codes = rng.integers(0, k, (n, m))
+    want = cb[np.arange(m)[None, :], codes].reshape(n, m * sd)
+    wide = k > 256
+    dcodes, dcb = ctx.to_device(codes.astype(np.uint16 if wide else np.uint8)), ctx.to_device(cb)
+    out = ctx.to_device(np.full((n + 1, m * sd), 0x5555, np.uint16))
+    (ctx.decode_f16_u16 if wide else ctx.decode_f16)(dcodes, n, m, sd, k, dcb, out)
+    got = out.download()
+    assert np.array_equal(got[:n], want.astype(np.float16).view(np.uint16)) and (got[n] == 0x5555).all()
+    out32 = ctx.to_device(np.full((n + 1, m * sd), 7.0, F))
+    (ctx.decode_f32_u16 if wide else ctx.decode_f32)(dcodes, n, m, sd, k, dcb, out32)
+    got = out32.download()
+    assert np.array_equal(got[:n], want) and (got[n] == 7.0).all()
+
+
+@pytest.mark.parametrize("dim", [8, 24, 128, 12, 7])
+def test_tree_decode(ctx, dim):
+    rng = np.random.default_rng(dim)
+    x = rng.standard_normal((3000, dim)).astype(F)
+    tree = ctx.tsvq_build(ctx.to_device(x), 3000, dim, dim, 5)
+    cen = tree.download()["centroids"]
+    leaf = rng.integers(0, len(cen), 2047).astype(np.int32)
+    out = ctx.to_device(np.full((2048, dim), 0x5555, np.uint16))
+    ctx.tsvq_decode_f16(tree, ctx.to_device(leaf), 2047, out)
+    got = out.download()
+    assert np.array_equal(got[:2047], cen[leaf].astype(np.float16).view(np.uint16)) and (got[2047] == 0x5555).all()

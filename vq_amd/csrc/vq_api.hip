@@ -17,6 +17,7 @@
 #include "ctx.hpp"
 #include "assign_exact.hpp"
 #include "assign_mfma.hpp"
+#include "decode.hpp"
 
 #ifndef VQ_MFMA_RUN
 #define VQ_MFMA_RUN 8    // tiles of 32 rows per wave in the matrix-core assignment (a power of two)
@@ -485,9 +486,9 @@ __global__ void k_decode_f16(const CodeT *__restrict__ codes, int64_t n, int m, 
 // Four consecutive components per thread (sub_dim a multiple of 4, 16-byte aligned codebooks and
 // output rows): one 16-byte load of the centroid, one 8- or 16-byte store.  F16: binary16 bit
 // patterns (round to nearest even), else f32.
-template <bool F16, typename CodeT>
+template <typename CodeT>
 __global__ void __launch_bounds__(256) k_decode_vec4(const CodeT *__restrict__ codes, int64_t n, int m, int sd,
-                                                     int k, const float *__restrict__ cb, void *__restrict__ out) {
+                                                     int k, const float *__restrict__ cb, uint2 *__restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;  // group of four components
     const int64_t dim4 = (int64_t)m * sd / 4;
     if (i >= n * dim4) return;
@@ -495,30 +496,31 @@ __global__ void __launch_bounds__(256) k_decode_vec4(const CodeT *__restrict__ c
     const int c = (int)(i % dim4) * 4;
     const int s = c / sd, t = c % sd;
     const float4 v = *reinterpret_cast<const float4 *>(cb + ((size_t)s * k + codes[row * m + s]) * sd + t);
-    if constexpr (F16) {
-        uint2 o;
-        o.x = (uint32_t)__half_as_ushort(__float2half_rn(v.x)) | ((uint32_t)__half_as_ushort(__float2half_rn(v.y)) << 16);
-        o.y = (uint32_t)__half_as_ushort(__float2half_rn(v.z)) | ((uint32_t)__half_as_ushort(__float2half_rn(v.w)) << 16);
-        reinterpret_cast<uint2 *>(out)[i] = o;
-    } else {
-        reinterpret_cast<float4 *>(out)[i] = v;
-    }
+    uint2 o;
+    o.x = (uint32_t)__half_as_ushort(__float2half_rn(v.x)) | ((uint32_t)__half_as_ushort(__float2half_rn(v.y)) << 16);
+    o.y = (uint32_t)__half_as_ushort(__float2half_rn(v.z)) | ((uint32_t)__half_as_ushort(__float2half_rn(v.w)) << 16);
+    out[i] = o;
 }
 
-// The same gather with the whole codebook table resident in LDS (up to 128 KB, one workgroup of
-// 1024 threads per compute unit walking over the output): a thread makes one 16-byte piece of the
+// The same gather with the codebook table resident in LDS (up to 128 KB, one workgroup of 1024 threads per
+// compute unit walking over the output): a thread makes one 16-byte piece of the
 // output per step — eight f16 values (F16; sub_dim a multiple of 8) or four f32 values (sub_dim a
-// multiple of 4) — so a wave's stores are 1 KB of consecutive bytes, its code reads consecutive
-// bytes, and the centroid comes from LDS instead of a scattered read of the 128 KB table through
-// the vector cache.  Four pieces per thread are in flight.
+// multiple of 4) — so a wave's stores are consecutive bytes, its code reads consecutive
+// bytes, and the centroid comes from LDS instead of a scattered read of the table through
+// the vector cache.  U pieces per thread are in flight.  blockIdx.y: a group of G column blocks, where the table
+// of all of them does not fit.  A workgroup takes runs of whole rows, so that a piece's place in its run is
+// divided in 32 bits.
 template <bool F16, typename CodeT>
 __global__ void __launch_bounds__(1024) k_decode_resident(const CodeT *__restrict__ codes, int64_t n, int m, int sd,
-                                                          int k, const float *__restrict__ cb,
+                                                          int k, int G, const float *__restrict__ cb,
                                                           vq::u32x4 *__restrict__ out) {
-    extern __shared__ __attribute__((aligned(16))) vq::u32x4 tab[];  // [m * k][pieces of a centroid]
-    const int pieces = F16 ? sd / 8 : sd / 4;                        // 16-byte output pieces per centroid
-    const int entries = m * k * pieces;
-    for (int e = threadIdx.x; e < entries; e += 1024) {
+    extern __shared__ __attribute__((aligned(16))) vq::u32x4 tab[];  // [blocks of the group * k][pieces of a centroid]
+    constexpr int U = F16 ? 4 : 8;  // pieces in flight per thread
+    const uint32_t pieces = F16 ? sd / 8 : sd / 4;  // 16-byte output pieces per centroid
+    const int s0 = (int)blockIdx.y * G, mg = m - s0 < G ? m - s0 : G;
+    const uint32_t entries = (uint32_t)mg * k * pieces;
+    cb += (size_t)s0 * k * sd;
+    for (uint32_t e = threadIdx.x; e < entries; e += 1024) {
         if constexpr (F16) {
             const float4 a = reinterpret_cast<const float4 *>(cb)[2 * (size_t)e];
             const float4 b = reinterpret_cast<const float4 *>(cb)[2 * (size_t)e + 1];
@@ -531,30 +533,30 @@ __global__ void __launch_bounds__(1024) k_decode_resident(const CodeT *__restric
         }
     }
     __syncthreads();
-    const int64_t total = n * m * pieces;
-    const int64_t stride = (int64_t)gridDim.x * 1024;
-    const int per_row = m * pieces;
-    constexpr int U = F16 ? 4 : 8;  // pieces in flight per thread
-    for (int64_t i0 = (int64_t)blockIdx.x * 1024 + threadIdx.x; i0 < total; i0 += U * stride) {
-        uint32_t code[U];
-        int64_t idx[U];
+    const uint32_t per_row = (uint32_t)mg * pieces;
+    const int64_t rows = U * 1024 / per_row > 1 ? U * 1024 / per_row : 1;  // of a run
+    for (int64_t row0 = blockIdx.x * rows; row0 < n; row0 += gridDim.x * rows) {
+        const uint32_t count = (uint32_t)(n - row0 < rows ? n - row0 : rows) * per_row;
+        const CodeT *run = codes + row0 * m + s0;
+        vq::u32x4 *to = out + (row0 * m + s0) * pieces;
+        for (uint32_t l0 = threadIdx.x; l0 < count; l0 += U * 1024) {
+            uint32_t code[U], at[U], entry[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            idx[u] = i0 + u * stride;
-            const int64_t ic = idx[u] < total ? idx[u] : i0;
-            code[u] = codes[ic / pieces];  // codes are n x m row-major: piece ic belongs to (row, block) ic / pieces
+            for (int u = 0; u < U; ++u) {
+                const uint32_t l = l0 + 1024u * u < count ? l0 + 1024u * u : l0;
+                const uint32_t row = l / per_row, within = l - row * per_row;
+                const uint32_t s = pieces == 1 ? within : within / pieces;
+                code[u] = run[row * (uint32_t)m + s];
+                at[u] = row * (uint32_t)m * pieces + within;
+                entry[u] = s * (uint32_t)k * pieces + (within - s * pieces);
+            }
+            vq::u32x4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = tab[entry[u] + code[u] * pieces];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (l0 + 1024u * u < count) __builtin_nontemporal_store(v[u], to + at[u]);
         }
-        vq::u32x4 v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t ic = idx[u] < total ? idx[u] : i0;
-            const int within = (int)(ic % per_row);  // (block, piece) of the row
-            const int s = within / pieces, pc = within % pieces;
-            v[u] = tab[(s * k + (int)code[u]) * pieces + pc];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (idx[u] < total) out[idx[u]] = v[u];
     }
 }
 
@@ -585,8 +587,18 @@ template <bool F16, typename CodeT>
 int32_t launch_decode_resident(vq_ctx *ctx, const CodeT *d_codes, int64_t n, int m, int sd, int k,
                                const float *d_codebooks, void *d_out, bool *done) {
     *done = false;
-    const size_t lds = (size_t)m * k * sd * (F16 ? 2 : 4);
-    if (sd % (F16 ? 8 : 4) != 0 || lds > 128 * 1024 || n * m < (1 << 16)) return VQ_OK;
+    // Where the table of all column blocks does not fit, a group of them whose pieces of a row fill whole lines, or
+    // half of one, if there are enough rows for the groups' tables (k_decode_gather: 50 us for the 36 above).
+    const size_t block = (size_t)k * sd * (F16 ? 2 : 4), line = (size_t)sd * (F16 ? 2 : 4);
+    if (sd % (F16 ? 8 : 4) != 0 || block > 128 * 1024 || n * m < (1 << 16)) return VQ_OK;
+    int G = m;
+    if (block * m > 128 * 1024) {
+        G = (int)(128 * 1024 / block);
+        if (G * line >= 128) G = (int)(G * line / 128 * 128 / line);
+        if (G < 1 || G * line < 64 || n * m < (1 << 20)) return VQ_OK;
+    }
+    if ((int64_t)m * sd >= (1 << 24)) return VQ_OK;  // 32-bit places in a run
+    const size_t lds = block * G;
     if ((reinterpret_cast<uintptr_t>(d_codebooks) | reinterpret_cast<uintptr_t>(d_out)) & 15) return VQ_OK;
     auto kern = k_decode_resident<F16, CodeT>;
     // the kernel's LDS limit and the number of compute units: asked for once per context and kernel
@@ -603,8 +615,10 @@ int32_t launch_decode_resident(vq_ctx *ctx, const CodeT *d_codes, int64_t n, int
     }
     const int64_t pieces = (int64_t)n * m * (F16 ? sd / 8 : sd / 4);
     const unsigned per_cu = lds <= 64 * 1024 ? 2u : 1u;
-    const unsigned wgs = (unsigned)std::min<int64_t>((int64_t)ctx->compute_units * per_cu, cdiv(pieces, 4096));
-    hipLaunchKernelGGL(kern, dim3(wgs), dim3(1024), lds, ctx->stream, d_codes, n, m, sd, k, d_codebooks,
+    const unsigned groups = cdiv(m, G);
+    const unsigned wgs = (unsigned)std::min<int64_t>(std::max<int64_t>(1, (int64_t)ctx->compute_units * per_cu / groups),
+                                                     cdiv(pieces, 4096 * groups));
+    hipLaunchKernelGGL(kern, dim3(wgs, groups), dim3(1024), lds, ctx->stream, d_codes, n, m, sd, k, G, d_codebooks,
                        (vq::u32x4 *)d_out);
     VQ_HIP(ctx, hipGetLastError());
     *done = true;
@@ -623,13 +637,19 @@ int32_t decode_codes(vq_ctx *ctx, const CodeT *d_codes, int64_t n, int32_t m, in
     bool done = false;
     VQ_TRY((launch_decode_resident<F16, CodeT>(ctx, d_codes, n, m, sd, k, d_codebooks, d_out, &done)));
     if (done) return VQ_OK;
-    if (sd % 4 == 0 && ((reinterpret_cast<uintptr_t>(d_codebooks) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0)
-        hipLaunchKernelGGL((k_decode_vec4<F16, CodeT>), dim3(cdiv(n * m * sd / 4, 256)), dim3(256), 0, ctx->stream,
-                           d_codes, n, m, sd, k, d_codebooks, d_out);
-    else if constexpr (F16)
-        hipLaunchKernelGGL(k_decode_f16<CodeT>, dim3(cdiv(n * m * sd, 256)), dim3(256), 0, ctx->stream, d_codes, n, m,
-                           sd, k, d_codebooks, (uint16_t *)d_out);
-    else
+    const bool aligned = ((reinterpret_cast<uintptr_t>(d_codebooks) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
+    constexpr int piece = F16 ? 8 : 4;
+    if (sd % piece == 0 && aligned && (int64_t)m * sd < (1LL << 31))
+        hipLaunchKernelGGL((vq::k_decode_gather<F16, CodeT>), dim3(cdiv(n * m * (sd / piece), 1024)), dim3(256), 0,
+                           ctx->stream, d_codes, n, m, sd, k, d_codebooks, (vq::u32x4_out *)d_out);
+    else if constexpr (F16) {
+        if (sd % 4 == 0 && aligned)
+            hipLaunchKernelGGL(k_decode_vec4<CodeT>, dim3(cdiv(n * m * sd / 4, 256)), dim3(256), 0, ctx->stream, d_codes, n,
+                               m, sd, k, d_codebooks, (uint2 *)d_out);
+        else
+            hipLaunchKernelGGL(k_decode_f16<CodeT>, dim3(cdiv(n * m * sd, 256)), dim3(256), 0, ctx->stream, d_codes, n, m,
+                               sd, k, d_codebooks, (uint16_t *)d_out);
+    } else
         hipLaunchKernelGGL(k_decode_f32<CodeT>, dim3(cdiv(n * m * sd, 256)), dim3(256), 0, ctx->stream, d_codes, n, m,
                            sd, k, d_codebooks, (float *)d_out);
     VQ_HIP(ctx, hipGetLastError());

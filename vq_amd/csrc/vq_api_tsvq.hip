@@ -13,6 +13,7 @@
 #include "host_batch.hpp"
 #include "assign_exact.hpp"
 #include "tsvq.hpp"
+#include "decode.hpp"
 #include "tsvq_kmeans.hpp"
 
 using namespace vqh;
@@ -838,8 +839,11 @@ int32_t vq_tsvq_decode_f16(vq_ctx *ctx, const vq_tree *tree, const int32_t *d_le
     if (n == 0) return VQ_OK;
     if (!d_leaf || !d_out || n < 0) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
     VQ_HIP(ctx, hipSetDevice(ctx->device));
-    if (tree->dim % 4 == 0 &&
-        ((reinterpret_cast<uintptr_t>(tree->d_centroids) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0)
+    const bool aligned = ((reinterpret_cast<uintptr_t>(tree->d_centroids) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
+    if (tree->dim % 8 == 0 && aligned)
+        hipLaunchKernelGGL((vq::k_decode_gather<true, int32_t>), dim3(cdiv(n * (tree->dim / 8), 1024)), dim3(256), 0, ctx->stream,
+                           d_leaf, n, 1, tree->dim, 0, tree->d_centroids, (vq::u32x4_out *)d_out);
+    else if (tree->dim % 4 == 0 && aligned)
         hipLaunchKernelGGL(vq::k_tsvq_decode4_f16, dim3(cdiv(n * (tree->dim / 4), 256)), dim3(256), 0, ctx->stream,
                            d_leaf, n, tree->dim, tree->d_centroids, reinterpret_cast<uint2 *>(d_out));
     else
