@@ -88,6 +88,21 @@ def test_lbg_fit_matches_oracle_bitwise(ctx, n, dim, m, k, iters, kind):
     assert np.array_equal(got.view(np.uint32), want["codebooks"].view(np.uint32))
 
 
+@pytest.mark.parametrize("n,sd,k", [(9000, 48, 2), (20_000, 256, 3), (13_000, 24, 2), (70_000, 16, 2)])
+def test_sorted_rows_first_cluster_absent_from_first_part(ctx, n, sd, k):
+    """Rows in the order of their clusters, the first cluster's last: its members begin after the first parts
+    of 4096 rows, so its leaf of part 0 is empty and lies at the very start of the member list."""
+    rng = np.random.default_rng(sd)
+    x = rng.standard_normal((n, sd)).astype(F)
+    x += (np.arange(n) < n - 4500)[:, None] * F(100.0)
+    init = np.array([[n - 1] + [5 + 7 * j for j in range(k - 1)]], np.uint32)
+    reseed = np.arange(8 * k, dtype=np.uint32)[None, :]
+    want = O.pq_fit(x, 1, k, 4, init, reseed)
+    got, it, used, _, _ = gpu_lbg(ctx, x, 1, k, 4, init, reseed)
+    assert np.array_equal(it, want["iters"]) and np.array_equal(used, want["reseeds"])
+    assert np.array_equal(got.view(np.uint32), want["codebooks"].view(np.uint32))
+
+
 def test_column_blocks_of_one_group_stop_at_different_iterations(ctx):
     """src/utils.rs:104-106 per column block: blocks 0 and 2 of a group of four hold constant rows and
     stop after their first pass, blocks 1 and 3 go on (the group's streaming sums are one workgroup)."""

@@ -436,7 +436,11 @@ static __global__ void __launch_bounds__(256) k_lbg_leafsum(LbgState st, const f
     // the row ids of the next batch are fetched while the current rows are in flight.
     constexpr int B = 16;
     uint32_t rn[B];
-    const uint32_t lastp = d.y - 1;  // leaves are never empty
+    if (d.x == d.y) {  // a large cluster has a leaf for every part, also where it has no member: nothing to read
+        st.leaf_sum[((size_t)s * st.leaf_cap + leaf) * sd + t] = 0.0f;
+        return;
+    }
+    const uint32_t lastp = d.y - 1;
 #pragma unroll
     for (int u = 0; u < B; ++u) rn[u] = perm[d.x + u < d.y ? d.x + u : lastp];
     for (uint32_t p = d.x; p < d.y; p += B) {
