@@ -1,0 +1,37 @@
+"""Sums of wide column blocks: leaves of every length class (short, long, very long, empty), several column blocks,
+widths at the edges of a workgroup, rows shuffled and in the order of their clusters; bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import vq_amd
+    c = vq_amd.Context(0)
+    yield c
+    c.close()
+
+
+SIZES = [1, 15, 16, 17, 64, 65, 127, 128, 129, 511, 512, 1024, 1025, 2500, 8000, 12_300]
+
+
+@pytest.mark.parametrize("order", ["shuffled", "sorted", "reversed"])
+@pytest.mark.parametrize("m,sd", [(1, 64), (2, 65), (1, 128), (1, 256), (1, 257), (3, 100), (1, 512)])
+def test_leaves(ctx, m, sd, order):
+    rng = np.random.default_rng(sd)
+    label = np.repeat(np.arange(len(SIZES)), SIZES)
+    label = label if order == "sorted" else label[::-1] if order == "reversed" else rng.permutation(label)
+    n, k = len(label), len(SIZES)
+    x = rng.standard_normal((n, m * sd)).astype(F) + (50 * label[:, None]).astype(F)
+    init = np.tile(np.array([np.flatnonzero(label == j)[0] for j in range(k)], np.uint32), (m, 1))
+    reseed = rng.integers(0, n, (m, 3 * k), dtype=np.uint32)
+    want = O.pq_fit(x, m, k, 3, init, reseed)
+    cb = ctx.empty((m, k, sd), F)
+    it, _ = ctx.lbg_fit(ctx.to_device(x), n, m * sd, m, sd, k, 3, init, reseed, cb)
+    assert np.array_equal(it, want["iters"])
+    assert np.array_equal(cb.download().view(np.uint32), want["codebooks"].view(np.uint32))

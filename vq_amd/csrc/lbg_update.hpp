@@ -54,7 +54,18 @@ struct LbgState {
     int nseg;
     int leaf_cap;
     int stream;            // 1: the large clusters are summed by k_lbg_stream8 / k_lbg_combine8
+    // wide column blocks (k_lbg_leafsum_wide): the leaves {lo, hi, leaf} in the order in which they are summed, else
+    // null: small clusters, then the large clusters' leaves part by part, long ones left out (leaf = kNoLeaf)
+    uint4 *order = nullptr;       // m*leaf_cap
+    uint4 *longs = nullptr;       // m*2*long_cap: leaves of kVeryLong members or more, leaves of kLong or more
+    uint32_t *place = nullptr;    // m*256 rank of a cluster among the small or among the large ones
+    int *nlong = nullptr;         // m*2
+    int long_cap = 0;
 };
+constexpr uint32_t kNoLeaf = 0xffffffffu;
+constexpr uint32_t kLong = 128, kVeryLong = 512;  // members
+
+__device__ __forceinline__ int long_class(uint32_t len) { return len >= kVeryLong ? 0 : len >= kLong ? 1 : 2; }
 
 // The short kernels of the gather path run beside the streaming kernel, whose waves keep the
 // vector ALU busy: their waves are given the higher issue priority, or they would wait for it.
@@ -171,6 +182,7 @@ static __global__ void __launch_bounds__(256) k_lbg_plan(LbgState st, int k) {
             run += v[u];
         }
     }
+    if (st.order && j < 2) st.nlong[2 * s + j] = 0;
     const bool live = j < k;
     const uint32_t cnt = live ? run : 0;
     const bool small = cnt > 0 && cnt <= (uint32_t)kSeqMax;
@@ -210,7 +222,15 @@ static __global__ void __launch_bounds__(256) k_lbg_plan(LbgState st, int k) {
     st.start[sj] = pc;
     st.leaf_start[sj] = pl;
     st.empty_rank[sj] = pe;
-    if (small) st.leaf_desc[(size_t)s * st.leaf_cap + pl] = make_uint2(pc, pc + cnt);
+    if (st.order) {
+        st.place[sj] = small ? ps : (pl - ps) / (uint32_t)st.nparts;
+        const int c = small ? long_class(cnt) : 2;  // (the counters were cleared before the barrier)
+        const uint4 leaf = make_uint4(pc, pc + cnt, pl, 0u);
+        if (c < 2) st.longs[((size_t)s * 2 + c) * st.long_cap + atomicAdd(&st.nlong[2 * s + c], 1)] = leaf;
+        if (small) st.order[(size_t)s * st.leaf_cap + ps] = c < 2 ? make_uint4(0u, 0u, kNoLeaf, 0u) : leaf;
+    } else if (small) {
+        st.leaf_desc[(size_t)s * st.leaf_cap + pl] = make_uint2(pc, pc + cnt);
+    }
     if (j == kMaxK - 1) {
         st.nleaves[s] = (int)(pl + nl);
         st.nsmall[s] = (int)(ps + (small ? 1u : 0u));
@@ -233,16 +253,58 @@ static __global__ void __launch_bounds__(256) k_lbg_scan_blocks(LbgState st) {
     const size_t sj = (size_t)s * kMaxK + j;
     const bool leaves = !st.stream && st.count[sj] > (uint32_t)kSeqMax;
     const uint32_t first = st.start[sj];
-    uint2 *desc = st.leaf_desc + (size_t)s * st.leaf_cap + st.leaf_start[sj] + b0;
+    const uint32_t leaf0 = st.leaf_start[sj] + (uint32_t)b0;  // (read here: the stores below may alias it)
+    uint2 *desc = st.leaf_desc + (size_t)s * st.leaf_cap + leaf0;
+    // (order: the large clusters' leaves of a part side by side)
+    const int nsmall = st.order ? st.nsmall[s] : 0, nbig = st.order ? (st.nleaves[s] - nsmall) / st.nparts : 0;
+    const int place = st.order ? nsmall + b0 * nbig + (int)st.place[sj] : 0;
     // the segment's entries in one memory round trip (unconditional loads, clamped to the last part)
     uint32_t v[kScanSeg];
 #pragma unroll
     for (int u = 0; u < kScanSeg; ++u) v[u] = h[(size_t)(b0 + u < b1 ? u : b1 - 1 - b0) * kMaxK];
+    if (st.order) {  // uniform
+        uint32_t need = 0;  // this thread's long leaves of the two classes, 16 bits each; one reservation per wave and class
+#pragma unroll
+        for (int u = 0; u < kScanSeg; ++u) {
+            const int c = leaves && b0 + u < b1 ? long_class(v[u]) : 2;
+            need += c == 0 ? 1u : c == 1 ? 0x10000u : 0u;
+        }
+        const int lane = j & 63;
+        uint32_t upto = need;  // of this lane and those before it
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_up(upto, off);
+            upto += lane >= off ? o : 0u;
+        }
+        const uint32_t all = __shfl(upto, 63);
+        int base = 0;
+        if (lane < 2 && all) base = atomicAdd(&st.nlong[2 * s + lane], (int)((all >> (16 * lane)) & 0xffffu));
+        // the leaves at their places while the reservation is on its way
+        uint4 *order = st.order + (size_t)s * st.leaf_cap + place;
+        uint32_t at = first + run;
+#pragma unroll
+        for (int u = 0; u < kScanSeg; ++u) {
+            if (b0 + u < b1 && leaves)
+                order[(size_t)u * nbig] = v[u] >= kLong ? make_uint4(0u, 0u, kNoLeaf, 0u) : make_uint4(at, at + v[u], leaf0 + (uint32_t)u, 0u);
+            at += v[u];
+        }
+        if (all) {  // uniform
+            int slot0 = __shfl(base, 0) + (int)((upto - need) & 0xffffu), slot1 = __shfl(base, 1) + (int)((upto - need) >> 16);
+            uint4 *longs = st.longs + (size_t)s * 2 * st.long_cap;
+            at = first + run;
+#pragma unroll
+            for (int u = 0; u < kScanSeg; ++u) {
+                if (b0 + u < b1 && leaves && v[u] >= kLong)
+                    longs[v[u] >= kVeryLong ? slot0++ : st.long_cap + slot1++] = make_uint4(at, at + v[u], leaf0 + (uint32_t)u, 0u);
+                at += v[u];
+            }
+        }
+    }
 #pragma unroll
     for (int u = 0; u < kScanSeg; ++u) {
         if (b0 + u < b1) {
             h[(size_t)u * kMaxK] = run;
-            if (leaves) desc[u] = make_uint2(first + run, first + run + v[u]);
+            if (leaves && !st.order) desc[u] = make_uint2(first + run, first + run + v[u]);
             run += v[u];
         }
     }
@@ -455,6 +517,53 @@ static __global__ void __launch_bounds__(256) k_lbg_leafsum(LbgState st, const f
             if ((uint32_t)u < cnt) acc = acc + v[u];
     }
     st.leaf_sum[((size_t)s * st.leaf_cap + leaf) * sd + t] = acc;
+}
+
+// Wide column blocks: one workgroup per leaf, a lane per component, sixteen members in flight and the next sixteen
+// behind them; the adds stay in list order.  What bounds it is HBM, if the rows of the leaves in flight lie together and
+// no leaf is left for the end: the long leaves come first (a cluster that takes a third of the rows has 1,600 of a
+// part's 4096: a chain of 100 memory round trips), then the others part by part.  Cluster by cluster, as
+// k_lbg_leafsum takes them, the workgroups read all over the rows at once: 1M x 256, k = 256, with the cluster
+// sizes of a residual fit's eight stages 225-240 us per pass against 185-205; in the fit 259 -> 208, which is 53.5 ->
+// 50.1 ms for its eight stages with k_lbg_scan_blocks at 11 us instead of 5.5.  (Workgroups that stay and draw
+// leaves from a counter: 230-550 us, the draws are in the way; the workgroups past the last leaf cost nothing.)
+static __global__ void __launch_bounds__(256) k_lbg_leafsum_wide(LbgState st, const float *__restrict__ x, int64_t n,
+                                                                 int64_t ld, int sd) {
+    const int s = blockIdx.y;
+    if (st.done[s]) return;
+    const int n0 = st.nlong[2 * s], n1 = st.nlong[2 * s + 1], i = (int)blockIdx.x - n0 - n1;
+    if (i >= st.nleaves[s]) return;
+    const uint4 *longs = st.longs + (size_t)s * 2 * st.long_cap;
+    const uint4 e = i >= 0 ? st.order[(size_t)s * st.leaf_cap + i] : longs[(int)blockIdx.x < n0 ? (int)blockIdx.x : st.long_cap + i + n1];
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)e.x), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)e.y);
+    if (e.z == kNoLeaf) return;
+    const int t = (int)blockIdx.z * (int)blockDim.x + (int)threadIdx.x, lane = threadIdx.x & 63;
+    const uint32_t *__restrict__ perm = st.perm + (size_t)s * n;
+    const float *__restrict__ xc = x + (int64_t)s * sd + (t < sd ? t : 0);
+    float acc = 0.0f;
+    if (lo != hi) {  // (a part may have no member of a large cluster: zero, nothing to read)
+        constexpr int B = 16;
+        float a[B], b[B];
+        const uint32_t count = hi - lo;
+        uint32_t ids = 0;  // of 64 members, one per lane
+        auto rows = [&](uint32_t m, float(&v)[B]) {  // past the end: the last member's again, not added
+            if ((m & 63u) == 0) ids = perm[lo + m + lane < hi ? lo + m + lane : hi - 1];
+#pragma unroll
+            for (int u = 0; u < B; ++u) v[u] = xc[(int64_t)(uint32_t)__builtin_amdgcn_readlane((int)ids, (int)(m & 63u) + u) * ld];
+        };
+        rows(0, a);
+        for (uint32_t m = 0; m < count; m += 2 * B) {
+            if (m + B < count) rows(m + B, b);
+#pragma unroll
+            for (int u = 0; u < B; ++u)
+                if (m + u < count) acc = acc + a[u];
+            if (m + 2 * B < count) rows(m + 2 * B, a);
+#pragma unroll
+            for (int u = 0; u < B; ++u)
+                if (m + B + u < count) acc = acc + b[u];
+        }
+    }
+    if (t < sd) st.leaf_sum[((size_t)s * st.leaf_cap + e.z) * sd + t] = acc;
 }
 
 // Narrow column blocks (sub_dim a power of two up to 32): one wave per leaf.  A lane-per-component

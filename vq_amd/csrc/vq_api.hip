@@ -1362,7 +1362,14 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
     VQ_TRY(ensure(ctx, ctx->perm, sizeof(uint32_t) * (size_t)m * n));
     // per-part sums of the streaming kernel, then one folded sum per cluster
     if (stream) VQ_TRY(ensure(ctx, ctx->part_sum, sizeof(float) * (size_t)m * (nparts + 1) * vq::kMaxK * 8));
-    VQ_TRY(ensure(ctx, ctx->leaf_desc, sizeof(uint2) * (size_t)m * leaf_cap));
+    // Blocks of 64 to 512 floats: leaves handed out long ones first, then part by part (k_lbg_leafsum_wide)
+    const bool wide_leaves = !stream && sd >= 64 && sd <= 512;
+    const size_t long_cap = (size_t)(n / vq::kLong + 1), leaf_slots = (size_t)m * leaf_cap;
+    if (wide_leaves)  // the leaves in order, the two lists of long ones, the places, the counters
+        VQ_TRY(ensure(ctx, ctx->leaf_desc, sizeof(uint4) * (leaf_slots + 2 * (size_t)m * long_cap) +
+                                               sizeof(uint32_t) * (size_t)m * (vq::kMaxK + 2)));
+    else
+        VQ_TRY(ensure(ctx, ctx->leaf_desc, sizeof(uint2) * leaf_slots));
     VQ_TRY(ensure(ctx, ctx->leaf_sum, sizeof(float) * (size_t)m * leaf_cap * sd));
     VQ_TRY(ensure(ctx, ctx->codes, (size_t)m * n));
     VQ_TRY(ensure(ctx, ctx->idx, sizeof(uint32_t) * (size_t)m * k));
@@ -1395,6 +1402,13 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
     S.nseg = nseg;
     S.leaf_cap = leaf_cap;
     S.stream = stream ? 1 : 0;
+    if (wide_leaves) {
+        S.order = (uint4 *)ctx->leaf_desc.p;
+        S.longs = S.order + leaf_slots;
+        S.place = (uint32_t *)(S.longs + 2 * (size_t)m * long_cap);
+        S.nlong = (int *)(S.place + (size_t)m * vq::kMaxK);
+        S.long_cap = (int)long_cap;
+    }
 
     VQ_HIP(ctx, hipMemcpyAsync(ctx->idx.p, h_init_idx, sizeof(uint32_t) * (size_t)m * k,
                                hipMemcpyHostToDevice, st));
@@ -1474,6 +1488,11 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
             // leaves are the few clusters of up to 1024 members beside the streaming kernel
             hipLaunchKernelGGL(vq::k_lbg_leafsum_wg, dim3(leaf_cap, m), dim3(256), 0, gs, S, d_x, n, ld, sd,
                                shift);
+        } else if (wide_leaves) {
+            // a workgroup per place and per long leaf; a block above 256 floats in two halves
+            const int z = sd > 256 ? 2 : 1, threads = (int)cdiv(cdiv(sd, z), 64) * 64;
+            hipLaunchKernelGGL(vq::k_lbg_leafsum_wide, dim3((unsigned)(leaf_cap + long_cap), m, z), dim3(threads), 0, gs, S, d_x,
+                               n, ld, sd);
         } else if (sd <= 32 && (1 << shift) == sd && (int64_t)leaf_cap * sd * m < (1 << 20)) {
             // few leaves: a wave each; from a million (leaf, component) pairs on a lane each fills the GPU
             // (600,000 rows in 12 blocks of 16, k = 256, 16 rows per leaf: 1.1 against 0.25 ms)
