@@ -104,3 +104,42 @@ def test_resident_fit(ctx):
             ctx.set_assign_path(0)
         out.append(cb.download())
     assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["crowded", "clumps", "nan0", "nan7"])
+@pytest.mark.parametrize("metric", [O.SQEUCLIDEAN, O.EUCLIDEAN])
+@pytest.mark.parametrize("n,m,sd,k", [(131_075, 1, 128, 256), (44_000, 3, 72, 250), (140_000, 1, 256, 70)])
+def test_rows_with_many_candidates(ctx, n, m, sd, k, metric, kind):
+    """What the resident pass leaves open to three and more centroids: clumps of 2 to 90 neighbours (more than one batch
+    of candidates, ties among them), a codebook that leaves every row open (more entries than have masks), NaN."""
+    rng = np.random.default_rng(sd + k)
+    x, cb = rng.standard_normal((n, m, sd)).astype(F), rng.standard_normal((m, k, sd)).astype(F)
+    if kind == "crowded":
+        cb = (cb[:, :1] + F(1e-6) * cb).astype(F)
+    else:
+        at = 0
+        for size in (2, 3, 5, 20, 90):
+            end = min(k, at + size)
+            cb[:, at:end] = cb[:, at:at + 1] + F(1e-6) * cb[:, at:end]
+            cb[:, end - 1] = cb[:, at]  # the last of a clump equal to its first
+            at = end
+        cb = cb[:, rng.permutation(k)].copy()
+        x[::2] = cb[np.arange(m)[None, :], rng.integers(0, k, (x[::2].shape[0], 1))] + F(0.3) * x[::2]
+        if kind == "nan0":
+            cb[:, 0, 3] = np.nan
+        elif kind == "nan7":
+            cb[:, 7, 3] = np.nan
+    x = np.ascontiguousarray(x.reshape(n, m * sd))
+    dx, dcb, codes = ctx.to_device(x), ctx.to_device(cb), ctx.empty((n, m), np.uint8)
+    ctx.assign(metric, dx, n, m * sd, m, sd, k, dcb, codes)
+    got = codes.download()
+    assert ctx.last_recheck_split()[0] > 0
+    pick = np.concatenate([np.arange(1500), np.arange(n - 1500, n)])
+    with np.errstate(all="ignore"):
+        assert np.array_equal(got[pick], O.pq_encode(metric, x[pick], cb).astype(np.uint8))
+    ctx.set_assign_path(1)
+    try:
+        ctx.assign(metric, dx, n, m * sd, m, sd, k, dcb, codes)
+    finally:
+        ctx.set_assign_path(0)
+    assert np.array_equal(got, codes.download())

@@ -1078,6 +1078,8 @@ struct MfmaWideBfTables {
     uint32_t *list;        // undecided pairs (row * m + s) for the exact kernel over all centroids
     uint32_t *list_count;  // [0] entries of list, [1] entries of pairs
     uint2 *pairs;          // undecided pairs with only two candidates: {row * m + s, c1 | c2 << 8}
+    u32x4 *masks;          // k_assign_mfma_wide_res: [mask_cap][2] the candidates of an entry of list (candidate_bit)
+    uint32_t mask_cap;
     int nb;
     int sd;
     float kappa;           // COS: error-bound coefficient on ||x||
@@ -1738,7 +1740,7 @@ constexpr int kWideResThreads = 512;
 constexpr int64_t kWideResMinRows = 256 * 8 * 32 * 2;  // rows x column blocks
 inline size_t wide_res_lds(int sd, int nb) {
     const size_t npair = (sd + 15) / 16;
-    return npair * nb * 1024 + 2 * (size_t)nb * 128 + ((sd + 31) / 32) * 128 + 8 * 64 * (sizeof(uint2) + sizeof(uint32_t));
+    return npair * nb * 1024 + 2 * (size_t)nb * 128 + ((sd + 31) / 32) * 128 + 8 * 64 * sizeof(uint2);
 }
 
 template <bool LBG, int NB>
@@ -1753,7 +1755,6 @@ __global__ void __launch_bounds__(kWideResThreads, 2) k_assign_mfma_wide_res(Ass
     const int sd = tb.sd, npair = (sd + 15) / 16, nst = (npair + 1) / 2, total16 = npair * NB * 64;
     float *lds_c2 = reinterpret_cast<float *>(res_a + total16), *lds_pen = lds_c2 + NB * 32, *lds_mu = lds_pen + NB * 32;
     uint2 *my_pairs = reinterpret_cast<uint2 *>(lds_mu + ((sd + 31) & ~31)) + wave * 64;
-    uint32_t *my_list = reinterpret_cast<uint32_t *>(reinterpret_cast<uint2 *>(lds_mu + ((sd + 31) & ~31)) + 8 * 64) + wave * 64;
     const float sg = tb.sigma[s];
     const bool shifted = tb.shifted[s] != 0;  // uniform
     const u32x4 *ag = tb.atab + (size_t)s * total16;
@@ -1814,7 +1815,7 @@ __global__ void __launch_bounds__(kWideResThreads, 2) k_assign_mfma_wide_res(Ass
     };
     next_rows(0);
     const uint32_t keep = opaque_vgpr(0xFFFFFF00u);
-    uint32_t npairs = 0, nlist = 0;  // uniform
+    uint32_t npairs = 0;  // uniform
     auto flush_pairs = [&]() {
         uint32_t base = 0;
         if (lane == 0) base = atomicAdd(tb.list_count + 1, npairs);
@@ -1824,16 +1825,6 @@ __global__ void __launch_bounds__(kWideResThreads, 2) k_assign_mfma_wide_res(Ass
         if ((uint32_t)lane < npairs) tb.pairs[base + lane] = my_pairs[lane];
         __builtin_amdgcn_wave_barrier();
         npairs = 0;
-    };
-    auto flush_list = [&]() {
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(tb.list_count, nlist);
-        base = __builtin_amdgcn_readfirstlane(base);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if ((uint32_t)lane < nlist) tb.list[base + lane] = my_list[lane];
-        __builtin_amdgcn_wave_barrier();
-        nlist = 0;
     };
     for (; tile < ntiles; tile += step_tiles) {
         const int64_t row = tile * 32 + r;
@@ -1922,13 +1913,223 @@ __global__ void __launch_bounds__(kWideResThreads, 2) k_assign_mfma_wide_res(Ass
             npairs += (uint32_t)__popcll(pm);
         }
         if (lm) {
-            if (nlist > 32) flush_list();
-            if ((lm >> lane) & 1) my_list[nlist + __popcll(lm & below)] = (uint32_t)(row * a.m + s);
-            nlist += (uint32_t)__popcll(lm);
+            // the candidates: every centroid that is not clear of the best one (2^-14: the tag's bits); for a row or
+            // a block that is not finite all of them
+            const float least = (s1 + slack) * (1.0f + 2.0f * tb.rel) * 1.00006103515625f;
+            uint32_t mk[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int c = 0; c < NB; ++c)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    mk[c >> 1] |= !(finite && acc[c][v] + lifted > least) ? 1u << (16 * (c & 1) + v) : 0u;
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(tb.list_count, (uint32_t)__popcll(lm));
+            base = __builtin_amdgcn_readfirstlane(base);
+            if ((lm >> r) & 1) {
+                const uint32_t e = base + (uint32_t)__popcll(lm & (((uint64_t)1 << r) - 1));
+                if (h == 0) tb.list[e] = (uint32_t)(row * a.m + s);
+                if (e < tb.mask_cap) tb.masks[2 * (size_t)e + h] = u32x4{mk[0], mk[1], mk[2], mk[3]};
+            }
         }
     }
     if (npairs) flush_pairs();
-    if (nlist) flush_list();
+}
+
+// ---- what k_assign_mfma_wide_res leaves open ------------------------------------------------------
+// Pairs with two candidates, and rows with a mask of candidates (three to a few dozen of the 256), decided by
+// distances in the reference's order: a lane per candidate, each its own sequential chain.  The vectors come through LDS
+// 32 dimensions at a time, eight lanes per 128-byte segment, the next 32 in flight meanwhile (the pieces' order
+// depends on the slot: the lanes' 16-byte reads fall into different banks; 48 KB, three workgroups in a compute unit).  A lane that read its own row and centroid from memory touched 64 lines
+// per load instruction and had 64 of them one after the other, and a row that more than two centroids could win was
+// compared with all of them: per pass of a residual fit of 1M x 256, k = 256 (15,000-60,000 pairs, 500-4,000 rows) 54 us,
+// 20 so, the fit 50.1 -> 47.3 ms.  Bound by the rows from HBM (up to 60 MB; slices of 16 dimensions, or four in flight, the same).
+constexpr int kFollowSlots = 96;  // 32 rows and 64 centroids per wave, 32 floats each
+constexpr unsigned kFollowPairBlocks = 512, kFollowRowBlocks = 2048;
+constexpr uint32_t kFollowMany = 16384;  // rows from which on their candidates may be all centroids for all we know
+
+// Bit of centroid j in an entry's masks: half (j / 4) % 2, then 16 bits per block of 32.
+__device__ __forceinline__ bool candidate_bit(const u32x4 *mask, int j) {
+    const int c = j >> 5, v = ((j >> 3) & 3) * 4 + (j & 3);
+    const uint32_t w = reinterpret_cast<const uint32_t *>(mask + ((j >> 2) & 1))[c >> 1];
+    return (w >> (16 * (c & 1) + v)) & 1u;
+}
+
+template <bool LBG> __device__ __forceinline__ void store_code(const AssignArgs &a, int64_t row, int s, int code) {
+    if constexpr (LBG) {
+        uint8_t *p = a.codes + (size_t)s * a.n + row;
+        if (*p != (uint8_t)code) {
+            *p = (uint8_t)code;
+            mark_changed(a.changed + s);
+        }
+    } else {
+        a.codes[row * a.m + s] = (uint8_t)code;
+    }
+}
+
+__device__ __forceinline__ float4 *follow_piece(float *st, int slot, int piece) {
+    return reinterpret_cast<float4 *>(st + slot * 32 + 4 * (piece ^ ((slot >> 1) & 7)));
+}
+// The distance of the row in slot x to the centroid in slot c: acc goes on over 32 dimensions (nd of them) in LDS.
+template <int METRIC> __device__ __forceinline__ void follow_slice(float &acc, float *st, int x, int c, int nd) {
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+        if (4 * p >= nd) break;  // uniform
+        const float4 xv = *follow_piece(st, x, p), cv = *follow_piece(st, c, p);
+        wide_step<METRIC>(acc, xv.x, cv.x);
+        wide_step<METRIC>(acc, xv.y, cv.y);
+        wide_step<METRIC>(acc, xv.z, cv.z);
+        wide_step<METRIC>(acc, xv.w, cv.w);
+    }
+}
+
+template <int METRIC, bool LBG>
+__global__ void __launch_bounds__(256) k_wide_follow(AssignArgs a, int sd, const uint32_t *__restrict__ list,
+                                                     const uint32_t *__restrict__ counts, const u32x4 *__restrict__ masks,
+                                                     uint32_t mask_cap, const uint2 *__restrict__ pairs) {
+    static_assert(METRIC == M_SQ || METRIC == M_EUCLID, "squared L2 / Euclidean");
+    __shared__ __attribute__((aligned(16))) float stage[4][kFollowSlots * 32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane >> 3, piece = lane & 7;
+    float *st = stage[wave];
+    const int nsl = (sd + 31) / 32, m = a.m, k = a.k;
+    const float inf = __builtin_inff();
+    auto at = [&](int sl) { return 32 * sl + 4 * piece < sd ? 32 * sl + 4 * piece : 0; };  // (past the width: not used)
+    auto put = [&](int slot, float4 v) { *follow_piece(st, slot, piece) = v; };
+    auto meet = []() {  // LDS of one wave: what the lanes have stored is there for all of them
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    if (blockIdx.x < kFollowPairBlocks) {
+        // lanes 2 i and 2 i + 1: the candidates of pair i; slots 0 .. 31 the rows, 32 + lane the centroids
+        const uint32_t total = counts[1];
+        for (uint64_t base = (blockIdx.x * 4 + wave) * 32; base < total; base += kFollowPairBlocks * 4 * 32) {
+            const uint64_t e = base + (uint32_t)(lane >> 1);
+            const uint2 ent = pairs[e < total ? e : base];
+            const int64_t row = ent.x / (uint32_t)m;
+            const int s = (int)(ent.x % (uint32_t)m), j = (int)((ent.y >> (8 * (lane & 1))) & 0xFFu);
+            const float *xr[4], *cr[8];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t en = __shfl(ent.x, 2 * (8 * u + sub));
+                xr[u] = a.x + (int64_t)(en / (uint32_t)m) * a.ld + (int64_t)(en % (uint32_t)m) * sd;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) cr[u] = a.cb + ((size_t)__shfl(s, 8 * u + sub) * k + __shfl(j, 8 * u + sub)) * sd;
+            float4 px[4], pc[8];
+            auto fetch = [&](int sl) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) px[u] = *reinterpret_cast<const float4 *>(xr[u] + at(sl));
+#pragma unroll
+                for (int u = 0; u < 8; ++u) pc[u] = *reinterpret_cast<const float4 *>(cr[u] + at(sl));
+            };
+            fetch(0);
+            float acc = 0.0f;
+            for (int sl = 0; sl < nsl; ++sl) {
+                meet();  // the slice before has been read
+#pragma unroll
+                for (int u = 0; u < 4; ++u) put(8 * u + sub, px[u]);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) put(32 + 8 * u + sub, pc[u]);
+                meet();
+                fetch(sl + 1 < nsl ? sl + 1 : sl);
+                follow_slice<METRIC>(acc, st, lane >> 1, 32 + lane, sd - 32 * sl);
+            }
+            float d = METRIC == M_EUCLID ? sqrtf(acc) : acc;
+            d = (d == d) ? d : inf;
+            const float od = __shfl_xor(d, 1);
+            const int oj = __shfl_xor(j, 1);
+            if (e < total && (lane & 1) == 0) store_code<LBG>(a, row, s, (od < d || (od == d && oj < j)) ? oj : j);
+        }
+        return;
+    }
+    const uint32_t total = counts[0];
+    if (total > kFollowMany) {  // uniform: a degenerate codebook or input; the codebook once per eight rows, all of it
+        constexpr int room = 4 * kFollowSlots * 32;
+        const unsigned block = blockIdx.x - kFollowPairBlocks;
+        if (m == 1 && kRowsWg * sd + kRowsWgLdsFloats <= room) {
+            wide_exact_rows_wg<METRIC, LBG>(a, sd, list, total, block, kFollowRowBlocks, stage[0]);
+            return;
+        }
+        if (m > 1 && 4 * kWideRows * sd <= room) {
+            wide_exact_groups<METRIC, LBG, true, true, kWideRows>(a, sd, list, total, stage[0] + wave * kWideRows * sd, lane, wave,
+                                                                  block, kFollowRowBlocks);
+            return;
+        }
+    }
+    // one wave per row: slot 0 the row, slots 32 .. 95 up to 64 candidates at a time, in ascending order
+    for (uint64_t e = (blockIdx.x - kFollowPairBlocks) * 4 + wave; e < total; e += kFollowRowBlocks * 4) {
+        const uint32_t ent = list[e];
+        const int64_t row = ent / (uint32_t)m;
+        const int s = (int)(ent % (uint32_t)m);
+        const float *xr = a.x + row * a.ld + (int64_t)s * sd;
+        unsigned long long has[4];
+        int nc = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int j = 64 * q + lane;
+            has[q] = __ballot(j < k && (e >= mask_cap || candidate_bit(masks + 2 * e, j)));
+            nc += __popcll(has[q]);
+        }
+        float bd = inf;
+        int bj = 0;
+        for (int c0 = 0; c0 < nc; c0 += 64) {
+            // candidate c0 + i -> its centroid
+            auto centroid = [&](int i) {
+                int left = c0 + i, j = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int here = __popcll(has[q]);
+                    if (left >= 0 && left < here) {
+                        unsigned long long w = has[q];
+                        for (int u = left; u > 0; --u) w &= w - 1;
+                        j = 64 * q + __ffsll(w) - 1;
+                    }
+                    left -= here;
+                }
+                return j;
+            };
+            const int live = nc - c0 < 64 ? nc - c0 : 64;
+            const int j = lane < live ? centroid(lane) : 0;
+            const int groups = (live + 7) / 8;  // uniform
+            float4 px, pc[8];
+            const float *cr[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) cr[u] = a.cb + ((size_t)s * k + __shfl(j, 8 * u + sub)) * sd;
+            auto fetch = [&](int sl) {
+                px = *reinterpret_cast<const float4 *>(xr + at(sl));
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (u < groups) pc[u] = *reinterpret_cast<const float4 *>(cr[u] + at(sl));
+            };
+            fetch(0);
+            float acc = 0.0f;
+            for (int sl = 0; sl < nsl; ++sl) {
+                meet();
+                if (lane < 8) put(0, px);
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (u < groups) put(32 + 8 * u + sub, pc[u]);
+                meet();
+                fetch(sl + 1 < nsl ? sl + 1 : sl);
+                follow_slice<METRIC>(acc, st, 0, 32 + (lane < live ? lane : 0), sd - 32 * sl);
+            }
+            const float raw = METRIC == M_EUCLID ? sqrtf(acc) : acc;
+            const float d = lane < live && raw == raw ? raw : inf;  // a NaN distance never wins
+            const uint32_t least = wave_umin(__float_as_uint(d));
+            const int first = __ffsll(__ballot(__float_as_uint(d) == least)) - 1;  // ascending candidates: the lowest index
+            const int fj = __builtin_amdgcn_readlane(j, first);
+            const float fd = __uint_as_float(least);
+            if (c0 == 0 || fd < bd) {
+                bd = fd;
+                bj = fj;
+            }
+            // ... unless it is centroid 0's, which is never displaced
+            if (c0 == 0 && (has[0] & 1) && __builtin_amdgcn_readlane((int)(raw != raw), 0)) {
+                bj = 0;
+                break;
+            }
+        }
+        if (lane == 0) store_code<LBG>(a, row, s, bj);
+    }
 }
 
 }  // namespace vq

@@ -289,7 +289,9 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + 2 * n_c2 + (size_t)a.m * nb + (size_t)a.m * sd + 2 * a.m + 2 * (size_t)a.m * nsl + 8) + 64));
     // header (two counts), the list for the all-centroid check, the list for the two-candidate check
     const size_t n_pairs = (size_t)a.n * a.m;
-    VQ_TRY(ensure(ctx, ctx->mfma_list, sizeof(uint32_t) * (4 + ((n_pairs + 1) & ~(size_t)1) + 2 * n_pairs)));
+    // ... and the candidates of an eighth of the pairs (a list beyond that goes over all centroids)
+    const size_t mask_cap = n_pairs / 8 + 4096, n_list = 4 + ((n_pairs + 3) & ~(size_t)3) + ((2 * n_pairs + 3) & ~(size_t)3);
+    VQ_TRY(ensure(ctx, ctx->mfma_list, sizeof(uint32_t) * (n_list + 8 * mask_cap)));
     float *atab = (float *)ctx->mfma_tab.p;
     float *c2perm = atab + n_atab;
     float *pen = c2perm + n_c2;
@@ -297,7 +299,8 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     float *mu = maxc2 + (((size_t)a.m * nb + 3) & ~(size_t)3);  // 16-byte aligned: read as float4
     uint32_t *count = (uint32_t *)ctx->mfma_list.p;
     uint32_t *list = count + 4;
-    uint2 *pairs = (uint2 *)(list + ((n_pairs + 1) & ~(size_t)1));  // 8-byte aligned
+    uint2 *pairs = (uint2 *)(list + ((n_pairs + 3) & ~(size_t)3));  // 16-byte aligned
+    vq::u32x4 *masks = (vq::u32x4 *)(count + n_list);               // likewise
     float2 *norms = (float2 *)(mu + (size_t)a.m * sd);  // sd is a multiple of 8: 8-byte aligned
     int *shifted = (int *)(norms + (size_t)a.m * nsl);
     float *sigma = (float *)(shifted + a.m);
@@ -333,7 +336,7 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
         void *args[] = {&cb, &mu, &norms, &shifted, &m, &k, &nbv, &sdv, &atab4, &c2perm, &maxc2, &count, &pen, &pc, &sigma, &pd, &cnorm};
         VQ_HIP(ctx, hipLaunchKernel(prep, dim3(a.m, nb), dim3(256), args, 0, ctx->stream));
     }
-    vq::MfmaWideBfTables tb{(const vq::u32x4 *)atab, c2perm, pen, maxc2, mu, shifted, sigma, list, count, pairs, nb, sd,
+    vq::MfmaWideBfTables tb{(const vq::u32x4 *)atab, c2perm, pen, maxc2, mu, shifted, sigma, list, count, pairs, masks, (uint32_t)mask_cap, nb, sd,
                             kappa, twice * cross * t, twice * t / rho, lift, rel};
     const size_t res_lds = vq::wide_res_lds(sd, nb);
     const bool resident = half && !a.pend_cb && res_lds <= 160 * 1024 && a.n * a.m >= vq::kWideResMinRows &&
@@ -381,6 +384,15 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     }
     VQ_HIP(ctx, hipGetLastError());
     ctx->recheck_src = 2;
+    if constexpr (!COS) {
+        if (resident) {
+            hipLaunchKernelGGL((vq::k_wide_follow<METRIC, LBG>), dim3(vq::kFollowPairBlocks + vq::kFollowRowBlocks), dim3(256), 0,
+                               ctx->stream, a, sd, (const uint32_t *)list, (const uint32_t *)count, (const vq::u32x4 *)masks,
+                               (uint32_t)mask_cap, (const uint2 *)pairs);
+            VQ_HIP(ctx, hipGetLastError());
+            return VQ_OK;
+        }
+    }
     // undecided pairs with two candidates and the few that need every centroid, in one launch
     return launch_wide_exact<METRIC, LBG>(ctx, a, sd, list, count, (const uint2 *)pairs,
                                           (const uint32_t *)(count + 1));
