@@ -1,4 +1,4 @@
-"""Column blocks of 8 floats (and of widths padded to 8) with 257 to 2048 centroids in one pass: codes against the
+"""Column blocks of 8 and 16 floats (and of widths padded to them) with 257 to 2048 and 1024 centroids in one pass: codes against the
 CPU oracle at the edges of the centroid tiles, of the two workgroup sizes and of the row tiles, for badly scaled,
 tied and non-finite input."""
 import numpy as np
@@ -34,17 +34,19 @@ def _check(ctx, x, cb, metric, ld=None):
 
 @pytest.mark.parametrize("kind", ["normal", "collapsed", "near_ties", "grid", "spread", "overflow", "tiny", "offset", "edges"])
 @pytest.mark.parametrize("metric", [O.SQEUCLIDEAN, O.EUCLIDEAN, O.COSINE])
-@pytest.mark.parametrize("n,m,k", [(700, 3, 257), (1300, 2, 1000), (333, 2, 2048)])
-def test_codes(ctx, n, m, k, metric, kind):
-    x, cb = _case(kind, n, m, 8, k)
+@pytest.mark.parametrize("n,m,k,sd", [(700, 3, 257, 8), (1300, 2, 1000, 8), (333, 2, 2048, 8), (700, 2, 300, 16), (300, 2, 1024, 16)])
+def test_codes(ctx, n, m, k, sd, metric, kind):
+    x, cb = _case(kind, n, m, sd, k)
     _check(ctx, x, cb, metric)
 
 
 @pytest.mark.parametrize("k", [300, 320, 321, 511, 513, 1024, 1216, 1217, 1985, 2047])
-@pytest.mark.parametrize("n,m,sd", [(1, 600, 8), (33, 20, 8), (5000, 1, 8), (2049, 3, 7), (900, 2, 5)])
+@pytest.mark.parametrize("n,m,sd", [(1, 600, 8), (33, 20, 8), (5000, 1, 8), (2049, 3, 7), (900, 2, 5), (2049, 2, 16), (700, 3, 11)])
 def test_sizes(ctx, n, m, sd, k):
     rng = np.random.default_rng(k + n)
     x, cb = rng.random((n, m * sd), dtype=F), rng.random((m, k, sd), dtype=F)
+    if sd > 8 and k > 1024:
+        pytest.skip("chunk by chunk: test_gpu_big_k.py")
     cb[:, k - 1] = cb[:, 3]  # a tie of the last centroid with an early one
     cb[:, k // 2] = cb[:, k // 2 - 1]  # and of neighbours
     x[: n // 3] = cb[np.arange(m), :][:, rng.integers(0, k, n // 3)].transpose(1, 0, 2).reshape(n // 3, m * sd)

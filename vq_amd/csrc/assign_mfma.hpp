@@ -181,10 +181,10 @@ __device__ __forceinline__ uint32_t bf16_pack2(float a, float b) {
 // candidates; the 2^-16 of both norms covers them.  Rows and centroids whose norm is outside [1e-15, 1e15]
 // and not zero, where the reference's products may over- or underflow, and rows of norm zero go to the exact
 // argmin (a centroid of norm zero has d = 1: its operand is zero and its ||c~||^2 kCosScale^2, in order).
-__device__ __forceinline__ float seq_norm8(const float (&c)[8]) {
+template <int SD> __device__ __forceinline__ float seq_norm8(const float (&c)[SD]) {
     float acc = 0.0f;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
+    for (int t = 0; t < SD; ++t) {
         const float p = c[t] * c[t];
         acc = acc + p;
     }
@@ -210,15 +210,15 @@ template <int METRIC> __device__ __forceinline__ float key_dist(uint32_t k) {
     if constexpr (METRIC == M_COS) return __uint_as_float(k ^ ((k & 0x80000000u) ? 0x80000000u : 0xffffffffu));
     return __uint_as_float(k);
 }
-// The distance of a row's eight floats to centroid c, in the reference's order; na, nb: the two norms.
-template <int METRIC>
-__device__ __forceinline__ float dist8(const float (&x)[8], const float (&c)[8], float na, float nb) {
+// The distance of a row's SD floats to centroid c, in the reference's order; na, nb: the two norms.
+template <int METRIC, int SD>
+__device__ __forceinline__ float dist8(const float (&x)[SD], const float (&c)[SD], float na, float nb) {
     if constexpr (METRIC == M_COS) {
-        const float dot = d_dot<8>(x, c);
+        const float dot = d_dot<SD>(x, c);
         const float den = na * nb, q = dot / den;
         return (na == 0.0f || nb == 0.0f) ? 1.0f : 1.0f - q;
     } else {
-        const float d = d_sq<8>(x, c);
+        const float d = d_sq<SD>(x, c);
         return METRIC == M_EUCLID ? sqrtf(d) : d;
     }
 }
@@ -230,11 +230,12 @@ __device__ __forceinline__ float mfma8_scale(float r2, int up = 2, float most = 
     if (r2 == 0.0f) return 1.0f;  // all centroids are the same
     return r2 > 1e-36f && r2 < most ? ldexpf(1.0f, up - (ilogbf(r2) >> 1)) : __builtin_nanf("");
 }
-// The A operand of one centroid and one lane half: a[t] = -2 c[t] of the half's four dimensions, scaled.
-// Elements below the normal range of binary16 count as zero, whatever the matrix cores make of them.
-// n2, d2: the half's shares of ||c~||^2 and of ||c - c~||^2.
-struct Half8 {
-    uint32_t h01, h23, l01;
+// The A operand of one centroid and one lane half: a[t] = -2 c[t] of the half's NH dimensions, scaled: NH / 2
+// words of high parts, then the low parts of the first NH - 2 dimensions, one instruction per 8 slots (the last
+// word of the last is c2_word's).  Elements below the normal range of binary16 count as zero, whatever the matrix
+// cores make of them.  n2, d2: the half's shares of ||c~||^2 and of ||c - c~||^2.
+template <int NH> struct HalfOp {
+    uint32_t w[NH - 1];
     float n2, d2;
 };
 __device__ __forceinline__ float f16_normal(float v) {
@@ -245,21 +246,22 @@ __device__ __forceinline__ uint32_t f16_pack2(float a, float b) {  // round to n
     using h2 = _Float16 __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(uint32_t, h2{(_Float16)a, (_Float16)b});
 }
-__device__ __forceinline__ Half8 half8(const float (&a)[4]) {
-    float hi[4], lo[4] = {0.f, 0.f, 0.f, 0.f};
-    Half8 o;
+template <int NH> __device__ __forceinline__ HalfOp<NH> half_op(const float (&a)[NH]) {
+    float hi[NH], lo[NH];
+    HalfOp<NH> o;
     o.n2 = o.d2 = 0.0f;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < NH; ++t) {
         hi[t] = f16_normal(a[t]);
-        if (t < 2) lo[t] = f16_normal(a[t] - hi[t]);
+        lo[t] = t < NH - 2 ? f16_normal(a[t] - hi[t]) : 0.0f;
         const float d = (a[t] - hi[t]) - lo[t], v = hi[t] + lo[t];
         o.n2 = __builtin_fmaf(0.25f * v, v, o.n2);
         o.d2 = __builtin_fmaf(0.25f * d, d, o.d2);
     }
-    o.h01 = f16_pack2(hi[0], hi[1]);
-    o.h23 = f16_pack2(hi[2], hi[3]);
-    o.l01 = f16_pack2(lo[0], lo[1]);
+#pragma unroll
+    for (int t = 0; t < NH / 2; ++t) o.w[t] = f16_pack2(hi[2 * t], hi[2 * t + 1]);
+#pragma unroll
+    for (int t = 0; t < NH / 2 - 1; ++t) o.w[NH / 2 + t] = f16_pack2(lo[2 * t], lo[2 * t + 1]);
     return o;
 }
 // The last word: 1 against the row's share of ||x||^2, and the half's part of c2 = ||c~||^2 against 1.
@@ -323,13 +325,13 @@ __device__ __forceinline__ void mfma8_prep_block(float (&c)[8], int s, int j, in
     if (j < nb * 32) {
         const int b = j / 32, i = j % 32;
         u32x4 *dst = atab + ((size_t)s * nb + b) * 64;
-        Half8 o[2];
+        HalfOp<4> o[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             float a[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) a[t] = j < k ? -2.0f * (c[4 * h + t] * sg) : 0.0f;
-            o[h] = half8(a);
+            o[h] = half_op<4>(a);
         }
         // (a centroid of norm zero has the cosine distance 1: as far as any at a right angle)
         const float c2 = COS && zero ? kCosScale * kCosScale : o[0].n2 + o[1].n2;
@@ -338,7 +340,7 @@ __device__ __forceinline__ void mfma8_prep_block(float (&c)[8], int s, int j, in
             md = o[0].d2 + o[1].d2;
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) dst[32 * h + i] = u32x4{o[h].h01, o[h].h23, o[h].l01, c2_word(c2, h, j < k)};
+        for (int h = 0; h < 2; ++h) dst[32 * h + i] = u32x4{o[h].w[0], o[h].w[1], o[h].w[2], c2_word(c2, h, j < k)};
     }
     // a NaN poisons the bound on purpose
 #pragma unroll
@@ -548,7 +550,7 @@ __device__ __forceinline__ void own_operands(const char *cl, const float *norms,
 #pragma unroll
         for (int u = 0; u < 4; ++u)
             a[u] = !live ? 0.0f : COS ? (scale * cv[b][u]) * kCosScale : scale * (cv[b][u] - sum[u]);
-        const Half8 o = half8(a);
+        const HalfOp<4> o = half_op<4>(a);
         int pa, pb;
         swap_halves(__float_as_int(o.n2), pa, pb);
         c2 = COS && nc == 0.0f ? kCosScale * kCosScale : __int_as_float(pa) + __int_as_float(pb);
@@ -557,7 +559,7 @@ __device__ __forceinline__ void own_operands(const char *cl, const float *norms,
         const float cx = live ? c2 + bad : 0.0f;
         mx = (mx == mx && cx == cx) ? fmaxf(mx, cx) : __builtin_nanf("");
         md = fmaxf(md, live ? d2 : 0.0f);
-        A[b] = u32x4{o.h01, o.h23, o.l01, c2_word(c2, h, live)};
+        A[b] = u32x4{o.w[0], o.w[1], o.w[2], c2_word(c2, h, live)};
     }
 #pragma unroll
     for (int off = 16; off > 0; off >>= 1) {
@@ -569,38 +571,39 @@ __device__ __forceinline__ void own_operands(const char *cl, const float *norms,
     mdc = md;
 }
 
-// The row operand of a tile: the lane's four dimensions relative to the centre (cosine: of length kCosScale).
-struct Row8 {
-    u32x4 b16;
-    float e2;            // what the rounding lost, squared, both halves
+// The row operand of a tile: the lane's NH dimensions relative to the centre (cosine: of length kCosScale), as
+// HalfOp's slots want them.
+template <int NH> struct RowOp {
+    u32x4 b16[NH / 4];
+    float e2;                    // what the rounding lost, squared, both halves
     float x2 = 0.0f, rx = 0.0f;  // cosine: ||x||^2 and 1 / ||x|| of the row as it is
 };
-template <int METRIC>
-__device__ __forceinline__ Row8 row8(const float (&xraw)[4], float sg, const float (&muh)[4]) {
-    Row8 o;
-    float xv[4];
+template <int METRIC, int NH>
+__device__ __forceinline__ RowOp<NH> row_op(const float (&xraw)[NH], float sg, const float (&muh)[NH]) {
+    RowOp<NH> o;
+    float xv[NH];
     int pa, pb;
     float p = 0.0f, d2 = 0.0f;
     if constexpr (METRIC == M_COS) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) p = __builtin_fmaf(xraw[u], xraw[u], p);
+        for (int u = 0; u < NH; ++u) p = __builtin_fmaf(xraw[u], xraw[u], p);
         swap_halves(__float_as_int(p), pa, pb);
         o.x2 = __int_as_float(pa) + __int_as_float(pb);
         o.rx = __builtin_amdgcn_rsqf(o.x2);
         const float f = kCosScale * o.rx;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) xv[u] = xraw[u] * f;
+        for (int u = 0; u < NH; ++u) xv[u] = xraw[u] * f;
         p = 0.0f;
     } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) xv[u] = __builtin_fmaf(xraw[u], sg, muh[u]);
+        for (int u = 0; u < NH; ++u) xv[u] = __builtin_fmaf(xraw[u], sg, muh[u]);
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) p = __builtin_fmaf(xv[u], xv[u], p);
+    for (int u = 0; u < NH; ++u) p = __builtin_fmaf(xv[u], xv[u], p);
     using h2 = _Float16 __attribute__((ext_vector_type(2)));
-    uint32_t w[2];
+    uint32_t w[NH];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < NH / 2; ++u) {
         w[u] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{xv[2 * u], xv[2 * u + 1]}), h2));
         float dl, dh;  // x~ - x: one instruction each that reads a half of the pair
         asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(dl) : "v"(w[u]), "v"(xv[2 * u]));
@@ -610,32 +613,34 @@ __device__ __forceinline__ Row8 row8(const float (&xraw)[4], float sg, const flo
     }
     swap_halves(__float_as_int(d2), pa, pb);
     o.e2 = __int_as_float(pa) + __int_as_float(pb);
-    o.b16 = u32x4{w[0], w[1], w[0],
-                  __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{p * kLift8, 1.0f}), h2))};
+#pragma unroll
+    for (int u = 0; u < NH / 2 - 1; ++u) w[NH / 2 + u] = w[u];
+    w[NH - 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{p * kLift8, 1.0f}), h2));
+#pragma unroll
+    for (int i = 0; i < NH / 4; ++i) o.b16[i] = u32x4{w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]};
     return o;
 }
 // Whether the best of the two smallest keys has won (false for NaN / inf - inf); e2c: the centroids' share of
-// the rounding, acc8: 3 * 2^-16 max ||c~||^2 (||x||^2 <= 2 (s2 + ||c||^2) stands for the row's norm).
-template <int METRIC>
-__device__ __forceinline__ bool decided8(float s1, float s2, const Row8 &row, float e2c, float acc8) {
-    const float E = (row.e2 + kFlush8) + e2c;
+// the rounding, acc8: 3 * NH / 4 * 2^-16 max ||c~||^2 (||x||^2 <= 2 (s2 + ||c||^2) stands for the row's norm).
+template <int METRIC, int NH>
+__device__ __forceinline__ bool decided8(float s1, float s2, const RowOp<NH> &row, float e2c, float acc8) {
+    const float E = (row.e2 + kFlush8 * (NH / 4)) + e2c;
     const float margin = __builtin_fmaf(4.001f, __builtin_amdgcn_sqrtf(2.0f * s2 * E), __builtin_fmaf(8.0f, E, acc8)) +
-                         9.1552734375e-05f * s2;
+                         (6.103515625e-05f + NH / 4 * 3.0517578125e-05f) * s2;
     // 1.2e5: below every padding centroid
     return (s2 - s1) > margin && s1 < 1.2e5f && (METRIC != M_COS || (row.x2 > 1e-30f && row.x2 < 1e30f));
 }
-// A lane half's share of the distance to a centroid: its four dimensions, fused.  Cosine: of the inner product.
-template <int METRIC> __device__ __forceinline__ float share8(const float (&xraw)[4], float4 v) {
-    const float c[4] = {v.x, v.y, v.z, v.w};
+// A lane half's share of the distance to a centroid: NH dimensions, fused.  Cosine: of the inner product.
+template <int METRIC, int NH> __device__ __forceinline__ float share8(const float (&xraw)[NH], const float (&c)[NH]) {
     if constexpr (METRIC == M_COS) {
         float p = xraw[0] * c[0];
 #pragma unroll
-        for (int u = 1; u < 4; ++u) p = __builtin_fmaf(xraw[u], c[u], p);
+        for (int u = 1; u < NH; ++u) p = __builtin_fmaf(xraw[u], c[u], p);
         return p;
     } else {
         float d = xraw[0] - c[0], p = d * d;
 #pragma unroll
-        for (int u = 1; u < 4; ++u) {
+        for (int u = 1; u < NH; ++u) {
             d = xraw[u] - c[u];
             p = __builtin_fmaf(d, d, p);
         }
@@ -785,8 +790,8 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
         xb = fetch_x(t + 2);
         if constexpr (LBG) ob = fetch_c(t + 2);
         const float xraw[4] = {xc.x, xc.y, xc.z, xc.w};
-        const Row8 row = row8<METRIC>(xraw, sg, muh);
-        const u32x4 xb16 = row.b16;
+        const RowOp<4> row = row_op<METRIC, 4>(xraw, sg, muh);
+        const u32x4 xb16 = row.b16[0];
         int m1 = 0x7f800000, m2 = 0x7f800000;  // +inf
         // One block of 32 centroids.  The tag leaves out the lane half (bit 2), so it is the same in
         // every lane and lives in scalar registers.
@@ -853,7 +858,7 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
         const float s1 = __int_as_float(imin(f1, g1));
         const float s2 = __int_as_float(imin(imax(f1, g1), imin(f2, g2)));
         const bool mine = h == 0 && t < lane_tiles;  // the lane's row of this tile exists
-        const bool near = decided8<METRIC>(s1, s2, row, mdc, acc8);
+        const bool near = decided8<METRIC, 4>(s1, s2, row, mdc, acc8);
         const int first = (int)(__float_as_uint(s1) & 0xFCu);  // first centroid of the best run
         // The best of the run's four centroids.  Each lane half takes its four dimensions of all of them (fused
         // multiply-adds), the halves' sums meet two centroids each; the smallest that is clear of the second by
@@ -864,7 +869,10 @@ __global__ void __launch_bounds__(256, 3) k_assign_mfma8(AssignArgs a, Mfma8Tabl
             const int run = Lds8<METRIC>::run(first, h);
             float p[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) p[i] = share8<METRIC>(xraw, Lds8<METRIC>::piece(cl, run, i));
+            for (int i = 0; i < 4; ++i) {
+                const float4 v = Lds8<METRIC>::piece(cl, run, i);
+                p[i] = share8<METRIC, 4>(xraw, {v.x, v.y, v.z, v.w});
+            }
             // lower half: centroids first, first + 1; upper half: first + 2, first + 3
             const auto r02 = __builtin_amdgcn_permlane32_swap(__float_as_int(p[0]), __float_as_int(p[2]), false, false);
             const auto r13 = __builtin_amdgcn_permlane32_swap(__float_as_int(p[1]), __float_as_int(p[3]), false, false);

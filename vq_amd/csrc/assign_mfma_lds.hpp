@@ -1,6 +1,6 @@
-// Nearest-centroid assignment for 8-float column blocks with 257 to 2048 centroids: one pass over the rows for
-// the whole codebook, 16-bit codes.  The scores, their bound and the decision are those of k_assign_mfma8
-// (assign_mfma.hpp); what differs is where the operands lie and how a row's best centroids are kept.
+// Nearest-centroid assignment with the operands of a whole column block in LDS: blocks of 8 floats with 257 to 2048
+// centroids (16-bit codes), blocks of 16 floats with up to 1024.  The scores, their bound and the decision are those of
+// k_assign_mfma8 (assign_mfma.hpp); what differs is where the operands lie and how a row's best centroids are kept.
 //
 // This translation unit must be compiled with -ffp-contract=off.
 #pragma once
@@ -8,40 +8,55 @@
 
 namespace vq {
 
-constexpr int kBig8Max = 2048;
+constexpr int kBig8Max = 2048, kLds16Max = 1024;
 constexpr float kBig8Far = 1e18f;   // components of the padding centroids: squares stay finite, and farther off than
                                     // any centroid of a block whose scale exists (kBig8Rms)
 constexpr float kBig8Rms = 1e30f;   // largest mean square norm about the centre that is scored
 
-struct Big8Args {
-    const float *x;
-    int64_t n, ld;
-    int m, k;
-    const float *cb;     // [m][k][8], 16-byte aligned
-    uint16_t *codes;     // [n][m]
-    int64_t stride;      // workgroups of a column block
+enum { CODES_LBG = 0, CODES_U8 = 1, CODES_U16 = 2 };  // [m][n] bytes in place (old -> new), [n][m] bytes, [n][m] 16 bits
+struct LdsArgs {
+    AssignArgs a;          // 16-byte aligned codebooks; codes: see above (CODES_U16: codes16)
+    uint16_t *codes16;
+    int64_t stride;        // workgroups of a column block
     uint32_t *stat, *stat_next;  // counters of undecided pairs: of this pass, and of the next (cleared)
 };
 
-// Centroids padded to whole pairs of blocks of 32; operands 32 bytes and the centroid itself 32 bytes each, under
+// Centroids padded to whole pairs of blocks of 32; the operand (4 bytes per float) and the centroid itself, under
 // cosine its norm and the reciprocal.
-inline int big8_padded(int k) { return (k + 63) / 64 * 64; }
-inline size_t big8_lds(bool cosine, int k) { return (size_t)big8_padded(k) * (64 + (cosine ? 8 : 0)); }
+inline int lds_padded(int k) { return (k + 63) / 64 * 64; }
+inline size_t assign_lds(bool cosine, int k, int sd) { return (size_t)lds_padded(k) * (8 * sd + (cosine ? 8 : 0)); }
 
-// The workgroup's copy of its block's centroids: planes as in Lds8, runs of 64 bytes with the order inside a
-// run depending on the run, so that a phase of the pick's reads, sixteen runs at random, meets all banks.
-struct LdsBig8 {
+// The workgroup's copy of its block's centroids: planes of four dimensions as in Lds8, runs of 64 bytes with the order
+// inside a run depending on the run, so that a phase of the pick's reads, sixteen runs at random, meets all banks.
+// A lane half's dimensions are SD / 8 planes side by side.
+template <int SD> struct LdsBlock {
+    static constexpr int NH = SD / 2, Q = SD / 8;  // dimensions and planes of a half
     char *cl;
     int plane;
-    __device__ __forceinline__ int run(int j, int h) const { return h * plane + j * 16 + ((j >> 4) & 3) * 16; }
-    __device__ __forceinline__ float4 piece(int at, int i) const { return *reinterpret_cast<const float4 *>(cl + (at ^ (i * 16))); }
-    __device__ __forceinline__ float4 half(int j, int h) const { return piece(run(j & ~3, h), j & 3); }
-    __device__ __forceinline__ void set(int j, int h, float4 v) const {
-        *reinterpret_cast<float4 *>(cl + (run(j & ~3, h) ^ ((j & 3) * 16))) = v;
+    __device__ __forceinline__ int run(int j, int h) const { return h * Q * plane + j * 16 + ((j >> 4) & 3) * 16; }
+    __device__ __forceinline__ float4 at(int run, int i, int q) const {
+        return *reinterpret_cast<const float4 *>(cl + (run ^ (i * 16)) + q * plane);
     }
-    __device__ __forceinline__ void load(int j, float (&c)[8]) const {
-        const float4 a = half(j, 0), b = half(j, 1);
-        c[0] = a.x, c[1] = a.y, c[2] = a.z, c[3] = a.w, c[4] = b.x, c[5] = b.y, c[6] = b.z, c[7] = b.w;
+    __device__ __forceinline__ void piece(int run, int i, float (&c)[NH]) const {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const float4 v = at(run, i, q);
+            c[4 * q] = v.x, c[4 * q + 1] = v.y, c[4 * q + 2] = v.z, c[4 * q + 3] = v.w;
+        }
+    }
+    __device__ __forceinline__ void set(int j, int piece16, float4 v) const {  // the centroid's 16-byte piece
+        *reinterpret_cast<float4 *>(cl + (run(j & ~3, 0) ^ ((j & 3) * 16)) + piece16 * plane) = v;
+    }
+    __device__ __forceinline__ float component(int j, int t) const {
+        return *reinterpret_cast<const float *>(cl + (run(j & ~3, 0) ^ ((j & 3) * 16)) + (t >> 2) * plane + (t & 3) * 4);
+    }
+    __device__ __forceinline__ void load(int j, float (&c)[SD]) const {
+        const int r = run(j & ~3, 0);
+#pragma unroll
+        for (int q = 0; q < 2 * Q; ++q) {
+            const float4 v = at(r, j & 3, q);
+            c[4 * q] = v.x, c[4 * q + 1] = v.y, c[4 * q + 2] = v.z, c[4 * q + 3] = v.w;
+        }
     }
 };
 
@@ -49,28 +64,31 @@ struct LdsBig8 {
 // sums and keeps the two smallest.  One lane with one centroid within 2^-16 of the smallest has the answer;
 // otherwise the reference's distances decide, the first of the smallest (a NaN sorts behind +inf, centroid 0 wins
 // where it is NaN or nothing is below +inf).
-template <int METRIC>
-__device__ __forceinline__ int exact_rows_big8(unsigned long long todo, int code, const LdsBig8 &cl, const float *norms,
-                                               int kp, const float (&xr)[8], float rx, int k, int lane) {
+template <int METRIC, int SD>
+__device__ __forceinline__ int exact_rows_lds(unsigned long long todo, int code, const LdsBlock<SD> &cl, const float *norms,
+                                              int kp, const float (&xr)[SD], float rx, int k, int lane) {
     constexpr uint32_t kInfKey = METRIC == M_COS ? 0xff800000u : 0x7f800000u;  // sort key of +inf
     constexpr int M = METRIC == M_COS ? M_COS : M_SQ;  // Euclidean: squares first
     const int at0 = cl.run(lane & ~3, 0) ^ ((lane & 3) * 16);  // of centroid lane; 64 centroids on is 1 KB on
     while (todo) {
         const int src = __builtin_amdgcn_readfirstlane(__ffsll(todo) - 1);
         todo &= todo - 1;
-        float xs[8];
+        float xs[SD];
 #pragma unroll
-        for (int d = 0; d < 8; ++d) xs[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xr[d]), src));
+        for (int d = 0; d < SD; ++d) xs[d] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xr[d]), src));
         int best = -1;
         {
             const float rxs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rx), src));
-            const float lo4[4] = {xs[0], xs[1], xs[2], xs[3]}, hi4[4] = {xs[4], xs[5], xs[6], xs[7]};
             uint32_t lo = 0xffffffffu, second = 0xffffffffu, first = 0;
             int at = 0;
             for (int q = 0; q < k; q += 64) {
-                const char *p = cl.cl + at0 + 16 * q;
-                float d = share8<METRIC>(lo4, *reinterpret_cast<const float4 *>(p)) +
-                          share8<METRIC>(hi4, *reinterpret_cast<const float4 *>(p + cl.plane));
+                float c[SD];
+#pragma unroll
+                for (int u = 0; u < SD / 4; ++u) {
+                    const float4 v = *reinterpret_cast<const float4 *>(cl.cl + at0 + 16 * q + u * cl.plane);
+                    c[4 * u] = v.x, c[4 * u + 1] = v.y, c[4 * u + 2] = v.z, c[4 * u + 3] = v.w;
+                }
+                float d = share8<METRIC, SD>(xs, c);
                 if constexpr (METRIC == M_COS) d = __builtin_fmaf(-(d * rxs), norms[kp + q + lane], 1.001f);
                 const uint32_t key = __float_as_uint(d);
                 if (q == 0) first = key;
@@ -90,7 +108,7 @@ __device__ __forceinline__ int exact_rows_big8(unsigned long long todo, int code
         if (best < 0) {  // uniform
             const float na = METRIC == M_COS ? seq_norm8(xs) : 0.0f;
             auto key_of = [&](int j) {
-                float c[8];
+                float c[SD];
                 cl.load(j, c);
                 const float d = dist8<M>(xs, c, na, METRIC == M_COS ? norms[j] : 0.0f);
                 return j < k && d == d ? dist_key<M>(d) : 0xffffffffu;
@@ -135,11 +153,14 @@ __device__ __forceinline__ int exact_rows_big8(unsigned long long todo, int code
 // k = 300 240 -> 140 us, 512 269 -> 170, 1024 515 -> 235; 200,000, k = 1500 568 -> 249; 150,000, k = 2048 613 -> 243;
 // 1,000, k = 257 20 -> 11, k = 2048 84 -> 30; 100,000 x 12 blocks of 7, k = 1024 269 -> 93.  Bound by vector-instruction
 // issue (26 per 64 centroids and tile) and the matrix instructions that only partly hide behind it.
-template <int METRIC>
-__global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
-    extern __shared__ __attribute__((aligned(16))) char lds[];
-    __shared__ float red[2][16][8];
-    constexpr bool COS = METRIC == M_COS;
+// LBG: codes in place, changed[s] set where one differs, converged blocks left out.
+template <int METRIC, int SD, int CODES>
+__global__ void __launch_bounds__(SD == 8 ? 1024 : 768, SD == 8 ? 4 : 3) k_assign_mfma_lds(LdsArgs args) {
+    extern __shared__ __attribute__((aligned(16))) char lds_block[];
+    __shared__ float red[2][16][SD], mu_all[SD];
+    constexpr bool COS = METRIC == M_COS, LBG = CODES == CODES_LBG;
+    constexpr int NH = SD / 2, NI = SD / 8;  // dimensions of a lane half, matrix instructions per 32 centroids
+    const AssignArgs &a = args.a;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int T = (int)blockDim.x, W = T >> 6;
     const int r = lane & 31, h = lane >> 5;
@@ -152,63 +173,57 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
     const int64_t ntiles = (a.n + 31) / 32;
     if (first_wg * W >= ntiles) return;
     if (blockIdx.x == 0)
-        for (int i = threadIdx.x; i < kStatSlots; i += T) a.stat_next[i * kStatStride] = 0u;
+        for (int i = threadIdx.x; i < kStatSlots; i += T) args.stat_next[i * kStatStride] = 0u;
+    if constexpr (LBG) {
+        if (block_done(a, s)) return;  // uniform
+    }
 
-    u32x4 *at = reinterpret_cast<u32x4 *>(lds);  // [kp / 32][64]
-    const LdsBig8 cl{lds + kp * 32, kp * 16};
-    float *norms = reinterpret_cast<float *>(lds + kp * 64);
+    u32x4 *at = reinterpret_cast<u32x4 *>(lds_block);  // [kp / 32][NI][64]
+    const LdsBlock<SD> cl{lds_block + kp * 4 * SD, kp * 16};
+    float *norms = reinterpret_cast<float *>(lds_block + kp * 8 * SD);
     {
-        const float4 *src = reinterpret_cast<const float4 *>(a.cb + (size_t)s * k * 8);
-        for (int i = threadIdx.x; i < 2 * kp; i += T)
-            cl.set(i >> 1, i & 1, i < 2 * k ? src[i] : make_float4(kBig8Far, kBig8Far, kBig8Far, kBig8Far));
+        constexpr int P = SD / 4;  // 16-byte pieces of a centroid
+        const float4 *src = reinterpret_cast<const float4 *>(a.cb + (size_t)s * k * SD);
+        for (int i = threadIdx.x; i < P * kp; i += T)
+            cl.set(i / P, i % P, i < P * k ? src[i] : make_float4(kBig8Far, kBig8Far, kBig8Far, kBig8Far));
     }
     __syncthreads();
-    float mu[8], sg = kCosScale, bad = 0.0f;
+    float mu[SD], sg = kCosScale, bad = 0.0f;
     if constexpr (COS) {
         for (int j = threadIdx.x; j < kp; j += T) {
-            float c[8];
+            float c[SD];
             cl.load(j, c);
             const float nc = seq_norm8(c);
             norms[j] = nc;
             norms[kp + j] = nc == 0.0f || j >= k ? 0.0f : 1.0f / nc;
         }
 #pragma unroll
-        for (int t = 0; t < 8; ++t) mu[t] = 0.0f;
+        for (int t = 0; t < SD; ++t) mu[t] = 0.0f;
     } else {
-        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        for (int j = threadIdx.x; j < k; j += T) {
-            float c[8];
-            cl.load(j, c);
+        // a thread per dimension and share of the centroids: two or three shuffles where a sum of all dimensions in
+        // every thread took six for each (1,000 rows x 10 blocks of 16: 17.7 -> 10.8 us)
+        const int t = threadIdx.x % SD, G = T / SD;
+        float v = 0.0f;
+        for (int j = threadIdx.x / SD; j < k; j += G) v += cl.component(j, t) * 0.00048828125f;  // / 2048: no overflow
 #pragma unroll
-            for (int t = 0; t < 8; ++t) v[t] += c[t] * 0.00048828125f;  // / 2048: no overflow
-        }
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) v[t] += __shfl_xor(v[t], off);
-            if (lane == 0) red[0][wave][t] = v[t];
-        }
+        for (int off = SD; off < 64; off <<= 1) v += __shfl_xor(v, off);
+        if (lane < SD) red[0][wave][t] = v;
         __syncthreads();
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            mu[t] = 0.0f;
-            for (int w = 0; w < W; ++w) mu[t] += red[0][w][t];
-            mu[t] *= 2048.0f / (float)k;
-        }
+        v = 0.0f;
+        for (int w = 0; w < W; ++w) v += red[0][w][t];
+        v *= 2048.0f / (float)k;
+        if ((int)threadIdx.x < SD) mu_all[t] = v;
         float p = 0.0f;
-        for (int j = threadIdx.x; j < k; j += T) {
-            float c[8];
-            cl.load(j, c);
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const float d = (c[t] - mu[t]) * 0.015625f;
-                p = __builtin_fmaf(d, d, p);  // / 4096
-            }
+        for (int j = threadIdx.x / SD; j < k; j += G) {
+            const float d = (cl.component(j, t) - v) * 0.015625f;
+            p = __builtin_fmaf(d, d, p);  // / 4096
         }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) p += __shfl_xor(p, off);
         if (lane == 0) red[1][wave][0] = p;
         __syncthreads();
+#pragma unroll
+        for (int u = 0; u < SD; ++u) mu[u] = mu_all[u];
         float r2 = 0.0f;
         for (int w = 0; w < W; ++w) r2 += red[1][w][0];
         sg = mfma8_scale(r2 * (4096.0f / (float)k), 1, kBig8Rms);  // root mean square 2 ... 4: none longer than 181
@@ -216,20 +231,20 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
     }
     float mc2 = 0.0f, mdc = 0.0f;
     for (int j = threadIdx.x; j < kp; j += T) {
-        float c[8];
+        float c[SD];
         cl.load(j, c);
         const bool live = j < k;
         const float nc = COS && live ? norms[j] : 1.0f;
-        Half8 o[2];
+        HalfOp<NH> o[2];
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
-            float v[4];
+            float v[NH];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const float e = c[4 * hh + t];
-                v[t] = !live ? 0.0f : COS ? (nc == 0.0f ? 0.0f : -2.0f * (e * (1.0f / nc)) * kCosScale) : -2.0f * ((e - mu[4 * hh + t]) * sg);
+            for (int t = 0; t < NH; ++t) {
+                const float e = c[NH * hh + t];
+                v[t] = !live ? 0.0f : COS ? (nc == 0.0f ? 0.0f : -2.0f * (e * (1.0f / nc)) * kCosScale) : -2.0f * ((e - mu[NH * hh + t]) * sg);
             }
-            o[hh] = half8(v);
+            o[hh] = half_op<NH>(v);
         }
         const float c2 = COS && nc == 0.0f ? kCosScale * kCosScale : o[0].n2 + o[1].n2;
         if (live) {
@@ -239,8 +254,15 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
             mdc = fmaxf(mdc, o[0].d2 + o[1].d2);
         }
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh)
-            at[(j / 32) * 64 + 32 * hh + j % 32] = u32x4{o[hh].h01, o[hh].h23, o[hh].l01, c2_word(c2, hh, live)};
+        for (int hh = 0; hh < 2; ++hh) {
+            uint32_t w[NH];
+#pragma unroll
+            for (int t = 0; t < NH - 1; ++t) w[t] = o[hh].w[t];
+            w[NH - 1] = c2_word(c2, hh, live);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                at[((j / 32) * NI + i) * 64 + 32 * hh + j % 32] = u32x4{w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]};
+        }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -258,36 +280,52 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
         mc2 = (mc2 == mc2 && o == o) ? fmaxf(mc2, o) : __builtin_nanf("");
         mdc = fmaxf(mdc, red[0][w][1]);
     }
-    float muh[4];
+    float muh[NH];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) muh[u] = COS ? 0.0f : -((h ? mu[4 + u] : mu[u]) * sg);
+    for (int u = 0; u < NH; ++u) muh[u] = COS ? 0.0f : -((h ? mu[NH + u] : mu[u]) * sg);
     const uint32_t keep = opaque_vgpr(0xFFFFFF00u);
-    const float acc8 = 4.57763671875e-05f * mc2;  // 3 * 2^-16: see decided8
+    const float acc8 = NH / 4 * 4.57763671875e-05f * mc2;  // see decided8
 
     // tiles t, t + step, ...; rows two tiles ahead
-    const int64_t step = a.stride * W;
+    const int64_t step = args.stride * W;
     int64_t t = first_wg * W + wave;
-    const uint32_t loff = 4u * ((uint32_t)r * (uint32_t)a.ld + 4u * (uint32_t)h);
+    const uint32_t loff = 4u * ((uint32_t)r * (uint32_t)a.ld + (uint32_t)NH * (uint32_t)h);
     typedef float rowpiece __attribute__((ext_vector_type(4), aligned(4)));
-    auto fetch = [&](int64_t tile) {
+    auto fetch = [&](int64_t tile, rowpiece(&v)[NH / 4]) {
         const int64_t row0 = (tile < ntiles ? tile : ntiles - 1) * 32;  // uniform
-        const char *base = reinterpret_cast<const char *>(a.x + row0 * a.ld + (int64_t)s * 8);
-        const rowpiece v = *reinterpret_cast<const rowpiece *>(base + (r < a.n - row0 ? loff : 16u * (uint32_t)h));
-        return make_float4(v[0], v[1], v[2], v[3]);
+        const char *base = reinterpret_cast<const char *>(a.x + row0 * a.ld + (int64_t)s * SD);
+        const uint32_t o = r < a.n - row0 ? loff : 4u * NH * (uint32_t)h;
+#pragma unroll
+        for (int q = 0; q < NH / 4; ++q) v[q] = *reinterpret_cast<const rowpiece *>(base + o + 16 * q);
+    };
+    uint8_t oa = 0, ob = 0;
+    auto fetch_c = [&](int64_t tile) {
+        const int64_t row0 = (tile < ntiles ? tile : ntiles - 1) * 32;
+        return a.codes[(size_t)s * a.n + row0 + (r < a.n - row0 ? r : 0)];
     };
     uint32_t n_exact = 0;
-    float4 xa = fetch(t), xb = fetch(t + step);
+    bool chg = false;
+    rowpiece xa[NH / 4], xb[NH / 4];
+    fetch(t, xa);
+    if constexpr (LBG) oa = fetch_c(t);
+    fetch(t + step, xb);
+    if constexpr (LBG) ob = fetch_c(t + step);
     for (; t < ntiles; t += step) {
-        const float xraw[4] = {xa.x, xa.y, xa.z, xa.w};
-        xa = xb;
-        xb = fetch(t + 2 * step);
-        const Row8 row = row8<METRIC>(xraw, sg, muh);
-        const u32x4 xb16 = row.b16;
+        float xraw[NH];
+#pragma unroll
+        for (int u = 0; u < NH; ++u) xraw[u] = xa[u / 4][u % 4];
+#pragma unroll
+        for (int q = 0; q < NH / 4; ++q) xa[q] = xb[q];
+        fetch(t + 2 * step, xb);
+        const uint8_t old = oa;
+        oa = ob;
+        if constexpr (LBG) ob = fetch_c(t + 2 * step);
+        const RowOp<NH> row = row_op<METRIC, NH>(xraw, sg, muh);
         const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         int m1 = 0x7f800000, m2 = 0x7f800000, o1 = 0x7f800000, o2 = 0x7f800000;  // +inf; even and odd pairs
         floatx16 p0, p1, q0, q1;
-#define VQ_MFMA(av, acc)                                                                                              \
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, av), __builtin_bit_cast(f16x8, xb16), zero, 0, 0, 0);
+#define VQ_MFMA(av, xv, from, acc)                                                                                    \
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, av), __builtin_bit_cast(f16x8, xv), from, 0, 0, 0);
 #define VQ_MIN8(c, d, p)                                                                                              \
     imin(imin(imin(imin(imin(imin(imin(__float_as_int(c[4 * p]), __float_as_int(c[4 * p + 1])),                       \
                                    __float_as_int(c[4 * p + 2])), __float_as_int(c[4 * p + 3])),                      \
@@ -298,13 +336,18 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
 #define VQ_PAIR(c, d, e, f, first, second, T0, T1, T2, T3, next)                                                      \
     {                                                                                                                 \
         int key[4];                                                                                                   \
-        VQ_MFMA(n0, e)                                                                                                \
+        VQ_MFMA(n0[0], row.b16[0], zero, e)                                                                           \
+        if constexpr (NI == 2) VQ_MFMA(n1[0], row.b16[0], zero, f)                                                    \
         __builtin_amdgcn_sched_barrier(0);                                                                            \
         VQ_KEY(c, d, 0, T0) VQ_KEY(c, d, 1, T1)                                                                       \
         __builtin_amdgcn_sched_barrier(0);                                                                            \
-        VQ_MFMA(n1, f)                                                                                                \
-        n0 = ap[(next) * 128];                                                                                        \
-        n1 = ap[(next) * 128 + 64];                                                                                   \
+        if constexpr (NI == 2) {                                                                                      \
+            VQ_MFMA(n0[NI - 1], row.b16[NI - 1], e, e)                                                                \
+            VQ_MFMA(n1[NI - 1], row.b16[NI - 1], f, f)                                                                \
+        } else {                                                                                                      \
+            VQ_MFMA(n1[0], row.b16[0], zero, f)                                                                       \
+        }                                                                                                             \
+        operands(next);                                                                                               \
         __builtin_amdgcn_sched_barrier(0);                                                                            \
         VQ_KEY(c, d, 2, T2) VQ_KEY(c, d, 3, T3)                                                                       \
         top2_push4(first, second, key[0], key[1], key[2], key[3]);                                                    \
@@ -314,11 +357,22 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
         uint32_t t0 = 0, t1 = 2, t2 = 4, t3 = 6, t4 = 8, t5 = 10, t6 = 12, t7 = 14;
         auto opaque = [](uint32_t &v) { asm volatile("" : "+s"(v)); };  // (else each is made again from one of them)
         const u32x4 *ap = at + lane;
-        u32x4 n0 = ap[0], n1 = ap[64];
-        VQ_MFMA(n0, p0)
-        VQ_MFMA(n1, p1)
-        n0 = ap[128];
-        n1 = ap[192];
+        u32x4 n0[NI], n1[NI];  // of the next pair's two blocks
+        auto operands = [&](int pair) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                n0[i] = ap[(pair * 2 * NI + i) * 64];
+                n1[i] = ap[((pair * 2 + 1) * NI + i) * 64];
+            }
+        };
+        operands(0);
+        VQ_MFMA(n0[0], row.b16[0], zero, p0)
+        VQ_MFMA(n1[0], row.b16[0], zero, p1)
+        if constexpr (NI == 2) {
+            VQ_MFMA(n0[NI - 1], row.b16[NI - 1], p0, p0)
+            VQ_MFMA(n1[NI - 1], row.b16[NI - 1], p1, p1)
+        }
+        operands(np > 1 ? 1 : 0);
         for (int p = 0; p < np; p += 2) {
             opaque(t0), opaque(t1), opaque(t2), opaque(t3), opaque(t4), opaque(t5), opaque(t6), opaque(t7);
             VQ_PAIR(p0, p1, q0, q1, m1, m2, t0, t1, t2, t3, p + 2 < np ? p + 2 : 0)
@@ -342,7 +396,7 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
         const float s1 = __int_as_float(set1), s2 = __int_as_float(imin(set2, others));
         const int64_t row0 = t * 32;
         const bool mine = h == 0 && r < a.n - row0;  // the lane's row exists
-        bool near = decided8<METRIC>(s1, s2, row, mdc, acc8);
+        bool near = decided8<METRIC, NH>(s1, s2, row, mdc, acc8);
         // The best of a set's eight centroids, runs first and first + 32: each lane half sums its four dimensions of
         // all of them, the lower half then holds the first run's distances, the upper half the second's, the place in
         // the run in the two low bits.  at: the best; lo, hi: the two smallest keys (lower lanes).
@@ -359,8 +413,11 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
             int ky[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(share8<METRIC>(xraw, cl.piece(ra, i))),
-                                                                 __float_as_int(share8<METRIC>(xraw, cl.piece(rb, i))), false, false);
+                float ca[NH], cb[NH];
+                cl.piece(ra, i, ca);
+                cl.piece(rb, i, cb);
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(share8<METRIC, NH>(xraw, ca)),
+                                                                 __float_as_int(share8<METRIC, NH>(xraw, cb)), false, false);
                 float d = __int_as_float((int)sw[0]) + __int_as_float((int)sw[1]);
                 if constexpr (COS) d = j0 + i < k ? __builtin_fmaf(-(d * row.rx), iv[i], 1.001f) : 1e30f;
                 ky[i] = (int)((__float_as_uint(d) & 0xFFFFFFFCu) | (uint32_t)i);
@@ -385,7 +442,7 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
         int other = -1;  // the second set, where it may have the answer
         unsigned long long todo = __ballot(mine && !near);
         if (todo) {  // the same in every lane
-            if (!near && decided8<METRIC>(s1, __int_as_float(others), row, mdc, acc8)) other = first_of(set2);
+            if (!near && decided8<METRIC, NH>(s1, __int_as_float(others), row, mdc, acc8)) other = first_of(set2);
             const bool two = other >= 0;
             if (__ballot(mine && two)) {
                 int code2, lo2, hi2;
@@ -402,13 +459,13 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
         }
         const unsigned long long ties = __ballot(mine && near && !clear);
         if (todo | ties) {  // the same in every lane
-            float xs[8];  // the lane's row
+            float xs[SD];  // the lane's row
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                int lo, hi;
-                swap_halves(__float_as_int(xraw[u]), lo, hi);
-                xs[u] = __int_as_float(lo);
-                xs[4 + u] = __int_as_float(hi);
+            for (int u = 0; u < NH; ++u) {
+                int xl, xh;
+                swap_halves(__float_as_int(xraw[u]), xl, xh);
+                xs[u] = __int_as_float(xl);
+                xs[NH + u] = __int_as_float(xh);
             }
             if (ties) {  // the sets' centroids by the reference's distances: the first of the smallest
                 const float na = COS ? seq_norm8(xs) : 0.0f;
@@ -416,7 +473,7 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
                 int bj = -1;
                 for (int i = 0; i < (__ballot(other >= 0 && !clear) ? 16 : 8); ++i) {
                     const int j = (i < 8 || other < 0 ? first : other) + (i & 3) + ((i >> 2) & 1) * 32;
-                    float c[8];
+                    float c[SD];
                     cl.load(j, c);
                     const float d = dist8<METRIC>(xs, c, na, COS ? norms[j] : 0.0f);
                     if (j < k && (bj < 0 || d < bd || (d == bd && j < bj))) {
@@ -428,13 +485,47 @@ __global__ void __launch_bounds__(1024) k_assign_mfma8_big(Big8Args a) {
             }
             if (todo) {
                 n_exact += (uint32_t)__popcll(todo);
-                code = exact_rows_big8<METRIC>(todo, code, cl, norms, kp, xs, row.rx, k, lane);
+                code = exact_rows_lds<METRIC, SD>(todo, code, cl, norms, kp, xs, row.rx, k, lane);
             }
         }
-        if (mine) a.codes[(size_t)(row0 + r) * m + s] = (uint16_t)code;
+        if (mine) {
+            if constexpr (CODES == CODES_U16) {
+                args.codes16[(size_t)(row0 + r) * m + s] = (uint16_t)code;
+            } else if constexpr (CODES == CODES_U8) {
+                a.codes[(size_t)(row0 + r) * m + s] = (uint8_t)code;
+            } else if (old != (uint8_t)code) {
+                a.codes[(size_t)s * a.n + row0 + r] = (uint8_t)code;
+                chg = true;
+            }
+        }
+    }
+    if constexpr (LBG) {
+        // once per wave, and only where the flag still reads 0 (see k_assign_mfma8)
+        if (__any(chg) && lane == 0 && a.changed[s] == 0) a.changed[s] = 1;
     }
     if (lane == 0 && n_exact)
-        atomicAdd(a.stat + ((first_wg * W + wave) & (kStatSlots - 1)) * kStatStride, n_exact);
+        atomicAdd(args.stat + ((first_wg * W + wave) & (kStatSlots - 1)) * kStatStride, n_exact);
+}
+
+// One round of workgroups: sixteen waves per compute unit (blocks of 8 floats; twelve with 16), as two workgroups, or
+// three, while their LDS leaves room.
+template <int METRIC, int SD, int CODES>
+inline hipError_t launch_mfma_lds(hipStream_t stream, LdsArgs &args) {
+    const size_t lds = assign_lds(METRIC == M_COS, args.a.k, SD);
+    const int waves_cu = SD == 8 ? 16 : 12;
+    const int wgs_cu = lds <= 50 * 1024 && SD == 16 ? 3 : lds <= 77 * 1024 ? 2 : 1, waves = waves_cu / wgs_cu;
+    const int64_t tiles = (args.a.n + 31) / 32;
+    int64_t stride = 256 * wgs_cu / args.a.m / 8 * 8;
+    if (stride < 8) stride = 8;
+    const int64_t most = ((tiles + waves - 1) / waves + 7) / 8 * 8;
+    if (stride > most) stride = most;
+    if (stride * args.a.m >= (1LL << 31)) return hipErrorInvalidConfiguration;
+    args.stride = stride;
+    const void *kern = reinterpret_cast<const void *>(k_assign_mfma_lds<METRIC, SD, CODES>);
+    const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    void *kargs[] = {&args};
+    return hipLaunchKernel(kern, dim3((unsigned)(stride * args.a.m)), dim3((unsigned)(64 * waves)), kargs, lds, stream);
 }
 
 }  // namespace vq

@@ -1,6 +1,6 @@
 // Codebooks of more than 256 centroids (16-bit codes).
 //
-// Assignment (blocks of 8 floats up to 2048 centroids: assign_mfma8_big.hpp): the codebook of every column block is
+// Assignment (blocks of 8 and 16 floats up to 2048 and 1024 centroids: assign_mfma_lds.hpp): the codebook of every column block is
 // cut into chunks of 256 consecutive centroids.
 // Each chunk goes through the 8-bit assignment kernels unchanged, which leave the chunk's own
 // winner (the lowest index of the smallest distance inside the chunk, src/utils.rs:62-70); a merge

@@ -17,6 +17,7 @@
 #include "ctx.hpp"
 #include "assign_exact.hpp"
 #include "assign_mfma.hpp"
+#include "assign_mfma_lds.hpp"
 #include "decode.hpp"
 
 #ifndef VQ_MFMA_RUN
@@ -420,6 +421,25 @@ bool mfma_applicable(const vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     return a.k <= 256;
 }
 
+// 16-float column blocks: one pass with the operands in LDS, undecided rows resolved in the same kernel
+// (assign_mfma_lds.hpp).  Against the kernel of wider blocks, its tables and its follow-up (an encode, Euclidean): 600,000 x
+// 8 blocks, k = 256 369 -> 195 us, 60,000 x 10 61 -> 37, k = 32 33 -> 26, 1,000 x 10 15.4 -> 10.8; cosine 376 -> 201, 64 -> 36.
+template <int METRIC, bool LBG>
+bool mfma16_applicable(const vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
+    if (ctx->assign_path == 1 || ctx->no_alloc || a.pend_cb) return false;
+    if (METRIC != vq::M_SQ && METRIC != vq::M_EUCLID && !(METRIC == vq::M_COS && !LBG)) return false;
+    // float4 centroid loads; 32 rows within 32-bit byte offsets
+    return sd == 16 && (reinterpret_cast<uintptr_t>(a.cb) & 15) == 0 && a.ld <= (1 << 20) && a.m <= 65535 && a.k <= 256;
+}
+template <int METRIC, bool LBG> int32_t launch_mfma16(vq_ctx *ctx, const vq::AssignArgs &a) {
+    vq::LdsArgs args{};
+    args.a = a;
+    VQ_TRY(next_counters(ctx, &args.stat, &args.stat_next));
+    ProfSpan sp(ctx, VQ_PROF_ASSIGN_KERNEL);
+    VQ_HIP(ctx, (vq::launch_mfma_lds<METRIC, 16, LBG ? vq::CODES_LBG : vq::CODES_U8>(ctx->stream, args)));
+    return VQ_OK;
+}
+
 // The width to pad every column block to so that the matrix-core kernels take the shape (squared L2,
 // Euclidean, cosine; 0: they take it as it is, or padding does not pay).  fit: for the passes of a fit,
 // which pads its rows once and whose update then streams blocks of 8 as well.
@@ -431,7 +451,9 @@ bool mfma_applicable(const vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
 int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bool fit) {
     if (ctx->assign_path == 1 || ctx->no_alloc || metric < VQ_SQEUCLIDEAN || metric > VQ_COSINE) return 0;
     if (sd == 1 || a.k < 32 || a.k > vq::kMaxK || a.m > 65535) return 0;
-    if (mfma_applicable<vq::M_SQ, true>(ctx, a, sd) || mfma_wide_applicable<vq::M_SQ, true>(ctx, a, sd)) return 0;
+    if (mfma_applicable<vq::M_SQ, true>(ctx, a, sd) || mfma16_applicable<vq::M_SQ, true>(ctx, a, sd) ||
+        mfma_wide_applicable<vq::M_SQ, true>(ctx, a, sd))
+        return 0;
     const int sdp = (sd + 7) / 8 * 8;
     // the limits of those kernels
     if ((int64_t)a.m * sdp > (1 << 20) || sdp > (1 << 16) || a.n * a.m >= (1LL << 32)) return 0;
@@ -466,6 +488,10 @@ int32_t launch_assign(vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, 
     if constexpr (!LBG)
         if (metric == VQ_COSINE && mfma_applicable<vq::M_COS, false>(ctx, a, sd))
             return launch_mfma<vq::M_COS, false>(ctx, a, tables_ready, started, done);
+    if (metric == VQ_SQEUCLIDEAN && mfma16_applicable<vq::M_SQ, LBG>(ctx, a, sd)) return launch_mfma16<vq::M_SQ, LBG>(ctx, a);
+    if (metric == VQ_EUCLIDEAN && mfma16_applicable<vq::M_EUCLID, LBG>(ctx, a, sd)) return launch_mfma16<vq::M_EUCLID, LBG>(ctx, a);
+    if constexpr (!LBG)
+        if (metric == VQ_COSINE && mfma16_applicable<vq::M_COS, false>(ctx, a, sd)) return launch_mfma16<vq::M_COS, false>(ctx, a);
     if constexpr (!LBG)
         if (metric == VQ_COSINE && mfma_wide_applicable<vq::M_COS, false>(ctx, a, sd))
             return launch_mfma_wide<vq::M_COS, false>(ctx, a, sd);
@@ -800,7 +826,8 @@ int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, i
     }
     ProfSpan sp(ctx, VQ_PROF_ENCODE);
     const int sdp = pend ? 0 : pad_width(ctx, metric, a, sd, false);
-    if (metric == VQ_COSINE && !mfma8 && sdp != 8) {  // the 8-float kernel makes the norms itself
+    // the kernels for 8 and 16 floats make the norms themselves
+    if (metric == VQ_COSINE && !mfma8 && sdp != 8 && sdp != 16 && !mfma16_applicable<vq::M_COS, false>(ctx, a, sd)) {
         float *cnorm = (float *)(ctx->static_scratch + kNoAllocNormOff);
         if (!ctx->no_alloc) {
             VQ_TRY(ensure(ctx, ctx->cnorm, sizeof(float) * (size_t)m * k));

@@ -10,7 +10,7 @@
 #include "ctx.hpp"
 #include "lbg_update.hpp"
 #include "bigk.hpp"
-#include "assign_mfma8_big.hpp"
+#include "assign_mfma_lds.hpp"
 
 using namespace vqh;
 
@@ -26,51 +26,53 @@ void launch_merge(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int m, i
                        k, chunks, base, count, win, win_d, stride, have_d, best, out);
 }
 
-// 8-float column blocks of up to kBig8Max centroids: the whole codebook in one pass over the rows.
-// One round of workgroups: two of 512 threads per compute unit while their LDS leaves room for two, one of 1024
-// threads above 1024 centroids (sixteen waves either way).
-int32_t launch_big8(vq_ctx *ctx, int metric, const float *d_x, int64_t n, int64_t ld, int m, int k, const float *d_codebooks,
-                    uint16_t *d_codes) {
-    const size_t lds = vq::big8_lds(metric == VQ_COSINE, k);
-    const int threads = lds <= 78 * 1024 ? 512 : 1024, waves = threads / 64;
-    const int64_t tiles = cdiv(n, 32);
-    int64_t stride = std::max<int64_t>(8, (1024 * 256 / threads) / m / 8 * 8);
-    stride = std::min<int64_t>(stride, cdiv(cdiv(tiles, waves), 8) * 8);
-    if (stride * m >= (1LL << 31)) return fail(ctx, VQ_ERR_UNSUPPORTED, "n * m too large for one launch");
-    vq::Big8Args a{d_x, n, ld, m, k, d_codebooks, d_codes, stride, nullptr, nullptr};
-    VQ_TRY(next_counters(ctx, &a.stat, &a.stat_next));
-    const void *kern = metric == VQ_SQEUCLIDEAN ? (const void *)vq::k_assign_mfma8_big<vq::M_SQ>
-                       : metric == VQ_EUCLIDEAN ? (const void *)vq::k_assign_mfma8_big<vq::M_EUCLID>
-                                                : (const void *)vq::k_assign_mfma8_big<vq::M_COS>;
-    VQ_HIP(ctx, hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    void *args[] = {&a};
-    VQ_HIP(ctx, hipLaunchKernel(kern, dim3((unsigned)(stride * m)), dim3((unsigned)threads), args, lds, ctx->stream));
+// Column blocks of 8 or 16 floats: the whole codebook in one pass over the rows.
+int32_t launch_big(vq_ctx *ctx, int metric, const float *d_x, int64_t n, int64_t ld, int m, int sd, int k, const float *d_codebooks,
+                   uint16_t *d_codes) {
+    vq::LdsArgs args{};
+    args.a.x = d_x;
+    args.a.n = n;
+    args.a.ld = ld;
+    args.a.m = m;
+    args.a.k = k;
+    args.a.cb = d_codebooks;
+    args.codes16 = d_codes;
+    VQ_TRY(next_counters(ctx, &args.stat, &args.stat_next));
+#define BIG(M) \
+    VQ_HIP(ctx, sd == 8 ? (vq::launch_mfma_lds<M, 8, vq::CODES_U16>(ctx->stream, args)) : (vq::launch_mfma_lds<M, 16, vq::CODES_U16>(ctx->stream, args)))
+    switch (metric) {
+    case VQ_SQEUCLIDEAN: BIG(vq::M_SQ); break;
+    case VQ_EUCLIDEAN: BIG(vq::M_EUCLID); break;
+    default: BIG(vq::M_COS); break;
+    }
+#undef BIG
     return VQ_OK;
 }
 
-// Blocks of 8 floats, or of a width that an encode pads to 8 (a slice of rows at a time).  *done: it ran.
-int32_t assign_big8(vq_ctx *ctx, int metric, const float *d_x, int64_t n, int64_t ld, int m, int sd, int k,
-                    const float *d_codebooks, uint16_t *d_codes, bool *done) {
+// Blocks of 8 or 16 floats, or of a width that an encode pads to one of them (a slice of rows at a time).  *done: it ran.
+int32_t assign_big(vq_ctx *ctx, int metric, const float *d_x, int64_t n, int64_t ld, int m, int sd, int k,
+                   const float *d_codebooks, uint16_t *d_codes, bool *done) {
     *done = false;
-    if (ctx->assign_path == 1 || k > vq::kBig8Max || sd > 8 || metric == VQ_MANHATTAN) return VQ_OK;
-    if (sd == 8) {
-        // float4 centroid loads; 32 rows within 32-bit byte offsets
-        if ((reinterpret_cast<uintptr_t>(d_codebooks) & 15) != 0 || ld > (1 << 20)) return VQ_OK;
+    if (ctx->assign_path == 1 || sd > 16 || metric == VQ_MANHATTAN) return VQ_OK;
+    auto fits = [&](int w) { return w == 8 ? k <= vq::kBig8Max : w == 16 && k <= vq::kLds16Max; };
+    // float4 centroid loads; 32 rows within 32-bit byte offsets
+    if (fits(sd) && (reinterpret_cast<uintptr_t>(d_codebooks) & 15) == 0 && ld <= (1 << 20)) {
         *done = true;
-        return launch_big8(ctx, metric, d_x, n, ld, m, k, d_codebooks, d_codes);
+        return launch_big(ctx, metric, d_x, n, ld, m, sd, k, d_codebooks, d_codes);
     }
-    if (encode_pad_width(ctx, metric, d_x, n, ld, m, sd, vq::kChunk, d_codebooks) != 8) return VQ_OK;
+    const int sdp = encode_pad_width(ctx, metric, d_x, n, ld, m, sd, vq::kChunk, d_codebooks);
+    if (!fits(sdp)) return VQ_OK;
     *done = true;
-    const int64_t row_bytes = (int64_t)sizeof(float) * m * 8;
+    const int64_t row_bytes = (int64_t)sizeof(float) * m * sdp;
     const int64_t slice = std::min<int64_t>(n, std::max<int64_t>(4096, kPadSlice / row_bytes / 4096 * 4096));
     VQ_TRY(ensure(ctx, ctx->pad_x, (size_t)(slice * row_bytes)));
-    VQ_TRY(ensure(ctx, ctx->pad_cb, sizeof(float) * (size_t)m * k * 8));
+    VQ_TRY(ensure(ctx, ctx->pad_cb, sizeof(float) * (size_t)m * k * sdp));
     float *px = (float *)ctx->pad_x.p, *pcb = (float *)ctx->pad_cb.p;
-    pad_blocks(ctx, d_codebooks, (int64_t)m * k, sd, 1, sd, 8, pcb);
+    pad_blocks(ctx, d_codebooks, (int64_t)m * k, sd, 1, sd, sdp, pcb);
     for (int64_t r0 = 0; r0 < n; r0 += slice) {
         const int64_t rows = std::min(slice, n - r0);
-        pad_blocks(ctx, d_x + r0 * ld, rows, ld, m, sd, 8, px);
-        VQ_TRY(launch_big8(ctx, metric, px, rows, (int64_t)m * 8, m, k, pcb, d_codes + r0 * m));
+        pad_blocks(ctx, d_x + r0 * ld, rows, ld, m, sd, sdp, px);
+        VQ_TRY(launch_big(ctx, metric, px, rows, (int64_t)m * sdp, m, sdp, k, pcb, d_codes + r0 * m));
     }
     VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;
@@ -107,7 +109,7 @@ int32_t assign_codes_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t 
         return VQ_OK;
     }
     bool done = false;
-    VQ_TRY(assign_big8(ctx, metric, d_x, n, ld, m, sd, k, d_codebooks, d_codes, &done));
+    VQ_TRY(assign_big(ctx, metric, d_x, n, ld, m, sd, k, d_codebooks, d_codes, &done));
     if (done) return VQ_OK;
     // The rows in slices of up to kSlicePairs (row, block) pairs: the chunks that one launch merges have their
     // winners and distances side by side, 24 bytes per pair for four and the running minimum, and the
