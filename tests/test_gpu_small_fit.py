@@ -46,3 +46,26 @@ def test_small_fit(ctx, n, m, sd, k, iters, kind):
     ref = O.pq_fit(x, m, k, iters, init, reseed)
     assert np.array_equal(dcb.download().view(np.uint32), ref["codebooks"].view(np.uint32))
     assert np.array_equal(it, ref["iters"]) and np.array_equal(used, ref["reseeds"])
+
+
+@pytest.mark.parametrize("sd,m,largest", [(8, 32, 3000), (8, 32, 9000), (16, 16, 5000), (16, 16, 9000), (4, 64, 3000),
+                                          (12, 16, 5000), (32, 12, 1025), (1028, 2, 1030)])
+def test_small_fit_cluster_sizes(ctx, sd, m, largest):
+    """Clusters of every size around the batches of eight members, of 1024 and 1025 (the order of summation
+    changes) and above 8192 rows in one workgroup's list (its sizes are not known when the sums begin), several
+    in a workgroup (m * k > 256) and at different places of it (a block's clusters are one further on)."""
+    rng = np.random.default_rng(sd + largest)
+    k = 64 if sd < 1024 else 140
+    sizes = [1, 2, 7, 8, 9, 15, 16, 17, 23, 24, 25, 31, 32, 33, 39, 40, 41, 1023, 1024, 1025, largest]
+    sizes += [200 if sd < 1024 else 90] * (k - len(sizes))
+    label = rng.permutation(np.repeat(np.arange(k), sizes))
+    n = len(label)
+    x = (50.0 * label[:, None] + rng.random((n, m * sd))).astype(F)
+    first = np.array([int(np.flatnonzero(label == j)[0]) for j in range(k)])
+    init = np.stack([first[(np.arange(k) + s) % k] for s in range(m)]).astype(np.uint32)
+    reseed = np.zeros((m, k), np.uint32)
+    want = O.pq_fit(x, m, k, 2, init, reseed)
+    dcb = ctx.empty((m, k, sd), F)
+    it, used = ctx.lbg_fit(ctx.to_device(x), n, m * sd, m, sd, k, 2, init, reseed, dcb)
+    assert want["rc"] == 0 and np.array_equal(it, want["iters"]) and np.array_equal(used, want["reseeds"])
+    assert np.array_equal(dcb.download().view(np.uint32), want["codebooks"].view(np.uint32))

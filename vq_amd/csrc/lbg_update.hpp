@@ -750,11 +750,11 @@ static __global__ void __launch_bounds__(256) k_lbg_finalize(LbgState st, const 
 // ---- the whole update of a small fit in one launch ------------------------------------------------
 // Below some ten thousand rows every kernel of the path above is a handful of waves and the update is
 // a chain of launches and memory round trips: 75 us per iteration at 10,000 x 128, m = 16, k = 256 (the
-// streaming kernel's 12 workgroups 47 of them), 11 us here; 29 us at 50,000 rows.  Here a workgroup owns C clusters of one column block:
+// streaming kernel's 12 workgroups 47 of them), 9.8 us here; 30 us at 50,000 rows.  Here a workgroup owns C clusters of one column block:
 // it reads all codes of the block, lists the rows of its own clusters in row order, sorts a window of
 // the list by cluster (a stable counting sort by ballots), brings the window's sub-vectors into LDS
 // (every load of up to 8192 floats in flight together), and one lane per (cluster, component) adds
-// them in list order, eight LDS reads ahead.  The orders of summation are those above: row order up
+// them in list order (add_members).  The orders of summation are those above: row order up
 // to 1024 members, part sums in part order above.
 // DEFER: clusters above 1024 members are counted and left to k_lbg_large.
 // STAGED: sub_dim a multiple of 4 up to 512, a thread per component.  Else (wider blocks) a wave takes
@@ -816,12 +816,103 @@ static __global__ void __launch_bounds__(256) k_lbg_small_report(const int *__re
     for (int i = threadIdx.x; i < count; i += 256) out[i] = flags[i];
 }
 
-template <bool STAGED, bool DEFER = false>
+// Which sums of a cluster's members are kept: in row order; by parts for the clusters above 1024 members;
+// or both, while the sizes are not known yet.
+enum { kRows, kParts, kBoth };
+
+// The members at positions i .. hi - 1 of the stage d[position][sd], rows in `row`, onto one (cluster,
+// component)'s sums: `part`, or (closed parts `total`, open part `part`) where `big`, a part closing where
+// the row leaves it; kBoth: and `seq` in row order.  One chain of additions bounds a stage, that of its
+// largest cluster: the next eight values are read while eight are added, at offsets that the instruction
+// holds where sd is known (SD of k_lbg_update_small).  A member took 12 ns with one batch at a time,
+// computed offsets and both sums in every cluster; with this, and the codes of three steps in flight instead
+// of one, the first update of 60,007 rows, m = 10, k = 200, blocks of 16, whose clusters are uneven, went from
+// 72.8 to 46.7 us (12.7 the list, 5 the sort, 12 the rows, 16 the sums), 60,000 rows, m = 32, blocks of 4, from
+// 79.0 to 66.2, m = 4, blocks of 32, from 83.7 to 65.7.
+template <int SUMS>
+__device__ __forceinline__ void add_members(const float *d, int sd, const uint32_t *row, uint32_t i, uint32_t hi, bool big,
+                                            float &seq, float &total, float &part, uint32_t &open) {
+    constexpr int B = 8;
+    auto load = [&](float (&t)[B], uint32_t &last, uint32_t at) {
+        const float *b = d + at * (uint32_t)sd;
+#pragma unroll
+        for (int u = 0; u < B; ++u) t[u] = b[u * sd];
+        if constexpr (SUMS != kRows) last = row[at + B - 1] / (uint32_t)kPartRows;
+    };
+    auto add_one = [&](float v, uint32_t r) {
+        const uint32_t p = big ? r / (uint32_t)kPartRows : open;
+        const bool close = p != open;
+        const float closed = total + part;
+        total = close ? closed : total;
+        part = close ? 0.0f : part;
+        open = p;
+        part = part + v;
+        if constexpr (SUMS == kBoth) seq = seq + v;
+    };
+    auto add = [&](const float (&t)[B], uint32_t last, uint32_t at) {
+        // (rows ascend: the last one in the open part means all eight)
+        if (SUMS != kRows && big && last != open) {
+#pragma unroll
+            for (int u = 0; u < B; ++u) add_one(t[u], row[at + u]);
+        } else {
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                part = part + t[u];
+                if constexpr (SUMS == kBoth) seq = seq + t[u];
+            }
+        }
+    };
+    float t[B], q[B];
+    uint32_t last_t = 0, last_q = 0;
+    if (i + B <= hi) {
+        load(t, last_t, i);
+        for (; i + 3 * B <= hi; i += 2 * B) {
+            load(q, last_q, i + B);
+            add(t, last_t, i);
+            load(t, last_t, i + 2 * B);
+            add(q, last_q, i + B);
+        }
+        if (i + 2 * B <= hi) {
+            load(q, last_q, i + B);
+            add(t, last_t, i);
+            i += B;
+            add(q, last_q, i);
+        } else {
+            add(t, last_t, i);
+        }
+        i += B;
+    }
+    if (i >= hi) return;
+#pragma unroll
+    for (int u = 0; u < B; ++u) t[u] = d[(i + u < hi ? i + u : hi - 1) * (uint32_t)sd];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+        if constexpr (SUMS == kRows) part = part + (i + u < hi ? t[u] : -0.0f);  // (a + -0 is a)
+        else if (i + u < hi) add_one(t[u], row[i + u]);
+    }
+}
+
+// The sum of v over the lanes up to this one.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
+    auto up = [&](auto ctrl, auto rows) {
+        v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    };
+    up(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});  // inside rows of 16 lanes
+    up(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    up(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+    up(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    up(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // lane 15 of a row to the odd row after it
+    up(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // lane 31 to the upper half
+    return v;
+}
+
+template <bool STAGED, bool DEFER = false, int SD = 0>
 static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSmall st, int it, int m,
                                                                            const float *__restrict__ x, int64_t n,
-                                                                           int64_t ld, int sd, int k, int C, int groups,
-                                                                           const uint32_t *__restrict__ reseed,
+                                                                           int64_t ld, int sub_dim, int k, int C,
+                                                                           int groups, const uint32_t *__restrict__ reseed,
                                                                            int n_reseed, float *__restrict__ cb) {
+    const int sd = SD ? SD : sub_dim;
     const unsigned id = xcd_contiguous(blockIdx.x, gridDim.x);
     const int s = (int)(id / (unsigned)groups), j0 = (int)(id % (unsigned)groups) * C;
     if (st.changed[it * m + s] == 0) return;  // converged before this iteration
@@ -850,7 +941,9 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
     uint32_t cur_part = 0;
     const int my_c = STAGED ? tid / sd : 0, my_t = STAGED ? tid % sd : 0;
     const bool summing = STAGED && my_c < jn;
-    bool track = false, drained = false;  // uniform; track: the part sums are needed as well
+    int track = kRows;  // uniform
+    bool drained = false;  // uniform
+    bool big = false;  // STAGED: this thread's cluster is above 1024 members
     uint32_t cnt = 0;                     // entries of list, uniform
 
     // one member's value into (row-order sum; closed parts, open part)
@@ -942,35 +1035,9 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
                         uint32_t i = c_lo > p0 ? c_lo - p0 : 0u;
                         const uint32_t end = c_hi > p0 ? c_hi - p0 : 0u, hi = end < pn ? end : pn;
                         const float *d = dyn + my_t;
-                        if (track) {
-                            for (; i + 8 <= hi; i += 8) {
-                                float t[8];
-#pragma unroll
-                                for (int u = 0; u < 8; ++u) t[u] = d[(i + u) * (uint32_t)sd];
-                                // (rows ascend: the last one in the open part means all eight)
-                                if (sorted[p0 + i + 7] / (uint32_t)kPartRows == cur_part) {
-#pragma unroll
-                                    for (int u = 0; u < 8; ++u) {
-                                        seq = seq + t[u];
-                                        part = part + t[u];
-                                    }
-                                } else {
-#pragma unroll
-                                    for (int u = 0; u < 8; ++u)
-                                        add_tracked(t[u], sorted[p0 + i + u], seq, total, part, cur_part);
-                                }
-                            }
-                            for (; i < hi; ++i) add_tracked(d[i * (uint32_t)sd], sorted[p0 + i], seq, total, part, cur_part);
-                        } else {
-                            for (; i + 8 <= hi; i += 8) {
-                                float t[8];
-#pragma unroll
-                                for (int u = 0; u < 8; ++u) t[u] = d[(i + u) * (uint32_t)sd];
-#pragma unroll
-                                for (int u = 0; u < 8; ++u) seq = seq + t[u];
-                            }
-                            for (; i < hi; ++i) seq = seq + d[i * (uint32_t)sd];
-                        }
+                        if (track == kBoth) add_members<kBoth>(d, sd, sorted + p0, i, hi, true, seq, total, part, cur_part);
+                        else if (track == kParts) add_members<kParts>(d, sd, sorted + p0, i, hi, big, seq, total, part, cur_part);
+                        else add_members<kRows>(d, sd, sorted + p0, i, hi, false, seq, total, part, cur_part);
                     }
                     __syncthreads();
                 }
@@ -994,7 +1061,7 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
 #pragma unroll
                         for (int u = 0; u < B; ++u)
                             if (i + u < hi) {
-                                if (track) add_tracked(v[u], r[u], a, tt, pp, open);
+                                if (track != kRows) add_tracked(v[u], r[u], a, tt, pp, open);
                                 else a = a + v[u];
                             }
                     }
@@ -1042,18 +1109,27 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
         const uint32_t w = u < 8u ? (u < 4u ? v[0] : v[1]) : (u < 12u ? v[2] : v[3]);
         return ((w >> (8u * (u & 3u))) & 0xffu) - (uint32_t)j0;
     };
-    uint32_t have_next;
-    codes16 next = fetch(16 * tid, have_next);
+    uint32_t have_next, have_2, have_3;
+    codes16 next = fetch(16 * tid, have_next), next2 = fetch(kStep + 16 * tid, have_2), next3 = fetch(2 * kStep + 16 * tid, have_3);
+    // the step that is next now; the one three steps on (from step p) into flight
+    auto advance = [&](int64_t p) {
+        next = next2;
+        have_next = have_2;
+        next2 = next3;
+        have_2 = have_3;
+        next3 = fetch((p + 3) * kStep + 16 * tid, have_3);
+    };
     uint32_t large = 0;  // (DEFER) bit c: cluster j0 + c is not summed here, uniform
     if constexpr (DEFER) {
         __syncthreads();
         for (int p = 0; p < nsteps; ++p) {
             const codes16 v = next;
             uint32_t mine = own_rows(v) & have_next;
-            next = fetch((int64_t)(p + 1 < nsteps ? p + 1 : 0) * kStep + 16 * tid, have_next);  // (then the first step again)
+            advance(p);
             for (; mine; mine &= mine - 1) atomicAdd(&cl_cnt[cluster_of(v, (uint32_t)__ffs(mine) - 1u)], 1u);
         }
         __syncthreads();
+        for (int p = -3; p < 0; ++p) advance(p);  // the first steps again
         for (int c = 0; c < jn; ++c) large |= (cl_cnt[c] > (uint32_t)kSeqMax ? 1u : 0u) << c;
         large = __builtin_amdgcn_readfirstlane(large);
         if (tid < jn && ((large >> tid) & 1u))
@@ -1063,18 +1139,13 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
         const uint32_t row0 = (uint32_t)p * (uint32_t)kStep + 16u * tid;
         const codes16 v = next;
         const uint32_t have = have_next;
-        next = fetch((int64_t)row0 + kStep, have_next);
+        advance(p);
         uint32_t mine = own_rows(v) & have;
         if (DEFER && large)
             for (uint32_t mm = mine; mm; mm &= mm - 1)
                 if ((large >> cluster_of(v, (uint32_t)__ffs(mm) - 1u)) & 1u) mine &= ~(mm & (0u - mm));
         const uint32_t m1 = __popc(mine);
-        uint32_t inc = m1;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t o = __shfl_up(inc, off);
-            if (lane >= off) inc += o;
-        }
+        const uint32_t inc = wave_prefix(m1);
         if (lane == 63) wave_tot[p & 1][wave] = inc;
         __syncthreads();
         uint32_t before = 0, all = 0;
@@ -1085,7 +1156,7 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
             all += t;
         }
         if (cnt + all > (uint32_t)kSmallList) {  // the sizes of the clusters are not known yet: keep both sums
-            track = !DEFER;
+            track = DEFER ? kRows : kBoth;
             drain();
         }
         uint32_t at = cnt + before + inc - m1;
@@ -1099,7 +1170,8 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
     }
     __syncthreads();
     if (!DEFER && !drained) {
-        for (int c = 0; c < jn; ++c) track = track || cl_cnt[c] > (uint32_t)kSeqMax;
+        for (int c = 0; c < jn; ++c) track = cl_cnt[c] > (uint32_t)kSeqMax ? (STAGED ? kParts : kBoth) : track;
+        big = summing && cl_cnt[my_c] > (uint32_t)kSeqMax;
     }
     drain();
     float *out = cb + ((size_t)s * k + j0) * sd;
@@ -1107,7 +1179,8 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
         if (summing) {
             const uint32_t cm = cl_cnt[my_c];
             if (cm && !((large >> my_c) & 1u))
-                out[my_c * sd + my_t] = (cm <= (uint32_t)kSeqMax ? seq : total + part) / __uint2float_rn(cm);
+                out[my_c * sd + my_t] =
+                    (cm > (uint32_t)kSeqMax ? total + part : (track == kBoth ? seq : part)) / __uint2float_rn(cm);
         }
     } else {
         for (int i = tid; i < jn * sd; i += kSmallThreads) {

@@ -1320,6 +1320,8 @@ static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
     const int groups = (int)cdiv(k, C);
     if (staged && !ctx->lbg_small_lds_set) {
         const void *kerns[] = {reinterpret_cast<const void *>(vq::k_lbg_update_small<true>),
+                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, false, 8>),
+                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, false, 16>),
                                reinterpret_cast<const void *>(vq::k_lbg_update_small<true, true>),
                                reinterpret_cast<const void *>(vq::k_lbg_large)};
         for (const void *kern : kerns)
@@ -1344,7 +1346,10 @@ static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
             hipLaunchKernelGGL(vq::k_lbg_large, dim3(nparts, std::min(most_large, 16)), dim3(vq::kSmallThreads),
                                sizeof(float) * vq::kSmallStage, st, S, it, d_x, n, ld, sd, k, d_codebooks);
         } else if (staged)
-            hipLaunchKernelGGL(vq::k_lbg_update_small<true>, dim3(groups * m), dim3(vq::kSmallThreads),
+            hipLaunchKernelGGL((sd == 8    ? vq::k_lbg_update_small<true, false, 8>
+                                : sd == 16 ? vq::k_lbg_update_small<true, false, 16>
+                                           : vq::k_lbg_update_small<true>),
+                               dim3(groups * m), dim3(vq::kSmallThreads),
                                sizeof(float) * vq::kSmallStage, st, S, it, m, d_x, n, ld, sd, k, C, groups,
                                (const uint32_t *)reseed, n_reseed, d_codebooks);
         else
