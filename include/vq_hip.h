@@ -342,6 +342,11 @@ int32_t vq_cross_cov(vq_ctx *ctx, const float *d_y, const float *d_x, int64_t n,
  * The result is a tolerance quantity (the reference's nalgebra SVD is not restated): both ways
  * agree to about 1e-10 for condition numbers up to 1e6.  Synchronises. */
 int32_t vq_procrustes_rotation(vq_ctx *ctx, const double *h_A, int32_t dim, double *h_R);
+/* d_R = the rotation update of one outer iteration (src/opq.rs:172-183), f32 on the device:
+ * vq_cross_cov, its result rounded to f32, and vq_procrustes_rotation, without A and R going through host
+ * memory while the Newton-Schulz steps take A (both norms and the start are made by kernels; the result is
+ * the same to rounding).  Synchronises. */
+int32_t vq_opq_rotation(vq_ctx *ctx, const float *d_y, const float *d_x, int64_t n, int32_t dim, float *d_R);
 /* 0 (default): as above; 1: the SVD only.  The switch exists for measurement and tests.  No
  * counterpart in the reference. */
 int32_t vq_ctx_set_procrustes_path(vq_ctx *ctx, int32_t path);

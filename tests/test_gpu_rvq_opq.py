@@ -336,6 +336,42 @@ def test_procrustes_rotation_of_a_singular_matrix_is_orthogonal(ctx, dim, rank):
         assert abs(np.trace(P) - np.linalg.svd(M, compute_uv=False).sum()) <= 1e-9 * np.abs(P).sum()
 
 
+@pytest.mark.parametrize("dim", [1, 2, 10, 15, 16, 17, 64, 100, 128, 130, 256, 271, 512])
+def test_opq_rotation_is_the_update_of_the_rounded_cross_covariance(ctx, dim):
+    """The update that stays on the device against the one through host memory: both are the polar factor of
+    the same f32 matrix to about 1e-11 (its condition number is below 1e4), then rounded to f32: an ulp of a
+    value up to 1, 6e-8.  A zero matrix leaves the steps at once and takes the SVD, which completes it to the
+    identity; so does the switch that allows the SVD only."""
+    rng = np.random.default_rng(dim)
+    n = 600
+    x = rng.standard_normal((n, dim)).astype(F)
+    y = (x + 0.3 * rng.standard_normal((n, dim))).astype(F)
+    dx, dy, dR = ctx.to_device(x), ctx.to_device(y), ctx.empty((dim, dim), F)
+    want = ctx.procrustes_rotation(ctx.cross_cov(dy, dx, n, dim).astype(F).astype(np.float64)).astype(F)
+    ctx.opq_rotation(dy, dx, n, dim, dR)
+    got = dR.download()
+    assert np.abs(got - want).max() <= 6e-8
+    ctx.opq_rotation(dy, dx, n, dim, dR)
+    assert np.array_equal(got, dR.download())  # deterministic
+    if dim <= 128:
+        ctx.opq_rotation(ctx.to_device(np.zeros((n, dim), F)), dx, n, dim, dR)
+        assert np.array_equal(dR.download(), np.eye(dim, dtype=F))
+        ctx.set_procrustes_path(1)
+        ctx.opq_rotation(dy, dx, n, dim, dR)
+        ctx.set_procrustes_path(0)
+        assert np.abs(dR.download() - want).max() <= 6e-8
+
+
+def test_opq_rotation_refuses_what_cross_cov_refuses(ctx):
+    d = ctx.to_device(np.zeros((4, 4), F))
+    for n, dim in ((0, 4), (4, 0), (4, 4097)):
+        with pytest.raises(Exception) as a:
+            ctx.cross_cov(d, d, n, dim)
+        with pytest.raises(Exception) as b:
+            ctx.opq_rotation(d, d, n, dim, d)
+        assert str(a.value) == str(b.value)
+
+
 @pytest.mark.parametrize("dim", [3, 9, 130, 200])
 def test_procrustes_rotation_sizes_outside_the_device_kernel(ctx, dim):
     rng = np.random.default_rng(dim)

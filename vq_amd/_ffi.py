@@ -67,6 +67,7 @@ SYMBOLS = {
                              _vp]),
     "vq_rotate": (_i32, [_vp, _vp, _i64, _i64, _i32, _vp, _vp]),
     "vq_cross_cov": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp]),
+    "vq_opq_rotation": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp]),
     "vq_tsvq_build": (_i32, [_vp, _vp, _i64, _i64, _i32, _i32, C.POINTER(_vp)]),
     "vq_tsvq_build_kmeans": (_i32, [_vp, _vp, _i64, _i64, _i32, _i32, _i32, _vp, _i32, C.POINTER(_vp)]),
     "vq_tree_create": (_i32, [_vp, _i32, _i32, _vp, _vp, _vp, C.POINTER(_vp)]),
@@ -395,6 +396,9 @@ class Context:
         A = np.empty((dim, dim), np.float64)
         self._check(_lib.vq_cross_cov(self._h, d_y.ptr, d_x.ptr, n, dim, A.ctypes.data))
         return A
+
+    def opq_rotation(self, d_y, d_x, n, dim, d_R):
+        self._check(_lib.vq_opq_rotation(self._h, d_y.ptr, d_x.ptr, n, dim, d_R.ptr))
 
     def set_tsvq_descend_path(self, path):
         """0: one inner product per node where it decides (default); 1: two distances per node always."""

@@ -154,4 +154,124 @@ static __global__ void __launch_bounds__(512) k_polar_step(const double *__restr
     }
 }
 
+// ---- the start and the end of the iteration on the device ------------------------------------------
+// A stays where the cross-covariance left it; the elements are rounded to f32 first (the reference's A is
+// a matrix of f32).  On the host the two norms, the transposed copy and the way there and back took 220 us of
+// a rotation update at 128 dimensions, the steps themselves 190.
+
+// The step tables of one iteration.
+struct PolarTables {
+    unsigned long long *errs;  // [kPolarMaxSteps]
+    int *fin;                  // [kPolarMaxSteps + 2]
+    int *bad;                  // A is zero or not finite: the steps return at once
+};
+
+__device__ __forceinline__ double polar_in(const double *A, size_t e) { return (double)(float)A[e]; }
+
+// Workgroup b: of rows 16 b .. 16 b + 15, the sums of |a| by column (col_part[b][dim]) and by row, and the
+// rows' sums of squares.  256 threads.
+static __global__ void __launch_bounds__(256) k_polar_norms(const double *__restrict__ A, int dim,
+                                                            double *__restrict__ col_part, double *__restrict__ row_sum,
+                                                            double *__restrict__ row_sq) {
+    const int i0 = 16 * blockIdx.x, rows = dim - i0 < 16 ? dim - i0 : 16;
+    for (int j = threadIdx.x; j < dim; j += 256) {
+        double v[16], c = 0.0;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = polar_in(A, (size_t)(i0 + (u < rows ? u : 0)) * dim + j);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) c += u < rows ? fabs(v[u]) : 0.0;
+        col_part[(size_t)blockIdx.x * dim + j] = c;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int u = wave; u < rows; u += 4) {
+        double a = 0.0, q = 0.0;
+        for (int j = lane; j < dim; j += 64) {
+            const double v = polar_in(A, (size_t)(i0 + u) * dim + j);
+            a += fabs(v);
+            q += v * v;
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            a += __shfl_xor(a, off);
+            q += __shfl_xor(q, off);
+        }
+        if (lane == 0) {
+            row_sum[i0 + u] = a;
+            row_sq[i0 + u] = q;
+        }
+    }
+}
+
+// X = A^T / scale, P x P, zero beyond dim, and cleared tables.  P / 16 workgroups of 256 threads, each with
+// its own copy of the scale.
+static __global__ void __launch_bounds__(256) k_polar_start(const double *__restrict__ A, int dim, int P,
+                                                            const double *__restrict__ col_part,
+                                                            const double *__restrict__ row_sum,
+                                                            const double *__restrict__ row_sq, PolarTables tb,
+                                                            double *__restrict__ X) {
+    __shared__ double red[3][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, strips = (dim + 15) / 16;
+    double n1 = 0.0, ni = 0.0, fro = 0.0;
+    for (int j = tid; j < dim; j += 256) {
+        double c = 0.0;
+        for (int b = 0; b < strips; ++b) c += col_part[(size_t)b * dim + j];
+        n1 = fmax(n1, c);
+        ni = fmax(ni, row_sum[j]);
+        fro += row_sq[j];  // (a NaN stays in this one)
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        n1 = fmax(n1, __shfl_xor(n1, off));
+        ni = fmax(ni, __shfl_xor(ni, off));
+        fro += __shfl_xor(fro, off);
+    }
+    if (lane == 0) {
+        red[0][wave] = n1;
+        red[1][wave] = ni;
+        red[2][wave] = fro;
+    }
+    __syncthreads();
+    n1 = fmax(fmax(red[0][0], red[0][1]), fmax(red[0][2], red[0][3]));
+    ni = fmax(fmax(red[1][0], red[1][1]), fmax(red[1][2], red[1][3]));
+    fro = (red[2][0] + red[2][1]) + (red[2][2] + red[2][3]);
+    // two upper bounds of the largest singular value; the smaller one
+    const double by_sums = sqrt(n1) * sqrt(ni), by_squares = sqrt(fro);
+    const double scale = by_sums < by_squares ? by_sums : by_squares;
+    const bool ok = scale > 0.0 && scale < __builtin_inf();
+    if (blockIdx.x == 0) {
+        if (tid < kPolarMaxSteps) tb.errs[tid] = 0ull;
+        if (tid < kPolarMaxSteps + 2) tb.fin[tid] = tid == 0 && !ok ? 1 : 0;
+        if (tid == 0) tb.bad[0] = ok ? 0 : 1;
+    }
+    const double inv = ok ? 1.0 / scale : 0.0;
+    const int i0 = 16 * blockIdx.x;
+    for (int j = tid; j < P; j += 256) {
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const bool in = i0 + u < dim && j < dim;
+            v[u] = polar_in(A, in ? (size_t)(i0 + u) * dim + j : 0);
+            v[u] = in && ok ? v[u] * inv : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) X[(size_t)j * P + i0 + u] = v[u];
+    }
+}
+
+// After `steps` steps: R = the iterate behind the first step whose error was below kPolarLastStepErr, in
+// f32, and status 1; 0 where there is none yet, -1 where the iteration could not begin.
+static __global__ void __launch_bounds__(256) k_polar_finish(const double *__restrict__ X0, const double *__restrict__ X1,
+                                                             int P, int dim, PolarTables tb, int steps,
+                                                             float *__restrict__ R, int *status) {
+    int last = -1;
+    for (int t = steps - 1; t >= 0; --t)
+        if (__longlong_as_double((long long)tb.errs[t]) < kPolarLastStepErr) last = t;
+    const bool bad = tb.bad[0] != 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *status = bad ? -1 : (last >= 0 ? 1 : 0);
+    if (bad || last < 0) return;
+    const double *X = (last + 1) & 1 ? X1 : X0;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < dim * dim; e += gridDim.x * 256)
+        R[e] = (float)X[(size_t)(e / dim) * P + e % dim];
+}
+
 }  // namespace vq

@@ -166,6 +166,29 @@ int32_t rvq_encode(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int
 
 namespace {
 
+// Enqueues the steps from .. upto - 1 of the iteration in X[0], X[1] (polar.hpp).  low: the assumed lower
+// bound of the singular values, 1e-3 before step 0.
+int32_t polar_steps(vq_ctx *ctx, double *const (&X)[2], int dim, int from, int upto, double &low, unsigned long long *errs,
+                    int *fin) {
+    const int P = (dim + 15) / 16 * 16;
+    const unsigned strips = (unsigned)(P / 16), waves = strips < 8u ? strips : 8u;
+    const size_t lds = sizeof(double) * 16 * (size_t)P;
+    if (lds > 48 * 1024)
+        VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_polar_step<0>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    for (int s = from; s < upto; ++s) {
+        double rho = 1.0;
+        if (s > 0 && low < 0.9) {
+            rho = std::sqrt(3.0 / (1.0 + low + low * low));
+            low = rho * low * (3.0 - rho * rho * low * low) * 0.5;
+        }
+        hipLaunchKernelGGL((P == 128 ? vq::k_polar_step<8> : vq::k_polar_step<0>), dim3(strips), dim3(64 * waves), lds,
+                           ctx->stream, (const double *)X[s & 1], P, dim, s, rho, errs, fin, X[(s + 1) & 1]);
+    }
+    VQ_HIP(ctx, hipGetLastError());
+    return VQ_OK;
+}
+
 // R = the orthogonal polar factor of A^T by Newton-Schulz steps (polar.hpp).  *done = false when the
 // iteration has not converged within its step limit (the caller then takes the SVD).
 int32_t polar_newton_schulz(vq_ctx *ctx, const double *h_A, int dim, double *h_R, bool *done) {
@@ -207,30 +230,13 @@ int32_t polar_newton_schulz(vq_ctx *ctx, const double *h_A, int dim, double *h_R
     hipStream_t st = ctx->stream;
     VQ_HIP(ctx, hipMemsetAsync(ctx->tmp_f.p, 0, 1024, st));
     VQ_HIP(ctx, hipMemcpyAsync(X[0], x0.data(), sizeof(double) * total, hipMemcpyHostToDevice, st));
-    const unsigned strips = (unsigned)(P / 16), waves = strips < 8u ? strips : 8u;
-    const size_t lds = sizeof(double) * 16 * (size_t)P;
-    if (lds > 48 * 1024)
-        VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_polar_step<0>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     unsigned long long h_errs[vq::kPolarMaxSteps];
     int s = 0, last = -1;
-    double low = 1e-3;  // assumed lower bound of the singular values after the first (plain) step
+    double low = 1e-3;
     while (s < vq::kPolarMaxSteps && last < 0) {
         const int upto = std::min(vq::kPolarMaxSteps, s == 0 ? 16 : s + 6);
-        for (; s < upto; ++s) {
-            double rho = 1.0;
-            if (s > 0 && low < 0.9) {
-                rho = std::sqrt(3.0 / (1.0 + low + low * low));
-                low = rho * low * (3.0 - rho * rho * low * low) * 0.5;
-            }
-            if (P == 128)
-                hipLaunchKernelGGL(vq::k_polar_step<8>, dim3(strips), dim3(64 * waves), lds, st,
-                                   (const double *)X[s & 1], P, dim, s, rho, errs, fin, X[(s + 1) & 1]);
-            else
-                hipLaunchKernelGGL(vq::k_polar_step<0>, dim3(strips), dim3(64 * waves), lds, st,
-                                   (const double *)X[s & 1], P, dim, s, rho, errs, fin, X[(s + 1) & 1]);
-        }
-        VQ_HIP(ctx, hipGetLastError());
+        VQ_TRY(polar_steps(ctx, X, dim, s, upto, low, errs, fin));
+        s = upto;
         VQ_HIP(ctx, hipMemcpyAsync(h_errs, errs, sizeof(unsigned long long) * s, hipMemcpyDeviceToHost, st));
         VQ_HIP(ctx, hipStreamSynchronize(st));
         for (int t = 0; t < s && last < 0; ++t) {
@@ -246,6 +252,105 @@ int32_t polar_newton_schulz(vq_ctx *ctx, const double *h_A, int dim, double *h_R
     for (int i = 0; i < dim; ++i)
         for (int j = 0; j < dim; ++j) h_R[(size_t)i * dim + j] = r[(size_t)i * P + j];
     *done = true;
+    return VQ_OK;
+}
+
+// R = V U^T of the one-sided Jacobi SVD: on the device for even dim up to kJacobiMax, else on the host.
+int32_t procrustes_svd(vq_ctx *ctx, const double *h_A, int dim, double *h_R) {
+    if (dim > vq::kJacobiMax || dim % 2 != 0) {
+        vqh::procrustes_host(h_A, (size_t)dim, h_R);
+        return VQ_OK;
+    }
+    const size_t total = (size_t)dim * dim;
+    const int half = dim / 2;
+    VQ_TRY(ensure(ctx, ctx->tmp_a, sizeof(double) * total));
+    VQ_TRY(ensure(ctx, ctx->tmp_b, sizeof(double) * total));
+    VQ_TRY(ensure(ctx, ctx->tmp_c, sizeof(double) * (total + dim)));
+    VQ_TRY(ensure(ctx, ctx->tmp_d, sizeof(double) * total));
+    VQ_TRY(ensure(ctx, ctx->tmp_e, sizeof(double2) * (size_t)vq::kJacobiSweeps * (dim - 1) * half));
+    VQ_TRY(ensure(ctx, ctx->tmp_f, 256));
+    double *d_A = (double *)ctx->tmp_a.p, *d_vt = (double *)ctx->tmp_b.p, *d_uhat = (double *)ctx->tmp_c.p;
+    double *d_sv = d_uhat + total;
+    double *d_out = (double *)ctx->tmp_d.p;
+    double2 *d_rot = (double2 *)ctx->tmp_e.p;
+    int *d_rounds = (int *)ctx->tmp_f.p;
+    VQ_HIP(ctx, hipMemcpyAsync(d_A, h_A, sizeof(double) * total, hipMemcpyHostToDevice, ctx->stream));
+    constexpr int kLanes = 8;
+    const size_t lds = sizeof(double) * (size_t)dim * vq::kJacobiStride;
+    VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_jacobi_sweeps<kLanes>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(vq::k_jacobi_sweeps<kLanes>, dim3(1), dim3(64 * kLanes), lds, ctx->stream, (const double *)d_A,
+                       dim, d_rot, d_rounds, d_uhat, d_sv);
+    hipLaunchKernelGGL(vq::k_jacobi_accumulate, dim3(dim), dim3(64), 0, ctx->stream, (const double2 *)d_rot,
+                       (const int *)d_rounds, dim, d_vt);
+    hipLaunchKernelGGL(vq::k_jacobi_product, dim3((unsigned)cdiv(total, 256)), dim3(256), 0, ctx->stream,
+                       (const double *)d_vt, (const double *)d_uhat, dim, d_out);
+    VQ_HIP(ctx, hipGetLastError());
+    std::vector<double> sv((size_t)dim);
+    VQ_HIP(ctx, hipMemcpyAsync(h_R, d_out, sizeof(double) * total, hipMemcpyDeviceToHost, ctx->stream));
+    VQ_HIP(ctx, hipMemcpyAsync(sv.data(), d_sv, sizeof(double) * dim, hipMemcpyDeviceToHost, ctx->stream));
+    VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    // A singular A leaves directions of U open (their columns came back as zero or as rounding
+    // noise): complete them on the host and form the product again.  Rare; a full-rank A ends here.
+    double top = 0.0;
+    for (double v : sv) top = std::max(top, v);
+    bool open = false;
+    for (double v : sv) open = open || !(top > 0.0 && v > vqh::kNullRel * top);
+    if (open) {
+        std::vector<double> Ut(total), Vt(total);
+        VQ_HIP(ctx, hipMemcpyAsync(Ut.data(), d_uhat, sizeof(double) * total, hipMemcpyDeviceToHost, ctx->stream));
+        VQ_HIP(ctx, hipMemcpyAsync(Vt.data(), d_vt, sizeof(double) * total, hipMemcpyDeviceToHost, ctx->stream));
+        VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        vqh::complete_null_columns(Ut, Vt, sv, (size_t)dim);
+        vqh::product_v_ut(Vt, Ut, (size_t)dim, h_R);
+    }
+    return VQ_OK;
+}
+
+// d_y^T d_x to tmp_b, dim x dim in f64.
+int32_t cross_cov_device(vq_ctx *ctx, const float *d_y, const float *d_x, int64_t n, int32_t dim) {
+    // chunks of 2048 rows up to dim 128; longer chunks for larger matrices, so that the partial
+    // sums (one dim x dim matrix per chunk) stay at about 64 B per row
+    const int64_t scale = ((int64_t)dim + 127) / 128;
+    // and shorter ones where that would leave fewer than 256 workgroups (a chunk has scale^2): 50,000 x 128
+    // was 25 workgroups and 265 us, now 34 us
+    const int64_t rows_per_chunk =
+        std::min<int64_t>(2048, std::max<int64_t>(128, (n / 256 + 3) / 4 * 4)) * scale * scale;
+    const int chunks = (int)cdiv(n, rows_per_chunk);
+    const int total = dim * dim;
+    VQ_TRY(ensure(ctx, ctx->tmp_a, sizeof(double) * (size_t)chunks * total));
+    VQ_TRY(ensure(ctx, ctx->tmp_b, sizeof(double) * (size_t)total));
+    VQ_TRY(ensure(ctx, ctx->tmp_c, sizeof(double) * (size_t)total * ((chunks + 31) / 32)));
+    if (dim % 16 == 0) {
+        const int nt_all = dim / 16, full = dim / 128, rest = nt_all % 8;
+        double *part = (double *)ctx->tmp_a.p;
+#define CROSSCOV(NT, B0, Z)                                                                                 \
+    hipLaunchKernelGGL((vq::k_crosscov_mfma<NT>), dim3(chunks, (nt_all + 7) / 8, Z), dim3(256), 0, ctx->stream, \
+                       d_y, d_x, n, dim, B0, rows_per_chunk, part)
+        if (full) CROSSCOV(8, 0, full);
+        switch (rest) {
+        case 1: CROSSCOV(1, 128 * full, 1); break;
+        case 2: CROSSCOV(2, 128 * full, 1); break;
+        case 3: CROSSCOV(3, 128 * full, 1); break;
+        case 4: CROSSCOV(4, 128 * full, 1); break;
+        case 5: CROSSCOV(5, 128 * full, 1); break;
+        case 6: CROSSCOV(6, 128 * full, 1); break;
+        case 7: CROSSCOV(7, 128 * full, 1); break;
+        default: break;
+        }
+#undef CROSSCOV
+    } else {
+        const int tiles = (dim + 127) / 128;
+        hipLaunchKernelGGL(vq::k_crosscov_partial, dim3(chunks, tiles * tiles), dim3(256), 0, ctx->stream, d_y, d_x,
+                           n, dim, rows_per_chunk, (double *)ctx->tmp_a.p);
+    }
+    // chunk sums in groups of 32 chunks, then the groups
+    const int per_group = 32, groups = (chunks + per_group - 1) / per_group;
+    hipLaunchKernelGGL(vq::k_crosscov_reduce, dim3(cdiv(total, 256), groups), dim3(256), 0, ctx->stream,
+                       (const double *)ctx->tmp_a.p, chunks, per_group, total, (double *)ctx->tmp_c.p);
+    hipLaunchKernelGGL(vq::k_crosscov_reduce, dim3(cdiv(total, 256), 1), dim3(256), 0, ctx->stream,
+                       (const double *)ctx->tmp_c.p, groups, groups, total, (double *)ctx->tmp_b.p);
+    VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;
 }
 
@@ -364,50 +469,64 @@ int32_t vq_cross_cov(vq_ctx *ctx, const float *d_y, const float *d_x, int64_t n,
     if (!d_y || !d_x || !h_A || n < 0 || dim <= 0) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
     if (dim > 4096) return fail(ctx, VQ_ERR_UNSUPPORTED, "cross-covariance: dim %d > 4096", dim);
     VQ_HIP(ctx, hipSetDevice(ctx->device));
-    // chunks of 2048 rows up to dim 128; longer chunks for larger matrices, so that the partial
-    // sums (one dim x dim matrix per chunk) stay at about 64 B per row
-    const int64_t scale = ((int64_t)dim + 127) / 128;
-    // and shorter ones where that would leave fewer than 256 workgroups (a chunk has scale^2): 50,000 x 128
-    // was 25 workgroups and 265 us, now 34 us
-    const int64_t rows_per_chunk =
-        std::min<int64_t>(2048, std::max<int64_t>(128, (n / 256 + 3) / 4 * 4)) * scale * scale;
-    const int chunks = (int)cdiv(n, rows_per_chunk);
-    const int total = dim * dim;
-    VQ_TRY(ensure(ctx, ctx->tmp_a, sizeof(double) * (size_t)chunks * total));
-    VQ_TRY(ensure(ctx, ctx->tmp_b, sizeof(double) * (size_t)total));
-    VQ_TRY(ensure(ctx, ctx->tmp_c, sizeof(double) * (size_t)total * ((chunks + 31) / 32)));
-    if (dim % 16 == 0) {
-        const int nt_all = dim / 16, full = dim / 128, rest = nt_all % 8;
-        double *part = (double *)ctx->tmp_a.p;
-#define CROSSCOV(NT, B0, Z)                                                                                 \
-    hipLaunchKernelGGL((vq::k_crosscov_mfma<NT>), dim3(chunks, (nt_all + 7) / 8, Z), dim3(256), 0, ctx->stream, \
-                       d_y, d_x, n, dim, B0, rows_per_chunk, part)
-        if (full) CROSSCOV(8, 0, full);
-        switch (rest) {
-        case 1: CROSSCOV(1, 128 * full, 1); break;
-        case 2: CROSSCOV(2, 128 * full, 1); break;
-        case 3: CROSSCOV(3, 128 * full, 1); break;
-        case 4: CROSSCOV(4, 128 * full, 1); break;
-        case 5: CROSSCOV(5, 128 * full, 1); break;
-        case 6: CROSSCOV(6, 128 * full, 1); break;
-        case 7: CROSSCOV(7, 128 * full, 1); break;
-        default: break;
-        }
-#undef CROSSCOV
-    } else {
-        const int tiles = (dim + 127) / 128;
-        hipLaunchKernelGGL(vq::k_crosscov_partial, dim3(chunks, tiles * tiles), dim3(256), 0, ctx->stream, d_y, d_x,
-                           n, dim, rows_per_chunk, (double *)ctx->tmp_a.p);
-    }
-    // chunk sums in groups of 32 chunks, then the groups
-    const int per_group = 32, groups = (chunks + per_group - 1) / per_group;
-    hipLaunchKernelGGL(vq::k_crosscov_reduce, dim3(cdiv(total, 256), groups), dim3(256), 0, ctx->stream,
-                       (const double *)ctx->tmp_a.p, chunks, per_group, total, (double *)ctx->tmp_c.p);
-    hipLaunchKernelGGL(vq::k_crosscov_reduce, dim3(cdiv(total, 256), 1), dim3(256), 0, ctx->stream,
-                       (const double *)ctx->tmp_c.p, groups, groups, total, (double *)ctx->tmp_b.p);
-    VQ_HIP(ctx, hipGetLastError());
+    VQ_TRY(cross_cov_device(ctx, d_y, d_x, n, dim));
+    const size_t total = (size_t)dim * dim;
     VQ_HIP(ctx, hipMemcpyAsync(h_A, ctx->tmp_b.p, sizeof(double) * total, hipMemcpyDeviceToHost, ctx->stream));
     VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return VQ_OK;
+}
+
+int32_t vq_opq_rotation(vq_ctx *ctx, const float *d_y, const float *d_x, int64_t n, int32_t dim, float *d_R) {
+    if (!ctx) return VQ_ERR_INVALID_ARG;
+    if (n == 0) return fail(ctx, VQ_ERR_EMPTY_INPUT, "Empty input: at least one vector is required.");
+    if (!d_y || !d_x || !d_R || n < 0 || dim <= 0) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
+    if (dim > 4096) return fail(ctx, VQ_ERR_UNSUPPORTED, "cross-covariance: dim %d > 4096", dim);
+    VQ_HIP(ctx, hipSetDevice(ctx->device));
+    hipStream_t st = ctx->stream;
+    VQ_TRY(cross_cov_device(ctx, d_y, d_x, n, dim));
+    const size_t total = (size_t)dim * dim;
+    if (dim <= vq::kPolarMaxDim && ctx->procrustes_path == 0) {
+        const int P = (dim + 15) / 16 * 16, strips = P / 16;
+        const double *A = (const double *)ctx->tmp_b.p;
+        VQ_TRY(ensure(ctx, ctx->tmp_a, sizeof(double) * (size_t)P * P));
+        VQ_TRY(ensure(ctx, ctx->tmp_d, sizeof(double) * (size_t)P * P));
+        VQ_TRY(ensure(ctx, ctx->tmp_c, sizeof(double) * (size_t)(strips + 2) * dim));
+        VQ_TRY(ensure(ctx, ctx->tmp_f, 1024));
+        VQ_TRY(ensure_pinned(ctx, ctx->lbg_pin, ctx->lbg_pin_cap, sizeof(int)));
+        double *X[2] = {(double *)ctx->tmp_a.p, (double *)ctx->tmp_d.p};
+        double *col_part = (double *)ctx->tmp_c.p, *row_sum = col_part + (size_t)strips * dim, *row_sq = row_sum + dim;
+        vq::PolarTables tb;
+        tb.errs = (unsigned long long *)ctx->tmp_f.p;
+        tb.fin = (int *)(tb.errs + vq::kPolarMaxSteps);
+        tb.bad = tb.fin + vq::kPolarMaxSteps + 2;
+        static_assert(sizeof(unsigned long long) * vq::kPolarMaxSteps + sizeof(int) * (vq::kPolarMaxSteps + 3) <= 1024,
+                      "step tables");
+        volatile int *status = (volatile int *)ctx->lbg_pin;
+        hipLaunchKernelGGL(vq::k_polar_norms, dim3(strips), dim3(256), 0, st, A, dim, col_part, row_sum, row_sq);
+        hipLaunchKernelGGL(vq::k_polar_start, dim3(strips), dim3(256), 0, st, A, dim, P, (const double *)col_part,
+                           (const double *)row_sum, (const double *)row_sq, tb, X[0]);
+        double low = 1e-3;
+        for (int s = 0; s < vq::kPolarMaxSteps;) {
+            const int upto = std::min(vq::kPolarMaxSteps, s == 0 ? 16 : s + 6);
+            VQ_TRY(polar_steps(ctx, X, dim, s, upto, low, tb.errs, tb.fin));
+            s = upto;
+            hipLaunchKernelGGL(vq::k_polar_finish, dim3(cdiv((int64_t)total, 1024)), dim3(256), 0, st,
+                               (const double *)X[0], (const double *)X[1], P, dim, tb, s, d_R, (int *)ctx->lbg_pin);
+            VQ_HIP(ctx, hipGetLastError());
+            VQ_HIP(ctx, hipStreamSynchronize(st));
+            if (*status > 0) return VQ_OK;
+            if (*status < 0) break;
+        }
+    }
+    // the SVD, from host memory
+    std::vector<double> A(total), R(total);
+    VQ_HIP(ctx, hipMemcpyAsync(A.data(), ctx->tmp_b.p, sizeof(double) * total, hipMemcpyDeviceToHost, st));
+    VQ_HIP(ctx, hipStreamSynchronize(st));
+    for (double &v : A) v = (double)(float)v;
+    VQ_TRY(procrustes_svd(ctx, A.data(), dim, R.data()));
+    std::vector<float> r(R.begin(), R.end());
+    VQ_HIP(ctx, hipMemcpyAsync(d_R, r.data(), sizeof(float) * total, hipMemcpyHostToDevice, st));
+    VQ_HIP(ctx, hipStreamSynchronize(st));
     return VQ_OK;
 }
 
@@ -421,7 +540,6 @@ int32_t vq_procrustes_rotation(vq_ctx *ctx, const double *h_A, int32_t dim, doub
     if (!ctx) return VQ_ERR_INVALID_ARG;
     if (!h_A || !h_R || dim < 1) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
     if (dim > 4096) return fail(ctx, VQ_ERR_UNSUPPORTED, "rotation update: dim %d above 4096", dim);
-    const size_t total = (size_t)dim * dim;
     // First the polar factor by Newton-Schulz steps on the f64 matrix cores (any dim up to 512); a
     // matrix that does not converge there — singular, badly conditioned, non-finite — takes the
     // one-sided Jacobi SVD: on the device for even dim up to 128, else the same routine on the host
@@ -436,53 +554,7 @@ int32_t vq_procrustes_rotation(vq_ctx *ctx, const double *h_A, int32_t dim, doub
         VQ_TRY(polar_newton_schulz(ctx, h_A, dim, h_R, &done));
         if (done) return VQ_OK;
     }
-    if (dim > vq::kJacobiMax || dim % 2 != 0) {
-        vqh::procrustes_host(h_A, (size_t)dim, h_R);
-        return VQ_OK;
-    }
-    const int half = dim / 2;
-    VQ_TRY(ensure(ctx, ctx->tmp_a, sizeof(double) * total));
-    VQ_TRY(ensure(ctx, ctx->tmp_b, sizeof(double) * total));
-    VQ_TRY(ensure(ctx, ctx->tmp_c, sizeof(double) * (total + dim)));
-    VQ_TRY(ensure(ctx, ctx->tmp_d, sizeof(double) * total));
-    VQ_TRY(ensure(ctx, ctx->tmp_e, sizeof(double2) * (size_t)vq::kJacobiSweeps * (dim - 1) * half));
-    VQ_TRY(ensure(ctx, ctx->tmp_f, 256));
-    double *d_A = (double *)ctx->tmp_a.p, *d_vt = (double *)ctx->tmp_b.p, *d_uhat = (double *)ctx->tmp_c.p;
-    double *d_sv = d_uhat + total;
-    double *d_out = (double *)ctx->tmp_d.p;
-    double2 *d_rot = (double2 *)ctx->tmp_e.p;
-    int *d_rounds = (int *)ctx->tmp_f.p;
-    VQ_HIP(ctx, hipMemcpyAsync(d_A, h_A, sizeof(double) * total, hipMemcpyHostToDevice, ctx->stream));
-    constexpr int kLanes = 8;
-    const size_t lds = sizeof(double) * (size_t)dim * vq::kJacobiStride;
-    VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_jacobi_sweeps<kLanes>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(vq::k_jacobi_sweeps<kLanes>, dim3(1), dim3(64 * kLanes), lds, ctx->stream, (const double *)d_A,
-                       dim, d_rot, d_rounds, d_uhat, d_sv);
-    hipLaunchKernelGGL(vq::k_jacobi_accumulate, dim3(dim), dim3(64), 0, ctx->stream, (const double2 *)d_rot,
-                       (const int *)d_rounds, dim, d_vt);
-    hipLaunchKernelGGL(vq::k_jacobi_product, dim3((unsigned)cdiv(total, 256)), dim3(256), 0, ctx->stream,
-                       (const double *)d_vt, (const double *)d_uhat, dim, d_out);
-    VQ_HIP(ctx, hipGetLastError());
-    std::vector<double> sv((size_t)dim);
-    VQ_HIP(ctx, hipMemcpyAsync(h_R, d_out, sizeof(double) * total, hipMemcpyDeviceToHost, ctx->stream));
-    VQ_HIP(ctx, hipMemcpyAsync(sv.data(), d_sv, sizeof(double) * dim, hipMemcpyDeviceToHost, ctx->stream));
-    VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    // A singular A leaves directions of U open (their columns came back as zero or as rounding
-    // noise): complete them on the host and form the product again.  Rare; a full-rank A ends here.
-    double top = 0.0;
-    for (double v : sv) top = std::max(top, v);
-    bool open = false;
-    for (double v : sv) open = open || !(top > 0.0 && v > vqh::kNullRel * top);
-    if (open) {
-        std::vector<double> Ut(total), Vt(total);
-        VQ_HIP(ctx, hipMemcpyAsync(Ut.data(), d_uhat, sizeof(double) * total, hipMemcpyDeviceToHost, ctx->stream));
-        VQ_HIP(ctx, hipMemcpyAsync(Vt.data(), d_vt, sizeof(double) * total, hipMemcpyDeviceToHost, ctx->stream));
-        VQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        vqh::complete_null_columns(Ut, Vt, sv, (size_t)dim);
-        vqh::product_v_ut(Vt, Ut, (size_t)dim, h_R);
-    }
-    return VQ_OK;
+    return procrustes_svd(ctx, h_A, dim, h_R);
 }
 
 }  // extern "C"

@@ -517,24 +517,19 @@ public:
         q.rotation_.assign(dim * dim, 0.f);
         for (size_t i = 0; i < dim; ++i) q.rotation_[i * dim + i] = 1.f;  // opq.rs:119
         q.d_rotation_ = DeviceBuffer<float>(dev, dim * dim);
-        std::vector<double> A(dim * dim), Rd;
         for (size_t it = 0; it < opq_iters; ++it) {
             dev->check(vq_lbg_fit(c, drot.get(), (int64_t)n, (int64_t)dim, (int32_t)m, (int32_t)sd, (int32_t)k,
                                   (int32_t)max_iters, streams->init.data(), streams->reseed.data(),
                                   streams->n_reseed, q.codebooks_.get(), nullptr, nullptr));  // 127-142
             dev->check(abi_assign(c, metric, drot.get(), n, dim, m, sd, k, q.codebooks_.get(), dcodes));  // 146-163
             dev->check(abi_decode_f32(c, dcodes, n, m, sd, k, q.codebooks_.get(), drec.get()));         // 164-167
-            dev->check(vq_cross_cov(c, drec.get(), drot.get(), (int64_t)n, (int32_t)dim, A.data())); // 172-179
-            for (double &v : A) v = (double)(float)v;  // the reference's A is a DMatrix<f32>
-            // 180-183 (the library runs the SVD on the device while its kernel takes the size,
-            // else on the host, and completes the directions a singular A leaves open)
-            Rd.resize(dim * dim);
-            dev->check(vq_procrustes_rotation(c, A.data(), (int32_t)dim, Rd.data()));
-            for (size_t i = 0; i < dim * dim; ++i) q.rotation_[i] = (float)Rd[i];
-            q.d_rotation_.upload(q.rotation_.data(), dim * dim);
+            // 172-183: A = Y X^T, rounded to f32 (the reference's A is a DMatrix<f32>), and R = V U^T; both stay
+            // on the device while the library's iteration takes A
+            dev->check(vq_opq_rotation(c, drec.get(), drot.get(), (int64_t)n, (int32_t)dim, q.d_rotation_.get()));
             dev->check(vq_rotate(c, dx.get(), (int64_t)n, (int64_t)dim, (int32_t)dim, q.d_rotation_.get(),
                                  drot.get()));                                                    // 186-194
         }
+        if (opq_iters > 0) q.rotation_ = q.d_rotation_.to_host();
         if (opq_iters == 0) {
             // no outer iteration: the reference keeps an identity rotation and NO codebooks
             // (src/opq.rs:122), so quantize returns an empty vector
