@@ -14,7 +14,7 @@
 // converge quadratically to the exact factor).  A matrix whose first error is below 0.005 is within
 // 0.64 of orthogonal in the 2-norm (128 x the largest entry bounds it), so every singular value is
 // above 0.6 already: it takes plain steps only — a scaled step would first spread them out.  A step is ONE launch (what a step costs is mostly the launch): a workgroup
-// owns a strip of 16 columns; its waves first make the strip of G = X^T X, one 16 x 16 tile each, in
+// owns a strip of 16 columns (or a quarter of its result); its waves first make the strip of G = X^T X, one 16 x 16 tile each, in
 // f64 on the matrix cores (v_mfma_f64_16x16x4_f64), leave M = 1.5 I - 0.5 G for the strip in LDS, meet,
 // and then make their tiles of the strip of X M (the operands sit in L2; every operand of a tile is
 // fetched before its first matrix instruction).  The first half also gives err_k = max |X_k^T X_k - I|;
@@ -71,10 +71,13 @@ __device__ __forceinline__ polar_d4 polar_tile(const double *__restrict__ pa, si
 
 // Step s: Xout = Xin (1.5 r I - 0.5 r^3 Xin^T Xin) with r = rho when the error of step 0 was at
 // least kPolarPlainBelow, else 1; errs[s] = max |Xin^T Xin - I| over the dim x dim block that holds
-// data (NaN counts as infinite).  P x P matrices, row-major, zero beyond dim.  Grid: P / 16
-// workgroups (column strips) of min(P / 16, 8) waves; dynamic LDS: P * 16 doubles.
-// PT = P / 16 when that is at most 8 (every operand of a tile fetched at once, and the rows of Xin
-// for the second half already on their way during the first), 0: any P.
+// data (NaN counts as infinite).  P x P matrices, row-major, zero beyond dim.  Grid: four workgroups per
+// column strip (P / 16 strips, of min(P / 16, 8) waves): a strip's products on one compute unit are bound by
+// its matrix instructions (64 cycles each, 4 us of a step at P = 128), so each of the four makes all of M and a
+// quarter of the tiles of the result.  P = 128: 13.2 us per step with one workgroup per strip, 7.7 with four.
+// Dynamic LDS: P * 16 doubles.
+// PT = 8: P = 128, every operand of a tile fetched at once, and the rows of Xin for the second half already
+// on their way during the first; 0: any P.
 template <int PT>
 static __global__ void __launch_bounds__(512) k_polar_step(const double *__restrict__ Xin, int P, int dim, int s,
                                                            double rho, unsigned long long *__restrict__ errs,
@@ -89,7 +92,7 @@ static __global__ void __launch_bounds__(512) k_polar_step(const double *__restr
     const double first = s > 0 ? __longlong_as_double((long long)errs[0]) : 0.0;
     const double r = first >= kPolarPlainBelow ? rho : 1.0;
     const double ca = 1.5 * r, cb = 0.5 * r * r * r;
-    const int nt = P / 16, tj = blockIdx.x;
+    const int nt = P / 16, tj = (int)blockIdx.x % nt, share = (int)blockIdx.x / nt;
     const int lane = threadIdx.x & 63, kk = lane >> 4, jj = lane & 15;
     const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     double e = 0.0;
@@ -105,22 +108,8 @@ static __global__ void __launch_bounds__(512) k_polar_step(const double *__restr
             }
         }
     };
-    if constexpr (PT > 0) {
-        constexpr int KS = 4 * PT, PP = 16 * PT;
-        const int ti = w;  // one tile per wave
-        // G[i][j] = sum_r X[r][i] X[r][j]: both operands run down a column of X, four rows per step
-        double a[KS], b[KS], a2[KS];
-        const double *pa = Xin + (size_t)kk * PP + 16 * ti + jj, *pb = Xin + (size_t)kk * PP + 16 * tj + jj;
-#pragma unroll
-        for (int u = 0; u < KS; ++u) {
-            a[u] = pa[(size_t)u * 4 * PP];
-            b[u] = pb[(size_t)u * 4 * PP];
-        }
-        // the second half's rows of Xin: Xout[r][j] = sum_c Xin[r][c] M[c][j], A runs along a row
-        const double *pr = Xin + (size_t)(16 * ti + jj) * PP + kk;
-#pragma unroll
-        for (int u = 0; u < KS; ++u) a2[u] = pr[4 * u];
-        emit(polar_mfma<KS>(a, b), ti);
+    auto report = [&]() {  // by one of a strip's workgroups
+        if (share) return;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
             const double o = __shfl_xor(e, off);
@@ -128,25 +117,53 @@ static __global__ void __launch_bounds__(512) k_polar_step(const double *__restr
         }
         // non-negative doubles order like their bit patterns
         if (lane == 0) atomicMax(errs + s, (unsigned long long)__double_as_longlong(e));
+    };
+    if constexpr (PT > 0) {
+        static_assert(PT == 8, "eight waves, a tile each");
+        constexpr int KS = 4 * PT, PP = 16 * PT;
+        const int ti = w;  // one tile per wave
+        // G[i][j] = sum_r X[r][i] X[r][j]: both operands run down a column of X, four rows per step
+        double a[KS], b[KS];
+        const double *pa = Xin + (size_t)kk * PP + 16 * ti + jj, *pb = Xin + (size_t)kk * PP + 16 * tj + jj;
+#pragma unroll
+        for (int u = 0; u < KS; ++u) {
+            a[u] = pa[(size_t)u * 4 * PP];
+            b[u] = pb[(size_t)u * 4 * PP];
+        }
+        // the second half's rows of Xin: Xout[r][j] = sum_c Xin[r][c] M[c][j], A runs along a row.  Two of
+        // the strip's tiles per workgroup, four waves a tile with a quarter of the sum each; a lane has two
+        // consecutive c of every eight (16-byte loads)
+        const int to = 2 * share + (w >> 2), c0 = (w & 3) * (PP / 4) + 2 * kk;
+        const double2 *pr = reinterpret_cast<const double2 *>(Xin + (size_t)(16 * to + jj) * PP + c0);
+        double2 r2[KS / 8];
+#pragma unroll
+        for (int v = 0; v < KS / 8; ++v) r2[v] = pr[4 * v];
+        emit(polar_mfma<KS>(a, b), ti);
+        report();
         __syncthreads();
+        double a2[KS / 4], b2[KS / 4];
 #pragma unroll
-        for (int u = 0; u < KS; ++u) b[u] = m_strip[(4 * u + kk) * 16 + jj];
-        const polar_d4 acc = polar_mfma<KS>(a2, b);
+        for (int v = 0; v < KS / 8; ++v) {
+            a2[2 * v] = r2[v].x;
+            a2[2 * v + 1] = r2[v].y;
+            b2[2 * v] = m_strip[(c0 + 8 * v) * 16 + jj];
+            b2[2 * v + 1] = m_strip[(c0 + 8 * v + 1) * 16 + jj];
+        }
+        const polar_d4 acc = polar_mfma<KS / 4>(a2, b2);
+        __syncthreads();  // the strip becomes the quarters' sums, [wave][v][lane]
 #pragma unroll
-        for (int v = 0; v < 4; ++v) Xout[(size_t)(16 * ti + 4 * v + kk) * PP + 16 * tj + jj] = acc[v];
+        for (int v = 0; v < 4; ++v) m_strip[(w * 4 + v) * 64 + lane] = acc[v];
+        __syncthreads();
+        const double *q = m_strip + (w & 4) * 256 + (w & 3) * 64 + lane;  // this thread: v = w % 4 of its tile
+        Xout[(size_t)(16 * to + 4 * (w & 3) + kk) * PP + 16 * tj + jj] = (q[0] + q[256]) + (q[512] + q[768]);
     } else {
         for (int ti = w; ti < nt; ti += nw)
             emit(polar_tile(Xin + (size_t)kk * P + 16 * ti + jj, 4 * (size_t)P, Xin + (size_t)kk * P + 16 * tj + jj,
                             4 * (size_t)P, P),
                  ti);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const double o = __shfl_xor(e, off);
-            e = o > e ? o : e;
-        }
-        if (lane == 0) atomicMax(errs + s, (unsigned long long)__double_as_longlong(e));
+        report();
         __syncthreads();
-        for (int ti = w; ti < nt; ti += nw) {
+        for (int ti = 4 * w + share; ti < nt; ti += 4 * nw) {
             const polar_d4 acc = polar_tile(Xin + (size_t)(16 * ti + jj) * P + kk, 4, m_strip + kk * 16 + jj, 64, P);
 #pragma unroll
             for (int v = 0; v < 4; ++v) Xout[(size_t)(16 * ti + 4 * v + kk) * P + 16 * tj + jj] = acc[v];

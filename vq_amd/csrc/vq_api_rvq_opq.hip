@@ -182,7 +182,7 @@ int32_t polar_steps(vq_ctx *ctx, double *const (&X)[2], int dim, int from, int u
             rho = std::sqrt(3.0 / (1.0 + low + low * low));
             low = rho * low * (3.0 - rho * rho * low * low) * 0.5;
         }
-        hipLaunchKernelGGL((P == 128 ? vq::k_polar_step<8> : vq::k_polar_step<0>), dim3(strips), dim3(64 * waves), lds,
+        hipLaunchKernelGGL((P == 128 ? vq::k_polar_step<8> : vq::k_polar_step<0>), dim3(4 * strips), dim3(64 * waves), lds,
                            ctx->stream, (const double *)X[s & 1], P, dim, s, rho, errs, fin, X[(s + 1) & 1]);
     }
     VQ_HIP(ctx, hipGetLastError());
