@@ -19,7 +19,12 @@ def ctx():
 
 
 @pytest.mark.parametrize("n,dim,ld,stages,k", [(513, 4, 4, 3, 9), (577, 32, 32, 4, 16), (640, 36, 40, 3, 16),
-                                               (1000, 100, 100, 3, 31), (703, 132, 136, 2, 300), (2049, 128, 129, 4, 16)])
+                                               (1000, 100, 100, 3, 31), (703, 132, 136, 2, 300), (2049, 128, 129, 4, 16),
+                                               # the tables of all stages in one launch: three parts and one product
+                                               (900, 40, 40, 4, 100), (3000, 64, 64, 5, 32), (1200, 256, 256, 3, 256),
+                                               # the codebooks of all stages in LDS for the reconstruction: whole groups
+                                               # of columns, a last group of 8, all columns in one
+                                               (16_400, 128, 128, 4, 256), (8000, 264, 264, 4, 256), (33_001, 64, 64, 8, 64)])
 def test_rows_stop_one_by_one(ctx, n, dim, ld, stages, k):
     rng = np.random.default_rng(dim + n)
     cb = rng.standard_normal((stages, k, dim)).astype(F)

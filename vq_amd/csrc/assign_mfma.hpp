@@ -1168,6 +1168,7 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
                                                                   uint32_t *__restrict__ list_count,
                                                                   float *__restrict__ pen, float pen_c2,
                                                                   float *__restrict__ sigma, float pen_dc,
+                                                                  int count_step,
                                                                   const float *__restrict__ cnorm = nullptr) {
     const int s = blockIdx.x, b = blockIdx.y;
     const int i = threadIdx.x & 31, g = threadIdx.x >> 5;
@@ -1331,7 +1332,7 @@ static __global__ void __launch_bounds__(256) k_mfma_wide_bf_prep(const float *_
             mx = (mx == mx && o == o) ? fmaxf(mx, o) : __builtin_nanf("");
         }
         if (i == 0) blockmax[(size_t)s * nb + b] = mx;
-        if (s == 0 && b == 0 && i < 2) list_count[i] = 0;
+        if (b == 0 && i < 2) list_count[(m - 1 - s) * count_step + i] = 0;  // (step 0: one pair for all column blocks)
     }
 }
 

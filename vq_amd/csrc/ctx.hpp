@@ -60,6 +60,13 @@ struct vq_ctx {
     int recheck_src = 0;         // where the last pass counted its undecided pairs: 1 mfma_stat, 2 mfma_list, 3 the fixed scratch
     int assign_path = 0;         // 0 = matrix cores where a kernel exists, 1 = vector ALU only
     int few_path = 0;            // 0 = a few rows in one launch, 1 = by the kernels of longer calls
+    // while an encode goes through stages that each have their own centroids: the operand tables of all of
+    // them are made in one launch, at the first (launch_mfma_wide)
+    struct StageTables {
+        const float *cb = nullptr;  // [stages][k][dim]
+        int stages = 0, stage = 0;
+        bool ready = false;
+    } stage_tables;
     bool lbg_small_lds_set = false;  // dynamic-LDS limit granted to k_lbg_update_small
     int compute_units = 0;       // of the context's GPU (0: not asked for yet)
     int decode_lds_set[4] = {0, 0, 0, 0};  // dynamic-LDS limit already granted to the four resident decode kernels

@@ -9,6 +9,8 @@
 
 namespace vq {
 
+typedef uint32_t rot_u32x4 __attribute__((ext_vector_type(4)));
+
 // res[i] -= codebook[code[i]]   (src/rvq.rs:127).  One lane per element.
 template <typename CodeT>
 static __global__ void __launch_bounds__(256) k_residual_sub(float *__restrict__ res, int64_t n, int64_t ld,
@@ -267,6 +269,89 @@ static __global__ void __launch_bounds__(256) k_rvq_recon4_f16(int64_t n, int di
     }
 }
 
+// The same with the stages' codebooks of G columns in LDS (blockIdx.y: which ones): a thread makes 16 bytes of
+// the output per step, U of them in flight, the next stage's codes on their way while one is added.  The
+// gather above reads 4 bytes of centroid per stage and element through the vector caches, which bounds it: gather ->
+// resident, 200,000 x 128, 4 stages of 256 (51 MB written) 31.2 -> 17.9 us, 100,000 x 256, 2 stages 20.8 -> 13.0, 200,000 x 64, 8
+// stages of 64 30.0 -> 15.1, 50,000 x 768, 4 stages 44.6 -> 22.3, 16,400 x 128 8.1 -> 6.4 (from 2^21 elements on).
+// Columns per group: the table within 128 KB, a row's share of the output no less than half a line; 0: none.
+inline int rvq_recon_columns(int stages, int k, int dim, int code_bytes) {
+    if (dim % 8 != 0 || stages < 1 || (int64_t)stages * k > 1024 || code_bytes != 1) return 0;
+    const int fit = 32 * 1024 / (stages * k) / 32 * 32;
+    return fit < dim ? fit : dim;
+}
+template <typename CodeT>
+static __global__ void __launch_bounds__(1024) k_rvq_recon_resident(int64_t n, int dim, int k, int G,
+                                                                    const float *__restrict__ codebooks,
+                                                                    const CodeT *__restrict__ codes, int stages,
+                                                                    const uint8_t *__restrict__ used,
+                                                                    rot_u32x4 *__restrict__ out) {
+    extern __shared__ __attribute__((aligned(16))) float4 tab4[];  // [stages * k][columns / 4]
+    constexpr int U = 2;
+    const int c0 = (int)blockIdx.y * G, cols = dim - c0 < G ? dim - c0 : G;
+    const uint32_t q4 = (uint32_t)cols / 4, pieces = (uint32_t)cols / 8, dim8 = (uint32_t)dim / 8;
+    for (uint32_t e = threadIdx.x; e < (uint32_t)(stages * k) * q4; e += 1024)
+        tab4[e] = *reinterpret_cast<const float4 *>(codebooks + (size_t)(e / q4) * dim + c0 + 4 * (e % q4));
+    __syncthreads();
+    const int64_t rows = U * 1024 / pieces > 1 ? U * 1024 / pieces : 1;  // of a run
+    for (int64_t row0 = blockIdx.x * rows; row0 < n; row0 += gridDim.x * rows) {
+        const uint32_t count = (uint32_t)(n - row0 < rows ? n - row0 : rows) * pieces;
+        const CodeT *run = codes + row0 * stages;
+        const uint8_t *run_used = used + row0;
+        rot_u32x4 *to = out + row0 * dim8 + c0 / 8;
+        for (uint32_t l0 = threadIdx.x; l0 < count; l0 += U * 1024) {
+            uint32_t row[U], at[U], code[U];
+            int nst[U];
+            float4 lo[U], hi[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t l = l0 + 1024u * u < count ? l0 + 1024u * u : l0;
+                row[u] = l / pieces;
+                at[u] = l - row[u] * pieces;
+                nst[u] = run_used[row[u]];
+                code[u] = run[row[u] * (uint32_t)stages];
+                lo[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+                hi[u] = lo[u];
+            }
+            for (int st = 0; st < stages; ++st) {
+                uint32_t next[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    next[u] = run[row[u] * (uint32_t)stages + (uint32_t)(st + 1 < stages ? st + 1 : st)];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const float4 *c = tab4 + ((uint32_t)(st * k) + (st < nst[u] ? code[u] : 0u)) * q4 + 2 * at[u];
+                    const float4 a = c[0], b = c[1];
+                    if (st < nst[u]) {
+                        lo[u] = make_float4(lo[u].x + a.x, lo[u].y + a.y, lo[u].z + a.z, lo[u].w + a.w);
+                        hi[u] = make_float4(hi[u].x + b.x, hi[u].y + b.y, hi[u].z + b.z, hi[u].w + b.w);
+                    }
+                    code[u] = next[u];
+                }
+            }
+            auto two = [](float x, float y) {
+                return (uint32_t)__half_as_ushort(__float2half_rn(x)) | ((uint32_t)__half_as_ushort(__float2half_rn(y)) << 16);
+            };
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (l0 + 1024u * u < count)
+                    __builtin_nontemporal_store(rot_u32x4{two(lo[u].x, lo[u].y), two(lo[u].z, lo[u].w), two(hi[u].x, hi[u].y),
+                                                          two(hi[u].z, hi[u].w)},
+                                                to + (row[u] * dim8 + at[u]));
+        }
+    }
+}
+
+// Every row active, no stage used.
+static __global__ void __launch_bounds__(256) k_rvq_begin(uint8_t *__restrict__ active, uint8_t *__restrict__ used,
+                                                          int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) {
+        active[i] = 1;
+        used[i] = 0;
+    }
+}
+
 // The row stops when ||residual|| < epsilon (src/rvq.rs:204-207).
 static __global__ void __launch_bounds__(256) k_rvq_stage_stop(const float *__restrict__ norms, int64_t n,
                                                         float epsilon, uint8_t *__restrict__ active) {
@@ -503,7 +588,6 @@ namespace vq {
 
 typedef float rot_floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 rot_bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t rot_u32x4 __attribute__((ext_vector_type(4)));
 
 // v -> (h, m, l) bf16 bit patterns, h + m + l == v
 __device__ __forceinline__ void rot_split3(float v, uint32_t &h, uint32_t &m, uint32_t &l) {

@@ -285,30 +285,38 @@ int32_t launch_wide_exact(vq_ctx *ctx, const vq::AssignArgs &a, int sd, const ui
 template <int METRIC, bool LBG>
 int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     const int nb = (a.k + 31) / 32, nkc = sd / 8, nsl = (sd + 31) / 32;
+    constexpr bool COS = METRIC == vq::M_COS;
+    // Stages of an encode: their tables lie one behind the other like those of column blocks and are made by the
+    // first one's launches (9.4 us a stage at k = 256, 128 floats); each has its own counts, the last one's in the header.
+    auto &stages = ctx->stage_tables;
+    const bool staged = !COS && !LBG && a.m == 1 && stages.cb && a.cb == stages.cb + (size_t)stages.stage * a.k * sd;
+    const int mt = staged ? stages.stages : a.m, at = staged ? stages.stage : 0;
     // A operands: 2 x 64 lanes x 16 bytes per (s, 16 dimensions, block of 32 centroids)
-    const size_t n_atab = (size_t)a.m * ((sd + 15) / 16) * nb * 128 * 4, n_c2 = (size_t)a.m * nb * 32;  // floats
-    VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + 2 * n_c2 + (size_t)a.m * nb + (size_t)a.m * sd + 2 * a.m + 2 * (size_t)a.m * nsl + 8) + 64));
+    const size_t n_atab = (size_t)mt * ((sd + 15) / 16) * nb * 128 * 4, n_c2 = (size_t)mt * nb * 32;  // floats
+    VQ_TRY(ensure(ctx, ctx->mfma_tab, sizeof(float) * (n_atab + 2 * n_c2 + (size_t)mt * nb + (size_t)mt * sd + 2 * mt + 2 * (size_t)mt * nsl + 8) + 64));
     // header (two counts), the list for the all-centroid check, the list for the two-candidate check
     const size_t n_pairs = (size_t)a.n * a.m;
     // ... and the candidates of an eighth of the pairs (a list beyond that goes over all centroids)
-    const size_t mask_cap = n_pairs / 8 + 4096, n_list = 4 + ((n_pairs + 3) & ~(size_t)3) + ((2 * n_pairs + 3) & ~(size_t)3);
+    const size_t n_head = staged ? 4 * (size_t)mt : 4;
+    const size_t mask_cap = n_pairs / 8 + 4096, n_list = n_head + ((n_pairs + 3) & ~(size_t)3) + ((2 * n_pairs + 3) & ~(size_t)3);
     VQ_TRY(ensure(ctx, ctx->mfma_list, sizeof(uint32_t) * (n_list + 8 * mask_cap)));
     float *atab = (float *)ctx->mfma_tab.p;
     float *c2perm = atab + n_atab;
     float *pen = c2perm + n_c2;
     float *maxc2 = pen + n_c2;  // per block of 32 centroids
-    float *mu = maxc2 + (((size_t)a.m * nb + 3) & ~(size_t)3);  // 16-byte aligned: read as float4
+    float *mu = maxc2 + (((size_t)mt * nb + 3) & ~(size_t)3);  // 16-byte aligned: read as float4
     uint32_t *count = (uint32_t *)ctx->mfma_list.p;
-    uint32_t *list = count + 4;
+    uint32_t *list = count + n_head;
     uint2 *pairs = (uint2 *)(list + ((n_pairs + 3) & ~(size_t)3));  // 16-byte aligned
     vq::u32x4 *masks = (vq::u32x4 *)(count + n_list);               // likewise
-    float2 *norms = (float2 *)(mu + (size_t)a.m * sd);  // sd is a multiple of 8: 8-byte aligned
-    int *shifted = (int *)(norms + (size_t)a.m * nsl);
-    float *sigma = (float *)(shifted + a.m);
-    constexpr bool COS = METRIC == vq::M_COS;
+    float2 *norms = (float2 *)(mu + (size_t)mt * sd);  // sd is a multiple of 8: 8-byte aligned
+    int *shifted = (int *)(norms + (size_t)mt * nsl);
+    float *sigma = (float *)(shifted + mt);
     const bool own_centre = !COS && vq::wide_own_centre(a.k, sd);
-    if (!COS && !own_centre)
-        hipLaunchKernelGGL(vq::k_block_centres, dim3(a.m, nsl), dim3(256), 0, ctx->stream, a.cb, a.k, sd, mu, norms);
+    const bool make = !staged || !stages.ready;
+    const float *tab_cb = staged ? stages.cb : a.cb;
+    if (!COS && !own_centre && make)
+        hipLaunchKernelGGL(vq::k_block_centres, dim3(mt, nsl), dim3(256), 0, ctx->stream, tab_cb, a.k, sd, mu, norms);
     // squared L2, Euclidean: see kWideT and kWideRho
     // cosine, in units of |x|, two candidates: the split of an operand twice as long, 2^-22 for the division by
     // the norm, fp32 accumulation (34 per 8 dimensions + 16) * 2^-24 of partial sums up to 4.2 |x|, the
@@ -329,13 +337,24 @@ int32_t launch_mfma_wide(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
                                          : (const void *)vq::k_mfma_wide_bf_prep<false, true>
                             : own_centre ? (const void *)vq::k_mfma_wide_bf_prep<false, false, true>
                                          : (const void *)vq::k_mfma_wide_bf_prep<COS, false>;
-    {
+    if (make) {
         vq::u32x4 *atab4 = (vq::u32x4 *)atab;
-        int m = a.m, k = a.k, nbv = nb, sdv = sd;
+        int m = mt, k = a.k, nbv = nb, sdv = sd, step = staged ? 4 : 0;
         float pc = pen_c2, pd = pen_dc;
-        const float *cb = a.cb, *cnorm = a.cnorm;
-        void *args[] = {&cb, &mu, &norms, &shifted, &m, &k, &nbv, &sdv, &atab4, &c2perm, &maxc2, &count, &pen, &pc, &sigma, &pd, &cnorm};
-        VQ_HIP(ctx, hipLaunchKernel(prep, dim3(a.m, nb), dim3(256), args, 0, ctx->stream));
+        const float *cb = tab_cb, *cnorm = a.cnorm;
+        void *args[] = {&cb, &mu, &norms, &shifted, &m, &k, &nbv, &sdv, &atab4, &c2perm, &maxc2, &count, &pen, &pc, &sigma, &pd, &step, &cnorm};
+        VQ_HIP(ctx, hipLaunchKernel(prep, dim3(mt, nb), dim3(256), args, 0, ctx->stream));
+        if (staged) stages.ready = true;
+    }
+    if (staged) {  // this stage's
+        atab += (size_t)at * ((sd + 15) / 16) * nb * (half ? 64 : 128) * 4;
+        c2perm += (size_t)at * nb * 32;
+        pen += (size_t)at * nb * 32;
+        maxc2 += (size_t)at * nb;
+        mu += (size_t)at * sd;
+        shifted += at;
+        sigma += at;
+        count += 4 * (mt - 1 - at);
     }
     vq::MfmaWideBfTables tb{(const vq::u32x4 *)atab, c2perm, pen, maxc2, mu, shifted, sigma, list, count, pairs, masks, (uint32_t)mask_cap, nb, sd,
                             kappa, twice * cross * t, twice * t / rho, lift, rel};

@@ -86,7 +86,7 @@ int32_t rvq_encode(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int
     float *res = (float *)ctx->tmp_c.p;
     CodeT *stage_codes[2] = {(CodeT *)ctx->tmp_e.p, (CodeT *)((uint8_t *)ctx->tmp_e.p + codes_bytes)};
     uint8_t *active = (uint8_t *)ctx->tmp_e.p + 2 * codes_bytes;
-    uint8_t *used = active + n;
+    uint8_t *used = d_stages_used ? d_stages_used : active + n;
     // With no norm test between the stages (epsilon <= 0: every row uses every stage) the update of
     // the residual by a stage's centroids waits for the next stage's assignment, where that pass can
     // take it along: one pass over the rows per stage instead of two.
@@ -97,13 +97,22 @@ int32_t rvq_encode(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int
     if (need_res && !direct)
         VQ_HIP(ctx, hipMemcpy2DAsync(res, sizeof(float) * dim, d_x, sizeof(float) * ld, sizeof(float) * dim,
                                      (size_t)n, hipMemcpyDeviceToDevice, st));
-    hipLaunchKernelGGL(vq::k_fill<uint8_t>, dim3(cdiv(n, 256)), dim3(256), 0, st, active, n, (uint8_t)1);
-    hipLaunchKernelGGL(vq::k_fill<uint8_t>, dim3(cdiv(n, 256)), dim3(256), 0, st, used, n, (uint8_t)0);
+    hipLaunchKernelGGL(vq::k_rvq_begin, dim3(cdiv(n, 256)), dim3(256), 0, st, active, used, n);
+    // the tables of all stages in one launch, as far as they are small beside the rows
+    struct Stages {
+        vq_ctx::StageTables &t;
+        ~Stages() { t = vq_ctx::StageTables(); }
+    } tables{ctx->stage_tables};
+    if (sizeof(CodeT) == 1 && stages > 1 && (int64_t)stages * k <= n) {
+        tables.t.cb = d_codebooks;
+        tables.t.stages = stages;
+    }
     const float *pend_cb = nullptr;  // the stage whose update of the residual is still to come
     const CodeT *pend_codes = nullptr;
     bool pend_from_x = false;        // ... and reads the caller's rows
     for (int s = 0; s < stages; ++s) {
         const float *cb = d_codebooks + (size_t)s * k * dim;
+        tables.t.stage = s;
         CodeT *cur = stage_codes[s & 1];
         const bool from_x = direct && s == 0;
         const float *rows = from_x ? d_x : res;
@@ -147,10 +156,17 @@ int32_t rvq_encode(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int
                                active);
         }
     }
-    if (d_stages_used)
-        VQ_HIP(ctx, hipMemcpyAsync(d_stages_used, used, (size_t)n, hipMemcpyDeviceToDevice, st));
     if (d_recon_f16) {
-        if (vec4 && (reinterpret_cast<uintptr_t>(d_recon_f16) & 7) == 0)
+        const int cols = vq::rvq_recon_columns(stages, k, dim, (int)sizeof(CodeT));
+        if (vec4 && cols && n * dim >= (1 << 21) && (reinterpret_cast<uintptr_t>(d_recon_f16) & 15) == 0) {
+            const size_t lds = sizeof(float) * (size_t)stages * k * cols;
+            auto kern = vq::k_rvq_recon_resident<CodeT>;
+            VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            const unsigned groups = cdiv(dim, cols), wgs = std::max(1u, 256u / groups);
+            hipLaunchKernelGGL(kern, dim3(wgs, groups), dim3(1024), lds, st, n, dim, k, cols, d_codebooks,
+                               (const CodeT *)d_codes, stages, (const uint8_t *)used, (vq::rot_u32x4 *)d_recon_f16);
+        } else if (vec4 && (reinterpret_cast<uintptr_t>(d_recon_f16) & 7) == 0)
             hipLaunchKernelGGL(vq::k_rvq_recon4_f16<CodeT>, dim3(cdiv(n * (dim / 4), 1024)), dim3(256), 0, st, n,
                                dim / 4, k, d_codebooks, (const CodeT *)d_codes, stages, (const uint8_t *)used,
                                d_recon_f16);
