@@ -274,10 +274,14 @@ static __global__ void __launch_bounds__(256) k_rvq_recon4_f16(int64_t n, int di
 // gather above reads 4 bytes of centroid per stage and element through the vector caches, which bounds it: gather ->
 // resident, 200,000 x 128, 4 stages of 256 (51 MB written) 31.2 -> 17.9 us, 100,000 x 256, 2 stages 20.8 -> 13.0, 200,000 x 64, 8
 // stages of 64 30.0 -> 15.1, 50,000 x 768, 4 stages 44.6 -> 22.3, 16,400 x 128 8.1 -> 6.4 (from 2^21 elements on).
-// Columns per group: the table within 128 KB, a row's share of the output no less than half a line; 0: none.
+// Columns per group: the table within 128 KB, 32 columns or more, or 16 (0: none).  A group's share of a row is then
+// half a line, or a quarter; the quarters come from four workgroups at about the same time (every group's workgroup x
+// lies on the same XCD and takes the same rows) and meet in its L2 if they are stored as ordinary lines: 1M x 256, eight
+// stages of 256, 425 -> 219 us (565 past the L2), 200,000 x 128 50 -> 31.  Halves of lines go past it: 200,000 x 128, four
+// stages, 18.3 us against 19.2.
 inline int rvq_recon_columns(int stages, int k, int dim, int code_bytes) {
-    if (dim % 8 != 0 || stages < 1 || (int64_t)stages * k > 1024 || code_bytes != 1) return 0;
-    const int fit = 32 * 1024 / (stages * k) / 32 * 32;
+    if (dim % 8 != 0 || stages < 1 || (int64_t)stages * k > 2048 || code_bytes != 1) return 0;
+    const int most = 32 * 1024 / (stages * k), fit = most < 32 ? 16 : most / 32 * 32;
     return fit < dim ? fit : dim;
 }
 template <typename CodeT>
@@ -334,10 +338,12 @@ static __global__ void __launch_bounds__(1024) k_rvq_recon_resident(int64_t n, i
             };
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                if (l0 + 1024u * u < count)
-                    __builtin_nontemporal_store(rot_u32x4{two(lo[u].x, lo[u].y), two(lo[u].z, lo[u].w), two(hi[u].x, hi[u].y),
-                                                          two(hi[u].z, hi[u].w)},
-                                                to + (row[u] * dim8 + at[u]));
+                if (l0 + 1024u * u < count) {
+                    const rot_u32x4 o = {two(lo[u].x, lo[u].y), two(lo[u].z, lo[u].w), two(hi[u].x, hi[u].y), two(hi[u].z, hi[u].w)};
+                    rot_u32x4 *p = to + (row[u] * dim8 + at[u]);
+                    if (G >= 32) __builtin_nontemporal_store(o, p);
+                    else *p = o;
+                }
         }
     }
 }
