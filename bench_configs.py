@@ -107,15 +107,18 @@ def opq_fit_device(ctx, dx, n, dim, m, k, iters, outer, streams, metric, bufs=No
         ctx.lbg_fit(drot, n, dim, m, sd, k, iters, init, reseed, dcb)       # 127-142
         ctx.assign(metric, drot, n, dim, m, sd, k, dcb, dcodes)             # 146-163
         ctx.decode_f32(dcodes, n, m, sd, k, dcb, drec)                      # 164-167
-        A = ctx.cross_cov(drec, drot, n, dim).astype(F).astype(np.float64)  # 172-179 (a DMatrix<f32>)
-        R = ctx.procrustes_rotation(A).astype(F)                            # 180-183
-        dR.upload(R)
+        if trace is not None:
+            A = ctx.cross_cov(drec, drot, n, dim).astype(F).astype(np.float64)  # 172-179 (a DMatrix<f32>)
+            R = ctx.procrustes_rotation(A).astype(F)                        # 180-183
+            dR.upload(R)
+        else:
+            ctx.opq_rotation(drec, drot, n, dim, dR)                        # both, A and R on the device
         ctx.rotate(dx, n, dim, dim, dR, drot)                               # 186-194
         if it + 1 in snapshots:
-            snaps[it + 1] = (R.copy(), dcb.download())
+            snaps[it + 1] = (dR.download(), dcb.download())
         if trace is not None:
             trace.append((rows, dcb.download(), dcodes.download(), A, R.copy()))
-    return R, bufs, snaps
+    return (dR.download() if outer else R), bufs, snaps
 
 
 def run_c3(ctx, log, x=None, dx=None, parity=True):
