@@ -144,7 +144,9 @@ __device__ __forceinline__ int exact_rows_lds(unsigned long long todo, int code,
 // workgroup itself, and its waves walk over tiles of 32 rows on their own, no barrier after the set-up.  The
 // 32 scores that a lane has of 64 centroids go into four sets of eight, {32 b + 8 p + 4 h + 0..3} of two neighbouring
 // blocks b: 16 minima, four tags and five operations for the two smallest keys, 25 instructions where sets of
-// four take 34 (k_assign_mfma8, whose pick among four instead of eight centroids weighs as much there).
+// four take 34.  FOUR: sets of four, the runs themselves, where there are at most four pairs of blocks and the pick
+// among eight centroids of 16 floats is more than that saves (eight -> four, Euclidean: 600,000 rows x 8 blocks, k = 256
+// 195 -> 181 us, 60,000 x 10 38.4 -> 34.0, k = 64 28.9 -> 24.2, 10,000 x 10 18.5 -> 15.5).
 // Even and odd pairs of blocks, and the two lane halves, each have two smallest keys of their own, so that the four
 // best sets are known with their tags and a row that only two sets can win is decided among their sixteen
 // centroids; the others, a tenth of the pairs that one bound leaves open, go through all k.
@@ -160,6 +162,7 @@ __global__ void __launch_bounds__(SD == 8 ? 1024 : 768, SD == 8 ? 4 : 3) k_assig
     __shared__ float red[2][16][SD], mu_all[SD];
     constexpr bool COS = METRIC == M_COS, LBG = CODES == CODES_LBG;
     constexpr int NH = SD / 2, NI = SD / 8;  // dimensions of a lane half, matrix instructions per 32 centroids
+    constexpr bool FOUR = SD == 16 && CODES != CODES_U16;  // sets of four (up to 256 centroids)
     const AssignArgs &a = args.a;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int T = (int)blockDim.x, W = T >> 6;
@@ -331,15 +334,23 @@ __global__ void __launch_bounds__(SD == 8 ? 1024 : 768, SD == 8 ? 4 : 3) k_assig
                                    __float_as_int(c[4 * p + 2])), __float_as_int(c[4 * p + 3])),                      \
                         __float_as_int(d[4 * p])), __float_as_int(d[4 * p + 1])), __float_as_int(d[4 * p + 2])),      \
          __float_as_int(d[4 * p + 3]))
+#define VQ_MIN4(c, p)                                                                                                 \
+    imin(imin(imin(__float_as_int(c[4 * p]), __float_as_int(c[4 * p + 1])), __float_as_int(c[4 * p + 2])),            \
+         __float_as_int(c[4 * p + 3]))
+#define VQ_KEY4(c, p, tag) (int)(((uint32_t)VQ_MIN4(c, p) & keep) | (tag))
 #define VQ_KEY(c, d, p, tag) key[p] = (int)(((uint32_t)VQ_MIN8(c, d, p) & keep) | (tag));
         // selection of 64 centroids (scores in c, d) with the matrix instructions of the next 64 (into e, f)
-#define VQ_PAIR(c, d, e, f, first, second, T0, T1, T2, T3, next)                                                      \
+#define VQ_PAIR(c, d, e, f, first, second, T0, T1, T2, T3, T4, T5, T6, T7, next)                                      \
     {                                                                                                                 \
         int key[4];                                                                                                   \
         VQ_MFMA(n0[0], row.b16[0], zero, e)                                                                           \
         if constexpr (NI == 2) VQ_MFMA(n1[0], row.b16[0], zero, f)                                                    \
         __builtin_amdgcn_sched_barrier(0);                                                                            \
-        VQ_KEY(c, d, 0, T0) VQ_KEY(c, d, 1, T1)                                                                       \
+        if constexpr (FOUR) {                                                                                         \
+            top2_push4(first, second, VQ_KEY4(c, 0, T0), VQ_KEY4(c, 1, T1), VQ_KEY4(c, 2, T2), VQ_KEY4(c, 3, T3));    \
+        } else {                                                                                                      \
+            VQ_KEY(c, d, 0, T0) VQ_KEY(c, d, 1, T1)                                                                   \
+        }                                                                                                             \
         __builtin_amdgcn_sched_barrier(0);                                                                            \
         if constexpr (NI == 2) {                                                                                      \
             VQ_MFMA(n0[NI - 1], row.b16[NI - 1], e, e)                                                                \
@@ -349,12 +360,17 @@ __global__ void __launch_bounds__(SD == 8 ? 1024 : 768, SD == 8 ? 4 : 3) k_assig
         }                                                                                                             \
         operands(next);                                                                                               \
         __builtin_amdgcn_sched_barrier(0);                                                                            \
-        VQ_KEY(c, d, 2, T2) VQ_KEY(c, d, 3, T3)                                                                       \
-        top2_push4(first, second, key[0], key[1], key[2], key[3]);                                                    \
+        if constexpr (FOUR) {                                                                                         \
+            top2_push4(first, second, VQ_KEY4(d, 0, T4), VQ_KEY4(d, 1, T5), VQ_KEY4(d, 2, T6), VQ_KEY4(d, 3, T7));    \
+        } else {                                                                                                      \
+            VQ_KEY(c, d, 2, T2) VQ_KEY(c, d, 3, T3)                                                                   \
+            top2_push4(first, second, key[0], key[1], key[2], key[3]);                                                \
+        }                                                                                                             \
         __builtin_amdgcn_sched_barrier(0);                                                                            \
     }
-        // the tags of the sets, one scalar register each: tag = 8 * pair + 2 * set
+        // the tags of the sets, one scalar register each: tag = 8 * pair + 2 * set (FOUR: 16 * pair + 2 * set)
         uint32_t t0 = 0, t1 = 2, t2 = 4, t3 = 6, t4 = 8, t5 = 10, t6 = 12, t7 = 14;
+        uint32_t u0 = 16, u1 = 18, u2 = 20, u3 = 22, u4 = 24, u5 = 26, u6 = 28, u7 = 30;  // FOUR, odd pairs
         auto opaque = [](uint32_t &v) { asm volatile("" : "+s"(v)); };  // (else each is made again from one of them)
         const u32x4 *ap = at + lane;
         u32x4 n0[NI], n1[NI];  // of the next pair's two blocks
@@ -375,12 +391,22 @@ __global__ void __launch_bounds__(SD == 8 ? 1024 : 768, SD == 8 ? 4 : 3) k_assig
         operands(np > 1 ? 1 : 0);
         for (int p = 0; p < np; p += 2) {
             opaque(t0), opaque(t1), opaque(t2), opaque(t3), opaque(t4), opaque(t5), opaque(t6), opaque(t7);
-            VQ_PAIR(p0, p1, q0, q1, m1, m2, t0, t1, t2, t3, p + 2 < np ? p + 2 : 0)
-            if (p + 1 < np) VQ_PAIR(q0, q1, p0, p1, o1, o2, t4, t5, t6, t7, p + 3 < np ? p + 3 : 0)
-            t0 += 16, t1 += 16, t2 += 16, t3 += 16, t4 += 16, t5 += 16, t6 += 16, t7 += 16;
+            if constexpr (FOUR) {
+                opaque(u0), opaque(u1), opaque(u2), opaque(u3), opaque(u4), opaque(u5), opaque(u6), opaque(u7);
+                VQ_PAIR(p0, p1, q0, q1, m1, m2, t0, t1, t2, t3, t4, t5, t6, t7, p + 2 < np ? p + 2 : 0)
+                if (p + 1 < np) VQ_PAIR(q0, q1, p0, p1, o1, o2, u0, u1, u2, u3, u4, u5, u6, u7, p + 3 < np ? p + 3 : 0)
+                t0 += 32, t1 += 32, t2 += 32, t3 += 32, t4 += 32, t5 += 32, t6 += 32, t7 += 32;
+                u0 += 32, u1 += 32, u2 += 32, u3 += 32, u4 += 32, u5 += 32, u6 += 32, u7 += 32;
+            } else {
+                VQ_PAIR(p0, p1, q0, q1, m1, m2, t0, t1, t2, t3, 0, 0, 0, 0, p + 2 < np ? p + 2 : 0)
+                if (p + 1 < np) VQ_PAIR(q0, q1, p0, p1, o1, o2, t4, t5, t6, t7, 0, 0, 0, 0, p + 3 < np ? p + 3 : 0)
+                t0 += 16, t1 += 16, t2 += 16, t3 += 16, t4 += 16, t5 += 16, t6 += 16, t7 += 16;
+            }
         }
 #undef VQ_MFMA
 #undef VQ_MIN8
+#undef VQ_MIN4
+#undef VQ_KEY4
 #undef VQ_KEY
 #undef VQ_PAIR
         m1 |= h;  // bit 0 of the tag: the lane half
@@ -402,9 +428,35 @@ __global__ void __launch_bounds__(SD == 8 ? 1024 : 768, SD == 8 ? 4 : 3) k_assig
         // the run in the two low bits.  at: the best; lo, hi: the two smallest keys (lower lanes).
         auto first_of = [](int set) {
             const uint32_t tag = (uint32_t)set & 0xFFu;
+            if constexpr (FOUR) return (int)((tag >> 3) * 32 + ((tag >> 1) & 3u) * 8 + (tag & 1u) * 4);
             return (int)((tag >> 3) * 64 + ((tag >> 1) & 3u) * 8 + (tag & 1u) * 4);
         };
+        // FOUR: the one run of a set, its first two centroids in the lower half, the others in the upper.
         auto pick = [&](int first, int &at, int &lo, int &hi) {
+            if constexpr (FOUR) {
+                const int ra = cl.run(first, h), j0 = first + 2 * h;
+                float2 inv = make_float2(0.f, 0.f);
+                if constexpr (COS) inv = *reinterpret_cast<const float2 *>(norms + kp + j0);
+                int ky[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    float ca[NH], cb[NH];
+                    cl.piece(ra, i, ca);
+                    cl.piece(ra, i + 2, cb);
+                    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(share8<METRIC, NH>(xraw, ca)),
+                                                                     __float_as_int(share8<METRIC, NH>(xraw, cb)), false, false);
+                    float d = __int_as_float((int)sw[0]) + __int_as_float((int)sw[1]);
+                    if constexpr (COS) d = j0 + i < k ? __builtin_fmaf(-(d * row.rx), i ? inv.y : inv.x, 1.001f) : 1e30f;
+                    ky[i] = (int)((__float_as_uint(d) & 0xFFFFFFFCu) | (uint32_t)(i + 2 * h));
+                }
+                int l0, l1, h0, h1;
+                swap_halves(imin(ky[0], ky[1]), l0, l1);
+                swap_halves(imax(ky[0], ky[1]), h0, h1);
+                lo = imin(l0, l1);
+                hi = imin3(imax(l0, l1), h0, h1);
+                at = first + (lo & 3);
+                return;
+            }
             const int ra = cl.run(first, h), rb = cl.run(first + 32, h);
             const int j0 = first + 32 * h;
             float4 inv = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -471,8 +523,9 @@ __global__ void __launch_bounds__(SD == 8 ? 1024 : 768, SD == 8 ? 4 : 3) k_assig
                 const float na = COS ? seq_norm8(xs) : 0.0f;
                 float bd = 0.0f;
                 int bj = -1;
-                for (int i = 0; i < (__ballot(other >= 0 && !clear) ? 16 : 8); ++i) {
-                    const int j = (i < 8 || other < 0 ? first : other) + (i & 3) + ((i >> 2) & 1) * 32;
+                constexpr int N = FOUR ? 4 : 8;  // centroids of a set
+                for (int i = 0; i < (__ballot(other >= 0 && !clear) ? 2 * N : N); ++i) {
+                    const int j = (i < N || other < 0 ? first : other) + (i & 3) + (FOUR ? 0 : ((i >> 2) & 1) * 32);
                     float c[SD];
                     cl.load(j, c);
                     const float d = dist8<METRIC>(xs, c, na, COS ? norms[j] : 0.0f);

@@ -442,7 +442,7 @@ bool mfma_applicable(const vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
 
 // 16-float column blocks: one pass with the operands in LDS, undecided rows resolved in the same kernel
 // (assign_mfma_lds.hpp).  Against the kernel of wider blocks, its tables and its follow-up (an encode, Euclidean): 600,000 x
-// 8 blocks, k = 256 369 -> 195 us, 60,000 x 10 61 -> 37, k = 32 33 -> 26, 1,000 x 10 15.4 -> 10.8; cosine 376 -> 201, 64 -> 36.
+// 8 blocks, k = 256 369 -> 181 us, 60,000 x 10 61 -> 34, k = 32 33 -> 24, 1,000 x 10 15.4 -> 11; cosine, with sets of eight, 376 -> 201, 64 -> 36.
 template <int METRIC, bool LBG>
 bool mfma16_applicable(const vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     if (ctx->assign_path == 1 || ctx->no_alloc || a.pend_cb) return false;
