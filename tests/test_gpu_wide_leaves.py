@@ -20,14 +20,19 @@ def ctx():
 SIZES = [1, 15, 16, 17, 64, 65, 127, 128, 129, 511, 512, 1024, 1025, 2500, 8000, 12_300]
 
 
-@pytest.mark.parametrize("order", ["shuffled", "sorted", "reversed"])
-@pytest.mark.parametrize("m,sd", [(1, 64), (2, 65), (1, 128), (1, 256), (1, 257), (3, 100), (1, 512)])
-def test_leaves(ctx, m, sd, order):
+# (the last: 100 million floats and 300,000 rows and more, where the leaves are taken in an order of their own)
+@pytest.mark.parametrize("m,sd,n,order", [(m, sd, 0, order) for order in ("shuffled", "sorted", "reversed") for m, sd in
+                                          [(1, 64), (2, 65), (1, 128), (1, 256), (1, 257), (3, 100), (1, 512)]] +
+                         [(1, 64, 1_570_000, "shuffled"), (2, 161, 311_000, "shuffled"), (1, 333, 302_000, "sorted"),
+                          (1, 257, 390_000, "reversed"), (1, 100, 1_001_000, "sorted")])
+def test_leaves(ctx, m, sd, n, order):
     rng = np.random.default_rng(sd)
-    label = np.repeat(np.arange(len(SIZES)), SIZES)
+    sizes = SIZES + ([n // 3, n - sum(SIZES) - n // 3] if n else [])
+    label = np.repeat(np.arange(len(sizes)), sizes)
     label = label if order == "sorted" else label[::-1] if order == "reversed" else rng.permutation(label)
-    n, k = len(label), len(SIZES)
-    x = rng.standard_normal((n, m * sd)).astype(F) + (50 * label[:, None]).astype(F)
+    n, k = len(label), len(sizes)
+    x = rng.standard_normal((n, m * sd), dtype=F)
+    x += (50 * label[:, None]).astype(F)
     init = np.tile(np.array([np.flatnonzero(label == j)[0] for j in range(k)], np.uint32), (m, 1))
     reseed = rng.integers(0, n, (m, 3 * k), dtype=np.uint32)
     want = O.pq_fit(x, m, k, 3, init, reseed)

@@ -1426,7 +1426,11 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
     // per-part sums of the streaming kernel, then one folded sum per cluster
     if (stream) VQ_TRY(ensure(ctx, ctx->part_sum, sizeof(float) * (size_t)m * (nparts + 1) * vq::kMaxK * 8));
     // Blocks of 64 to 512 floats: leaves handed out long ones first, then part by part (k_lbg_leafsum_wide)
-    const bool wide_leaves = !stream && sd >= 64 && sd <= 512;
+    // where the rows are well beyond the memory-side cache (256 MB): the order costs 5 us per iteration in the scan, and rows
+    // that lie in the cache may be read in any order.  An iteration of a residual fit, k = 256, without -> with:
+    // 150,000 x 256 172 -> 179 us, 300,000 240 -> 241, 500,000 351 -> 343, 1,000,000 620 -> 589; x 128: 300,000 164 -> 169, 600,000
+    // 258 -> 252 (k = 121 2 % slower), 1,000,000 384 -> 360; x 512: 250,000 384 -> 390, 500,000 646 -> 633; 3,000,000 x 64 589 -> 565.
+    const bool wide_leaves = !stream && sd >= 64 && sd <= 512 && n >= 300'000 && n * m * sd >= 100'000'000;
     const size_t long_cap = (size_t)(n / vq::kLong + 1), leaf_slots = (size_t)m * leaf_cap;
     if (wide_leaves)  // the leaves in order, the two lists of long ones, the places, the counters
         VQ_TRY(ensure(ctx, ctx->leaf_desc, sizeof(uint4) * (leaf_slots + 2 * (size_t)m * long_cap) +
