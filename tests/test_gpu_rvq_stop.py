@@ -26,7 +26,8 @@ def ctx():
                                                # of columns, a last group of 8, all columns in one
                                                (16_400, 128, 128, 4, 256), (8000, 264, 264, 4, 256), (33_001, 64, 64, 8, 64),
                                                # 16 columns in a group, a last group of 8
-                                               (16_391, 128, 128, 8, 256), (29_200, 72, 72, 8, 200)])
+                                               (16_391, 128, 128, 8, 256), (29_200, 72, 72, 8, 200),
+                                               (16_400, 128, 128, 3, 300)])  # 16-bit codes
 def test_rows_stop_one_by_one(ctx, n, dim, ld, stages, k):
     rng = np.random.default_rng(dim + n)
     cb = rng.standard_normal((stages, k, dim)).astype(F)

@@ -279,8 +279,8 @@ static __global__ void __launch_bounds__(256) k_rvq_recon4_f16(int64_t n, int di
 // lies on the same XCD and takes the same rows) and meet in its L2 if they are stored as ordinary lines: 1M x 256, eight
 // stages of 256, 425 -> 219 us (565 past the L2), 200,000 x 128 50 -> 31.  Halves of lines go past it: 200,000 x 128, four
 // stages, 18.3 us against 19.2.
-inline int rvq_recon_columns(int stages, int k, int dim, int code_bytes) {
-    if (dim % 8 != 0 || stages < 1 || (int64_t)stages * k > 2048 || code_bytes != 1) return 0;
+inline int rvq_recon_columns(int stages, int k, int dim) {
+    if (dim % 8 != 0 || stages < 1 || (int64_t)stages * k > 2048) return 0;
     const int most = 32 * 1024 / (stages * k), fit = most < 32 ? 16 : most / 32 * 32;
     return fit < dim ? fit : dim;
 }

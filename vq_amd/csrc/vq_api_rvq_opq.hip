@@ -157,7 +157,7 @@ int32_t rvq_encode(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int
         }
     }
     if (d_recon_f16) {
-        const int cols = vq::rvq_recon_columns(stages, k, dim, (int)sizeof(CodeT));
+        const int cols = vq::rvq_recon_columns(stages, k, dim);
         if (vec4 && cols && n * dim >= (1 << 21) && (reinterpret_cast<uintptr_t>(d_recon_f16) & 15) == 0) {
             const size_t lds = sizeof(float) * (size_t)stages * k * cols;
             auto kern = vq::k_rvq_recon_resident<CodeT>;
