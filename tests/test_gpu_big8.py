@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
+from tests import data
 from tests.test_gpu_wide_bound import _case
 
 pytestmark = pytest.mark.gpu
@@ -63,3 +64,29 @@ def test_codebook_off_alignment(ctx):
     assert np.array_equal(codes.download(), O.pq_encode(O.SQEUCLIDEAN, x, cb).astype(np.uint16))
     big = rng.standard_normal((1, 2100, 8)).astype(F)
     _check(ctx, x[:, :8].copy(), big, O.SQEUCLIDEAN)
+
+
+@pytest.mark.parametrize("metric", [O.SQEUCLIDEAN, O.EUCLIDEAN])
+@pytest.mark.parametrize("sd,k", [(16, 35), (16, 63), (16, 319), (16, 1023), (8, 319), (8, 2047)])  # one padding centroid in the last set
+def test_block_around_the_padding(ctx, sd, k, metric):
+    """A block far from the origin, by any place that padding centroids could be given: none of them is ever chosen."""
+    rng = np.random.default_rng(k)
+    for off in (1e18, -1e18, 1e15, 0.0):
+        x = (F(off) + F(3e12) * rng.standard_normal((4000, 2 * sd)).astype(F)).astype(F)
+        cb = (F(off) + F(1e13) * rng.standard_normal((2, k, sd)).astype(F)).astype(F)
+        if k > 256:
+            _check(ctx, x, cb, metric)
+            continue
+        codes = ctx.empty((4000, 2), np.uint8)
+        ctx.assign(metric, ctx.to_device(x), 4000, 2 * sd, 2, sd, k, ctx.to_device(cb), codes)
+        assert np.array_equal(codes.download(), O.pq_encode(metric, x, cb).astype(np.uint8))
+
+
+def test_fit_around_the_padding(ctx):
+    n, m, sd, k = 5000, 2, 16, 35
+    rng = np.random.default_rng(3)
+    x = (F(1e18) + F(1e13) * rng.standard_normal((n, m * sd)).astype(F)).astype(F)
+    init, reseed = data.index_streams(n, m, k, 4, seed=k)
+    cb = ctx.empty((m, k, sd), F)
+    ctx.lbg_fit(ctx.to_device(x), n, sd * m, m, sd, k, 4, init, reseed, cb)
+    assert np.array_equal(cb.download().view(np.uint32), O.pq_fit(x, m, k, 4, init, reseed)["codebooks"].view(np.uint32))

@@ -9,8 +9,10 @@
 namespace vq {
 
 constexpr int kBig8Max = 2048, kLds16Max = 1024;
-constexpr float kBig8Far = 1e18f;   // components of the padding centroids: squares stay finite, and farther off than
-                                    // any centroid of a block whose scale exists (kBig8Rms)
+// Components of the padding centroids: +inf, so that their distance to every finite row is +inf wherever the block's
+// centroids lie (a scale bounds their spread, not their place).  In a pick they are never clear of a centroid whose
+// distance is finite, and beside one that overflows they tie, which the reference's distances of j < k decide.
+constexpr float kLdsFar = __builtin_inff();
 constexpr float kBig8Rms = 1e30f;   // largest mean square norm about the centre that is scored
 
 enum { CODES_LBG = 0, CODES_U8 = 1, CODES_U16 = 2 };  // [m][n] bytes in place (old -> new), [n][m] bytes, [n][m] 16 bits
@@ -188,7 +190,7 @@ __global__ void __launch_bounds__(SD == 8 ? 1024 : 768, SD == 8 ? 4 : 3) k_assig
         constexpr int P = SD / 4;  // 16-byte pieces of a centroid
         const float4 *src = reinterpret_cast<const float4 *>(a.cb + (size_t)s * k * SD);
         for (int i = threadIdx.x; i < P * kp; i += T)
-            cl.set(i / P, i % P, i < P * k ? src[i] : make_float4(kBig8Far, kBig8Far, kBig8Far, kBig8Far));
+            cl.set(i / P, i % P, i < P * k ? src[i] : make_float4(kLdsFar, kLdsFar, kLdsFar, kLdsFar));
     }
     __syncthreads();
     float mu[SD], sg = kCosScale, bad = 0.0f;
