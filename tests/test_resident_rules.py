@@ -1,0 +1,60 @@
+"""Which reconstructions take their table into LDS (vq_amd/csrc/resident_rules.hpp): the rules are compiled by g++ and
+asked for sizes up to the limits of the entry points.  What they admit has its places within a run in 32 bits and its
+groups within a grid's second dimension; what they refuse goes to the gather kernels, which take any size."""
+import os
+import random
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+MAIN = """
+#include <cstdio>
+#include "resident_rules.hpp"
+int main() {
+    long long n; int f16, m, sd, k;
+    while (scanf("%d %lld %d %d %d", &f16, &n, &m, &sd, &k) == 5) printf("%d\\n", vq::decode_resident_blocks(f16, n, m, sd, k));
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("rules") / "rules")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-x", "c++", "-", "-I", os.path.join(ROOT, "vq_amd", "csrc"),
+                    "-o", exe], input=MAIN, text=True, check=True)
+
+    def ask(cases):
+        text = "\n".join(" ".join(str(int(v)) for v in c) for c in cases)
+        return [int(v) for v in subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.split()]
+    return ask
+
+
+def _decode_ok(f16, n, m, sd, k, G):
+    pieces, block = sd // (8 if f16 else 4), k * sd * (2 if f16 else 4)
+    groups = -(-m // G)
+    for mg in {min(G, m), m - (groups - 1) * G}:  # a whole group, the last one
+        rows = min(n, max(1, 1024 * (4 if f16 else 8) // (mg * pieces)))  # of a run, as k_decode_resident takes them
+        if (rows - 1) * m * pieces + mg * pieces > 2 ** 32:
+            return False
+    return sd % (8 if f16 else 4) == 0 and block * G <= 128 * 1024 and groups <= 65535
+
+
+def test_decode_at_the_limits(rules):
+    rng = random.Random(1)
+    edges = [(1 << e) + d for e in range(8, 24) for d in (-1, 0, 1, 5)] + [1064961, 532481]
+    cases = [(f16, n, m, sd, k) for f16 in (0, 1) for m in edges for sd in (4, 8, 16, 24) for k in (1, 5, 256, 2048)
+             for n in (1, 2, 5, 100, 4096, 8192, 1 << 20, 1 << 31)]
+    cases += [(rng.random() < 0.5, int(2 ** rng.uniform(0, 32)), int(2 ** rng.uniform(0, 24)), rng.choice([4, 8, 8, 16, 32, 100, 512]),
+               int(2 ** rng.uniform(0, 16))) for _ in range(20_000)]
+    got = rules(cases)
+    assert sum(G > 0 for G in got) > 1000
+    assert [c for c, G in zip(cases, got) if G and not _decode_ok(*c, G)] == []
+
+
+def test_decode_of_ordinary_sizes(rules):
+    """(binary16, n, m, sub_dim, k): column blocks per group."""
+    want = {(1, 1_000_000, 16, 8, 256): 16, (1, 300_000, 16, 8, 1024): 8, (0, 300_000, 16, 8, 1024): 4, (1, 200_000, 12, 8, 256): 12,
+            (1, 66_000, 17, 8, 2048): 4, (1, 130_000, 9, 16, 5000): 0, (1, 1000, 16, 8, 256): 0, (1, 50_000, 16, 12, 256): 0,
+            (0, 100_000, 10, 12, 200): 10, (1, 4_194_304, 1, 8, 1): 1, (1, 3, 500_000, 8, 2048): 0, (1, 4096, 1064961, 8, 1): 0}
+    assert rules(list(want)) == list(want.values())

@@ -19,6 +19,7 @@
 #include "assign_mfma.hpp"
 #include "assign_mfma_lds.hpp"
 #include "decode.hpp"
+#include "resident_rules.hpp"
 
 #ifndef VQ_MFMA_RUN
 #define VQ_MFMA_RUN 8    // tiles of 32 rows per wave in the matrix-core assignment (a power of two)
@@ -644,18 +645,9 @@ template <bool F16, typename CodeT>
 int32_t launch_decode_resident(vq_ctx *ctx, const CodeT *d_codes, int64_t n, int m, int sd, int k,
                                const float *d_codebooks, void *d_out, bool *done) {
     *done = false;
-    // Where the table of all column blocks does not fit, a group of them whose pieces of a row fill whole lines, or
-    // half of one, if there are enough rows for the groups' tables (k_decode_gather: 50 us for the 36 above).
-    const size_t block = (size_t)k * sd * (F16 ? 2 : 4), line = (size_t)sd * (F16 ? 2 : 4);
-    if (sd % (F16 ? 8 : 4) != 0 || block > 128 * 1024 || n * m < (1 << 16)) return VQ_OK;
-    int G = m;
-    if (block * m > 128 * 1024) {
-        G = (int)(128 * 1024 / block);
-        if (G * line >= 128) G = (int)(G * line / 128 * 128 / line);
-        if (G < 1 || G * line < 64 || n * m < (1 << 20)) return VQ_OK;
-    }
-    if ((int64_t)m * sd >= (1 << 24)) return VQ_OK;  // 32-bit places in a run
-    const size_t lds = block * G;
+    const int G = vq::decode_resident_blocks(F16, n, m, sd, k);
+    if (G == 0) return VQ_OK;
+    const size_t lds = (size_t)k * sd * (F16 ? 2 : 4) * G;
     if ((reinterpret_cast<uintptr_t>(d_codebooks) | reinterpret_cast<uintptr_t>(d_out)) & 15) return VQ_OK;
     auto kern = k_decode_resident<F16, CodeT>;
     // the kernel's LDS limit and the number of compute units: asked for once per context and kernel
