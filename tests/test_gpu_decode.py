@@ -18,7 +18,10 @@ def ctx():
 @pytest.mark.parametrize("n,m,sd,k", [
     (1, 1, 8, 2), (1025, 3, 8, 40), (70_001, 1, 8, 256), (5463, 12, 16, 256), (70_000, 1, 512, 20),  # whole table / gather
     (110_001, 10, 8, 1024), (66_000, 17, 8, 2048), (33_001, 33, 24, 300), (263_000, 4, 16, 3000),   # groups, the last short
-    (130_000, 9, 16, 5000), (4097, 2, 64, 700), (999, 5, 12, 300)])                                 # a block too large: gather
+    (130_000, 9, 16, 5000), (4097, 2, 64, 700), (999, 5, 12, 300),                                  # a block too large: gather
+    (87_401, 12, 8, 1024), (53_003, 20, 8, 2048), (262_145, 4, 8, 256), (52_429, 10, 8, 300),  # table in LDS: binary16
+    (21_001, 25, 8, 200), (10_699, 49, 8, 11),
+    (87_401, 12, 4, 1024), (53_003, 20, 4, 2048), (33_000, 17, 4, 256), (175_001, 3, 4, 2000)])  # table in LDS: f32
 def test_decode(ctx, n, m, sd, k):
     rng = np.random.default_rng(n + k)
     cb = (rng.standard_normal((m, k, sd)) * 100).astype(F)
@@ -34,6 +37,23 @@ def test_decode(ctx, n, m, sd, k):
     (ctx.decode_f32_u16 if wide else ctx.decode_f32)(dcodes, n, m, sd, k, dcb, out32)
     got = out32.download()
     assert np.array_equal(got[:n], want) and (got[n] == 7.0).all()
+
+
+@pytest.mark.parametrize("off", [2, 16, 32, 64])
+def test_output_off_alignment(ctx, off):
+    """An output that starts anywhere in a line: the table in LDS only where lines are filled."""
+    rng = np.random.default_rng(off)
+    n, m, k = 35_537, 16, 200
+    cb, codes = rng.standard_normal((m, k, 8)).astype(F), rng.integers(0, k, (n, m))
+    out = ctx.to_device(np.full(n * m * 8 + 64, 0x5555, np.uint16))
+
+    class Part:
+        ptr = out.ptr + off
+    ctx.decode_f16(ctx.to_device(codes.astype(np.uint8)), n, m, 8, k, ctx.to_device(cb), Part())
+    got = out.download()
+    want = cb[np.arange(m)[None, :], codes].reshape(-1).astype(np.float16).view(np.uint16)
+    assert np.array_equal(got[off // 2:off // 2 + len(want)], want)
+    assert (got[:off // 2] == 0x5555).all() and (got[off // 2 + len(want):] == 0x5555).all()
 
 
 @pytest.mark.parametrize("dim", [8, 24, 128, 12, 7])
