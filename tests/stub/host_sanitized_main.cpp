@@ -102,6 +102,7 @@ int main() {
         CHECK(q.quantize(rows[1]).len() == dim);
         CHECK(q.quantize_batch(rows).size() == n);
         CHECK(q.rotation().size() == dim * dim);
+        CHECK(q.rotation()[dim - 1] == 1.0f && q.rotation()[0] == 0.0f);  // the stand-in's vq_opq_rotation
         CHECK(q.encode(rows).size() == n * 3);
         auto none = OptimizedProductQuantizer::fit(rows, 3, 4, 2, 0, Distance(Distance::Euclidean), 0);
         CHECK(!none.trained());

@@ -209,17 +209,11 @@ int32_t vq_rotate(vq_ctx *, const float *x, int64_t n, int64_t ld, int32_t dim, 
         for (int t = 0; t < dim; ++t) y[i * dim + t] = x[i * ld + t];
     return VQ_OK;
 }
-int32_t vq_cross_cov(vq_ctx *, const float *y, const float *x, int64_t n, int32_t dim, double *A) {
+int32_t vq_opq_rotation(vq_ctx *, const float *y, const float *x, int64_t n, int32_t dim, float *R) {  // reverses a row
     touch(y, (size_t)n * dim);
     touch(x, (size_t)n * dim);
     for (int a = 0; a < dim; ++a)
-        for (int b = 0; b < dim; ++b) A[(size_t)a * dim + b] = a == b ? 1.0 : 0.0;
-    return VQ_OK;
-}
-int32_t vq_procrustes_rotation(vq_ctx *, const double *A, int32_t dim, double *R) {
-    touch(A, (size_t)dim * dim);
-    for (int a = 0; a < dim; ++a)
-        for (int b = 0; b < dim; ++b) R[(size_t)a * dim + b] = a == b ? 1.0 : 0.0;
+        for (int b = 0; b < dim; ++b) R[(size_t)a * dim + b] = a + b == dim - 1 ? 1.0f : 0.0f;
     return VQ_OK;
 }
 

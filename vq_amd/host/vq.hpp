@@ -33,10 +33,6 @@
 
 #include "../../include/vq_hip.h"
 
-// Newer than the other entry points: a program may be linked with a library that does not have it.
-extern "C" int32_t vq_opq_rotation(vq_ctx *ctx, const float *d_y, const float *d_x, int64_t n, int32_t dim, float *d_R)
-    __attribute__((weak));
-
 namespace vq {
 
 // ---- errors (src/exceptions.rs) ----------------------------------------------------------------
@@ -529,15 +525,7 @@ public:
             dev->check(abi_decode_f32(c, dcodes, n, m, sd, k, q.codebooks_.get(), drec.get()));         // 164-167
             // 172-183: A = Y X^T, rounded to f32 (the reference's A is a DMatrix<f32>), and R = V U^T; both stay
             // on the device while the library's iteration takes A
-            if (vq_opq_rotation) {
-                dev->check(vq_opq_rotation(c, drec.get(), drot.get(), (int64_t)n, (int32_t)dim, q.d_rotation_.get()));
-            } else {
-                std::vector<double> A(dim * dim), R(dim * dim);
-                dev->check(vq_cross_cov(c, drec.get(), drot.get(), (int64_t)n, (int32_t)dim, A.data()));
-                for (double &v : A) v = (double)(float)v;
-                dev->check(vq_procrustes_rotation(c, A.data(), (int32_t)dim, R.data()));
-                q.d_rotation_.upload(std::vector<float>(R.begin(), R.end()).data(), dim * dim);
-            }
+            dev->check(vq_opq_rotation(c, drec.get(), drot.get(), (int64_t)n, (int32_t)dim, q.d_rotation_.get()));
             dev->check(vq_rotate(c, dx.get(), (int64_t)n, (int64_t)dim, (int32_t)dim, q.d_rotation_.get(),
                                  drot.get()));                                                    // 186-194
         }
