@@ -100,7 +100,6 @@ def opq_fit_device(ctx, dx, n, dim, m, k, iters, outer, streams, metric, bufs=No
                     cb=ctx.empty((m, k, sd), F), R=ctx.empty((dim, dim), F))
     drot, drec, dcodes, dcb, dR = bufs["rot"], bufs["rec"], bufs["codes"], bufs["cb"], bufs["R"]
     ctx.copy_f32(drot, dx, n * dim)                                         # opq.rs:121
-    R = np.eye(dim, dtype=F)
     snaps = {}
     for it in range(outer):
         rows = drot.download() if trace is not None else None
@@ -108,17 +107,14 @@ def opq_fit_device(ctx, dx, n, dim, m, k, iters, outer, streams, metric, bufs=No
         ctx.assign(metric, drot, n, dim, m, sd, k, dcb, dcodes)             # 146-163
         ctx.decode_f32(dcodes, n, m, sd, k, dcb, drec)                      # 164-167
         if trace is not None:
-            A = ctx.cross_cov(drec, drot, n, dim).astype(F).astype(np.float64)  # 172-179 (a DMatrix<f32>)
-            R = ctx.procrustes_rotation(A).astype(F)                        # 180-183
-            dR.upload(R)
-        else:
-            ctx.opq_rotation(drec, drot, n, dim, dR)                        # both, A and R on the device
+            A = ctx.cross_cov(drec, drot, n, dim).astype(F).astype(np.float64)  # 172-179 (a DMatrix<f32>), for the record
+        ctx.opq_rotation(drec, drot, n, dim, dR)                            # 172-183, A and R on the device
         ctx.rotate(dx, n, dim, dim, dR, drot)                               # 186-194
         if it + 1 in snapshots:
             snaps[it + 1] = (dR.download(), dcb.download())
         if trace is not None:
-            trace.append((rows, dcb.download(), dcodes.download(), A, R.copy()))
-    return (dR.download() if outer else R), bufs, snaps
+            trace.append((rows, dcb.download(), dcodes.download(), A, dR.download()))
+    return (dR.download() if outer else np.eye(dim, dtype=F)), bufs, snaps
 
 
 def run_c3(ctx, log, x=None, dx=None, parity=True):
