@@ -27,6 +27,9 @@ def ctx():
                                                (16_400, 128, 128, 4, 256), (8000, 264, 264, 4, 256), (33_001, 64, 64, 8, 64),
                                                # 16 columns in a group, a last group of 8
                                                (16_391, 128, 128, 8, 256), (29_200, 72, 72, 8, 200),
+                                               # groups of widths that are no multiple of 32, one of all columns
+                                               (10_600, 200, 200, 6, 256), (8100, 264, 264, 8, 256), (29_200, 72, 72, 2, 256),
+                                               (15_500, 136, 136, 2, 16),
                                                (16_400, 128, 128, 3, 300)])  # 16-bit codes
 def test_rows_stop_one_by_one(ctx, n, dim, ld, stages, k):
     rng = np.random.default_rng(dim + n)

@@ -12,8 +12,9 @@ MAIN = """
 #include <cstdio>
 #include "resident_rules.hpp"
 int main() {
-    long long n; int f16, m, sd, k;
-    while (scanf("%d %lld %d %d %d", &f16, &n, &m, &sd, &k) == 5) printf("%d\\n", vq::decode_resident_blocks(f16, n, m, sd, k));
+    long long n; int what, a, b, c;  // what: 0 decode to f32, 1 to binary16, 2 residual sums
+    while (scanf("%d %lld %d %d %d", &what, &n, &a, &b, &c) == 5)
+        printf("%d\\n", what == 2 ? vq::rvq_recon_columns(n, a, b, c) : vq::decode_resident_blocks(what, n, a, b, c));
 }
 """
 
@@ -61,3 +62,27 @@ def test_decode_of_ordinary_sizes(rules):
             # a table that the vector cache holds
             (1, 1_000_000, 16, 8, 16): 0, (0, 1_000_000, 16, 4, 200): 0, (0, 1_000_000, 16, 4, 256): 16}
     assert rules(list(want)) == list(want.values())
+
+
+def _recon_ok(n, stages, k, dim, G):
+    groups = -(-dim // G)
+    for cols in {G, dim - (groups - 1) * G}:
+        rows = min(n, max(1, 2048 // (cols // 8)))  # of a run, as k_rvq_recon_resident takes them
+        if cols % 8 or (rows - 1) * (dim // 8) + cols // 8 > 2 ** 32:
+            return False
+    return 4 * stages * k * G <= 128 * 1024 and groups <= 65535
+
+
+def test_residual_sums(rules):
+    rng = random.Random(2)
+    dims = [(1 << e) + d for e in range(3, 31) for d in (-8, 0, 8, 24)] + [32 * 65535, 32 * 65535 + 8, 16 * 65535 + 16]
+    cases = [(2, n, stages, k, dim) for dim in dims if dim > 0 for stages in (1, 2, 4, 8, 255) for k in (1, 8, 100, 256, 300)
+             for n in (1, 3, 2048, 1 << 20)]
+    cases += [(2, int(2 ** rng.uniform(0, 32)), rng.randint(1, 40), int(2 ** rng.uniform(0, 10)), rng.randint(1, 500)) for _ in range(5000)]
+    got = rules(cases)
+    assert sum(G > 0 for G in got) > 1000
+    assert [c for c, G in zip(cases, got) if G and not _recon_ok(*c[1:], G)] == []
+    want = {(200_000, 4, 256, 128): 32, (1_000_000, 8, 256, 256): 16, (200_000, 6, 256, 200): 16, (100_000, 2, 256, 256): 64,
+            (400_000, 2, 256, 72): 0, (100_000, 2, 16, 136): 136, (100_000, 9, 256, 64): 0, (100_000, 4, 256, 100): 0,
+            (1, 4, 256, 32 * 65535 + 32): 0}
+    assert rules([(2, *c) for c in want]) == list(want.values())

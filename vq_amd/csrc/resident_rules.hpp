@@ -35,4 +35,18 @@ inline int decode_resident_blocks(bool f16, int64_t n, int m, int sd, int k) {
     return (int)G;
 }
 
+// Columns per group of k_rvq_recon_resident; 0: the gather.  The stages' table within 128 KB, 32 columns or more, or 16.
+// Where groups share rows that are not whole halves of lines, from four stages on: gather -> resident of 256 centroids
+// 200,000 x 72, two stages 14.9 -> 15.0 us, 400,000 33.6 -> 42.8, 400,000 x 104 38 -> 50; four stages 200,000 x 136 39 -> 31, 400,000 60 -> 63,
+// 200,000 x 264 65 -> 56; six 49 -> 37 (200,000 x 136); geometric means over seven widths 1.08, 0.87, 0.83.
+inline int rvq_recon_columns(int64_t n, int stages, int k, int dim) {
+    if (dim % 8 != 0 || stages < 1 || (int64_t)stages * k > 2048) return 0;
+    const int most = 32 * 1024 / (stages * k), fit = most < 32 ? 16 : most / 32 * 32;
+    if (fit >= dim) return dim;
+    const int64_t groups = (dim + fit - 1) / fit, last = dim - (groups - 1) * fit;
+    const int64_t rows = std::min<int64_t>(n, std::max<int64_t>(1, 2048 / (last / 8)));  // of a run of the last group
+    if (groups > kMaxGridY || rows * (dim / 8) >= (1LL << 32)) return 0;  // places in a run: 32 bits
+    return dim % 32 != 0 && stages < 4 ? 0 : fit;
+}
+
 }  // namespace vq

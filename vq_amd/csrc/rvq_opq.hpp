@@ -269,21 +269,16 @@ static __global__ void __launch_bounds__(256) k_rvq_recon4_f16(int64_t n, int di
     }
 }
 
-// The same with the stages' codebooks of G columns in LDS (blockIdx.y: which ones): a thread makes 16 bytes of
-// the output per step, U of them in flight, the next stage's codes on their way while one is added.  The
+// The same with the stages' codebooks of G columns in LDS (blockIdx.y: which ones; rvq_recon_columns): a thread makes 16
+// bytes of the output per step, U of them in flight, the next stage's codes on their way while one is added.  The
 // gather above reads 4 bytes of centroid per stage and element through the vector caches, which bounds it: gather ->
 // resident, 200,000 x 128, 4 stages of 256 (51 MB written) 31.2 -> 17.9 us, 100,000 x 256, 2 stages 20.8 -> 13.0, 200,000 x 64, 8
 // stages of 64 30.0 -> 15.1, 50,000 x 768, 4 stages 44.6 -> 22.3, 16,400 x 128 8.1 -> 6.4 (from 2^21 elements on).
-// Columns per group: the table within 128 KB, 32 columns or more, or 16 (0: none).  A group's share of a row is then
-// half a line, or a quarter; the quarters come from four workgroups at about the same time (every group's workgroup x
-// lies on the same XCD and takes the same rows) and meet in its L2 if they are stored as ordinary lines: 1M x 256, eight
-// stages of 256, 425 -> 219 us (565 past the L2), 200,000 x 128 50 -> 31.  Halves of lines go past it: 200,000 x 128, four
-// stages, 18.3 us against 19.2.
-inline int rvq_recon_columns(int stages, int k, int dim) {
-    if (dim % 8 != 0 || stages < 1 || (int64_t)stages * k > 2048) return 0;
-    const int most = 32 * 1024 / (stages * k), fit = most < 32 ? 16 : most / 32 * 32;
-    return fit < dim ? fit : dim;
-}
+// The workgroups of a group are a multiple of eight, so that every group's workgroup x lies on the same XCD and
+// takes the same rows: shares of a row that end inside a line, quarters of lines or those of a width that is no multiple
+// of 32, meet in its L2 if they are stored as ordinary lines: 1M x 256, eight stages of 256, 425 -> 219 us (565 past the
+// L2), 200,000 x 200 (13 groups of 16) 57 -> 34, where 19 workgroups a group took 57.  Halves of lines, and runs of whole rows, go
+// past it: 200,000 x 128, four stages, 18.3 us against 19.2.
 template <typename CodeT>
 static __global__ void __launch_bounds__(1024) k_rvq_recon_resident(int64_t n, int dim, int k, int G,
                                                                     const float *__restrict__ codebooks,
@@ -293,11 +288,13 @@ static __global__ void __launch_bounds__(1024) k_rvq_recon_resident(int64_t n, i
     extern __shared__ __attribute__((aligned(16))) float4 tab4[];  // [stages * k][columns / 4]
     constexpr int U = 2;
     const int c0 = (int)blockIdx.y * G, cols = dim - c0 < G ? dim - c0 : G;
+    const bool past_l2 = G == dim || (G >= 32 && dim % 32 == 0);
     const uint32_t q4 = (uint32_t)cols / 4, pieces = (uint32_t)cols / 8, dim8 = (uint32_t)dim / 8;
     for (uint32_t e = threadIdx.x; e < (uint32_t)(stages * k) * q4; e += 1024)
         tab4[e] = *reinterpret_cast<const float4 *>(codebooks + (size_t)(e / q4) * dim + c0 + 4 * (e % q4));
     __syncthreads();
-    const int64_t rows = U * 1024 / pieces > 1 ? U * 1024 / pieces : 1;  // of a run
+    // rows of a run: eight at a time, which end with a line whatever the width
+    const int64_t rows = U * 1024 / pieces >= 8 ? U * 1024 / pieces / 8 * 8 : U * 1024 / pieces > 1 ? U * 1024 / pieces : 1;
     for (int64_t row0 = blockIdx.x * rows; row0 < n; row0 += gridDim.x * rows) {
         const uint32_t count = (uint32_t)(n - row0 < rows ? n - row0 : rows) * pieces;
         const CodeT *run = codes + row0 * stages;
@@ -341,7 +338,7 @@ static __global__ void __launch_bounds__(1024) k_rvq_recon_resident(int64_t n, i
                 if (l0 + 1024u * u < count) {
                     const rot_u32x4 o = {two(lo[u].x, lo[u].y), two(lo[u].z, lo[u].w), two(hi[u].x, hi[u].y), two(hi[u].z, hi[u].w)};
                     rot_u32x4 *p = to + (row[u] * dim8 + at[u]);
-                    if (G >= 32) __builtin_nontemporal_store(o, p);
+                    if (past_l2) __builtin_nontemporal_store(o, p);
                     else *p = o;
                 }
         }

@@ -10,6 +10,7 @@
 
 #include "ctx.hpp"
 #include "rvq_opq.hpp"
+#include "resident_rules.hpp"
 #include "procrustes_host.hpp"
 #include "polar.hpp"
 
@@ -157,13 +158,14 @@ int32_t rvq_encode(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int
         }
     }
     if (d_recon_f16) {
-        const int cols = vq::rvq_recon_columns(stages, k, dim);
+        const int cols = vq::rvq_recon_columns(n, stages, k, dim);
         if (vec4 && cols && n * dim >= (1 << 21) && (reinterpret_cast<uintptr_t>(d_recon_f16) & 15) == 0) {
             const size_t lds = sizeof(float) * (size_t)stages * k * cols;
             auto kern = vq::k_rvq_recon_resident<CodeT>;
             VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            const unsigned groups = cdiv(dim, cols), wgs = std::max(1u, 256u / groups);
+            // (up to 32 groups: a multiple of eight workgroups each, see the kernel)
+            const unsigned groups = cdiv(dim, cols), wgs = groups <= 32 ? 256u / groups / 8 * 8 : std::max(1u, 256u / groups);
             hipLaunchKernelGGL(kern, dim3(wgs, groups), dim3(1024), lds, st, n, dim, k, cols, d_codebooks,
                                (const CodeT *)d_codes, stages, (const uint8_t *)used, (vq::rot_u32x4 *)d_recon_f16);
         } else if (vec4 && (reinterpret_cast<uintptr_t>(d_recon_f16) & 7) == 0)
