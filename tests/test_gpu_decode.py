@@ -21,11 +21,13 @@ def ctx():
     (130_000, 9, 16, 5000), (4097, 2, 64, 700), (999, 5, 12, 300),                                  # a block too large: gather
     (87_401, 12, 8, 1024), (53_003, 20, 8, 2048), (262_145, 4, 8, 256), (52_429, 10, 8, 300),  # table in LDS: binary16
     (21_001, 25, 8, 200), (10_699, 49, 8, 11),
-    (87_401, 12, 4, 1024), (53_003, 20, 4, 2048), (33_000, 17, 4, 256), (175_001, 3, 4, 2000)])  # table in LDS: f32
+    (87_401, 12, 4, 1024), (53_003, 20, 4, 2048), (33_000, 17, 4, 256), (175_001, 3, 4, 2000),  # table in LDS: f32
+    # 60 million components and more: also centroids of several pieces, f16 and f32
+    (470_001, 8, 16, 256), (157_003, 12, 32, 256), (500_009, 5, 24, 40)])
 def test_decode(ctx, n, m, sd, k):
     rng = np.random.default_rng(n + k)
     cb = (rng.standard_normal((m, k, sd)) * 100).astype(F)
-    codes = rng.integers(0, k, (n, m))
+    codes = rng.integers(0, k, (n, m), dtype=np.uint16)
     want = cb[np.arange(m)[None, :], codes].reshape(n, m * sd)
     wide = k > 256
     dcodes, dcb = ctx.to_device(codes.astype(np.uint16 if wide else np.uint8)), ctx.to_device(cb)

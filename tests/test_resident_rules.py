@@ -32,17 +32,18 @@ def rules(tmp_path_factory):
 
 
 def _decode_ok(f16, n, m, sd, k, G):
+    pieces, block = sd // (8 if f16 else 4), k * sd * (2 if f16 else 4)
     groups = -(-m // G)
     for mg in {min(G, m), m - (groups - 1) * G}:  # a whole group, the last one
-        rows = min(n, max(1, 1024 * (4 if f16 else 8) // mg))  # of a run, as k_decode_resident takes them
-        if (rows - 1) * m + mg > 2 ** 32 or (groups > 1 and mg % 4):  # (64-byte shares)
+        rows = min(n, max(1, 1024 * (4 if f16 else 8) // (mg * pieces)))  # of a run, as k_decode_resident takes them
+        if (rows - 1) * m * pieces + mg * pieces > 2 ** 32 or (groups > 1 and mg * pieces % 4):  # (64-byte shares)
             return False
-    return sd == (8 if f16 else 4) and k * 16 * G <= 128 * 1024 and groups <= 65535
+    return sd % (8 if f16 else 4) == 0 and block * G <= 128 * 1024 and groups <= 65535
 
 
 def test_decode_at_the_limits(rules):
     rng = random.Random(1)
-    edges = [(1 << e) + d for e in range(8, 24) for d in (-1, 0, 1, 5)] + [2_097_156, 4_194_308]
+    edges = [(1 << e) + d for e in range(8, 24) for d in (-1, 0, 1, 5)] + [1064961, 532481, 8_388_612]
     cases = [(f16, n, m, sd, k) for f16 in (0, 1) for m in edges for sd in (4, 8, 16, 24) for k in (1, 5, 256, 2048)
              for n in (1, 2, 5, 100, 4096, 8192, 1 << 20, 1 << 31)]
     cases += [(rng.random() < 0.5, int(2 ** rng.uniform(0, 32)), int(2 ** rng.uniform(0, 24)), rng.choice([4, 8, 8, 16, 32, 100, 512]),
@@ -55,12 +56,14 @@ def test_decode_at_the_limits(rules):
 def test_decode_of_ordinary_sizes(rules):
     """(binary16, n, m, sub_dim, k): column blocks per group."""
     want = {(1, 1_000_000, 16, 8, 256): 16, (1, 300_000, 16, 8, 1024): 8, (0, 300_000, 16, 4, 1024): 8, (1, 200_000, 12, 8, 256): 12,
-            (1, 66_000, 20, 8, 2048): 4, (1, 262_144, 10, 8, 100): 10, (0, 4096, 2_097_156, 4, 2): 0, (1, 6, 500_000, 8, 2048): 0,
-            # shares of a row that end inside a half line, more than one piece to a centroid, few pieces, no room in LDS
-            (1, 1_000_000, 10, 8, 1024): 0, (1, 1_000_000, 17, 8, 2048): 0, (1, 130_000, 8, 16, 256): 0, (0, 300_000, 16, 8, 256): 0,
-            (1, 50_000, 16, 12, 256): 0, (1, 32_000, 16, 8, 256): 0, (1, 1_000_000, 16, 8, 2049): 0,
-            # a table that the vector cache holds
-            (1, 1_000_000, 16, 8, 16): 0, (0, 1_000_000, 16, 4, 200): 0, (0, 1_000_000, 16, 4, 256): 16}
+            (1, 66_000, 20, 8, 2048): 4, (1, 262_144, 10, 8, 100): 10, (1, 6, 500_000, 8, 2048): 0, (0, 4096, 8_388_612, 4, 1): 0,
+            # shares of a row that end inside a half line, few pieces, no room in LDS
+            (1, 1_000_000, 10, 8, 1024): 0, (1, 1_000_000, 17, 8, 2048): 0, (1, 32_000, 16, 8, 256): 0, (1, 1_000_000, 16, 8, 2049): 0,
+            # a table that the vector cache holds, also with rows beyond the memory-side cache
+            (1, 400_000, 16, 8, 16): 0, (0, 800_000, 16, 4, 200): 0, (0, 800_000, 16, 4, 256): 16, (1, 1_000_000, 16, 8, 16): 16,
+            # more than one piece to a centroid
+            (1, 130_000, 8, 16, 256): 0, (1, 1_000_000, 8, 16, 256): 8, (0, 400_000, 16, 8, 256): 0, (0, 1_000_000, 16, 8, 256): 16,
+            (0, 300_000, 16, 8, 512): 0, (0, 1_000_000, 16, 8, 512): 8, (1, 1_000_000, 10, 12, 256): 0}
     assert rules(list(want)) == list(want.values())
 
 

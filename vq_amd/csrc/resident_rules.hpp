@@ -8,30 +8,35 @@ namespace vq {
 
 constexpr int64_t kMaxGridY = 65535;  // workgroups in the second dimension of a grid
 
-// Column blocks per group of k_decode_resident; 0: the gather (k_decode_gather).
-// The table in LDS pays where a centroid is one 16-byte piece of the output and the codebook is more than the vector
-// cache holds, from 2^19 pieces on.  Gather -> table, f16 blocks of 8, output not in a cache: 1M x 16, k = 256 67 -> 50 us, 200,000 x 12
-// 12.0 -> 9.5, 1M x 10 41 -> 34; geometric means by table size 1.03 (1-4 KB), 0.97 (8 KB), 0.92 (16 KB), 0.84 (32), 0.80 (64-128); below
-// 2^19 pieces 1.08 (5.4 -> 5.8 us).  f32 blocks of 4: 1.1-1.2 up to 32 KB (200,000 x 12, k = 256 9.4 -> 12.3), 0.97 at 64 KB, 0.86
-// at 128.
+// Column blocks per group of k_decode_resident; 0: the gather (k_decode_gather).  Kernel times behind an assignment of
+// as many rows, gather -> table.
+// A centroid of one 16-byte piece of the output: the table in LDS once the codebook is more than the vector
+// cache holds, from 2^19 pieces on.  f16 blocks of 8: 200,000 x 12, k = 256 11.9 -> 9.6 us, 1M x 16, k = 256 91 -> 54; geometric
+// means 1.04 below 2^19 pieces, 0.96 (8 MB written), 0.85 (16 to 64 MB).  f32 blocks of 4: 1.1-1.2 with tables up to 32 KB, 0.97 at
+// 64 KB, 0.86 at 128.
+// More pieces, which the gather reads as one run of bytes: the gather, until the rows (240 MB of f32) leave
+// nothing of the output in the memory-side cache.  Stores that go to memory want the table's long runs, others do not:
+// f16 100,000 x 12 blocks of 32 1.05-1.3, from 60M elements on 0.65-0.88 (1M x 8 of 16, k = 256 71 -> 54); f32 1.05-1.3, then
+// 0.74-0.92 (1M x 16 of 8, k = 256 123 -> 104).
 // Where the blocks' tables exceed LDS a group's share of every row has to be whole 64-byte halves of lines, the stores
 // pass the caches: 1M x 16, k = 1024 (two groups) 75 -> 50, 300,000 x 32, k = 512 47 -> 31, 66,000 x 64, k = 2048 (64-byte shares) 32.6 ->
 // 22.3; with shares that end inside: 1M x 10, k = 1024 48 -> 121, 300,000 x 17, k = 2048, f32 30 -> 129.
-// Centroids of more than one piece are read by the gather as one run of bytes: 1M x 4 blocks of 32, k = 1024
-// 41 -> 51, 110,000 x 12 of 32, k = 16 14.6 -> 20.5 (geometric means 1.04-1.7 by width).
 // The last group may be short and its runs long: their places are counted in 32 bits.
 inline int decode_resident_blocks(bool f16, int64_t n, int m, int sd, int k) {
-    const int64_t table = (int64_t)k * 16 * m, room = 128 * 1024;
-    if (sd != (f16 ? 8 : 4) || n * m < (1 << 19) || table < (f16 ? 8 : 64) * 1024) return 0;
+    const int64_t line = (int64_t)sd * (f16 ? 2 : 4), pieces = line / 16, block = k * line, room = 128 * 1024;
+    if (line % 16 != 0 || block > room || n * m < (1 << 16)) return 0;
+    const bool beyond = n * m * sd >= 60'000'000;
     int64_t G = m;
-    if (table > room) {
-        G = room / ((int64_t)k * 16);
-        G = G >= 8 ? G / 8 * 8 : G / 4 * 4;
-        if (G == 0 || m % 4 != 0 || n * m < (1 << 20)) return 0;
+    if (block * m <= room) {
+        if (!beyond && (pieces > 1 || n * m < (1 << 19) || block * m < (f16 ? 8 : 64) * 1024)) return 0;
+    } else {
+        G = room / block;
+        if (G * line >= 128) G = G * line / 128 * 128 / line;
+        if (G < 1 || G * line % 64 != 0 || m * line % 64 != 0 || n * m < (1 << 20) || (pieces > 1 && !beyond)) return 0;
     }
     const int64_t groups = (m + G - 1) / G, last = m - (groups - 1) * G;
-    const int64_t rows = std::min<int64_t>(n, std::max<int64_t>(1, (f16 ? 4096 : 8192) / last));
-    if (groups > kMaxGridY || rows * m >= (1LL << 32)) return 0;
+    const int64_t rows = std::min<int64_t>(n, std::max<int64_t>(1, (f16 ? 4096 : 8192) / (last * pieces)));
+    if (groups > kMaxGridY || rows * m * pieces >= (1LL << 32)) return 0;
     return (int)G;
 }
 

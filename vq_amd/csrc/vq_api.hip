@@ -560,23 +560,25 @@ __global__ void __launch_bounds__(256) k_decode_vec4(const CodeT *__restrict__ c
     out[i] = o;
 }
 
-// Blocks whose centroid is ONE 16-byte piece of the output (eight f16 values, F16, or four f32), with the codebook table
-// resident in LDS: up to 128 KB, one workgroup of 1024 threads per compute unit walking over the output, two where the
-// table leaves room.  A wave's stores are consecutive bytes, its code reads consecutive
+// The same gather with the codebook table resident in LDS (up to 128 KB, one workgroup of 1024 threads per
+// compute unit walking over the output, two where the table leaves room): a thread makes one 16-byte piece of the
+// output per step, eight f16 values (F16; sub_dim a multiple of 8) or four f32 values (sub_dim a
+// multiple of 4), so a wave's stores are consecutive bytes, its code reads consecutive
 // bytes, and the centroid comes from LDS instead of a scattered read of the table through
 // the vector cache.  U pieces per thread are in flight.  blockIdx.y: a group of G column blocks, where the table
 // of all of them does not fit.  A workgroup takes runs of whole rows, so that a piece's place in its run is
-// divided in 32 bits; the stores pass the caches, so a group's share of a row has to fill its lines.
-// Bound by the stores (49.5 us for 256 MB: 1M x 16 blocks of 8, k = 1024); decode_resident_blocks has the gather's times.
+// divided in 32 bits; the stores pass the caches, so runs, and a group's share of a row, have to fill their lines.
+// Bound by the stores; decode_resident_blocks has its times and the gather's.
 template <bool F16, typename CodeT>
-__global__ void __launch_bounds__(1024) k_decode_resident(const CodeT *__restrict__ codes, int64_t n, int m,
+__global__ void __launch_bounds__(1024) k_decode_resident(const CodeT *__restrict__ codes, int64_t n, int m, int sd,
                                                           int k, int G, const float *__restrict__ cb,
                                                           vq::u32x4 *__restrict__ out) {
-    extern __shared__ __attribute__((aligned(16))) vq::u32x4 tab[];  // [blocks of the group * k]
+    extern __shared__ __attribute__((aligned(16))) vq::u32x4 tab[];  // [blocks of the group * k][pieces of a centroid]
     constexpr int U = F16 ? 4 : 8;  // pieces in flight per thread
+    const uint32_t pieces = F16 ? sd / 8 : sd / 4;  // 16-byte output pieces per centroid
     const int s0 = (int)blockIdx.y * G, mg = m - s0 < G ? m - s0 : G;
-    const uint32_t entries = (uint32_t)mg * k;
-    cb += (size_t)s0 * k * (F16 ? 8 : 4);
+    const uint32_t entries = (uint32_t)mg * k * pieces;
+    cb += (size_t)s0 * k * sd;
     for (uint32_t e = threadIdx.x; e < entries; e += 1024) {
         if constexpr (F16) {
             const float4 a = reinterpret_cast<const float4 *>(cb)[2 * (size_t)e];
@@ -590,25 +592,27 @@ __global__ void __launch_bounds__(1024) k_decode_resident(const CodeT *__restric
         }
     }
     __syncthreads();
-    const uint32_t per_row = (uint32_t)mg;
+    const uint32_t per_row = (uint32_t)mg * pieces;
     // rows of a run: eight at a time, which end with a line whatever m is
     const int64_t rows = U * 1024 / per_row >= 8 ? U * 1024 / per_row / 8 * 8 : U * 1024 / per_row > 1 ? U * 1024 / per_row : 1;
     for (int64_t row0 = blockIdx.x * rows; row0 < n; row0 += gridDim.x * rows) {
         const uint32_t count = (uint32_t)(n - row0 < rows ? n - row0 : rows) * per_row;
         const CodeT *run = codes + row0 * m + s0;
-        vq::u32x4 *to = out + row0 * m + s0;
+        vq::u32x4 *to = out + (row0 * m + s0) * pieces;
         for (uint32_t l0 = threadIdx.x; l0 < count; l0 += U * 1024) {
-            uint32_t at[U], entry[U];
+            uint32_t code[U], at[U], entry[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const uint32_t l = l0 + 1024u * u < count ? l0 + 1024u * u : l0;
-                const uint32_t row = l / per_row, s = l - row * per_row;
-                at[u] = row * (uint32_t)m + s;
-                entry[u] = s * (uint32_t)k + run[at[u]];
+                const uint32_t row = l / per_row, within = l - row * per_row;
+                const uint32_t s = pieces == 1 ? within : within / pieces;
+                code[u] = run[row * (uint32_t)m + s];
+                at[u] = row * (uint32_t)m * pieces + within;
+                entry[u] = s * (uint32_t)k * pieces + (within - s * pieces);
             }
             vq::u32x4 v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = tab[entry[u]];
+            for (int u = 0; u < U; ++u) v[u] = tab[entry[u] + code[u] * pieces];
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 if (l0 + 1024u * u < count) __builtin_nontemporal_store(v[u], to + at[u]);
@@ -645,7 +649,7 @@ int32_t launch_decode_resident(vq_ctx *ctx, const CodeT *d_codes, int64_t n, int
     *done = false;
     const int G = vq::decode_resident_blocks(F16, n, m, sd, k);
     if (G == 0) return VQ_OK;
-    const size_t lds = (size_t)k * 16 * G;
+    const size_t lds = (size_t)k * sd * (F16 ? 2 : 4) * G;
     if ((reinterpret_cast<uintptr_t>(d_codebooks) & 15) || (reinterpret_cast<uintptr_t>(d_out) & 63)) return VQ_OK;
     auto kern = k_decode_resident<F16, CodeT>;
     // the kernel's LDS limit and the number of compute units: asked for once per context and kernel
@@ -660,12 +664,12 @@ int32_t launch_decode_resident(vq_ctx *ctx, const CodeT *d_codes, int64_t n, int
         VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
         ctx->compute_units = cus > 0 ? cus : 1;
     }
-    const int64_t pieces = (int64_t)n * m;
+    const int64_t pieces = (int64_t)n * m * (F16 ? sd / 8 : sd / 4);
     const unsigned per_cu = lds <= 64 * 1024 ? 2u : 1u;
     const unsigned groups = cdiv(m, G);
     const unsigned wgs = (unsigned)std::min<int64_t>(std::max<int64_t>(1, (int64_t)ctx->compute_units * per_cu / groups),
                                                      cdiv(pieces, 4096 * groups));
-    hipLaunchKernelGGL(kern, dim3(wgs, groups), dim3(1024), lds, ctx->stream, d_codes, n, m, k, G, d_codebooks,
+    hipLaunchKernelGGL(kern, dim3(wgs, groups), dim3(1024), lds, ctx->stream, d_codes, n, m, sd, k, G, d_codebooks,
                        (vq::u32x4 *)d_out);
     VQ_HIP(ctx, hipGetLastError());
     *done = true;
