@@ -194,9 +194,12 @@ __device__ __forceinline__ int argmin_lds(const float (&x)[SD], const float *lds
 
 // One lane = one row, G consecutive column blocks per lane (G*SD floats in registers, G
 // codebooks in LDS).  blockIdx.x = tile * (m/G) + block group.
-template <int SD, int G, int METRIC, bool LBG>
-__global__ void __launch_bounds__(256) k_assign_static(AssignArgs a) {
+// PAD: blocks of sub_dim < SD floats, zeros behind them in the registers and in LDS.  A component that is zero on both
+// sides adds +0 to a sum that started at +0, so every distance keeps its bits.
+template <int SD, int G, int METRIC, bool LBG, bool PAD>
+__global__ void __launch_bounds__(256) k_assign_static(AssignArgs a, int sub_dim) {
     extern __shared__ float lds[];
+    const int sd = PAD ? sub_dim : SD;
     const int groups = a.m / G;
     const int sg = blockIdx.x % groups;
     const int64_t tile = blockIdx.x / groups;
@@ -213,9 +216,14 @@ __global__ void __launch_bounds__(256) k_assign_static(AssignArgs a) {
     }
     // codebooks of blocks s0..s0+G-1 are contiguous: G*k*SD floats
     {
-        const float *src = a.cb + (size_t)s0 * k * SD;
+        const float *src = a.cb + (size_t)s0 * k * sd;
         const int total = G * k * SD;
-        for (int i = threadIdx.x; i < total; i += 256) lds[i] = src[i];
+        for (int i = threadIdx.x; i < total; i += 256) {
+            if constexpr (PAD)
+                lds[i] = i % SD < sd ? src[i / SD * sd + i % SD] : 0.0f;
+            else
+                lds[i] = src[i];
+        }
         if constexpr (METRIC == M_COS) {
             const float *cn = a.cnorm + (size_t)s0 * k;
             for (int i = threadIdx.x; i < G * k; i += 256) lds_cn[i] = cn[i];
@@ -228,8 +236,16 @@ __global__ void __launch_bounds__(256) k_assign_static(AssignArgs a) {
 
     float x[G][SD];
     {
-        const float *xr = a.x + row * a.ld + (int64_t)s0 * SD;
-        if constexpr ((G * SD) % 4 == 0) {
+        const float *xr = a.x + row * a.ld + (int64_t)s0 * sd;
+        if constexpr (PAD) {
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int t = 0; t < SD; ++t) {  // unconditional loads, all in flight together
+                    const float v = xr[g * sd + (t < sd ? t : sd - 1)];
+                    x[g][t] = t < sd ? v : 0.0f;
+                }
+        } else if constexpr ((G * SD) % 4 == 0) {
             if ((a.ld % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.x) & 15) == 0)) {
                 const float4 *p = reinterpret_cast<const float4 *>(xr);
                 float *xf = &x[0][0];
@@ -279,101 +295,6 @@ __global__ void __launch_bounds__(256) k_assign_static(AssignArgs a) {
     if constexpr (!LBG && G == 4) {
         // m % 4 == 0 here, so the 4 codes of this lane are one aligned 32-bit word
         *reinterpret_cast<uint32_t *>(a.codes + row * a.m + s0) = packed;
-    }
-}
-
-// Fallback for any sub_dim: one lane = one row, one column block per blockIdx.y, sub-vector
-// re-read from memory for every group of 4 centroids; centroids read through wave-uniform
-// addresses.  Same operation order as above.
-template <int METRIC, bool LBG>
-__global__ void __launch_bounds__(256) k_assign_dyn(AssignArgs a, int sd) {
-    const int s = blockIdx.y;
-    if constexpr (LBG) {
-        if (block_done(a, s)) return;
-    }
-    const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (row >= a.n) return;
-    const int k = a.k;
-    const float *__restrict__ xr = a.x + row * a.ld + (int64_t)s * sd;
-    const float *__restrict__ cb = a.cb + (size_t)s * k * sd;
-    const float *__restrict__ cn = a.cnorm ? a.cnorm + (size_t)s * k : nullptr;
-    int best = 0;
-    float bd = 0.0f, pd = __builtin_inff();
-    float na = 0.0f;
-    if constexpr (METRIC == M_COS) {
-        float sa = 0.0f;
-        for (int t = 0; t < sd; ++t) {
-            float p = xr[t] * xr[t];
-            sa = sa + p;
-        }
-        na = sqrtf(sa);
-    }
-    for (int j0 = 0; j0 < k; j0 += 4) {
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        const int jn = (k - j0 < 4) ? (k - j0) : 4;
-        for (int t = 0; t < sd; ++t) {
-            float xv = xr[t];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (u < jn) {
-                    float cv = cb[(size_t)(j0 + u) * sd + t];
-                    if constexpr (METRIC == M_COS) {
-                        float p = xv * cv;
-                        acc[u] = acc[u] + p;
-                    } else if constexpr (METRIC == M_L1) {
-                        float d = xv - cv;
-                        acc[u] = acc[u] + fabsf(d);
-                    } else {
-                        float d = xv - cv;
-                        float p = d * d;
-                        acc[u] = acc[u] + p;
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (u < jn) {
-                float d = acc[u];
-                if constexpr (METRIC == M_COS) {
-                    float nb = cn[j0 + u];
-                    float den = na * nb;
-                    float q = d / den;
-                    d = 1.0f - q;
-                    d = (na == 0.0f || nb == 0.0f) ? 1.0f : d;
-                }
-                bool upd = (j0 + u == 0) || (d < bd);
-                if constexpr (METRIC == M_EUCLID) pd = (upd && (j0 + u) != 0) ? bd : pd;
-                bd = upd ? d : bd;
-                best = upd ? (j0 + u) : best;
-            }
-        }
-    }
-    if constexpr (METRIC == M_EUCLID) {
-        float sr = sqrtf(bd);
-        if (sqrtf(pd) == sr) {
-            for (int j = 0; j < best; ++j) {
-                float acc = 0.0f;
-                for (int t = 0; t < sd; ++t) {
-                    float d = xr[t] - cb[(size_t)j * sd + t];
-                    float p = d * d;
-                    acc = acc + p;
-                }
-                if (sqrtf(acc) == sr) {
-                    best = j;
-                    break;
-                }
-            }
-        }
-    }
-    if constexpr (LBG) {
-        uint8_t *p = a.codes + (size_t)s * a.n + row;
-        if (*p != (uint8_t)best) {
-            *p = (uint8_t)best;
-            mark_changed(a.changed + s);
-        }
-    } else {
-        a.codes[row * a.m + s] = (uint8_t)best;
     }
 }
 

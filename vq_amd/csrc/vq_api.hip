@@ -45,6 +45,8 @@ std::string &create_error() {
 
 using namespace vqh;
 
+static bool lbg_small(int64_t n, int m, int sd, int k);
+
 namespace {
 
 // ---- the scratch of vq_assign_noalloc --------------------------------------------------------
@@ -74,11 +76,11 @@ template <int METRIC, bool LBG>
 int32_t launch_wide_exact(vq_ctx *ctx, const vq::AssignArgs &a, int sd, const uint32_t *list,
                           const uint32_t *count, const uint2 *pairs = nullptr, const uint32_t *pair_count = nullptr);
 
-template <int SD, int G, int METRIC, bool LBG>
-int32_t launch_static(vq_ctx *ctx, const vq::AssignArgs &a) {
+template <int SD, int G, int METRIC, bool LBG, bool PAD>
+int32_t launch_static(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     size_t lds = (size_t)G * a.k * SD * sizeof(float);
     if (METRIC == vq::M_COS) lds += (size_t)G * a.k * sizeof(float);
-    auto kern = vq::k_assign_static<SD, G, METRIC, LBG>;
+    auto kern = vq::k_assign_static<SD, G, METRIC, LBG, PAD>;
     if (lds > 48 * 1024)
         VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -87,53 +89,56 @@ int32_t launch_static(vq_ctx *ctx, const vq::AssignArgs &a) {
     if (blocks > 0x7fffffffLL) return fail(ctx, VQ_ERR_UNSUPPORTED, "grid too large");
     {
         ProfSpan sp(ctx, VQ_PROF_ASSIGN_KERNEL);
-        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), lds, ctx->stream, a);
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), lds, ctx->stream, a, sd);
     }
     VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;
 }
 
-template <int SD, int METRIC, bool LBG>
-int32_t launch_static_g(vq_ctx *ctx, const vq::AssignArgs &a) {
+template <int SD, int METRIC, bool LBG, bool PAD = false>
+int32_t launch_static_g(vq_ctx *ctx, const vq::AssignArgs &a, int sd = SD) {
     // G column blocks per lane: as many as keep the lane's floats within 32 registers and the
     // codebooks within 64 KB of LDS.
     size_t per = (size_t)a.k * SD * sizeof(float) + (METRIC == vq::M_COS ? a.k * sizeof(float) : 0);
     if constexpr (SD * 4 <= 32) {
-        if (a.m % 4 == 0 && 4 * per <= 64 * 1024) return launch_static<SD, 4, METRIC, LBG>(ctx, a);
+        if (a.m % 4 == 0 && 4 * per <= 64 * 1024) return launch_static<SD, 4, METRIC, LBG, PAD>(ctx, a, sd);
     }
     if constexpr (SD * 2 <= 32) {
-        if (a.m % 2 == 0 && 2 * per <= 64 * 1024) return launch_static<SD, 2, METRIC, LBG>(ctx, a);
+        if (a.m % 2 == 0 && 2 * per <= 64 * 1024) return launch_static<SD, 2, METRIC, LBG, PAD>(ctx, a, sd);
     }
-    return launch_static<SD, 1, METRIC, LBG>(ctx, a);
+    return launch_static<SD, 1, METRIC, LBG, PAD>(ctx, a, sd);
+}
+
+// The register width that k_assign_static holds blocks of sd floats in (0: it does not take them): their own, or
+// the next of a few widths, whose last floats are zeros.  (256 centroids of 48 floats are 48 KB of LDS.)
+int static_width(int sd) {
+    return sd <= 6 ? sd : sd <= 8 ? 8 : sd <= 12 ? 12 : sd <= 16 ? 16 : sd <= 24 ? 24 : sd <= 32 ? 32 : sd <= 48 ? 48 : 0;
 }
 
 template <int METRIC, bool LBG>
 int32_t launch_assign_m(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
-    size_t per = (size_t)a.k * sd * sizeof(float) + a.k * sizeof(float);
-    if (per <= 64 * 1024) {
-        switch (sd) {
-        case 1: return launch_static_g<1, METRIC, LBG>(ctx, a);
-        case 2: return launch_static_g<2, METRIC, LBG>(ctx, a);
-        case 3: return launch_static_g<3, METRIC, LBG>(ctx, a);
-        case 4: return launch_static_g<4, METRIC, LBG>(ctx, a);
-        case 5: return launch_static_g<5, METRIC, LBG>(ctx, a);
-        case 6: return launch_static_g<6, METRIC, LBG>(ctx, a);
-        case 8: return launch_static_g<8, METRIC, LBG>(ctx, a);
-        case 12: return launch_static_g<12, METRIC, LBG>(ctx, a);
-        case 16: return launch_static_g<16, METRIC, LBG>(ctx, a);
-        case 32: return launch_static_g<32, METRIC, LBG>(ctx, a);
-        default: break;
-        }
+    const bool pad = static_width(sd) != sd;
+    switch (static_width(sd)) {
+    case 1: return launch_static_g<1, METRIC, LBG>(ctx, a);
+    case 2: return launch_static_g<2, METRIC, LBG>(ctx, a);
+    case 3: return launch_static_g<3, METRIC, LBG>(ctx, a);
+    case 4: return launch_static_g<4, METRIC, LBG>(ctx, a);
+    case 5: return launch_static_g<5, METRIC, LBG>(ctx, a);
+    case 6: return launch_static_g<6, METRIC, LBG>(ctx, a);
+#define PADDED(W) \
+    case W: return pad ? launch_static_g<W, METRIC, LBG, true>(ctx, a, sd) : launch_static_g<W, METRIC, LBG>(ctx, a)
+    PADDED(8);
+    PADDED(12);
+    PADDED(16);
+    PADDED(24);
+    PADDED(32);
+    PADDED(48);
+#undef PADDED
+    default: break;
     }
     if (a.m > 65535) return fail(ctx, VQ_ERR_UNSUPPORTED, "m too large for the generic kernel");
-    if (sd >= 24) {
-        ProfSpan sp(ctx, VQ_PROF_ASSIGN_KERNEL);
-        return launch_wide_exact<METRIC, LBG>(ctx, a, sd, nullptr, nullptr);
-    }
-    hipLaunchKernelGGL((vq::k_assign_dyn<METRIC, LBG>), dim3(cdiv(a.n, 256), (unsigned)a.m),
-                       dim3(256), 0, ctx->stream, a, sd);
-    VQ_HIP(ctx, hipGetLastError());
-    return VQ_OK;
+    ProfSpan sp(ctx, VQ_PROF_ASSIGN_KERNEL);
+    return launch_wide_exact<METRIC, LBG>(ctx, a, sd, nullptr, nullptr);
 }
 
 // 8-float column blocks: bf16-split scores on the matrix cores, undecided rows resolved in the
@@ -463,28 +468,36 @@ template <int METRIC, bool LBG> int32_t launch_mfma16(vq_ctx *ctx, const vq::Ass
 // The width to pad every column block to so that the matrix-core kernels take the shape (squared L2,
 // Euclidean, cosine; 0: they take it as it is, or padding does not pay).  fit: for the passes of a fit,
 // which pads its rows once and whose update then streams blocks of 8 as well.
-// Widths without a register kernel always gain (10 floats, 60,007 rows x 10 blocks, k = 200: 3.94 ms per
-// pass on k_assign_dyn).  k_assign_static does 3 sd + 1 vector instructions per row and centroid (cosine:
-// about 2 sd + 26), the padded kernels about 600 per row and block and half the bytes more to read; the
-// lines below are where the two took the same time at 20,000-600,000 rows, 12 and 25 blocks.  One float
-// per block leaves most rows to the exact path of the matrix-core kernels: never.
+// k_assign_static does 3 w + 1 vector instructions per row and centroid (cosine: about 2 w + 26; w: its register
+// width), the padded kernels about 600 per row and block and half the bytes more to read.  Its own widths: the
+// lines below are where the two took the same time at 20,000-600,000 rows, 12 and 25 blocks; one float
+// per block leaves most rows to the exact path of the matrix-core kernels: never.  Widths that it holds with zeros
+// behind them (150,000 rows x 12 blocks, an encode, microseconds padded against static): 7 floats k = 31 85 / 72, 48
+// 86 / 87, 80 89 / 117; 10 floats k = 48 128 / 115, 80 134 / 152; 20 floats 195 / 156, 208 / 230; 25 floats 289 / 243,
+// 298 / 331; cosine, 11 blocks: 7 floats k = 31 87 / 84, 48 87 / 100, 15 floats 136 / 119, 137 / 144, 20 floats k = 48 165 / 140, 64
+// 168 / 174: so the line is a number of centroids, about the same for all of them.  The passes of a fit lie no
+// further apart, but its update needs fewer launches where the padded blocks make it a small one (12,000 x 12
+// blocks of 10, k = 24, six iterations: 241 against 705 us).  Widths that neither takes always gain.
 int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bool fit) {
     if (ctx->assign_path == 1 || ctx->no_alloc || metric < VQ_SQEUCLIDEAN || metric > VQ_COSINE) return 0;
-    if (sd == 1 || a.k < 32 || a.k > vq::kMaxK || a.m > 65535) return 0;
+    if (sd == 1 || a.k < 2 || a.k > vq::kMaxK || a.m > 65535) return 0;
     if (mfma_applicable<vq::M_SQ, true>(ctx, a, sd) || mfma16_applicable<vq::M_SQ, true>(ctx, a, sd) ||
         mfma_wide_applicable<vq::M_SQ, true>(ctx, a, sd))
         return 0;
     const int sdp = (sd + 7) / 8 * 8;
     // the limits of those kernels
     if ((int64_t)a.m * sdp > (1 << 20) || sdp > (1 << 16) || a.n * a.m >= (1LL << 32)) return 0;
-    const bool has_static = (sd <= 6 || sd == 12 || sd == 16 || sd == 32) && ((size_t)a.k * (sd + 1)) * sizeof(float) <= 64 * 1024;
-    if (has_static) {
+    const int w = static_width(sd);
+    if (fit && sd != sdp && lbg_small(a.n, a.m, sdp, a.k)) return sdp;
+    if (w == sd) {
         const int cost = a.k * (metric == VQ_COSINE ? 2 * sd + 26 : 3 * sd + 1);
         if (metric == VQ_COSINE ? cost < (sd < 8 ? 1500 : 3500)
             : sd > 8            ? cost < (fit ? 4700 : 3500)
             : fit               ? a.k < 40
                                 : sd == 2 || cost < 1600 || (a.m % 4 != 0 && (cost - 1600) * (double)(a.n * a.m) < 5e8))
             return 0;
+    } else if (w && a.k < (w > 16 ? 60 : metric == VQ_COSINE ? (w == 8 ? 32 : 40) : w == 8 ? 48 : 60)) {
+        return 0;
     }
     return sdp;
 }
@@ -519,13 +532,13 @@ int32_t launch_assign(vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, 
         return launch_mfma_wide<vq::M_SQ, LBG>(ctx, a, sd);
     if (metric == VQ_EUCLIDEAN && mfma_wide_applicable<vq::M_EUCLID, LBG>(ctx, a, sd))
         return launch_mfma_wide<vq::M_EUCLID, LBG>(ctx, a, sd);
-    switch (metric) {
-    case VQ_SQEUCLIDEAN: return launch_assign_m<vq::M_SQ, LBG>(ctx, a, sd);
-    case VQ_EUCLIDEAN: return launch_assign_m<vq::M_EUCLID, LBG>(ctx, a, sd);
-    case VQ_COSINE: return launch_assign_m<vq::M_COS, LBG>(ctx, a, sd);
-    case VQ_MANHATTAN: return launch_assign_m<vq::M_L1, LBG>(ctx, a, sd);
-    default: return fail(ctx, VQ_ERR_UNSUPPORTED, "metric %d has no kernel", metric);
+    if (metric == VQ_SQEUCLIDEAN) return launch_assign_m<vq::M_SQ, LBG>(ctx, a, sd);
+    if constexpr (!LBG) {  // the passes of a fit are squared Euclidean
+        if (metric == VQ_EUCLIDEAN) return launch_assign_m<vq::M_EUCLID, false>(ctx, a, sd);
+        if (metric == VQ_COSINE) return launch_assign_m<vq::M_COS, false>(ctx, a, sd);
+        if (metric == VQ_MANHATTAN) return launch_assign_m<vq::M_L1, false>(ctx, a, sd);
     }
+    return fail(ctx, VQ_ERR_UNSUPPORTED, "metric %d has no kernel", metric);
 }
 
 template <typename CodeT>
