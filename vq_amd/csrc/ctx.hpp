@@ -266,6 +266,9 @@ bool assign_pending_fusable(const vq_ctx *ctx, int32_t metric, const float *d_x,
 int encode_pad_width(const vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd,
                      int32_t k, const float *d_codebooks);
 void pad_blocks(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t sdp, float *d_y);
+// ... and back: n rows of sd floats from rows of sdp.
+void unpad_rows(vq_ctx *ctx, const float *d_y, int64_t n, int32_t sd, int32_t sdp, float *d_x);
+constexpr size_t kPadKeep = 2u << 30;  // bytes that the context keeps of a padded copy of a call's rows
 // Turns to the other set of counters of undecided pairs: this pass's (cleared by the pass before), and the
 // next pass's, which this pass clears.
 int32_t next_counters(vq_ctx *ctx, uint32_t **now, uint32_t **next);

@@ -1098,7 +1098,8 @@ static __global__ void __launch_bounds__(64) k_seg_select_pick(uint32_t *__restr
 // element winning (Iterator::max_by, src/tsvq.rs:102-106); one thread per segment.
 // The same launch starts the radix select of the middle values: bins cleared, ranks of the two
 // targets of every segment (the lower and the upper middle).  Grid over nseg * 512 bins.
-static __global__ void k_seg_argmax_last(const float *__restrict__ var, int nseg, int dim, int *__restrict__ sdim,
+// var: rows of `stride` values, the first dim of them the row's components (padded rows: zeros behind them).
+static __global__ void k_seg_argmax_last(const float *__restrict__ var, int nseg, int dim, int stride, int *__restrict__ sdim,
                                          const uint2 *__restrict__ seg_range, SegSelect *__restrict__ sel,
                                          uint32_t *__restrict__ hist) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1110,7 +1111,7 @@ static __global__ void k_seg_argmax_last(const float *__restrict__ var, int nseg
         sel[2 * i] = SegSelect{0u, (c % 2 == 0) ? c / 2 - 1 : c / 2};
         sel[2 * i + 1] = SegSelect{0u, c / 2};
     }
-    const float *v = var + (size_t)i * dim;
+    const float *v = var + (size_t)i * stride;
     int best = 0;
     float vb = v[0];
     for (int t0 = 1; t0 < dim; t0 += 16) {
@@ -1151,7 +1152,7 @@ inline size_t split_wg_lds(uint32_t longest) { return sizeof(uint32_t) * ((size_
 
 static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__restrict__ perm,
                                                               const uint2 *__restrict__ seg_range,
-                                                              const float *__restrict__ var, int dim,
+                                                              const float *__restrict__ var, int dim, int stride,
                                                               const float *__restrict__ x, int64_t ld,
                                                               int *__restrict__ split_dim, float *__restrict__ median,
                                                               uint32_t *__restrict__ nleft, uint32_t *__restrict__ perm_out) {
@@ -1164,7 +1165,7 @@ static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__
     // NaN or what follows one is always taken.  A run of values acts on what came before as its own result
     // does, unless it holds a NaN: then it decides alone; so runs compose in order, one per lane.
     if (wave == 0) {
-        const float *v = var + (size_t)g * dim;
+        const float *v = var + (size_t)g * stride;
         const int per = (dim + 63) / 64, t0 = lane * per, t1 = t0 + per < dim ? t0 + per : dim;
         int best = t0;
         float vb = t0 < dim ? v[t0] : 0.0f;

@@ -502,8 +502,6 @@ int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bo
     return sdp;
 }
 
-constexpr size_t kPadKeep = 2u << 30;    // bytes that the context keeps of a fit's padded copy of its rows
-
 void launch_pad(vq_ctx *ctx, const float *x, int64_t n, int64_t ld, int m, int sd, int sdp, float *y) {
     hipLaunchKernelGGL(vq::k_pad_blocks, dim3(cdiv(n * m * (sdp / 4), 1024)), dim3(256), 0, ctx->stream, x, n, ld, m, sd,
                        sdp, y);
@@ -794,6 +792,10 @@ int encode_pad_width(const vq_ctx *ctx, int32_t metric, const float *d_x, int64_
 
 void pad_blocks(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t sdp, float *d_y) {
     launch_pad(ctx, d_x, n, ld, m, sd, sdp, d_y);
+}
+
+void unpad_rows(vq_ctx *ctx, const float *d_y, int64_t n, int32_t sd, int32_t sdp, float *d_x) {
+    hipLaunchKernelGGL(vq::k_unpad_rows, dim3(cdiv(n * sd, 256)), dim3(256), 0, ctx->stream, d_y, n, sd, sdp, d_x);
 }
 
 int32_t next_counters(vq_ctx *ctx, uint32_t **now, uint32_t **next) {
@@ -1255,9 +1257,7 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
             launch_pad(ctx, d_x, n, ld, m, sd, sdp, px);
             rc = lbg_fit_run(ctx, px, n, (int64_t)m * sdp, m, sdp, k, max_iters, h_init_idx, h_reseed_stream, n_reseed,
                              pcb, h_iters_run, h_reseeds_used, nullptr, nullptr, [&] {
-                                 hipLaunchKernelGGL(vq::k_unpad_rows, dim3(cdiv((int64_t)m * k * sd, 256)), dim3(256), 0,
-                                                    ctx->stream, (const float *)pcb, (int64_t)m * k, sd, sdp,
-                                                    d_codebooks);
+                                 unpad_rows(ctx, pcb, (int64_t)m * k, sd, sdp, d_codebooks);
                              });
         }
         // a large copy is not held for later calls (taking 2.3 GB again costs a fit of 1,500,000 x 96 in

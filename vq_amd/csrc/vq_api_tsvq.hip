@@ -126,6 +126,16 @@ int32_t vq_tsvq_build_kmeans(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
     return tsvq_build_impl(ctx, d_x, n, ld, dim, max_depth, &km, out);
 }
 
+// Levels whose longest node is no longer than this: a workgroup per node (k_seg_variance_wg, 11 ns per row of
+// 128 and node, one launch) instead of the composed maps (four launches, 115 us at one node of 100,000 rows,
+// 62 at 16 nodes, 275 at 512, where the walks over many short columns cost most): 16 nodes of 6,250 rows
+// 78 and 62 us, 32 of 3,125 44 and 71, 512 of 195 22 and 275
+constexpr uint32_t kVarWgRows = 4096;
+
+// The build on validated arguments.  real_dim: the components that count; the others, up to dim, are zeros.
+static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t dim, int32_t real_dim,
+                               int32_t max_depth, const KmOpts *km, vq_tree **out);
+
 static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t dim, int32_t max_depth,
                                const KmOpts *km, vq_tree **out) {
     if (!ctx || !out) return VQ_ERR_INVALID_ARG;
@@ -134,6 +144,33 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     if (!d_x || n < 0 || dim <= 0 || ld < dim || max_depth < 0) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
     if (n >= (1LL << 31)) return fail(ctx, VQ_ERR_UNSUPPORTED, "n must be below 2^31");
     VQ_HIP(ctx, hipSetDevice(ctx->device));
+    // The variances are made by kernels for rows of whole groups of eight components (the composed maps) or of whole,
+    // aligned 16-byte pieces (k_seg_variance_wg).  Other rows are copied once with zeros behind them, for all levels: a
+    // column of zeros has the variance 0 and takes no part in the choice of the split dimension.  Builds of nine
+    // levels over the rows as they are (a lane per column that adds its squares one after the other; whole pieces: a
+    // workgroup per node) against the copy: 600,000 x 50 55.7 -> 2.6 ms, 20,000 2.17 -> 0.83, 2,000 0.585 -> 0.605; 600,000 x
+    // 100 17.7 -> 3.3 ms, 20,000 1.16 -> 0.88, 5,000 0.66 -> 0.71.
+    const bool whole = dim % 4 == 0 && dim <= 1024 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;
+    if (!km && dim % 8 != 0 && dim < (1 << 20) && n > (whole ? 2 * (int64_t)kVarWgRows : (int64_t)kVarWgRows / 2)) {
+        const int32_t dimp = (dim + 7) / 8 * 8;
+        int32_t rc = ensure(ctx, ctx->pad_x, sizeof(float) * (size_t)n * dimp);
+        if (rc == VQ_OK) {
+            float *px = (float *)ctx->pad_x.p;
+            pad_blocks(ctx, d_x, n, ld, 1, dim, dimp, px);
+            rc = tsvq_build_rows(ctx, px, n, dimp, dimp, dim, max_depth, km, out);
+        }
+        if (rc == VQ_ERR_OOM || ctx->pad_x.cap > kPadKeep) {  // a large copy is not held for later calls
+            const int32_t gone = release(ctx, ctx->pad_x);
+            if (rc == VQ_OK && gone != VQ_OK) return gone;  // (the tree is the caller's)
+        }
+        if (rc != VQ_ERR_OOM) return rc;  // no room for the copy beside the workspace: the rows as they are, the same tree
+    }
+    return tsvq_build_rows(ctx, d_x, n, ld, dim, dim, max_depth, km, out);
+}
+
+static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t dim, int32_t real_dim,
+                               int32_t max_depth, const KmOpts *km, vq_tree **out) {
+    const bool padded = real_dim != dim;
     hipStream_t st = ctx->stream;
 
     // workspace: two row-id lists, column values, flags, scan
@@ -145,11 +182,6 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     VQ_TRY(ensure(ctx, ctx->tmp_f, sizeof(uint32_t) * (size_t)n));
     // two-step variance (squares on the whole GPU, then the chains): dim a multiple of 8, and room
     // for a level's squares with every node starting on its own group of 32 positions
-    // levels whose longest node is no longer than this: a workgroup per node (k_seg_variance_wg, 11 ns per row of
-    // 128 and node, one launch) instead of the composed maps (four launches, 115 us at one node of 100,000 rows,
-    // 62 at 16 nodes, 275 at 512, where the walks over many short columns cost most): 16 nodes of 6,250 rows
-    // 78 and 62 us, 32 of 3,125 44 and 71, 512 of 195 22 and 275
-    constexpr uint32_t kVarWgRows = 4096;
     constexpr int64_t kLeafWgSums = 65536;  // a lane per sum fills half of the chip: both take the same time there
     constexpr int kChainSegs = 2048;  // levels with more nodes than this take the other kernels
     const bool var_chain = dim % 8 == 0;
@@ -172,7 +204,7 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
 
     vq_tree *T = new vq_tree;
     T->device = ctx->device;
-    T->dim = dim;
+    T->dim = real_dim;
     std::vector<Seg> level{{0, 0u, (uint32_t)n, 1}};
     T->h_left.push_back(-1);
     T->h_right.push_back(-1);
@@ -544,12 +576,12 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                 SP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_seg_split_wg),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             hipLaunchKernelGGL(vq::k_seg_split_wg, dim3((unsigned)ns), dim3(longest > 1024 ? 1024u : 256u), lds, st, perm,
-                               (const uint2 *)d_range, (const float *)d_var, dim, d_x, ld, d_sdim, d_median, d_nleft, perm2);
+                               (const uint2 *)d_range, (const float *)d_var, real_dim, dim, d_x, ld, d_sdim, d_median, d_nleft, perm2);
             SP_HIP(hipGetLastError());
         } else {
         // split dimension on the device (src/tsvq.rs:102-106); read back with the left counts below
         hipLaunchKernelGGL(vq::k_seg_argmax_last, dim3(cdiv((int64_t)ns * 512, 256)), dim3(256), 0, st,
-                           (const float *)d_var, ns, dim, (int *)d_sdim, (const uint2 *)d_range, (vq::SegSelect *)d_sel,
+                           (const float *)d_var, ns, real_dim, dim, (int *)d_sdim, (const uint2 *)d_range, (vq::SegSelect *)d_sel,
                            (uint32_t *)d_hist);
         // split column, middle values by radix select (src/tsvq.rs:109-117)
         hipLaunchKernelGGL(vq::k_seg_gather_col, dim3(cdiv(n, 256)), dim3(256), 0, st, perm, n,
@@ -620,9 +652,22 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
         --depth_left;
     }
     T->n_nodes = (int32_t)T->h_left.size();
-    T->h_centroids.resize((size_t)T->n_nodes * dim);
-    if (means_arena)
-        LV_HIP(hipMemcpyAsync(T->h_centroids.data(), ctx->tsvq_means.p, sizeof(float) * (size_t)T->n_nodes * dim,
+    T->h_centroids.resize((size_t)T->n_nodes * real_dim);
+    const float *d_nodes = means_arena ? (const float *)ctx->tsvq_means.p : nullptr;
+    if (padded) {
+        rc = ensure(ctx, ctx->pad_cb, sizeof(float) * (size_t)T->n_nodes * real_dim);
+        if (rc != VQ_OK) {
+            free_means();
+            return cleanup_fail(rc);
+        }
+        float *real = (float *)ctx->pad_cb.p;
+        for (auto &lm : level_means)
+            unpad_rows(ctx, (const float *)lm.d, lm.nseg, real_dim, dim, real + (size_t)lm.first_node * real_dim);
+        LV_HIP(hipGetLastError());
+        d_nodes = real;
+    }
+    if (d_nodes)
+        LV_HIP(hipMemcpyAsync(T->h_centroids.data(), d_nodes, sizeof(float) * (size_t)T->n_nodes * real_dim,
                               hipMemcpyDeviceToHost, st));
     else
         for (auto &lm : level_means)
@@ -631,7 +676,7 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     LV_HIP(hipStreamSynchronize(st));
 #undef LV_HIP
 #undef SP_HIP
-    rc = tree_to_device(ctx, T, means_arena ? (const float *)ctx->tsvq_means.p : nullptr);
+    rc = tree_to_device(ctx, T, d_nodes);
     free_means();
     if (rc != VQ_OK) return cleanup_fail(rc);
     *out = T;
