@@ -1598,12 +1598,18 @@ __global__ void __launch_bounds__(512) k_tsvq_descend_reg(const float *__restric
 // reference, huge ones overflow), non-finite values (they fail the comparison) — is decided for that
 // lane by the two sums in the reference's order, read from global memory.  Manhattan has no such form
 // and keeps the two-centroid kernel.
-constexpr float kDescendCosMargin = 600.0f * 5.9604644775390625e-08f;
-constexpr float kDescendL2Margin = 300.0f * 5.9604644775390625e-08f;
+// With D components the bounds are (4 D + 15) u and (2 D + 12) u; wider rows take margins that grow with them
+// (600 u and 300 u at 128).
+__host__ __device__ inline float descend_cos_margin(int dim) {
+    return (float)(4 * (dim > 128 ? dim : 128) + 88) * 5.9604644775390625e-08f;
+}
+__host__ __device__ inline float descend_l2_margin(int dim) {
+    return (float)(2 * (dim > 128 ? dim : 128) + 44) * 5.9604644775390625e-08f;
+}
 
 // Tables for the nodes below kTopNodes, one wave per node: w[node][DIM], and per node
-//   cosine: sc[node] = kDescendCosMargin, or +inf when a child's norm is outside [1e-15, 1e15]
-//   L2:     sc[2 node] = b, sc[2 node + 1] = kDescendL2Margin * s (+inf when s is not in [1e-30, 1e30])
+//   cosine: sc[node] = descend_cos_margin, or +inf when a child's norm is outside [1e-15, 1e15]
+//   L2:     sc[2 node] = b, sc[2 node + 1] = descend_l2_margin * s (+inf when s is not in [1e-30, 1e30])
 // Nodes without two children get zeros and +inf (they are never consulted).
 template <bool COS>
 static __global__ void __launch_bounds__(64) k_tsvq_wtable(const float *__restrict__ cen,
@@ -1635,7 +1641,7 @@ static __global__ void __launch_bounds__(64) k_tsvq_wtable(const float *__restri
             w[(size_t)node * dim + t] = a - b;
         }
         const bool ok = nl >= 1e-15f && nl <= 1e15f && nr >= 1e-15f && nr <= 1e15f;
-        if (lane == 0) sc[node] = ok ? kDescendCosMargin : inf;
+        if (lane == 0) sc[node] = ok ? descend_cos_margin(dim) : inf;
     } else {
         double sl = 0.0, sr = 0.0;
         for (int t = lane; t < dim; t += 64) {
@@ -1653,7 +1659,7 @@ static __global__ void __launch_bounds__(64) k_tsvq_wtable(const float *__restri
             const double s = 2.0 * (sl + sr);
             const bool ok = s >= 1e-30 && s <= 1e30;  // false for NaN
             sc[2 * node] = (float)(sr - sl);
-            sc[2 * node + 1] = ok ? (float)(s * 1.000001) * kDescendL2Margin : inf;
+            sc[2 * node + 1] = ok ? (float)(s * 1.000001) * descend_l2_margin(dim) : inf;
         }
     }
 }
@@ -1722,7 +1728,7 @@ __global__ void __launch_bounds__(512) k_tsvq_descend_w(const float *__restrict_
         if constexpr (COS)
             mrow = (na >= 1e-15f && na <= 1e15f) ? na : inf;
         else
-            mrow = (sa <= 1e30f) ? 4.0f * kDescendL2Margin * sa : inf;  // false for NaN
+            mrow = (sa <= 1e30f) ? 4.0f * descend_l2_margin(DIM) * sa : inf;  // false for NaN
         int node = 0;
         bool active = row0 + lane < n;
         while (__any(active)) {
@@ -1808,11 +1814,253 @@ __global__ void __launch_bounds__(512) k_tsvq_descend_w(const float *__restrict_
     }  // batches
 }
 
+// The walk for every width up to 256 and rows of any alignment: four lanes per row, lane q with the pieces 4 p + q of
+// four components (zeros behind the last one), so that a row's four lanes read 64 consecutive bytes and a wave holds
+// 16 rows in NP * 4 registers per lane.  The inner product decides as above where the node has a table (below ntab; the
+// first ntop of it in LDS).  Else both children's sums are made from memory, each lane its pieces with fused
+// multiply-adds, and their difference decides where it exceeds the bounds on both roundings:
+//   L2         |ar - al| > (2 D + 13) u (al + ar), al + ar >= 1e-30 (no square has lost bits below the smallest number)
+//   Manhattan  |ar - al| > (2 D + 2) u (al + ar)
+//   cosine     |pl / |cl| - pr / |cr|| > (4 D + 17) u |x|, norms as above
+// (the margins of descend_l2_margin and descend_cos_margin cover them; those of L2 are the distances' share and not
+// the vectors': rows far from the origin, as uniform ones are, 16 times closer at 248 components).  What that cannot
+// decide takes the two sums in the reference's order, lane 0 the left one, lane 1 the right one.  Manhattan has no
+// table: its LDS holds the first ntop centroids.
+// The nodes' stride of an odd number of 64-byte pieces spreads the rows of a wave over the banks.
+typedef float quad_piece __attribute__((ext_vector_type(4), aligned(4)));
+
+__host__ __device__ constexpr int quad_stride(int np) { return 16 * (np | 1); }
+
+// Workgroups of 512 threads per compute unit: what the registers allow.
+__host__ __device__ constexpr int quad_per_cu(int np) { return np <= 2 ? 3 : np <= 7 ? 2 : 1; }
+
+__device__ __forceinline__ quad_piece quad_load(const float *__restrict__ p, int at, int dim) {
+    quad_piece v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (at + 4 <= dim) {
+        v = *reinterpret_cast<const quad_piece *>(p + at);
+    } else {
+        if (at < dim) v.x = p[at];
+        if (at + 1 < dim) v.y = p[at + 1];
+        if (at + 2 < dim) v.z = p[at + 2];
+    }
+    return v;
+}
+
+// What lane LANE of a row's four holds.
+template <int LANE>
+__device__ __forceinline__ float quad_from(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), LANE * 0x55, 0xf, 0xf, false));
+}
+
+// The sum over a row's four lanes, the same bits in each of them.
+__device__ __forceinline__ float quad_sum(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));  // lanes 1 0 3 2
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));  // lanes 2 3 0 1
+    return v;
+}
+
+// Both children's sums over a lane's pieces, in an order of their own.
+template <int METRIC, int NP, typename Load>
+__device__ __forceinline__ void quad_pair(const quad_piece (&xr)[NP], float &sl, float &sr, Load load) {
+    float al[2] = {0.0f, 0.0f}, ar[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        quad_piece a, b;
+        load(p, a, b);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float xv = xr[p][e];
+            if constexpr (METRIC == M_COS) {
+                al[e & 1] = __builtin_fmaf(xv, a[e], al[e & 1]);
+                ar[e & 1] = __builtin_fmaf(xv, b[e], ar[e & 1]);
+            } else if constexpr (METRIC == M_L1) {
+                al[e & 1] += fabsf(xv - a[e]);
+                ar[e & 1] += fabsf(xv - b[e]);
+            } else {
+                const float dl = xv - a[e], dr = xv - b[e];
+                al[e & 1] = __builtin_fmaf(dl, dl, al[e & 1]);
+                ar[e & 1] = __builtin_fmaf(dr, dr, ar[e & 1]);
+            }
+        }
+    }
+    sl = quad_sum(al[0] + al[1]);
+    sr = quad_sum(ar[0] + ar[1]);
+}
+
+// tab: the table of k_tsvq_wtable with sctab, of ntab nodes, or the centroids themselves (Manhattan); ntop: the nodes of it in
+// LDS.  out16 (nullable): the leaves' centroids.
+template <int METRIC, int NP>
+__global__ void __launch_bounds__(512, 2 * quad_per_cu(NP)) k_tsvq_descend_quad(const float *__restrict__ x, int64_t n, int64_t ld, int dim,
+                                                           const float *__restrict__ cen,
+                                                           const float *__restrict__ cnorm,
+                                                           const int *__restrict__ left,
+                                                           const int *__restrict__ right,
+                                                           const float *__restrict__ tab,
+                                                           const float *__restrict__ sctab, int ntop, int ntab,
+                                                           int *__restrict__ leaf, uint16_t *__restrict__ out16) {
+    constexpr int S = quad_stride(NP);
+    constexpr bool COS = METRIC == M_COS, L1 = METRIC == M_L1;
+    extern __shared__ float4 lds_quad[];  // [ntop][S] the nodes, [2 ntop] their children, [2 ntop] their scalars
+    float *top = reinterpret_cast<float *>(lds_quad);
+    int *child = reinterpret_cast<int *>(top + (size_t)ntop * S);
+    float *sc = reinterpret_cast<float *>(child + 2 * ntop);
+    const float inf = __builtin_inff();
+    for (int e = threadIdx.x; e < ntop; e += blockDim.x) {
+        child[2 * e] = left[e];
+        child[2 * e + 1] = right[e];
+        if constexpr (COS) {
+            sc[e] = sctab[e];
+        } else if constexpr (!L1) {
+            sc[2 * e] = sctab[2 * e];
+            sc[2 * e + 1] = sctab[2 * e + 1];
+        }
+    }
+    for (int e = threadIdx.x; e < ntop * NP * 4; e += blockDim.x) {
+        const int nd = e / (NP * 4), pc = e % (NP * 4);
+        *reinterpret_cast<float4 *>(&top[nd * S + pc * 4]) =
+            __builtin_bit_cast(float4, quad_load(tab + (size_t)nd * dim, pc * 4, dim));
+    }
+    __syncthreads();
+    const int q = threadIdx.x & 3, waves = blockDim.x >> 6;
+    const float l2m = descend_l2_margin(dim), cosm = descend_cos_margin(dim);
+    const int64_t nbatch = (n + 15) / 16;
+    for (int64_t batch = (int64_t)blockIdx.x * waves + (threadIdx.x >> 6); batch < nbatch; batch += (int64_t)gridDim.x * waves) {
+        const int64_t row = batch * 16 + ((threadIdx.x & 63) >> 2);
+        const float *__restrict__ xp = x + (row < n ? row : n - 1) * ld;  // past the end: the last row, not stored
+        quad_piece xr[NP];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) xr[p] = quad_load(xp, (p * 4 + q) * 4, dim);
+        float mrow = 0.0f;  // the row's own share of the margin, +inf where its norm is out of range or not finite
+        if constexpr (!L1) {
+            float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                s0 = __builtin_fmaf(xr[p][0], xr[p][0], s0);
+                s1 = __builtin_fmaf(xr[p][1], xr[p][1], s1);
+                s0 = __builtin_fmaf(xr[p][2], xr[p][2], s0);
+                s1 = __builtin_fmaf(xr[p][3], xr[p][3], s1);
+            }
+            const float sa = quad_sum(s0 + s1), na = sqrtf(sa);
+            if constexpr (COS)
+                mrow = (na >= 1e-15f && na <= 1e15f) ? na : inf;
+            else
+                mrow = (sa <= 1e30f) ? 4.0f * l2m * sa : inf;  // false for NaN
+        }
+        int node = 0;
+        bool active = row < n;
+        while (__any(active)) {
+            int l = -1, r = -1;
+            if (active) {
+                if (node < ntop) {
+                    l = child[2 * node];
+                    r = child[2 * node + 1];
+                } else {
+                    l = left[node];
+                    r = right[node];
+                }
+            }
+            if (l >= 0 && r >= 0) {  // (the four lanes of a row agree here and below)
+                float f = 0.0f, theta = inf;
+                if (!L1 && node < ntab) {
+                    float f0 = 0.0f, f1 = 0.0f, f2 = 0.0f, f3 = 0.0f;
+                    auto dot = [&](auto load) {
+#pragma unroll
+                        for (int p = 0; p < NP; ++p) {
+                            const quad_piece a = load(p);
+                            f0 = __builtin_fmaf(xr[p][0], a[0], f0);
+                            f1 = __builtin_fmaf(xr[p][1], a[1], f1);
+                            f2 = __builtin_fmaf(xr[p][2], a[2], f2);
+                            f3 = __builtin_fmaf(xr[p][3], a[3], f3);
+                        }
+                    };
+                    if (node < ntop) {
+                        const float *pw = &top[node * S + q * 4];
+                        dot([&](int p) { return __builtin_bit_cast(quad_piece, *reinterpret_cast<const float4 *>(pw + p * 16)); });
+                    } else {
+                        const float *pw = tab + (size_t)node * dim;
+                        dot([&](int p) { return quad_load(pw, (p * 4 + q) * 4, dim); });
+                    }
+                    const float *sn = node < ntop ? sc : sctab;
+                    f = quad_sum((f0 + f1) + (f2 + f3));
+                    if constexpr (COS) {
+                        theta = sn[node] * mrow;
+                    } else {
+                        f += sn[2 * node];
+                        theta = sn[2 * node + 1] + mrow;
+                    }
+                }
+                if (!(fabsf(f) > theta)) {  // (also for NaN)
+                    float sl, sr;
+                    if (L1 && l < ntop && r < ntop) {
+                        const float *pl = &top[l * S + q * 4], *pr = &top[r * S + q * 4];
+                        quad_pair<METRIC, NP>(xr, sl, sr, [&](int p, quad_piece &a, quad_piece &b) {
+                            a = __builtin_bit_cast(quad_piece, *reinterpret_cast<const float4 *>(pl + p * 16));
+                            b = __builtin_bit_cast(quad_piece, *reinterpret_cast<const float4 *>(pr + p * 16));
+                        });
+                    } else {
+                        const float *pl = cen + (size_t)l * dim, *pr = cen + (size_t)r * dim;
+                        quad_pair<METRIC, NP>(xr, sl, sr, [&](int p, quad_piece &a, quad_piece &b) {
+                            a = quad_load(pl, (p * 4 + q) * 4, dim);
+                            b = quad_load(pr, (p * 4 + q) * 4, dim);
+                        });
+                    }
+                    if constexpr (COS) {
+                        const float nl = cnorm[l], nr = cnorm[r];
+                        const bool ok = nl >= 1e-15f && nl <= 1e15f && nr >= 1e-15f && nr <= 1e15f;
+                        f = sl / nl - sr / nr;
+                        theta = ok ? cosm * mrow : inf;
+                    } else {
+                        f = sr - sl;
+                        theta = (L1 || sl + sr >= 1e-30f) ? l2m * (sl + sr) : inf;
+                    }
+                }
+                if (f > theta) {  // (NaN fails both tests)
+                    node = l;
+                } else if (f < -theta) {
+                    node = r;
+                } else {
+                    // the two sums in the reference's order (src/tsvq.rs:167-171)
+                    const float *__restrict__ c = cen + (size_t)((q & 1) ? r : l) * dim;
+                    float d = 0.0f, sa = 0.0f;
+#pragma unroll 8
+                    for (int t = 0; t < dim; ++t) {
+                        const float xv = xp[t];
+                        wide_step<METRIC>(d, xv, c[t]);
+                        if constexpr (COS) {
+                            const float xx = xv * xv;
+                            sa = sa + xx;
+                        }
+                    }
+                    if constexpr (COS) {
+                        const float na = sqrtf(sa), nc = cnorm[(q & 1) ? r : l];
+                        const float quot = d / (na * nc);
+                        d = (na == 0.0f || nc == 0.0f) ? 1.0f : 1.0f - quot;
+                    }
+                    if constexpr (METRIC == M_EUCLID) d = sqrtf(d);
+                    const float dl = quad_from<0>(d), dr = quad_from<1>(d);
+                    node = dl <= dr ? l : r;
+                }
+            } else if (l >= 0) {
+                node = l;
+            } else if (r >= 0) {
+                node = r;
+            } else {
+                active = false;
+            }
+        }
+        if (q == 0 && row < n) leaf[row] = node;
+        if (out16)  // a row at a time by the whole wave: runs of 128 bytes, also into host memory
+            for (int i = 0; i < 16 && batch * 16 + i < n; ++i) {
+                const float *__restrict__ c = cen + (size_t)__shfl(node, 4 * i) * dim;
+                for (int t = threadIdx.x & 63; t < dim; t += 64) out16[(batch * 16 + i) * dim + t] = __half_as_ushort(__float2half_rn(c[t]));
+            }
+    }  // batches
+}
+
 // TSVQNode::quantize_with_distance (src/tsvq.rs:162-181) for a few rows: one wave per row, which brings
 // both children's centroids of a node into LDS with whole-line loads; lane 0 adds up the left distance
 // and lane 1 the right one, each in the reference's order.  out16 (nullable): the leaf's centroid.
-// (A lane of k_tsvq_descend reads its centroids alone; where the kernels that hold rows in registers are
-// faster, regs_rows says up to how many rows.)
+// (For widths beyond k_tsvq_descend_quad.)
 template <int METRIC>
 __global__ void __launch_bounds__(64) k_tsvq_few(const float *__restrict__ x, int64_t ld, int dim,
                                                  const float *__restrict__ cen, const float *__restrict__ cnorm,

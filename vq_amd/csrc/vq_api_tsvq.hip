@@ -23,6 +23,7 @@ using namespace vqh;
 struct vq_tree {
     int device = 0;
     int32_t n_nodes = 0;
+    int32_t n_inner = 0;  // nodes up to the last one with a child
     int32_t dim = 0;
     std::vector<float> h_centroids;
     std::vector<int32_t> h_left, h_right, h_split_dim;
@@ -63,6 +64,7 @@ struct KmOpts {
 // go up from the host copy.
 int32_t tree_to_device(vq_ctx *ctx, vq_tree *t, const float *d_means = nullptr) {
     size_t nn = (size_t)t->n_nodes, dim = (size_t)t->dim;
+    for (t->n_inner = t->n_nodes; t->n_inner > 0 && t->h_left[t->n_inner - 1] < 0 && t->h_right[t->n_inner - 1] < 0;) --t->n_inner;
     auto pad = [](size_t z) { return (z + 255) & ~(size_t)255; };
     const size_t cen_b = pad(sizeof(float) * nn * dim), idx_b = pad(sizeof(int32_t) * nn);
     const size_t ntop = std::min<size_t>(nn, (size_t)vq::kTopNodes);
@@ -100,6 +102,78 @@ void tree_release(vq_tree *t) {
     if (!t) return;
     (void)hipFree(t->d_block);
     delete t;
+}
+
+// The kernel with four lanes per row (k_tsvq_descend_quad): every width its registers hold.  Against a lane per row
+// with its sums from memory (k_tsvq_descend): 222,240 x 100, seven levels 982 -> 37 us, 69,233 x 200, five levels,
+// Manhattan 434 -> 42, 300,000 x 256, ten levels 5703 -> 212; against a wave per row (k_tsvq_few): 400 x 200,
+// five levels 19.9 -> 11.2 us, 100 x 128, nine levels 15.2 -> 9.4.
+constexpr int kQuadDims = 256;
+
+bool quad_applicable(const vq_ctx *ctx, const vq_tree *tree) {
+    return ctx->tsvq_descend_path == 0 && tree->dim <= kQuadDims;
+}
+
+template <int METRIC, int NP>
+int32_t descend_quad_np(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, const vq_tree *tree, int32_t *d_leaf,
+                        uint16_t *d_out) {
+    constexpr bool l1 = METRIC == vq::M_L1, cosine = METRIC == vq::M_COS;
+    // As many workgroups on a compute unit as its registers hold, the LDS shared among them: the nodes that do not
+    // fit are read from the L2, which costs less than the waves a larger table displaces (480,000 x 32, ten levels: a third
+    // of the LDS 40 us, half 46, all of it 76; x 64: 70, 59, 93; x 128: 140, 137, 134).
+    constexpr unsigned kPerCu = vq::quad_per_cu(NP);
+    constexpr size_t kBudget = (156u << 10) / kPerCu;
+    const size_t per_node = sizeof(float) * (size_t)vq::quad_stride(NP) + 2 * sizeof(int32_t) + (l1 ? 0 : 2 * sizeof(float));
+    const int32_t most = l1 ? tree->n_nodes : std::min(tree->n_inner, (int32_t)vq::kTopNodes);
+    // 129 to 2048 rows: a wave per workgroup and no table, so that the rows spread over the compute units (500 host rows
+    // x 128, ten levels 57 -> 47 us, 400 x 256 in GPU memory 20.6 -> 18.9)
+    const bool few = n > 128 && n <= 2048;
+    const unsigned threads = few ? 64 : 512;
+    const int32_t ntop = few ? 0 : (int32_t)std::min<size_t>((size_t)most, kBudget / per_node);
+    const size_t lds = per_node * (size_t)std::max(ntop, 1);
+    VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_tsvq_descend_quad<METRIC, NP>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    int cus = 0;
+    VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    const dim3 grid(std::min<unsigned>(cdiv(n, threads / 4), few ? ~0u : (unsigned)std::max(cus, 1) * kPerCu));
+    hipLaunchKernelGGL((vq::k_tsvq_descend_quad<METRIC, NP>), grid, dim3(threads), lds, ctx->stream, d_x, n, ld, tree->dim, tree->d_centroids,
+                       tree->d_cnorm, tree->d_left, tree->d_right, l1 ? tree->d_centroids : cosine ? tree->d_wcos : tree->d_wl2,
+                       cosine ? tree->d_sccos : tree->d_scl2, ntop, std::min(tree->n_nodes, (int32_t)vq::kTopNodes), d_leaf, d_out);
+    VQ_HIP(ctx, hipGetLastError());
+    return VQ_OK;
+}
+
+template <int METRIC>
+int32_t descend_quad_m(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, const vq_tree *tree, int32_t *d_leaf, uint16_t *d_out) {
+#define QUAD(NP) return descend_quad_np<METRIC, NP>(ctx, d_x, n, ld, tree, d_leaf, d_out)
+    switch ((tree->dim + 15) / 16) {
+    case 1: QUAD(1);
+    case 2: QUAD(2);
+    case 3: QUAD(3);
+    case 4: QUAD(4);
+    case 5: QUAD(5);
+    case 6: QUAD(6);
+    case 7: QUAD(7);
+    case 8: QUAD(8);
+    case 9:
+    case 10: QUAD(10);
+    case 11:
+    case 12:
+    case 13: QUAD(13);
+    default: QUAD(16);
+    }
+#undef QUAD
+}
+
+int32_t descend_quad(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, const vq_tree *tree, int32_t *d_leaf,
+                     uint16_t *d_out) {
+    switch (metric) {
+    case VQ_SQEUCLIDEAN: return descend_quad_m<vq::M_SQ>(ctx, d_x, n, ld, tree, d_leaf, d_out);
+    case VQ_EUCLIDEAN: return descend_quad_m<vq::M_EUCLID>(ctx, d_x, n, ld, tree, d_leaf, d_out);
+    case VQ_COSINE: return descend_quad_m<vq::M_COS>(ctx, d_x, n, ld, tree, d_leaf, d_out);
+    case VQ_MANHATTAN: return descend_quad_m<vq::M_L1>(ctx, d_x, n, ld, tree, d_leaf, d_out);
+    default: return fail(ctx, VQ_ERR_UNSUPPORTED, "metric %d has no kernel", metric);
+    }
 }
 
 }  // namespace
@@ -752,16 +826,6 @@ static bool few_applicable(const vq_ctx *ctx, int64_t n, int32_t dim) {
     return ctx->few_path == 0 && n <= kFewPairs && dim <= 4096;
 }
 
-// Up to how many rows the kernels that hold rows in registers (regs; inner: by one inner product per node) are
-// faster than k_tsvq_few.  They walk a level in half the time, but the rows of a wave read the levels that are not
-// in LDS (beyond 255 inner nodes) one after the other.  128 floats, Euclidean: 511 nodes 64 rows 11.1 us against
-// 19.4, 384 17.0 and 20.2, 512 19.2 and 20.9 (31 nodes: 14.1 and 11.4); 8191 nodes 64 rows 20.7 and 27.9, 128
-// 27.3 and 28.0, 256 41.7 and 28.1; Manhattan, 32 floats, 511 nodes: 64 rows 6.8 and 8.5, 384 8.9 and 8.5.
-// k_tsvq_descend, one lane per row with its centroids read by that lane alone, is slower at every number of rows.
-static int64_t regs_rows(bool regs, bool inner, int32_t n_nodes) {
-    return !regs ? 0 : !inner ? 64 : n_nodes <= 511 ? 384 : n_nodes <= 1023 ? 256 : 160;
-}
-
 static int32_t descend_few(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, const vq_tree *tree,
                            int32_t *d_leaf, uint16_t *d_out) {
     const size_t lds = sizeof(float) * 3 * ((size_t)tree->dim + 1);
@@ -793,12 +857,17 @@ int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n
     // cosine and (squared) Euclidean: a step decided by one inner product with the node's vector,
     // the two sums of the reference only where that cannot decide
     const bool inner = ctx->tsvq_descend_path == 0 && metric >= VQ_SQEUCLIDEAN && metric <= VQ_COSINE;
-    if (n > regs_rows(regs, inner, tree->n_nodes) && few_applicable(ctx, n, tree->dim))
-        return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
+    int cus = 0;
+    VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    // The kernels with a row per lane read half the LDS bytes per row where every inner node is in LDS (255) and
+    // half of their workgroups of 512 rows, one per compute unit, have rows: 131,072 x 128, eight levels 30.6 us
+    // against 38.7, 480,000 x 32, eight levels 28 against 32; but 66,000 x 128 27.9 against 27.4, 20,000 23.5 against
+    // 15.7, and ten levels 500,000 x 128 179 against 137.
+    if (quad_applicable(ctx, tree) && !(regs && tree->n_inner <= vq::kTopNodes && n > (int64_t)cus * 256))
+        return descend_quad(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
+    if (few_applicable(ctx, n, tree->dim)) return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
     if (regs) {
         // one workgroup per compute unit (the staged centroids fill its LDS), walking over the rows
-        int cus = 0;
-        VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
         dim3 g(std::min<unsigned>(cdiv(n, 512), (unsigned)std::max(cus, 1))), b(512);
         if (inner) {
             const bool cosine = metric == VQ_COSINE;
@@ -872,8 +941,11 @@ int32_t vq_tsvq_quantize_host(vq_ctx *ctx, int32_t metric, const float *h_x, int
     return host_batch(ctx, h_x, n, sizeof(float) * (size_t)dim, outs, 4u << 20, true,
                       [&](const float *d_x, int64_t rows, void *d_out, void *d_leaf) -> int32_t {
                           uint16_t *out = h_out ? (uint16_t *)d_out : nullptr;
-                          if (few_applicable(ctx, rows, dim))
+                          if (few_applicable(ctx, rows, dim)) {
+                              if (quad_applicable(ctx, tree))
+                                  return descend_quad(ctx, metric, d_x, rows, dim, tree, (int32_t *)d_leaf, out);
                               return descend_few(ctx, metric, d_x, rows, dim, tree, (int32_t *)d_leaf, out);
+                          }
                           VQ_TRY(vq_tsvq_descend(ctx, metric, d_x, rows, dim, tree, (int32_t *)d_leaf));
                           return out ? vq_tsvq_decode_f16(ctx, tree, (const int32_t *)d_leaf, rows, out) : VQ_OK;
                       });
