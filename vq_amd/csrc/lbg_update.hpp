@@ -566,60 +566,84 @@ static __global__ void __launch_bounds__(256) k_lbg_leafsum_wide(LbgState st, co
     if (t < sd) st.leaf_sum[((size_t)s * st.leaf_cap + e.z) * sd + t] = acc;
 }
 
-// Narrow column blocks (sub_dim a power of two up to 32): one wave per leaf.  A lane-per-component
-// walk as above leaves most of the wave idle and pays one memory round trip per 32 members; here
-// the 64 lanes fetch up to 2048 / sub_dim members at a time into LDS (row ids first, then the
-// sub-vectors, all loads of a chunk in flight together), and lanes 0..sub_dim-1 add them in list
-// order.
-constexpr int kLeafStage = 2048;  // floats staged per wave
-
-static __global__ void __launch_bounds__(256) k_lbg_leafsum_wave(LbgState st, const float *__restrict__ x,
-                                                                 int64_t n, int64_t ld, int sd, int sd_shift) {
+// A workgroup per leaf and tile of up to 4 P components (grid z), P pieces of VEC floats per member: the threads
+// fetch a chunk of members into registers, eight loads of each in flight while the chunk before is added, and store
+// them transposed in LDS; a lane per component adds them in list order, sixteen members read ahead of the adds.
+// The last piece of a tile begins at the tile's end less VEC and the last tile at the block's end less its width, so that
+// pieces of any width are whole (what two of them share is written twice, with the same values).  Its time is a chain of memory round trips, one per chunk of 128
+// to 512 members, beside the adds: 7,930 x 300, k = 22 41 -> 17 us per launch, 50,019 x 28 blocks of 10, k = 78 110 -> 28.
+// (With chunks of twice the members by 256 threads the same, where the leaves are long; the LDS then holds half the leaves.)
+template <int NT, int VEC>
+static __global__ void __launch_bounds__(NT) k_lbg_leafsum_tile(LbgState st, const float *__restrict__ x, int64_t n, int64_t ld,
+                                                                int sd, int width, int pieces) {
     const int s = blockIdx.y;
     if (st.done[s]) return;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t leaf = (int64_t)blockIdx.x * 4 + w;
-    if (leaf >= st.nleaves[s]) return;  // uniform per wave; the waves never synchronise
-    __shared__ float stage_all[4][kLeafStage];
-    float *stage = stage_all[w];
+    const int64_t leaf = blockIdx.x;
+    if (leaf >= st.nleaves[s]) return;  // uniform per workgroup
+    typedef float piece_t __attribute__((ext_vector_type(VEC), aligned(4)));
+    constexpr int E = 8;
+    extern __shared__ float4 lds_tile[];
+    float *stage = reinterpret_cast<float *>(lds_tile);
+    const int tid = threadIdx.x;
+    const int first = (int)blockIdx.z * width < sd - width ? (int)blockIdx.z * width : sd - width;
     const uint2 d = st.leaf_desc[(size_t)s * st.leaf_cap + leaf];
     const uint32_t *__restrict__ perm = st.perm + (size_t)s * n;
-    const float *__restrict__ xs = x + (int64_t)s * sd;
-    const uint32_t chunk = (uint32_t)(kLeafStage >> sd_shift);  // members per chunk
-    constexpr int E = kLeafStage / 64;                          // elements per lane and chunk
+    const int step = NT / pieces, mine = tid / pieces, at = VEC * (tid % pieces);
+    const int t0 = at + VEC <= width ? at : width - VEC;
+    const bool fetches = mine < step;
+    const float *__restrict__ xs = x + (int64_t)s * sd + first + t0;
+    const uint32_t chunk = (uint32_t)(E * step), stride = chunk + 4;
+    uint32_t row[E];
+    piece_t v[E];
+    auto rows = [&](uint32_t p) {  // past the end: the last member's
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const uint32_t q = p + (uint32_t)(mine + step * i);
+            row[i] = perm[q < d.y ? q : d.y - 1];
+        }
+    };
+    auto load = [&](uint32_t p) {
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+            if (p + (uint32_t)(step * i) < d.y) v[i] = *reinterpret_cast<const piece_t *>(xs + (int64_t)row[i] * ld);
+    };
     float acc = 0.0f;
-    for (uint32_t p = d.x; p < d.y; p += chunk) {
-        const uint32_t cm = (d.y - p < chunk) ? d.y - p : chunk;
-        const uint32_t tot = cm << sd_shift;
-        uint32_t row[E];
-        float v[E];
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-            const uint32_t e = (uint32_t)lane + 64u * i;
-            row[i] = (e < tot) ? perm[p + (e >> sd_shift)] : 0u;
-        }
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-            const uint32_t e = (uint32_t)lane + 64u * i;
-            v[i] = (e < tot) ? xs[(int64_t)row[i] * ld + (e & (uint32_t)(sd - 1))] : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < E; ++i) stage[lane + 64 * i] = v[i];
-        __builtin_amdgcn_wave_barrier();
-        if (lane < sd) {
-            uint32_t mbr = 0;
-            for (; mbr + 8 <= cm; mbr += 8) {
-                float t[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) t[u] = stage[((mbr + u) << sd_shift) + lane];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) acc = acc + t[u];
-            }
-            for (; mbr < cm; ++mbr) acc = acc + stage[(mbr << sd_shift) + lane];
-        }
-        __builtin_amdgcn_wave_barrier();
+    if (fetches && d.x < d.y) {
+        rows(d.x);
+        load(d.x);
     }
-    if (lane < sd) st.leaf_sum[((size_t)s * st.leaf_cap + leaf) * sd + lane] = acc;
+    for (uint32_t p = d.x; p < d.y; p += chunk) {
+        const uint32_t cm = d.y - p < chunk ? d.y - p : chunk;
+        if (fetches && p + chunk < d.y) rows(p + chunk);
+        if (p != d.x) __syncthreads();  // the chunk before has been added
+        if (fetches) {
+#pragma unroll
+            for (int i = 0; i < E; ++i)
+                if ((uint32_t)(step * i) < cm)
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) stage[(uint32_t)(t0 + e) * stride + (uint32_t)(mine + step * i)] = v[i][e];
+            if (p + chunk < d.y) load(p + chunk);
+        }
+        __syncthreads();
+        if (tid < width) {
+            const float *col = stage + (uint32_t)tid * stride;
+            uint32_t mbr = 0;
+            for (; mbr + 16 <= cm; mbr += 16) {
+                float4 q[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) q[u] = *reinterpret_cast<const float4 *>(col + mbr + 4 * u);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    acc = acc + q[u].x;
+                    acc = acc + q[u].y;
+                    acc = acc + q[u].z;
+                    acc = acc + q[u].w;
+                }
+            }
+            for (; mbr < cm; ++mbr) acc = acc + col[mbr];
+        }
+    }
+    if (tid < width) st.leaf_sum[((size_t)s * st.leaf_cap + leaf) * sd + first + tid] = acc;
 }
 
 // Few, long leaves (the small clusters beside the streaming kernel: up to 1024 members each): one

@@ -1438,6 +1438,13 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
     // 150,000 x 256 172 -> 179 us, 300,000 240 -> 241, 500,000 351 -> 343, 1,000,000 620 -> 589; x 128: 300,000 164 -> 169, 600,000
     // 258 -> 252 (k = 121 2 % slower), 1,000,000 384 -> 360; x 512: 250,000 384 -> 390, 500,000 646 -> 633; 3,000,000 x 64 589 -> 565.
     const bool wide_leaves = !stream && sd >= 64 && sd <= 512 && n >= 300'000 && n * m * sd >= 100'000'000;
+    // Else a workgroup per leaf and 32 components (k_lbg_leafsum_tile), of one wave where the leaves are parts of under 64
+    // members (500,000 x 8 blocks of 16, k = 160: 284 us per iteration, with two waves 341, a lane per component 309; 50,019 x 28 of
+    // 10, k = 78: two waves 141, one 142, a wave of 4-byte loads per leaf 223; 100,000 x 32, k = 128: 75, 83, a lane 155),
+    // but a lane per component where leaves of under 20 members fill the GPU that way (600,000 x 12 of 16, k = 256: 525
+    // against 583; 1M x 32, k = 256, on the other side: 221 and 198).
+    const bool parted = n > (int64_t)vq::kSeqMax * k;  // an average cluster is summed part by part
+    const bool lane_leaves = parted && vq::kPartRows < 20 * k && leaf_cap64 * sd * m >= (1 << 22);
     const size_t long_cap = (size_t)(n / vq::kLong + 1), leaf_slots = (size_t)m * leaf_cap;
     if (wide_leaves)  // the leaves in order, the two lists of long ones, the places, the counters
         VQ_TRY(ensure(ctx, ctx->leaf_desc, sizeof(uint4) * (leaf_slots + 2 * (size_t)m * long_cap) +
@@ -1567,11 +1574,14 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
             const int z = sd > 256 ? 2 : 1, threads = (int)cdiv(cdiv(sd, z), 64) * 64;
             hipLaunchKernelGGL(vq::k_lbg_leafsum_wide, dim3((unsigned)(leaf_cap + long_cap), m, z), dim3(threads), 0, gs, S, d_x,
                                n, ld, sd);
-        } else if (sd <= 32 && (1 << shift) == sd && (int64_t)leaf_cap * sd * m < (1 << 20)) {
-            // few leaves: a wave each; from a million (leaf, component) pairs on a lane each fills the GPU
-            // (600,000 rows in 12 blocks of 16, k = 256, 16 rows per leaf: 1.1 against 0.25 ms)
-            hipLaunchKernelGGL(vq::k_lbg_leafsum_wave, dim3(cdiv(leaf_cap, 4), m), dim3(256), 0, gs, S, d_x, n,
-                               ld, sd, shift);
+        } else if (!lane_leaves) {
+            const int tiles = (int)cdiv(sd, 32), width = tiles == 1 ? sd : (int)cdiv(cdiv(sd, tiles), 4) * 4;
+            const int threads = parted && vq::kPartRows < 64 * k ? 64 : 128, vec = sd >= 4 ? 4 : 1, pieces = (int)cdiv(width, vec);
+            const size_t lds = sizeof(float) * (size_t)width * (8 * (threads / pieces) + 4);
+            const dim3 grid(leaf_cap, m, (unsigned)cdiv(sd, width));
+            auto *kern = threads == 64 ? (vec == 4 ? vq::k_lbg_leafsum_tile<64, 4> : vq::k_lbg_leafsum_tile<64, 1>)
+                                       : (vec == 4 ? vq::k_lbg_leafsum_tile<128, 4> : vq::k_lbg_leafsum_tile<128, 1>);
+            hipLaunchKernelGGL(kern, grid, dim3(threads), lds, gs, S, d_x, n, ld, sd, width, pieces);
         } else {
             hipLaunchKernelGGL(vq::k_lbg_leafsum, dim3(cdiv((int64_t)leaf_cap * sd, 256), m), dim3(256), 0, gs,
                                S, d_x, n, ld, sd);
