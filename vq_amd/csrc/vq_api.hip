@@ -465,6 +465,31 @@ template <int METRIC, bool LBG> int32_t launch_mfma16(vq_ctx *ctx, const vq::Ass
     return VQ_OK;
 }
 
+// Whether the sums of a fit's blocks of 8 floats are streamed (k_lbg_stream8) or go by the lists of members.  The
+// streaming kernel's time does not depend on where the rows of a cluster are, but the fewer clusters share a tile of rows, the
+// more rounds it takes (one wave's chain over a part: 270 us per iteration at 4 clusters, 150 at 16, 120 at 40); the lists
+// and their leaves take 60 us and 32 per million (row, block) pairs, k = 4 to 100.  Per iteration, lists / streamed:
+// 250,000 x 12 k = 4 148 / 287, 16 150 / 176, 32 152 / 151, 112 170 / 138, 256 226 / 177; x 33 k = 4 309 / 400,
+// 10 310 / 289, 40 312 / 221; 1M x 16 k = 4 579 / 628, 10 578 / 459; 60,000 x 48 k = 16 153 / 181, 40 156 / 149, 80 (fewer
+// than 1024 rows per centroid: short lists) 168 / 190; 250,000 x 4 k = 56 89 / 116, 256 117 / 130.
+bool stream_pays(int64_t n, int m, int k) {
+    const double pairs = (double)n * m;
+    return pairs >= 1.5e6 + 6e7 / k && (n > (int64_t)vq::kSeqMax * k || pairs >= 2.95e6);
+}
+
+// Microseconds per iteration of a fit of blocks of 8 floats, and of narrower blocks of their own width, for the choice between
+// them (within 15 % at 30,000 to 1M rows, 4 to 48 blocks, k = 4 to 256).  Narrow blocks are cheaper where
+// memory bounds both: 250,000 x 12 blocks of 3, k = 32 137 / 152, 80 174 / 147; x 33 of 6, k = 4 389 / 323, 46 blocks of 7
+// 430 / 240; 60,000 x 12 of 6, k = 24 85 / 86, 56 99 / 89.
+double fit8_us(int64_t n, int m, int k) {
+    const double mp = (double)n * m * 1e-6;
+    return stream_pays(n, m, k) ? 95 + 650.0 / k + mp * (16 + 40.0 / k) : 60 + 33 * mp;
+}
+double fit_static_us(int64_t n, int m, int sd, int k) {
+    const double mp = (double)n * m * 1e-6, spread = m % 2 ? 0.6 + 0.15 * sd : 1.0;  // (odd: one block per lane)
+    return 55 + mp * (19 + std::max(13 * spread, 0.022 * (3 * (sd == 7 ? 8 : sd) + 1) * k));
+}
+
 // The width to pad every column block to so that the matrix-core kernels take the shape (squared L2,
 // Euclidean, cosine; 0: they take it as it is, or padding does not pay).  fit: for the passes of a fit,
 // which pads its rows once and whose update then streams blocks of 8 as well.
@@ -489,11 +514,12 @@ int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bo
     if ((int64_t)a.m * sdp > (1 << 20) || sdp > (1 << 16) || a.n * a.m >= (1LL << 32)) return 0;
     const int w = static_width(sd);
     if (fit && sd != sdp && lbg_small(a.n, a.m, sdp, a.k)) return sdp;
+    if (fit && sd < 8) return fit8_us(a.n, a.m, a.k) < fit_static_us(a.n, a.m, sd, a.k) ? sdp : 0;
+    if (fit && w != sd && (w <= 16 || w == 32)) return a.k >= (w == 32 ? 36 : 40) || (w <= 16 && a.m % 2 == 0) ? sdp : 0;
     if (w == sd) {
         const int cost = a.k * (metric == VQ_COSINE ? 2 * sd + 26 : 3 * sd + 1);
         if (metric == VQ_COSINE ? cost < (sd < 8 ? 1500 : 3500)
-            : sd > 8            ? cost < (fit ? 4700 : 3500)
-            : fit               ? a.k < 40
+            : sd > 8            ? (fit ? a.k < 40 : cost < 3500)
                                 : sd == 2 || cost < 1600 || (a.m % 4 != 0 && (cost - 1600) * (double)(a.n * a.m) < 5e8))
             return 0;
     } else if (w && a.k < (w > 16 ? 60 : metric == VQ_COSINE ? (w == 8 ? 32 : 40) : w == 8 ? 48 : 60)) {
@@ -1418,9 +1444,8 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
     const int nparts = (int)((n + vq::kPartRows - 1) / vq::kPartRows);
     const int nseg = (nparts + vq::kScanSeg - 1) / vq::kScanSeg;
     // streaming sums of the large clusters: 32-byte sub-vectors, 4 to a workgroup, aligned rows (a last
-    // group with idle waves pays from some 60,000 rows on: 25 blocks, k = 16: 20,000 rows 117 us per
-    // iteration without, 150 with; 200,000 rows 283 and 223)
-    const bool stream = sd == 8 && (m % 4 == 0 || nparts >= 16) && ld % 4 == 0 && ld <= (1 << 20) &&
+    // group with idle waves pays from some 60,000 rows on)
+    const bool stream = sd == 8 && stream_pays(n, m, k) && (m % 4 == 0 || nparts >= 16) && ld % 4 == 0 && ld <= (1 << 20) &&
                         (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;  // (32-bit lane offsets inside a chunk)
     const int64_t leaf_cap64 = stream ? (int64_t)k : (int64_t)k * nparts;
     if (leaf_cap64 * sd > (1LL << 31)) return fail(ctx, VQ_ERR_UNSUPPORTED, "n * k * sub_dim too large");
