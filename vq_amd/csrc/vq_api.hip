@@ -515,7 +515,7 @@ int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bo
     const int w = static_width(sd);
     if (fit && sd != sdp && lbg_small(a.n, a.m, sdp, a.k)) return sdp;
     if (fit && sd < 8) return fit8_us(a.n, a.m, a.k) < fit_static_us(a.n, a.m, sd, a.k) ? sdp : 0;
-    if (fit && w != sd && (w <= 16 || w == 32)) return a.k >= (w == 32 ? 36 : 40) || (w <= 16 && a.m % 2 == 0) ? sdp : 0;
+    if (fit && w && w != sd && (w <= 16 || w == 32)) return a.k >= (w == 32 ? 36 : 40) || (w <= 16 && a.m % 2 == 0) ? sdp : 0;
     if (w == sd) {
         const int cost = a.k * (metric == VQ_COSINE ? 2 * sd + 26 : 3 * sd + 1);
         if (metric == VQ_COSINE ? cost < (sd < 8 ? 1500 : 3500)
