@@ -30,7 +30,8 @@ constexpr int kSeqMax = 1024;        // PARALLEL_THRESHOLD, src/vector.rs:16
 struct LbgState {
     // per column block s
     int *changed;          // m
-    int *done;             // m
+    int *done;             // m   of this iteration
+    int *done_next = nullptr;  // m   of the next one: written with the plan where no later kernel controls the loop, else null
     int *iters;            // m
     int *used;             // m   re-seed entries consumed so far
     int *ubase;            // m   value of used[s] at the start of the current update
@@ -76,6 +77,7 @@ static __global__ void k_lbg_init(LbgState st, int m) {
     if (s < m) {
         st.changed[s] = 0;
         st.done[s] = 0;
+        if (st.done_next) st.done_next[s] = 0;
         st.iters[s] = 0;
         st.used[s] = 0;
         st.ubase[s] = 0;
@@ -143,6 +145,32 @@ static __global__ void __launch_bounds__(64) k_lbg_hist(LbgState st, int64_t n) 
     for (int j = threadIdx.x; j < kMaxK; j += 64) h[j] = cnt[j];
 }
 
+// The same by four waves with a histogram each, where no streaming kernel runs beside it (12 -> 6 us at 2 to 47 parts: the
+// time is a wave's chain of LDS additions, and of few parts no other wave hides it).
+static __global__ void __launch_bounds__(256) k_lbg_hist_wg(LbgState st, int64_t n) {
+    const int s = blockIdx.y, b = blockIdx.x, w = threadIdx.x >> 6;
+    if (st.done[s]) return;
+    __shared__ uint32_t cnt[4][kMaxK];
+    for (int j = threadIdx.x; j < 4 * kMaxK; j += 256) (&cnt[0][0])[j] = 0;
+    __syncthreads();
+    const uint8_t *codes = st.codes + (size_t)s * n;
+    const int64_t lo = (int64_t)b * kPartRows;
+    const int64_t hi = lo + kPartRows < n ? lo + kPartRows : n;
+    if (hi - lo == kPartRows && ((uintptr_t)(codes + lo) & 15) == 0) {
+        const uint4 v = reinterpret_cast<const uint4 *>(codes + lo)[threadIdx.x];
+        const uint32_t q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int sh = 0; sh < 32; sh += 8) atomicAdd(&cnt[w][(q[u] >> sh) & 255u], 1u);
+    } else {
+        for (int64_t i = lo + threadIdx.x; i < hi; i += 256) atomicAdd(&cnt[w][codes[i]], 1u);
+    }
+    __syncthreads();
+    const int j = threadIdx.x;
+    st.hist[((size_t)s * st.nparts + b) * kMaxK + j] = cnt[0][j] + cnt[1][j] + cnt[2][j] + cnt[3][j];
+}
+
 // Scan step 1: per (column block, segment of kScanSeg parts) sum of the histograms.
 static __global__ void __launch_bounds__(256) k_lbg_scan_seg(LbgState st) {
     side_chain_priority();
@@ -165,24 +193,9 @@ static __global__ void __launch_bounds__(256) k_lbg_scan_seg(LbgState st) {
 // the re-seed cursor advanced by the number of empty clusters.
 // Leaves: a small cluster (1..1024 members) is one leaf over its whole member list; a large
 // cluster has one leaf per part, unless the streaming kernel sums the large clusters.
-static __global__ void __launch_bounds__(256) k_lbg_plan(LbgState st, int k) {
-    side_chain_priority();
-    const int s = blockIdx.x, j = threadIdx.x;
-    if (st.done[s]) return;
+// Thread j of 256, in group g of as many (group 0 writes): run members of cluster j; pc, pl: its first position and leaf.
+__device__ __forceinline__ void lbg_plan_clusters(const LbgState &st, int s, int j, int k, int g, uint32_t run, uint32_t &pc, uint32_t &pl) {
     __shared__ uint32_t sh_cnt[4], sh_leaf[4], sh_empty[4], sh_small[4];  // totals of the four waves
-    uint32_t run = 0;
-    uint32_t *h = st.seg + (size_t)s * st.nseg * kMaxK + j;
-    for (int g0 = 0; g0 < st.nseg; g0 += 8) {
-        uint32_t v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = (g0 + u < st.nseg) ? h[(size_t)(g0 + u) * kMaxK] : 0u;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            if (g0 + u < st.nseg) h[(size_t)(g0 + u) * kMaxK] = run;
-            run += v[u];
-        }
-    }
-    if (st.order && j < 2) st.nlong[2 * s + j] = 0;
     const bool live = j < k;
     const uint32_t cnt = live ? run : 0;
     const bool small = cnt > 0 && cnt <= (uint32_t)kSeqMax;
@@ -210,13 +223,16 @@ static __global__ void __launch_bounds__(256) k_lbg_plan(LbgState st, int k) {
         sh_small[wv] = is;
     }
     __syncthreads();
-    uint32_t pc = ic - cnt, pl = il - nl, pe = ie - emp, ps = is - (small ? 1u : 0u);
+    pc = ic - cnt;
+    pl = il - nl;
+    uint32_t pe = ie - emp, ps = is - (small ? 1u : 0u);
     for (int u = 0; u < wv; ++u) {
         pc += sh_cnt[u];
         pl += sh_leaf[u];
         pe += sh_empty[u];
         ps += sh_small[u];
     }
+    if (g) return;
     const size_t sj = (size_t)s * kMaxK + j;
     st.count[sj] = cnt;
     st.start[sj] = pc;
@@ -237,6 +253,74 @@ static __global__ void __launch_bounds__(256) k_lbg_plan(LbgState st, int k) {
         int u = st.used[s];
         st.ubase[s] = u;
         st.used[s] = u + (int)(pe + emp);
+        if (st.done_next) {  // the loop control of src/utils.rs:57,104-106: this update is the last one if no code changed
+            st.iters[s] += 1;
+            st.done_next[s] = st.changed[s] ? 0 : 1;
+            st.changed[s] = 0;
+        }
+    }
+}
+
+static __global__ void __launch_bounds__(256) k_lbg_plan(LbgState st, int k) {
+    side_chain_priority();
+    const int s = blockIdx.x, j = threadIdx.x;
+    if (st.done[s]) {
+        if (st.done_next && j == 0) st.done_next[s] = 1;
+        return;
+    }
+    uint32_t run = 0;
+    uint32_t *h = st.seg + (size_t)s * st.nseg * kMaxK + j;
+    for (int g0 = 0; g0 < st.nseg; g0 += 8) {
+        uint32_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = (g0 + u < st.nseg) ? h[(size_t)(g0 + u) * kMaxK] : 0u;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if (g0 + u < st.nseg) h[(size_t)(g0 + u) * kMaxK] = run;
+            run += v[u];
+        }
+    }
+    if (st.order && j < 2) st.nlong[2 * s + j] = 0;
+    uint32_t pc, pl;
+    lbg_plan_clusters(st, s, j, k, 0, run, pc, pl);
+}
+
+// The three steps in one launch for up to kScanMost segments (524,288 rows) where no streaming kernel runs beside
+// them: 256 threads per segment, thread j of each with its cluster's kScanSeg entries.  14 -> 6 us; beyond, a
+// single workgroup cannot keep the loads of a column block in flight.
+constexpr int kScanMost = 4;
+static __global__ void __launch_bounds__(256 * kScanMost) k_lbg_scan(LbgState st, int k) {
+    const int s = blockIdx.x, g = threadIdx.x >> 8, j = threadIdx.x & 255;
+    if (st.done[s]) {
+        if (st.done_next && threadIdx.x == 0) st.done_next[s] = 1;
+        return;
+    }
+    __shared__ uint32_t sums[kScanMost][kMaxK];
+    const int b0 = g * kScanSeg, b1 = (b0 + kScanSeg < st.nparts) ? b0 + kScanSeg : st.nparts;
+    uint32_t *h = st.hist + ((size_t)s * st.nparts + b0) * kMaxK + j;
+    uint32_t v[kScanSeg], sum = 0;
+#pragma unroll
+    for (int u = 0; u < kScanSeg; ++u) v[u] = h[(size_t)(b0 + u < b1 ? u : b1 - 1 - b0) * kMaxK];
+#pragma unroll
+    for (int u = 0; u < kScanSeg; ++u) sum += (b0 + u < b1) ? v[u] : 0u;
+    sums[g][j] = sum;
+    __syncthreads();
+    uint32_t all = 0, run = 0;
+    for (int u = 0; u < st.nseg; ++u) {
+        if (u < g) run += sums[u][j];
+        all += sums[u][j];
+    }
+    uint32_t pc, pl;
+    lbg_plan_clusters(st, s, j, k, g, all, pc, pl);
+    const bool leaves = j < k && !st.stream && all > (uint32_t)kSeqMax;
+    uint2 *desc = st.leaf_desc + (size_t)s * st.leaf_cap + pl + (uint32_t)b0;
+#pragma unroll
+    for (int u = 0; u < kScanSeg; ++u) {
+        if (b0 + u < b1) {
+            h[(size_t)u * kMaxK] = run;
+            if (leaves) desc[u] = make_uint2(pc + run, pc + run + v[u]);
+            run += v[u];
+        }
     }
 }
 
@@ -396,20 +480,20 @@ static __global__ void __launch_bounds__(64) k_lbg_scatter(LbgState st, int64_t 
     }
 }
 
-// The same scatter by a workgroup of four waves per (part, column block): wave w ranks the rows
-// [1024 w, 1024 w + 1024) of the part.  A first sweep counts the listed codes of each quarter, so
-// that a wave's first position inside cluster j is the part's position plus the members in the
-// quarters before its own; the order of the rows inside a cluster stays the row order.  One wave
-// per part is a chain of 64 dependent LDS round trips per part (and a handful of waves on the whole
-// GPU when there is one column block).
-static __global__ void __launch_bounds__(256) k_lbg_scatter_wg(LbgState st, int64_t n) {
+// The same scatter by a workgroup of W waves per (part, column block): wave w ranks the w-th W-th of the part's
+// rows.  A first sweep counts the listed codes of each share, so that a wave's first position inside
+// cluster j is the part's position plus the members in the shares before its own; the order of the rows inside a
+// cluster stays the row order.  A wave is a chain of 4096 / 64 W dependent LDS round trips (and there is a handful of workgroups
+// on the whole GPU when there is one column block): four waves per part 13 us, sixteen 9.
+constexpr int kScatterWaves = 16;
+
+static __global__ void __launch_bounds__(64 * kScatterWaves) k_lbg_scatter_wg(LbgState st, int64_t n) {
     side_chain_priority();
     const int s = blockIdx.y, b = blockIdx.x;
     if (st.done[s]) return;
     if (st.stream && st.nsmall[s] == 0) return;
-    constexpr int kQuarter = kPartRows / 4;
-    __shared__ uint32_t cntq[4][kMaxK];
-    __shared__ uint32_t base[4][kMaxK];
+    constexpr int W = kScatterWaves, kShare = kPartRows / W;
+    __shared__ uint32_t cntq[W][kMaxK];
     __shared__ uint8_t listed[kMaxK];
     __shared__ __attribute__((aligned(16))) uint8_t pcodes[kPartRows];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -418,10 +502,11 @@ static __global__ void __launch_bounds__(256) k_lbg_scatter_wg(LbgState st, int6
     const int64_t lo = (int64_t)b * kPartRows;
     const int64_t hi = lo + kPartRows < n ? lo + kPartRows : n;
     const int rows = (int)(hi - lo);
-    for (int j = threadIdx.x; j < 4 * kMaxK; j += 256) (&cntq[0][0])[j] = 0u;
-    listed[threadIdx.x] = (!st.stream || st.count[(size_t)s * kMaxK + threadIdx.x] <= (uint32_t)kSeqMax) ? 1 : 0;
+    for (int j = threadIdx.x; j < W * kMaxK; j += 64 * W) (&cntq[0][0])[j] = 0u;
+    if (threadIdx.x < kMaxK)
+        listed[threadIdx.x] = (!st.stream || st.count[(size_t)s * kMaxK + threadIdx.x] <= (uint32_t)kSeqMax) ? 1 : 0;
     // the part's codes into LDS, 16 per thread
-    {
+    if (threadIdx.x < kPartRows / 16) {
         const int64_t r0 = lo + 16 * (int64_t)threadIdx.x;
         uint4 v = make_uint4(0u, 0u, 0u, 0u);
         if (((uintptr_t)(codes + lo) & 15) == 0 && r0 + 16 <= hi) {
@@ -435,25 +520,26 @@ static __global__ void __launch_bounds__(256) k_lbg_scatter_wg(LbgState st, int6
         reinterpret_cast<uint4 *>(pcodes)[threadIdx.x] = v;
     }
     __syncthreads();
-    const int q0 = w * kQuarter, q1 = q0 + kQuarter < rows ? q0 + kQuarter : rows;
+    const int q0 = w * kShare, q1 = q0 + kShare < rows ? q0 + kShare : rows;
     for (int i = q0 + lane; i < q1; i += 64) {
         const uint32_t c = pcodes[i];
         if (listed[c]) atomicAdd(&cntq[w][c], 1u);
     }
     __syncthreads();
-    {
+    if (threadIdx.x < kMaxK) {
         const uint32_t *h = st.hist + ((size_t)s * st.nparts + b) * kMaxK;
         const uint32_t *start = st.start + (size_t)s * kMaxK;
-        const int j = threadIdx.x;  // kMaxK == 256 threads
+        const int j = threadIdx.x;
         uint32_t run = start[j] + h[j];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            base[q][j] = run;
-            run += cntq[q][j];
+        for (int q = 0; q < W; ++q) {
+            const uint32_t c = cntq[q][j];
+            cntq[q][j] = run;
+            run += c;
         }
     }
     __syncthreads();
-    uint32_t *mybase = base[w];
+    uint32_t *mybase = cntq[w];
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     for (int i0 = q0; i0 < q1; i0 += 64) {
         const int i = i0 + lane;
@@ -1538,15 +1624,6 @@ static __global__ void __launch_bounds__(256) k_lbg_fold8(LbgState st, int k, fl
             if (p + u < np) sum = sum + v[u];
     }
     big_sum[((size_t)s * kMaxK + j) * 8 + t] = sum;
-}
-
-// Loop control of src/utils.rs:57,104-106, one thread per column block.
-static __global__ void k_lbg_advance(LbgState st, int m) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= m || st.done[s]) return;
-    st.iters[s] += 1;
-    if (!st.changed[s]) st.done[s] = 1;
-    st.changed[s] = 0;
 }
 
 // The end of an update and the start of the next assignment pass, one workgroup per column block

@@ -468,13 +468,13 @@ template <int METRIC, bool LBG> int32_t launch_mfma16(vq_ctx *ctx, const vq::Ass
 // Whether the sums of a fit's blocks of 8 floats are streamed (k_lbg_stream8) or go by the lists of members.  The
 // streaming kernel's time does not depend on where the rows of a cluster are, but the fewer clusters share a tile of rows, the
 // more rounds it takes (one wave's chain over a part: 270 us per iteration at 4 clusters, 150 at 16, 120 at 40); the lists
-// and their leaves take 60 us and 32 per million (row, block) pairs, k = 4 to 100.  Per iteration, lists / streamed:
+// and their leaves take 48 us and 32 per million (row, block) pairs, k = 4 to 100 (60 and 32 when the figures below were taken).  Per iteration, lists / streamed:
 // 250,000 x 12 k = 4 148 / 287, 16 150 / 176, 32 152 / 151, 112 170 / 138, 256 226 / 177; x 33 k = 4 309 / 400,
 // 10 310 / 289, 40 312 / 221; 1M x 16 k = 4 579 / 628, 10 578 / 459; 60,000 x 48 k = 16 153 / 181, 40 156 / 149, 80 (fewer
 // than 1024 rows per centroid: short lists) 168 / 190; 250,000 x 4 k = 56 89 / 116, 256 117 / 130.
 bool stream_pays(int64_t n, int m, int k) {
     const double pairs = (double)n * m;
-    return pairs >= 1.5e6 + 6e7 / k && (n > (int64_t)vq::kSeqMax * k || pairs >= 2.95e6);
+    return pairs >= 2e6 + 6e7 / k && (n > (int64_t)vq::kSeqMax * k || pairs >= 2.95e6);
 }
 
 // Microseconds per iteration of a fit of blocks of 8 floats, and of narrower blocks of their own width, for the choice between
@@ -483,11 +483,11 @@ bool stream_pays(int64_t n, int m, int k) {
 // 430 / 240; 60,000 x 12 of 6, k = 24 85 / 86, 56 99 / 89.
 double fit8_us(int64_t n, int m, int k) {
     const double mp = (double)n * m * 1e-6;
-    return stream_pays(n, m, k) ? 95 + 650.0 / k + mp * (16 + 40.0 / k) : 60 + 33 * mp;
+    return stream_pays(n, m, k) ? 95 + 650.0 / k + mp * (16 + 40.0 / k) : 48 + 33 * mp;
 }
 double fit_static_us(int64_t n, int m, int sd, int k) {
     const double mp = (double)n * m * 1e-6, spread = m % 2 ? 0.6 + 0.15 * sd : 1.0;  // (odd: one block per lane)
-    return 55 + mp * (19 + std::max(13 * spread, 0.022 * (3 * (sd == 7 ? 8 : sd) + 1) * k));
+    return 42 + mp * (19 + std::max(13 * spread, 0.022 * (3 * (sd == 7 ? 8 : sd) + 1) * k));
 }
 
 // The width to pad every column block to so that the matrix-core kernels take the shape (squared L2,
@@ -1450,7 +1450,7 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
     const int64_t leaf_cap64 = stream ? (int64_t)k : (int64_t)k * nparts;
     if (leaf_cap64 * sd > (1LL << 31)) return fail(ctx, VQ_ERR_UNSUPPORTED, "n * k * sub_dim too large");
     const int leaf_cap = (int)leaf_cap64;
-    VQ_TRY(ensure(ctx, ctx->flags, sizeof(int) * (7 * (size_t)m + 1)));
+    VQ_TRY(ensure(ctx, ctx->flags, sizeof(int) * (8 * (size_t)m + 1)));
     VQ_TRY(ensure(ctx, ctx->tables, sizeof(uint32_t) * 4 * (size_t)m * vq::kMaxK));
     VQ_TRY(ensure(ctx, ctx->hist, sizeof(uint32_t) * (size_t)m * nparts * vq::kMaxK));
     VQ_TRY(ensure(ctx, ctx->seg, sizeof(uint32_t) * (size_t)m * nseg * vq::kMaxK));
@@ -1491,6 +1491,7 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
     S.nleaves = f + 5 * m;
     S.nsmall = f + 6 * m;
     S.err = f + 7 * m;
+    S.done_next = f + 7 * m + 1;
     uint32_t *tb = (uint32_t *)ctx->tables.p;
     const size_t mk = (size_t)m * vq::kMaxK;
     S.count = tb;
@@ -1547,7 +1548,10 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
     // centroids, the loop control and the tables of the next assignment pass.
     const bool fused_tail = stream && mfma_applicable<vq::M_SQ, true>(ctx, a, sd);
     MfmaTabPtrs tabs{};
-    if (fused_tail) VQ_TRY(mfma_tab_ptrs(ctx, m, k, tabs));
+    if (fused_tail) {
+        VQ_TRY(mfma_tab_ptrs(ctx, m, k, tabs));
+        S.done_next = nullptr;
+    }
     // Timing classes of the loop: where the assignment kernel carries its own events (started,
     // done) the assignment span is the kernel's and an update span runs from one kernel's end to
     // the next one's start, so nothing is recorded between the kernels of an iteration.
@@ -1582,14 +1586,21 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
             VQ_HIP(ctx, hipStreamWaitEvent(gs, done, 0));
             hipLaunchKernelGGL(vq::k_lbg_stream8, dim3(nparts, cdiv(m, 4)), dim3(256), 0, st, S, d_x, n, ld, m);
         }
-        hipLaunchKernelGGL(vq::k_lbg_hist, dim3(nparts, m), dim3(64), 0, gs, S, n);
-        hipLaunchKernelGGL(vq::k_lbg_scan_seg, dim3(nseg, m), dim3(256), 0, gs, S);
-        hipLaunchKernelGGL(vq::k_lbg_plan, dim3(m), dim3(256), 0, gs, S, k);
-        hipLaunchKernelGGL(vq::k_lbg_scan_blocks, dim3(nseg, m), dim3(256), 0, gs, S);
+        if (stream)
+            hipLaunchKernelGGL(vq::k_lbg_hist, dim3(nparts, m), dim3(64), 0, gs, S, n);
+        else
+            hipLaunchKernelGGL(vq::k_lbg_hist_wg, dim3(nparts, m), dim3(256), 0, gs, S, n);
+        if (!stream && nseg <= vq::kScanMost && !wide_leaves) {
+            hipLaunchKernelGGL(vq::k_lbg_scan, dim3(m), dim3(256 * nseg), 0, gs, S, k);
+        } else {
+            hipLaunchKernelGGL(vq::k_lbg_scan_seg, dim3(nseg, m), dim3(256), 0, gs, S);
+            hipLaunchKernelGGL(vq::k_lbg_plan, dim3(m), dim3(256), 0, gs, S, k);
+            hipLaunchKernelGGL(vq::k_lbg_scan_blocks, dim3(nseg, m), dim3(256), 0, gs, S);
+        }
         if (stream)  // beside the streaming kernel: one wave per part (four waves per part take its resources: 40 us, and 15 us more for the streaming kernel)
             hipLaunchKernelGGL(vq::k_lbg_scatter, dim3(nparts, m), dim3(64), 0, gs, S, n);
-        else  // every row is listed: four waves per part
-            hipLaunchKernelGGL(vq::k_lbg_scatter_wg, dim3(nparts, m), dim3(256), 0, gs, S, n);
+        else  // every row is listed: sixteen waves per part (four: 3-5 us more of an iteration)
+            hipLaunchKernelGGL(vq::k_lbg_scatter_wg, dim3(nparts, m), dim3(64 * vq::kScatterWaves), 0, gs, S, n);
         if (leaf_wg) {
             // leaves are the few clusters of up to 1024 members beside the streaming kernel
             hipLaunchKernelGGL(vq::k_lbg_leafsum_wg, dim3(leaf_cap, m), dim3(256), 0, gs, S, d_x, n, ld, sd,
@@ -1628,7 +1639,8 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
         } else {
             hipLaunchKernelGGL(vq::k_lbg_finalize, dim3(cdiv((int64_t)k * sd, 256), m), dim3(256), 0, st, S,
                                d_x, ld, k, sd, (const uint32_t *)ctx->reseed.p, n_reseed, d_codebooks);
-            hipLaunchKernelGGL(vq::k_lbg_advance, dim3(cdiv(m, 64)), dim3(64), 0, st, S, m);
+            std::swap(S.done, S.done_next);
+            a.done = S.done;
         }
         VQ_HIP(ctx, hipGetLastError());
     }
