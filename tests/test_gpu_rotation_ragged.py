@@ -1,0 +1,55 @@
+"""Rotation and cross-covariance of dimensions that are no multiple of the matrix-core tiles: against 64-bit products, with
+the bound of a chain of fused multiply-adds, rows spaced and unaligned, and what is not finite in the components behind a row."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+@pytest.mark.parametrize("n,dim,extra,offset", [
+    (2, 1, 0, 0), (127, 5, 0, 0), (128, 31, 0, 1), (129, 33, 2, 0), (300, 50, 0, 0), (65, 64, 1, 0), (64, 96, 0, 2), (257, 100, 0, 0), (700, 130, 0, 0),
+    (1000, 180, 0, 0), (33, 250, 5, 3), (200, 300, 0, 0), (40, 639, 0, 0)])
+def test_rotate(n, dim, extra, offset):
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    rng = np.random.default_rng(dim)
+    ld = dim + extra
+    buf = np.full(n * ld + offset, np.nan, F)  # what lies between the rows is no number
+    x = np.lib.stride_tricks.as_strided(buf[offset:], (n, dim), (4 * ld, 4))
+    x[:] = rng.standard_normal((n, dim))
+    x[n // 2, dim // 2] = np.inf
+    R = rng.standard_normal((dim, dim)).astype(F)
+    y = ctx.empty((n, dim), F)
+    dx = ctx.to_device(buf)
+    ctx.rotate(SimpleNamespace(ptr=dx.ptr + 4 * offset), n, ld, dim, ctx.to_device(R), y)
+    got = y.download()
+    X, R64 = x.astype(np.float64), R.astype(np.float64)
+    rest = np.arange(n) != n // 2
+    want, size = X @ R64.T, np.abs(X) @ np.abs(R64).T
+    chain = np.zeros((n, dim), F)  # fused multiply-adds in ascending order (but for sums that 64 bits of fraction round as well)
+    for t in range(dim):
+        chain = (x[:, t, None].astype(np.longdouble) * R[:, t].astype(np.longdouble) + chain).astype(F)
+    if dim % 32 or extra or offset:
+        assert np.sum(got[rest] != chain[rest]) <= n * dim // 1000
+    with np.errstate(invalid="ignore"):
+        err = np.abs(got - want)
+    assert np.all(err[rest] <= (dim + 1) * 2.0 ** -24 * size[rest])
+    assert np.array_equal(got[n // 2], want[n // 2].astype(F))  # infinities, not NaN
+    with pytest.raises(Exception):
+        ctx.rotate(dx, 1, 700, 640 + 3, ctx.to_device(R), y)
+    ctx.close()
+
+
+@pytest.mark.parametrize("n,dim", [(1, 1), (3, 15), (130, 7), (129, 17), (131, 18), (1, 33), (4, 33), (700, 50), (1025, 100), (514, 130), (2050, 180), (520, 250), (516, 300)])
+def test_cross_cov(n, dim):
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    rng = np.random.default_rng(n + dim)
+    y, x = rng.standard_normal((n, dim)).astype(F), rng.standard_normal((n, dim)).astype(F)
+    got = ctx.cross_cov(ctx.to_device(y), ctx.to_device(x), n, dim)
+    Y, X = y.astype(np.float64), x.astype(np.float64)
+    assert np.all(np.abs(got - Y.T @ X) <= 2 * n * 2.0 ** -53 * (np.abs(Y).T @ np.abs(X)) + 1e-300)
+    ctx.close()

@@ -369,80 +369,140 @@ static __global__ void __launch_bounds__(256) k_fill(T *__restrict__ p, int64_t 
 }
 
 // ---- rotation ------------------------------------------------------------------------------
-// y[i][a] = sum_b R[a][b] * x[i][b].  Generic dimension: one workgroup = 64 rows, x tile and
-// (a slab of) R staged in LDS, fused multiply-add accumulation in ascending b.
-static __global__ void __launch_bounds__(256) k_rotate_generic(const float *__restrict__ x, int64_t n,
-                                                        int64_t ld, int dim,
-                                                        const float *__restrict__ R,
-                                                        float *__restrict__ y) {
-    extern __shared__ float lds[];  // 64 * (dim + 1) floats of x
-    const int stride = dim + 1;
-    const int64_t row0 = (int64_t)blockIdx.x * 64;
-    for (int i = threadIdx.x; i < 64 * dim; i += 256) {
-        int r = i / dim, t = i % dim;
-        int64_t row = row0 + r;
-        lds[r * stride + t] = row < n ? x[row * ld + t] : 0.0f;
+// y[i][a] = sum_b R[a][b] * x[i][b] on the fp32 matrix cores (v_mfma_f32_32x32x2_f32: two fused multiply-adds in
+// ascending order, so the result is one chain over b) for dimensions and alignments that the bf16 kernels below do not
+// take.  A wave owns 32 rows and NB blocks of 32 outputs (grid y).  Step u of kc takes the components 8 kc + 2 u + h, lane
+// 32 h + r those of row r; rtab holds the same of R (zeros beyond dim on both sides), 1 KB per block and kc, read
+// through the vector cache two to eight kc ahead.  Against a thread per (row, four outputs) with its factors from LDS, the
+// same bits: 15,127 x 180 130 -> 24 us, 100,000 x 250 1230 -> 170, 3 x 248 189 -> 12.
+typedef float rot_acc __attribute__((ext_vector_type(16)));
+typedef float rot_piece __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ rot_piece rot_load(const float *__restrict__ p, int at, int dim) {
+    rot_piece v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (at + 4 <= dim) {
+        v = *reinterpret_cast<const rot_piece *>(p + at);
+    } else {
+        if (at < dim) v.x = p[at];
+        if (at + 1 < dim) v.y = p[at + 1];
+        if (at + 2 < dim) v.z = p[at + 2];
     }
-    __syncthreads();
-    // thread -> (row r = tid % 64, outputs a = tid / 64, +4, +8, ...)
-    const int r = threadIdx.x % 64;
-    const int64_t row = row0 + r;
-    for (int a = threadIdx.x / 64; a < dim; a += 4) {
-        const float *Ra = R + (size_t)a * dim;  // wave-uniform
-        float acc = 0.0f;
-        for (int b = 0; b < dim; ++b) acc = __builtin_fmaf(Ra[b], lds[r * stride + b], acc);
-        if (row < n) y[row * dim + a] = acc;
+    return v;
+}
+
+// rtab[kc][b][lane][u] = R[32 b + lane % 32][8 kc + 2 u + lane / 32], blocks = ceil(dim / 32)
+static __global__ void __launch_bounds__(256) k_rotate_prep_f32(const float *__restrict__ R, int dim, int blocks, int total,
+                                                                float4 *__restrict__ rtab) {
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= total) return;
+    const int lane = e % 64, b = (e / 64) % blocks, kc = e / (64 * blocks);
+    const int a = 32 * b + lane % 32, t = 8 * kc + lane / 32;
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = a < dim && t + 2 * u < dim ? R[(size_t)a * dim + t + 2 * u] : 0.0f;
+    rtab[e] = make_float4(v[0], v[1], v[2], v[3]);
+}
+
+template <int NB>
+static __global__ void __launch_bounds__(256) k_rotate_mfma_f32(const float *__restrict__ x, int64_t n, int64_t ld, int dim,
+                                                                int blocks, const float4 *__restrict__ rtab,
+                                                                float *__restrict__ y) {
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 32 + (lane & 31);
+    const float *__restrict__ xr = x + (row < n ? row : n - 1) * ld;  // past the end: the last row, not stored
+    const int b0 = (int)blockIdx.y * NB < blocks - NB ? (int)blockIdx.y * NB : blocks - NB, nkc = (dim + 7) / 8;
+    const float4 *__restrict__ rt = rtab + (size_t)b0 * 64 + lane;
+    rot_acc acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[b][v] = 0.0f;
+    // pieces of the next kAhead kc in flight
+    constexpr int kAhead = NB == 1 ? 8 : NB == 2 ? 4 : 2;
+    rot_piece xn[kAhead];
+    float4 rn[kAhead][NB];
+    auto fetch = [&](int kc, rot_piece &xv, float4(&rv)[NB]) {
+        xv = rot_load(xr, 8 * kc + 4 * h, dim);  // zeros past the end
+        const float4 *from = rt + (size_t)(kc < nkc ? kc : nkc - 1) * blocks * 64;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) rv[b] = from[b * 64];
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) fetch(i, xn[i], rn[i]);
+    for (int kc0 = 0; kc0 < nkc; kc0 += kAhead) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            // components {0..3} of lanes h = 0 and {4..7} of lanes h = 1 -> 2 u + h: the upper half of the first with the
+            // lower half of the second
+            const auto p02 = __builtin_amdgcn_permlane32_swap(__float_as_uint(xn[i].x), __float_as_uint(xn[i].y), false, false);
+            const auto p13 = __builtin_amdgcn_permlane32_swap(__float_as_uint(xn[i].z), __float_as_uint(xn[i].w), false, false);
+            const float xv[4] = {__uint_as_float(p02[0]), __uint_as_float(p13[0]), __uint_as_float(p02[1]), __uint_as_float(p13[1])};
+            float4 rv[NB];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) rv[b] = rn[i][b];
+            fetch(kc0 + i + kAhead, xn[i], rn[i]);
+            if (kc0 + i >= nkc) continue;  // uniform
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const float a = u == 0 ? rv[b].x : u == 1 ? rv[b].y : u == 2 ? rv[b].z : rv[b].w;
+                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, xv[u], acc[b], 0, 0, 0);
+                }
+        }
     }
+    // register v of a block holds output 32 b + 8 (v / 4) + 4 h + v % 4 of this lane's row
+    if (row >= n) return;
+    float *__restrict__ yr = y + row * dim;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int at = 32 * (b0 + b) + 8 * g + 4 * h;
+            const rot_piece v = {acc[b][4 * g], acc[b][4 * g + 1], acc[b][4 * g + 2], acc[b][4 * g + 3]};
+            if (at + 4 <= dim) {
+                *reinterpret_cast<rot_piece *>(yr + at) = v;
+            } else {
+                if (at < dim) yr[at] = v.x;
+                if (at + 1 < dim) yr[at + 1] = v.y;
+                if (at + 2 < dim) yr[at + 2] = v.z;
+            }
+        }
 }
 
 // ---- cross-covariance ----------------------------------------------------------------------
 // part[c][a][b] = sum over the rows of chunk c of yr[i][a] * x[i][b], accumulated in f64 in row
-// order; chunks are combined in chunk order by k_crosscov_reduce.  Generic dimension: a workgroup
-// takes one tile of up to 128 x 128 outputs of one chunk (grid.y walks the tiles row by row).
+// order; chunks are combined in chunk order by k_crosscov_reduce.  Fewer than 16 dimensions: a workgroup per chunk.
 static __global__ void __launch_bounds__(256) k_crosscov_partial(const float *__restrict__ yr,
                                                           const float *__restrict__ x, int64_t n,
                                                           int dim, int64_t rows_per_chunk,
                                                           double *__restrict__ part) {
-    __shared__ float ly[32 * 128], lx[32 * 128];
-    const int tiles = (dim + 127) / 128;
-    const int a0 = (int)(blockIdx.y / tiles) * 128, b0 = (int)(blockIdx.y % tiles) * 128;
-    const int da = dim - a0 < 128 ? dim - a0 : 128, db = dim - b0 < 128 ? dim - b0 : 128;
+    __shared__ float ly[128 * 15], lx[128 * 15];
     const int64_t lo = (int64_t)blockIdx.x * rows_per_chunk;
     const int64_t hi = lo + rows_per_chunk < n ? lo + rows_per_chunk : n;
-    const int total = da * db;
-    // each thread owns outputs e = tid, tid+256, ... of the tile (at most 64 per thread)
-    double acc[64];
-#pragma unroll
-    for (int u = 0; u < 64; ++u) acc[u] = 0.0;
-    for (int64_t r0 = lo; r0 < hi; r0 += 32) {
-        int rows = (int)((hi - r0) < 32 ? (hi - r0) : 32);
+    const int total = dim * dim, e = threadIdx.x, a = e / dim, b = e % dim;  // thread e owns output e
+    double acc = 0.0;
+    for (int64_t r0 = lo; r0 < hi; r0 += 128) {
+        const int rows = (int)((hi - r0) < 128 ? (hi - r0) : 128);
         __syncthreads();
-        for (int i = threadIdx.x; i < rows * da; i += 256) ly[i] = yr[(r0 + i / da) * dim + a0 + i % da];
-        for (int i = threadIdx.x; i < rows * db; i += 256) lx[i] = x[(r0 + i / db) * dim + b0 + i % db];
+        for (int i = threadIdx.x; i < rows * dim; i += 256) {
+            ly[i] = yr[r0 * dim + i];
+            lx[i] = x[r0 * dim + i];
+        }
         __syncthreads();
-#pragma unroll
-        for (int u = 0; u < 64; ++u) {
-            int e = threadIdx.x + u * 256;
-            if (e < total) {
-                int a = e / db, b = e % db;
-                double s = acc[u];
-#pragma unroll 1
-                for (int r = 0; r < rows; ++r) s += (double)ly[r * da + a] * (double)lx[r * db + b];
-                acc[u] = s;
-            }
+        if (e < total) {
+#pragma unroll 4
+            for (int r = 0; r < rows; ++r) acc += (double)ly[r * dim + a] * (double)lx[r * dim + b];
         }
     }
-    double *out = part + (size_t)blockIdx.x * dim * dim;
-#pragma unroll
-    for (int u = 0; u < 64; ++u) {
-        int e = threadIdx.x + u * 256;
-        if (e < total) out[(size_t)(a0 + e / db) * dim + b0 + e % db] = acc[u];
-    }
+    if (e < total) part[(size_t)blockIdx.x * total + e] = acc;
 }
 
-// The same partial sums on the f64 matrix cores (v_mfma_f64_16x16x4_f64) for dim a multiple of 16:
+// The same partial sums on the f64 matrix cores (v_mfma_f64_16x16x4_f64) for 16 dimensions and more:
 // a launch covers the output columns [b0 + 128 z, b0 + 128 z + 16 NT) for z = blockIdx.z and every
-// output row.
+// output row.  Where dim is no multiple of 16 the last tiles' operands beyond it are the row behind's first (they reach no
+// output that is stored), and the chunk's last rows, which may have none behind them, are read under a mask.
+// (15,127 x 180: 1655 -> 47 us against a thread per output with its factors from LDS.)
 // One wave owns the 32 output rows [16 ti, 16 ti + 32) of a chunk and NT column tiles; a
 // contraction step takes 4 rows: lane l supplies y[row + l/16][16 ti + l%16] and, per column
 // tile, x[row + l/16][16 tj + l%16], converted to f64 (the products are then exact).  The result
@@ -456,7 +516,7 @@ __global__ void __launch_bounds__(256) k_crosscov_mfma(const float *__restrict__
     // a wave owns TWO tiles of 16 output rows (32 dimensions of y), so every operand of x it
     // fetches feeds two matrix instructions
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ti = 2 * (blockIdx.y * 4 + w), nti = DIM / 16;
+    const int ti = 2 * (blockIdx.y * 4 + w), nti = (DIM + 15) / 16;
     if (ti >= nti) return;
     const bool two = ti + 1 < nti;  // without a second tile acc1 repeats acc0 and is not stored
     b0 += 128 * blockIdx.z;
@@ -473,8 +533,8 @@ __global__ void __launch_bounds__(256) k_crosscov_mfma(const float *__restrict__
     // offset (and the column tile as the instruction's immediate), so the loop spends no vector
     // instruction on them; the vector ALU and the matrix cores take turns on a SIMD, and what the
     // loop still needs of the first is the conversions to f64.
-    const int nsteps = (int)((hi - lo) / 4);  // steps in which every lane has a row
-    const int tail = (int)((hi - lo) % 4);
+    const int rows = (int)(hi - lo), whole = DIM % 16 ? (rows - 1) / 4 : rows / 4;
+    const int nsteps = whole;  // steps in which every lane has a row (and, ragged, there is a row behind them)
     uint32_t lane_off = 4u * ((uint32_t)kk * (uint32_t)DIM + (uint32_t)jj);
     const int64_t stepb = 16 * (int64_t)DIM;
     const char *ybase = reinterpret_cast<const char *>(yr + lo * (int64_t)DIM + 16 * ti);
@@ -533,14 +593,18 @@ __global__ void __launch_bounds__(256) k_crosscov_mfma(const float *__restrict__
             }
         }
     }
-    if (tail) {  // the chunk's last one to three rows: zeros in the lanes of the missing rows
-        const bool ok = kk < tail;
+    if (4 * nsteps < rows) {  // the chunk's last one to four rows: zeros in the lanes of missing rows and columns
+        const bool ok = 4 * nsteps + kk < rows;
         const char *yb = ybase + nsteps * stepb, *xb = xbase + nsteps * stepb;
-        const uint32_t off = ok ? lane_off : 4u * (uint32_t)jj;
-        const double ac0 = ok ? (double)ldf(yb, off, 0) : 0.0, ac1 = ok ? (double)ldf(yb + ysec, off, 0) : 0.0;
+        const uint32_t off = ok ? lane_off : 0u;
+        auto masked = [&](const char *base, int col, int imm) {
+            const bool in = ok && col < DIM;
+            return in ? (double)ldf(base, off, imm) : 0.0;
+        };
+        const double ac0 = masked(yb, 16 * ti + jj, 0), ac1 = masked(yb, 16 * ti + ysec / 4 + jj, ysec);
 #pragma unroll
         for (int tj = 0; tj < NT; ++tj) {
-            const double bc = ok ? (double)ldf(xb, off, 64 * tj) : 0.0;
+            const double bc = masked(xb, b0 + 16 * tj + jj, 64 * tj);
             acc0[tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac0, bc, acc0[tj], 0, 0, 0);
             acc1[tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac1, bc, acc1[tj], 0, 0, 0);
         }
@@ -550,8 +614,9 @@ __global__ void __launch_bounds__(256) k_crosscov_mfma(const float *__restrict__
     for (int tj = 0; tj < NT; ++tj)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            out[(size_t)(16 * ti + 4 * v + kk) * DIM + b0 + 16 * tj + jj] = acc0[tj][v];
-            if (two) out[(size_t)(16 * ti + 16 + 4 * v + kk) * DIM + b0 + 16 * tj + jj] = acc1[tj][v];
+            const int a = 16 * ti + 4 * v + kk, b = b0 + 16 * tj + jj;
+            if (a < DIM && b < DIM) out[(size_t)a * DIM + b] = acc0[tj][v];
+            if (two && a + 16 < DIM && b < DIM) out[(size_t)(a + 16) * DIM + b] = acc1[tj][v];
         }
 }
 

@@ -339,8 +339,8 @@ int32_t cross_cov_device(vq_ctx *ctx, const float *d_y, const float *d_x, int64_
     VQ_TRY(ensure(ctx, ctx->tmp_a, sizeof(double) * (size_t)chunks * total));
     VQ_TRY(ensure(ctx, ctx->tmp_b, sizeof(double) * (size_t)total));
     VQ_TRY(ensure(ctx, ctx->tmp_c, sizeof(double) * (size_t)total * ((chunks + 31) / 32)));
-    if (dim % 16 == 0) {
-        const int nt_all = dim / 16, full = dim / 128, rest = nt_all % 8;
+    if (dim >= 16) {
+        const int nt_all = (int)cdiv(dim, 16), full = nt_all / 8, rest = nt_all % 8;
         double *part = (double *)ctx->tmp_a.p;
 #define CROSSCOV(NT, B0, Z)                                                                                 \
     hipLaunchKernelGGL((vq::k_crosscov_mfma<NT>), dim3(chunks, (nt_all + 7) / 8, Z), dim3(256), 0, ctx->stream, \
@@ -358,8 +358,7 @@ int32_t cross_cov_device(vq_ctx *ctx, const float *d_y, const float *d_x, int64_
         }
 #undef CROSSCOV
     } else {
-        const int tiles = (dim + 127) / 128;
-        hipLaunchKernelGGL(vq::k_crosscov_partial, dim3(chunks, tiles * tiles), dim3(256), 0, ctx->stream, d_y, d_x,
+        hipLaunchKernelGGL(vq::k_crosscov_partial, dim3(chunks), dim3(256), 0, ctx->stream, d_y, d_x,
                            n, dim, rows_per_chunk, (double *)ctx->tmp_a.p);
     }
     // chunk sums in groups of 32 chunks, then the groups
@@ -430,7 +429,7 @@ int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t 
     if (n == 0) return VQ_OK;
     if (!d_x || !d_R || !d_y || n < 0 || dim <= 0 || ld < dim) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
     VQ_HIP(ctx, hipSetDevice(ctx->device));
-    // matrix-core kernel: dim a multiple of 32 up to 256, rows and output 16-byte aligned
+    // bf16 matrix cores: dim a multiple of 32 up to 256, rows and output 16-byte aligned
     if (dim % 32 == 0 && dim <= 256 && ld % 4 == 0 &&
         ((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_y)) & 15) == 0) {
         // operand table: 32 bytes per (output dimension, 4 input dimensions)
@@ -470,13 +469,20 @@ int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t 
         VQ_HIP(ctx, hipGetLastError());
         return VQ_OK;
     }
-    size_t lds = sizeof(float) * 64 * ((size_t)dim + 1);
-    if (lds > 160 * 1024) return fail(ctx, VQ_ERR_UNSUPPORTED, "rotation: dim %d too large", dim);
-    if (lds > 48 * 1024)
-        VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_rotate_generic),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(vq::k_rotate_generic, dim3(cdiv(n, 64)), dim3(256), lds, ctx->stream, d_x, n, ld,
-                       dim, d_R, d_y);
+    if (dim > 639) return fail(ctx, VQ_ERR_UNSUPPORTED, "rotation: dim %d too large", dim);
+    // up to four blocks of 32 outputs per wave, the same number in every wave (the last ones overlap), fewer where that
+    // leaves compute units without rows
+    const int blocks = (int)cdiv(dim, 32);
+    int per = 4;
+    while (per > 1 && (int64_t)cdiv(n, 128) * cdiv(blocks, per) < 256) per /= 2;
+    per = (int)cdiv(blocks, cdiv(blocks, per));
+    const unsigned groups = cdiv(blocks, per);
+    const int entries = (int)cdiv(dim, 8) * blocks * 64;
+    VQ_TRY(ensure(ctx, ctx->tmp_f, sizeof(float4) * (size_t)entries));
+    float4 *rtab = (float4 *)ctx->tmp_f.p;
+    hipLaunchKernelGGL(vq::k_rotate_prep_f32, dim3(cdiv(entries, 256)), dim3(256), 0, ctx->stream, d_R, dim, blocks, entries, rtab);
+    auto *kern = per == 1 ? vq::k_rotate_mfma_f32<1> : per == 2 ? vq::k_rotate_mfma_f32<2> : per == 3 ? vq::k_rotate_mfma_f32<3> : vq::k_rotate_mfma_f32<4>;
+    hipLaunchKernelGGL(kern, dim3(cdiv(n, 128), groups), dim3(256), 0, ctx->stream, d_x, n, ld, dim, blocks, (const float4 *)rtab, d_y);
     VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;
 }
