@@ -1,0 +1,49 @@
+"""More than 256 centroids chunk by chunk: blocks padded before the chunks, winners' distances from the assignment kernel or
+from the merge, whole pieces and remainders of its sums; fits on rows padded once, both means kernels: against the oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests import data
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+METRICS = [O.SQEUCLIDEAN, O.EUCLIDEAN, O.COSINE, O.MANHATTAN]
+
+
+@pytest.mark.parametrize("metric", METRICS)
+@pytest.mark.parametrize("n,m,sd,k,extra", [(700, 3, 10, 1030, 0), (600, 4, 20, 300, 1), (520, 4, 5, 2060, 0), (513, 4, 8, 2305, 0), (600, 1, 47, 258, 0),
+                                            (300, 2, 51, 513, 0), (257, 8, 2, 600, 0), (600, 2, 16, 1281, 2)])
+def test_encode(metric, n, m, sd, k, extra):
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    ctx.set_few_path(1)
+    rng = np.random.default_rng(n + sd + k)
+    buf = np.round(rng.standard_normal((n, m * sd + extra)) * 4).astype(F)  # ties inside and between chunks
+    cb = np.round(rng.standard_normal((m, k, sd)) * 4).astype(F)
+    buf[::9] = rng.standard_normal((len(buf[::9]), m * sd + extra))
+    buf[5] = 0.0
+    buf[7, 0] = np.nan
+    buf[11, -1 - extra] = np.inf
+    cb[0, 256, 0] = np.nan  # a chunk whose first distance is no number
+    cb[0, 3] = 0.0
+    codes = ctx.empty((n, m), np.uint16)
+    ctx.assign_u16(metric, ctx.to_device(buf), n, m * sd + extra, m, sd, k, ctx.to_device(cb), codes)
+    with np.errstate(all="ignore"):
+        want = O.pq_encode(metric, np.ascontiguousarray(buf[:, :m * sd]), cb)
+    assert np.array_equal(codes.download(), want.astype(np.uint16))
+    ctx.close()
+
+
+@pytest.mark.parametrize("n,m,sd,k", [(9000, 9, 3, 280), (8959, 3, 9, 280), (12_000, 2, 33, 260), (3000, 17, 10, 1100), (20_000, 1, 2, 300), (40_000, 2, 20, 300)])
+def test_fit(n, m, sd, k):
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    x = np.random.default_rng(n + sd).random((n, m * sd), dtype=F)
+    x[: n // 4] *= F(0.01)  # clusters of more than 1024 members
+    init, reseed = data.index_streams(n, m, k, 2, seed=5)
+    cb = ctx.empty((m, k, sd), F)
+    ctx.lbg_fit(ctx.to_device(x), n, m * sd, m, sd, k, 2, init, reseed, cb)
+    want = O.pq_fit(x, m, k, 2, init, reseed)["codebooks"]
+    assert np.array_equal(cb.download().view(np.uint32), want.view(np.uint32))
+    ctx.close()

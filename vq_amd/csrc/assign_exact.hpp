@@ -29,7 +29,7 @@ struct AssignArgs {
     int *changed;         // LBG mode: changed[s] set to 1 when any code of block s differs
     const int *done;      // LBG mode: blocks with done[s] != 0 are skipped
     const int *before = nullptr;  // LBG mode, instead of done: the changed flags of the pass before (0: skipped)
-    float *dist = nullptr;  // encode mode, k_assign_mfma8 only: [n][m] distance of the chosen centroid, or null
+    float *dist = nullptr;  // encode mode, k_assign_mfma8 and k_assign_static only: [n][m] distance of the chosen centroid, or null
     uint16_t *out16 = nullptr;  // encode mode, k_assign_mfma8 only: [n][8 m] chosen centroids as binary16, or null
     // A residual update that the pass applies before it scores the rows (single wide column block,
     // k_assign_mfma_wide_bf only): x[i] = src[i] - pend_cb[pend_codes[i]], where src is the rows
@@ -121,10 +121,10 @@ __device__ __forceinline__ void lds_centroid(const float *lds, int j, float (&c)
     }
 }
 
-// Argmin of one row's sub-vector against the k centroids held in LDS.
+// Argmin of one row's sub-vector against the k centroids held in LDS; dist: its distance.
 template <int SD, int METRIC>
 __device__ __forceinline__ int argmin_lds(const float (&x)[SD], const float *lds, const float *cn,
-                                          int k) {
+                                          int k, float &dist) {
     float c[SD];
     int best = 0;
     if constexpr (METRIC == M_SQ || METRIC == M_EUCLID) {
@@ -145,7 +145,8 @@ __device__ __forceinline__ int argmin_lds(const float (&x)[SD], const float *lds
             // its running minimum is the first element of the strictly decreasing chain of d2
             // minima whose root equals the root of the smallest d2.  Only when the previous
             // chain element shares that root can the answer be an earlier index: rescan.
-            float s = sqrtf(bd);
+            const float s = sqrtf(bd);
+            bd = s;
             if (sqrtf(pd) == s) {
                 for (int j = 0; j < best; ++j) {
                     lds_centroid<SD>(lds, j, c);
@@ -156,6 +157,7 @@ __device__ __forceinline__ int argmin_lds(const float (&x)[SD], const float *lds
                 }
             }
         }
+        dist = bd;
     } else if constexpr (METRIC == M_L1) {
         lds_centroid<SD>(lds, 0, c);
         float bd = d_l1<SD>(x, c);
@@ -167,6 +169,7 @@ __device__ __forceinline__ int argmin_lds(const float (&x)[SD], const float *lds
             bd = u ? d : bd;
             best = u ? j : best;
         }
+        dist = bd;
     } else {  // cosine, src/distances.rs:141-151
         float sa = 0.0f;
 #pragma unroll
@@ -188,6 +191,7 @@ __device__ __forceinline__ int argmin_lds(const float (&x)[SD], const float *lds
             bd = u ? d : bd;
             best = u ? j : best;
         }
+        dist = bd;
     }
     return best;
 }
@@ -278,7 +282,8 @@ __global__ void __launch_bounds__(256) k_assign_static(AssignArgs a, int sub_dim
         if constexpr (LBG) {
             if (block_done(a, s)) continue;  // uniform
         }
-        int best = argmin_lds<SD, METRIC>(x[g], lds + (size_t)g * k * SD, lds_cn + g * k, k);
+        float dist;
+        const int best = argmin_lds<SD, METRIC>(x[g], lds + (size_t)g * k * SD, lds_cn + g * k, k, dist);
         if constexpr (LBG) {
             uint8_t *p = a.codes + (size_t)s * a.n + row;
             if (*p != (uint8_t)best) {
@@ -290,6 +295,7 @@ __global__ void __launch_bounds__(256) k_assign_static(AssignArgs a, int sub_dim
                 packed |= (uint32_t)best << (8 * g);
             else
                 a.codes[row * a.m + s] = (uint8_t)best;
+            if (a.dist) a.dist[row * a.m + s] = dist;  // uniform
         }
     }
     if constexpr (!LBG && G == 4) {

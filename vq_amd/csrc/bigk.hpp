@@ -21,6 +21,7 @@
 #include <stdint.h>
 
 #include "assign_exact.hpp"
+#include "lbg_update.hpp"
 
 namespace vq {
 
@@ -39,39 +40,56 @@ static __global__ void k_chunk_tables(const float *__restrict__ cb, int m, int k
 
 // Distance of one row's sub-vector to one centroid in the reference's operation order
 // (src/distances.rs:129-152; the squared form of src/vector.rs:214-220 for the LBG).
+// Pieces of 16 components are loaded whole: a component at a time is a memory round trip each (11,523 x 48 blocks of
+// 16, k = 1258: 126 us per merge of four chunks, now 33).
 template <int METRIC>
 __device__ __forceinline__ float pair_distance(const float *__restrict__ x, const float *__restrict__ c, int sd) {
-    if constexpr (METRIC == M_SQ || METRIC == M_EUCLID) {
-        float acc = 0.0f;
-        for (int t = 0; t < sd; ++t) {
-            const float d = x[t] - c[t];
+    typedef float piece4 __attribute__((ext_vector_type(4), aligned(4)));
+    float acc = 0.0f, sa = 0.0f, sb = 0.0f;
+    auto step = [&](float xv, float cv) {
+        if constexpr (METRIC == M_COS) {
+            const float p = xv * cv;
+            acc = acc + p;
+            const float pa = xv * xv;
+            sa = sa + pa;
+            const float pb = cv * cv;
+            sb = sb + pb;
+        } else if constexpr (METRIC == M_L1) {
+            const float d = xv - cv;
+            acc = acc + fabsf(d);
+        } else {
+            const float d = xv - cv;
             const float p = d * d;
             acc = acc + p;
         }
-        return METRIC == M_EUCLID ? sqrtf(acc) : acc;
-    } else if constexpr (METRIC == M_L1) {
-        float acc = 0.0f;
-        for (int t = 0; t < sd; ++t) {
-            const float d = x[t] - c[t];
-            acc = acc + fabsf(d);
+    };
+    int t = 0;
+    auto pieces = [&](auto count) {
+        constexpr int P = decltype(count)::value;
+        for (; t + 4 * P <= sd; t += 4 * P) {
+            piece4 xv[P], cv[P];
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                xv[u] = *reinterpret_cast<const piece4 *>(x + t + 4 * u);
+                cv[u] = *reinterpret_cast<const piece4 *>(c + t + 4 * u);
+            }
+#pragma unroll
+            for (int u = 0; u < P; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) step(xv[u][e], cv[u][e]);
         }
-        return acc;
-    } else {
-        float dot = 0.0f, sa = 0.0f, sb = 0.0f;
-        for (int t = 0; t < sd; ++t) {
-            const float p = x[t] * c[t];
-            dot = dot + p;
-            const float pa = x[t] * x[t];
-            sa = sa + pa;
-            const float pb = c[t] * c[t];
-            sb = sb + pb;
-        }
+    };
+    pieces(std::integral_constant<int, 4>{});
+    pieces(std::integral_constant<int, 1>{});
+    for (; t < sd; ++t) step(x[t], c[t]);
+    if constexpr (METRIC == M_COS) {
         const float na = sqrtf(sa), nb = sqrtf(sb);
         const float den = na * nb;
-        const float q = dot / den;
+        const float q = acc / den;
         const float d = 1.0f - q;
         return (na == 0.0f || nb == 0.0f) ? 1.0f : d;
     }
+    return METRIC == M_EUCLID ? sqrtf(acc) : acc;
 }
 
 // One thread per (row, column block): folds the winners of `count` chunks from `base` on into the running
@@ -160,22 +178,32 @@ static __global__ void k_big_init(BigLbg st, int m) {
 // sort key of the pair: the row in bits 0-31, the code in the code_bits above them, the column
 // block above that.  The keys are written block by block in row order, so a stable sort on the
 // bits from 32 up lists every cluster's members in row order.
+// Eight column blocks per thread: their codes lie side by side in a row (a block at a time every row's line was
+// fetched once per block: 200,131 x 36 87 us, now 41).
+constexpr int kCommitBlocks = 8;
 static __global__ void __launch_bounds__(256) k_big_commit(BigLbg st, const uint16_t *__restrict__ fresh, int64_t n,
                                                            int m, int code_bits, uint64_t *__restrict__ keys) {
-    const int s = blockIdx.y;
+    const int s0 = blockIdx.y * kCommitBlocks, count = m - s0 < kCommitBlocks ? m - s0 : kCommitBlocks;
     const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (row >= n) return;
-    uint16_t *cur = st.codes + (size_t)s * n + row;
-    uint16_t c = *cur;
-    if (!st.done[s]) {
-        const uint16_t f = fresh[row * m + s];
-        if (f != c) {
-            *cur = f;
-            c = f;
+    uint16_t f[kCommitBlocks], c[kCommitBlocks];
+#pragma unroll
+    for (int u = 0; u < kCommitBlocks; ++u) {  // all loads in flight (past the last block: its again, not used)
+        const int s = s0 + (u < count ? u : count - 1);
+        f[u] = fresh[row * m + s];
+        c[u] = st.codes[(size_t)s * n + row];
+    }
+#pragma unroll
+    for (int u = 0; u < kCommitBlocks; ++u) {
+        if (u >= count) break;
+        const int s = s0 + u;
+        if (f[u] != c[u] && !st.done[s]) {
+            st.codes[(size_t)s * n + row] = f[u];
+            c[u] = f[u];
             mark_changed(st.changed + s);
         }
+        keys[(size_t)s * n + row] = ((uint64_t)s << (32 + code_bits)) | ((uint64_t)c[u] << 32) | (uint64_t)row;
     }
-    keys[(size_t)s * n + row] = ((uint64_t)s << (32 + code_bits)) | ((uint64_t)c << 32) | (uint64_t)row;
 }
 
 // Sorted keys -> first position and size of every cluster that has members.
@@ -268,6 +296,36 @@ static __global__ void __launch_bounds__(256) k_big_small_means(BigLbg st, const
             if (p + u < cnt) sum = sum + v[u];
     }
     *out = sum / __uint2float_rn(cnt);
+}
+
+// The same by two waves per cluster and tile of 32 components (grid z), where a cluster has 32 members on average:
+// 200,131 x 36 blocks of 3 (held in 8), k = 280 167 -> 123 us, which is the rate at which the lines of the rows come, a line per member.
+template <int VEC>
+static __global__ void __launch_bounds__(128) k_big_means_tile(BigLbg st, const uint64_t *__restrict__ sorted, const float *__restrict__ x,
+                                                               int64_t n, int64_t ld, int k, int sd, int width, int pieces,
+                                                               const uint32_t *__restrict__ reseed, int n_reseed,
+                                                               float *__restrict__ cb) {
+    const int s = blockIdx.y, j = blockIdx.x;
+    if (st.done[s]) return;
+    extern __shared__ float4 lds_tile[];
+    const int first = (int)blockIdx.z * width < sd - width ? (int)blockIdx.z * width : sd - width;
+    const size_t sj = (size_t)s * k + j;
+    const uint32_t cnt = st.count[sj];
+    const float *col = x + (int64_t)s * sd + first;
+    float *out = cb + sj * sd + first + threadIdx.x;
+    if (cnt > (uint32_t)kBigSeqMax) return;
+    if (cnt == 0) {
+        const int pos = st.ubase[s] + (int)st.empty_rank[sj];
+        if (pos >= n_reseed)
+            st.err[0] = 1;
+        else if ((int)threadIdx.x < width)
+            *out = col[(int64_t)reseed[(size_t)s * n_reseed + pos] * ld + threadIdx.x];
+        return;
+    }
+    const uint64_t *__restrict__ mem = sorted + (size_t)s * n + st.start[sj];
+    const float sum = member_tile_sum<128, VEC>(reinterpret_cast<float *>(lds_tile), col, ld, 0u, cnt, width, pieces,
+                                                [&](uint32_t p) { return (uint32_t)mem[p]; });
+    if ((int)threadIdx.x < width) *out = sum / __uint2float_rn(cnt);
 }
 
 // One workgroup per cluster above 1024 members.  Thread (p, l): part q0 + p of a round, component

@@ -55,6 +55,7 @@ struct vq_ctx {
     DevBuf tsvq_bsum, tsvq_segmaps;           // per block of groups: f64 sum; per run of groups: composed map
     int tsvq_var_path = 0;       // 0 = composed integer maps, 1 = one chain of adds per column
     DevBuf pad_x, pad_cb;        // rows and codebooks whose column blocks are padded to a multiple of 8 floats
+    DevBuf pad_rows;             // the same for a fit of more than 256 centroids, whose passes may pad slices of their own
     DevBuf mfma_tab, mfma_list, mfma_stat;  // tables, re-check list and counters of the matrix-core assignment
     int mfma_stat_cur = 0;       // which of the two sets of counters in mfma_stat the last pass used
     int recheck_src = 0;         // where the last pass counted its undecided pairs: 1 mfma_stat, 2 mfma_list, 3 the fixed scratch

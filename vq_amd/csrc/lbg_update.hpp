@@ -652,32 +652,24 @@ static __global__ void __launch_bounds__(256) k_lbg_leafsum_wide(LbgState st, co
     if (t < sd) st.leaf_sum[((size_t)s * st.leaf_cap + e.z) * sd + t] = acc;
 }
 
-// A workgroup per leaf and tile of up to 4 P components (grid z), P pieces of VEC floats per member: the threads
-// fetch a chunk of members into registers, eight loads of each in flight while the chunk before is added, and store
-// them transposed in LDS; a lane per component adds them in list order, sixteen members read ahead of the adds.
-// The last piece of a tile begins at the tile's end less VEC and the last tile at the block's end less its width, so that
-// pieces of any width are whole (what two of them share is written twice, with the same values).  Its time is a chain of memory round trips, one per chunk of 128
+// The sum of members lo .. hi - 1 of a list (row_of: position -> row) over a tile of up to VEC P components, by a
+// workgroup: P pieces of VEC floats per member; the threads fetch a chunk of members into registers, eight loads of each in
+// flight while the chunk before is added, and store them transposed in LDS (stage: width * (8 NT / P + 4) floats); a lane per
+// component adds them in list order, sixteen members read ahead of the adds.  xs: row 0's tile.  Returned in the lanes
+// below width.  The last piece of a tile begins at the tile's end less VEC, so that pieces of any width are whole (what
+// two of them share is written twice, with the same values).  Its time is a chain of memory round trips, one per chunk of 128
 // to 512 members, beside the adds: 7,930 x 300, k = 22 41 -> 17 us per launch, 50,019 x 28 blocks of 10, k = 78 110 -> 28.
 // (With chunks of twice the members by 256 threads the same, where the leaves are long; the LDS then holds half the leaves.)
-template <int NT, int VEC>
-static __global__ void __launch_bounds__(NT) k_lbg_leafsum_tile(LbgState st, const float *__restrict__ x, int64_t n, int64_t ld,
-                                                                int sd, int width, int pieces) {
-    const int s = blockIdx.y;
-    if (st.done[s]) return;
-    const int64_t leaf = blockIdx.x;
-    if (leaf >= st.nleaves[s]) return;  // uniform per workgroup
+template <int NT, int VEC, typename RowOf>
+__device__ __forceinline__ float member_tile_sum(float *stage, const float *__restrict__ xs, int64_t ld, uint32_t lo, uint32_t hi, int width,
+                                                 int pieces, RowOf row_of) {
     typedef float piece_t __attribute__((ext_vector_type(VEC), aligned(4)));
     constexpr int E = 8;
-    extern __shared__ float4 lds_tile[];
-    float *stage = reinterpret_cast<float *>(lds_tile);
     const int tid = threadIdx.x;
-    const int first = (int)blockIdx.z * width < sd - width ? (int)blockIdx.z * width : sd - width;
-    const uint2 d = st.leaf_desc[(size_t)s * st.leaf_cap + leaf];
-    const uint32_t *__restrict__ perm = st.perm + (size_t)s * n;
     const int step = NT / pieces, mine = tid / pieces, at = VEC * (tid % pieces);
     const int t0 = at + VEC <= width ? at : width - VEC;
     const bool fetches = mine < step;
-    const float *__restrict__ xs = x + (int64_t)s * sd + first + t0;
+    xs += t0;
     const uint32_t chunk = (uint32_t)(E * step), stride = chunk + 4;
     uint32_t row[E];
     piece_t v[E];
@@ -685,30 +677,30 @@ static __global__ void __launch_bounds__(NT) k_lbg_leafsum_tile(LbgState st, con
 #pragma unroll
         for (int i = 0; i < E; ++i) {
             const uint32_t q = p + (uint32_t)(mine + step * i);
-            row[i] = perm[q < d.y ? q : d.y - 1];
+            row[i] = row_of(q < hi ? q : hi - 1);
         }
     };
     auto load = [&](uint32_t p) {
 #pragma unroll
         for (int i = 0; i < E; ++i)
-            if (p + (uint32_t)(step * i) < d.y) v[i] = *reinterpret_cast<const piece_t *>(xs + (int64_t)row[i] * ld);
+            if (p + (uint32_t)(step * i) < hi) v[i] = *reinterpret_cast<const piece_t *>(xs + (int64_t)row[i] * ld);
     };
     float acc = 0.0f;
-    if (fetches && d.x < d.y) {
-        rows(d.x);
-        load(d.x);
+    if (fetches && lo < hi) {
+        rows(lo);
+        load(lo);
     }
-    for (uint32_t p = d.x; p < d.y; p += chunk) {
-        const uint32_t cm = d.y - p < chunk ? d.y - p : chunk;
-        if (fetches && p + chunk < d.y) rows(p + chunk);
-        if (p != d.x) __syncthreads();  // the chunk before has been added
+    for (uint32_t p = lo; p < hi; p += chunk) {
+        const uint32_t cm = hi - p < chunk ? hi - p : chunk;
+        if (fetches && p + chunk < hi) rows(p + chunk);
+        if (p != lo) __syncthreads();  // the chunk before has been added
         if (fetches) {
 #pragma unroll
             for (int i = 0; i < E; ++i)
                 if ((uint32_t)(step * i) < cm)
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) stage[(uint32_t)(t0 + e) * stride + (uint32_t)(mine + step * i)] = v[i][e];
-            if (p + chunk < d.y) load(p + chunk);
+            if (p + chunk < hi) load(p + chunk);
         }
         __syncthreads();
         if (tid < width) {
@@ -729,7 +721,24 @@ static __global__ void __launch_bounds__(NT) k_lbg_leafsum_tile(LbgState st, con
             for (; mbr < cm; ++mbr) acc = acc + col[mbr];
         }
     }
-    if (tid < width) st.leaf_sum[((size_t)s * st.leaf_cap + leaf) * sd + first + tid] = acc;
+    return acc;
+}
+
+// A workgroup per leaf and tile of components (grid z); the last tile begins at the block's end less its width.
+template <int NT, int VEC>
+static __global__ void __launch_bounds__(NT) k_lbg_leafsum_tile(LbgState st, const float *__restrict__ x, int64_t n, int64_t ld,
+                                                                int sd, int width, int pieces) {
+    const int s = blockIdx.y;
+    if (st.done[s]) return;
+    const int64_t leaf = blockIdx.x;
+    if (leaf >= st.nleaves[s]) return;  // uniform per workgroup
+    extern __shared__ float4 lds_tile[];
+    const int first = (int)blockIdx.z * width < sd - width ? (int)blockIdx.z * width : sd - width;
+    const uint2 d = st.leaf_desc[(size_t)s * st.leaf_cap + leaf];
+    const uint32_t *__restrict__ perm = st.perm + (size_t)s * n;
+    const float acc = member_tile_sum<NT, VEC>(reinterpret_cast<float *>(lds_tile), x + (int64_t)s * sd + first, ld, d.x, d.y, width, pieces,
+                                               [&](uint32_t p) { return perm[p]; });
+    if ((int)threadIdx.x < width) st.leaf_sum[((size_t)s * st.leaf_cap + leaf) * sd + first + threadIdx.x] = acc;
 }
 
 // Few, long leaves (the small clusters beside the streaming kernel: up to 1024 members each): one

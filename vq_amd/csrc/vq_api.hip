@@ -510,6 +510,7 @@ int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bo
         mfma_wide_applicable<vq::M_SQ, true>(ctx, a, sd))
         return 0;
     const int sdp = (sd + 7) / 8 * 8;
+    if (sdp == sd && a.ld % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.cb)) & 15) == 0) return 0;
     // the limits of those kernels
     if ((int64_t)a.m * sdp > (1 << 20) || sdp > (1 << 16) || a.n * a.m >= (1LL << 32)) return 0;
     const int w = static_width(sd);
@@ -891,7 +892,14 @@ int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, i
                            ctx->stream, d_codebooks, (int64_t)m * k, sd, cnorm);
         a.cnorm = cnorm;
     }
-    if (!sdp) return launch_assign<false>(ctx, metric, a, sd);
+    if (!sdp) {
+        // k_assign_static has the distance too: Manhattan, and blocks too narrow for the other kernels
+        if (d_dist && dist_written && !mfma8 && !pend && (metric == VQ_MANHATTAN ? static_width(sd) != 0 : sd <= 6)) {
+            a.dist = d_dist;
+            *dist_written = true;
+        }
+        return launch_assign<false>(ctx, metric, a, sd);
+    }
     // padded a slice of rows at a time: the copy is read back from the memory-side cache (256 MB)
     // and the workspace stays small whatever n is
     const int64_t row_bytes = (int64_t)sizeof(float) * m * sdp;
@@ -960,7 +968,7 @@ int32_t vq_ctx_destroy(vq_ctx *ctx) {
     if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     DevBuf *bufs[] = {&ctx->flags, &ctx->tables, &ctx->hist, &ctx->perm, &ctx->leaf_desc,
                       &ctx->leaf_sum, &ctx->codes, &ctx->idx, &ctx->reseed, &ctx->cnorm,
-                      &ctx->seg, &ctx->part_sum, &ctx->pad_x, &ctx->pad_cb, &ctx->pipe_dev, &ctx->pipe_rot, &ctx->mfma_tab, &ctx->mfma_list, &ctx->mfma_stat, &ctx->tsvq_sq, &ctx->tsvq_split, &ctx->tsvq_level, &ctx->tsvq_means, &ctx->tsvq_scan, &ctx->tsvq_km, &ctx->tsvq_bsum, &ctx->tsvq_segmaps, &ctx->tsvq_gsum, &ctx->tsvq_guess, &ctx->tsvq_maps, &ctx->tmp_a, &ctx->tmp_b, &ctx->tmp_c, &ctx->tmp_d, &ctx->tmp_e, &ctx->tmp_f,
+                      &ctx->seg, &ctx->part_sum, &ctx->pad_x, &ctx->pad_cb, &ctx->pad_rows, &ctx->pipe_dev, &ctx->pipe_rot, &ctx->mfma_tab, &ctx->mfma_list, &ctx->mfma_stat, &ctx->tsvq_sq, &ctx->tsvq_split, &ctx->tsvq_level, &ctx->tsvq_means, &ctx->tsvq_scan, &ctx->tsvq_km, &ctx->tsvq_bsum, &ctx->tsvq_segmaps, &ctx->tsvq_gsum, &ctx->tsvq_guess, &ctx->tsvq_maps, &ctx->tmp_a, &ctx->tmp_b, &ctx->tmp_c, &ctx->tmp_d, &ctx->tmp_e, &ctx->tmp_f,
                       &ctx->big_chunk, &ctx->big_win, &ctx->big_wind, &ctx->big_best, &ctx->big_fresh, &ctx->big_codes, &ctx->big_keys,
                       &ctx->big_sorted, &ctx->big_sort_tmp, &ctx->big_tables, &ctx->big_flags};
     for (DevBuf *b : bufs)
@@ -1262,9 +1270,26 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
         if (h_reseed_stream[i] >= (uint64_t)n)
             return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter: reseed index %u out of range", h_reseed_stream[i]);
     VQ_HIP(ctx, hipSetDevice(ctx->device));
-    if (k > vq::kMaxK)
+    if (k > vq::kMaxK) {
+        // rows that every pass would pad, once for the fit, as below (200,131 x 36 blocks of 3, k = 280: 62 of 920 us per
+        // iteration; 5,851 x 23 of 9, k = 1953: 97 of 400)
+        const int w = max_iters > 0 ? encode_pad_width(ctx, VQ_SQEUCLIDEAN, d_x, n, ld, m, sd, vq::kMaxK, d_codebooks) : 0;
+        int32_t rc = VQ_ERR_OOM;
+        if (w && ensure(ctx, ctx->pad_rows, sizeof(float) * ((size_t)n * m + (size_t)m * k) * w) == VQ_OK) {
+            float *px = (float *)ctx->pad_rows.p, *pcb = px + (size_t)n * m * w;
+            launch_pad(ctx, d_x, n, ld, m, sd, w, px);
+            rc = vqh::lbg_fit_big(ctx, px, n, (int64_t)m * w, m, w, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, pcb,
+                                  h_iters_run, h_reseeds_used);
+            if (rc == VQ_OK) unpad_rows(ctx, pcb, (int64_t)m * k, sd, w, d_codebooks);
+        }
+        if (rc == VQ_ERR_OOM || ctx->pad_rows.cap > kPadKeep) {
+            const int32_t gone = release(ctx, ctx->pad_rows);
+            if (rc == VQ_OK) rc = gone;
+        }
+        if (rc != VQ_ERR_OOM) return rc;
         return vqh::lbg_fit_big(ctx, d_x, n, ld, m, sd, k, max_iters, h_init_idx, h_reseed_stream, n_reseed,
                                 d_codebooks, h_iters_run, h_reseeds_used);
+    }
     vq::AssignArgs shape;
     shape.x = d_x;
     shape.n = n;

@@ -49,11 +49,12 @@ int32_t launch_big(vq_ctx *ctx, int metric, const float *d_x, int64_t n, int64_t
     return VQ_OK;
 }
 
-// Blocks of 8 or 16 floats, or of a width that an encode pads to one of them (a slice of rows at a time).  *done: it ran.
+// Blocks of 8 or 16 floats in one pass, blocks of a width that an encode pads padded first (a slice of rows at a time).
+// *done: it ran.
 int32_t assign_big(vq_ctx *ctx, int metric, const float *d_x, int64_t n, int64_t ld, int m, int sd, int k,
                    const float *d_codebooks, uint16_t *d_codes, bool *done) {
     *done = false;
-    if (ctx->assign_path == 1 || sd > 16 || metric == VQ_MANHATTAN) return VQ_OK;
+    if (ctx->assign_path == 1 || metric == VQ_MANHATTAN) return VQ_OK;
     auto fits = [&](int w) { return w == 8 ? k <= vq::kBig8Max : w == 16 && k <= vq::kLds16Max; };
     // float4 centroid loads; 32 rows within 32-bit byte offsets
     if (fits(sd) && (reinterpret_cast<uintptr_t>(d_codebooks) & 15) == 0 && ld <= (1 << 20)) {
@@ -61,7 +62,7 @@ int32_t assign_big(vq_ctx *ctx, int metric, const float *d_x, int64_t n, int64_t
         return launch_big(ctx, metric, d_x, n, ld, m, sd, k, d_codebooks, d_codes);
     }
     const int sdp = encode_pad_width(ctx, metric, d_x, n, ld, m, sd, vq::kChunk, d_codebooks);
-    if (!fits(sdp)) return VQ_OK;
+    if (!sdp) return VQ_OK;
     *done = true;
     const int64_t row_bytes = (int64_t)sizeof(float) * m * sdp;
     const int64_t slice = std::min<int64_t>(n, std::max<int64_t>(4096, kPadSlice / row_bytes / 4096 * 4096));
@@ -72,7 +73,10 @@ int32_t assign_big(vq_ctx *ctx, int metric, const float *d_x, int64_t n, int64_t
     for (int64_t r0 = 0; r0 < n; r0 += slice) {
         const int64_t rows = std::min(slice, n - r0);
         pad_blocks(ctx, d_x + r0 * ld, rows, ld, m, sd, sdp, px);
-        VQ_TRY(launch_big(ctx, metric, px, rows, (int64_t)m * sdp, m, sdp, k, pcb, d_codes + r0 * m));
+        if (fits(sdp))
+            VQ_TRY(launch_big(ctx, metric, px, rows, (int64_t)m * sdp, m, sdp, k, pcb, d_codes + r0 * m));
+        else  // chunk by chunk
+            VQ_TRY(assign_codes_u16(ctx, metric, px, rows, (int64_t)m * sdp, m, sdp, k, pcb, d_codes + r0 * m, nullptr, nullptr));
     }
     VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;
@@ -221,7 +225,7 @@ int32_t lbg_fit_big(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_
             VQ_TRY(assign_codes_u16(ctx, VQ_SQEUCLIDEAN, d_x, n, ld, m, sd, k, d_codebooks, fresh));
         }
         ProfSpan sp(ctx, VQ_PROF_LBG_UPDATE);
-        hipLaunchKernelGGL(vq::k_big_commit, dim3(cdiv(n, 256), m), dim3(256), 0, st, S, (const uint16_t *)fresh, n, m,
+        hipLaunchKernelGGL(vq::k_big_commit, dim3(cdiv(n, 256), cdiv(m, vq::kCommitBlocks)), dim3(256), 0, st, S, (const uint16_t *)fresh, n, m,
                            code_bits, keys);
         VQ_HIP(ctx, hipGetLastError());
         VQ_HIP(ctx, rocprim::radix_sort_keys(ctx->big_sort_tmp.p, sort_bytes, keys, sorted, pairs, 32u, end_bit, st));
@@ -229,9 +233,18 @@ int32_t lbg_fit_big(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_
         hipLaunchKernelGGL(vq::k_big_bounds, dim3(cdiv((int64_t)pairs, 256)), dim3(256), 0, st, S,
                            (const uint64_t *)sorted, n, m, k, code_bits);
         hipLaunchKernelGGL(vq::k_big_plan, dim3(m), dim3(256), 0, st, S, k);
-        hipLaunchKernelGGL(vq::k_big_small_means, dim3(cdiv((int64_t)k * sd, 256), m), dim3(256), 0, st, S,
-                           (const uint64_t *)sorted, d_x, n, ld, k, sd, (const uint32_t *)ctx->reseed.p, n_reseed,
-                           d_codebooks);
+        if (n >= 32 * (int64_t)k) {  // two waves per cluster and 32 components
+            const int tiles = (int)cdiv(sd, 32), width = tiles == 1 ? sd : (int)cdiv(cdiv(sd, tiles), 4) * 4;
+            const int vec = sd >= 4 ? 4 : 1, pieces = (int)cdiv(width, vec);
+            const size_t lds = sizeof(float) * (size_t)width * (8 * (128 / pieces) + 4);
+            hipLaunchKernelGGL(vec == 4 ? vq::k_big_means_tile<4> : vq::k_big_means_tile<1>, dim3(k, m, cdiv(sd, width)), dim3(128), lds, st, S,
+                               (const uint64_t *)sorted, d_x, n, ld, k, sd, width, pieces, (const uint32_t *)ctx->reseed.p,
+                               n_reseed, d_codebooks);
+        } else {
+            hipLaunchKernelGGL(vq::k_big_small_means, dim3(cdiv((int64_t)k * sd, 256), m), dim3(256), 0, st, S,
+                               (const uint64_t *)sorted, d_x, n, ld, k, sd, (const uint32_t *)ctx->reseed.p, n_reseed,
+                               d_codebooks);
+        }
         hipLaunchKernelGGL(vq::k_big_large_means, dim3(big_cap, m), dim3(256), 0, st, S, (const uint64_t *)sorted, d_x,
                            n, ld, k, sd, d_codebooks);
         hipLaunchKernelGGL(vq::k_big_advance, dim3(cdiv(m, 64)), dim3(64), 0, st, S, m);
