@@ -14,6 +14,7 @@
 #include <stdint.h>
 
 #include "assign_exact.hpp"
+#include "member_tile.hpp"
 
 namespace vq {
 
@@ -156,39 +157,22 @@ static __global__ void __launch_bounds__(256) k_seg_mean_wg(const float *__restr
     if (q == 0 && c < sd) out[(out_first + g) * sd + c] = tree[0][t] / __uint2float_rn(info.z);
 }
 
-// One lane per (segment, dimension): sequential sum of squared deviations in row order.
-// seg_range[g] = {lo, hi} positions in perm; mean of segment g at means[(first + g) * dim].
-static __global__ void __launch_bounds__(64) k_seg_variance(const uint32_t *__restrict__ perm,
-                                                     const uint2 *__restrict__ seg_range, int nseg,
-                                                     const float *__restrict__ means, int64_t first,
-                                                     const float *__restrict__ x, int64_t ld, int dim,
-                                                     float *__restrict__ var) {
-    int64_t gid = (int64_t)blockIdx.x * 64 + threadIdx.x;
-    int g = (int)(gid / dim);
-    int t = (int)(gid % dim);
-    if (g >= nseg) return;
-    uint2 r = seg_range[g];
-    const float mu = means[(first + g) * dim + t];
-    const float *__restrict__ xc = x + t;
-    float acc = 0.0f;
-    uint32_t p = r.x;
-    for (; p + 16 <= r.y; p += 16) {
-        float v[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = xc[(int64_t)perm[p + u] * ld];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            float d = v[u] - mu;
-            float q = d * d;
-            acc = acc + q;
-        }
-    }
-    for (; p < r.y; ++p) {
-        float d = xc[(int64_t)perm[p] * ld] - mu;
-        float q = d * d;
-        acc = acc + q;
-    }
-    var[(size_t)g * dim + t] = acc;
+// Sums of squared deviations in row order, a workgroup per segment and tile of up to 16 components (grid y; the last
+// one begins at dim less its width): seg_range[g] = {lo, hi} positions in perm; mean of segment g at means[(first + g) * dim].
+// Bound by the chain of adds, 3 ns a row, and the first chunk's memory round trips.  Against one workgroup per segment with all
+// columns, whose one lane per column read its squares one by one: a root of 5,964 x 100 90 -> 25 us.
+template <int VEC>
+static __global__ void __launch_bounds__(256) k_seg_variance_tile(const uint32_t *__restrict__ perm, const uint2 *__restrict__ seg_range,
+                                                                 const float *__restrict__ means, int64_t first,
+                                                                 const float *__restrict__ x, int64_t ld, int dim, int width, int pieces,
+                                                                 float *__restrict__ var) {
+    extern __shared__ float4 lds_var[];
+    const int g = blockIdx.x;
+    const int c0 = (int)blockIdx.y * width < dim - width ? (int)blockIdx.y * width : dim - width;
+    const uint2 r = seg_range[g];
+    const float sum = member_tile_sum<256, VEC, true>(reinterpret_cast<float *>(lds_var), x + c0, ld, r.x, r.y, width, pieces,
+                                                      [&](uint32_t p) { return perm[p]; }, means + (first + g) * dim + c0);
+    if ((int)threadIdx.x < width) var[(size_t)g * dim + c0 + threadIdx.x] = sum;
 }
 
 // ---- per-dimension sums of squared deviations in two steps (dim a multiple of 8) --------------
@@ -779,150 +763,7 @@ static __global__ void __launch_bounds__(256) k_seg_chain_compose(const uint32_t
     if (lane == 0) var[(size_t)g * dim + c] = S;
 }
 
-// The same sums with everything but the adds taken off the chain of dependent adds.  One workgroup
-// of 1024 threads per segment: all threads fetch rows (16-byte pieces, whole rows contiguous)
-// eight chunks ahead into registers, turn them into squared deviations (v - mean)^2 — the same
-// two roundings as in the chain — and hand those over through two LDS tiles; threads 0..dim-1
-// add the squares of the current tile in row order, one add per row.  A chunk is 8192 / dim rows;
-// about 512 rows (256 KB at dim = 128) are in flight per workgroup, which is what one chain of adds
-// consumes per memory round trip.  The barrier waits for LDS only, so the loads in flight are not
-// drained.
-constexpr int kVarStage = 8192;  // floats per LDS tile
-constexpr int kVarAhead = 8;     // chunks in flight
-
 __device__ __forceinline__ void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// acc + the squares of one component over the rows of one LDS tile, in row order.  DIM > 0: the row
-// stride as a constant, so that the reads pair up with constant offsets and the next sixteen
-// values are on their way while sixteen are added; DIM = 0: any stride.
-template <int DIM>
-__device__ __forceinline__ float seg_variance_chunk(const float *t, int rows, int dim, float acc) {
-    const int stride = DIM > 0 ? DIM : dim;
-    int r = 0;
-    if (rows >= 16) {
-        float v[16];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = t[q * stride];
-        for (; r + 32 <= rows; r += 16) {
-            float w[16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) w[q] = t[(r + 16 + q) * stride];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc = acc + v[q];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) v[q] = w[q];
-        }
-#pragma unroll
-        for (int q = 0; q < 16; ++q) acc = acc + v[q];
-        r += 16;
-    }
-    for (; r < rows; ++r) acc = acc + t[r * stride];
-    return acc;
-}
-
-template <int DIM>
-static __global__ void __launch_bounds__(1024) k_seg_variance_wg(const uint32_t *__restrict__ perm,
-                                                                const uint2 *__restrict__ seg_range,
-                                                                const float *__restrict__ means, int64_t first,
-                                                                const float *__restrict__ x, int64_t ld, int dim,
-                                                                float *__restrict__ var) {
-    __shared__ float4 tile[2][kVarStage / 4];
-    const int g = blockIdx.x, tid = threadIdx.x;
-    const uint2 range = seg_range[g];
-    const uint32_t count = range.y - range.x;
-    const int ppr = dim / 4;                  // 16-byte pieces per row
-    const int R = kVarStage / dim;            // rows per chunk
-    const int pieces = R * ppr;               // pieces per chunk (<= 2048)
-    const int nch = (int)((count + R - 1) / R);
-    // this thread's two pieces of every chunk
-    int rr[2], pc[2];
-    bool has[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int e = tid + 1024 * j;
-        has[j] = e < pieces;
-        rr[j] = has[j] ? e / ppr : 0;
-        pc[j] = has[j] ? e % ppr : 0;
-    }
-    if (count == 0) {  // uniform
-        if (tid < dim) var[(size_t)g * dim + tid] = 0.0f;
-        return;
-    }
-    const uint32_t *pm = perm + range.x;
-    // Loads are unconditional (positions clamped into the segment; surplus rows are fetched and
-    // never read): loads under a branch would make the compiler wait for every outstanding load
-    // at each use instead of counting them.  The rings are plain arrays with constant indices.
-    // (Eight named slots instead of an array: an array of this size is left in scratch memory.)
-    const float *xp0 = x + 4 * pc[0], *xp1 = x + 4 * pc[1];
-    // the means of this thread's columns
-    const float *mrow = means + (first + g) * dim;
-    const float4 mu0 = *reinterpret_cast<const float4 *>(mrow + 4 * pc[0]);
-    const float4 mu1 = *reinterpret_cast<const float4 *>(mrow + 4 * pc[1]);
-    auto sq_dev = [](float4 v, float4 m) {
-        float4 d, p;
-        d.x = v.x - m.x;
-        d.y = v.y - m.y;
-        d.z = v.z - m.z;
-        d.w = v.w - m.w;
-        p.x = d.x * d.x;
-        p.y = d.y * d.y;
-        p.z = d.z * d.z;
-        p.w = d.w * d.w;
-        return p;
-    };
-#define VAR_DECL(S) uint32_t ida_##S, idb_##S; float4 xa_##S, xb_##S;
-    VAR_DECL(0) VAR_DECL(1) VAR_DECL(2) VAR_DECL(3) VAR_DECL(4) VAR_DECL(5) VAR_DECL(6) VAR_DECL(7)
-#define VAR_IDS(S, chunk)                                                     \
-    {                                                                         \
-        const uint32_t m0 = (uint32_t)(chunk) * R + rr[0], m1 = (uint32_t)(chunk) * R + rr[1]; \
-        ida_##S = pm[m0 < count ? m0 : count - 1];                            \
-        idb_##S = pm[m1 < count ? m1 : count - 1];                            \
-    }
-#define VAR_ROWS(S)                                                           \
-    {                                                                         \
-        xa_##S = *reinterpret_cast<const float4 *>(xp0 + (int64_t)ida_##S * ld); \
-        xb_##S = *reinterpret_cast<const float4 *>(xp1 + (int64_t)idb_##S * ld); \
-    }
-#define VAR_STORE(buf, S)                                                     \
-    {                                                                         \
-        if (has[0]) tile[buf][rr[0] * ppr + pc[0]] = sq_dev(xa_##S, mu0);     \
-        if (has[1]) tile[buf][rr[1] * ppr + pc[1]] = sq_dev(xb_##S, mu1);     \
-    }
-    // prologue: ids of chunks 0..15, rows of chunks 0..7, chunk 0 in LDS
-    VAR_IDS(0, 0) VAR_IDS(1, 1) VAR_IDS(2, 2) VAR_IDS(3, 3) VAR_IDS(4, 4) VAR_IDS(5, 5) VAR_IDS(6, 6) VAR_IDS(7, 7)
-#define VAR_PRO(S) VAR_ROWS(S) VAR_IDS(S, S + kVarAhead)
-    VAR_PRO(0) VAR_PRO(1) VAR_PRO(2) VAR_PRO(3) VAR_PRO(4) VAR_PRO(5) VAR_PRO(6) VAR_PRO(7)
-    VAR_STORE(0, 0)
-    lds_only_barrier();
-    float acc = 0.0f;
-    // One step: rows of chunk i + 8 into the slot chunk i has left, ids of chunk i + 16 behind
-    // them; chunk i + 1 (fetched seven steps ago) into the other tile; chunk i added.  Chunks past
-    // the end run empty, so every thread reaches every barrier.
-#define VAR_STEP(S, SN)                                                       \
-    {                                                                         \
-        const int i = base + S;                                               \
-        VAR_ROWS(S)                                                           \
-        VAR_IDS(S, i + 2 * kVarAhead)                                         \
-        VAR_STORE((i + 1) & 1, SN)                                            \
-        if (tid < dim && i < nch) {                                           \
-            const float *t = reinterpret_cast<const float *>(tile[i & 1]) + tid; \
-            const int rows = (int)(((uint32_t)(i + 1) * R <= count) ? R : count - (uint32_t)i * R); \
-            acc = seg_variance_chunk<DIM>(t, rows, dim, acc);                 \
-        }                                                                     \
-        lds_only_barrier();                                                   \
-    }
-    for (int base = 0; base < nch; base += kVarAhead) {
-        VAR_STEP(0, 1) VAR_STEP(1, 2) VAR_STEP(2, 3) VAR_STEP(3, 4)
-        VAR_STEP(4, 5) VAR_STEP(5, 6) VAR_STEP(6, 7) VAR_STEP(7, 0)
-    }
-#undef VAR_DECL
-#undef VAR_PRO
-#undef VAR_STEP
-#undef VAR_IDS
-#undef VAR_ROWS
-#undef VAR_STORE
-    if (tid < dim) var[(size_t)g * dim + tid] = acc;
-}
 
 __device__ __forceinline__ int find_segment(const uint2 *__restrict__ seg_range, int nseg, uint32_t p) {
     // segments are sorted by position and disjoint; returns -1 when p lies in none

@@ -200,11 +200,11 @@ int32_t vq_tsvq_build_kmeans(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
     return tsvq_build_impl(ctx, d_x, n, ld, dim, max_depth, &km, out);
 }
 
-// Levels whose longest node is no longer than this: a workgroup per node (k_seg_variance_wg, 11 ns per row of
-// 128 and node, one launch) instead of the composed maps (four launches, 115 us at one node of 100,000 rows,
-// 62 at 16 nodes, 275 at 512, where the walks over many short columns cost most): 16 nodes of 6,250 rows
-// 78 and 62 us, 32 of 3,125 44 and 71, 512 of 195 22 and 275
-constexpr uint32_t kVarWgRows = 4096;
+// Levels whose longest node is no longer than this: a workgroup per node and 16 columns (k_seg_variance_tile, one launch,
+// 3-6 ns per row of the longest node) instead of the composed maps (four launches, 45 us and what the columns take).  Builds
+// with 4096 / 8192 / 16,384 rows: 100,000 x 16 641 / 661 / 675 us, 40,000 x 96 692 / 690 / 707, 220,611 x 128 1624 / 1567 / 1556,
+// 60,000 x 256 1064 / 1050 / 1065.
+static uint32_t var_tile_rows(int32_t dim) { return dim >= 96 ? 8192 : 4096; }
 
 // The build on validated arguments.  real_dim: the components that count; the others, up to dim, are zeros.
 static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t dim, int32_t real_dim,
@@ -218,14 +218,10 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     if (!d_x || n < 0 || dim <= 0 || ld < dim || max_depth < 0) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
     if (n >= (1LL << 31)) return fail(ctx, VQ_ERR_UNSUPPORTED, "n must be below 2^31");
     VQ_HIP(ctx, hipSetDevice(ctx->device));
-    // The variances are made by kernels for rows of whole groups of eight components (the composed maps) or of whole,
-    // aligned 16-byte pieces (k_seg_variance_wg).  Other rows are copied once with zeros behind them, for all levels: a
-    // column of zeros has the variance 0 and takes no part in the choice of the split dimension.  Builds of nine
-    // levels over the rows as they are (a lane per column that adds its squares one after the other; whole pieces: a
-    // workgroup per node) against the copy: 600,000 x 50 55.7 -> 2.6 ms, 20,000 2.17 -> 0.83, 2,000 0.585 -> 0.605; 600,000 x
-    // 100 17.7 -> 3.3 ms, 20,000 1.16 -> 0.88, 5,000 0.66 -> 0.71.
-    const bool whole = dim % 4 == 0 && dim <= 1024 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;
-    if (!km && dim % 8 != 0 && dim < (1 << 20) && n > (whole ? 2 * (int64_t)kVarWgRows : (int64_t)kVarWgRows / 2)) {
+    // The composed maps take rows of whole groups of eight components.  Other rows with nodes that need them are copied
+    // once with zeros behind them, for all levels: a column of zeros has the variance 0 and takes no part in the choice of the
+    // split dimension.  (600,000 x 50, nine levels: 55.7 -> 2.6 ms against a lane per column that adds its squares one after the other.)
+    if (!km && dim % 8 != 0 && dim < (1 << 20) && n > (int64_t)var_tile_rows(dim)) {
         const int32_t dimp = (dim + 7) / 8 * 8;
         int32_t rc = ensure(ctx, ctx->pad_x, sizeof(float) * (size_t)n * dimp);
         if (rc == VQ_OK) {
@@ -576,8 +572,7 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
         hipLaunchKernelGGL(vq::k_gather_means, dim3(cdiv((int64_t)ns * dim, 256)), dim3(256), 0, st,
                            (const float *)d_means, (const int *)d_split, ns, dim, (float *)d_smeans);
         // per-dimension sums of squared deviations (src/tsvq.rs:88-99)
-        const bool var_wg = dim % 4 == 0 && dim <= 1024 && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;
-        if (var_chain && ns <= kChainSegs && !(var_wg && ctx->tsvq_var_path == 0 && longest <= kVarWgRows)) {
+        if (var_chain && ns <= kChainSegs && !(ctx->tsvq_var_path == 0 && longest <= var_tile_rows(dim))) {
             hipLaunchKernelGGL(vq::k_seg_sqdev32, dim3((unsigned)cdiv((int64_t)longest, 64), (unsigned)ns), dim3(256),
                                0, st, perm, (const uint2 *)d_range, (const float *)d_smeans, (int64_t)0, d_x, ld, dim,
                                var_maps ? (float *)nullptr : d_sq, var_maps ? (float *)ctx->tsvq_gsum.p : (float *)nullptr);
@@ -627,22 +622,13 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                 hipLaunchKernelGGL(vq::k_seg_chain32, dim3((unsigned)ns, (unsigned)cdiv(dim, 32)), dim3(256), 0, st,
                                    (const float *)d_sq, (const uint2 *)d_range, dim, (float *)d_var);
             }
-        } else if (var_wg) {
-#define VARIANCE_WG(D)                                                                                     \
-    hipLaunchKernelGGL((vq::k_seg_variance_wg<D>), dim3(ns), dim3(1024), 0, st, perm, (const uint2 *)d_range, \
-                       (const float *)d_smeans, (int64_t)0, d_x, ld, dim, (float *)d_var)
-            switch (dim) {  // the common row lengths get constant LDS strides
-            case 32: VARIANCE_WG(32); break;
-            case 64: VARIANCE_WG(64); break;
-            case 128: VARIANCE_WG(128); break;
-            case 256: VARIANCE_WG(256); break;
-            default: VARIANCE_WG(0); break;
-            }
-#undef VARIANCE_WG
-        } else
-            hipLaunchKernelGGL(vq::k_seg_variance, dim3(cdiv((int64_t)ns * dim, 64)), dim3(64), 0, st, perm,
-                               (const uint2 *)d_range, ns, (const float *)d_smeans, (int64_t)0, d_x, ld, dim,
-                               (float *)d_var);
+        } else {
+            const int tiles = (int)cdiv(dim, 16), width = tiles == 1 ? dim : (int)cdiv(cdiv(dim, tiles), 4) * 4;
+            const int vec = dim >= 4 ? 4 : 1, pieces = (int)cdiv(width, vec);
+            hipLaunchKernelGGL(vec == 4 ? vq::k_seg_variance_tile<4> : vq::k_seg_variance_tile<1>, dim3(ns, cdiv(dim, width)), dim3(256),
+                               sizeof(float) * (size_t)width * (8 * (256 / pieces) + 4), st, perm, (const uint2 *)d_range, (const float *)d_smeans,
+                               (int64_t)0, d_x, ld, dim, width, pieces, (float *)d_var);
+        }
         SP_HIP(hipGetLastError());
         if (split_wg) {  // (a leaf's rows are not moved: nothing reads them again)
             const size_t lds = vq::split_wg_lds(longest);
