@@ -12,7 +12,7 @@ namespace vq {
 // workgroup: P pieces of VEC floats per member; the threads fetch a chunk of members into registers, eight loads of each in
 // flight while the chunk before is added, and store them transposed in LDS (stage: width * (8 NT / P + 4) floats); a lane per
 // component adds them in list order, sixteen members read at a time (with the next sixteen read
-// beside the adds 5-10 % slower).  xs: row 0's tile.  Returned in the lanes
+// beside the adds no faster).  xs: row 0's tile.  Returned in the lanes
 // below width.  The last piece of a tile begins at the tile's end less VEC, so that pieces of any width are whole (what
 // two of them share is written twice, with the same values).  Its time is a chain of memory round trips, one per chunk of 128
 // to 512 members, beside the adds: 7,930 x 300, k = 22 41 -> 17 us per launch, 50,019 x 28 blocks of 10, k = 78 110 -> 28.

@@ -159,8 +159,8 @@ static __global__ void __launch_bounds__(256) k_seg_mean_wg(const float *__restr
 
 // Sums of squared deviations in row order, a workgroup per segment and tile of up to 16 components (grid y; the last
 // one begins at dim less its width): seg_range[g] = {lo, hi} positions in perm; mean of segment g at means[(first + g) * dim].
-// Bound by the chain of adds, 3 ns a row, and the first chunk's memory round trips.  Against one workgroup per segment with all
-// columns, whose one lane per column read its squares one by one: a root of 5,964 x 100 90 -> 25 us.
+// A chunk of 512 rows is a memory round trip, two barriers and their adds, 3.5 us in all: 7 ns a row.  Against one workgroup per segment with all
+// columns, whose one lane per column read its squares one by one: a root of 5,964 x 100 90 -> 41 us.
 template <int VEC>
 static __global__ void __launch_bounds__(256) k_seg_variance_tile(const uint32_t *__restrict__ perm, const uint2 *__restrict__ seg_range,
                                                                  const float *__restrict__ means, int64_t first,

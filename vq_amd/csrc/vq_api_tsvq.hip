@@ -201,7 +201,7 @@ int32_t vq_tsvq_build_kmeans(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
 }
 
 // Levels whose longest node is no longer than this: a workgroup per node and 16 columns (k_seg_variance_tile, one launch,
-// 3-6 ns per row of the longest node) instead of the composed maps (four launches, 45 us and what the columns take).  Builds
+// 7 ns per row of the longest node) instead of the composed maps (four launches, 45 us and what the columns take).  Builds
 // with 4096 / 8192 / 16,384 rows: 100,000 x 16 641 / 661 / 675 us, 40,000 x 96 692 / 690 / 707, 220,611 x 128 1624 / 1567 / 1556,
 // 60,000 x 256 1064 / 1050 / 1065.
 static uint32_t var_tile_rows(int32_t dim) { return dim >= 96 ? 8192 : 4096; }
