@@ -53,3 +53,17 @@ def test_cross_cov(n, dim):
     Y, X = y.astype(np.float64), x.astype(np.float64)
     assert np.all(np.abs(got - Y.T @ X) <= 2 * n * 2.0 ** -53 * (np.abs(Y).T @ np.abs(X)) + 1e-300)
     ctx.close()
+
+
+@pytest.mark.parametrize("n,dim", [(300, 50), (40_000, 50), (300, 180), (70_000, 130), (5, 250)])
+def test_rotate_in_place(n, dim):
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    rng = np.random.default_rng(dim)
+    x, R = rng.standard_normal((n, dim)).astype(F), ctx.to_device(rng.standard_normal((dim, dim)).astype(F))
+    dx, y = ctx.to_device(x), ctx.empty((n, dim), F)
+    ctx.rotate(dx, n, dim, dim, R, y)
+    want = y.download()
+    ctx.rotate(dx, n, dim, dim, R, dx)
+    assert np.array_equal(dx.download().view(np.uint32), want.view(np.uint32))
+    ctx.close()

@@ -496,6 +496,15 @@ int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t 
     VQ_TRY(ensure(ctx, ctx->tmp_f, sizeof(float4) * (size_t)entries));
     float4 *rtab = (float4 *)ctx->tmp_f.p;
     hipLaunchKernelGGL(vq::k_rotate_prep_f32, dim3(cdiv(entries, 256)), dim3(256), 0, ctx->stream, d_R, dim, blocks, entries, rtab);
+    // rows rotated in place: a row's groups are different workgroups, which then read a copy
+    const float *d_end = d_x + (n - 1) * ld + dim;
+    if (groups > 1 && d_y < d_end && d_x < d_y + n * (int64_t)dim) {
+        VQ_TRY(ensure(ctx, ctx->tmp_e, sizeof(float) * (size_t)n * dim));
+        VQ_HIP(ctx, hipMemcpy2DAsync(ctx->tmp_e.p, sizeof(float) * dim, d_x, sizeof(float) * ld, sizeof(float) * dim, (size_t)n,
+                                     hipMemcpyDeviceToDevice, ctx->stream));
+        d_x = (const float *)ctx->tmp_e.p;
+        ld = dim;
+    }
     auto *kern = per == 1 ? vq::k_rotate_mfma_f32<1> : per == 2 ? vq::k_rotate_mfma_f32<2> : per == 3 ? vq::k_rotate_mfma_f32<3> : vq::k_rotate_mfma_f32<4>;
     hipLaunchKernelGGL(kern, dim3(cdiv(n, 128), groups), dim3(256), 0, ctx->stream, d_x, n, ld, dim, blocks, (const float4 *)rtab, d_y);
     VQ_HIP(ctx, hipGetLastError());

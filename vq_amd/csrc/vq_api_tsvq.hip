@@ -131,8 +131,9 @@ int32_t descend_quad_np(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, co
     const unsigned threads = few ? 64 : 512;
     const int32_t ntop = few ? 0 : (int32_t)std::min<size_t>((size_t)most, kBudget / per_node);
     const size_t lds = per_node * (size_t)std::max(ntop, 1);
-    VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_tsvq_descend_quad<METRIC, NP>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (lds > 48 * 1024)
+        VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_tsvq_descend_quad<METRIC, NP>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int cus = 0;
     VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
     const dim3 grid(std::min<unsigned>(cdiv(n, threads / 4), few ? ~0u : (unsigned)std::max(cus, 1) * kPerCu));
