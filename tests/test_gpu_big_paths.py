@@ -47,3 +47,30 @@ def test_fit(n, m, sd, k):
     want = O.pq_fit(x, m, k, 2, init, reseed)["codebooks"]
     assert np.array_equal(cb.download().view(np.uint32), want.view(np.uint32))
     ctx.close()
+
+
+@pytest.mark.parametrize("iters", [1, 3])  # (ends with the last iteration, ends when no code changed)
+@pytest.mark.parametrize("sd", [31, 32])
+def test_fit_is_done_on_return(sd, iters):
+    """The codebooks are in place when the call returns: nothing of it is left on the stream, whether the rows were padded or not."""
+    import ctypes
+    import vq_amd
+    from vq_amd._ffi import lib
+    ctx = vq_amd.Context(0)
+    hip = ctypes.CDLL("libamdhip64.so")
+    n, m, k = 4096, 64, 2048  # 4 MB of codebooks: tens of microseconds for what follows the last update
+    rng = np.random.default_rng(sd)
+    x = rng.random((n, m * sd), dtype=F) if iters == 1 else np.tile(rng.random((k, m * sd), dtype=F), (n // k, 1))
+    init = np.stack([rng.permutation(n)[:k] if iters == 1 else np.arange(k) for _ in range(m)]).astype(np.uint32)
+    reseed = rng.integers(0, n, (m, k * iters)).astype(np.uint32)
+    ran = np.zeros(m, np.int32)
+    dx, cb = ctx.to_device(x), ctx.empty((m, k, sd), F)
+    for _ in range(2):
+        ctx.sync()
+        ctx._check(lib().vq_lbg_fit(ctx._h, dx.ptr, n, m * sd, m, sd, k, iters, init.ctypes.data, reseed.ctypes.data, k * iters, cb.ptr,
+                                    ran.ctypes.data, None))
+        assert hip.hipStreamQuery(ctypes.c_void_p(lib().vq_ctx_stream(ctx._h))) == 0
+        assert ran.max() < 3  # (rows that are their own centroids: the first or second pass changes nothing)
+    want = O.pq_fit(np.ascontiguousarray(x[:, :sd]), 1, k, iters, init[:1], reseed[:1])["codebooks"]
+    assert np.array_equal(cb.download()[:1].view(np.uint32), want.view(np.uint32))
+    ctx.close()

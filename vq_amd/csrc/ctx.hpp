@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -279,12 +280,14 @@ constexpr int64_t kPadSlice = 96 << 20;  // bytes of padded rows that an encode 
 void drop_crew(vq_ctx *ctx);
 
 // Defined in vq_api_bigk.hip: the same for any k up to 65536 with 16-bit codes, and the LBG above
-// 256 centroids (arguments as vq_lbg_fit, already validated).
+// 256 centroids (arguments as vq_lbg_fit, already validated).  last: enqueues what follows the last update; the stream has
+// been waited for when the call returns.
 int32_t assign_codes_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m,
                          int32_t sd, int32_t k, const float *d_codebooks, uint16_t *d_codes,
                          uint16_t *d_out16 = nullptr, bool *out_written = nullptr);
 int32_t lbg_fit_big(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
                     int32_t max_iters, const uint32_t *h_init_idx, const uint32_t *h_reseed_stream,
-                    int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used);
+                    int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used,
+                    const std::function<void()> &last = {});
 
 }  // namespace vqh

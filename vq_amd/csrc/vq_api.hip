@@ -1279,8 +1279,7 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
             float *px = (float *)ctx->pad_rows.p, *pcb = px + (size_t)n * m * w;
             launch_pad(ctx, d_x, n, ld, m, sd, w, px);
             rc = vqh::lbg_fit_big(ctx, px, n, (int64_t)m * w, m, w, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, pcb,
-                                  h_iters_run, h_reseeds_used);
-            if (rc == VQ_OK) unpad_rows(ctx, pcb, (int64_t)m * k, sd, w, d_codebooks);
+                                  h_iters_run, h_reseeds_used, [&] { unpad_rows(ctx, pcb, (int64_t)m * k, sd, w, d_codebooks); });
         }
         if (rc == VQ_ERR_OOM || ctx->pad_rows.cap > kPadKeep) {
             const int32_t gone = release(ctx, ctx->pad_rows);

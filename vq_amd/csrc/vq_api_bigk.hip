@@ -165,7 +165,8 @@ int32_t assign_codes_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t 
 
 int32_t lbg_fit_big(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
                     int32_t max_iters, const uint32_t *h_init_idx, const uint32_t *h_reseed_stream,
-                    int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used) {
+                    int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used,
+                    const std::function<void()> &last) {
     hipStream_t st = ctx->stream;
     const size_t pairs = (size_t)n * m;
     if (pairs >= (1ULL << 32)) return fail(ctx, VQ_ERR_UNSUPPORTED, "n * m must be below 2^32 when k is above 256");
@@ -248,13 +249,21 @@ int32_t lbg_fit_big(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_
         hipLaunchKernelGGL(vq::k_big_large_means, dim3(big_cap, m), dim3(256), 0, st, S, (const uint64_t *)sorted, d_x,
                            n, ld, k, sd, d_codebooks);
         hipLaunchKernelGGL(vq::k_big_advance, dim3(cdiv(m, 64)), dim3(64), 0, st, S, m);
+        if (last && it == max_iters - 1) last();
         VQ_HIP(ctx, hipGetLastError());
         // every column block converged (src/utils.rs:104-106): the remaining passes would change nothing
         VQ_HIP(ctx, hipMemcpyAsync(host.data(), f, sizeof(int) * host.size(), hipMemcpyDeviceToHost, st));
         VQ_HIP(ctx, hipStreamSynchronize(st));
         bool all_done = true;
         for (int s = 0; s < m; ++s) all_done = all_done && host[(size_t)m + s] != 0;
-        if (all_done || host[6 * (size_t)m]) break;
+        if (all_done || host[6 * (size_t)m]) {
+            if (last && it < max_iters - 1) {
+                last();
+                VQ_HIP(ctx, hipGetLastError());
+                VQ_HIP(ctx, hipStreamSynchronize(st));
+            }
+            break;
+        }
     }
     if (max_iters == 0) {
         VQ_HIP(ctx, hipMemcpyAsync(host.data(), f, sizeof(int) * host.size(), hipMemcpyDeviceToHost, st));
