@@ -74,3 +74,29 @@ def test_fit_is_done_on_return(sd, iters):
     want = O.pq_fit(np.ascontiguousarray(x[:, :sd]), 1, k, iters, init[:1], reseed[:1])["codebooks"]
     assert np.array_equal(cb.download()[:1].view(np.uint32), want.view(np.uint32))
     ctx.close()
+
+
+def test_fit_keeps_the_copy_of_other_calls():
+    """A fit whose rows need no copy leaves the one that a padded residual encode has made with the context."""
+    import ctypes
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        ctx.sync()
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+    rng = np.random.default_rng(1)
+    n, dim, k = 50_000, 300, 300
+    dx, dcb = ctx.to_device(rng.random((n, dim), dtype=F)), ctx.to_device(rng.random((2, 64, dim), dtype=F))
+    codes = ctx.empty((n, 2), np.uint8)
+    init, reseed = data.index_streams(4096, 2, k, 1, seed=5)
+    x8, cb8 = ctx.to_device(rng.random((4096, 16), dtype=F)), ctx.empty((2, k, 8), F)
+    ctx.lbg_fit(x8, 4096, 16, 2, 8, k, 1, init, reseed, cb8)
+    ctx.rvq_encode(O.EUCLIDEAN, dx, n, dim, dim, 2, 64, dcb, 0.0, codes)
+    before = free_bytes()
+    ctx.lbg_fit(x8, 4096, 16, 2, 8, k, 1, init, reseed, cb8)
+    assert abs(free_bytes() - before) < 16 << 20
+    ctx.close()

@@ -1274,18 +1274,20 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
         // rows that every pass would pad, once for the fit, as below (200,131 x 36 blocks of 3, k = 280: 62 of 920 us per
         // iteration; 5,851 x 23 of 9, k = 1953: 97 of 400)
         const int w = max_iters > 0 ? encode_pad_width(ctx, VQ_SQEUCLIDEAN, d_x, n, ld, m, sd, vq::kMaxK, d_codebooks) : 0;
-        int32_t rc = VQ_ERR_OOM;
-        if (w && ensure(ctx, ctx->pad_rows, sizeof(float) * ((size_t)n * m + (size_t)m * k) * w) == VQ_OK) {
-            float *px = (float *)ctx->pad_rows.p, *pcb = px + (size_t)n * m * w;
-            launch_pad(ctx, d_x, n, ld, m, sd, w, px);
-            rc = vqh::lbg_fit_big(ctx, px, n, (int64_t)m * w, m, w, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, pcb,
-                                  h_iters_run, h_reseeds_used, [&] { unpad_rows(ctx, pcb, (int64_t)m * k, sd, w, d_codebooks); });
+        if (w) {
+            int32_t rc = ensure(ctx, ctx->pad_rows, sizeof(float) * ((size_t)n * m + (size_t)m * k) * w);
+            if (rc == VQ_OK) {
+                float *px = (float *)ctx->pad_rows.p, *pcb = px + (size_t)n * m * w;
+                launch_pad(ctx, d_x, n, ld, m, sd, w, px);
+                rc = vqh::lbg_fit_big(ctx, px, n, (int64_t)m * w, m, w, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, pcb,
+                                      h_iters_run, h_reseeds_used, [&] { unpad_rows(ctx, pcb, (int64_t)m * k, sd, w, d_codebooks); });
+            }
+            if (rc == VQ_ERR_OOM || ctx->pad_rows.cap > kPadKeep) {
+                const int32_t gone = release(ctx, ctx->pad_rows);
+                if (rc == VQ_OK) rc = gone;
+            }
+            if (rc != VQ_ERR_OOM) return rc;
         }
-        if (rc == VQ_ERR_OOM || ctx->pad_rows.cap > kPadKeep) {
-            const int32_t gone = release(ctx, ctx->pad_rows);
-            if (rc == VQ_OK) rc = gone;
-        }
-        if (rc != VQ_ERR_OOM) return rc;
         return vqh::lbg_fit_big(ctx, d_x, n, ld, m, sd, k, max_iters, h_init_idx, h_reseed_stream, n_reseed,
                                 d_codebooks, h_iters_run, h_reseeds_used);
     }
