@@ -125,3 +125,23 @@ def lbg(X, k, max_iters, init_idx, reseed_stream):
         if not changed:
             break
     return cen, assign, iters, used
+
+
+def fma(a, b, c):
+    """a * b + c with one rounding to float32, element by element: the product is exact in 64 bits, and the sum is rounded to
+    an odd last bit there where it is not exact, so that the second rounding sees on which side it lies."""
+    p, c = np.asarray(a, F).astype(np.float64) * np.asarray(b, F).astype(np.float64), np.asarray(c, F).astype(np.float64)
+    s = p + c
+    back = s - p
+    rest = (p - (s - back)) + (c - back)
+    bits = s.view(np.int64)
+    away = np.where((rest > 0) == (s > 0), 1, -1)
+    return np.where((rest != 0) & (bits & 1 == 0), bits + away, bits).view(np.float64).astype(F)
+
+
+def rotate_chain(x, R):
+    """y[i][a]: one chain of fused multiply-adds over ascending b from +0."""
+    y = np.zeros((len(x), len(R)), F)
+    for b in range(x.shape[1]):
+        y = fma(x[:, b, None], R[None, :, b], y)
+    return y

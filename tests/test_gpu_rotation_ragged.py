@@ -5,6 +5,8 @@ from types import SimpleNamespace
 import numpy as np
 import pytest
 
+from tests import np_ref
+
 pytestmark = pytest.mark.gpu
 F = np.float32
 
@@ -29,11 +31,8 @@ def test_rotate(n, dim, extra, offset):
     X, R64 = x.astype(np.float64), R.astype(np.float64)
     rest = np.arange(n) != n // 2
     want, size = X @ R64.T, np.abs(X) @ np.abs(R64).T
-    chain = np.zeros((n, dim), F)  # fused multiply-adds in ascending order (but for sums that 64 bits of fraction round as well)
-    for t in range(dim):
-        chain = (x[:, t, None].astype(np.longdouble) * R[:, t].astype(np.longdouble) + chain).astype(F)
     if dim % 32 or extra or offset:
-        assert np.sum(got[rest] != chain[rest]) <= n * dim // 1000
+        assert np.array_equal(got[rest].view(np.uint32), np_ref.rotate_chain(x[rest], R).view(np.uint32))
     with np.errstate(invalid="ignore"):
         err = np.abs(got - want)
     assert np.all(err[rest] <= (dim + 1) * 2.0 ** -24 * size[rest])
@@ -66,4 +65,33 @@ def test_rotate_in_place(n, dim):
     want = y.download()
     ctx.rotate(dx, n, dim, dim, R, dx)
     assert np.array_equal(dx.download().view(np.uint32), want.view(np.uint32))
+    ctx.close()
+
+
+@pytest.mark.parametrize("n,dim,extra", [(70, 1, 0), (70, 5, 0), (70, 16, 3), (40, 23, 0), (70, 31, 0), (40, 32, 1), (70, 33, 0), (100, 50, 0), (33, 100, 0), (40, 250, 2)])
+@pytest.mark.parametrize("kind", ["rows", "matrix", "products", "sums", "minus_zero"])
+def test_rotate_below_the_smallest_normal_number(n, dim, extra, kind):
+    """Rows, matrices, products and partial sums without a normal exponent, and sums that come down to -0: the bits of the
+    chain of fused multiply-adds, also behind the last component."""
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    rng = np.random.default_rng(dim)
+    x, R = rng.standard_normal((n, dim + extra)), rng.standard_normal((dim, dim))
+    if kind == "rows":
+        x *= 1e-41
+    elif kind == "matrix":
+        R *= 1e-41
+    elif kind == "products":
+        x, R = x * 1e-20, R * 1e-21
+    elif kind == "sums":
+        x, R = x * np.exp2(rng.integers(-75, -60, x.shape)), R * np.exp2(rng.integers(-75, -60, R.shape))
+    else:  # zeros, then one product below the smallest number
+        x[:, :dim - 1] = 0.0
+        x[:, dim - 1], R[:, dim - 1] = -1e-30, 1e-30
+    x, R = x.astype(F), R.astype(F)
+    y = ctx.empty((n, dim), F)
+    ctx.rotate(ctx.to_device(x), n, dim + extra, dim, ctx.to_device(R), y)
+    want = np_ref.rotate_chain(np.ascontiguousarray(x[:, :dim]), R)
+    assert kind != "minus_zero" or np.all(np.signbit(want) & (want == 0))
+    assert np.array_equal(y.download().view(np.uint32), want.view(np.uint32))
     ctx.close()

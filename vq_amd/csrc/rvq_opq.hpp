@@ -372,8 +372,9 @@ static __global__ void __launch_bounds__(256) k_fill(T *__restrict__ p, int64_t 
 // y[i][a] = sum_b R[a][b] * x[i][b] on the fp32 matrix cores (v_mfma_f32_32x32x2_f32: two fused multiply-adds in
 // ascending order, so the result is one chain over b) for dimensions and alignments that the bf16 kernels below do not
 // take.  A wave owns 32 rows and NB blocks of 32 outputs (grid y).  Step u of kc takes the components 8 kc + 2 u + h, lane
-// 32 h + r those of row r; rtab holds the same of R (zeros beyond dim on both sides), 1 KB per block and kc, read
-// through the vector cache two to eight kc ahead.  Against a thread per (row, four outputs) with its factors from LDS, the
+// 32 h + r those of row r; rtab holds the same of R, 1 KB per block and kc, read
+// through the vector cache two to eight kc ahead.  Beyond dim the rows are +0 and R is -0: a product of -0 leaves every
+// sum as it is, also one that has come down to -0.  Against a thread per (row, four outputs) with its factors from LDS, the
 // same bits: 15,127 x 180 130 -> 24 us, 100,000 x 250 1230 -> 170, 3 x 248 189 -> 12.
 typedef float rot_acc __attribute__((ext_vector_type(16)));
 typedef float rot_piece __attribute__((ext_vector_type(4), aligned(4)));
@@ -399,7 +400,7 @@ static __global__ void __launch_bounds__(256) k_rotate_prep_f32(const float *__r
     const int a = 32 * b + lane % 32, t = 8 * kc + lane / 32;
     float v[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = a < dim && t + 2 * u < dim ? R[(size_t)a * dim + t + 2 * u] : 0.0f;
+    for (int u = 0; u < 4; ++u) v[u] = a < dim && t + 2 * u < dim ? R[(size_t)a * dim + t + 2 * u] : -0.0f;
     rtab[e] = make_float4(v[0], v[1], v[2], v[3]);
 }
 
