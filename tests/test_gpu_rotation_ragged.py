@@ -12,7 +12,7 @@ F = np.float32
 
 
 @pytest.mark.parametrize("n,dim,extra,offset", [
-    (2, 1, 0, 0), (127, 5, 0, 0), (128, 31, 0, 1), (129, 33, 2, 0), (300, 50, 0, 0), (65, 64, 1, 0), (64, 96, 0, 2), (257, 100, 0, 0), (700, 130, 0, 0),
+    (2, 1, 0, 0), (257, 2, 1, 1), (300, 3, 0, 0), (130, 4, 0, 2), (127, 5, 0, 0), (33, 8, 0, 0), (31, 9, 0, 1), (1, 16, 0, 0), (129, 17, 1, 0), (500, 24, 0, 0), (64, 25, 0, 0), (40, 32, 0, 1), (128, 31, 0, 1), (129, 33, 2, 0), (300, 50, 0, 0), (65, 64, 1, 0), (64, 96, 0, 2), (257, 100, 0, 0), (700, 130, 0, 0),
     (1000, 180, 0, 0), (33, 250, 5, 3), (200, 300, 0, 0), (40, 639, 0, 0)])
 def test_rotate(n, dim, extra, offset):
     import vq_amd
@@ -54,7 +54,7 @@ def test_cross_cov(n, dim):
     ctx.close()
 
 
-@pytest.mark.parametrize("n,dim", [(300, 50), (40_000, 50), (300, 180), (70_000, 130), (5, 250)])
+@pytest.mark.parametrize("n,dim", [(700, 3), (40_000, 20), (300, 50), (40_000, 50), (300, 180), (70_000, 130), (5, 250)])
 def test_rotate_in_place(n, dim):
     import vq_amd
     ctx = vq_amd.Context(0)

@@ -379,8 +379,8 @@ static __global__ void __launch_bounds__(256) k_fill(T *__restrict__ p, int64_t 
 typedef float rot_acc __attribute__((ext_vector_type(16)));
 typedef float rot_piece __attribute__((ext_vector_type(4), aligned(4)));
 
-__device__ __forceinline__ rot_piece rot_load(const float *__restrict__ p, int at, int dim) {
-    rot_piece v = {0.0f, 0.0f, 0.0f, 0.0f};
+__device__ __forceinline__ rot_piece rot_load(const float *__restrict__ p, int at, int dim, float behind) {
+    rot_piece v = {behind, behind, behind, behind};
     if (at + 4 <= dim) {
         v = *reinterpret_cast<const rot_piece *>(p + at);
     } else {
@@ -389,6 +389,33 @@ __device__ __forceinline__ rot_piece rot_load(const float *__restrict__ p, int a
         if (at + 2 < dim) v.z = p[at + 2];
     }
     return v;
+}
+
+// Components {0..3} of lanes h = 0 and {4..7} of lanes h = 1 -> 2 u + h: the upper half of the first with the lower half of the
+// second.
+__device__ __forceinline__ void rot_spread(const rot_piece &p, float (&v)[4]) {
+    const auto p02 = __builtin_amdgcn_permlane32_swap(__float_as_uint(p.x), __float_as_uint(p.y), false, false);
+    const auto p13 = __builtin_amdgcn_permlane32_swap(__float_as_uint(p.z), __float_as_uint(p.w), false, false);
+    v[0] = __uint_as_float(p02[0]);
+    v[1] = __uint_as_float(p13[0]);
+    v[2] = __uint_as_float(p02[1]);
+    v[3] = __uint_as_float(p13[1]);
+}
+
+// A block's outputs of a row: register v holds output 8 (v / 4) + 4 h + v % 4 of the block; first: 32 b + 4 h.
+__device__ __forceinline__ void rot_store(const rot_acc &acc, float *__restrict__ yr, int first, int dim) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const int at = first + 8 * g;
+        const rot_piece v = {acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+        if (at + 4 <= dim) {
+            *reinterpret_cast<rot_piece *>(yr + at) = v;
+        } else {
+            if (at < dim) yr[at] = v.x;
+            if (at + 1 < dim) yr[at + 1] = v.y;
+            if (at + 2 < dim) yr[at + 2] = v.z;
+        }
+    }
 }
 
 // rtab[kc][b][lane][u] = R[32 b + lane % 32][8 kc + 2 u + lane / 32], blocks = ceil(dim / 32)
@@ -423,7 +450,7 @@ static __global__ void __launch_bounds__(256) k_rotate_mfma_f32(const float *__r
     rot_piece xn[kAhead];
     float4 rn[kAhead][NB];
     auto fetch = [&](int kc, rot_piece &xv, float4(&rv)[NB]) {
-        xv = rot_load(xr, 8 * kc + 4 * h, dim);  // zeros past the end
+        xv = rot_load(xr, 8 * kc + 4 * h, dim, 0.0f);
         const float4 *from = rt + (size_t)(kc < nkc ? kc : nkc - 1) * blocks * 64;
 #pragma unroll
         for (int b = 0; b < NB; ++b) rv[b] = from[b * 64];
@@ -433,11 +460,8 @@ static __global__ void __launch_bounds__(256) k_rotate_mfma_f32(const float *__r
     for (int kc0 = 0; kc0 < nkc; kc0 += kAhead) {
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) {
-            // components {0..3} of lanes h = 0 and {4..7} of lanes h = 1 -> 2 u + h: the upper half of the first with the
-            // lower half of the second
-            const auto p02 = __builtin_amdgcn_permlane32_swap(__float_as_uint(xn[i].x), __float_as_uint(xn[i].y), false, false);
-            const auto p13 = __builtin_amdgcn_permlane32_swap(__float_as_uint(xn[i].z), __float_as_uint(xn[i].w), false, false);
-            const float xv[4] = {__uint_as_float(p02[0]), __uint_as_float(p13[0]), __uint_as_float(p02[1]), __uint_as_float(p13[1])};
+            float xv[4];
+            rot_spread(xn[i], xv);
             float4 rv[NB];
 #pragma unroll
             for (int b = 0; b < NB; ++b) rv[b] = rn[i][b];
@@ -452,23 +476,58 @@ static __global__ void __launch_bounds__(256) k_rotate_mfma_f32(const float *__r
                 }
         }
     }
-    // register v of a block holds output 32 b + 8 (v / 4) + 4 h + v % 4 of this lane's row
     if (row >= n) return;
-    float *__restrict__ yr = y + row * dim;
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+    for (int b = 0; b < NB; ++b) rot_store(acc[b], y + row * dim, 32 * (b0 + b) + 4 * h, dim);
+}
+
+// The same for up to 32 dimensions, 8 NK of them at most, in one launch: the matrix is 4 KB, its pieces are read as the rows' are.
+// (A table costs a launch of its own, and the loads that are ahead for a long chain: 60 x 8 6.0 -> 3.6 us, 400,000 x 2
+// 18.7 -> 5.9, x 32 38 -> 24; a thread per (row, output) with its factors from LDS took 3.6, 4.4 and 85.)
+template <int NK>
+static __global__ void __launch_bounds__(256) k_rotate_mfma_small(const float *__restrict__ x, int64_t n, int64_t ld, int dim,
+                                                                  const float *__restrict__ R, float *__restrict__ y) {
+    const int lane = threadIdx.x & 63, h = lane >> 5, r = lane & 31;
+    const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 32 + r;
+    const float *__restrict__ xr = x + (row < n ? row : n - 1) * ld;  // past the end: the last row, not stored
+    const float *__restrict__ Rr = R + (size_t)(r < dim ? r : dim - 1) * dim;
+    rot_piece xp[NK], rp[NK];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int at = 32 * (b0 + b) + 8 * g + 4 * h;
-            const rot_piece v = {acc[b][4 * g], acc[b][4 * g + 1], acc[b][4 * g + 2], acc[b][4 * g + 3]};
-            if (at + 4 <= dim) {
-                *reinterpret_cast<rot_piece *>(yr + at) = v;
-            } else {
-                if (at < dim) yr[at] = v.x;
-                if (at + 1 < dim) yr[at + 1] = v.y;
-                if (at + 2 < dim) yr[at + 2] = v.z;
-            }
-        }
+    for (int kc = 0; kc < NK; ++kc) {
+        xp[kc] = rot_load(xr, 8 * kc + 4 * h, dim, 0.0f);
+        rp[kc] = rot_load(Rr, 8 * kc + 4 * h, dim, -0.0f);
+    }
+    rot_acc acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+#pragma unroll
+    for (int kc = 0; kc < NK; ++kc) {
+        float xv[4], rv[4];
+        rot_spread(xp[kc], xv);
+        rot_spread(rp[kc], rv);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(rv[u], xv[u], acc, 0, 0, 0);
+    }
+    if (row < n) rot_store(acc, y + row * dim, 4 * h, dim);
+}
+
+// Up to three dimensions: a row per lane (1M x 1 8.8 -> 3.4 us, x 3 11.4 -> 3.9 against the tiles above).
+template <int D>
+static __global__ void __launch_bounds__(256) k_rotate_narrow(const float *__restrict__ x, int64_t n, int64_t ld, const float *__restrict__ R,
+                                                              float *__restrict__ y) {
+    const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (row >= n) return;
+    float v[D], out[D];
+#pragma unroll
+    for (int b = 0; b < D; ++b) v[b] = x[row * ld + b];
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        out[a] = 0.0f;
+#pragma unroll
+        for (int b = 0; b < D; ++b) out[a] = __builtin_fmaf(R[a * D + b], v[b], out[a]);
+    }
+#pragma unroll
+    for (int a = 0; a < D; ++a) y[row * D + a] = out[a];
 }
 
 // ---- cross-covariance ----------------------------------------------------------------------

@@ -485,6 +485,19 @@ int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t 
         return VQ_OK;
     }
     if (dim > 639) return fail(ctx, VQ_ERR_UNSUPPORTED, "rotation: dim %d too large", dim);
+    if (dim <= 3) {
+        auto *kern = dim == 1 ? vq::k_rotate_narrow<1> : dim == 2 ? vq::k_rotate_narrow<2> : vq::k_rotate_narrow<3>;
+        hipLaunchKernelGGL(kern, dim3(cdiv(n, 256)), dim3(256), 0, ctx->stream, d_x, n, ld, d_R, d_y);
+        VQ_HIP(ctx, hipGetLastError());
+        return VQ_OK;
+    }
+    if (dim <= 32) {
+        const int nk = (int)cdiv(dim, 8);
+        auto *kern = nk == 1 ? vq::k_rotate_mfma_small<1> : nk == 2 ? vq::k_rotate_mfma_small<2> : nk == 3 ? vq::k_rotate_mfma_small<3> : vq::k_rotate_mfma_small<4>;
+        hipLaunchKernelGGL(kern, dim3(cdiv(n, 128)), dim3(256), 0, ctx->stream, d_x, n, ld, dim, d_R, d_y);
+        VQ_HIP(ctx, hipGetLastError());
+        return VQ_OK;
+    }
     // up to four blocks of 32 outputs per wave, the same number in every wave (the last ones overlap), fewer where that
     // leaves compute units without rows
     const int blocks = (int)cdiv(dim, 32);
