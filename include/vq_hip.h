@@ -320,7 +320,8 @@ int32_t vq_rvq_encode_u16(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t
 /* ---- optimized product quantizer (src/opq.rs) ---------------------------------------------- */
 
 /* d_y[i] = R * d_x[i] for every row, R row-major dim x dim (src/opq.rs:186-194, 232-234).
- * d_y is n x dim, compact.  f32 fused multiply-add accumulation (the reference's nalgebra
+ * d_y is n x dim, compact; it may overlap the rows (they are read from a copy then, except where they are compact
+ * and d_y == d_x and a wave makes all outputs of a row).  f32 fused multiply-add accumulation (the reference's nalgebra
  * rounding is implementation-defined).  Asynchronous. */
 int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t dim, const float *d_R,
                   float *d_y);

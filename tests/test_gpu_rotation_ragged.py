@@ -95,3 +95,25 @@ def test_rotate_below_the_smallest_normal_number(n, dim, extra, kind):
     assert kind != "minus_zero" or np.all(np.signbit(want) & (want == 0))
     assert np.array_equal(y.download().view(np.uint32), want.view(np.uint32))
     ctx.close()
+
+
+@pytest.mark.parametrize("dim,extra", [(2, 1), (20, 3), (50, 2), (64, 1), (64, 4), (160, 32), (180, 1)])
+@pytest.mark.parametrize("shift", [0, 4, -52])  # of the output against the rows, in floats (multiples of 16 bytes)
+def test_rotate_over_the_rows(dim, extra, shift):
+    """An output that lies over rows of other waves, spaced or shifted: as into a buffer of its own."""
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    n, ld = 100_000, dim + (extra if shift >= 0 else 0)
+    rng = np.random.default_rng(dim)
+    front = max(0, -shift)
+    buf = rng.standard_normal(front + n * ld + max(0, shift)).astype(F)
+    dx, R, y = ctx.to_device(buf), ctx.to_device(rng.standard_normal((dim, dim)).astype(F)), ctx.empty((n, dim), F)
+    rows = SimpleNamespace(ptr=dx.ptr + 4 * front)
+    ctx.rotate(rows, n, ld, dim, R, y)
+    want = y.download().view(np.uint32).ravel()
+    for _ in range(6):
+        dx.upload(buf)
+        ctx.rotate(rows, n, ld, dim, R, SimpleNamespace(ptr=rows.ptr + 4 * shift))
+        got = dx.download()[front + shift:front + shift + n * dim]
+        assert np.array_equal(got.view(np.uint32), want)
+    ctx.close()

@@ -438,15 +438,18 @@ int32_t vq_mean_l2norm(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int
     return VQ_OK;
 }
 
-int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t dim, const float *d_R,
-                  float *d_y) {
-    if (!ctx) return VQ_ERR_INVALID_ARG;
-    if (n == 0) return VQ_OK;
-    if (!d_x || !d_R || !d_y || n < 0 || dim <= 0 || ld < dim) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
-    VQ_HIP(ctx, hipSetDevice(ctx->device));
-    // bf16 matrix cores: dim a multiple of 32 up to 256, rows and output 16-byte aligned
-    if (dim % 32 == 0 && dim <= 256 && ld % 4 == 0 &&
-        ((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_y)) & 15) == 0) {
+// Up to four blocks of 32 outputs per wave of k_rotate_mfma_f32, the same number in every wave (the last ones overlap), fewer
+// where that leaves compute units without rows.
+static int rotate_blocks_per_wave(int64_t n, int32_t dim) {
+    const int blocks = (int)cdiv(dim, 32);
+    int per = 4;
+    while (per > 1 && (int64_t)cdiv(n, 128) * cdiv(blocks, per) < 256) per /= 2;
+    return (int)cdiv(blocks, cdiv(blocks, per));
+}
+
+// The rotation by the kernels that bf16 and the dimension ask for.
+static int32_t rotate_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t dim, const float *d_R, float *d_y, bool bf16) {
+    if (bf16) {
         // operand table: 32 bytes per (output dimension, 4 input dimensions)
         VQ_TRY(ensure(ctx, ctx->tmp_f, 8 * (size_t)dim * dim));
         vq::rot_u32x4 *rtab = (vq::rot_u32x4 *)ctx->tmp_f.p;
@@ -484,7 +487,6 @@ int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t 
         VQ_HIP(ctx, hipGetLastError());
         return VQ_OK;
     }
-    if (dim > 639) return fail(ctx, VQ_ERR_UNSUPPORTED, "rotation: dim %d too large", dim);
     if (dim <= 3) {
         auto *kern = dim == 1 ? vq::k_rotate_narrow<1> : dim == 2 ? vq::k_rotate_narrow<2> : vq::k_rotate_narrow<3>;
         hipLaunchKernelGGL(kern, dim3(cdiv(n, 256)), dim3(256), 0, ctx->stream, d_x, n, ld, d_R, d_y);
@@ -498,30 +500,40 @@ int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t 
         VQ_HIP(ctx, hipGetLastError());
         return VQ_OK;
     }
-    // up to four blocks of 32 outputs per wave, the same number in every wave (the last ones overlap), fewer where that
-    // leaves compute units without rows
-    const int blocks = (int)cdiv(dim, 32);
-    int per = 4;
-    while (per > 1 && (int64_t)cdiv(n, 128) * cdiv(blocks, per) < 256) per /= 2;
-    per = (int)cdiv(blocks, cdiv(blocks, per));
+    const int blocks = (int)cdiv(dim, 32), per = rotate_blocks_per_wave(n, dim);
     const unsigned groups = cdiv(blocks, per);
     const int entries = (int)cdiv(dim, 8) * blocks * 64;
     VQ_TRY(ensure(ctx, ctx->tmp_f, sizeof(float4) * (size_t)entries));
     float4 *rtab = (float4 *)ctx->tmp_f.p;
     hipLaunchKernelGGL(vq::k_rotate_prep_f32, dim3(cdiv(entries, 256)), dim3(256), 0, ctx->stream, d_R, dim, blocks, entries, rtab);
-    // rows rotated in place: a row's groups are different workgroups, which then read a copy
-    const float *d_end = d_x + (n - 1) * ld + dim;
-    if (groups > 1 && d_y < d_end && d_x < d_y + n * (int64_t)dim) {
+    auto *kern = per == 1 ? vq::k_rotate_mfma_f32<1> : per == 2 ? vq::k_rotate_mfma_f32<2> : per == 3 ? vq::k_rotate_mfma_f32<3> : vq::k_rotate_mfma_f32<4>;
+    hipLaunchKernelGGL(kern, dim3(cdiv(n, 128), groups), dim3(256), 0, ctx->stream, d_x, n, ld, dim, blocks, (const float4 *)rtab, d_y);
+    VQ_HIP(ctx, hipGetLastError());
+    return VQ_OK;
+}
+
+int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t dim, const float *d_R,
+                  float *d_y) {
+    if (!ctx) return VQ_ERR_INVALID_ARG;
+    if (n == 0) return VQ_OK;
+    if (!d_x || !d_R || !d_y || n < 0 || dim <= 0 || ld < dim) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter");
+    VQ_HIP(ctx, hipSetDevice(ctx->device));
+    // bf16 matrix cores: dim a multiple of 32 up to 256, rows and output 16-byte aligned
+    const bool bf16 = dim % 32 == 0 && dim <= 256 && ld % 4 == 0 &&
+                      ((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_y)) & 15) == 0;
+    if (!bf16 && dim > 639) return fail(ctx, VQ_ERR_UNSUPPORTED, "rotation: dim %d too large", dim);
+    // An output over the rows: a wave reads all of its rows before it writes, so compact rows may be replaced by their own
+    // results where one wave makes all outputs of a row; else an output lies over rows that other waves still read.
+    const bool overlap = d_y < d_x + (n - 1) * ld + dim && d_x < d_y + n * (int64_t)dim;
+    const bool own = d_x == d_y && ld == dim && (bf16 || rotate_blocks_per_wave(n, dim) * 32 >= dim);
+    if (overlap && !own) {
         VQ_TRY(ensure(ctx, ctx->tmp_e, sizeof(float) * (size_t)n * dim));
         VQ_HIP(ctx, hipMemcpy2DAsync(ctx->tmp_e.p, sizeof(float) * dim, d_x, sizeof(float) * ld, sizeof(float) * dim, (size_t)n,
                                      hipMemcpyDeviceToDevice, ctx->stream));
         d_x = (const float *)ctx->tmp_e.p;
         ld = dim;
     }
-    auto *kern = per == 1 ? vq::k_rotate_mfma_f32<1> : per == 2 ? vq::k_rotate_mfma_f32<2> : per == 3 ? vq::k_rotate_mfma_f32<3> : vq::k_rotate_mfma_f32<4>;
-    hipLaunchKernelGGL(kern, dim3(cdiv(n, 128), groups), dim3(256), 0, ctx->stream, d_x, n, ld, dim, blocks, (const float4 *)rtab, d_y);
-    VQ_HIP(ctx, hipGetLastError());
-    return VQ_OK;
+    return rotate_rows(ctx, d_x, n, ld, dim, d_R, d_y, bf16);
 }
 
 int32_t vq_cross_cov(vq_ctx *ctx, const float *d_y, const float *d_x, int64_t n, int32_t dim, double *h_A) {
