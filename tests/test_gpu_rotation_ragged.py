@@ -117,3 +117,35 @@ def test_rotate_over_the_rows(dim, extra, shift):
         got = dx.download()[front + shift:front + shift + n * dim]
         assert np.array_equal(got.view(np.uint32), want)
     ctx.close()
+
+
+def test_rotate_over_many_rows():
+    """More rows than one copy takes: the same rows, in slices where the output begins no later than they do, whole where it begins
+    later (the one that exceeds the bound is given back)."""
+    import ctypes
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        ctx.sync()
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+    n, dim, slack = 1_300_000, 500, 1000  # 2.6 GB
+    x = np.random.default_rng(1).standard_normal((1300, dim)).astype(F)
+    R = ctx.to_device(np.random.default_rng(2).standard_normal((dim, dim)).astype(F))
+    y, dx = ctx.empty((1300, dim), F), ctx.empty(n * dim + slack, F)
+    ctx.rotate(ctx.to_device(x), 1300, dim, dim, R, y)
+    want = y.download().view(np.uint32)
+    rows = np.tile(x, (n // 1300, 1)).ravel()
+    for at, to in ((0, 0), (slack, 0), (0, slack)):
+        host = np.zeros(n * dim + slack, F)
+        host[at:at + n * dim] = rows
+        dx.upload(host)
+        before = free_bytes()
+        ctx.rotate(SimpleNamespace(ptr=dx.ptr + 4 * at), n, dim, dim, R, SimpleNamespace(ptr=dx.ptr + 4 * to))
+        assert before - free_bytes() < 128 << 20
+        got = dx.download()[to:to + n * dim].view(np.uint32).reshape(-1, *want.shape)
+        assert np.array_equal(got, np.broadcast_to(want, got.shape))
+    ctx.close()

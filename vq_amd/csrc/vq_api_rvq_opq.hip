@@ -526,14 +526,23 @@ int32_t vq_rotate(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t 
     // results where one wave makes all outputs of a row; else an output lies over rows that other waves still read.
     const bool overlap = d_y < d_x + (n - 1) * ld + dim && d_x < d_y + n * (int64_t)dim;
     const bool own = d_x == d_y && ld == dim && (bf16 || rotate_blocks_per_wave(n, dim) * 32 >= dim);
-    if (overlap && !own) {
-        VQ_TRY(ensure(ctx, ctx->tmp_e, sizeof(float) * (size_t)n * dim));
-        VQ_HIP(ctx, hipMemcpy2DAsync(ctx->tmp_e.p, sizeof(float) * dim, d_x, sizeof(float) * ld, sizeof(float) * dim, (size_t)n,
-                                     hipMemcpyDeviceToDevice, ctx->stream));
-        d_x = (const float *)ctx->tmp_e.p;
-        ld = dim;
+    if (!overlap || own) return rotate_rows(ctx, d_x, n, ld, dim, d_R, d_y, bf16);
+    // An output that begins no later than the rows reaches none behind the ones it is made of: a slice is copied at a time
+    // (64 MB).  Else all rows are, and a large copy is given back.
+    const int64_t slice = d_y <= d_x ? std::min<int64_t>(n, (64 << 20) / (int64_t)sizeof(float) / dim) : n;
+    VQ_TRY(ensure(ctx, ctx->tmp_e, sizeof(float) * (size_t)slice * dim));
+    int32_t rc = VQ_OK;
+    for (int64_t r0 = 0; r0 < n && rc == VQ_OK; r0 += slice) {
+        const int64_t rows = std::min(slice, n - r0);
+        VQ_HIP(ctx, hipMemcpy2DAsync(ctx->tmp_e.p, sizeof(float) * dim, d_x + r0 * ld, sizeof(float) * ld, sizeof(float) * dim,
+                                     (size_t)rows, hipMemcpyDeviceToDevice, ctx->stream));
+        rc = rotate_rows(ctx, (const float *)ctx->tmp_e.p, rows, dim, dim, d_R, d_y + r0 * dim, bf16);
     }
-    return rotate_rows(ctx, d_x, n, ld, dim, d_R, d_y, bf16);
+    if (ctx->tmp_e.cap > kPadKeep) {
+        const int32_t gone = release(ctx, ctx->tmp_e);
+        if (rc == VQ_OK) rc = gone;
+    }
+    return rc;
 }
 
 int32_t vq_cross_cov(vq_ctx *ctx, const float *d_y, const float *d_x, int64_t n, int32_t dim, double *h_A) {
