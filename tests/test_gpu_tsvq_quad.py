@@ -27,7 +27,10 @@ def ctx():
     (1, 1, 0, 0, 3), (15, 3, 0, 0, 4), (17, 5, 2, 1, 4), (129, 15, 0, 0, 5), (700, 16, 1, 3, 6), (700, 17, 0, 0, 6),
     (700, 31, 0, 2, 9), (3000, 50, 0, 0, 10), (700, 64, 0, 0, 10), (700, 100, 0, 0, 8), (700, 112, 3, 0, 5),
     (5000, 128, 0, 0, 9), (700, 129, 0, 0, 5), (700, 161, 0, 0, 7), (700, 208, 0, 0, 6), (2500, 248, 0, 0, 11),
-    (700, 256, 4, 0, 8), (700, 257, 0, 0, 4), (70_000, 9, 0, 0, 12)])
+    (700, 256, 4, 0, 8), (700, 257, 0, 0, 4), (70_000, 9, 0, 0, 12),
+    # a lane per row, and the first that are not
+    (700, 1, 1, 0, 10), (70_000, 2, 0, 1, 6), (700, 3, 2, 0, 8), (700, 3, 0, 1, 9), (700, 4, 0, 0, 3), (700, 4, 1, 1, 4), (3000, 7, 0, 0, 2), (600, 15, 0, 0, 1),
+    (600, 16, 0, 0, 1), (100_001, 5, 0, 0, 4), (600, 32, 0, 0, 0)])
 def test_widths_and_depths(ctx, metric, n, dim, extra, offset, depth):
     rng = np.random.default_rng(n + dim)
     nn = 2 ** (depth + 1) - 1

@@ -72,6 +72,7 @@ struct vq_ctx {
     bool lbg_small_lds_set = false;  // dynamic-LDS limit granted to k_lbg_update_small
     int compute_units = 0;       // of the context's GPU (0: not asked for yet)
     int decode_lds_set[4] = {0, 0, 0, 0};  // dynamic-LDS limit already granted to the four resident decode kernels
+    uint64_t quad_lds_set = 0;   // dynamic-LDS limit granted to k_tsvq_descend_quad, a bit per instance
     int tsvq_descend_path = 0;   // 0 = one inner product per node where it decides (cosine, L2), 1 = two distances per node always
     int procrustes_path = 0;     // 0 = Newton-Schulz polar factor first, SVD when it does not converge; 1 = SVD only
     // vq_assign_noalloc: the device address of this GPU's file-scope scratch array, and whether a
@@ -168,6 +169,16 @@ inline int32_t ensure_pinned(vq_ctx *ctx, void *&p, size_t &cap, size_t bytes) {
     const size_t want = bytes + bytes / 8 + 4096;
     VQ_HIP(ctx, hipHostMalloc(&p, want, hipHostMallocDefault));
     cap = want;
+    return VQ_OK;
+}
+
+// Sets ctx->compute_units.  (The runtime's query is 0.3 us, a tenth of a small call.)
+inline int32_t know_compute_units(vq_ctx *ctx) {
+    if (ctx->compute_units == 0) {
+        int cus = 0;
+        VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+        ctx->compute_units = cus > 0 ? cus : 1;
+    }
     return VQ_OK;
 }
 

@@ -690,18 +690,14 @@ int32_t launch_decode_resident(vq_ctx *ctx, const CodeT *d_codes, int64_t n, int
     const size_t lds = (size_t)k * sd * (F16 ? 2 : 4) * G;
     if ((reinterpret_cast<uintptr_t>(d_codebooks) & 15) || (reinterpret_cast<uintptr_t>(d_out) & 63)) return VQ_OK;
     auto kern = k_decode_resident<F16, CodeT>;
-    // the kernel's LDS limit and the number of compute units: asked for once per context and kernel
+    // the kernel's LDS limit: asked for once per context and kernel
     const int slot = (F16 ? 2 : 0) + (sizeof(CodeT) == 2 ? 1 : 0);
     if ((size_t)ctx->decode_lds_set[slot] < lds) {
         VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));
         ctx->decode_lds_set[slot] = 128 * 1024;
     }
-    if (ctx->compute_units == 0) {
-        int cus = 0;
-        VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-        ctx->compute_units = cus > 0 ? cus : 1;
-    }
+    VQ_TRY(know_compute_units(ctx));
     const int64_t pieces = (int64_t)n * m * (F16 ? sd / 8 : sd / 4);
     const unsigned per_cu = lds <= 64 * 1024 ? 2u : 1u;
     const unsigned groups = cdiv(m, G);

@@ -114,6 +114,16 @@ bool quad_applicable(const vq_ctx *ctx, const vq_tree *tree) {
     return ctx->tsvq_descend_path == 0 && tree->dim <= kQuadDims;
 }
 
+// Narrow rows on few levels go to the kernel with a lane per row (k_tsvq_descend): a node is a load or two then, and four lanes
+// hold a row of one piece.  Times of the four lanes over the lane's, 600 to 1M rows: 1 component 1.1 to 4 at any depth, 3
+// components 1.1-2.9 (one level), 1.04-1.4 (six), 0.8-1.06 (ten), 5 components 1.06-1.5 (two levels), 1.0-1.2 (three), 0.9-1.0 (four;
+// 1.06-1.13 from 131,000 rows on), 8 components 0.9-1.1 (one level), 0.6-0.9 (two), 16 components 0.5-1 (one level).
+bool lane_per_row(const vq_tree *tree, int64_t n) {
+    int levels = 0;  // of a complete tree with as many inner nodes
+    while (tree->n_inner >> levels) ++levels;
+    return tree->dim <= 2 || (tree->dim == 3 && levels <= 8) || tree->dim * levels <= (n > 100'000 && tree->dim <= 6 ? 20 : 15);
+}
+
 template <int METRIC, int NP>
 int32_t descend_quad_np(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, const vq_tree *tree, int32_t *d_leaf,
                         uint16_t *d_out) {
@@ -131,12 +141,15 @@ int32_t descend_quad_np(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, co
     const unsigned threads = few ? 64 : 512;
     const int32_t ntop = few ? 0 : (int32_t)std::min<size_t>((size_t)most, kBudget / per_node);
     const size_t lds = per_node * (size_t)std::max(ntop, 1);
-    if (lds > 48 * 1024)
+    static_assert(NP <= 16 && METRIC >= 0 && METRIC < 4, "a bit per instance");
+    constexpr uint64_t instance = 1ull << (METRIC * 16 + NP - 1);
+    if (lds > 48 * 1024 && !(ctx->quad_lds_set & instance)) {
         VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_tsvq_descend_quad<METRIC, NP>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    int cus = 0;
-    VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-    const dim3 grid(std::min<unsigned>(cdiv(n, threads / 4), few ? ~0u : (unsigned)std::max(cus, 1) * kPerCu));
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBudget));
+        ctx->quad_lds_set |= instance;
+    }
+    VQ_TRY(know_compute_units(ctx));
+    const dim3 grid(std::min<unsigned>(cdiv(n, threads / 4), few ? ~0u : (unsigned)ctx->compute_units * kPerCu));
     hipLaunchKernelGGL((vq::k_tsvq_descend_quad<METRIC, NP>), grid, dim3(threads), lds, ctx->stream, d_x, n, ld, tree->dim, tree->d_centroids,
                        tree->d_cnorm, tree->d_left, tree->d_right, l1 ? tree->d_centroids : cosine ? tree->d_wcos : tree->d_wl2,
                        cosine ? tree->d_sccos : tree->d_scl2, ntop, std::min(tree->n_nodes, (int32_t)vq::kTopNodes), d_leaf, d_out);
@@ -844,18 +857,18 @@ int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n
     // cosine and (squared) Euclidean: a step decided by one inner product with the node's vector,
     // the two sums of the reference only where that cannot decide
     const bool inner = ctx->tsvq_descend_path == 0 && metric >= VQ_SQEUCLIDEAN && metric <= VQ_COSINE;
-    int cus = 0;
-    VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    VQ_TRY(know_compute_units(ctx));
     // The kernels with a row per lane read half the LDS bytes per row where every inner node is in LDS (255) and
     // half of their workgroups of 512 rows, one per compute unit, have rows: 131,072 x 128, eight levels 30.6 us
     // against 38.7, 480,000 x 32, eight levels 28 against 32; but 66,000 x 128 27.9 against 27.4, 20,000 23.5 against
     // 15.7, and ten levels 500,000 x 128 179 against 137.
-    if (quad_applicable(ctx, tree) && !(regs && tree->n_inner <= vq::kTopNodes && n > (int64_t)cus * 256))
+    const bool narrow = quad_applicable(ctx, tree) && lane_per_row(tree, n);
+    if (!narrow && quad_applicable(ctx, tree) && !(regs && tree->n_inner <= vq::kTopNodes && n > (int64_t)ctx->compute_units * 256))
         return descend_quad(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
-    if (few_applicable(ctx, n, tree->dim)) return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
-    if (regs) {
+    if (!narrow && few_applicable(ctx, n, tree->dim)) return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
+    if (regs && !narrow) {
         // one workgroup per compute unit (the staged centroids fill its LDS), walking over the rows
-        dim3 g(std::min<unsigned>(cdiv(n, 512), (unsigned)std::max(cus, 1))), b(512);
+        dim3 g(std::min<unsigned>(cdiv(n, 512), (unsigned)ctx->compute_units)), b(512);
         if (inner) {
             const bool cosine = metric == VQ_COSINE;
             const float *wt = cosine ? tree->d_wcos : tree->d_wl2, *sc = cosine ? tree->d_sccos : tree->d_scl2;
