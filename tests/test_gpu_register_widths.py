@@ -70,3 +70,17 @@ def test_encode_in_slices(ctx):
     ctx.assign(vq_amd.EUCLIDEAN, ctx.to_device(x), n, m * sd, m, sd, k, ctx.to_device(cb), codes)
     at = np.concatenate([np.arange(500), rng.integers(0, n, 3000), np.arange(n - 500, n), 520_000 + np.arange(10_000)])
     assert np.array_equal(codes.download()[at], O.pq_encode(O.EUCLIDEAN, x[at], cb).astype(np.uint8))
+
+
+@pytest.mark.parametrize("n,m,sd,k", [(65_281, 4, 3, 6), (65_280, 4, 5, 9), (65_281, 8, 7, 17), (65_281, 2, 12, 9), (65_300, 2, 15, 5), (65_281, 4, 4, 2), (44_000, 6, 10, 3)])
+def test_encode_with_several_blocks_per_lane(ctx, n, m, sd, k):
+    """Two or four blocks per lane: only where that leaves a workgroup per compute unit (65,281 rows x 4 by fours)."""
+    import vq_amd
+    rng = np.random.default_rng(n + sd)
+    x, cb = np.round(rng.standard_normal((n, m * sd)) * 3).astype(F), np.round(rng.standard_normal((m, k, sd)) * 3).astype(F)
+    x[n // 3, 1] = np.inf
+    dx, dcb = ctx.to_device(x), ctx.to_device(cb)
+    for metric, om in ((vq_amd.SQEUCLIDEAN, O.SQEUCLIDEAN), (vq_amd.EUCLIDEAN, O.EUCLIDEAN), (vq_amd.COSINE, O.COSINE), (vq_amd.MANHATTAN, O.MANHATTAN)):
+        codes = ctx.to_device(np.full((n, m), 255, np.uint8))
+        ctx.assign(metric, dx, n, m * sd, m, sd, k, dcb, codes)
+        assert np.array_equal(codes.download(), O.pq_encode(om, x, cb).astype(np.uint8)), metric

@@ -97,14 +97,16 @@ int32_t launch_static(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
 
 template <int SD, int METRIC, bool LBG, bool PAD = false>
 int32_t launch_static_g(vq_ctx *ctx, const vq::AssignArgs &a, int sd = SD) {
-    // G column blocks per lane: as many as keep the lane's floats within 32 registers and the
-    // codebooks within 64 KB of LDS.
+    // G column blocks per lane: as many as keep the lane's floats within 32 registers and the codebooks within 64 KB of LDS,
+    // where that leaves a workgroup per compute unit: a lane takes its blocks one after the
+    // other (6000 x 16 blocks of four, k = 256, Manhattan 44 -> 12.5 us, x 4 of seven, k = 33 13.5 -> 5; but 20,000 x 16 of five, k = 4 9 -> 4.6).
     size_t per = (size_t)a.k * SD * sizeof(float) + (METRIC == vq::M_COS ? a.k * sizeof(float) : 0);
+    auto fills = [&](int G) { return (a.n + 255) / 256 * (a.m / G) >= 256; };
     if constexpr (SD * 4 <= 32) {
-        if (a.m % 4 == 0 && 4 * per <= 64 * 1024) return launch_static<SD, 4, METRIC, LBG, PAD>(ctx, a, sd);
+        if (a.m % 4 == 0 && 4 * per <= 64 * 1024 && fills(4)) return launch_static<SD, 4, METRIC, LBG, PAD>(ctx, a, sd);
     }
     if constexpr (SD * 2 <= 32) {
-        if (a.m % 2 == 0 && 2 * per <= 64 * 1024) return launch_static<SD, 2, METRIC, LBG, PAD>(ctx, a, sd);
+        if (a.m % 2 == 0 && 2 * per <= 64 * 1024 && fills(2)) return launch_static<SD, 2, METRIC, LBG, PAD>(ctx, a, sd);
     }
     return launch_static<SD, 1, METRIC, LBG, PAD>(ctx, a, sd);
 }
