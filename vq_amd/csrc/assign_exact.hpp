@@ -200,7 +200,8 @@ __device__ __forceinline__ int argmin_lds(const float (&x)[SD], const float *lds
 // codebooks in LDS).  blockIdx.x = tile * (m/G) + block group.
 // PAD: blocks of sub_dim < SD floats, zeros behind them in the registers and in LDS.  A component that is zero on both
 // sides adds +0 to a sum that started at +0, so every distance keeps its bits.
-template <int SD, int G, int METRIC, bool LBG, bool PAD>
+// DIST: the chosen centroids' distances, too, where the caller asks for them (as a run-time choice it cost every call 0.2 us).
+template <int SD, int G, int METRIC, bool LBG, bool PAD, bool DIST>
 __global__ void __launch_bounds__(256) k_assign_static(AssignArgs a, int sub_dim) {
     extern __shared__ float lds[];
     const int sd = PAD ? sub_dim : SD;
@@ -295,7 +296,7 @@ __global__ void __launch_bounds__(256) k_assign_static(AssignArgs a, int sub_dim
                 packed |= (uint32_t)best << (8 * g);
             else
                 a.codes[row * a.m + s] = (uint8_t)best;
-            if (a.dist) a.dist[row * a.m + s] = dist;  // uniform
+            if constexpr (DIST) a.dist[row * a.m + s] = dist;
         }
     }
     if constexpr (!LBG && G == 4) {

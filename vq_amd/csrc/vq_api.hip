@@ -76,11 +76,14 @@ template <int METRIC, bool LBG>
 int32_t launch_wide_exact(vq_ctx *ctx, const vq::AssignArgs &a, int sd, const uint32_t *list,
                           const uint32_t *count, const uint2 *pairs = nullptr, const uint32_t *pair_count = nullptr);
 
-template <int SD, int G, int METRIC, bool LBG, bool PAD>
+template <int SD, int G, int METRIC, bool LBG, bool PAD, bool DIST = false>
 int32_t launch_static(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
+    if constexpr (!LBG && !DIST && (METRIC == vq::M_L1 || SD <= 6)) {  // (assign_codes asks for no others)
+        if (a.dist) return launch_static<SD, G, METRIC, LBG, PAD, true>(ctx, a, sd);
+    }
     size_t lds = (size_t)G * a.k * SD * sizeof(float);
     if (METRIC == vq::M_COS) lds += (size_t)G * a.k * sizeof(float);
-    auto kern = vq::k_assign_static<SD, G, METRIC, LBG, PAD>;
+    auto kern = vq::k_assign_static<SD, G, METRIC, LBG, PAD, DIST>;
     if (lds > 48 * 1024)
         VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
