@@ -84,3 +84,18 @@ def test_encode_with_several_blocks_per_lane(ctx, n, m, sd, k):
         codes = ctx.to_device(np.full((n, m), 255, np.uint8))
         ctx.assign(metric, dx, n, m * sd, m, sd, k, dcb, codes)
         assert np.array_equal(codes.download(), O.pq_encode(om, x, cb).astype(np.uint8)), metric
+
+
+@pytest.mark.parametrize("n,m,sd,k", [(300, 3, 24, 256), (7000, 3, 24, 60), (300, 2, 25, 200), (300, 4, 28, 100), (9000, 4, 28, 100), (513, 1, 33, 256), (3000, 16, 33, 90),
+                                      (260, 2, 47, 256), (257, 4, 48, 130), (20_000, 3, 48, 40)])
+def test_manhattan_by_waves_and_by_lanes(ctx, n, m, sd, k):
+    """Blocks of 24 to 48 floats, few and many rows, short and long codebooks: whichever kernel takes them, also chunk by chunk."""
+    import vq_amd
+    rng = np.random.default_rng(n + sd)
+    x, cb = np.round(rng.standard_normal((n, m * sd)) * 2).astype(F), np.round(rng.standard_normal((m, k + 256, sd)) * 2).astype(F)
+    dx = ctx.to_device(x)
+    codes, wide = ctx.to_device(np.full((n, m), 255, np.uint8)), ctx.to_device(np.full((n, m), 65535, np.uint16))
+    ctx.assign(vq_amd.MANHATTAN, dx, n, m * sd, m, sd, k, ctx.to_device(np.ascontiguousarray(cb[:, :k])), codes)
+    assert np.array_equal(codes.download(), O.pq_encode(O.MANHATTAN, x, np.ascontiguousarray(cb[:, :k])).astype(np.uint8))
+    ctx.assign_u16(vq_amd.MANHATTAN, dx, n, m * sd, m, sd, k + 256, ctx.to_device(cb), wide)
+    assert np.array_equal(wide.download(), O.pq_encode(O.MANHATTAN, x, cb).astype(np.uint16))

@@ -120,10 +120,31 @@ int static_width(int sd) {
     return sd <= 6 ? sd : sd <= 8 ? 8 : sd <= 12 ? 12 : sd <= 16 ? 16 : sd <= 24 ? 24 : sd <= 32 ? 32 : sd <= 48 ? 48 : 0;
 }
 
+// Whether blocks of 24 floats and more (but 32) go to k_assign_wide_exact instead of k_assign_static: its waves share a
+// row's centroids, while a lane takes them one after the other, however few rows there are.  The model is within
+// 25 % at 600 to 150,000 rows, 1 to 16 blocks, Manhattan; microseconds, waves / lanes: 24 floats, k = 256, 600 x 4 12 / 41, 6000 x 16 55 / 42, k = 60 600 x 4
+// 12 / 11; 40 floats, k = 256, 600 x 4 16 / 70, 20,000 x 4 79 / 77, k = 100, 2000 x 4 16 / 32; 33 floats, k = 256, 2000 x 4 29 / 69, x 16 117 / 71
+// (whole pieces are read as such; of other widths a component at a time, and a codebook of more than 32 KB from beyond the
+// vector cache).
+bool wide_pays(int64_t n, int m, int sd, int k, bool vec) {
+    const int w = static_width(sd);
+    if (sd < 24 || sd == 32 || w == 0) return false;
+    const double pairs = (double)n * m, start = vec ? 7 + 0.2 * sd : 11 + 0.25 * sd;
+    const double lanes = (0.19 * w - 2.2 + k * (0.0043 * w + 0.04)) * std::max(1.0, pairs / 120e3);
+    const double step = vec ? 8.5e-8 : k * sd > 8192 ? 3.6e-7 : 1.2e-7;
+    const double waves = std::max({start, (7 + 0.2 * sd) * (0.35 + pairs / 22e3), 0.5 * start + pairs * k * sd * step});
+    return waves < lanes;
+}
+
+// The register width that an assignment by k_assign_static takes; 0: k_assign_wide_exact.
+int exact_width(const vq::AssignArgs &a, int sd) {
+    return wide_pays(a.n, a.m, sd, a.k, sd % 4 == 0 && (reinterpret_cast<uintptr_t>(a.cb) & 15) == 0) ? 0 : static_width(sd);
+}
+
 template <int METRIC, bool LBG>
 int32_t launch_assign_m(vq_ctx *ctx, const vq::AssignArgs &a, int sd) {
     const bool pad = static_width(sd) != sd;
-    switch (static_width(sd)) {
+    switch (exact_width(a, sd)) {
     case 1: return launch_static_g<1, METRIC, LBG>(ctx, a);
     case 2: return launch_static_g<2, METRIC, LBG>(ctx, a);
     case 3: return launch_static_g<3, METRIC, LBG>(ctx, a);
@@ -895,7 +916,7 @@ int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, i
     }
     if (!sdp) {
         // k_assign_static has the distance too: Manhattan, and blocks too narrow for the other kernels
-        if (d_dist && dist_written && !mfma8 && !pend && (metric == VQ_MANHATTAN ? static_width(sd) != 0 : sd <= 6)) {
+        if (d_dist && dist_written && !mfma8 && !pend && (metric == VQ_MANHATTAN ? exact_width(a, sd) != 0 : sd <= 6)) {
             a.dist = d_dist;
             *dist_written = true;
         }
