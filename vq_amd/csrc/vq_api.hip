@@ -526,7 +526,8 @@ double fit_static_us(int64_t n, int m, int sd, int k) {
 // behind them (150,000 rows x 12 blocks, an encode, microseconds padded against static): 7 floats k = 31 85 / 72, 48
 // 86 / 87, 80 89 / 117; 10 floats k = 48 128 / 115, 80 134 / 152; 20 floats 195 / 156, 208 / 230; 25 floats 289 / 243,
 // 298 / 331; cosine, 11 blocks: 7 floats k = 31 87 / 84, 48 87 / 100, 15 floats 136 / 119, 137 / 144, 20 floats k = 48 165 / 140, 64
-// 168 / 174: so the line is a number of centroids, about the same for all of them.  The passes of a fit lie no
+// 168 / 174; 33 floats, k = 48, 400,000 x 1 52 / 64, 150,000 x 4 81 / 92, k = 33 81 / 72; cosine, 15 floats, k = 33, 20,000 x 16 24.5 /
+// 30: so the line is a number of centroids, about the same for all of them.  The passes of a fit lie no
 // further apart, but its update needs fewer launches where the padded blocks make it a small one (12,000 x 12
 // blocks of 10, k = 24, six iterations: 241 against 705 us).  Widths that neither takes always gain.
 int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bool fit) {
@@ -549,7 +550,7 @@ int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bo
             : sd > 8            ? (fit ? a.k < 40 : cost < 3500)
                                 : sd == 2 || cost < 1600 || (a.m % 4 != 0 && (cost - 1600) * (double)(a.n * a.m) < 5e8))
             return 0;
-    } else if (w && a.k < (w > 16 ? 60 : metric == VQ_COSINE ? (w == 8 ? 32 : 40) : w == 8 ? 48 : 60)) {
+    } else if (w && a.k < (w == 48 ? 40 : w > 16 ? 60 : metric == VQ_COSINE ? (w == 8 ? 32 : 33) : w == 8 ? 48 : 60)) {
         return 0;
     }
     return sdp;
@@ -915,8 +916,9 @@ int32_t assign_codes(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, i
         a.cnorm = cnorm;
     }
     if (!sdp) {
-        // k_assign_static has the distance too: Manhattan, and blocks too narrow for the other kernels
-        if (d_dist && dist_written && !mfma8 && !pend && (metric == VQ_MANHATTAN ? exact_width(a, sd) != 0 : sd <= 6)) {
+        // k_assign_static has the distance too: Manhattan, and blocks too narrow for the other kernels (a distance of one
+        // component costs the merge less than reading it: 60,000 x 5, k = 600 40 -> 36.7 us)
+        if (d_dist && dist_written && !mfma8 && !pend && sd > 1 && (metric == VQ_MANHATTAN ? exact_width(a, sd) != 0 : sd <= 6)) {
             a.dist = d_dist;
             *dist_written = true;
         }
