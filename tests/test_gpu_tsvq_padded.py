@@ -34,3 +34,25 @@ def test_build(n, dim, extra, depth, kind):
         got["centroids"][nan] = want["centroids"][nan] = F(0)
     assert_same_tree(got, want)
     ctx.close()
+
+
+@pytest.mark.parametrize("n,dim,depth", [(8193, 262_133, 1), (8193, 262_139, 1), (8193, 262_144, 1), (5, 1_048_603, 2)])
+def test_widths_around_the_grids_limit(n, dim, depth):
+    """Rows whose columns, four or sixteen to a workgroup, pass 65,535 workgroups: all zeros but eight columns, so that the tree is
+    the one of those columns."""
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    rng = np.random.default_rng(dim)
+    cols = np.concatenate([[0], np.sort(rng.choice(np.arange(1, dim - 1), 6, replace=False)), [dim - 1]])
+    part = rng.standard_normal((n, 8)).astype(F)
+    x = np.zeros((n, dim), F)
+    x[:, cols] = part
+    got = ctx.tsvq_build(ctx.to_device(x), n, dim, dim, depth).download()
+    want, _ = bfs_order(O.tsvq_fit(part, depth))
+    rest = np.ones(dim, bool)
+    rest[cols] = False
+    assert not got["centroids"][:, rest].any()
+    got["centroids"] = np.ascontiguousarray(got["centroids"][:, cols])
+    want["split_dim"] = np.where(want["split_dim"] < 0, -1, cols[want["split_dim"]]).astype(want["split_dim"].dtype)
+    assert_same_tree(got, want)
+    ctx.close()

@@ -157,18 +157,18 @@ static __global__ void __launch_bounds__(256) k_seg_mean_wg(const float *__restr
     if (q == 0 && c < sd) out[(out_first + g) * sd + c] = tree[0][t] / __uint2float_rn(info.z);
 }
 
-// Sums of squared deviations in row order, a workgroup per segment and tile of up to 16 components (grid y; the last
-// one begins at dim less its width): seg_range[g] = {lo, hi} positions in perm; mean of segment g at means[(first + g) * dim].
+// Sums of squared deviations in row order, a workgroup per segment and tile of up to 16 components (block
+// tile * nseg + segment, as y would end at 65,535 tiles; the last tile begins at dim less its width): seg_range[g] = {lo, hi} positions in perm; mean of segment g at means[(first + g) * dim].
 // A chunk of 512 rows is a memory round trip, two barriers and their adds, 3.5 us in all: 7 ns a row.  Against one workgroup per segment with all
 // columns, whose one lane per column read its squares one by one: a root of 5,964 x 100 90 -> 41 us.
 template <int VEC>
-static __global__ void __launch_bounds__(256) k_seg_variance_tile(const uint32_t *__restrict__ perm, const uint2 *__restrict__ seg_range,
+static __global__ void __launch_bounds__(256) k_seg_variance_tile(const uint32_t *__restrict__ perm, const uint2 *__restrict__ seg_range, int nseg,
                                                                  const float *__restrict__ means, int64_t first,
                                                                  const float *__restrict__ x, int64_t ld, int dim, int width, int pieces,
                                                                  float *__restrict__ var) {
     extern __shared__ float4 lds_var[];
-    const int g = blockIdx.x;
-    const int c0 = (int)blockIdx.y * width < dim - width ? (int)blockIdx.y * width : dim - width;
+    const int g = blockIdx.x % (unsigned)nseg, tile = blockIdx.x / (unsigned)nseg;
+    const int c0 = tile * width < dim - width ? tile * width : dim - width;
     const uint2 r = seg_range[g];
     const float sum = member_tile_sum<256, VEC, true>(reinterpret_cast<float *>(lds_var), x + c0, ld, r.x, r.y, width, pieces,
                                                       [&](uint32_t p) { return perm[p]; }, means + (first + g) * dim + c0);

@@ -220,6 +220,9 @@ int32_t vq_tsvq_build_kmeans(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
 // 60,000 x 256 1064 / 1050 / 1065.
 static uint32_t var_tile_rows(int32_t dim) { return dim >= 96 ? 8192 : 4096; }
 
+// The columns that the composed maps take: their grids have a workgroup per four of them in y.
+constexpr int32_t kMapColumns = 4 * 65535;
+
 // The build on validated arguments.  real_dim: the components that count; the others, up to dim, are zeros.
 static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t dim, int32_t real_dim,
                                int32_t max_depth, const KmOpts *km, vq_tree **out);
@@ -235,8 +238,8 @@ static int32_t tsvq_build_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     // The composed maps take rows of whole groups of eight components.  Other rows with nodes that need them are copied
     // once with zeros behind them, for all levels: a column of zeros has the variance 0 and takes no part in the choice of the
     // split dimension.  (600,000 x 50, nine levels: 55.7 -> 2.6 ms against a lane per column that adds its squares one after the other.)
-    if (!km && dim % 8 != 0 && dim < (1 << 20) && n > (int64_t)var_tile_rows(dim)) {
-        const int32_t dimp = (dim + 7) / 8 * 8;
+    const int32_t dimp = dim <= kMapColumns ? (dim + 7) / 8 * 8 : dim;
+    if (!km && dim % 8 != 0 && dimp <= kMapColumns && n > (int64_t)var_tile_rows(dim)) {
         int32_t rc = ensure(ctx, ctx->pad_x, sizeof(float) * (size_t)n * dimp);
         if (rc == VQ_OK) {
             float *px = (float *)ctx->pad_x.p;
@@ -268,7 +271,7 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     // for a level's squares with every node starting on its own group of 32 positions
     constexpr int64_t kLeafWgSums = 65536;  // a lane per sum fills half of the chip: both take the same time there
     constexpr int kChainSegs = 2048;  // levels with more nodes than this take the other kernels
-    const bool var_chain = dim % 8 == 0;
+    const bool var_chain = dim % 8 == 0 && dim <= kMapColumns;
     // per group of 32 squares (composed-maps path): approximate sum, binade guess, integer maps;
     // the chain path keeps the squares themselves
     const bool var_maps = var_chain && ctx->tsvq_var_path == 0;
@@ -639,8 +642,8 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
         } else {
             const int tiles = (int)cdiv(dim, 16), width = tiles == 1 ? dim : (int)cdiv(cdiv(dim, tiles), 4) * 4;
             const int vec = dim >= 4 ? 4 : 1, pieces = (int)cdiv(width, vec);
-            hipLaunchKernelGGL(vec == 4 ? vq::k_seg_variance_tile<4> : vq::k_seg_variance_tile<1>, dim3(ns, cdiv(dim, width)), dim3(256),
-                               sizeof(float) * (size_t)width * (8 * (256 / pieces) + 4), st, perm, (const uint2 *)d_range, (const float *)d_smeans,
+            hipLaunchKernelGGL(vec == 4 ? vq::k_seg_variance_tile<4> : vq::k_seg_variance_tile<1>, dim3((unsigned)((int64_t)ns * cdiv(dim, width))), dim3(256),
+                               sizeof(float) * (size_t)width * (8 * (256 / pieces) + 4), st, perm, (const uint2 *)d_range, ns, (const float *)d_smeans,
                                (int64_t)0, d_x, ld, dim, width, pieces, (float *)d_var);
         }
         SP_HIP(hipGetLastError());
