@@ -56,6 +56,7 @@ struct vq_ctx {
     DevBuf tsvq_bsum, tsvq_segmaps;           // per block of groups: f64 sum; per run of groups: composed map
     int tsvq_var_path = 0;       // 0 = composed integer maps, 1 = one chain of adds per column
     DevBuf pad_x, pad_cb;        // rows and codebooks whose column blocks are padded to a multiple of 8 floats
+    bool pad_held = false;       // pad_x holds rows that a call still reads: nothing pads into it meanwhile
     DevBuf pad_rows;             // the same for a fit of more than 256 centroids, whose passes may pad slices of their own
     DevBuf mfma_tab, mfma_list, mfma_stat;  // tables, re-check list and counters of the matrix-core assignment
     int mfma_stat_cur = 0;       // which of the two sets of counters in mfma_stat the last pass used

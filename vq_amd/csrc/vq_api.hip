@@ -531,7 +531,7 @@ double fit_static_us(int64_t n, int m, int sd, int k) {
 // further apart, but its update needs fewer launches where the padded blocks make it a small one (12,000 x 12
 // blocks of 10, k = 24, six iterations: 241 against 705 us).  Widths that neither takes always gain.
 int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bool fit) {
-    if (ctx->assign_path == 1 || ctx->no_alloc || metric < VQ_SQEUCLIDEAN || metric > VQ_COSINE) return 0;
+    if (ctx->assign_path == 1 || ctx->no_alloc || ctx->pad_held || metric < VQ_SQEUCLIDEAN || metric > VQ_COSINE) return 0;
     if (sd == 1 || a.k < 2 || a.k > vq::kMaxK || a.m > 65535) return 0;
     if (mfma_applicable<vq::M_SQ, true>(ctx, a, sd) || mfma16_applicable<vq::M_SQ, true>(ctx, a, sd) ||
         mfma_wide_applicable<vq::M_SQ, true>(ctx, a, sd))

@@ -70,6 +70,11 @@ int32_t assign_big(vq_ctx *ctx, int metric, const float *d_x, int64_t n, int64_t
     VQ_TRY(ensure(ctx, ctx->pad_cb, sizeof(float) * (size_t)m * k * sdp));
     float *px = (float *)ctx->pad_x.p, *pcb = (float *)ctx->pad_cb.p;
     pad_blocks(ctx, d_codebooks, (int64_t)m * k, sd, 1, sd, sdp, pcb);
+    struct Held {  // the chunks of a slice never pad into the buffer that they read
+        bool &on;
+        explicit Held(bool &b) : on(b) { on = true; }
+        ~Held() { on = false; }
+    } held{ctx->pad_held};
     for (int64_t r0 = 0; r0 < n; r0 += slice) {
         const int64_t rows = std::min(slice, n - r0);
         pad_blocks(ctx, d_x + r0 * ld, rows, ld, m, sd, sdp, px);
