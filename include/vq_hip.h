@@ -75,10 +75,11 @@ void *vq_ctx_stream(vq_ctx *ctx);
  * Both give bit-identical codes; the switch exists for measurement and tests. */
 int32_t vq_ctx_set_assign_path(vq_ctx *ctx, int32_t path);
 
-/* Which kernels take an encode or a descent of a few rows (up to 512 (row, column block) pairs):
+/* Which kernels take an encode of a few rows (up to 512 (row, column block) pairs), or a descent of up to 512 rows:
  *   0 (default)  one workgroup per pair or row in one launch, where that is the faster way
  *   1            the kernels of longer calls
- * Both give the reference's results bit for bit; the switch exists for measurement and tests. */
+ * A descent has a wave per row for rows above 256 components, and below that only where vq_ctx_set_tsvq_descend_path
+ * is 1; other descents do not look at this switch.  Both give the reference's results bit for bit; the switch exists for measurement and tests. */
 int32_t vq_ctx_set_few_path(vq_ctx *ctx, int32_t path);
 
 /* How vq_tsvq_build sums a node's squared deviations per dimension in row order (src/tsvq.rs:88-99)
@@ -394,15 +395,17 @@ int32_t vq_tree_download(const vq_tree *tree, float *h_centroids, int32_t *h_lef
  * leaf reached; `<=` goes left, single children are followed.  Asynchronous. */
 int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld,
                         const vq_tree *tree, int32_t *d_leaf);
-/* How vq_tsvq_descend decides a node under cosine, squared Euclidean and Euclidean distance when
- * the row fits in registers (dim a multiple of 32 up to 128):
- *   0 (default)  by the sign of one inner product with a vector of the node (the difference of the
- *                children's normalised centroids, or of the centroids with a norm term), whenever
- *                its value clears a proven bound on every rounding error of the reference's two
- *                sums; otherwise, for that row, by those two sums
- *   1            by the two sums always
- * Both give the reference's leaves bit for bit; the switch exists for measurement and tests.
- * Manhattan always takes the two sums.  No counterpart in the reference. */
+/* How vq_tsvq_descend decides a node of rows of up to 256 components:
+ *   0 (default)  from sums in an order of their own, whenever they clear a proven bound on every rounding error of theirs
+ *                and of the reference's two sums; otherwise, for that row, by those two sums.  Cosine, squared Euclidean
+ *                and Euclidean: one inner product with a vector of the node (the difference of the children's
+ *                normalised centroids, or of the centroids with a norm term); Manhattan, and nodes beyond the
+ *                table of those vectors: both children's sums.  Narrow rows on few levels, where a sum is a load or
+ *                two, take the reference's sums; so does Manhattan where a lane holds a whole row (many rows of 32,
+ *                64, 96 or 128 components, 16-byte aligned, in a tree of up to 255 inner nodes)
+ *   1            by the two sums always: a wave per row for up to 512 rows (vq_ctx_set_few_path), a lane per row beyond
+ * Rows above 256 components always take the two sums.  Both give the reference's leaves bit for bit; the switch
+ * exists for measurement and tests.  No counterpart in the reference. */
 int32_t vq_ctx_set_tsvq_descend_path(vq_ctx *ctx, int32_t path);
 /* d_out[i] = f16(centroid of leaf d_leaf[i]) (src/tsvq.rs:241-248), n x dim.  Asynchronous. */
 int32_t vq_tsvq_decode_f16(vq_ctx *ctx, const vq_tree *tree, const int32_t *d_leaf, int64_t n,
