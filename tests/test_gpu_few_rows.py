@@ -103,7 +103,7 @@ def test_rvq_few(ctx, metric, n, dim, stages, k, eps):
 
 
 @pytest.mark.parametrize("metric", METRICS)
-@pytest.mark.parametrize("n,dim,depth", [(1, 3, 2), (40, 70, 6), (512, 128, 9)])
+@pytest.mark.parametrize("n,dim,depth", [(1, 3, 2), (40, 70, 6), (512, 128, 9), (1, 257, 4), (100, 300, 7), (512, 1031, 5)])
 def test_tsvq_few(ctx, metric, n, dim, depth):
     rng = np.random.default_rng(dim + depth)
     x = rng.standard_normal((max(n, 300), dim)).astype(F)
@@ -111,9 +111,15 @@ def test_tsvq_few(ctx, metric, n, dim, depth):
     t = tree.download()
     q = x[:n].copy()
     q[0] = 0.0
-    leaf = ctx.empty(n, np.int32)
-    ctx.tsvq_descend(metric, ctx.to_device(q), n, dim, tree, leaf)
-    assert np.array_equal(leaf.download(), O.tsvq_descend(metric, q, t))
+    want = O.tsvq_descend(metric, q, t)
+    try:
+        for path in (0, 1):  # 1, and rows above 256 components: a wave per row
+            ctx.set_tsvq_descend_path(path)
+            leaf = ctx.to_device(np.full(n, -1, np.int32))
+            ctx.tsvq_descend(metric, ctx.to_device(q), n, dim, tree, leaf)
+            assert np.array_equal(leaf.download(), want), path
+    finally:
+        ctx.set_tsvq_descend_path(0)
 
 
 @pytest.mark.parametrize("metric", METRICS)

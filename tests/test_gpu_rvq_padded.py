@@ -21,15 +21,23 @@ def test_encode(metric, n, dim, extra, stages, k, eps):
     buf[::50] *= F(1e-3)
     buf[3] = 0.0
     buf[9, 0] = np.inf
+    for r in range(10, n, 7):  # rows that stop after one or two stages
+        buf[r, :dim] = cb[:1 + r % 2, r % k].sum(0) + F(1e-5) * rng.standard_normal(dim).astype(F)
     x = np.ascontiguousarray(buf[:, :dim])
     dx, dcb = ctx.to_device(buf), ctx.to_device(cb)
-    codes, used, rec = ctx.empty((n, stages), np.uint8), ctx.empty(n, np.uint8), ctx.empty((n, dim), np.uint16)
     with np.errstate(all="ignore"):
         want, want_rec = O.rvq_quantize(metric, x, cb, eps)
+    reached = want != 0xFFFFFFFF
+    assert reached.all() == (eps == 0.0 or stages == 1)
     fine = np.arange(n) != 9  # (sums of infinities of both signs: no number, whatever its bits)
     for with_used, with_rec in ((True, True), (False, True), (False, False)):
+        # (what each call has to write is something else before it)
+        codes, used = ctx.to_device(~np.where(reached, want, 0).astype(np.uint8)), ctx.to_device(np.full(n, 99, np.uint8))
+        rec = ctx.to_device(~np.asarray(want_rec).view(np.uint16))
         ctx.rvq_encode(metric, dx, n, dim + extra, dim, stages, k, dcb, eps, codes, used if with_used else None, rec if with_rec else None)
-        assert np.array_equal(codes.download()[fine], want.astype(np.uint8)[fine])
+        assert np.array_equal(codes.download()[fine], np.where(reached, want, 0).astype(np.uint8)[fine])
+        if with_used:
+            assert np.array_equal(used.download()[fine], reached.sum(1)[fine])
         if with_rec:
             assert np.array_equal(rec.download()[fine], np.asarray(want_rec).view(np.uint16)[fine])
     assert np.array_equal(dx.download(), buf, equal_nan=True)

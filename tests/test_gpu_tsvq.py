@@ -184,7 +184,7 @@ def _hand_tree(ctx, cen, depth):
 
 
 @pytest.mark.parametrize("metric", [O.SQEUCLIDEAN, O.EUCLIDEAN, O.COSINE])
-@pytest.mark.parametrize("dim", [32, 64, 128])
+@pytest.mark.parametrize("dim", [32, 64, 96, 128])
 @pytest.mark.parametrize("kind", ["ties", "near_ties", "scales", "zero_norms", "non_finite", "far_offset",
                                   "equal_children"])
 def test_descent_by_one_inner_product_agrees_with_the_two_distances(ctx, metric, dim, kind):
@@ -251,3 +251,10 @@ def test_descent_by_one_inner_product_agrees_with_the_two_distances(ctx, metric,
             assert np.array_equal(got, want), (path, int((got != want).sum()))
     finally:
         ctx.set_tsvq_descend_path(0)
+    # the same rows over and over, beyond 65,536 of them: a row per lane, and per lane another one each time (3000 is no multiple of 64)
+    times = 23
+    many = ctx.to_device(np.tile(q, (times, 1)))
+    leaves = ctx.to_device(np.full(times * n, -1, np.int32))
+    ctx.tsvq_descend(metric, many, times * n, dim, tree, leaves)
+    got = leaves.download().reshape(times, n)
+    assert np.array_equal(got, np.broadcast_to(want, got.shape)), int((got != want).sum())
