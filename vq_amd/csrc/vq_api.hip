@@ -491,29 +491,35 @@ template <int METRIC, bool LBG> int32_t launch_mfma16(vq_ctx *ctx, const vq::Ass
     return VQ_OK;
 }
 
-// Whether the sums of a fit's blocks of 8 floats are streamed (k_lbg_stream8) or go by the lists of members.  The
-// streaming kernel's time does not depend on where the rows of a cluster are, but the fewer clusters share a tile of rows, the
-// more rounds it takes (one wave's chain over a part: 270 us per iteration at 4 clusters, 150 at 16, 120 at 40); the lists
-// and their leaves take 48 us and 32 per million (row, block) pairs, k = 4 to 100 (60 and 32 when the figures below were taken).  Per iteration, lists / streamed:
-// 250,000 x 12 k = 4 148 / 287, 16 150 / 176, 32 152 / 151, 112 170 / 138, 256 226 / 177; x 33 k = 4 309 / 400,
-// 10 310 / 289, 40 312 / 221; 1M x 16 k = 4 579 / 628, 10 578 / 459; 60,000 x 48 k = 16 153 / 181, 40 156 / 149, 80 (fewer
-// than 1024 rows per centroid: short lists) 168 / 190; 250,000 x 4 k = 56 89 / 116, 256 117 / 130.
+// Microseconds per iteration of a fit of blocks of 8 floats whose sums go by the lists of members, or are streamed
+// (k_lbg_stream8).  The lists and their leaves cost by the (row, block) pair, and more with the centroids among which a
+// part's rows are spread.  The streaming kernel costs less per pair, but takes more rounds the fewer clusters share a tile of rows (one wave's
+// chain over a part), and its clusters of up to 1024 members go by the lists as well.  Within 17 % of (lists / streamed): 250,000 x 12 k = 4 129 / 256, 16 129 / 157, 40 132 / 134, 112 155 / 125, 256
+// 212 / 162; x 33 k = 6 288 / 317, 10 287 / 266, 40 290 / 205; 1M x 16 k = 4 575 / 583, 6 572 / 497; 600,000 x 4 k = 64
+// 133 / 122, 128 140 / 118; 500,000 x 5 k = 64 132 / 119, 200 170 / 123, x 8 k = 24 167 / 154; 100,000 x 32 k = 48 142 / 133, 96
+// 153 / 160; 60,000 x 48 k = 40 132 / 132, 80 143 / 179; 150,000 x 16 k = 128 133 / 142; 250,000 x 4 k = 56 68 / 105, 256 98 / 122.
+double fit8_lists_us(int64_t n, int m, int k) {
+    return 28 + (double)n * m * 1e-6 * (33.5 + 0.09 * k);
+}
+double fit8_streamed_us(int64_t n, int m, int k) {
+    const double members = (double)n / k;  // of an average cluster
+    return 80 + 420.0 / k + (double)n * m * 1e-6 * (13 + 50.0 / k) + std::max(0.0, 0.066 * (1600 - members));
+}
+// (four blocks to a workgroup: a last group with idle waves from 61,441 rows on only)
 bool stream_pays(int64_t n, int m, int k) {
-    const double pairs = (double)n * m;
-    return pairs >= 2e6 + 6e7 / k && (n > (int64_t)vq::kSeqMax * k || pairs >= 2.95e6);
+    return (m % 4 == 0 || n > 15 * vq::kPartRows) && fit8_streamed_us(n, m, k) < fit8_lists_us(n, m, k);
 }
 
-// Microseconds per iteration of a fit of blocks of 8 floats, and of narrower blocks of their own width, for the choice between
-// them (within 15 % at 30,000 to 1M rows, 4 to 48 blocks, k = 4 to 256).  Narrow blocks are cheaper where
-// memory bounds both: 250,000 x 12 blocks of 3, k = 32 137 / 152, 80 174 / 147; x 33 of 6, k = 4 389 / 323, 46 blocks of 7
-// 430 / 240; 60,000 x 12 of 6, k = 24 85 / 86, 56 99 / 89.
+// The same of a fit of 8 floats by the faster way and of narrower blocks of their own width, for the choice between them.
+// Own width / padded, measured: 250,000 x 12 blocks of 3, k = 32 121 / 131, 80 148 / 131; x 33 of 6, k = 4 362 / 288, x 46 of 7 474 / 386;
+// 60,000 x 12 of 6, k = 24 57 / 55, 56 74 / 65; 100,000 x 13 of 5, k = 48 80 / 76, 200 139 / 91; 200,000 x 16 of two, k = 64
+// 139 / 130; 500,000 x 12 of 6, k = 40 267 / 175, 100 405 / 170; 1M x 4 of 4, k = 64 195 / 138, 200 354 / 155; 60,007 x 25 of 4, k = 60 90 / 99.
 double fit8_us(int64_t n, int m, int k) {
-    const double mp = (double)n * m * 1e-6;
-    return stream_pays(n, m, k) ? 95 + 650.0 / k + mp * (16 + 40.0 / k) : 48 + 33 * mp;
+    return stream_pays(n, m, k) ? fit8_streamed_us(n, m, k) : fit8_lists_us(n, m, k);
 }
 double fit_static_us(int64_t n, int m, int sd, int k) {
     const double mp = (double)n * m * 1e-6, spread = m % 2 ? 0.6 + 0.15 * sd : 1.0;  // (odd: one block per lane)
-    return 42 + mp * (19 + std::max(13 * spread, 0.022 * (3 * (sd == 7 ? 8 : sd) + 1) * k));
+    return 28 + mp * (22 + std::max(13 * spread, 0.022 * (3 * (sd == 7 ? 8 : sd) + 1) * k));
 }
 
 // The width to pad every column block to so that the matrix-core kernels take the shape (squared L2,
@@ -1493,9 +1499,8 @@ static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld,
 
     const int nparts = (int)((n + vq::kPartRows - 1) / vq::kPartRows);
     const int nseg = (nparts + vq::kScanSeg - 1) / vq::kScanSeg;
-    // streaming sums of the large clusters: 32-byte sub-vectors, 4 to a workgroup, aligned rows (a last
-    // group with idle waves pays from some 60,000 rows on)
-    const bool stream = sd == 8 && stream_pays(n, m, k) && (m % 4 == 0 || nparts >= 16) && ld % 4 == 0 && ld <= (1 << 20) &&
+    // streaming sums of the large clusters: 32-byte sub-vectors, 4 to a workgroup, aligned rows
+    const bool stream = sd == 8 && stream_pays(n, m, k) && ld % 4 == 0 && ld <= (1 << 20) &&
                         (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;  // (32-bit lane offsets inside a chunk)
     const int64_t leaf_cap64 = stream ? (int64_t)k : (int64_t)k * nparts;
     if (leaf_cap64 * sd > (1LL << 31)) return fail(ctx, VQ_ERR_UNSUPPORTED, "n * k * sub_dim too large");
