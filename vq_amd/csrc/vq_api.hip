@@ -535,7 +535,10 @@ double fit_static_us(int64_t n, int m, int sd, int k) {
 // 168 / 174; 33 floats, k = 48, 400,000 x 1 52 / 64, 150,000 x 4 81 / 92, k = 33 81 / 72; cosine, 15 floats, k = 33, 20,000 x 16 24.5 /
 // 30: so the line is a number of centroids, about the same for all of them.  The passes of a fit lie no
 // further apart, but its update needs fewer launches where the padded blocks make it a small one (12,000 x 12
-// blocks of 10, k = 24, six iterations: 241 against 705 us).  Widths that neither takes always gain.
+// blocks of 10, k = 24, six iterations: 241 against 705 us).  Where the update is a small one at both widths (multiples
+// of four floats; per iteration own / padded): 431 x 15 blocks of 4, k = 16 12.5 / 14.8, k = 32 12.9 / 14.7, 10,000 x 15 of 4, k = 64 19.6 / 20.1, 256
+// 31 / 24; of 12, k = 16 13 / 15.4, 32 15.4 / 15.9, 64 18.9 / 16; of 20, k = 16 16.8 / 23.5, 32 19.3 / 22.8, 64 26 / 22.7; of 28, k = 32 22.5 / 23.5,
+// 64 30 / 23.  Widths that neither takes always gain.
 int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bool fit) {
     if (ctx->assign_path == 1 || ctx->no_alloc || ctx->pad_held || metric < VQ_SQEUCLIDEAN || metric > VQ_COSINE) return 0;
     if (sd == 1 || a.k < 2 || a.k > vq::kMaxK || a.m > 65535) return 0;
@@ -547,6 +550,8 @@ int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bo
     // the limits of those kernels
     if ((int64_t)a.m * sdp > (1 << 20) || sdp > (1 << 16) || a.n * a.m >= (1LL << 32)) return 0;
     const int w = static_width(sd);
+    // few rows, whose update is one launch at either width: padding adds its own launches and pays by the scores alone
+    if (fit && sd <= 28 && a.k < 40 && lbg_small(a.n, a.m, sd, a.k)) return 0;
     if (fit && sd != sdp && lbg_small(a.n, a.m, sdp, a.k)) return sdp;
     if (fit && sd < 8) return fit8_us(a.n, a.m, a.k) < fit_static_us(a.n, a.m, sd, a.k) ? sdp : 0;
     if (fit && w && w != sd && (w <= 16 || w == 32)) return a.k >= (w == 32 ? 36 : 40) || (w <= 16 && a.m % 2 == 0) ? sdp : 0;
