@@ -123,6 +123,27 @@ def test_tsvq_few(ctx, metric, n, dim, depth):
 
 
 @pytest.mark.parametrize("metric", METRICS)
+@pytest.mark.parametrize("dim,depth", [(7, 3), (16, 4), (16, 6), (24, 8), (36, 3), (72, 3), (100, 9), (130, 1), (200, 1), (200, 4), (256, 3), (257, 2)])
+def test_tsvq_few_levels_and_host_rows(ctx, metric, dim, depth):
+    """On both sides of the line between a wave and four lanes per row, in GPU memory, and from host rows to f16 rows."""
+    from vq_amd import api
+    dist = {O.SQEUCLIDEAN: api.Distance.SquaredEuclidean, O.EUCLIDEAN: api.Distance.Euclidean, O.COSINE: api.Distance.CosineDistance,
+            O.MANHATTAN: api.Distance.Manhattan}[metric]
+    x = np.round(np.random.default_rng(dim).standard_normal((1000, dim)) * 4).astype(F)  # ties
+    q = api.TSVQ.new(x, depth, dist)
+    t = q.tree()
+    want = O.tsvq_descend(metric, x[:512], t)
+    rows = t["centroids"][want].astype(np.float16).view(np.uint16)
+    tree = ctx.tsvq_build(ctx.to_device(x), len(x), dim, dim, depth)
+    dx = ctx.to_device(x)
+    for n in (1, 17, 32, 33, 129, 512):
+        leaf = ctx.to_device(np.full(n, -1, np.int32))
+        ctx.tsvq_descend(metric, dx, n, dim, tree, leaf)
+        assert np.array_equal(leaf.download(), want[:n]), n
+        assert np.array_equal(q.quantize_batch(x[:n]).view(np.uint16), rows[:n]), n
+
+
+@pytest.mark.parametrize("metric", METRICS)
 @pytest.mark.parametrize("dim,depth", [(32, 8), (128, 9)])
 def test_tsvq_rows_on_both_sides_of_the_lines(ctx, metric, dim, depth):
     """Row widths that fit registers: which kernel takes a few rows depends on their number and the tree's size."""

@@ -1729,9 +1729,10 @@ __device__ __forceinline__ void quad_pair(const quad_piece (&xr)[NP], float &sl,
 }
 
 // tab: the table of k_tsvq_wtable with sctab, of ntab nodes, or the centroids themselves (Manhattan); ntop: the nodes of it in
-// LDS.  out16 (nullable): the leaves' centroids.
-template <int METRIC, int NP>
-__global__ void __launch_bounds__(512, 2 * quad_per_cu(NP)) k_tsvq_descend_quad(const float *__restrict__ x, int64_t n, int64_t ld, int dim,
+// LDS.  OUT: the leaves' centroids into out16 as well, for a few rows: an instance of its own with registers for the loads of 16 rows
+// (a row's load behind the store of the one before was 2 to 4 us of a call; with four rows' loads in the common instance it spills).
+template <int METRIC, int NP, bool OUT>
+__global__ void __launch_bounds__(512, OUT ? 2 : 2 * quad_per_cu(NP)) k_tsvq_descend_quad(const float *__restrict__ x, int64_t n, int64_t ld, int dim,
                                                            const float *__restrict__ cen,
                                                            const float *__restrict__ cnorm,
                                                            const int *__restrict__ left,
@@ -1890,11 +1891,19 @@ __global__ void __launch_bounds__(512, 2 * quad_per_cu(NP)) k_tsvq_descend_quad(
             }
         }
         if (q == 0 && row < n) leaf[row] = node;
-        if (out16)  // a row at a time by the whole wave: runs of 128 bytes, also into host memory
-            for (int i = 0; i < 16 && batch * 16 + i < n; ++i) {
-                const float *__restrict__ c = cen + (size_t)__shfl(node, 4 * i) * dim;
-                for (int t = threadIdx.x & 63; t < dim; t += 64) out16[(batch * 16 + i) * dim + t] = __half_as_ushort(__float2half_rn(c[t]));
+        if constexpr (OUT) {  // a row at a time by the whole wave: runs of 128 bytes, also into host memory; all rows' loads in flight
+            const float *c[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) c[i] = cen + (size_t)__builtin_amdgcn_readlane(node, 4 * i) * dim;
+            for (int t = threadIdx.x & 63; t < dim; t += 64) {
+                float v[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[i] = c[i][t];
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (batch * 16 + i < n) out16[(batch * 16 + i) * dim + t] = __half_as_ushort(__float2half_rn(v[i]));
             }
+        }
     }  // batches
 }
 

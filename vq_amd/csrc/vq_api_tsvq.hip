@@ -114,19 +114,38 @@ bool quad_applicable(const vq_ctx *ctx, const vq_tree *tree) {
     return ctx->tsvq_descend_path == 0 && tree->dim <= kQuadDims;
 }
 
+int tree_levels(const vq_tree *tree) {  // of a complete tree with as many inner nodes
+    int levels = 0;
+    while (tree->n_inner >> levels) ++levels;
+    return levels;
+}
+
 // Narrow rows on few levels go to the kernel with a lane per row (k_tsvq_descend): a node is a load or two then, and four lanes
 // hold a row of one piece.  Times of the four lanes over the lane's, 600 to 1M rows: 1 component 1.1 to 4 at any depth, 3
 // components 1.1-2.9 (one level), 1.04-1.4 (six), 0.8-1.06 (ten), 5 components 1.06-1.5 (two levels), 1.0-1.2 (three), 0.9-1.0 (four;
 // 1.06-1.13 from 131,000 rows on), 8 components 0.9-1.1 (one level), 0.6-0.9 (two), 16 components 0.5-1 (one level).
 bool lane_per_row(const vq_tree *tree, int64_t n) {
-    int levels = 0;  // of a complete tree with as many inner nodes
-    while (tree->n_inner >> levels) ++levels;
+    const int levels = tree_levels(tree);
     return tree->dim <= 2 || (tree->dim == 3 && levels <= 8) || tree->dim * levels <= (n > 100'000 && tree->dim <= 6 ? 20 : 15);
 }
 
-template <int METRIC, int NP>
+// A few rows (few_applicable) on few levels go to the kernel with a wave per row (k_tsvq_few), which starts without a table of
+// nodes.  Microseconds, waves / four lanes, 256 rows in GPU memory, cosine: one level of 36 components 5.6 / 6.1, 128 5.7 / 5.7, 200 7.5 / 6.2, three levels
+// of 16 5.6 / 6.1, 36 5.7 / 6.0, 72 7.5 / 6.3; Manhattan, one level of 200 5.8 / 6.2, three of 36 5.6 / 6.1, 72 6.6 / 6.4.  host: the kernel writes
+// the f16 rows as well, where a wave per row spreads the writes: 256 rows, three levels of 8 24.0 / 25.4, Manhattan, 200 40.9 / 44.3, 256
+// 45.3 / 48.6, one level of 256 38.6 / 41.4.
+bool wave_per_row(const vq_tree *tree, int32_t metric, int64_t n, bool host) {
+    const int levels = tree_levels(tree), dim = tree->dim;
+    const bool l1 = metric == VQ_MANHATTAN;
+    if (host && (dim < 12 || (l1 && dim > 128 && dim * levels <= 800 && n > 32))) return true;
+    return dim >= 8 && levels <= 4 && levels * (l1 ? 0.1 + 0.006 * dim : 0.2 + 0.009 * dim) < 1.6;
+}
+
+template <int METRIC, int NP, bool OUT = false>
 int32_t descend_quad_np(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, const vq_tree *tree, int32_t *d_leaf,
                         uint16_t *d_out) {
+    if constexpr (!OUT)
+        if (d_out) return descend_quad_np<METRIC, NP, true>(ctx, d_x, n, ld, tree, d_leaf, d_out);
     constexpr bool l1 = METRIC == vq::M_L1, cosine = METRIC == vq::M_COS;
     // As many workgroups on a compute unit as its registers hold, the LDS shared among them: the nodes that do not
     // fit are read from the L2, which costs less than the waves a larger table displaces (480,000 x 32, ten levels: a third
@@ -143,14 +162,14 @@ int32_t descend_quad_np(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, co
     const size_t lds = per_node * (size_t)std::max(ntop, 1);
     static_assert(NP <= 16 && METRIC >= 0 && METRIC < 4, "a bit per instance");
     constexpr uint64_t instance = 1ull << (METRIC * 16 + NP - 1);
-    if (lds > 48 * 1024 && !(ctx->quad_lds_set & instance)) {
-        VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_tsvq_descend_quad<METRIC, NP>),
+    if (lds > 48 * 1024 && !(ctx->quad_lds_set[OUT] & instance)) {
+        VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_tsvq_descend_quad<METRIC, NP, OUT>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBudget));
-        ctx->quad_lds_set |= instance;
+        ctx->quad_lds_set[OUT] |= instance;
     }
     VQ_TRY(know_compute_units(ctx));
     const dim3 grid(std::min<unsigned>(cdiv(n, threads / 4), few ? ~0u : (unsigned)ctx->compute_units * kPerCu));
-    hipLaunchKernelGGL((vq::k_tsvq_descend_quad<METRIC, NP>), grid, dim3(threads), lds, ctx->stream, d_x, n, ld, tree->dim, tree->d_centroids,
+    hipLaunchKernelGGL((vq::k_tsvq_descend_quad<METRIC, NP, OUT>), grid, dim3(threads), lds, ctx->stream, d_x, n, ld, tree->dim, tree->d_centroids,
                        tree->d_cnorm, tree->d_left, tree->d_right, l1 ? tree->d_centroids : cosine ? tree->d_wcos : tree->d_wl2,
                        cosine ? tree->d_sccos : tree->d_scl2, ntop, std::min(tree->n_nodes, (int32_t)vq::kTopNodes), d_leaf, d_out);
     VQ_HIP(ctx, hipGetLastError());
@@ -866,9 +885,10 @@ int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n
     // against 38.7, 480,000 x 32, eight levels 28 against 32; but 66,000 x 128 27.9 against 27.4, 20,000 23.5 against
     // 15.7, and ten levels 500,000 x 128 179 against 137.
     const bool narrow = quad_applicable(ctx, tree) && lane_per_row(tree, n);
-    if (!narrow && quad_applicable(ctx, tree) && !(regs && tree->n_inner <= vq::kTopNodes && n > (int64_t)ctx->compute_units * 256))
+    const bool few = few_applicable(ctx, n, tree->dim) && (!quad_applicable(ctx, tree) || wave_per_row(tree, metric, n, false));
+    if (!narrow && !few && quad_applicable(ctx, tree) && !(regs && tree->n_inner <= vq::kTopNodes && n > (int64_t)ctx->compute_units * 256))
         return descend_quad(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
-    if (!narrow && few_applicable(ctx, n, tree->dim)) return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
+    if (!narrow && few) return descend_few(ctx, metric, d_x, n, ld, tree, d_leaf, nullptr);
     if (regs && !narrow) {
         // one workgroup per compute unit (the staged centroids fill its LDS), walking over the rows
         dim3 g(std::min<unsigned>(cdiv(n, 512), (unsigned)ctx->compute_units)), b(512);
@@ -945,7 +965,7 @@ int32_t vq_tsvq_quantize_host(vq_ctx *ctx, int32_t metric, const float *h_x, int
                       [&](const float *d_x, int64_t rows, void *d_out, void *d_leaf) -> int32_t {
                           uint16_t *out = h_out ? (uint16_t *)d_out : nullptr;
                           if (few_applicable(ctx, rows, dim)) {
-                              if (quad_applicable(ctx, tree))
+                              if (quad_applicable(ctx, tree) && !wave_per_row(tree, metric, rows, true))
                                   return descend_quad(ctx, metric, d_x, rows, dim, tree, (int32_t *)d_leaf, out);
                               return descend_few(ctx, metric, d_x, rows, dim, tree, (int32_t *)d_leaf, out);
                           }
