@@ -26,7 +26,10 @@ CASES = [(16, 4, 8, 16, 3, "normal"),          # one row per cluster
          (9000, 2, 12, 40, 4, "same"),         # one cluster, every other one re-seeded
          (2000, 5, 8, 7, 30, "blobs"),         # early stop
          (3000, 2, 32, 20, 3, "normal"), (5000, 1, 36, 64, 3, "normal"), (4097, 1, 100, 33, 3, "normal"),
-         (12_000, 1, 256, 256, 2, "skewed"), (20_001, 2, 40, 64, 3, "skewed"), (10_000, 1, 48, 16, 3, "same"), (6000, 2, 64, 32, 3, "skewed"), (300, 1, 1000, 5, 2, "normal")]
+         (12_000, 1, 256, 256, 2, "skewed"), (20_001, 2, 40, 64, 3, "skewed"), (10_000, 1, 48, 16, 3, "same"), (6000, 2, 64, 32, 3, "skewed"), (300, 1, 1000, 5, 2, "normal"),
+         # blocks of their own width up to 39 centroids, padded from 40 on
+         (431, 15, 4, 32, 4, "normal"), (900, 3, 4, 39, 3, "normal"), (900, 3, 4, 40, 3, "normal"), (2000, 3, 12, 39, 3, "blobs"), (2000, 3, 12, 40, 3, "blobs"),
+         (2000, 5, 20, 39, 3, "normal"), (2000, 5, 20, 40, 3, "normal"), (3000, 2, 28, 39, 3, "skewed"), (3000, 2, 28, 40, 3, "skewed")]
 
 
 @pytest.mark.parametrize("n,m,sd,k,iters,kind", CASES)
