@@ -173,16 +173,6 @@ inline int32_t ensure_pinned(vq_ctx *ctx, void *&p, size_t &cap, size_t bytes) {
     return VQ_OK;
 }
 
-// Sets ctx->compute_units.  (The runtime's query is 0.3 us, a tenth of a small call.)
-inline int32_t know_compute_units(vq_ctx *ctx) {
-    if (ctx->compute_units == 0) {
-        int cus = 0;
-        VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-        ctx->compute_units = cus > 0 ? cus : 1;
-    }
-    return VQ_OK;
-}
-
 inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
 inline hipEvent_t prof_event(vq_ctx *ctx) {
@@ -274,6 +264,9 @@ inline bool assign_few_applicable(const vq_ctx *ctx, int64_t n, int32_t m, int32
 // take a pending update along.
 bool assign_pending_fusable(const vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t sd,
                             int32_t k, const float *d_codebook);
+
+// Sets ctx->compute_units.  (The runtime's query is 0.3 us, a tenth of a small call.)
+int32_t know_compute_units(vq_ctx *ctx);
 
 // The width to which an encode pads the column blocks of such rows (0: not at all), and the copy itself:
 // n rows of m blocks of sd floats to m blocks of sdp floats, zeros after each block.

@@ -851,6 +851,15 @@ int encode_pad_width(const vq_ctx *ctx, int32_t metric, const float *d_x, int64_
     return pad_width(ctx, metric, a, sd, false);
 }
 
+int32_t know_compute_units(vq_ctx *ctx) {
+    if (ctx->compute_units == 0) {
+        int cus = 0;
+        VQ_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+        ctx->compute_units = cus > 0 ? cus : 1;
+    }
+    return VQ_OK;
+}
+
 void pad_blocks(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t sdp, float *d_y) {
     launch_pad(ctx, d_x, n, ld, m, sd, sdp, d_y);
 }
