@@ -78,7 +78,7 @@ int32_t vq_ctx_set_assign_path(vq_ctx *ctx, int32_t path);
 /* Which kernels take an encode of a few rows (up to 512 (row, column block) pairs), or a descent of up to 512 rows:
  *   0 (default)  one workgroup per pair or row in one launch, where that is the faster way
  *   1            the kernels of longer calls
- * A descent has a wave per row for rows above 256 components, and below that only where vq_ctx_set_tsvq_descend_path
+ * A descent has a wave per row for rows above 256 components, on few levels, and where vq_ctx_set_tsvq_descend_path
  * is 1; other descents do not look at this switch.  Both give the reference's results bit for bit; the switch exists for measurement and tests. */
 int32_t vq_ctx_set_few_path(vq_ctx *ctx, int32_t path);
 
@@ -401,7 +401,7 @@ int32_t vq_tsvq_descend(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n
  *                and Euclidean: one inner product with a vector of the node (the difference of the children's
  *                normalised centroids, or of the centroids with a norm term); Manhattan, and nodes beyond the
  *                table of those vectors: both children's sums.  Narrow rows on few levels, where a sum is a load or
- *                two, take the reference's sums; so does Manhattan where a lane holds a whole row (many rows of 32,
+ *                two, and up to 512 rows on few levels take the reference's sums; so does Manhattan where a lane holds a whole row (many rows of 32,
  *                64, 96 or 128 components, 16-byte aligned, in a tree of up to 255 inner nodes)
  *   1            by the two sums always: a wave per row for up to 512 rows (vq_ctx_set_few_path), a lane per row beyond
  * Rows above 256 components always take the two sums.  Both give the reference's leaves bit for bit; the switch

@@ -1910,7 +1910,7 @@ __global__ void __launch_bounds__(512, OUT ? 2 : 2 * quad_per_cu(NP)) k_tsvq_des
 // TSVQNode::quantize_with_distance (src/tsvq.rs:162-181) for a few rows: one wave per row, which brings
 // both children's centroids of a node into LDS with whole-line loads; lane 0 adds up the left distance
 // and lane 1 the right one, each in the reference's order.  out16 (nullable): the leaf's centroid.
-// (For widths beyond k_tsvq_descend_quad.)
+// (For widths beyond k_tsvq_descend_quad, and where few levels are over before that kernel's table is read.)
 template <int METRIC>
 __global__ void __launch_bounds__(64) k_tsvq_few(const float *__restrict__ x, int64_t ld, int dim,
                                                  const float *__restrict__ cen, const float *__restrict__ cnorm,

@@ -529,11 +529,13 @@ double fit_static_us(int64_t n, int m, int sd, int k) {
 // width), the padded kernels about 600 per row and block and half the bytes more to read.  Its own widths: the
 // lines below are where the two took the same time at 20,000-600,000 rows, 12 and 25 blocks; one float
 // per block leaves most rows to the exact path of the matrix-core kernels: never.  Widths that it holds with zeros
-// behind them (150,000 rows x 12 blocks, an encode, microseconds padded against static): 7 floats k = 31 85 / 72, 48
-// 86 / 87, 80 89 / 117; 10 floats k = 48 128 / 115, 80 134 / 152; 20 floats 195 / 156, 208 / 230; 25 floats 289 / 243,
-// 298 / 331; cosine, 11 blocks: 7 floats k = 31 87 / 84, 48 87 / 100, 15 floats 136 / 119, 137 / 144, 20 floats k = 48 165 / 140, 64
-// 168 / 174; 33 floats, k = 48, 400,000 x 1 52 / 64, 150,000 x 4 81 / 92, k = 33 81 / 72; cosine, 15 floats, k = 33, 20,000 x 16 24.5 /
-// 30: so the line is a number of centroids, about the same for all of them.  The passes of a fit lie no
+// behind them (150,000 rows, an assignment, microseconds padded / static, 12 blocks, then 11): 7 floats k = 31 58 / 43, 55 / 46, 48
+// 55 / 54, 55 / 49, 64 56 / 67, 53 / 58; 10 floats k = 48 86 / 70, 82 / 62, 60 88 / 83, 83 / 74, 80 94 / 111, 88 / 95; 20 floats
+// k = 48 166 / 144, 140 / 121, 60 165 / 156, 139 / 148, 80 173 / 200, 149 / 189; 25 floats k = 60 201 / 193, 185 / 181, 80 210 / 255, 194 / 244;
+// cosine, 11 blocks: 7 floats k = 31 56 / 53, 48 57 / 67, 15 floats k = 33 83 / 69, 40 85 / 80, 60 85 / 112, 20 floats k = 48 136 / 123, 60
+// 135 / 142; 33 floats, k = 48, 400,000 x 1 52 / 64, 150,000 x 4 81 / 92, k = 33 81 / 72; cosine, 15 floats, k = 33, 20,000 x 16 24.5 /
+// 30: so the line is a number of centroids, about the same for all of them and for odd numbers of blocks (few rows have it higher: 30,000 x 11
+// of 7, k = 48 24 / 16, of 10, k = 60 29 / 23).  The passes of a fit lie no
 // further apart, but its update needs fewer launches where the padded blocks make it a small one (12,000 x 12
 // blocks of 10, k = 24, six iterations: 241 against 705 us).  Where the update is a small one at both widths (multiples
 // of four floats; per iteration own / padded): 431 x 15 blocks of 4, k = 16 12.5 / 14.8, k = 32 12.9 / 14.7, 10,000 x 15 of 4, k = 64 19.6 / 20.1, 256
