@@ -143,3 +143,28 @@ def test_rows_with_many_candidates(ctx, n, m, sd, k, metric, kind):
     finally:
         ctx.set_assign_path(0)
     assert np.array_equal(got, codes.download())
+
+
+@pytest.mark.parametrize("n,m,sd,k", [(600, 26, 32, 2), (4000, 26, 104, 2), (4000, 26, 100, 2), (5100, 26, 64, 256)])
+def test_blocks_whose_only_change_is_an_undecided_pair(ctx, n, m, sd, k):
+    """The same rows in every column block: in the second pass one row changes its cluster, by a margin of 2e-5 that only the
+    check of two candidates decides, in all blocks at once.  No block has converged before the third pass."""
+    far = k - 2
+    h, nb = (n - far) // 2, n - far - (n - far) // 2
+    v = np.zeros(n)
+    v[1:h], v[h:n - far - 1] = 0.02, 1.0
+    # the row is nearer to the second cluster's first centre, and 2.5e-6 below the middle of the two means
+    v[n - far - 1] = ((v[:h].mean() + (nb - 1) / nb) / 2 - 2.5e-6) / (1 - 0.5 / nb)
+    x = np.zeros((n, m, sd), F)
+    x[:, :, 0] = v.astype(F)[:, None]
+    for j in range(far):  # clusters of one row each
+        x[n - far + j, :, 1 + j % (sd - 1)] = (4.0 + j // (2 * (sd - 1))) * (-1) ** (j // (sd - 1))
+    x = x.reshape(n, m * sd)
+    init = np.tile(np.concatenate([[0, h], np.arange(n - far, n)]).astype(np.uint32), (m, 1))
+    reseed = np.zeros((m, 6 * k), np.uint32)
+    dcb = ctx.empty((m, k, sd), F)
+    iters, used = ctx.lbg_fit(ctx.to_device(x), n, m * sd, m, sd, k, 6, init, reseed, dcb)
+    want = O.pq_fit(x, m, k, 6, init, reseed)
+    assert np.all(want["iters"] == 3)
+    assert np.array_equal(iters, want["iters"]) and np.array_equal(used, want["reseeds"])
+    assert np.array_equal(dcb.download().view(np.uint32), want["codebooks"].view(np.uint32))

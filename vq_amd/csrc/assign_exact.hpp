@@ -46,12 +46,17 @@ __device__ __forceinline__ bool block_done(const AssignArgs &a, int s) {
     return a.before ? a.before[s] == 0 : a.done[s] != 0;
 }
 
-// Called by the lanes of a wave that changed a code.  Every store to one address is serialised
+// Called by the lanes of a wave that changed a code of one column block (the same flag for all).  Every store to one address is serialised
 // in its L2 channel and a million rows may change in a pass, so one lane of the wave stores, and
 // only when it still reads 0 (a stale 0 from the vector cache costs a store, nothing else).
 __device__ __forceinline__ void mark_changed(int *flag) {
     const unsigned long long active = __ballot(1);
     if ((int)__lane_id() == __ffsll(active) - 1 && *flag == 0) *flag = 1;
+}
+
+// The same for lanes of different column blocks, each with its own block's flag.
+__device__ __forceinline__ void mark_each_changed(int *flag) {
+    if (*flag == 0) *flag = 1;
 }
 
 // sqrt(sum of squares) of every centroid, sequential order (map_sum, src/distances.rs:66-69,144)
@@ -867,7 +872,7 @@ __device__ __forceinline__ void wide_pair_blocks(const AssignArgs &a, int sd, co
                 uint8_t *p = a.codes + (size_t)s * a.n + row;
                 if (*p != (uint8_t)best) {
                     *p = (uint8_t)best;
-                    mark_changed(a.changed + s);
+                    mark_each_changed(a.changed + s);
                 }
             } else {
                 a.codes[row * a.m + s] = (uint8_t)best;

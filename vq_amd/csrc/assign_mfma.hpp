@@ -1968,7 +1968,7 @@ template <bool LBG> __device__ __forceinline__ void store_code(const AssignArgs 
         uint8_t *p = a.codes + (size_t)s * a.n + row;
         if (*p != (uint8_t)code) {
             *p = (uint8_t)code;
-            mark_changed(a.changed + s);
+            mark_each_changed(a.changed + s);
         }
     } else {
         a.codes[row * a.m + s] = (uint8_t)code;
