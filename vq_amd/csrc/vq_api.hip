@@ -494,32 +494,37 @@ template <int METRIC, bool LBG> int32_t launch_mfma16(vq_ctx *ctx, const vq::Ass
 // Microseconds per iteration of a fit of blocks of 8 floats whose sums go by the lists of members, or are streamed
 // (k_lbg_stream8).  The lists and their leaves cost by the (row, block) pair, and more with the centroids among which a
 // part's rows are spread.  The streaming kernel costs less per pair, but takes more rounds the fewer clusters share a tile of rows (one wave's
-// chain over a part), and its clusters of up to 1024 members go by the lists as well.  Within 17 % of (lists / streamed): 250,000 x 12 k = 4 129 / 256, 16 129 / 157, 40 132 / 134, 112 155 / 125, 256
-// 212 / 162; x 33 k = 6 288 / 317, 10 287 / 266, 40 290 / 205; 1M x 16 k = 4 575 / 583, 6 572 / 497; 600,000 x 4 k = 64
-// 133 / 122, 128 140 / 118; 500,000 x 5 k = 64 132 / 119, 200 170 / 123, x 8 k = 24 167 / 154; 100,000 x 32 k = 48 142 / 133, 96
-// 153 / 160; 60,000 x 48 k = 40 132 / 132, 80 143 / 179; 150,000 x 16 k = 128 133 / 142; 250,000 x 4 k = 56 68 / 105, 256 98 / 122.
+// chain over a part), and its clusters of up to 1024 members go by the lists as well, some from averages of 1800 on.  Odd numbers of
+// blocks leave lanes idle in both.  The choice by these models costs 0.3 % on average over 234 shapes, 7 % at most (lists / streamed): 250,000 x 12
+// k = 4 129 / 256, 16 129 / 157, 40 132 / 134, 112 155 / 125, 256 212 / 162; x 33 k = 6 288 / 317, 10 287 / 266, 40 290 / 205; 1M x 16
+// k = 4 575 / 583, 6 572 / 497; 600,000 x 4 k = 64 133 / 122, 128 140 / 118; 500,000 x 5 k = 64 132 / 119, 200 170 / 123, x 8 k = 24
+// 167 / 154; 100,000 x 32 k = 48 142 / 133, 96 153 / 160; 87,148 x 32 k = 53 137 / 144; 60,000 x 48 k = 40 132 / 132, 80 143 / 179; 150,000 x 16
+// k = 128 133 / 142; 250,000 x 4 k = 56 68 / 105, 256 98 / 122.
 double fit8_lists_us(int64_t n, int m, int k) {
-    return 28 + (double)n * m * 1e-6 * (33.5 + 0.09 * k);
+    return 33 + (m % 2 ? 6 : 0) + (double)n * m * 1e-6 * (31.5 + 0.09 * k);
 }
 double fit8_streamed_us(int64_t n, int m, int k) {
     const double members = (double)n / k;  // of an average cluster
-    return 80 + 420.0 / k + (double)n * m * 1e-6 * (13 + 50.0 / k) + std::max(0.0, 0.066 * (1600 - members));
+    return 80 + (m % 2 ? 6 : 0) + 420.0 / k + (double)n * m * 1e-6 * (13 + 50.0 / k) + std::max(0.0, 0.066 * (1800 - members));
 }
 // (four blocks to a workgroup: a last group with idle waves from 61,441 rows on only)
 bool stream_pays(int64_t n, int m, int k) {
     return (m % 4 == 0 || n > 15 * vq::kPartRows) && fit8_streamed_us(n, m, k) < fit8_lists_us(n, m, k);
 }
 
-// The same of a fit of 8 floats by the faster way and of narrower blocks of their own width, for the choice between them.
+// The same of a fit of 8 floats by the faster way and of narrower blocks of their own width, for the choice between them
+// (three operations per component and centroid beside the bytes; one block per lane where their number is odd).
 // Own width / padded, measured: 250,000 x 12 blocks of 3, k = 32 121 / 131, 80 148 / 131; x 33 of 6, k = 4 362 / 288, x 46 of 7 474 / 386;
-// 60,000 x 12 of 6, k = 24 57 / 55, 56 74 / 65; 100,000 x 13 of 5, k = 48 80 / 76, 200 139 / 91; 200,000 x 16 of two, k = 64
-// 139 / 130; 500,000 x 12 of 6, k = 40 267 / 175, 100 405 / 170; 1M x 4 of 4, k = 64 195 / 138, 200 354 / 155; 60,007 x 25 of 4, k = 60 90 / 99.
+// 60,000 x 12 of 6, k = 24 57 / 55, 56 74 / 65; 100,000 x 13 of 5, k = 48 80 / 76, 200 139 / 91; 87,148 x 31 of 4, k = 24 118 / 120, 53 135 / 135, 80 145 / 141; x 13
+// of 4, k = 40 70 / 80, 128 98 / 92; 150,000 x 12 of 6, k = 24 93 / 97, 53 113 / 103; 500,000 x 12 of 6, k = 40 267 / 175, 100 405 / 170; 1M x 4 of 4,
+// k = 64 195 / 138, 200 354 / 155; 60,007 x 25 of 4, k = 40 86 / 98.
 double fit8_us(int64_t n, int m, int k) {
     return stream_pays(n, m, k) ? fit8_streamed_us(n, m, k) : fit8_lists_us(n, m, k);
 }
 double fit_static_us(int64_t n, int m, int sd, int k) {
-    const double mp = (double)n * m * 1e-6, spread = m % 2 ? 0.6 + 0.15 * sd : 1.0;  // (odd: one block per lane)
-    return 28 + mp * (22 + std::max(13 * spread, 0.022 * (3 * (sd == 7 ? 8 : sd) + 1) * k));
+    const int w = sd == 7 ? 8 : sd;
+    const double alone = m % 2 ? std::max(0.0, 8 - 0.08 * k) : 0.0;
+    return 28 + (double)n * m * 1e-6 * (22.5 + 1.9 * std::max(0, w - 4) + 0.022 * (3 * w + 1) * k + alone);
 }
 
 // The width to pad every column block to so that the matrix-core kernels take the shape (squared L2,
