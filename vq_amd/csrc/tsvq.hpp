@@ -1729,8 +1729,9 @@ __device__ __forceinline__ void quad_pair(const quad_piece (&xr)[NP], float &sl,
 }
 
 // tab: the table of k_tsvq_wtable with sctab, of ntab nodes, or the centroids themselves (Manhattan); ntop: the nodes of it in
-// LDS.  OUT: the leaves' centroids into out16 as well, for a few rows: an instance of its own with registers for the loads of 16 rows
-// (a row's load behind the store of the one before was 2 to 4 us of a call; with four rows' loads in the common instance it spills).
+// LDS.  OUT: the leaves' centroids into out16 as well, for a few rows: an instance of its own, as the common one has no registers for the loads of
+// R rows (a row's load behind the store of the one before was 2 to 4 us of a call; 16 rows' loads are 1 us faster than four for 16 rows
+// and more, and as much slower for one to three; above 208 components they spill).
 template <int METRIC, int NP, bool OUT>
 __global__ void __launch_bounds__(512, OUT ? 2 : 2 * quad_per_cu(NP)) k_tsvq_descend_quad(const float *__restrict__ x, int64_t n, int64_t ld, int dim,
                                                            const float *__restrict__ cen,
@@ -1740,7 +1741,7 @@ __global__ void __launch_bounds__(512, OUT ? 2 : 2 * quad_per_cu(NP)) k_tsvq_des
                                                            const float *__restrict__ tab,
                                                            const float *__restrict__ sctab, int ntop, int ntab,
                                                            int *__restrict__ leaf, uint16_t *__restrict__ out16) {
-    constexpr int S = quad_stride(NP);
+    constexpr int S = quad_stride(NP), R = 4;
     constexpr bool COS = METRIC == M_COS, L1 = METRIC == M_L1;
     extern __shared__ float4 lds_quad[];  // [ntop][S] the nodes, [2 ntop] their children, [2 ntop] their scalars
     float *top = reinterpret_cast<float *>(lds_quad);
@@ -1891,19 +1892,20 @@ __global__ void __launch_bounds__(512, OUT ? 2 : 2 * quad_per_cu(NP)) k_tsvq_des
             }
         }
         if (q == 0 && row < n) leaf[row] = node;
-        if constexpr (OUT) {  // a row at a time by the whole wave: runs of 128 bytes, also into host memory; all rows' loads in flight
-            const float *c[16];
+        if constexpr (OUT)  // a row at a time by the whole wave: runs of 128 bytes, also into host memory; the loads of R rows in flight
+            for (int i0 = 0; i0 < 16 && batch * 16 + i0 < n; i0 += R) {
+                const float *c[R];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) c[i] = cen + (size_t)__builtin_amdgcn_readlane(node, 4 * i) * dim;
-            for (int t = threadIdx.x & 63; t < dim; t += 64) {
-                float v[16];
+                for (int i = 0; i < R; ++i) c[i] = cen + (size_t)__builtin_amdgcn_readlane(node, 4 * (i0 + i)) * dim;
+                for (int t = threadIdx.x & 63; t < dim; t += 64) {
+                    float v[R];
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[i] = c[i][t];
+                    for (int i = 0; i < R; ++i) v[i] = c[i][t];
 #pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    if (batch * 16 + i < n) out16[(batch * 16 + i) * dim + t] = __half_as_ushort(__float2half_rn(v[i]));
+                    for (int i = 0; i < R; ++i)
+                        if (batch * 16 + i0 + i < n) out16[(batch * 16 + i0 + i) * dim + t] = __half_as_ushort(__float2half_rn(v[i]));
+                }
             }
-        }
     }  // batches
 }
 
