@@ -69,3 +69,42 @@ def test_tree_decode(ctx, dim):
     ctx.tsvq_decode_f16(tree, ctx.to_device(leaf), 2047, out)
     got = out.download()
     assert np.array_equal(got[:2047], cen[leaf].astype(np.float16).view(np.uint16)) and (got[2047] == 0x5555).all()
+
+
+@pytest.mark.parametrize("off", [0, 2, 8])
+@pytest.mark.parametrize("n,m,sd,k", [
+    # read from memory: units of one, two and four components, ends inside a thread's and a workgroup's share
+    (1, 1, 1, 1), (1023, 3, 7, 40), (1500, 2, 6, 300), (2049, 5, 12, 300), (90_001, 3, 5, 2000), (300_001, 3, 2, 30_000),
+    # the table in LDS: two codes per eight components or more, narrow blocks, whole and short last pieces, 160 KB
+    (2_600_003, 1, 1, 256), (650_001, 2, 2, 256), (280_001, 3, 3, 200), (200_003, 7, 4, 256), (180_001, 3, 5, 300), (160_001, 3, 6, 256),
+    (120_007, 3, 7, 256), (46_003, 11, 5, 1024), (70_001, 4, 9, 2000), (60_001, 7, 12, 256), (9_001, 7, 45, 30), (66_001, 8, 10, 1024)])
+def test_decode_any_width(ctx, n, m, sd, k, off):
+    rng = np.random.default_rng(n + sd)
+    cb = (rng.standard_normal((m, k, sd)) * 100).astype(F)
+    codes = rng.integers(0, k, (n, m), dtype=np.uint16)
+    want = cb[np.arange(m)[None, :], codes].reshape(-1).astype(np.float16).view(np.uint16)
+    out = ctx.to_device(np.full(n * m * sd + 16, 0x5555, np.uint16))
+
+    class Part:
+        ptr = out.ptr + off
+    if k > 256:
+        ctx.decode_f16_u16(ctx.to_device(codes), n, m, sd, k, ctx.to_device(cb), Part())
+    else:
+        ctx.decode_f16(ctx.to_device(codes.astype(np.uint8)), n, m, sd, k, ctx.to_device(cb), Part())
+    got = out.download()
+    assert np.array_equal(got[off // 2:off // 2 + len(want)], want)
+    assert (got[:off // 2] == 0x5555).all() and (got[off // 2 + len(want):] == 0x5555).all()
+
+
+def test_tree_decode_from_a_table(ctx):
+    """More leaves than a tree's table in LDS needs to pay, widths of every unit."""
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((4000, 50)).astype(F)
+    for dim, n in ((50, 60_001), (44, 120_001), (25, 110_003)):
+        tree = ctx.tsvq_build(ctx.to_device(np.ascontiguousarray(x[:, :dim])), 4000, dim, dim, 4)
+        cen = tree.download()["centroids"]
+        leaf = rng.integers(0, len(cen), n).astype(np.int32)
+        out = ctx.to_device(np.full((n + 1, dim), 0x5555, np.uint16))
+        ctx.tsvq_decode_f16(tree, ctx.to_device(leaf), n, out)
+        got = out.download()
+        assert np.array_equal(got[:n], cen[leaf].astype(np.float16).view(np.uint16)) and (got[n] == 0x5555).all()

@@ -40,6 +40,20 @@ inline int decode_resident_blocks(bool f16, int64_t n, int m, int sd, int k) {
     return (int)G;
 }
 
+// Whether binary16 rows of blocks that fill no 16-byte pieces are made from a table in LDS (k_decode_flat; else
+// k_decode_units): the table is filled once per workgroup, so from 64 values of the output per value of the table on, and from
+// sizes on where a launch is not most of the time.  Alone, units -> table: 372,160 x 21 blocks of 15, k = 33 147 -> 59 us (4.0 TB/s),
+// 755,499 x 8 of 7, k = 216 59 -> 25, 322,755 x 49 of 7, k = 227 (156 KB) 156 -> 67, 122,321 x 55 of 2, k = 189 23.5 -> 10.5, 300,000 x 10 of 12,
+// k = 256 22 -> 17, x 16 of 4 18.8 -> 9.4, 20,000 x 60 of 5, k = 256 (79 values per value) 12.3 -> 11.5, 6,000 x 30 of 15, k = 30 6.4 -> 6.0;
+// below the lines 6,404 x 17 of 7, k = 98 4.9 -> 6.1, 20,000 x 16 of 6, k = 256 5.1 -> 5.9, 8,000 x 50 of 3, k = 256 5.2 -> 7.7.
+constexpr int kDecodeFlatLds = 160 * 1024;  // the largest table, bytes
+inline bool decode_flat_resident(int64_t n, int64_t m, int64_t sd, int64_t k) {
+    constexpr int64_t most = kDecodeFlatLds / 2;
+    if (m > most || sd > most || m * sd * k > most) return false;
+    const int64_t total = n * m * sd;
+    return total >= (sd % 4 == 0 ? 5'000'000 : 2'500'000) && total >= 64 * (m * sd * k);
+}
+
 // Columns per group of k_rvq_recon_resident; 0: the gather.  The stages' table within 128 KB, 32 columns or more, or 16.
 // Where groups share rows that are not whole halves of lines, from four stages on: gather -> resident of 256 centroids
 // 200,000 x 72, two stages 14.9 -> 15.0 us, 400,000 33.6 -> 42.8, 400,000 x 104 38 -> 50; four stages 200,000 x 136 39 -> 31, 400,000 60 -> 63,

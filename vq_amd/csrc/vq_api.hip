@@ -611,39 +611,7 @@ int32_t launch_assign(vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, 
     return fail(ctx, VQ_ERR_UNSUPPORTED, "metric %d has no kernel", metric);
 }
 
-template <typename CodeT>
-__global__ void k_decode_f16(const CodeT *__restrict__ codes, int64_t n, int m, int sd, int k,
-                             const float *__restrict__ cb, uint16_t *__restrict__ out) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t dim = (int64_t)m * sd;
-    if (i >= n * dim) return;
-    int64_t row = i / dim;
-    int c = (int)(i % dim);
-    int s = c / sd, t = c % sd;
-    float v = cb[((size_t)s * k + codes[row * m + s]) * sd + t];
-    out[i] = __half_as_ushort(__float2half_rn(v));
-}
-
-// Four consecutive components per thread (sub_dim a multiple of 4, 16-byte aligned codebooks and
-// output rows): one 16-byte load of the centroid, one 8- or 16-byte store.  F16: binary16 bit
-// patterns (round to nearest even), else f32.
-template <typename CodeT>
-__global__ void __launch_bounds__(256) k_decode_vec4(const CodeT *__restrict__ codes, int64_t n, int m, int sd,
-                                                     int k, const float *__restrict__ cb, uint2 *__restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;  // group of four components
-    const int64_t dim4 = (int64_t)m * sd / 4;
-    if (i >= n * dim4) return;
-    const int64_t row = i / dim4;
-    const int c = (int)(i % dim4) * 4;
-    const int s = c / sd, t = c % sd;
-    const float4 v = *reinterpret_cast<const float4 *>(cb + ((size_t)s * k + codes[row * m + s]) * sd + t);
-    uint2 o;
-    o.x = (uint32_t)__half_as_ushort(__float2half_rn(v.x)) | ((uint32_t)__half_as_ushort(__float2half_rn(v.y)) << 16);
-    o.y = (uint32_t)__half_as_ushort(__float2half_rn(v.z)) | ((uint32_t)__half_as_ushort(__float2half_rn(v.w)) << 16);
-    out[i] = o;
-}
-
-// The same gather with the codebook table resident in LDS (up to 128 KB, one workgroup of 1024 threads per
+// Reconstruction with the codebook table resident in LDS (up to 128 KB, one workgroup of 1024 threads per
 // compute unit walking over the output, two where the table leaves room): a thread makes one 16-byte piece of the
 // output per step, eight f16 values (F16; sub_dim a multiple of 8) or four f32 values (sub_dim a
 // multiple of 4), so a wave's stores are consecutive bytes, its code reads consecutive
@@ -703,18 +671,6 @@ __global__ void __launch_bounds__(1024) k_decode_resident(const CodeT *__restric
     }
 }
 
-template <typename CodeT>
-__global__ void k_decode_f32(const CodeT *__restrict__ codes, int64_t n, int m, int sd, int k,
-                             const float *__restrict__ cb, float *__restrict__ out) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t dim = (int64_t)m * sd;
-    if (i >= n * dim) return;
-    int64_t row = i / dim;
-    int c = (int)(i % dim);
-    int s = c / sd, t = c % sd;
-    out[i] = cb[((size_t)s * k + codes[row * m + s]) * sd + t];
-}
-
 __global__ void __launch_bounds__(256) k_copy_f32(const float4 *__restrict__ src,
                                                   float4 *__restrict__ dst, int64_t n4,
                                                   const float *__restrict__ src_tail,
@@ -772,16 +728,10 @@ int32_t decode_codes(vq_ctx *ctx, const CodeT *d_codes, int64_t n, int32_t m, in
     if (sd % piece == 0 && aligned && (int64_t)m * sd < (1LL << 31))
         hipLaunchKernelGGL((vq::k_decode_gather<F16, CodeT>), dim3(cdiv(n * m * (sd / piece), 1024)), dim3(256), 0,
                            ctx->stream, d_codes, n, m, sd, k, d_codebooks, (vq::u32x4_out *)d_out);
-    else if constexpr (F16) {
-        if (sd % 4 == 0 && aligned)
-            hipLaunchKernelGGL(k_decode_vec4<CodeT>, dim3(cdiv(n * m * sd / 4, 256)), dim3(256), 0, ctx->stream, d_codes, n,
-                               m, sd, k, d_codebooks, (uint2 *)d_out);
-        else
-            hipLaunchKernelGGL(k_decode_f16<CodeT>, dim3(cdiv(n * m * sd, 256)), dim3(256), 0, ctx->stream, d_codes, n, m,
-                               sd, k, d_codebooks, (uint16_t *)d_out);
-    } else
-        hipLaunchKernelGGL(k_decode_f32<CodeT>, dim3(cdiv(n * m * sd, 256)), dim3(256), 0, ctx->stream, d_codes, n, m,
-                           sd, k, d_codebooks, (float *)d_out);
+    else {
+        VQ_TRY(know_compute_units(ctx));
+        VQ_HIP(ctx, (vq::launch_decode_any<F16, CodeT>(ctx->stream, ctx->compute_units, d_codes, n, m, sd, k, d_codebooks, d_out)));
+    }
     VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;
 }

@@ -983,12 +983,11 @@ int32_t vq_tsvq_decode_f16(vq_ctx *ctx, const vq_tree *tree, const int32_t *d_le
     if (tree->dim % 8 == 0 && aligned)
         hipLaunchKernelGGL((vq::k_decode_gather<true, int32_t>), dim3(cdiv(n * (tree->dim / 8), 1024)), dim3(256), 0, ctx->stream,
                            d_leaf, n, 1, tree->dim, 0, tree->d_centroids, (vq::u32x4_out *)d_out);
-    else if (tree->dim % 4 == 0 && aligned)
-        hipLaunchKernelGGL(vq::k_tsvq_decode4_f16, dim3(cdiv(n * (tree->dim / 4), 256)), dim3(256), 0, ctx->stream,
-                           d_leaf, n, tree->dim, tree->d_centroids, reinterpret_cast<uint2 *>(d_out));
-    else
-        hipLaunchKernelGGL(vq::k_tsvq_decode_f16, dim3(cdiv(n * tree->dim, 256)), dim3(256), 0, ctx->stream, d_leaf,
-                           n, tree->dim, tree->d_centroids, d_out);
+    else {
+        VQ_TRY(know_compute_units(ctx));
+        VQ_HIP(ctx, (vq::launch_decode_any<true, int32_t>(ctx->stream, ctx->compute_units, d_leaf, n, 1, tree->dim, tree->n_nodes,
+                                                          tree->d_centroids, d_out)));
+    }
     VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;
 }
