@@ -1,0 +1,36 @@
+"""TSVQ levels built without the host between them (k_node_leafsum, k_node_stats, k_node_split): trees that are not
+balanced, so that nodes are longer than a launch expects (their keys in memory, their leaves summed in rounds), slots
+without a node, levels by the host above them, more levels than one table holds, few components; against the oracle."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests.test_gpu_tsvq import assert_same_tree, bfs_order
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import vq_amd
+    c = vq_amd.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("n,dim,depth,kind", [
+    (4096, 10, 6, "lopsided"), (8192, 100, 7, "lopsided"), (8000, 97, 5, "lopsided"), (3000, 3, 8, "normal"),
+    (20000, 8, 8, "lopsided"), (30000, 96, 7, "lopsided"), (700, 1, 10, "normal"), (40, 6, 13, "normal"), (2100, 4, 14, "lopsided"),
+    (6000, 17, 12, "copies"), (257, 20, 1, "normal"), (5, 2, 3, "copies"), (9000, 33, 9, "copies"),
+])
+def test_levels_on_device(ctx, n, dim, depth, kind):
+    rng = np.random.default_rng(17 * n + dim)
+    x = rng.standard_normal((n, dim)).astype(F)
+    if kind == "lopsided":  # every column: four rows of five share the least value, which is the median
+        x = np.where(rng.random((n, dim)) < 0.8, F(0.0), np.abs(x) * F(10) + F(1)).astype(F) * np.arange(1, dim + 1, dtype=F)
+    elif kind == "copies":  # few distinct rows: nodes of equal rows have no children
+        x = x[rng.integers(0, min(n, 9), n)]
+    got = ctx.tsvq_build(ctx.to_device(x), n, dim, dim, depth).download()
+    want, _ = bfs_order(O.tsvq_fit(x, depth))
+    assert_same_tree(got, want)

@@ -991,22 +991,17 @@ static __global__ void k_seg_median(const SegSelect *__restrict__ sel, const uin
 constexpr uint32_t kSplitWgMax = 16384;  // rows: 64 KB of keys
 inline size_t split_wg_lds(uint32_t longest) { return sizeof(uint32_t) * ((size_t)longest + 512 + 64); }
 
-static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__restrict__ perm,
-                                                              const uint2 *__restrict__ seg_range,
-                                                              const float *__restrict__ var, int dim, int stride,
-                                                              const float *__restrict__ x, int64_t ld,
-                                                              int *__restrict__ split_dim, float *__restrict__ median,
-                                                              uint32_t *__restrict__ nleft, uint32_t *__restrict__ perm_out) {
-    extern __shared__ uint32_t lds_split[];
-    uint32_t *hist = lds_split, *part = hist + 512, *key = part + 64;
-    const int g = blockIdx.x, tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
-    const uint2 r = seg_range[g];
+// One node of a workgroup: v its per-dimension sums, r its positions in perm, key room for its rows' keys (LDS or
+// memory).  Split dimension, median and left count through the pointers (thread 0).  Returns the left count.
+__device__ __forceinline__ uint32_t split_node(uint32_t *hist, uint32_t *part, uint32_t *key, const uint32_t *__restrict__ perm, const uint2 r,
+                                               const float *__restrict__ v, int dim, const float *__restrict__ x, int64_t ld,
+                                               int *split_dim, float *median, uint32_t *nleft, uint32_t *__restrict__ perm_out) {
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
     const uint32_t cnt = r.y - r.x;
     // The reference's scan keeps an index for which !(v[t] < best so far): the last of the largest values, and a
     // NaN or what follows one is always taken.  A run of values acts on what came before as its own result
     // does, unless it holds a NaN: then it decides alone; so runs compose in order, one per lane.
     if (wave == 0) {
-        const float *v = var + (size_t)g * stride;
         const int per = (dim + 63) / 64, t0 = lane * per, t1 = t0 + per < dim ? t0 + per : dim;
         int best = t0;
         float vb = t0 < dim ? v[t0] : 0.0f;
@@ -1032,7 +1027,7 @@ static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__
         }
         if (lane == 0) {
             part[0] = (uint32_t)best;
-            split_dim[g] = best;
+            *split_dim = best;
         }
     }
     for (int i = tid; i < 512; i += nt) hist[i] = 0u;
@@ -1100,8 +1095,8 @@ static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__
     uint32_t total = 0;
     for (int w = 0; w < nw; ++w) total += part[w];
     if (tid == 0) {
-        median[g] = med;
-        nleft[g] = total;
+        *median = med;
+        *nleft = total;
     }
     uint32_t before = 0;  // left rows of the stretches so far
     for (uint32_t base = 0; base < cnt; base += nt) {
@@ -1119,8 +1114,140 @@ static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__
         }
         if (in) perm_out[left ? r.x + mybefore : r.x + total + (p - mybefore)] = perm[r.x + p];
     }
+    return total;
 }
 
+static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__restrict__ perm,
+                                                              const uint2 *__restrict__ seg_range,
+                                                              const float *__restrict__ var, int dim, int stride,
+                                                              const float *__restrict__ x, int64_t ld,
+                                                              int *__restrict__ split_dim, float *__restrict__ median,
+                                                              uint32_t *__restrict__ nleft, uint32_t *__restrict__ perm_out) {
+    extern __shared__ uint32_t lds_split[];
+    const int g = blockIdx.x;
+    split_node(lds_split, lds_split + 512, lds_split + 576, perm, seg_range[g], var + (size_t)g * stride, dim, x, ld, split_dim + g,
+               median + g, nleft + g, perm_out);
+}
+
+// ---- levels of short nodes, without the host between them ------------------------------------
+// Where no node of a level is longer than var_tile_rows, the levels below it are built from tables on the device: the nodes of
+// level d are the slots of a complete tree (children of slot g: 2 g and 2 g + 1 of the next table), a slot without a node
+// is {0, 0}.  Every launch covers all slots of its level; the host reads the decisions of all levels at once and
+// numbers the nodes.  (A level that waits for the host costs two copies, the wait and the time until its first kernel
+// starts, 30 us on a level of 70-100, and its means were three launches where they are one or two.  Builds: 2,295 x 128, seven levels 391 -> 247 us,
+// 4,157 x 100, ten 614 -> 404, 12,557 x 96, six 507 -> 414, 100,000 x 128, ten 1284 -> 1171.)  The host knows no node's
+// size here, only the longest one's above: what a launch is sized for is the balanced tree's, and a longer node
+// (equal values all go left) takes more rounds of the same loops.
+constexpr int kNodeLeaves = 8;  // leaves of 1024 rows of the longest node
+
+// Rows lo .. hi - 1 (of cnt) of leaf l, by the midpoints of src/vector.rs's recursion.
+__device__ __forceinline__ uint2 leaf_range(uint32_t cnt, int dep, uint32_t l) {
+    uint32_t lo = 0, hi = cnt;
+    for (int bit = dep - 1; bit >= 0; --bit) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        if ((l >> bit) & 1u)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return make_uint2(lo, hi);
+}
+
+__device__ __forceinline__ int leaf_depth(uint32_t cnt) {
+    int dep = 0;
+    while (cnt > (1024u << dep)) ++dep;
+    return dep;
+}
+
+// Sums of the leaves of a level's nodes, a workgroup per (node, one of every `per` leaves, tile of up to 16 components, as
+// k_node_stats has them): leaf_sum[(node * kNodeLeaves + leaf) * dim + component].
+template <int VEC>
+static __global__ void __launch_bounds__(256) k_node_leafsum(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, int slots,
+                                                             int per, const float *__restrict__ x, int64_t ld, int dim, int width,
+                                                             int pieces, float *__restrict__ leaf_sum) {
+    extern __shared__ float4 lds_node[];
+    const int g = blockIdx.x % (unsigned)slots, rest = blockIdx.x / (unsigned)slots, tile = rest / per;
+    const int c0 = tile * width < dim - width ? tile * width : dim - width;
+    const uint2 r = range[g];
+    const uint32_t cnt = r.y - r.x;
+    const int dep = leaf_depth(cnt);
+    for (uint32_t l = (uint32_t)(rest % per); cnt && l < (1u << dep); l += (uint32_t)per) {
+        const uint2 lr = leaf_range(cnt, dep, l);
+        const float sum = member_tile_sum<256, VEC>(reinterpret_cast<float *>(lds_node), x + c0, ld, r.x + lr.x, r.x + lr.y, width, pieces,
+                                                    [&](uint32_t p) { return perm[p]; });
+        if ((int)threadIdx.x < width) leaf_sum[((size_t)g * kNodeLeaves + l) * dim + c0 + threadIdx.x] = sum;
+        __syncthreads();  // (the stage has been read)
+    }
+}
+
+// Means, and with var the sums of squared deviations, of a level's nodes: a workgroup per node and tile, as
+// k_seg_variance_tile.  SUMS: the leaves are summed here, one after the other (nodes of up to 1024 rows have one); else from leaf_sum.
+// NT threads: 64 for nodes of up to 256 rows, whose chunks of 128 members leave room for more workgroups (the last levels
+// of 100,000 x 128, nodes of 195 and 98 rows: 23 -> 15 us each).
+template <int VEC, bool SUMS, int NT>
+static __global__ void __launch_bounds__(NT) k_node_stats(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, int slots,
+                                                           const float *__restrict__ x, int64_t ld, int dim, int width, int pieces,
+                                                           const float *__restrict__ leaf_sum, float *__restrict__ means,
+                                                           float *__restrict__ var) {
+    extern __shared__ float4 lds_node[];
+    __shared__ float leaf[kNodeLeaves][16];
+    float *stage = reinterpret_cast<float *>(lds_node);
+    const int g = blockIdx.x % (unsigned)slots, tile = blockIdx.x / (unsigned)slots, tid = threadIdx.x;
+    const int c0 = tile * width < dim - width ? tile * width : dim - width;
+    const uint2 r = range[g];
+    const uint32_t cnt = r.y - r.x;
+    if (cnt == 0) return;
+    const int dep = leaf_depth(cnt);
+    const uint32_t nl = 1u << dep;
+    for (uint32_t l = 0; l < nl; ++l) {
+        if constexpr (SUMS) {
+            const uint2 lr = leaf_range(cnt, dep, l);
+            const float sum = member_tile_sum<NT, VEC>(stage, x + c0, ld, r.x + lr.x, r.x + lr.y, width, pieces,
+                                                        [&](uint32_t p) { return perm[p]; });
+            if (tid < width) leaf[l][tid] = sum;
+            __syncthreads();  // (the stage has been read)
+        } else if (tid < width) {
+            leaf[l][tid] = leaf_sum[((size_t)g * kNodeLeaves + l) * dim + c0 + tid];
+        }
+    }
+    if (tid < width) {  // (a lane reads what it wrote itself)
+        for (uint32_t h = 1; h < nl; h <<= 1)
+            for (uint32_t q = 0; q < nl; q += 2 * h) leaf[q][tid] = leaf[q][tid] + leaf[q + h][tid];
+        leaf[0][tid] = leaf[0][tid] / __uint2float_rn(cnt);
+        means[(size_t)g * dim + c0 + tid] = leaf[0][tid];
+    }
+    if (!var || cnt < 2) return;
+    __syncthreads();
+    const float sum = member_tile_sum<NT, VEC, true>(stage, x + c0, ld, r.x, r.y, width, pieces, [&](uint32_t p) { return perm[p]; }, leaf[0]);
+    if (tid < width) var[(size_t)g * dim + c0 + tid] = sum;
+}
+
+// k_seg_split_wg for the slots of a level; the children's positions go into the next level's table.  room: rows whose keys the
+// workgroup's LDS holds; a longer node's keys lie in memory (keys, by position).  nleft stays 0 where nothing is split.
+static __global__ void __launch_bounds__(1024) k_node_split(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, uint32_t room,
+                                                            const float *__restrict__ var, int dim, int stride,
+                                                            const float *__restrict__ x, int64_t ld, uint32_t *__restrict__ keys,
+                                                            int *__restrict__ split_dim, float *__restrict__ median,
+                                                            uint32_t *__restrict__ nleft, uint32_t *__restrict__ perm_out,
+                                                            uint2 *__restrict__ child) {
+    extern __shared__ uint32_t lds_split[];
+    uint32_t *hist = lds_split, *part = hist + 512;
+    const int g = blockIdx.x;
+    const uint2 r = range[g];
+    const uint32_t cnt = r.y - r.x;
+    uint32_t nl = 0;
+    const float *v = var + (size_t)g * stride;
+    if (cnt >= 2 && cnt <= room)
+        nl = split_node(hist, part, part + 64, perm, r, v, dim, x, ld, split_dim + g, median + g, nleft + g, perm_out);
+    else if (cnt >= 2)
+        nl = split_node(hist, part, keys + r.x, perm, r, v, dim, x, ld, split_dim + g, median + g, nleft + g, perm_out);
+    if (threadIdx.x == 0) {
+        const bool both = nl > 0 && nl < cnt;  // (no child holds all rows)
+        if (cnt < 2) nleft[g] = 0u;
+        child[2 * g] = both ? make_uint2(r.x, r.x + nl) : make_uint2(0u, 0u);
+        child[2 * g + 1] = both ? make_uint2(r.x + nl, r.y) : make_uint2(0u, 0u);
+    }
+}
 
 // out[i][t] = means[idx[i]][t]: the means of the nodes that split, side by side
 static __global__ void __launch_bounds__(256) k_gather_means(const float *__restrict__ means,

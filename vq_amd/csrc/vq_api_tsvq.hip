@@ -359,7 +359,149 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     };
     auto pad = [](size_t z) { return (z + 255) & ~(size_t)255; };
 
+    // The columns of a workgroup of the kernels that take a node's rows by tiles.
+    const int tiles = (int)cdiv(dim, 16), width = tiles == 1 ? dim : (int)cdiv(cdiv(dim, tiles), 4) * 4;
+    const int vec = dim >= 4 ? 4 : 1, pieces = (int)cdiv(width, vec), wtiles = (int)cdiv(dim, width);
+    const auto tile_lds = [&](int threads) { return sizeof(float) * (size_t)width * (8 * (threads / pieces) + 4); };
+    // Levels of short nodes without the host between them (k_node_stats, k_node_split): as many as their tables
+    // take at once, then the host numbers the nodes.  Sets done, or leaves level and depth_left at the first level not built.
+    auto device_levels = [&](bool &ran, bool &done) -> int32_t {
+        const int nseg = (int)level.size(), first_node = level[0].node;
+        uint32_t longest = 0;
+        for (const Seg &sg : level) longest = std::max(longest, sg.hi - sg.lo);
+        if (km || ctx->tsvq_var_path != 0 || !means_arena || depth_left < 1 || longest < 2 || longest > var_tile_rows(dim)) return VQ_OK;
+        // the slots of the last level, and what they take
+        const int64_t most = std::max<int64_t>(4096, 4 * (int64_t)nseg);
+        int D = 0;
+        while (D < depth_left && ((int64_t)nseg << (D + 1)) <= most && ((int64_t)nseg << (D + 2)) * dim <= (16 << 20)) ++D;
+        if (D < std::min(depth_left, 2)) return VQ_OK;
+        const size_t last = (size_t)nseg << D, inner = last - nseg, slots = inner + last;  // (nseg (2^D - 1), and with the last level's)
+        int leafy = 0;  // levels whose leaves are summed ahead
+        while (leafy <= D && (longest >> leafy) > (uint32_t)kLeafMaxRows) ++leafy;
+        const bool direct = (uint64_t)first_node + slots <= max_nodes;  // (slots without a node may exceed the arena)
+        const size_t sizes[5] = {sizeof(uint2) * slots, 3 * sizeof(uint32_t) * inner, sizeof(float) * (inner ? last / 2 : 0) * dim,
+                                 leafy ? sizeof(float) * vq::kNodeLeaves * ((size_t)nseg << (leafy - 1)) * dim : 0,
+                                 direct ? 0 : sizeof(float) * slots * dim};
+        size_t total = 0;
+        for (size_t z : sizes) total += pad(z);
+        VQ_TRY(ensure(ctx, ctx->tsvq_level, total));
+        VQ_TRY(pinned(std::max(sizes[1], sizeof(uint2) * (size_t)nseg)));
+        char *at[5], *p = (char *)ctx->tsvq_level.p;
+        for (int z = 0; z < 5; ++z) {
+            at[z] = p;
+            p += pad(sizes[z]);
+        }
+        uint2 *d_range = (uint2 *)at[0], *h_range = (uint2 *)ctx->tsvq_pin;
+        int *d_sdim = (int *)at[1];
+        float *d_median = (float *)d_sdim + inner, *d_var = (float *)at[2], *d_lsum = (float *)at[3];
+        uint32_t *d_nleft = (uint32_t *)d_sdim + 2 * inner;
+        float *d_means = direct ? (float *)ctx->tsvq_means.p + (size_t)first_node * dim : (float *)at[4];
+        for (int g = 0; g < nseg; ++g) h_range[g] = make_uint2(level[g].lo, level[g].hi);
+        VQ_HIP(ctx, hipMemcpyAsync(d_range, h_range, sizeof(uint2) * (size_t)nseg, hipMemcpyHostToDevice, st));
+        for (int d = 0; d <= D; ++d) {
+            if (d == D && D < depth_left) break;  // the next call's first level
+            const size_t o = ((size_t)nseg << d) - nseg;
+            const int ns = nseg << d;
+            const uint32_t usual = std::max(longest >> d, 1u);
+            const uint2 *r = d_range + o;
+            float *means = d_means + o * dim, *var = d < D ? d_var : nullptr;
+            const dim3 grid((unsigned)((int64_t)ns * wtiles)), block(256);
+            if (d < leafy) {
+                const int per = 1 << tree_depth(usual);
+                hipLaunchKernelGGL(vec == 4 ? vq::k_node_leafsum<4> : vq::k_node_leafsum<1>, dim3((unsigned)((int64_t)ns * wtiles * per)), block,
+                                   tile_lds(256), st, perm, r, ns, per, d_x, ld, dim, width, pieces, d_lsum);
+                hipLaunchKernelGGL((vec == 4 ? vq::k_node_stats<4, false, 256> : vq::k_node_stats<1, false, 256>), grid, block, tile_lds(256), st, perm, r, ns,
+                                   d_x, ld, dim, width, pieces, (const float *)d_lsum, means, var);
+            } else {
+                const bool wave = usual <= 256;
+                hipLaunchKernelGGL((vec == 4 ? (wave ? vq::k_node_stats<4, true, 64> : vq::k_node_stats<4, true, 256>)
+                                             : (wave ? vq::k_node_stats<1, true, 64> : vq::k_node_stats<1, true, 256>)),
+                                   grid, dim3(wave ? 64 : 256), tile_lds(wave ? 64 : 256), st, perm, r, ns, d_x, ld, dim, width, pieces,
+                                   (const float *)nullptr, means, var);
+            }
+            if (d == D) break;
+            const uint32_t room = std::min(longest, usual + usual / 8 + 64);
+            hipLaunchKernelGGL(vq::k_node_split, dim3((unsigned)ns), dim3(usual > 1024 ? 1024u : 256u), vq::split_wg_lds(room), st, perm, r, room,
+                               (const float *)d_var, real_dim, dim, d_x, ld, (uint32_t *)vals, d_sdim + o, d_median + o, d_nleft + o, perm2,
+                               d_range + o + ns);
+            std::swap(perm, perm2);
+        }
+        VQ_HIP(ctx, hipGetLastError());
+        VQ_HIP(ctx, hipMemcpyAsync(ctx->tsvq_pin, d_sdim, sizes[1], hipMemcpyDeviceToHost, st));
+        VQ_HIP(ctx, hipStreamSynchronize(st));
+        const int *sdim = (const int *)ctx->tsvq_pin;
+        const float *median = (const float *)sdim + inner;
+        const uint32_t *nleft = (const uint32_t *)sdim + 2 * inner;
+        // the nodes, level by level, as the loop below numbers them (src/tsvq.rs:126-141)
+        std::vector<uint32_t> slot(nseg), from;  // of the level's nodes; of all nodes with means, in node order
+        for (int g = 0; g < nseg; ++g) slot[g] = (uint32_t)g;
+        for (int d = 0;; ++d) {
+            const size_t o = ((size_t)nseg << d) - nseg;
+            if (d < D || D == depth_left)
+                for (uint32_t g : slot) from.push_back((uint32_t)o + g);
+            if (d == D) break;
+            std::vector<Seg> next;
+            std::vector<uint32_t> next_slot;
+            for (size_t i = 0; i < level.size(); ++i) {
+                const Seg sg = level[i];
+                const uint32_t cnt = sg.hi - sg.lo;
+                if (cnt < 2) continue;
+                const size_t q = o + slot[i];
+                const uint32_t nl = nleft[q];
+                T->h_split_dim[sg.node] = sdim[q];
+                T->h_split_val[sg.node] = median[q];
+                if (nl == 0 || nl >= cnt) continue;
+                for (int side = 0; side < 2; ++side) {
+                    const uint32_t lo = side ? sg.lo + nl : sg.lo, hi = side ? sg.hi : sg.lo + nl;
+                    const int32_t id = (int32_t)T->h_left.size();
+                    (side ? T->h_right : T->h_left)[sg.node] = id;
+                    T->h_left.push_back(-1);
+                    T->h_right.push_back(-1);
+                    T->h_split_dim.push_back(-1);
+                    T->h_split_val.push_back(0.f);
+                    T->h_count.push_back((int64_t)hi - lo);
+                    next.push_back({id, lo, hi, 2 * sg.heap + (uint64_t)side});
+                    next_slot.push_back(2 * slot[i] + (uint32_t)side);
+                }
+            }
+            level.swap(next);
+            slot.swap(next_slot);
+            if (level.empty()) break;
+        }
+        // means of slots without gaps are where the nodes' means belong
+        if (!direct || from.back() + 1 != from.size()) {
+            const size_t cnt = from.size();
+            VQ_TRY(ensure(ctx, ctx->tsvq_split, pad(sizeof(float) * cnt * dim) + sizeof(uint32_t) * cnt));
+            VQ_TRY(pinned(sizeof(uint32_t) * cnt));
+            float *packed = (float *)ctx->tsvq_split.p;
+            int *d_from = (int *)((char *)packed + pad(sizeof(float) * cnt * dim));
+            memcpy(ctx->tsvq_pin, from.data(), sizeof(uint32_t) * cnt);
+            VQ_HIP(ctx, hipMemcpyAsync(d_from, ctx->tsvq_pin, sizeof(uint32_t) * cnt, hipMemcpyHostToDevice, st));
+            hipLaunchKernelGGL(vq::k_gather_means, dim3(cdiv((int64_t)cnt * dim, 256)), dim3(256), 0, st, (const float *)d_means,
+                               (const int *)d_from, (int)cnt, dim, packed);
+            VQ_HIP(ctx, hipGetLastError());
+            VQ_HIP(ctx, hipMemcpyAsync((float *)ctx->tsvq_means.p + (size_t)first_node * dim, packed, sizeof(float) * cnt * dim,
+                                       hipMemcpyDeviceToDevice, st));
+            VQ_HIP(ctx, hipStreamSynchronize(st));  // (the page-locked memory is free again)
+        }
+        level_means.push_back({(float *)ctx->tsvq_means.p + (size_t)first_node * dim, first_node, (int)from.size()});
+        ran = true;
+        done = level.empty() || D == depth_left;
+        depth_left -= D;
+        return VQ_OK;
+    };
+
     while (!level.empty()) {
+        {
+            bool ran = false, done = false;
+            const int32_t rc = device_levels(ran, done);
+            if (rc != VQ_OK) {
+                free_means();
+                return cleanup_fail(rc);
+            }
+            if (done) break;
+            if (ran) continue;
+        }
         const int nseg = (int)level.size();
         // ---- means of every node of the level ------------------------------------------------
         desc.clear();  // (both outlive the level: their uploads are enqueued, not waited for)
@@ -659,10 +801,8 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                                    (const float *)d_sq, (const uint2 *)d_range, dim, (float *)d_var);
             }
         } else {
-            const int tiles = (int)cdiv(dim, 16), width = tiles == 1 ? dim : (int)cdiv(cdiv(dim, tiles), 4) * 4;
-            const int vec = dim >= 4 ? 4 : 1, pieces = (int)cdiv(width, vec);
-            hipLaunchKernelGGL(vec == 4 ? vq::k_seg_variance_tile<4> : vq::k_seg_variance_tile<1>, dim3((unsigned)((int64_t)ns * cdiv(dim, width))), dim3(256),
-                               sizeof(float) * (size_t)width * (8 * (256 / pieces) + 4), st, perm, (const uint2 *)d_range, ns, (const float *)d_smeans,
+            hipLaunchKernelGGL(vec == 4 ? vq::k_seg_variance_tile<4> : vq::k_seg_variance_tile<1>, dim3((unsigned)((int64_t)ns * wtiles)), dim3(256),
+                               tile_lds(256), st, perm, (const uint2 *)d_range, ns, (const float *)d_smeans,
                                (int64_t)0, d_x, ld, dim, width, pieces, (float *)d_var);
         }
         SP_HIP(hipGetLastError());
