@@ -159,9 +159,10 @@ static __global__ void __launch_bounds__(256) k_seg_mean_wg(const float *__restr
 
 // Sums of squared deviations in row order, a workgroup per segment and tile of up to 16 components (block
 // tile * nseg + segment, as y would end at 65,535 tiles; the last tile begins at dim less its width): seg_range[g] = {lo, hi} positions in perm; mean of segment g at means[(first + g) * dim].
-// A chunk of 512 rows is a memory round trip, two barriers and their adds, 3.5 us in all: 7 ns a row.  Against one workgroup per segment with all
+// A chunk of 512 rows was a memory round trip, two barriers and their adds, 3.5 us in all or 7 ns a row; 4 ns where the chunks overlap the adds (CHAIN).  Against one workgroup per segment with all
 // columns, whose one lane per column read its squares one by one: a root of 5,964 x 100 90 -> 41 us.
-template <int VEC>
+// CHAIN: few workgroups, whose chains of adds decide (member_chain_sum).
+template <int VEC, bool CHAIN>
 static __global__ void __launch_bounds__(256) k_seg_variance_tile(const uint32_t *__restrict__ perm, const uint2 *__restrict__ seg_range, int nseg,
                                                                  const float *__restrict__ means, int64_t first,
                                                                  const float *__restrict__ x, int64_t ld, int dim, int width, int pieces,
@@ -170,7 +171,7 @@ static __global__ void __launch_bounds__(256) k_seg_variance_tile(const uint32_t
     const int g = blockIdx.x % (unsigned)nseg, tile = blockIdx.x / (unsigned)nseg;
     const int c0 = tile * width < dim - width ? tile * width : dim - width;
     const uint2 r = seg_range[g];
-    const float sum = member_tile_sum<256, VEC, true>(reinterpret_cast<float *>(lds_var), x + c0, ld, r.x, r.y, width, pieces,
+    const float sum = tile_sum<256, VEC, true, CHAIN>(reinterpret_cast<float *>(lds_var), x + c0, ld, r.x, r.y, width, pieces,
                                                       [&](uint32_t p) { return perm[p]; }, means + (first + g) * dim + c0);
     if ((int)threadIdx.x < width) var[(size_t)g * dim + c0 + threadIdx.x] = sum;
 }
@@ -1161,7 +1162,7 @@ __device__ __forceinline__ int leaf_depth(uint32_t cnt) {
 
 // Sums of the leaves of a level's nodes, a workgroup per (node, one of every `per` leaves, tile of up to 16 components, as
 // k_node_stats has them): leaf_sum[(node * kNodeLeaves + leaf) * dim + component].
-template <int VEC>
+template <int VEC, bool CHAIN>
 static __global__ void __launch_bounds__(256) k_node_leafsum(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, int slots,
                                                              int per, const float *__restrict__ x, int64_t ld, int dim, int width,
                                                              int pieces, float *__restrict__ leaf_sum) {
@@ -1173,7 +1174,7 @@ static __global__ void __launch_bounds__(256) k_node_leafsum(const uint32_t *__r
     const int dep = leaf_depth(cnt);
     for (uint32_t l = (uint32_t)(rest % per); cnt && l < (1u << dep); l += (uint32_t)per) {
         const uint2 lr = leaf_range(cnt, dep, l);
-        const float sum = member_tile_sum<256, VEC>(reinterpret_cast<float *>(lds_node), x + c0, ld, r.x + lr.x, r.x + lr.y, width, pieces,
+        const float sum = tile_sum<256, VEC, false, CHAIN>(reinterpret_cast<float *>(lds_node), x + c0, ld, r.x + lr.x, r.x + lr.y, width, pieces,
                                                     [&](uint32_t p) { return perm[p]; });
         if ((int)threadIdx.x < width) leaf_sum[((size_t)g * kNodeLeaves + l) * dim + c0 + threadIdx.x] = sum;
         __syncthreads();  // (the stage has been read)
@@ -1184,7 +1185,7 @@ static __global__ void __launch_bounds__(256) k_node_leafsum(const uint32_t *__r
 // k_seg_variance_tile.  SUMS: the leaves are summed here, one after the other (nodes of up to 1024 rows have one); else from leaf_sum.
 // NT threads: 64 for nodes of up to 256 rows, whose chunks of 128 members leave room for more workgroups (the last levels
 // of 100,000 x 128, nodes of 195 and 98 rows: 23 -> 15 us each).
-template <int VEC, bool SUMS, int NT>
+template <int VEC, bool SUMS, int NT, bool CHAIN>
 static __global__ void __launch_bounds__(NT) k_node_stats(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, int slots,
                                                            const float *__restrict__ x, int64_t ld, int dim, int width, int pieces,
                                                            const float *__restrict__ leaf_sum, float *__restrict__ means,
@@ -1202,8 +1203,8 @@ static __global__ void __launch_bounds__(NT) k_node_stats(const uint32_t *__rest
     for (uint32_t l = 0; l < nl; ++l) {
         if constexpr (SUMS) {
             const uint2 lr = leaf_range(cnt, dep, l);
-            const float sum = member_tile_sum<NT, VEC>(stage, x + c0, ld, r.x + lr.x, r.x + lr.y, width, pieces,
-                                                        [&](uint32_t p) { return perm[p]; });
+            const auto row = [&](uint32_t p) { return perm[p]; };
+            const float sum = tile_sum<NT, VEC, false, CHAIN>(stage, x + c0, ld, r.x + lr.x, r.x + lr.y, width, pieces, row);
             if (tid < width) leaf[l][tid] = sum;
             __syncthreads();  // (the stage has been read)
         } else if (tid < width) {
@@ -1218,7 +1219,8 @@ static __global__ void __launch_bounds__(NT) k_node_stats(const uint32_t *__rest
     }
     if (!var || cnt < 2) return;
     __syncthreads();
-    const float sum = member_tile_sum<NT, VEC, true>(stage, x + c0, ld, r.x, r.y, width, pieces, [&](uint32_t p) { return perm[p]; }, leaf[0]);
+    const auto row = [&](uint32_t p) { return perm[p]; };
+    const float sum = tile_sum<NT, VEC, true, CHAIN>(stage, x + c0, ld, r.x, r.y, width, pieces, row, leaf[0]);
     if (tid < width) var[(size_t)g * dim + c0 + tid] = sum;
 }
 

@@ -362,7 +362,9 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     // The columns of a workgroup of the kernels that take a node's rows by tiles.
     const int tiles = (int)cdiv(dim, 16), width = tiles == 1 ? dim : (int)cdiv(cdiv(dim, tiles), 4) * 4;
     const int vec = dim >= 4 ? 4 : 1, pieces = (int)cdiv(width, vec), wtiles = (int)cdiv(dim, width);
-    const auto tile_lds = [&](int threads) { return sizeof(float) * (size_t)width * (8 * (threads / pieces) + 4); };
+    const auto tile_lds = [&](int threads, bool chain) {
+        return sizeof(float) * (chain ? vq::chain_stage_floats(threads, width, pieces) : (size_t)width * (8 * (threads / pieces) + 4));
+    };
     // Levels of short nodes without the host between them (k_node_stats, k_node_split): as many as their tables
     // take at once, then the host numbers the nodes.  Sets done, or leaves level and depth_left at the first level not built.
     auto device_levels = [&](bool &ran, bool &done) -> int32_t {
@@ -408,15 +410,24 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
             const dim3 grid((unsigned)((int64_t)ns * wtiles)), block(256);
             if (d < leafy) {
                 const int per = 1 << tree_depth(usual);
-                hipLaunchKernelGGL(vec == 4 ? vq::k_node_leafsum<4> : vq::k_node_leafsum<1>, dim3((unsigned)((int64_t)ns * wtiles * per)), block,
-                                   tile_lds(256), st, perm, r, ns, per, d_x, ld, dim, width, pieces, d_lsum);
-                hipLaunchKernelGGL((vec == 4 ? vq::k_node_stats<4, false, 256> : vq::k_node_stats<1, false, 256>), grid, block, tile_lds(256), st, perm, r, ns,
-                                   d_x, ld, dim, width, pieces, (const float *)d_lsum, means, var);
+                const int64_t groups = (int64_t)ns * wtiles * per;
+                const bool chain = groups <= vq::kChainGroups, chain2 = grid.x <= (unsigned)vq::kChainGroups;
+                hipLaunchKernelGGL((vec == 4 ? (chain ? vq::k_node_leafsum<4, true> : vq::k_node_leafsum<4, false>)
+                                             : (chain ? vq::k_node_leafsum<1, true> : vq::k_node_leafsum<1, false>)),
+                                   dim3((unsigned)groups), block, tile_lds(256, chain), st, perm, r, ns, per, d_x, ld, dim, width, pieces, d_lsum);
+                hipLaunchKernelGGL((vec == 4 ? (chain2 ? vq::k_node_stats<4, false, 256, true> : vq::k_node_stats<4, false, 256, false>)
+                                             : (chain2 ? vq::k_node_stats<1, false, 256, true> : vq::k_node_stats<1, false, 256, false>)),
+                                   grid, block, tile_lds(256, chain2), st, perm, r, ns, d_x, ld, dim, width, pieces, (const float *)d_lsum, means, var);
             } else {
-                const bool wave = usual <= 256;
-                hipLaunchKernelGGL((vec == 4 ? (wave ? vq::k_node_stats<4, true, 64> : vq::k_node_stats<4, true, 256>)
-                                             : (wave ? vq::k_node_stats<1, true, 64> : vq::k_node_stats<1, true, 256>)),
-                                   grid, dim3(wave ? 64 : 256), tile_lds(wave ? 64 : 256), st, perm, r, ns, d_x, ld, dim, width, pieces,
+                // (a wave, or the usual workgroup, or that with its chains)
+                const int kind = usual <= 256 ? 0 : grid.x > (unsigned)vq::kChainGroups ? 1 : 2, threads = kind ? 256 : 64;
+                const auto kern = vec == 4 ? (kind == 0   ? vq::k_node_stats<4, true, 64, false>
+                                              : kind == 1 ? vq::k_node_stats<4, true, 256, false>
+                                                          : vq::k_node_stats<4, true, 256, true>)
+                                           : (kind == 0   ? vq::k_node_stats<1, true, 64, false>
+                                              : kind == 1 ? vq::k_node_stats<1, true, 256, false>
+                                                          : vq::k_node_stats<1, true, 256, true>);
+                hipLaunchKernelGGL(kern, grid, dim3(threads), tile_lds(threads, kind == 2), st, perm, r, ns, d_x, ld, dim, width, pieces,
                                    (const float *)nullptr, means, var);
             }
             if (d == D) break;
@@ -801,9 +812,12 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                                    (const float *)d_sq, (const uint2 *)d_range, dim, (float *)d_var);
             }
         } else {
-            hipLaunchKernelGGL(vec == 4 ? vq::k_seg_variance_tile<4> : vq::k_seg_variance_tile<1>, dim3((unsigned)((int64_t)ns * wtiles)), dim3(256),
-                               tile_lds(256), st, perm, (const uint2 *)d_range, ns, (const float *)d_smeans,
-                               (int64_t)0, d_x, ld, dim, width, pieces, (float *)d_var);
+            const int64_t groups = (int64_t)ns * wtiles;
+            const bool chain = groups <= vq::kChainGroups;
+            hipLaunchKernelGGL((vec == 4 ? (chain ? vq::k_seg_variance_tile<4, true> : vq::k_seg_variance_tile<4, false>)
+                                         : (chain ? vq::k_seg_variance_tile<1, true> : vq::k_seg_variance_tile<1, false>)),
+                               dim3((unsigned)groups), dim3(256), tile_lds(256, chain), st, perm, (const uint2 *)d_range, ns,
+                               (const float *)d_smeans, (int64_t)0, d_x, ld, dim, width, pieces, (float *)d_var);
         }
         SP_HIP(hipGetLastError());
         if (split_wg) {  // (a leaf's rows are not moved: nothing reads them again)
