@@ -10,7 +10,8 @@ namespace vq {
 
 // acc and the count values of a column in LDS (16-byte aligned), one after the other: sixteen are added while the next sixteen are
 // read.  The scheduler is held to that order: left to itself it puts the reads behind the adds, and every sixteen members
-// wait for LDS.
+// wait for LDS.  (A chain alone on its compute unit gains by it; where other workgroups fill the wait the registers cost more:
+// add_column_plain.)
 __device__ __forceinline__ float add_column(const float *col, uint32_t count, float acc) {
     float4 q[2][4];
     auto read = [&](float4 (&d)[4], uint32_t at) {
@@ -51,14 +52,32 @@ __device__ __forceinline__ float add_column(const float *col, uint32_t count, fl
     return acc;
 }
 
+// The same, sixteen read and then added.
+__device__ __forceinline__ float add_column_plain(const float *col, uint32_t count, float acc) {
+    uint32_t m = 0;
+    for (; m + 16 <= count; m += 16) {
+        float4 q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = *reinterpret_cast<const float4 *>(col + m + 4 * u);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            acc = acc + q[u].x;
+            acc = acc + q[u].y;
+            acc = acc + q[u].z;
+            acc = acc + q[u].w;
+        }
+    }
+    for (; m < count; ++m) acc = acc + col[m];
+    return acc;
+}
+
 // The sum of members lo .. hi - 1 of a list (row_of: position -> row) over a tile of up to VEC P components, by a
 // workgroup: P pieces of VEC floats per member; the threads fetch a chunk of members into registers, eight loads of each in
 // flight while the chunk before is added, and store them transposed in LDS (stage: width * (8 NT / P + 4) floats); a lane per
-// component adds them in list order, sixteen members read at a time (with the next sixteen read
-// beside the adds no faster).  xs: row 0's tile.  Returned in the lanes
+// component adds them in list order, sixteen members read at a time.  xs: row 0's tile.  Returned in the lanes
 // below width.  The last piece of a tile begins at the tile's end less VEC, so that pieces of any width are whole (what
 // two of them share is written twice, with the same values).  Its time is a chain of memory round trips, one per chunk of 128
-// to 512 members, beside the adds: 7,930 x 300, k = 22 41 -> 17 us per launch, 50,019 x 28 blocks of 10, k = 78 110 -> 28.
+// to 512 members, beside the adds (reading ahead as add_column does costs fits 1 to 3 %: 84,443 x 100, k = 108 3351 -> 3424 us): 7,930 x 300, k = 22 41 -> 17 us per launch, 50,019 x 28 blocks of 10, k = 78 110 -> 28.
 // (With chunks of twice the members by 256 threads the same, where the leaves are long; the LDS then holds half the leaves.)
 // DEV: of the squared deviations from mean (the tile's), two roundings each, made as they are stored.
 template <int NT, int VEC, bool DEV = false, typename RowOf>
@@ -112,7 +131,7 @@ __device__ __forceinline__ float member_tile_sum(float *stage, const float *__re
             if (p + chunk < hi) load(p + chunk);
         }
         __syncthreads();
-        if (tid < width) acc = add_column(stage + (uint32_t)tid * stride, cm, acc);
+        if (tid < width) acc = add_column_plain(stage + (uint32_t)tid * stride, cm, acc);
     }
     return acc;
 }
