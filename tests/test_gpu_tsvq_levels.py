@@ -23,6 +23,10 @@ def ctx():
     (4096, 10, 6, "lopsided"), (8192, 100, 7, "lopsided"), (8000, 97, 5, "lopsided"), (3000, 3, 8, "normal"),
     (20000, 8, 8, "lopsided"), (30000, 96, 7, "lopsided"), (700, 1, 10, "normal"), (40, 6, 13, "normal"), (2100, 4, 14, "lopsided"),
     (6000, 17, 12, "copies"), (257, 20, 1, "normal"), (5, 2, 3, "copies"), (9000, 33, 9, "copies"),
+    # a chain's chunks of 336 members (16 components) and the ends of its two stages, three components, a last tile that overlaps
+    (335, 16, 1, "normal"), (336, 16, 1, "normal"), (337, 16, 1, "normal"), (672, 16, 1, "normal"), (1009, 20, 1, "normal"), (900, 3, 1, "normal"),
+    # more workgroups than a round: tiles of up to 32 components, nodes of some hundred rows and of two leaves
+    (30_000, 256, 7, "normal"), (40_000, 100, 8, "normal"), (26_000, 250, 6, "lopsided"), (90_000, 130, 6, "normal"),
 ])
 def test_levels_on_device(ctx, n, dim, depth, kind):
     rng = np.random.default_rng(17 * n + dim)

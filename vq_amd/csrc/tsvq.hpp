@@ -157,7 +157,7 @@ static __global__ void __launch_bounds__(256) k_seg_mean_wg(const float *__restr
     if (q == 0 && c < sd) out[(out_first + g) * sd + c] = tree[0][t] / __uint2float_rn(info.z);
 }
 
-// Sums of squared deviations in row order, a workgroup per segment and tile of up to 16 components (block
+// Sums of squared deviations in row order, a workgroup per segment and tile of up to 32 components (block
 // tile * nseg + segment, as y would end at 65,535 tiles; the last tile begins at dim less its width): seg_range[g] = {lo, hi} positions in perm; mean of segment g at means[(first + g) * dim].
 // A chunk of 512 rows was a memory round trip, two barriers and their adds, 3.5 us in all or 7 ns a row; 4 ns where the chunks overlap the adds (CHAIN).  Against one workgroup per segment with all
 // columns, whose one lane per column read its squares one by one: a root of 5,964 x 100 90 -> 41 us.
@@ -1160,7 +1160,7 @@ __device__ __forceinline__ int leaf_depth(uint32_t cnt) {
     return dep;
 }
 
-// Sums of the leaves of a level's nodes, a workgroup per (node, one of every `per` leaves, tile of up to 16 components, as
+// Sums of the leaves of a level's nodes, a workgroup per (node, one of every `per` leaves, tile of up to 32 components, as
 // k_node_stats has them): leaf_sum[(node * kNodeLeaves + leaf) * dim + component].
 template <int VEC, bool CHAIN>
 static __global__ void __launch_bounds__(256) k_node_leafsum(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, int slots,
@@ -1191,7 +1191,7 @@ static __global__ void __launch_bounds__(NT) k_node_stats(const uint32_t *__rest
                                                            const float *__restrict__ leaf_sum, float *__restrict__ means,
                                                            float *__restrict__ var) {
     extern __shared__ float4 lds_node[];
-    __shared__ float leaf[kNodeLeaves][16];
+    __shared__ float leaf[kNodeLeaves][32];
     float *stage = reinterpret_cast<float *>(lds_node);
     const int g = blockIdx.x % (unsigned)slots, tile = blockIdx.x / (unsigned)slots, tid = threadIdx.x;
     const int c0 = tile * width < dim - width ? tile * width : dim - width;

@@ -359,11 +359,21 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     };
     auto pad = [](size_t z) { return (z + 255) & ~(size_t)255; };
 
-    // The columns of a workgroup of the kernels that take a node's rows by tiles.
-    const int tiles = (int)cdiv(dim, 16), width = tiles == 1 ? dim : (int)cdiv(cdiv(dim, tiles), 4) * 4;
-    const int vec = dim >= 4 ? 4 : 1, pieces = (int)cdiv(width, vec), wtiles = (int)cdiv(dim, width);
-    const auto tile_lds = [&](int threads, bool chain) {
-        return sizeof(float) * (chain ? vq::chain_stage_floats(threads, width, pieces) : (size_t)width * (8 * (threads / pieces) + 4));
+    // The columns of a workgroup of the kernels that take a node's rows by tiles: 16, or 32 where chains do not decide
+    // (kChainGroups): those are whole lines of the rows, and with 16 a level of rows that the L2 does not hold reads its lines
+    // twice.  Builds, 16 -> 32: 1,000,000 x 128, ten levels 5278 -> 4845 us, 471,568 x 96, eight 2073 -> 1965, 200,000 x 128, ten 1583 -> 1535,
+    // 500,000 x 64, ten 2139 -> 1994, 100,000 x 256, nine 1356 -> 1328.
+    const int vec = dim >= 4 ? 4 : 1;
+    struct Tiles {
+        int width, pieces, count;
+    };
+    const auto tiles_of = [&](int most) {
+        const int t = (int)cdiv(dim, most), w = t == 1 ? dim : (int)cdiv(cdiv(dim, t), 4) * 4;
+        return Tiles{w, (int)cdiv(w, vec), (int)cdiv(dim, w)};
+    };
+    const Tiles narrow = tiles_of(16), broad = tiles_of(32);
+    const auto tile_lds = [&](const Tiles &t, int threads, bool chain) {
+        return sizeof(float) * (chain ? vq::chain_stage_floats(threads, t.width, t.pieces) : (size_t)t.width * (8 * (threads / t.pieces) + 4));
     };
     // Levels of short nodes without the host between them (k_node_stats, k_node_split): as many as their tables
     // take at once, then the host numbers the nodes.  Sets done, or leaves level and depth_left at the first level not built.
@@ -407,28 +417,33 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
             const uint32_t usual = std::max(longest >> d, 1u);
             const uint2 *r = d_range + o;
             float *means = d_means + o * dim, *var = d < D ? d_var : nullptr;
-            const dim3 grid((unsigned)((int64_t)ns * wtiles)), block(256);
+            const dim3 block(256);
+            const bool chain2 = (int64_t)ns * narrow.count <= vq::kChainGroups;
+            const Tiles &t2 = chain2 ? narrow : broad;
             if (d < leafy) {
                 const int per = 1 << tree_depth(usual);
-                const int64_t groups = (int64_t)ns * wtiles * per;
-                const bool chain = groups <= vq::kChainGroups, chain2 = grid.x <= (unsigned)vq::kChainGroups;
+                const bool chain = (int64_t)ns * narrow.count * per <= vq::kChainGroups;
+                const Tiles &t = chain ? narrow : broad;
                 hipLaunchKernelGGL((vec == 4 ? (chain ? vq::k_node_leafsum<4, true> : vq::k_node_leafsum<4, false>)
                                              : (chain ? vq::k_node_leafsum<1, true> : vq::k_node_leafsum<1, false>)),
-                                   dim3((unsigned)groups), block, tile_lds(256, chain), st, perm, r, ns, per, d_x, ld, dim, width, pieces, d_lsum);
+                                   dim3((unsigned)((int64_t)ns * t.count * per)), block, tile_lds(t, 256, chain), st, perm, r, ns, per, d_x, ld,
+                                   dim, t.width, t.pieces, d_lsum);
                 hipLaunchKernelGGL((vec == 4 ? (chain2 ? vq::k_node_stats<4, false, 256, true> : vq::k_node_stats<4, false, 256, false>)
                                              : (chain2 ? vq::k_node_stats<1, false, 256, true> : vq::k_node_stats<1, false, 256, false>)),
-                                   grid, block, tile_lds(256, chain2), st, perm, r, ns, d_x, ld, dim, width, pieces, (const float *)d_lsum, means, var);
+                                   dim3((unsigned)((int64_t)ns * t2.count)), block, tile_lds(t2, 256, chain2), st, perm, r, ns, d_x, ld, dim,
+                                   t2.width, t2.pieces, (const float *)d_lsum, means, var);
             } else {
                 // (a wave, or the usual workgroup, or that with its chains)
-                const int kind = usual <= 256 ? 0 : grid.x > (unsigned)vq::kChainGroups ? 1 : 2, threads = kind ? 256 : 64;
+                const int kind = usual <= 256 ? 0 : chain2 ? 2 : 1, threads = kind ? 256 : 64;
+                const Tiles &t = kind == 1 ? broad : narrow;
                 const auto kern = vec == 4 ? (kind == 0   ? vq::k_node_stats<4, true, 64, false>
                                               : kind == 1 ? vq::k_node_stats<4, true, 256, false>
                                                           : vq::k_node_stats<4, true, 256, true>)
                                            : (kind == 0   ? vq::k_node_stats<1, true, 64, false>
                                               : kind == 1 ? vq::k_node_stats<1, true, 256, false>
                                                           : vq::k_node_stats<1, true, 256, true>);
-                hipLaunchKernelGGL(kern, grid, dim3(threads), tile_lds(threads, kind == 2), st, perm, r, ns, d_x, ld, dim, width, pieces,
-                                   (const float *)nullptr, means, var);
+                hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)ns * t.count)), dim3(threads), tile_lds(t, threads, kind == 2), st, perm, r,
+                                   ns, d_x, ld, dim, t.width, t.pieces, (const float *)nullptr, means, var);
             }
             if (d == D) break;
             const uint32_t room = std::min(longest, usual + usual / 8 + 64);
@@ -812,12 +827,12 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                                    (const float *)d_sq, (const uint2 *)d_range, dim, (float *)d_var);
             }
         } else {
-            const int64_t groups = (int64_t)ns * wtiles;
-            const bool chain = groups <= vq::kChainGroups;
+            const bool chain = (int64_t)ns * narrow.count <= vq::kChainGroups;
+            const Tiles &t = chain ? narrow : broad;
             hipLaunchKernelGGL((vec == 4 ? (chain ? vq::k_seg_variance_tile<4, true> : vq::k_seg_variance_tile<4, false>)
                                          : (chain ? vq::k_seg_variance_tile<1, true> : vq::k_seg_variance_tile<1, false>)),
-                               dim3((unsigned)groups), dim3(256), tile_lds(256, chain), st, perm, (const uint2 *)d_range, ns,
-                               (const float *)d_smeans, (int64_t)0, d_x, ld, dim, width, pieces, (float *)d_var);
+                               dim3((unsigned)((int64_t)ns * t.count)), dim3(256), tile_lds(t, 256, chain), st, perm, (const uint2 *)d_range, ns,
+                               (const float *)d_smeans, (int64_t)0, d_x, ld, dim, t.width, t.pieces, (float *)d_var);
         }
         SP_HIP(hipGetLastError());
         if (split_wg) {  // (a leaf's rows are not moved: nothing reads them again)
