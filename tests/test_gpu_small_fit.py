@@ -72,3 +72,27 @@ def test_small_fit_cluster_sizes(ctx, sd, m, largest):
     it, used = ctx.lbg_fit(ctx.to_device(x), n, m * sd, m, sd, k, 2, init, reseed, dcb)
     assert want["rc"] == 0 and np.array_equal(it, want["iters"]) and np.array_equal(used, want["reseeds"])
     assert np.array_equal(dcb.download().view(np.uint32), want["codebooks"].view(np.uint32))
+
+
+@pytest.mark.parametrize("n,m,sd,k", [(12_000, 1, 36, 64), (12_289, 2, 36, 200), (12_000, 1, 100, 64), (12_288, 1, 300, 256), (10_000, 1, 512, 256),
+                                      (8192, 1, 48, 30), (8193, 2, 52, 60), (12_000, 20, 48, 100), (32_768, 1, 40, 200), (32_769, 1, 40, 200)])
+def test_small_fit_tiles(ctx, n, m, sd, k):
+    """Blocks above 32 floats by tiles whose last one overlaps (or whole, where there are many): clusters on both sides
+    of the size from which each part's members are added by tiles too, and one that is re-seeded."""
+    rng = np.random.default_rng(n + sd)
+    line = 1024 * -(-n // 4096)
+    sizes = [line + 1, line, 1025] if 2 * line + 1100 + k < n else [line + 1, 1024]
+    rest = n - sum(sizes)
+    sizes += [rest // (k - len(sizes))] * (k - len(sizes) - 1)
+    sizes.append(n - sum(sizes))
+    label = rng.permutation(np.repeat(np.arange(k), sizes))
+    x = (50.0 * label[:, None] + rng.random((n, m * sd))).astype(F)
+    first = np.array([int(np.flatnonzero(label == j)[0]) for j in range(k)])
+    first[k // 2] = first[k // 2 + 1]
+    init = np.stack([first[(np.arange(k) + s) % k] for s in range(m)]).astype(np.uint32)
+    reseed = rng.integers(0, n, (m, 2 * k), dtype=np.uint32)
+    want = O.pq_fit(x, m, k, 2, init, reseed)
+    dcb = ctx.empty((m, k, sd), F)
+    it, used = ctx.lbg_fit(ctx.to_device(x), n, m * sd, m, sd, k, 2, init, reseed, dcb)
+    assert want["rc"] == 0 and np.array_equal(it, want["iters"]) and np.array_equal(used, want["reseeds"]) and used.min() > 0
+    assert np.array_equal(dcb.download().view(np.uint32), want["codebooks"].view(np.uint32))

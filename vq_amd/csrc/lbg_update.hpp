@@ -805,6 +805,11 @@ static __global__ void __launch_bounds__(256) k_lbg_finalize(LbgState st, const 
 // them in list order (add_members).  The orders of summation are those above: row order up
 // to 1024 members, part sums in part order above.
 // DEFER: clusters above 1024 members are counted and left to k_lbg_large.
+// Blocks above 32 floats (SD 16, 32 and tiles > 1): a workgroup takes a tile of the components of C clusters.  The floats that it
+// brings in are those of a whole block of C / tiles clusters, but a stage holds 1024 or 512 members instead of 170 of 96 floats, and a
+// long cluster's are spread over several workgroups: what bounded it was one memory round trip per stage of the longest cluster.
+// An iteration of a residual fit of 6,264 x 96, k = 186 61 -> 49 us, 7,143 x 100, k = 214 87 -> 63; fits, three or four stages of six iterations, of
+// 8,000 x 256, k = 256 2356 -> 1647 us, 10,000 x 512 2729 -> 1830, 12,000 x 300, k = 100 3540 -> 2520.
 // STAGED: sub_dim a multiple of 4 up to 512, a thread per component.  Else (wider blocks) a wave takes
 // one cluster and 64 components at a time and reads the rows themselves, 16 rows in flight.
 constexpr int kSmallList = 8192;    // listed rows held before the list is worked off: at least 16 per thread
@@ -957,12 +962,14 @@ __device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
 template <bool STAGED, bool DEFER = false, int SD = 0>
 static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSmall st, int it, int m,
                                                                            const float *__restrict__ x, int64_t n,
-                                                                           int64_t ld, int sub_dim, int k, int C,
-                                                                           int groups, const uint32_t *__restrict__ reseed,
+                                                                           int64_t ld, int sub_dim, int tiles, int k,
+                                                                           int C, int groups, const uint32_t *__restrict__ reseed,
                                                                            int n_reseed, float *__restrict__ cb) {
-    const int sd = SD ? SD : sub_dim;
-    const unsigned id = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int s = (int)(id / (unsigned)groups), j0 = (int)(id % (unsigned)groups) * C;
+    constexpr bool TILES = STAGED && (SD == 16 || SD == 32);
+    const int sd = SD ? SD : sub_dim, full = TILES ? sub_dim : sd;
+    const unsigned id = xcd_contiguous(blockIdx.x, gridDim.x), unit = TILES ? id / (unsigned)tiles : id;  // (tiles of the same rows side by side)
+    const int tile = TILES ? (int)(id % (unsigned)tiles) : 0, c0 = tile * sd < full - sd ? tile * sd : full - sd;
+    const int s = (int)(unit / (unsigned)groups), j0 = (int)(unit % (unsigned)groups) * C;
     if (st.changed[it * m + s] == 0) return;  // converged before this iteration
     const int jn = k - j0 < C ? k - j0 : C;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -975,7 +982,7 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
     __shared__ uint32_t wave_tot[2][kSmallWaves];
     extern __shared__ float dyn[];  // STAGED: the sub-vectors; else three sums per (cluster, component)
     const uint8_t *codes = st.codes + (size_t)s * n;
-    const float *xs = x + (int64_t)s * sd;
+    const float *xs = x + (int64_t)s * full + c0;
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     if (tid < kSmallClusters) {
         cl_cnt[tid] = 0u;
@@ -1180,7 +1187,7 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
         for (int p = -3; p < 0; ++p) advance(p);  // the first steps again
         for (int c = 0; c < jn; ++c) large |= (cl_cnt[c] > (uint32_t)kSeqMax ? 1u : 0u) << c;
         large = __builtin_amdgcn_readfirstlane(large);
-        if (tid < jn && ((large >> tid) & 1u))
+        if (tile == 0 && tid < jn && ((large >> tid) & 1u))
             st.large[atomicAdd(st.n_large + it, 1)] = make_uint2((uint32_t)(s * kMaxK + j0 + tid), cl_cnt[tid]);
     }
     for (int p = 0; p < nsteps; ++p) {
@@ -1222,12 +1229,12 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
         big = summing && cl_cnt[my_c] > (uint32_t)kSeqMax;
     }
     drain();
-    float *out = cb + ((size_t)s * k + j0) * sd;
+    float *out = cb + ((size_t)s * k + j0) * full + c0;
     if constexpr (STAGED) {
         if (summing) {
             const uint32_t cm = cl_cnt[my_c];
             if (cm && !((large >> my_c) & 1u))
-                out[my_c * sd + my_t] =
+                out[my_c * full + my_t] =
                     (cm > (uint32_t)kSeqMax ? total + part : (track == kBoth ? seq : part)) / __uint2float_rn(cm);
         }
     } else {
@@ -1254,7 +1261,7 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
             cl_off[c] = (uint32_t)(used + mine);  // place in the stream
             mine += cl_cnt[c] == 0u;
         }
-        atomicAdd(st.empties + it * m + s, mine);
+        if (tile == 0) atomicAdd(st.empties + it * m + s, mine);
     }
     __syncthreads();
     for (int i = tid; i < jn * sd; i += kSmallThreads) {
@@ -1264,20 +1271,28 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
         if (pos >= n_reseed)
             st.err[0] = 1;  // the centroid stays
         else
-            out[i] = xs[(int64_t)reseed[(size_t)s * n_reseed + pos] * ld + t];
+            out[c * full + t] = xs[(int64_t)reseed[(size_t)s * n_reseed + pos] * ld + t];
     }
 }
 
 // The clusters above 1024 members of a small fit over wide blocks (rows that are residuals gather in a
-// few of them): workgroup (part p, y) takes the listed clusters y, y + gridDim.y, ... and adds the
+// few of them): workgroup (part p, y) takes the listed clusters y, y + whole, ... and adds the
 // members in part p in row order, staged through LDS as above; the workgroup that brings a cluster's
 // last part adds the part sums in part order and divides.  One workgroup that adds such a cluster alone
 // is bound by what it has in flight, 64 KB per memory round trip: 6,000 rows of 128 took 200 us.
+// SD: a cluster with more than kLargeTiled members per part (three of a column block at most) is taken by tiles of SD components, which
+// hold 1024 or 512 members per memory round trip: workgroups (p, whole + tile), which look for such clusters.  For the others a
+// fence per tile is more than what the tiles save (20,000 x 128, k = 256, tiles of all clusters 22.7 us a launch, of these 17.1;
+// 15,980 x 96, k = 63 28.6 without tiles).
+constexpr int kLargeTiled = 1024;
+template <int SD>
 static __global__ void __launch_bounds__(kSmallThreads) k_lbg_large(LbgSmall st, int it, const float *__restrict__ x,
-                                                                    int64_t n, int64_t ld, int sd, int k,
+                                                                    int64_t n, int64_t ld, int full, int k, int whole,
                                                                     float *__restrict__ cb) {
     const int count = st.n_large[it];
-    if ((int)blockIdx.y >= count) return;
+    const bool tiled = SD != 0 && (int)blockIdx.y >= whole;
+    if (tiled ? count == 0 : (int)blockIdx.y >= count) return;
+    const int tile = tiled ? (int)blockIdx.y - whole : 0, tiles = SD ? (int)gridDim.y - whole : 1;
     const int p = blockIdx.x, nparts = gridDim.x, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ uint16_t list[kPartRows];
@@ -1287,9 +1302,10 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_large(LbgSmall st,
     const int64_t lo = (int64_t)p * kPartRows;
     const int rows = n - lo < kPartRows ? (int)(n - lo) : kPartRows;
     typedef float piece4 __attribute__((ext_vector_type(4), aligned(4)));
-    for (int e = blockIdx.y; e < count; e += gridDim.y) {
+    auto by_tiles = [&](uint32_t members) { return SD != 0 && members > (uint32_t)(kLargeTiled * nparts); };
+    auto cluster = [&](int e) {
         const uint2 ent = st.large[e];
-        const int s = (int)(ent.x / kMaxK);
+        const int s = (int)(ent.x / kMaxK), c0 = !tiled ? 0 : tile * SD < full - SD ? tile * SD : full - SD;
         const uint32_t j = ent.x % kMaxK;
         const uint8_t *codes = st.codes + (size_t)s * n + lo;
         uint32_t mine = 0;  // of the thread's eight consecutive rows
@@ -1315,59 +1331,67 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_large(LbgSmall st,
         }
         for (; mine; mine &= mine - 1) list[at++] = (uint16_t)(8 * tid + __ffs(mine) - 1);
         __syncthreads();
-        const float *xs = x + lo * ld + (int64_t)s * sd;
-        const uint32_t per = (uint32_t)sd / 4u, most = (uint32_t)kSmallStage / (uint32_t)sd;
-        constexpr int E = kSmallStage / 4 / kSmallThreads;
-        piece4 v[E];
-        auto gather = [&](uint32_t p0) {
-            const uint32_t pn = cnt - p0 < most ? cnt - p0 : most;
+        const float *xs = x + lo * ld + (int64_t)s * full + c0;
+        float sum = 0.0f;
+        auto add_part = [&](auto fixed) {
+            constexpr int W = decltype(fixed)::value;
+            const uint32_t sd = W ? W : full, per = sd / 4u, most = (uint32_t)kSmallStage / sd;
+            constexpr int E = kSmallStage / 4 / kSmallThreads;
+            piece4 v[E];
+            float unused = 0.0f;
+            uint32_t open = 0;
+            auto gather = [&](uint32_t p0) {
+                const uint32_t pn = cnt - p0 < most ? cnt - p0 : most;
 #pragma unroll
-            for (int u = 0; u < E; ++u) {
-                const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * u, ic = i < pn * per ? i : 0u;
-                v[u] = *reinterpret_cast<const piece4 *>(xs + (int64_t)list[p0 + ic / per] * ld + 4u * (ic % per));
+                for (int u = 0; u < E; ++u) {
+                    const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * u, ic = i < pn * per ? i : 0u;
+                    v[u] = *reinterpret_cast<const piece4 *>(xs + (int64_t)list[p0 + ic / per] * ld + 4u * (ic % per));
+                }
+            };
+            if (cnt) gather(0);
+            for (uint32_t p0 = 0; p0 < cnt; p0 += most) {
+                const uint32_t pn = cnt - p0 < most ? cnt - p0 : most;
+#pragma unroll
+                for (int u = 0; u < E; ++u) {
+                    const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * u;
+                    if (i < pn * per) *reinterpret_cast<float4 *>(dyn + 4u * i) = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
+                }
+                __syncthreads();
+                if (p0 + most < cnt) gather(p0 + most);
+                if ((uint32_t)tid < sd) add_members<kRows>(dyn + tid, (int)sd, nullptr, 0, pn, false, unused, unused, sum, open);
+                __syncthreads();
             }
         };
-        float sum = 0.0f;
-        if (cnt) gather(0);
-        for (uint32_t p0 = 0; p0 < cnt; p0 += most) {
-            const uint32_t pn = cnt - p0 < most ? cnt - p0 : most;
-#pragma unroll
-            for (int u = 0; u < E; ++u) {
-                const uint32_t i = (uint32_t)tid + (uint32_t)kSmallThreads * u;
-                if (i < pn * per) *reinterpret_cast<float4 *>(dyn + 4u * i) = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
-            }
-            __syncthreads();
-            if (p0 + most < cnt) gather(p0 + most);
-            if (tid < sd) {
-                uint32_t i = 0;
-                for (; i + 8 <= pn; i += 8) {
-                    float t[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) t[u] = dyn[(i + u) * (uint32_t)sd + tid];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) sum = sum + t[u];
-                }
-                for (; i < pn; ++i) sum = sum + dyn[i * (uint32_t)sd + tid];
-            }
-            __syncthreads();
-        }
-        float *sums = st.large_sum + (size_t)e * nparts * sd;
-        if (tid < sd) sums[(size_t)p * sd + tid] = sum;
+        const int sd = tiled ? SD : full;
+        if (tiled) add_part(std::integral_constant<int, SD>{});
+        else add_part(std::integral_constant<int, 0>{});
+        float *sums = st.large_sum + (size_t)e * nparts * full + c0;
+        int *arrived = st.arrived + (size_t)e * tiles + tile;
+        if (tid < sd) sums[(size_t)p * full + tid] = sum;
         __threadfence();
         __syncthreads();
-        if (tid == 0) last = atomicAdd(st.arrived + e, 1) == nparts - 1;
+        if (tid == 0) last = atomicAdd(arrived, 1) == nparts - 1;
         __syncthreads();
         if (last) {
             __threadfence();
             if (tid < sd) {
                 float total = 0.0f;
                 for (int q = 0; q < nparts; ++q)
-                    total = total + __hip_atomic_load(sums + (size_t)q * sd + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                cb[((size_t)s * k + j) * sd + tid] = total / __uint2float_rn(ent.y);
+                    total = total + __hip_atomic_load(sums + (size_t)q * full + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                cb[((size_t)s * k + j) * full + c0 + tid] = total / __uint2float_rn(ent.y);
             }
-            if (tid == 0) st.arrived[e] = 0;  // for the next iteration
+            if (tid == 0) *arrived = 0;  // for the next iteration
         }
         __syncthreads();
+    };
+    if (!tiled) {
+        for (int e = blockIdx.y; e < count; e += whole)
+            if (!by_tiles(st.large[e].y)) cluster(e);  // uniform
+        return;
+    }
+    for (int e0 = 0; e0 < count; e0 += 64) {  // every wave finds the same entries
+        const bool mine = e0 + lane < count && by_tiles(st.large[e0 + lane < count ? e0 + lane : 0].y);
+        for (uint64_t mask = __ballot(mine); mask; mask &= mask - 1) cluster(e0 + __ffsll((unsigned long long)mask) - 1);
     }
 }
 

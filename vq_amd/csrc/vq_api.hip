@@ -1335,16 +1335,32 @@ static int lbg_small_clusters(int m, int sd, int k) {
     return c;
 }
 
+// Components of a workgroup of k_lbg_update_small: blocks above 32 floats are taken by tiles of 16 or 32 where those are a
+// round of the GPU; the last tile begins at the block's end less its width.
+static int lbg_small_width(int m, int sd, int k) {
+    if (sd <= 32) return sd;
+    for (int w : {16, 32})
+        if ((int64_t)m * (int64_t)cdiv(sd, w) * (int64_t)cdiv(k, vq::kSmallClusters) <= 256) return w;
+    return sd;
+}
+
 // Whether the update of a fit runs as k_lbg_update_small.  Its time follows the members of a cluster
 // (one chain of additions each) and the floats that a workgroup brings in, the other path's the number
 // of its launches.  The two take the same time near 700 members where the chain decides (blocks of
 // 8 floats, k = 116) and near 75,000 floats per workgroup in narrow blocks, 45,000-70,000 in wide ones, on
 // uniform rows and on mixtures.  Ten iterations, m = 16, k = 256, blocks of 8: 2,000 rows 0.83 -> 0.22 ms,
 // 10,000 1.07 -> 0.29 ms, 50,000 1.35 -> 0.74 ms; m = 1, k = 256, 20,000 x 128: 0.78 -> 0.45 ms.
+// Blocks above 32 floats: a block that is the whole row is a stage of a residual fit, whose rows gather in a few clusters, and every
+// workgroup lists all rows.  Three stages of five iterations, other path -> this one: k = 256, 30,000 x 64 1077 -> 994 us,
+// 45,000 1175 -> 1171, 65,000 1186 -> 1625, 130,000 1320 -> 3915; 20,000 x 128 1097 -> 1002, 40,000 1196 -> 1471; 16,000 x 256
+// 1314 -> 1276, 24,000 1332 -> 1533; k = 63, 16,000 x 96 1054 -> 1064.  Five iterations, k = 256: 40,000 x 2 of 48 393 -> 353, 80,000
+// 472 -> 663; 40,000 x 8 of 40 645 -> 660.  Narrower rows likewise, three stages, k = 256: 40,000 x 32 959 -> 933, 80,000 1058 -> 1321,
+// 130,000 1152 -> 1920; 40,000 x 24 954 -> 827, 80,000 1047 -> 1291; 80,000 x 16 875 -> 816, 130,000 930 -> 1201.
 static bool lbg_small(int64_t n, int m, int sd, int k) {
     if (sd % 4 != 0 || sd > 4096 || n > 131072) return false;
     if (sd > vq::kSmallThreads) return n <= 128 * (int64_t)k;
-    return n <= 640 * (int64_t)k && n * lbg_small_clusters(m, sd, k) * sd <= (sd <= 32 ? 57344 : 40960) * (int64_t)k;
+    if (sd > 32 ? n > 32768 : m == 1 && sd >= 16 && n > (sd > 16 ? 45056 : 90112)) return false;
+    return n <= 640 * (int64_t)k && n * lbg_small_clusters(m, sd, k) * sd <= (sd <= 32 ? 57344 : m == 1 ? 20480 : 40960) * (int64_t)k;
 }
 
 // The LBG loop of a small fit, two launches per iteration: the assignment and k_lbg_update_small.  The
@@ -1361,8 +1377,9 @@ static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
     const bool staged = sd <= vq::kSmallThreads;
     const int nparts = (int)cdiv(n, vq::kPartRows);
     const bool defer = staged && sd > 32 && nparts > 2;
+    const int width = staged ? lbg_small_width(m, sd, k) : sd, tiles = (int)cdiv(sd, width);
     const int most_large = defer ? (int)(m * (n / (vq::kSeqMax + 1))) : 0;
-    VQ_TRY(ensure(ctx, ctx->flags, sizeof(int) * (n_flags + max_iters + most_large)));
+    VQ_TRY(ensure(ctx, ctx->flags, sizeof(int) * (n_flags + max_iters + (size_t)most_large * tiles)));
     VQ_TRY(ensure(ctx, ctx->codes, (size_t)m * n + 4));
     if (defer) {
         VQ_TRY(ensure(ctx, ctx->leaf_desc, sizeof(uint2) * (size_t)most_large));
@@ -1384,7 +1401,7 @@ static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
     S.large_sum = (float *)ctx->leaf_sum.p;
     const int64_t init_items = std::max<int64_t>((int64_t)m * k * sd, (int64_t)m * n / 4);
     hipLaunchKernelGGL(vq::k_lbg_small_init, dim3(std::min<unsigned>(cdiv(init_items, 256), 1024u)), dim3(256), 0, st, S,
-                       d_x, n, ld, m, k, sd, max_iters, most_large, (const uint32_t *)idx, d_codebooks, pend_cb, pend_codes);
+                       d_x, n, ld, m, k, sd, max_iters, most_large * tiles, (const uint32_t *)idx, d_codebooks, pend_cb, pend_codes);
     vq::AssignArgs a;
     a.x = d_x;
     a.n = n;
@@ -1395,14 +1412,19 @@ static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
     a.cnorm = nullptr;
     a.codes = S.codes;
     a.done = nullptr;
-    const int C = lbg_small_clusters(m, sd, k);
+    const int C = lbg_small_clusters(m * tiles, width, k);
     const int groups = (int)cdiv(k, C);
     if (staged && !ctx->lbg_small_lds_set) {
         const void *kerns[] = {reinterpret_cast<const void *>(vq::k_lbg_update_small<true>),
                                reinterpret_cast<const void *>(vq::k_lbg_update_small<true, false, 8>),
                                reinterpret_cast<const void *>(vq::k_lbg_update_small<true, false, 16>),
+                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, false, 32>),
                                reinterpret_cast<const void *>(vq::k_lbg_update_small<true, true>),
-                               reinterpret_cast<const void *>(vq::k_lbg_large)};
+                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, true, 16>),
+                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, true, 32>),
+                               reinterpret_cast<const void *>(vq::k_lbg_large<0>),
+                               reinterpret_cast<const void *>(vq::k_lbg_large<16>),
+                               reinterpret_cast<const void *>(vq::k_lbg_large<32>)};
         for (const void *kern : kerns)
             VQ_HIP(ctx, hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                             (int)(sizeof(float) * vq::kSmallStage)));
@@ -1418,23 +1440,19 @@ static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
             VQ_TRY(launch_assign<true>(ctx, VQ_SQEUCLIDEAN, a, sd));
         }
         ProfSpan sp(ctx, VQ_PROF_LBG_UPDATE);
-        if (defer) {
-            hipLaunchKernelGGL((vq::k_lbg_update_small<true, true>), dim3(groups * m), dim3(vq::kSmallThreads),
-                               sizeof(float) * vq::kSmallStage, st, S, it, m, d_x, n, ld, sd, k, C, groups,
-                               (const uint32_t *)reseed, n_reseed, d_codebooks);
-            hipLaunchKernelGGL(vq::k_lbg_large, dim3(nparts, std::min(most_large, 16)), dim3(vq::kSmallThreads),
-                               sizeof(float) * vq::kSmallStage, st, S, it, d_x, n, ld, sd, k, d_codebooks);
-        } else if (staged)
-            hipLaunchKernelGGL((sd == 8    ? vq::k_lbg_update_small<true, false, 8>
-                                : sd == 16 ? vq::k_lbg_update_small<true, false, 16>
-                                           : vq::k_lbg_update_small<true>),
-                               dim3(groups * m), dim3(vq::kSmallThreads),
-                               sizeof(float) * vq::kSmallStage, st, S, it, m, d_x, n, ld, sd, k, C, groups,
-                               (const uint32_t *)reseed, n_reseed, d_codebooks);
-        else
-            hipLaunchKernelGGL(vq::k_lbg_update_small<false>, dim3(groups * m), dim3(vq::kSmallThreads),
-                               sizeof(float) * 3 * C * sd, st, S, it, m, d_x, n, ld, sd, k, C, groups,
-                               (const uint32_t *)reseed, n_reseed, d_codebooks);
+        const unsigned wgs = (unsigned)groups * m * tiles;
+        const size_t lds = sizeof(float) * (staged ? vq::kSmallStage : 3 * (size_t)C * sd);
+        const auto kern = !staged       ? vq::k_lbg_update_small<false>
+                          : width == 8  ? vq::k_lbg_update_small<true, false, 8>
+                          : width == 16 ? (defer ? vq::k_lbg_update_small<true, true, 16> : vq::k_lbg_update_small<true, false, 16>)
+                          : width == 32 ? (defer ? vq::k_lbg_update_small<true, true, 32> : vq::k_lbg_update_small<true, false, 32>)
+                                        : (defer ? vq::k_lbg_update_small<true, true> : vq::k_lbg_update_small<true>);
+        hipLaunchKernelGGL(kern, dim3(wgs), dim3(vq::kSmallThreads), lds, st, S, it, m, d_x, n, ld, sd, tiles, k, C, groups,
+                           (const uint32_t *)reseed, n_reseed, d_codebooks);
+        const int whole = std::min(most_large, 16);
+        if (defer)
+            hipLaunchKernelGGL(width == 16 ? vq::k_lbg_large<16> : width == 32 ? vq::k_lbg_large<32> : vq::k_lbg_large<0>, dim3(nparts, whole + (tiles > 1 ? tiles : 0)),
+                               dim3(vq::kSmallThreads), lds, st, S, it, d_x, n, ld, sd, k, whole, d_codebooks);
     }
     last();
     hipLaunchKernelGGL(vq::k_lbg_small_report, dim3(1), dim3(256), 0, st, (const int *)S.changed, (int)n_flags, report);
