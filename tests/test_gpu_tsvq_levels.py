@@ -25,6 +25,8 @@ def ctx():
     (6000, 17, 12, "copies"), (257, 20, 1, "normal"), (5, 2, 3, "copies"), (9000, 33, 9, "copies"),
     # a chain's chunks of 336 members (16 components) and the ends of its two stages, three components, a last tile that overlaps
     (335, 16, 1, "normal"), (336, 16, 1, "normal"), (337, 16, 1, "normal"), (672, 16, 1, "normal"), (1009, 20, 1, "normal"), (900, 3, 1, "normal"),
+    # the longest nodes: sixteen leaves, 68 KB of LDS for the split
+    (16_384, 100, 6, "normal"), (16_385, 100, 4, "normal"), (16_384, 96, 5, "lopsided"), (8193, 50, 5, "lopsided"),
     # more workgroups than a round: tiles of up to 32 components, nodes of some hundred rows and of two leaves
     (30_000, 256, 7, "normal"), (40_000, 100, 8, "normal"), (26_000, 250, 6, "lopsided"), (90_000, 130, 6, "normal"),
 ])

@@ -1136,10 +1136,10 @@ static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__
 // is {0, 0}.  Every launch covers all slots of its level; the host reads the decisions of all levels at once and
 // numbers the nodes.  (A level that waits for the host costs two copies, the wait and the time until its first kernel
 // starts, 30 us on a level of 70-100, and its means were three launches where they are one or two.  Builds: 2,295 x 128, seven levels 391 -> 247 us,
-// 4,157 x 100, ten 614 -> 404, 12,557 x 96, six 507 -> 414, 100,000 x 128, ten 1284 -> 1171.)  The host knows no node's
+// 4,157 x 100, ten 614 -> 404, 12,557 x 96, six 507 -> 343, 100,000 x 128, ten 1284 -> 1083.)  The host knows no node's
 // size here, only the longest one's above: what a launch is sized for is the balanced tree's, and a longer node
 // (equal values all go left) takes more rounds of the same loops.
-constexpr int kNodeLeaves = 8;  // leaves of 1024 rows of the longest node
+constexpr int kNodeLeaves = 16;  // leaves of 1024 rows of the longest node
 
 // Rows lo .. hi - 1 (of cnt) of leaf l, by the midpoints of src/vector.rs's recursion.
 __device__ __forceinline__ uint2 leaf_range(uint32_t cnt, int dep, uint32_t l) {

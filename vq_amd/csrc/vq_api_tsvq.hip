@@ -234,10 +234,11 @@ int32_t vq_tsvq_build_kmeans(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
 }
 
 // Levels whose longest node is no longer than this: a workgroup per node and 16 columns (k_seg_variance_tile, one launch,
-// 7 ns per row of the longest node) instead of the composed maps (four launches, 45 us and what the columns take).  Builds
-// with 4096 / 8192 / 16,384 rows: 100,000 x 16 641 / 661 / 675 us, 40,000 x 96 692 / 690 / 707, 220,611 x 128 1624 / 1567 / 1556,
-// 60,000 x 256 1064 / 1050 / 1065.
-static uint32_t var_tile_rows(int32_t dim) { return dim >= 96 ? 8192 : 4096; }
+// 4 ns per row of the longest node) and no wait for the host, instead of the composed maps (four launches, 45 us and what the
+// columns take).  Half as many rows -> as many: 7,000 x 50, six levels 326 -> 279 us, 6,000 x 16, eight 311 -> 291, 12,557 x 96, six
+// 370 -> 343, 16,000 x 100, six 435 -> 407, 100,000 x 128, ten 1108 -> 1083, 500,000 x 64, ten 2027 -> 1921, 1,000,000 x 128, ten
+// 4821 -> 4585; 30,000 x 64, ten 660 -> 665.
+static uint32_t var_tile_rows(int32_t dim) { return dim >= 96 ? 16384 : 8192; }
 
 // The columns that the composed maps take: their grids have a workgroup per four of them in y.
 constexpr int32_t kMapColumns = 4 * 65535;
@@ -447,7 +448,11 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
             }
             if (d == D) break;
             const uint32_t room = std::min(longest, usual + usual / 8 + 64);
-            hipLaunchKernelGGL(vq::k_node_split, dim3((unsigned)ns), dim3(usual > 1024 ? 1024u : 256u), vq::split_wg_lds(room), st, perm, r, room,
+            const size_t split_lds = vq::split_wg_lds(room);
+            if (split_lds > 48 * 1024)
+                VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_node_split),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_lds));
+            hipLaunchKernelGGL(vq::k_node_split, dim3((unsigned)ns), dim3(usual > 1024 ? 1024u : 256u), split_lds, st, perm, r, room,
                                (const float *)d_var, real_dim, dim, d_x, ld, (uint32_t *)vals, d_sdim + o, d_median + o, d_nleft + o, perm2,
                                d_range + o + ns);
             std::swap(perm, perm2);
