@@ -168,3 +168,17 @@ def test_blocks_whose_only_change_is_an_undecided_pair(ctx, n, m, sd, k):
     assert np.all(want["iters"] == 3)
     assert np.array_equal(iters, want["iters"]) and np.array_equal(used, want["reseeds"])
     assert np.array_equal(dcb.download().view(np.uint32), want["codebooks"].view(np.uint32))
+
+
+# rounds of 16,384 rows (64 compute units per column block): tiles of the last one dealt to all workgroups below half a round, and a
+# workgroup's eight side by side beyond; one tile more than whole rounds, one row more than a tile
+@pytest.mark.parametrize("n", [32_768, 32_769, 33_000, 40_928, 40_960, 40_961, 49_151])
+def test_last_round_of_tiles(n):
+    import vq_amd
+    ctx = vq_amd.Context(0)
+    rng = np.random.default_rng(n)
+    x, cb = rng.random((n, 256), dtype=np.float32), rng.random((4, 256, 64), dtype=np.float32)
+    codes = ctx.empty((n, 4), np.uint8)
+    ctx.assign(O.EUCLIDEAN, ctx.to_device(x), n, 256, 4, 64, 256, ctx.to_device(cb), codes)
+    assert np.array_equal(codes.download(), O.pq_encode(O.EUCLIDEAN, x, cb).astype(np.uint8))
+    ctx.close()
