@@ -69,16 +69,26 @@ __global__ void __launch_bounds__(256) k_decode_units(const CodeT *__restrict__ 
     using OutT = typename std::conditional<F16, uint16_t, float>::type;
     constexpr int RUN = 256 * U * UNIT;
     const int64_t blocks = n * m, total = blocks * sd, first = (int64_t)blockIdx.x * RUN;
-    const int64_t b0 = total <= 0xFFFFFFFFll ? (uint32_t)first / (uint32_t)sd : first / sd;  // uniform
-    const uint32_t t0 = (uint32_t)(first - b0 * sd), s0 = total <= 0xFFFFFFFFll ? (uint32_t)b0 % (uint32_t)m : (uint32_t)(b0 % m);
-    const CodeT *run = codes + b0;
     const float *src[U];
+    if (m == 1 && total <= 0xFFFFFFFFll) {  // the rows of a tree: one division on the way to the code (20,000 x 100 with its descent 25.4 -> 24.8 us)
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-        uint32_t e = t0 + (threadIdx.x + 256u * u) * UNIT;
-        if (first + (threadIdx.x + 256u * u) * UNIT >= total) e = t0;  // (not stored)
-        const uint32_t b = e / (uint32_t)sd, t = e - b * (uint32_t)sd, s = s0 + b;
-        src[u] = cb + ((size_t)(s - s / (uint32_t)m * (uint32_t)m) * k + (size_t)run[b]) * sd + t;
+        for (int u = 0; u < U; ++u) {
+            uint32_t e = (uint32_t)first + (threadIdx.x + 256u * u) * UNIT;
+            if (first + (threadIdx.x + 256u * u) * UNIT >= total) e = (uint32_t)first;  // (not stored)
+            const uint32_t b = e / (uint32_t)sd;
+            src[u] = cb + (size_t)codes[b] * sd + (e - b * (uint32_t)sd);
+        }
+    } else {
+        const int64_t b0 = total <= 0xFFFFFFFFll ? (uint32_t)first / (uint32_t)sd : first / sd;  // uniform
+        const uint32_t t0 = (uint32_t)(first - b0 * sd), s0 = total <= 0xFFFFFFFFll ? (uint32_t)b0 % (uint32_t)m : (uint32_t)(b0 % m);
+        const CodeT *run = codes + b0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            uint32_t e = t0 + (threadIdx.x + 256u * u) * UNIT;
+            if (first + (threadIdx.x + 256u * u) * UNIT >= total) e = t0;  // (not stored)
+            const uint32_t b = e / (uint32_t)sd, t = e - b * (uint32_t)sd, s = s0 + b;
+            src[u] = cb + ((size_t)(s - s / (uint32_t)m * (uint32_t)m) * k + (size_t)run[b]) * sd + t;
+        }
     }
     typedef float fv __attribute__((ext_vector_type(UNIT == 1 ? 2 : UNIT)));  // (of two, one is used where UNIT is 1)
     fv v[U];
