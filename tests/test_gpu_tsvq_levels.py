@@ -29,12 +29,21 @@ def ctx():
     (16_384, 100, 6, "normal"), (16_385, 100, 4, "normal"), (16_384, 96, 5, "lopsided"), (8193, 50, 5, "lopsided"),
     # more workgroups than a round: tiles of up to 32 components, nodes of some hundred rows and of two leaves
     (30_000, 256, 7, "normal"), (40_000, 100, 8, "normal"), (26_000, 250, 6, "lopsided"), (90_000, 130, 6, "normal"),
+    # levels that end because a node is longer than three times a balanced tree's: once and again, at the last level of the tree,
+    # one above it, an odd and an even number of levels early, many nodes above them, three components
+    (16_384, 100, 9, "one of fifty"), (9000, 100, 2, "one of fifty"), (9000, 100, 3, "one of fifty"), (8000, 96, 4, "one of fifty"), (5000, 17, 5, "one of fifty"),
+    (8192, 3, 10, "one of fifty"), (60_000, 130, 8, "one of fifty"), (6000, 24, 7, "even above"), (6001, 24, 8, "even above"),
 ])
 def test_levels_on_device(ctx, n, dim, depth, kind):
     rng = np.random.default_rng(17 * n + dim)
     x = rng.standard_normal((n, dim)).astype(F)
     if kind == "lopsided":  # every column: four rows of five share the least value, which is the median
         x = np.where(rng.random((n, dim)) < 0.8, F(0.0), np.abs(x) * F(10) + F(1)).astype(F) * np.arange(1, dim + 1, dtype=F)
+    elif kind == "one of fifty":  # a node loses one row in fifty per level
+        x = np.where(rng.random((n, dim)) < 0.98, F(0.0), np.abs(x) + F(1)).astype(F)
+    elif kind == "even above":  # three balanced levels, then equal values
+        x = np.where(rng.random((n, dim)) < 0.9, F(0.0), F(1.0)).astype(F) * np.arange(1, dim + 1, dtype=F) * F(0.01)
+        x[:, :3] = rng.standard_normal((n, 3)) * [400, 200, 100]
     elif kind == "copies":  # few distinct rows: nodes of equal rows have no children
         x = x[rng.integers(0, min(n, 9), n)]
     got = ctx.tsvq_build(ctx.to_device(x), n, dim, dim, depth).download()

@@ -1135,10 +1135,13 @@ static __global__ void __launch_bounds__(1024) k_seg_split_wg(const uint32_t *__
 // level d are the slots of a complete tree (children of slot g: 2 g and 2 g + 1 of the next table), a slot without a node
 // is {0, 0}.  Every launch covers all slots of its level; the host reads the decisions of all levels at once and
 // numbers the nodes.  (A level that waits for the host costs two copies, the wait and the time until its first kernel
-// starts, 30 us on a level of 70-100, and its means were three launches where they are one or two.  Builds: 2,295 x 128, seven levels 391 -> 247 us,
-// 4,157 x 100, ten 614 -> 404, 12,557 x 96, six 507 -> 343, 100,000 x 128, ten 1284 -> 1083.)  The host knows no node's
+// starts, 30 us on a level of 70-100, and its means were three launches where they are one or two.  Builds: 2,295 x 128, seven levels 398 -> 226 us,
+// 4,157 x 100, ten 625 -> 361, 16,000 x 100, ten 871 -> 550, 100,000 x 128, ten 1268 -> 1088.)  The host knows no node's
 // size here, only the longest one's above: what a launch is sized for is the balanced tree's, and a longer node
-// (equal values all go left) takes more rounds of the same loops.
+// (equal values all go left) takes more rounds of the same loops.  Where that would be many (kUneven), the split of the level
+// above sets the level's word of stop: its kernels and those of the levels below return, and the host takes up there with
+// the true length.  (A tree that ends early pays for the launches of its empty levels: thirteen levels of 2,000 rows of which three
+// differ 170 -> 220 us, ten of 16,000 of which nine differ 573 -> 490.)
 constexpr int kNodeLeaves = 16;  // leaves of 1024 rows of the longest node
 
 // Rows lo .. hi - 1 (of cnt) of leaf l, by the midpoints of src/vector.rs's recursion.
@@ -1163,14 +1166,16 @@ __device__ __forceinline__ int leaf_depth(uint32_t cnt) {
 // Sums of the leaves of a level's nodes, a workgroup per (node, one of every `per` leaves, tile of up to 32 components, as
 // k_node_stats has them): leaf_sum[(node * kNodeLeaves + leaf) * dim + component].
 template <int VEC, bool CHAIN>
-static __global__ void __launch_bounds__(256) k_node_leafsum(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, int slots,
-                                                             int per, const float *__restrict__ x, int64_t ld, int dim, int width,
-                                                             int pieces, float *__restrict__ leaf_sum) {
+static __global__ void __launch_bounds__(256) k_node_leafsum(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range,
+                                                             const uint32_t *__restrict__ stop, int slots, int per,
+                                                             const float *__restrict__ x, int64_t ld, int dim, int width, int pieces,
+                                                             float *__restrict__ leaf_sum) {
     extern __shared__ float4 lds_node[];
     const int g = blockIdx.x % (unsigned)slots, rest = blockIdx.x / (unsigned)slots, tile = rest / per;
     const int c0 = tile * width < dim - width ? tile * width : dim - width;
     const uint2 r = range[g];
     const uint32_t cnt = r.y - r.x;
+    if (*stop) return;
     const int dep = leaf_depth(cnt);
     for (uint32_t l = (uint32_t)(rest % per); cnt && l < (1u << dep); l += (uint32_t)per) {
         const uint2 lr = leaf_range(cnt, dep, l);
@@ -1186,7 +1191,8 @@ static __global__ void __launch_bounds__(256) k_node_leafsum(const uint32_t *__r
 // NT threads: 64 for nodes of up to 256 rows, whose chunks of 128 members leave room for more workgroups (the last levels
 // of 100,000 x 128, nodes of 195 and 98 rows: 23 -> 15 us each).
 template <int VEC, bool SUMS, int NT, bool CHAIN>
-static __global__ void __launch_bounds__(NT) k_node_stats(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, int slots,
+static __global__ void __launch_bounds__(NT) k_node_stats(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range,
+                                                           const uint32_t *__restrict__ stop, int slots,
                                                            const float *__restrict__ x, int64_t ld, int dim, int width, int pieces,
                                                            const float *__restrict__ leaf_sum, float *__restrict__ means,
                                                            float *__restrict__ var) {
@@ -1197,7 +1203,7 @@ static __global__ void __launch_bounds__(NT) k_node_stats(const uint32_t *__rest
     const int c0 = tile * width < dim - width ? tile * width : dim - width;
     const uint2 r = range[g];
     const uint32_t cnt = r.y - r.x;
-    if (cnt == 0) return;
+    if (*stop || cnt == 0) return;
     const int dep = leaf_depth(cnt);
     const uint32_t nl = 1u << dep;
     for (uint32_t l = 0; l < nl; ++l) {
@@ -1226,8 +1232,9 @@ static __global__ void __launch_bounds__(NT) k_node_stats(const uint32_t *__rest
 
 // k_seg_split_wg for the slots of a level; the children's positions go into the next level's table.  room: rows whose keys the
 // workgroup's LDS holds; a longer node's keys lie in memory (keys, by position).  nleft stays 0 where nothing is split.
-static __global__ void __launch_bounds__(1024) k_node_split(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, uint32_t room,
-                                                            const float *__restrict__ var, int dim, int stride,
+// most: rows of a child above which the next level stops (*stop: this level has).
+static __global__ void __launch_bounds__(1024) k_node_split(const uint32_t *__restrict__ perm, const uint2 *__restrict__ range, uint32_t *stop,
+                                                            uint32_t room, uint32_t most, const float *__restrict__ var, int dim, int stride,
                                                             const float *__restrict__ x, int64_t ld, uint32_t *__restrict__ keys,
                                                             int *__restrict__ split_dim, float *__restrict__ median,
                                                             uint32_t *__restrict__ nleft, uint32_t *__restrict__ perm_out,
@@ -1237,6 +1244,10 @@ static __global__ void __launch_bounds__(1024) k_node_split(const uint32_t *__re
     const int g = blockIdx.x;
     const uint2 r = range[g];
     const uint32_t cnt = r.y - r.x;
+    if (*stop) {
+        if (g == 0 && threadIdx.x == 0) stop[1] = 1u;
+        return;
+    }
     uint32_t nl = 0;
     const float *v = var + (size_t)g * stride;
     if (cnt >= 2 && cnt <= room)
@@ -1246,6 +1257,7 @@ static __global__ void __launch_bounds__(1024) k_node_split(const uint32_t *__re
     if (threadIdx.x == 0) {
         const bool both = nl > 0 && nl < cnt;  // (no child holds all rows)
         if (cnt < 2) nleft[g] = 0u;
+        if (both && (nl > cnt - nl ? nl : cnt - nl) > most) stop[1] = 1u;
         child[2 * g] = both ? make_uint2(r.x, r.x + nl) : make_uint2(0u, 0u);
         child[2 * g + 1] = both ? make_uint2(r.x + nl, r.y) : make_uint2(0u, 0u);
     }

@@ -240,6 +240,14 @@ int32_t vq_tsvq_build_kmeans(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
 // 4821 -> 4585; 30,000 x 64, ten 660 -> 665.
 static uint32_t var_tile_rows(int32_t dim) { return dim >= 96 ? 16384 : 8192; }
 
+// Levels on the device end before one whose longest node has more than kUnevenRows rows and kUneven times those of a balanced
+// tree, for which its launches are sized; the next ones start from the node's true length, as many at a time as were built, until
+// they are even again.  16,000 x 100, ten levels (before levels on the device / without this line / with it): 80 % zeros 1358 / 1406 / 1232 us, 90 %
+// 1658 / 2318 / 1645, 98 % 1936 / 3581 / 2042 (the first launches that are for nothing); 8000 x 50, 98 % 1330 / 1813 / 1174, 5000 x 64 1077 / 1228 / 852,
+// 2000 x 20, 80 % 557 / 411 / 394; balanced 100,000 x 128 1268 / 1120 / 1088, 16,000 x 100 877 / 564 / 553.  Twice the rows of a balanced tree: the
+// same; four times: 98 % 2107; from 256 rows on 2000 x 20 476, from 2048 on 2000 x 20, 98 % 606 -> 661.
+constexpr uint32_t kUneven = 3, kUnevenRows = 1024;
+
 // The columns that the composed maps take: their grids have a workgroup per four of them in y.
 constexpr int32_t kMapColumns = 4 * 65535;
 
@@ -378,6 +386,7 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
     };
     // Levels of short nodes without the host between them (k_node_stats, k_node_split): as many as their tables
     // take at once, then the host numbers the nodes.  Sets done, or leaves level and depth_left at the first level not built.
+    int level_cap = 64;  // levels at a time while the nodes are uneven
     auto device_levels = [&](bool &ran, bool &done) -> int32_t {
         const int nseg = (int)level.size(), first_node = level[0].node;
         uint32_t longest = 0;
@@ -386,37 +395,44 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
         // the slots of the last level, and what they take
         const int64_t most = std::max<int64_t>(4096, 4 * (int64_t)nseg);
         int D = 0;
-        while (D < depth_left && ((int64_t)nseg << (D + 1)) <= most && ((int64_t)nseg << (D + 2)) * dim <= (16 << 20)) ++D;
+        while (D < depth_left && D < level_cap && ((int64_t)nseg << (D + 1)) <= most && ((int64_t)nseg << (D + 2)) * dim <= (16 << 20)) ++D;
         if (D < std::min(depth_left, 2)) return VQ_OK;
         const size_t last = (size_t)nseg << D, inner = last - nseg, slots = inner + last;  // (nseg (2^D - 1), and with the last level's)
         int leafy = 0;  // levels whose leaves are summed ahead
         while (leafy <= D && (longest >> leafy) > (uint32_t)kLeafMaxRows) ++leafy;
         const bool direct = (uint64_t)first_node + slots <= max_nodes;  // (slots without a node may exceed the arena)
-        const size_t sizes[5] = {sizeof(uint2) * slots, 3 * sizeof(uint32_t) * inner, sizeof(float) * (inner ? last / 2 : 0) * dim,
+        // decisions (split dimensions, medians, left counts), the levels' stops and the nodes' rows: what comes back and what goes up
+        // are one run each
+        const size_t down = (3 * inner + 1) / 2 * 2, stops = 64;
+        const size_t sizes[4] = {sizeof(uint32_t) * (down + stops) + sizeof(uint2) * slots, sizeof(float) * (inner ? last / 2 : 0) * dim,
                                  leafy ? sizeof(float) * vq::kNodeLeaves * ((size_t)nseg << (leafy - 1)) * dim : 0,
                                  direct ? 0 : sizeof(float) * slots * dim};
         size_t total = 0;
         for (size_t z : sizes) total += pad(z);
         VQ_TRY(ensure(ctx, ctx->tsvq_level, total));
-        VQ_TRY(pinned(std::max(sizes[1], sizeof(uint2) * (size_t)nseg)));
-        char *at[5], *p = (char *)ctx->tsvq_level.p;
-        for (int z = 0; z < 5; ++z) {
+        VQ_TRY(pinned(sizeof(uint32_t) * stops + std::max(sizeof(uint32_t) * down, sizeof(uint2) * (size_t)nseg)));
+        char *at[4], *p = (char *)ctx->tsvq_level.p;
+        for (int z = 0; z < 4; ++z) {
             at[z] = p;
             p += pad(sizes[z]);
         }
-        uint2 *d_range = (uint2 *)at[0], *h_range = (uint2 *)ctx->tsvq_pin;
-        int *d_sdim = (int *)at[1];
-        float *d_median = (float *)d_sdim + inner, *d_var = (float *)at[2], *d_lsum = (float *)at[3];
-        uint32_t *d_nleft = (uint32_t *)d_sdim + 2 * inner;
-        float *d_means = direct ? (float *)ctx->tsvq_means.p + (size_t)first_node * dim : (float *)at[4];
+        int *d_sdim = (int *)at[0];
+        float *d_median = (float *)d_sdim + inner, *d_var = (float *)at[1], *d_lsum = (float *)at[2];
+        uint32_t *d_nleft = (uint32_t *)d_sdim + 2 * inner, *d_stop = (uint32_t *)d_sdim + down;
+        uint2 *d_range = (uint2 *)(d_stop + stops), *h_range = (uint2 *)((uint32_t *)ctx->tsvq_pin + stops);
+        float *d_means = direct ? (float *)ctx->tsvq_means.p + (size_t)first_node * dim : (float *)at[3];
+        memset(ctx->tsvq_pin, 0, sizeof(uint32_t) * stops);
         for (int g = 0; g < nseg; ++g) h_range[g] = make_uint2(level[g].lo, level[g].hi);
-        VQ_HIP(ctx, hipMemcpyAsync(d_range, h_range, sizeof(uint2) * (size_t)nseg, hipMemcpyHostToDevice, st));
+        VQ_HIP(ctx, hipMemcpyAsync(d_stop, ctx->tsvq_pin, sizeof(uint32_t) * stops + sizeof(uint2) * (size_t)nseg, hipMemcpyHostToDevice, st));
+        const auto expected = [&](int d) { return std::max(longest >> d, 1u); };
+        const auto stops_above = [&](int d) { return std::max(kUnevenRows, kUneven * expected(d)); };
         for (int d = 0; d <= D; ++d) {
             if (d == D && D < depth_left) break;  // the next call's first level
             const size_t o = ((size_t)nseg << d) - nseg;
             const int ns = nseg << d;
-            const uint32_t usual = std::max(longest >> d, 1u);
+            const uint32_t usual = expected(d);
             const uint2 *r = d_range + o;
+            const uint32_t *stop = d_stop + d;
             float *means = d_means + o * dim, *var = d < D ? d_var : nullptr;
             const dim3 block(256);
             const bool chain2 = (int64_t)ns * narrow.count <= vq::kChainGroups;
@@ -427,11 +443,11 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                 const Tiles &t = chain ? narrow : broad;
                 hipLaunchKernelGGL((vec == 4 ? (chain ? vq::k_node_leafsum<4, true> : vq::k_node_leafsum<4, false>)
                                              : (chain ? vq::k_node_leafsum<1, true> : vq::k_node_leafsum<1, false>)),
-                                   dim3((unsigned)((int64_t)ns * t.count * per)), block, tile_lds(t, 256, chain), st, perm, r, ns, per, d_x, ld,
+                                   dim3((unsigned)((int64_t)ns * t.count * per)), block, tile_lds(t, 256, chain), st, perm, r, stop, ns, per, d_x, ld,
                                    dim, t.width, t.pieces, d_lsum);
                 hipLaunchKernelGGL((vec == 4 ? (chain2 ? vq::k_node_stats<4, false, 256, true> : vq::k_node_stats<4, false, 256, false>)
                                              : (chain2 ? vq::k_node_stats<1, false, 256, true> : vq::k_node_stats<1, false, 256, false>)),
-                                   dim3((unsigned)((int64_t)ns * t2.count)), block, tile_lds(t2, 256, chain2), st, perm, r, ns, d_x, ld, dim,
+                                   dim3((unsigned)((int64_t)ns * t2.count)), block, tile_lds(t2, 256, chain2), st, perm, r, stop, ns, d_x, ld, dim,
                                    t2.width, t2.pieces, (const float *)d_lsum, means, var);
             } else {
                 // (a wave, or the usual workgroup, or that with its chains)
@@ -443,7 +459,7 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                                            : (kind == 0   ? vq::k_node_stats<1, true, 64, false>
                                               : kind == 1 ? vq::k_node_stats<1, true, 256, false>
                                                           : vq::k_node_stats<1, true, 256, true>);
-                hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)ns * t.count)), dim3(threads), tile_lds(t, threads, kind == 2), st, perm, r,
+                hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)ns * t.count)), dim3(threads), tile_lds(t, threads, kind == 2), st, perm, r, stop,
                                    ns, d_x, ld, dim, t.width, t.pieces, (const float *)nullptr, means, var);
             }
             if (d == D) break;
@@ -452,25 +468,30 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
             if (split_lds > 48 * 1024)
                 VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_node_split),
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_lds));
-            hipLaunchKernelGGL(vq::k_node_split, dim3((unsigned)ns), dim3(usual > 1024 ? 1024u : 256u), split_lds, st, perm, r, room,
-                               (const float *)d_var, real_dim, dim, d_x, ld, (uint32_t *)vals, d_sdim + o, d_median + o, d_nleft + o, perm2,
+            hipLaunchKernelGGL(vq::k_node_split, dim3((unsigned)ns), dim3(usual > 1024 ? 1024u : 256u), split_lds, st, perm, r, d_stop + d, room,
+                               stops_above(d + 1), (const float *)d_var, real_dim, dim, d_x, ld, (uint32_t *)vals, d_sdim + o, d_median + o, d_nleft + o, perm2,
                                d_range + o + ns);
             std::swap(perm, perm2);
         }
         VQ_HIP(ctx, hipGetLastError());
-        VQ_HIP(ctx, hipMemcpyAsync(ctx->tsvq_pin, d_sdim, sizes[1], hipMemcpyDeviceToHost, st));
+        VQ_HIP(ctx, hipMemcpyAsync(ctx->tsvq_pin, d_sdim, sizeof(uint32_t) * (down + stops), hipMemcpyDeviceToHost, st));
         VQ_HIP(ctx, hipStreamSynchronize(st));
         const int *sdim = (const int *)ctx->tsvq_pin;
         const float *median = (const float *)sdim + inner;
-        const uint32_t *nleft = (const uint32_t *)sdim + 2 * inner;
+        const uint32_t *nleft = (const uint32_t *)sdim + 2 * inner, *stopped = (const uint32_t *)sdim + down;
+        int built = 0;  // levels split (the first one always is)
+        while (++built < D && !stopped[built]) {}
+        const bool ends = D == depth_left && built == D && !stopped[D];  // the last level's means are there
+        if ((D - built) % 2) std::swap(perm, perm2);
+        level_cap = stopped[built] ? std::max(built, 2) : 64;
         // the nodes, level by level, as the loop below numbers them (src/tsvq.rs:126-141)
         std::vector<uint32_t> slot(nseg), from;  // of the level's nodes; of all nodes with means, in node order
         for (int g = 0; g < nseg; ++g) slot[g] = (uint32_t)g;
         for (int d = 0;; ++d) {
             const size_t o = ((size_t)nseg << d) - nseg;
-            if (d < D || D == depth_left)
+            if (d < built || ends)
                 for (uint32_t g : slot) from.push_back((uint32_t)o + g);
-            if (d == D) break;
+            if (d == built) break;
             std::vector<Seg> next;
             std::vector<uint32_t> next_slot;
             for (size_t i = 0; i < level.size(); ++i) {
@@ -517,8 +538,8 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
         }
         level_means.push_back({(float *)ctx->tsvq_means.p + (size_t)first_node * dim, first_node, (int)from.size()});
         ran = true;
-        done = level.empty() || D == depth_left;
-        depth_left -= D;
+        done = level.empty() || ends;
+        depth_left -= built;
         return VQ_OK;
     };
 
