@@ -75,7 +75,9 @@ def test_small_fit_cluster_sizes(ctx, sd, m, largest):
 
 
 @pytest.mark.parametrize("n,m,sd,k", [(12_000, 1, 36, 64), (12_289, 2, 36, 200), (12_000, 1, 100, 64), (12_288, 1, 300, 256), (10_000, 1, 512, 256),
-                                      (8192, 1, 48, 30), (8193, 2, 52, 60), (12_000, 20, 48, 100), (32_768, 1, 40, 200), (32_769, 1, 40, 200)])
+                                      (8192, 1, 48, 30), (8193, 2, 52, 60), (12_000, 20, 48, 100), (32_768, 1, 40, 200), (32_769, 1, 40, 200),
+                                      # several blocks: the line rises with the number of clusters
+                                      (36_000, 3, 36, 100), (36_001, 3, 36, 100), (39_872, 4, 64, 256), (39_873, 4, 64, 256), (50_041, 2, 48, 256), (32_769, 2, 100, 200)])
 def test_small_fit_tiles(ctx, n, m, sd, k):
     """Blocks above 32 floats by tiles whose last one overlaps (or whole, where there are many): clusters on both sides
     of the size from which each part's members are added by tiles too, and one that is re-seeded."""

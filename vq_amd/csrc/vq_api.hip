@@ -1353,13 +1353,17 @@ static int lbg_small_width(int m, int sd, int k) {
 // Blocks above 32 floats: a block that is the whole row is a stage of a residual fit, whose rows gather in a few clusters, and every
 // workgroup lists all rows.  Three stages of five iterations, other path -> this one: k = 256, 30,000 x 64 1077 -> 994 us,
 // 45,000 1175 -> 1171, 65,000 1186 -> 1625, 130,000 1320 -> 3915; 20,000 x 128 1097 -> 1002, 40,000 1196 -> 1471; 16,000 x 256
-// 1314 -> 1276, 24,000 1332 -> 1533; k = 63, 16,000 x 96 1054 -> 1064.  Five iterations, k = 256: 40,000 x 2 of 48 393 -> 353, 80,000
-// 472 -> 663; 40,000 x 8 of 40 645 -> 660.  Narrower rows likewise, three stages, k = 256: 40,000 x 32 959 -> 933, 80,000 1058 -> 1321,
+// 1314 -> 1276, 24,000 1332 -> 1533; k = 63, 16,000 x 96 1054 -> 1064.  Of several wide blocks the rows spread over the clusters, and the
+// line rises with k.  Fit of five iterations and encode: two blocks of 48, k = 256 33,000 rows 400 -> 345, 40,000 393 -> 358, 48,000 404 -> 385,
+// 65,000 468 -> 508, k = 128 36,000 364 -> 356, 44,000 371 -> 395; three of 36, k = 180 36,000 424 -> 396, 44,000 448 -> 434, k = 100 33,000 429 -> 388,
+// 40,000 423 -> 439; four of 64, k = 256 36,000 465 -> 439, 44,000 495 -> 502, k = 180 33,000 466 -> 447, 36,000 467 -> 499; two of 96, k = 256 36,000
+// 435 -> 404, 44,000 457 -> 520; two of 128, k = 256 33,000 498 -> 513, 40,000 492 -> 523.  Narrower rows likewise, three stages, k = 256: 40,000 x 32 959 -> 933, 80,000 1058 -> 1321,
 // 130,000 1152 -> 1920; 40,000 x 24 954 -> 827, 80,000 1047 -> 1291; 80,000 x 16 875 -> 816, 130,000 930 -> 1201.
 static bool lbg_small(int64_t n, int m, int sd, int k) {
     if (sd % 4 != 0 || sd > 4096 || n > 131072) return false;
     if (sd > vq::kSmallThreads) return n <= 128 * (int64_t)k;
-    if (sd > 32 ? n > 32768 : m == 1 && sd >= 16 && n > (sd > 16 ? 45056 : 90112)) return false;
+    const int64_t wide = m == 1 || sd > 96 ? 0 : sd <= 48 ? 27000 + 90 * (int64_t)k : 24000 + 62 * (int64_t)k;
+    if (sd > 32 ? n > std::max<int64_t>(32768, wide) : m == 1 && sd >= 16 && n > (sd > 16 ? 45056 : 90112)) return false;
     return n <= 640 * (int64_t)k && n * lbg_small_clusters(m, sd, k) * sd <= (sd <= 32 ? 57344 : m == 1 ? 20480 : 40960) * (int64_t)k;
 }
 
