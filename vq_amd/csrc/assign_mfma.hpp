@@ -1782,10 +1782,12 @@ __global__ void __launch_bounds__(kWideResThreads, 2) k_assign_mfma_wide_res(Ass
     __syncthreads();
 
     const int64_t ntiles = (a.n + 31) / 32, step_tiles = (int64_t)gridDim.x * 8;
-    // Where less than half of the waves have a tile in the last round, those tiles lie on all compute units and not eight on a
-    // few: encode of 200,000 x 128, k = 256, four stages (3.05 rounds) 340 -> 328 us, 100,000 x 4 blocks of 64 73 -> 70, a residual fit of 1M x 256
-    // (15.26) 45.36 -> 45.07 ms.  Beyond, eight neighbouring tiles to a workgroup are the faster ones: 180,000 x 96 (2.75) 1055 against 1068 us.
-    int64_t tile = ntiles % step_tiles * 2 < step_tiles ? (int64_t)wave * gridDim.x + blockIdx.x : (int64_t)blockIdx.x * 8 + wave;
+    // Where some, but less than half, of the waves have a tile in the last round, those tiles lie on all compute units and not
+    // eight on a few: encode of 200,000 x 128, k = 256, four stages (3.05 rounds) 337 -> 325 us, 100,000 x 4 blocks of 64 72.5 -> 70.4; a residual
+    // fit of 1M x 256 (15.26) the same within 0.5 %.  Beyond, eight neighbouring tiles to a workgroup are the faster ones: 180,000 x 96 (2.75)
+    // 1055 against 1068 us; after whole rounds (65,536 to 1,048,576 rows of one to four blocks) both take the same time.
+    const int64_t over = ntiles % step_tiles;
+    int64_t tile = over != 0 && over * 2 < step_tiles ? (int64_t)wave * gridDim.x + blockIdx.x : (int64_t)blockIdx.x * 8 + wave;
     if (tile >= ntiles) return;  // (no barrier follows)
     const char *xs = reinterpret_cast<const char *>(a.x + (int64_t)s * sd);
     const int64_t tile_bytes = 128 * a.ld;
