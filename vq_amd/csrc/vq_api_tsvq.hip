@@ -235,10 +235,10 @@ int32_t vq_tsvq_build_kmeans(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
 
 // Levels whose longest node is no longer than this: a workgroup per node and 16 columns (k_seg_variance_tile, one launch,
 // 4 ns per row of the longest node) and no wait for the host, instead of the composed maps (four launches, 45 us and what the
-// columns take).  Half as many rows -> as many: 7,000 x 50, six levels 326 -> 279 us, 6,000 x 16, eight 311 -> 291, 12,557 x 96, six
-// 370 -> 343, 16,000 x 100, six 435 -> 407, 100,000 x 128, ten 1108 -> 1083, 500,000 x 64, ten 2027 -> 1921, 1,000,000 x 128, ten
-// 4821 -> 4585; 30,000 x 64, ten 660 -> 665.
-static uint32_t var_tile_rows(int32_t dim) { return dim >= 96 ? 16384 : 8192; }
+// columns take).  Half as many rows -> as many: 7,000 x 50, six levels 336 -> 296 us, 6,000 x 16, eight 331 -> 309, 12,557 x 96, six
+// 370 -> 371, 16,000 x 100, six 432 -> 422, 100,000 x 128, ten 1109 -> 1123, 500,000 x 64, ten 1956 -> 1914, 1,000,000 x 128, ten
+// 4769 -> 4531, 30,000 x 64, ten 700 -> 665, 60,000 x 256, ten 1227 -> 1212.  (89 columns are 96 where they are padded.)
+static uint32_t var_tile_rows(int32_t dim) { return dim > 88 ? 16384 : 8192; }
 
 // Levels on the device end before one whose longest node has more than kUnevenRows rows and kUneven times those of a balanced
 // tree, for which its launches are sized; the next ones start from the node's true length, as many at a time as were built, until
