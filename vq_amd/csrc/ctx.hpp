@@ -72,6 +72,7 @@ struct vq_ctx {
     } stage_tables;
     bool lbg_small_lds_set = false;  // dynamic-LDS limit granted to k_lbg_update_small
     int compute_units = 0;       // of the context's GPU (0: not asked for yet)
+    uint32_t decode_flat_set = 0;  // the kernels of launch_decode_any whose dynamic-LDS limit is granted, a bit each
     int decode_lds_set[4] = {0, 0, 0, 0};  // dynamic-LDS limit already granted to the four resident decode kernels
     uint64_t quad_lds_set[2] = {0, 0};  // dynamic-LDS limit granted to k_tsvq_descend_quad without and with its output, a bit per instance
     int tsvq_descend_path = 0;   // 0 = one inner product per node where it decides (cosine, L2), 1 = two distances per node always

@@ -191,9 +191,10 @@ __global__ void __launch_bounds__(1024) k_decode_flat(const CodeT *__restrict__ 
 }
 
 // Widths and alignments that k_decode_gather does not take, launched.  k: entries per block (of a tree: its nodes).
+// lds_set: the caller's, a bit per kernel whose LDS limit has been set.
 template <bool F16, typename CodeT>
-hipError_t launch_decode_any(hipStream_t st, int compute_units, const CodeT *codes, int64_t n, int m, int sd, int k, const float *cb,
-                             void *out) {
+hipError_t launch_decode_any(hipStream_t st, int compute_units, uint32_t &lds_set, const CodeT *codes, int64_t n, int m, int sd, int k,
+                             const float *cb, void *out) {
     const size_t lds = F16 && decode_flat_resident(n, m, sd, k) ? 2 * (size_t)m * k * sd : 0;
     const unsigned lds_groups = (unsigned)compute_units * (lds <= kDecodeFlatLds / 2 ? 2u : 1u);
     const uintptr_t at = reinterpret_cast<uintptr_t>(cb);
@@ -203,9 +204,13 @@ hipError_t launch_decode_any(hipStream_t st, int compute_units, const CodeT *cod
         if constexpr (F16) {
             if (lds) {
                 auto kern = sd >= 8 - UNIT ? k_decode_flat<UNIT, true, CodeT> : k_decode_flat<UNIT, false, CodeT>;
-                const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, kDecodeFlatLds);
-                if (e != hipSuccess) return e;
+                const uint32_t bit = 1u << ((UNIT / 2 * 2 + (sd >= 8 - UNIT ? 1 : 0)) * 3 + sizeof(CodeT) / 2);
+                if (!(lds_set & bit)) {
+                    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                                             hipFuncAttributeMaxDynamicSharedMemorySize, kDecodeFlatLds);
+                    if (e != hipSuccess) return e;
+                    lds_set |= bit;
+                }
                 const int64_t runs = (total + 16383) / 16384;
                 hipLaunchKernelGGL(kern, dim3((unsigned)(runs < lds_groups ? runs : lds_groups)), dim3(1024), lds, st, codes, n, m, sd, k,
                                    cb, (uint16_t *)out);

@@ -730,7 +730,8 @@ int32_t decode_codes(vq_ctx *ctx, const CodeT *d_codes, int64_t n, int32_t m, in
                            ctx->stream, d_codes, n, m, sd, k, d_codebooks, (vq::u32x4_out *)d_out);
     else {
         VQ_TRY(know_compute_units(ctx));
-        VQ_HIP(ctx, (vq::launch_decode_any<F16, CodeT>(ctx->stream, ctx->compute_units, d_codes, n, m, sd, k, d_codebooks, d_out)));
+        VQ_HIP(ctx, (vq::launch_decode_any<F16, CodeT>(ctx->stream, ctx->compute_units, ctx->decode_flat_set, d_codes, n, m, sd, k, d_codebooks,
+                                                       d_out)));
     }
     VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;

@@ -465,9 +465,9 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
             if (d == D) break;
             const uint32_t room = std::min(longest, usual + usual / 8 + 64);
             const size_t split_lds = vq::split_wg_lds(room);
-            if (split_lds > 48 * 1024)
-                VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_node_split),
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_lds));
+            if (split_lds > 48 * 1024)  // (a first level; the same limit in every thread)
+                VQ_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_node_split), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                (int)vq::split_wg_lds(vq::kSplitWgMax)));
             hipLaunchKernelGGL(vq::k_node_split, dim3((unsigned)ns), dim3(usual > 1024 ? 1024u : 256u), split_lds, st, perm, r, d_stop + d, room,
                                stops_above(d + 1), (const float *)d_var, real_dim, dim, d_x, ld, (uint32_t *)vals, d_sdim + o, d_median + o, d_nleft + o, perm2,
                                d_range + o + ns);
@@ -865,7 +865,7 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
             const size_t lds = vq::split_wg_lds(longest);
             if (lds > 48 * 1024)
                 SP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(vq::k_seg_split_wg),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)vq::split_wg_lds(vq::kSplitWgMax)));
             hipLaunchKernelGGL(vq::k_seg_split_wg, dim3((unsigned)ns), dim3(longest > 1024 ? 1024u : 256u), lds, st, perm,
                                (const uint2 *)d_range, (const float *)d_var, real_dim, dim, d_x, ld, d_sdim, d_median, d_nleft, perm2);
             SP_HIP(hipGetLastError());
@@ -1180,8 +1180,8 @@ int32_t vq_tsvq_decode_f16(vq_ctx *ctx, const vq_tree *tree, const int32_t *d_le
                            d_leaf, n, 1, tree->dim, 0, tree->d_centroids, (vq::u32x4_out *)d_out);
     else {
         VQ_TRY(know_compute_units(ctx));
-        VQ_HIP(ctx, (vq::launch_decode_any<true, int32_t>(ctx->stream, ctx->compute_units, d_leaf, n, 1, tree->dim, tree->n_nodes,
-                                                          tree->d_centroids, d_out)));
+        VQ_HIP(ctx, (vq::launch_decode_any<true, int32_t>(ctx->stream, ctx->compute_units, ctx->decode_flat_set, d_leaf, n, 1, tree->dim,
+                                                          tree->n_nodes, tree->d_centroids, d_out)));
     }
     VQ_HIP(ctx, hipGetLastError());
     return VQ_OK;
