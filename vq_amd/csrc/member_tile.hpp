@@ -208,10 +208,9 @@ __device__ __forceinline__ float member_chain_sum(float *stage, const float *__r
 }
 
 // One or the other.  Chains are the faster ones while the workgroups, at 44 KB of LDS for 16 components, are a round of the GPU
-// (kChainGroups); beyond, more fetching threads
-// in each are.  100,000 x 128, the levels of 16, 32 and 64 nodes 28.5 -> 20.6 us on average, of 128 and 256 nodes (1024 and 2048 workgroups) 22.7 -> 28.0;
+// (kChainGroups on a compute unit); beyond, more fetching threads in each are.  100,000 x 128, the levels of 16, 32 and 64 nodes 28.5 -> 20.6 us on average, of 128 and 256 nodes (1024 and 2048 workgroups) 22.7 -> 28.0;
 // 4,157 x 100, of one, two and four nodes 20.2 -> 15.2.
-constexpr int kChainGroups = 768;
+constexpr int kChainGroups = 3;
 template <int NT, int VEC, bool DEV, bool CHAIN, typename RowOf>
 __device__ __forceinline__ float tile_sum(float *stage, const float *__restrict__ xs, int64_t ld, uint32_t lo, uint32_t hi, int width, int pieces,
                                           RowOf row_of, const float *__restrict__ mean = nullptr) {

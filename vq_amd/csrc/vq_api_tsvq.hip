@@ -287,6 +287,8 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                                int32_t max_depth, const KmOpts *km, vq_tree **out) {
     const bool padded = real_dim != dim;
     hipStream_t st = ctx->stream;
+    VQ_TRY(know_compute_units(ctx));
+    const int64_t chain_groups = (int64_t)vq::kChainGroups * ctx->compute_units;
 
     // workspace: two row-id lists, column values, flags, scan
     VQ_TRY(ensure(ctx, ctx->tmp_a, sizeof(uint32_t) * (size_t)n));
@@ -435,11 +437,11 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
             const uint32_t *stop = d_stop + d;
             float *means = d_means + o * dim, *var = d < D ? d_var : nullptr;
             const dim3 block(256);
-            const bool chain2 = (int64_t)ns * narrow.count <= vq::kChainGroups;
+            const bool chain2 = (int64_t)ns * narrow.count <= chain_groups;
             const Tiles &t2 = chain2 ? narrow : broad;
             if (d < leafy) {
                 const int per = 1 << tree_depth(usual);
-                const bool chain = (int64_t)ns * narrow.count * per <= vq::kChainGroups;
+                const bool chain = (int64_t)ns * narrow.count * per <= chain_groups;
                 const Tiles &t = chain ? narrow : broad;
                 hipLaunchKernelGGL((vec == 4 ? (chain ? vq::k_node_leafsum<4, true> : vq::k_node_leafsum<4, false>)
                                              : (chain ? vq::k_node_leafsum<1, true> : vq::k_node_leafsum<1, false>)),
@@ -853,7 +855,7 @@ static int32_t tsvq_build_rows(vq_ctx *ctx, const float *d_x, int64_t n, int64_t
                                    (const float *)d_sq, (const uint2 *)d_range, dim, (float *)d_var);
             }
         } else {
-            const bool chain = (int64_t)ns * narrow.count <= vq::kChainGroups;
+            const bool chain = (int64_t)ns * narrow.count <= chain_groups;
             const Tiles &t = chain ? narrow : broad;
             hipLaunchKernelGGL((vec == 4 ? (chain ? vq::k_seg_variance_tile<4, true> : vq::k_seg_variance_tile<4, false>)
                                          : (chain ? vq::k_seg_variance_tile<1, true> : vq::k_seg_variance_tile<1, false>)),
