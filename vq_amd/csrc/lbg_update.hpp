@@ -805,7 +805,7 @@ static __global__ void __launch_bounds__(256) k_lbg_finalize(LbgState st, const 
 // them in list order (add_members).  The orders of summation are those above: row order up
 // to 1024 members, part sums in part order above.
 // DEFER: clusters above 1024 members are counted and left to k_lbg_large.
-// Blocks above 32 floats (SD 16, 32 and tiles > 1): a workgroup takes a tile of the components of C clusters.  The floats that it
+// Blocks above 32 floats (TILES, of SD 16 or 32): a workgroup takes a tile of the components of C clusters.  The floats that it
 // brings in are those of a whole block of C / tiles clusters, but a stage holds 1024 or 512 members instead of 170 of 96 floats, and a
 // long cluster's are spread over several workgroups: what bounded it was one memory round trip per stage of the longest cluster.
 // An iteration of a residual fit of 6,264 x 96, k = 186 61 -> 49 us, 7,143 x 100, k = 214 87 -> 63; fits, three or four stages of six iterations, of
@@ -959,13 +959,12 @@ __device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
     return v;
 }
 
-template <bool STAGED, bool DEFER = false, int SD = 0>
+template <bool STAGED, bool DEFER = false, int SD = 0, bool TILES = false>
 static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSmall st, int it, int m,
                                                                            const float *__restrict__ x, int64_t n,
-                                                                           int64_t ld, int sub_dim, int tiles, int k,
-                                                                           int C, int groups, const uint32_t *__restrict__ reseed,
-                                                                           int n_reseed, float *__restrict__ cb) {
-    constexpr bool TILES = STAGED && (SD == 16 || SD == 32);
+                                                                           int64_t ld, int sub_dim, int k, int C,
+                                                                           int groups, const uint32_t *__restrict__ reseed,
+                                                                           int n_reseed, float *__restrict__ cb, int tiles) {
     const int sd = SD ? SD : sub_dim, full = TILES ? sub_dim : sd;
     const unsigned id = xcd_contiguous(blockIdx.x, gridDim.x), unit = TILES ? id / (unsigned)tiles : id;  // (tiles of the same rows side by side)
     const int tile = TILES ? (int)(id % (unsigned)tiles) : 0, c0 = tile * sd < full - sd ? tile * sd : full - sd;

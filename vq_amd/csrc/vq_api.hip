@@ -1425,8 +1425,10 @@ static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
                                reinterpret_cast<const void *>(vq::k_lbg_update_small<true, false, 16>),
                                reinterpret_cast<const void *>(vq::k_lbg_update_small<true, false, 32>),
                                reinterpret_cast<const void *>(vq::k_lbg_update_small<true, true>),
-                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, true, 16>),
-                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, true, 32>),
+                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, false, 16, true>),
+                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, false, 32, true>),
+                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, true, 16, true>),
+                               reinterpret_cast<const void *>(vq::k_lbg_update_small<true, true, 32, true>),
                                reinterpret_cast<const void *>(vq::k_lbg_large<0>),
                                reinterpret_cast<const void *>(vq::k_lbg_large<16>),
                                reinterpret_cast<const void *>(vq::k_lbg_large<32>)};
@@ -1447,13 +1449,17 @@ static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
         ProfSpan sp(ctx, VQ_PROF_LBG_UPDATE);
         const unsigned wgs = (unsigned)groups * m * tiles;
         const size_t lds = sizeof(float) * (staged ? vq::kSmallStage : 3 * (size_t)C * sd);
-        const auto kern = !staged       ? vq::k_lbg_update_small<false>
-                          : width == 8  ? vq::k_lbg_update_small<true, false, 8>
-                          : width == 16 ? (defer ? vq::k_lbg_update_small<true, true, 16> : vq::k_lbg_update_small<true, false, 16>)
-                          : width == 32 ? (defer ? vq::k_lbg_update_small<true, true, 32> : vq::k_lbg_update_small<true, false, 32>)
-                                        : (defer ? vq::k_lbg_update_small<true, true> : vq::k_lbg_update_small<true>);
-        hipLaunchKernelGGL(kern, dim3(wgs), dim3(vq::kSmallThreads), lds, st, S, it, m, d_x, n, ld, sd, tiles, k, C, groups,
-                           (const uint32_t *)reseed, n_reseed, d_codebooks);
+        const auto tiled = width == 16 ? (defer ? vq::k_lbg_update_small<true, true, 16, true> : vq::k_lbg_update_small<true, false, 16, true>)
+                                       : (defer ? vq::k_lbg_update_small<true, true, 32, true> : vq::k_lbg_update_small<true, false, 32, true>);
+        const auto kern = !staged    ? vq::k_lbg_update_small<false>
+                          : tiles > 1 ? tiled
+                          : sd == 8   ? vq::k_lbg_update_small<true, false, 8>
+                          : sd == 16  ? vq::k_lbg_update_small<true, false, 16>
+                          : sd == 32  ? vq::k_lbg_update_small<true, false, 32>
+                          : defer     ? vq::k_lbg_update_small<true, true>
+                                      : vq::k_lbg_update_small<true>;
+        hipLaunchKernelGGL(kern, dim3(wgs), dim3(vq::kSmallThreads), lds, st, S, it, m, d_x, n, ld, sd, k, C, groups,
+                           (const uint32_t *)reseed, n_reseed, d_codebooks, tiles);
         const int whole = std::min(most_large, 16);
         if (defer)
             hipLaunchKernelGGL(width == 16 ? vq::k_lbg_large<16> : width == 32 ? vq::k_lbg_large<32> : vq::k_lbg_large<0>, dim3(nparts, whole + (tiles > 1 ? tiles : 0)),
