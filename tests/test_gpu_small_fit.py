@@ -98,3 +98,46 @@ def test_small_fit_tiles(ctx, n, m, sd, k):
     it, used = ctx.lbg_fit(ctx.to_device(x), n, m * sd, m, sd, k, 2, init, reseed, dcb)
     assert want["rc"] == 0 and np.array_equal(it, want["iters"]) and np.array_equal(used, want["reseeds"]) and used.min() > 0
     assert np.array_equal(dcb.download().view(np.uint32), want["codebooks"].view(np.uint32))
+
+
+@pytest.mark.parametrize("n,m,sd,k", [(12_288, 1, 36, 64), (12_288, 2, 52, 60), (16_000, 3, 100, 40), (9000, 1, 512, 30)])
+def test_small_fit_three_large_clusters(ctx, n, m, sd, k):
+    """Three clusters of every block that are taken by tiles, side by side, and of several blocks more than there are turns."""
+    rng = np.random.default_rng(n + m)
+    line = 1024 * -(-n // 4096)
+    sizes = [line + 1, line + 2, line + 1] if 3 * line + 4 + k < n else [line + 1, line + 2]
+    rest = n - sum(sizes)
+    sizes += [rest // (k - len(sizes))] * (k - len(sizes) - 1)
+    sizes.append(n - sum(sizes))
+    label = rng.permutation(np.repeat(np.arange(k), sizes))
+    x = (50.0 * label[:, None] + rng.random((n, m * sd))).astype(F)
+    first = np.array([int(np.flatnonzero(label == j)[0]) for j in range(k)])
+    init = np.stack([first[(np.arange(k) + 7 * s) % k] for s in range(m)]).astype(np.uint32)
+    reseed = rng.integers(0, n, (m, 2 * k), dtype=np.uint32)
+    want = O.pq_fit(x, m, k, 2, init, reseed)
+    dcb = ctx.empty((m, k, sd), F)
+    it, used = ctx.lbg_fit(ctx.to_device(x), n, m * sd, m, sd, k, 2, init, reseed, dcb)
+    assert want["rc"] == 0 and np.array_equal(it, want["iters"]) and np.array_equal(used, want["reseeds"])
+    assert np.array_equal(dcb.download().view(np.uint32), want["codebooks"].view(np.uint32))
+
+
+# both sides of the lines of one block that is the whole row, of a first fit and of a residual stage
+@pytest.mark.parametrize("residual,n,sd,k", [
+    (False, 54_000, 40, 200), (False, 54_001, 40, 200), (False, 58_000, 24, 100), (False, 58_001, 24, 100), (False, 20_480, 128, 64), (False, 20_481, 128, 64),
+    (True, 40_480, 32, 64), (True, 40_481, 32, 64), (True, 33_760, 64, 64), (True, 33_761, 64, 64), (True, 30_000, 128, 100), (True, 30_001, 128, 100),
+    (True, 16_071, 224, 128), (True, 16_072, 224, 128), (True, 104_001, 16, 170), (True, 30_001, 100, 100)])
+def test_fit_of_one_block_at_its_lines(ctx, residual, n, sd, k):
+    rng = np.random.default_rng(n + sd)
+    x = (rng.random((n, sd)) + 3 * rng.integers(0, 4, (n, 1))).astype(F)
+    init = rng.choice(n, k, replace=False).astype(np.uint32)[None]
+    reseed = rng.integers(0, n, (1, 2 * k), dtype=np.uint32)
+    dx, dcb = ctx.to_device(x), ctx.empty((1, k, sd), F)
+    if residual:
+        pcb, pcodes = rng.random((9, sd)).astype(F), rng.integers(0, 9, n, dtype=np.uint8)
+        it, used = ctx.lbg_fit_residual(dx, n, sd, sd, k, 2, init[0], reseed[0], dcb, ctx.to_device(pcb), 9, ctx.to_device(pcodes))
+        x = x - pcb[pcodes]
+    else:
+        it, used = ctx.lbg_fit(dx, n, sd, 1, sd, k, 2, init, reseed, dcb)
+    want = O.pq_fit(x, 1, k, 2, init, reseed)
+    assert want["rc"] == 0 and np.all(it == want["iters"]) and np.all(used == want["reseeds"])
+    assert np.array_equal(dcb.download().view(np.uint32), want["codebooks"].view(np.uint32))

@@ -1280,10 +1280,12 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_update_small(LbgSm
 // last part adds the part sums in part order and divides.  One workgroup that adds such a cluster alone
 // is bound by what it has in flight, 64 KB per memory round trip: 6,000 rows of 128 took 200 us.
 // SD: a cluster with more than kLargeTiled members per part (three of a column block at most) is taken by tiles of SD components, which
-// hold 1024 or 512 members per memory round trip: workgroups (p, whole + tile), which look for such clusters.  For the others a
+// hold 1024 or 512 members per memory round trip: workgroups (p, whole + tile + tiles t), which look for such clusters and take the t-th, the
+// (t + kLargeTurns)-th ... of them (one turn: three clusters of a block one after the other, 23,405 x 224, k = 160 95 us a launch, of 12,288 x
+// 128, k = 64 55; without tiles 50 and 39).  For the others a
 // fence per tile is more than what the tiles save (20,000 x 128, k = 256, tiles of all clusters 22.7 us a launch, of these 17.1;
 // 15,980 x 96, k = 63 28.6 without tiles).
-constexpr int kLargeTiled = 1024;
+constexpr int kLargeTiled = 1024, kLargeTurns = 3;
 template <int SD>
 static __global__ void __launch_bounds__(kSmallThreads) k_lbg_large(LbgSmall st, int it, const float *__restrict__ x,
                                                                     int64_t n, int64_t ld, int full, int k, int whole,
@@ -1291,7 +1293,7 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_large(LbgSmall st,
     const int count = st.n_large[it];
     const bool tiled = SD != 0 && (int)blockIdx.y >= whole;
     if (tiled ? count == 0 : (int)blockIdx.y >= count) return;
-    const int tile = tiled ? (int)blockIdx.y - whole : 0, tiles = SD ? (int)gridDim.y - whole : 1;
+    const int tiles = SD ? (full + SD - 1) / (SD ? SD : 1) : 1, tile = tiled ? ((int)blockIdx.y - whole) % tiles : 0;
     const int p = blockIdx.x, nparts = gridDim.x, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ uint16_t list[kPartRows];
@@ -1388,9 +1390,13 @@ static __global__ void __launch_bounds__(kSmallThreads) k_lbg_large(LbgSmall st,
             if (!by_tiles(st.large[e].y)) cluster(e);  // uniform
         return;
     }
+    int turn = ((int)blockIdx.y - whole) / tiles;
     for (int e0 = 0; e0 < count; e0 += 64) {  // every wave finds the same entries
         const bool mine = e0 + lane < count && by_tiles(st.large[e0 + lane < count ? e0 + lane : 0].y);
-        for (uint64_t mask = __ballot(mine); mask; mask &= mask - 1) cluster(e0 + __ffsll((unsigned long long)mask) - 1);
+        for (uint64_t mask = __ballot(mine); mask; mask &= mask - 1) {
+            if (turn == 0) cluster(e0 + __ffsll((unsigned long long)mask) - 1);
+            turn = turn == 0 ? kLargeTurns - 1 : turn - 1;
+        }
     }
 }
 

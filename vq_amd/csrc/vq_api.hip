@@ -1462,7 +1462,7 @@ static int32_t lbg_fit_small(vq_ctx *ctx, const float *d_x, int64_t n, int64_t l
                            (const uint32_t *)reseed, n_reseed, d_codebooks, tiles);
         const int whole = std::min(most_large, 16);
         if (defer)
-            hipLaunchKernelGGL(width == 16 ? vq::k_lbg_large<16> : width == 32 ? vq::k_lbg_large<32> : vq::k_lbg_large<0>, dim3(nparts, whole + (tiles > 1 ? tiles : 0)),
+            hipLaunchKernelGGL(width == 16 ? vq::k_lbg_large<16> : width == 32 ? vq::k_lbg_large<32> : vq::k_lbg_large<0>, dim3(nparts, whole + (tiles > 1 ? vq::kLargeTurns * tiles : 0)),
                                dim3(vq::kSmallThreads), lds, st, S, it, d_x, n, ld, sd, k, whole, d_codebooks);
     }
     last();
