@@ -45,7 +45,7 @@ std::string &create_error() {
 
 using namespace vqh;
 
-static bool lbg_small(int64_t n, int m, int sd, int k);
+static bool lbg_small(int64_t n, int m, int sd, int k, bool residual);
 
 namespace {
 
@@ -529,7 +529,7 @@ double fit_static_us(int64_t n, int m, int sd, int k) {
 
 // The width to pad every column block to so that the matrix-core kernels take the shape (squared L2,
 // Euclidean, cosine; 0: they take it as it is, or padding does not pay).  fit: for the passes of a fit,
-// which pads its rows once and whose update then streams blocks of 8 as well.
+// which pads its rows once and whose update then streams blocks of 8 as well (residual: of a residual stage).
 // k_assign_static does 3 w + 1 vector instructions per row and centroid (cosine: about 2 w + 26; w: its register
 // width), the padded kernels about 600 per row and block and half the bytes more to read.  Its own widths: the
 // lines below are where the two took the same time at 20,000-600,000 rows, 12 and 25 blocks; one float
@@ -546,7 +546,7 @@ double fit_static_us(int64_t n, int m, int sd, int k) {
 // of four floats; per iteration own / padded): 431 x 15 blocks of 4, k = 16 12.5 / 14.8, k = 32 12.9 / 14.7, 10,000 x 15 of 4, k = 64 19.6 / 20.1, 256
 // 31 / 24; of 12, k = 16 13 / 15.4, 32 15.4 / 15.9, 64 18.9 / 16; of 20, k = 16 16.8 / 23.5, 32 19.3 / 22.8, 64 26 / 22.7; of 28, k = 32 22.5 / 23.5,
 // 64 30 / 23.  Widths that neither takes always gain.
-int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bool fit) {
+int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bool fit, bool residual = false) {
     if (ctx->assign_path == 1 || ctx->no_alloc || ctx->pad_held || metric < VQ_SQEUCLIDEAN || metric > VQ_COSINE) return 0;
     if (sd == 1 || a.k < 2 || a.k > vq::kMaxK || a.m > 65535) return 0;
     if (mfma_applicable<vq::M_SQ, true>(ctx, a, sd) || mfma16_applicable<vq::M_SQ, true>(ctx, a, sd) ||
@@ -558,8 +558,8 @@ int pad_width(const vq_ctx *ctx, int metric, const vq::AssignArgs &a, int sd, bo
     if ((int64_t)a.m * sdp > (1 << 20) || sdp > (1 << 16) || a.n * a.m >= (1LL << 32)) return 0;
     const int w = static_width(sd);
     // few rows, whose update is one launch at either width: padding adds its own launches and pays by the scores alone
-    if (fit && sd <= 28 && a.k < 40 && lbg_small(a.n, a.m, sd, a.k)) return 0;
-    if (fit && sd != sdp && lbg_small(a.n, a.m, sdp, a.k)) return sdp;
+    if (fit && sd <= 28 && a.k < 40 && lbg_small(a.n, a.m, sd, a.k, residual)) return 0;
+    if (fit && sd != sdp && lbg_small(a.n, a.m, sdp, a.k, residual)) return sdp;
     if (fit && sd < 8) return fit8_us(a.n, a.m, a.k) < fit_static_us(a.n, a.m, sd, a.k) ? sdp : 0;
     if (fit && w && w != sd && (w <= 16 || w == 32)) return a.k >= (w == 32 ? 36 : 40) || (w <= 16 && a.m % 2 == 0) ? sdp : 0;
     if (w == sd) {
@@ -1247,16 +1247,16 @@ template <typename Last>
 static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
                            int32_t max_iters, const uint32_t *h_init_idx, const uint32_t *h_reseed_stream,
                            int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used,
-                           const float *pend_cb, const uint8_t *pend_codes, const Last &last);
+                           const float *pend_cb, const uint8_t *pend_codes, bool residual, const Last &last);
 
 // pend_cb / pend_codes: a residual update x[i] -= pend_cb[pend_codes[i]] that the fit applies to the
 // rows in place as its first assignment pass reads them (the caller has checked that this shape's
-// first pass is the kernel that can: lbg_pending_fusable).
+// first pass is the kernel that can: lbg_pending_fusable).  residual: the rows are (or become so) what a stage left.
 static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd,
                             int32_t k, int32_t max_iters, const uint32_t *h_init_idx,
                             const uint32_t *h_reseed_stream, int32_t n_reseed, float *d_codebooks,
                             int32_t *h_iters_run, int32_t *h_reseeds_used, const float *pend_cb,
-                            const uint8_t *pend_codes) {
+                            const uint8_t *pend_codes, bool residual) {
     if (!ctx) return VQ_ERR_INVALID_ARG;
     if (k == 0) return fail(ctx, VQ_ERR_INVALID_ARG, "Invalid parameter: k must be greater than 0");
     VQ_TRY(check_common(ctx, d_x, n, ld, m, sd, k, 65536));
@@ -1300,7 +1300,7 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
     shape.m = m;
     shape.k = k;
     shape.cb = d_codebooks;
-    const int sdp = max_iters > 0 ? pad_width(ctx, VQ_SQEUCLIDEAN, shape, sd, true) : 0;
+    const int sdp = max_iters > 0 ? pad_width(ctx, VQ_SQEUCLIDEAN, shape, sd, true, residual) : 0;
     if (sdp && (int64_t)k * cdiv(n, vq::kPartRows) * sdp <= (1LL << 31)) {
         // the rows padded once for all passes of the fit (where the second copy of the rows and the fit's
         // workspace do not fit together, it trains on the rows as they are: the same results)
@@ -1310,7 +1310,7 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
             float *px = (float *)ctx->pad_x.p, *pcb = (float *)ctx->pad_cb.p;
             launch_pad(ctx, d_x, n, ld, m, sd, sdp, px);
             rc = lbg_fit_run(ctx, px, n, (int64_t)m * sdp, m, sdp, k, max_iters, h_init_idx, h_reseed_stream, n_reseed,
-                             pcb, h_iters_run, h_reseeds_used, nullptr, nullptr, [&] {
+                             pcb, h_iters_run, h_reseeds_used, nullptr, nullptr, residual, [&] {
                                  unpad_rows(ctx, pcb, (int64_t)m * k, sd, sdp, d_codebooks);
                              });
         }
@@ -1323,7 +1323,7 @@ static int32_t lbg_fit_impl(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld
         if (rc != VQ_ERR_OOM) return rc;
     }
     return lbg_fit_run(ctx, d_x, n, ld, m, sd, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, d_codebooks,
-                       h_iters_run, h_reseeds_used, pend_cb, pend_codes, [] {});
+                       h_iters_run, h_reseeds_used, pend_cb, pend_codes, residual, [] {});
 }
 
 // Clusters per workgroup of k_lbg_update_small: the fewest with which the workgroups (106 KB of LDS each) are one
@@ -1351,21 +1351,28 @@ static int lbg_small_width(int m, int sd, int k) {
 // 8 floats, k = 116) and near 75,000 floats per workgroup in narrow blocks, 45,000-70,000 in wide ones, on
 // uniform rows and on mixtures.  Ten iterations, m = 16, k = 256, blocks of 8: 2,000 rows 0.83 -> 0.22 ms,
 // 10,000 1.07 -> 0.29 ms, 50,000 1.35 -> 0.74 ms; m = 1, k = 256, 20,000 x 128: 0.78 -> 0.45 ms.
-// Blocks above 32 floats: a block that is the whole row is a stage of a residual fit, whose rows gather in a few clusters, and every
-// workgroup lists all rows.  Three stages of five iterations, other path -> this one: k = 256, 30,000 x 64 1077 -> 994 us,
-// 45,000 1175 -> 1171, 65,000 1186 -> 1625, 130,000 1320 -> 3915; 20,000 x 128 1097 -> 1002, 40,000 1196 -> 1471; 16,000 x 256
-// 1314 -> 1276, 24,000 1332 -> 1533; k = 63, 16,000 x 96 1054 -> 1064.  Of several wide blocks the rows spread over the clusters, and the
-// line rises with k.  Fit of five iterations and encode: two blocks of 48, k = 256 33,000 rows 400 -> 345, 40,000 393 -> 358, 48,000 404 -> 385,
-// 65,000 468 -> 508, k = 128 36,000 364 -> 356, 44,000 371 -> 395; three of 36, k = 180 36,000 424 -> 396, 44,000 448 -> 434, k = 100 33,000 429 -> 388,
-// 40,000 423 -> 439; four of 64, k = 256 36,000 465 -> 439, 44,000 495 -> 502, k = 180 33,000 466 -> 447, 36,000 467 -> 499; two of 96, k = 256 36,000
-// 435 -> 404, 44,000 457 -> 520; two of 128, k = 256 33,000 498 -> 513, 40,000 492 -> 523.  Narrower rows likewise, three stages, k = 256: 40,000 x 32 959 -> 933, 80,000 1058 -> 1321,
-// 130,000 1152 -> 1920; 40,000 x 24 954 -> 827, 80,000 1047 -> 1291; 80,000 x 16 875 -> 816, 130,000 930 -> 1201.
-static bool lbg_small(int64_t n, int m, int sd, int k) {
+// A block that is the whole row (m == 1).  What decides is the longest cluster: even rows keep the clusters even in every
+// stage, the residuals of clustered rows gather in a few of them, and every workgroup lists all rows.  So the lines lie lower where
+// the rows are what a stage left, where both kinds of rows lose as much on one side as on the other.  A fit of five iterations, k = 256, other
+// path -> this one: uniform rows, first stage 52,428 x 24 307 -> 227 us, 78,643 x 32 337 -> 273, 52,428 x 64 355 -> 298, 78,643 389 -> 410, 32,768 x
+// 128 405 -> 331, 65,536 452 -> 441; a mixture of 1024 Gaussians, first stage 104,857 x 24 365 -> 372, 52,428 x 64 374 -> 323, 78,643 402 -> 529.
+// Residuals: uniform 52,428 x 24 305 -> 234, 78,643 328 -> 314, 52,428 x 64 360 -> 304, 78,643 392 -> 412, 28,086 x 224 446 -> 417; mixture 52,428 x
+// 24 322 -> 360, 78,643 357 -> 477, 32,768 x 64 337 -> 360, 52,428 365 -> 460, 28,086 x 224 451 -> 518, 131,072 x 64 441 -> 1377.  k = 64, residuals of a
+// mixture: 32,768 x 64 1.02 times the other path's time, 40,960 1.19, 9,361 x 224 1.00; uniform 0.75, 0.86, 0.77.  Above 160 floats the residuals'
+// line is a number of floats.
+// Several wide blocks: their rows spread over the clusters too.  Fit of five iterations and encode: two blocks of 48, k = 256 33,000 rows
+// 400 -> 345, 40,000 393 -> 358, 48,000 404 -> 385, 65,000 468 -> 508, k = 128 36,000 364 -> 356, 44,000 371 -> 395; three of 36, k = 180 36,000 424 -> 396,
+// 44,000 448 -> 434, k = 100 33,000 429 -> 388, 40,000 423 -> 439; four of 64, k = 256 36,000 465 -> 439, 44,000 495 -> 502, k = 180 33,000 466 -> 447,
+// 36,000 467 -> 499; two of 96, k = 256 36,000 435 -> 404, 44,000 457 -> 520; two of 128, k = 256 33,000 498 -> 513, 40,000 492 -> 523.
+static bool lbg_small(int64_t n, int m, int sd, int k, bool residual) {
     if (sd % 4 != 0 || sd > 4096 || n > 131072) return false;
     if (sd > vq::kSmallThreads) return n <= 128 * (int64_t)k;
-    const int64_t wide = m == 1 || sd > 96 ? 0 : sd <= 48 ? 27000 + 90 * (int64_t)k : 24000 + 62 * (int64_t)k;
-    if (sd > 32 ? n > std::max<int64_t>(32768, wide) : m == 1 && sd >= 16 && n > (sd > 16 ? 45056 : 90112)) return false;
-    return n <= 640 * (int64_t)k && n * lbg_small_clusters(m, sd, k) * sd <= (sd <= 32 ? 57344 : m == 1 ? 20480 : 40960) * (int64_t)k;
+    if (n > 640 * (int64_t)k || n * lbg_small_clusters(m, sd, k) * sd > (sd <= 32 ? 57344 : 40960) * (int64_t)k) return false;
+    if (m > 1) return sd <= 32 || n <= std::max(32768, sd > 96 ? 0 : sd <= 48 ? 27000 + 90 * k : 24000 + 62 * k);
+    if (sd < 16) return true;
+    if (residual)
+        return sd > 160 ? n * sd <= 3'600'000 : n <= (sd == 16 ? 104'000 : sd <= 32 ? 36000 + 70 * k : sd <= 64 ? 28000 + 90 * k : 25000 + 50 * k);
+    return sd == 16 || n <= (sd <= 32 ? 30000 + 280 * k : sd <= 64 ? 35000 + 95 * k : 30000 + 70 * k);
 }
 
 // The LBG loop of a small fit, two launches per iteration: the assignment and k_lbg_update_small.  The
@@ -1491,8 +1498,8 @@ template <typename Last>
 static int32_t lbg_fit_run(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t m, int32_t sd, int32_t k,
                            int32_t max_iters, const uint32_t *h_init_idx, const uint32_t *h_reseed_stream,
                            int32_t n_reseed, float *d_codebooks, int32_t *h_iters_run, int32_t *h_reseeds_used,
-                           const float *pend_cb, const uint8_t *pend_codes, const Last &last) {
-    if (lbg_small(n, m, sd, k))
+                           const float *pend_cb, const uint8_t *pend_codes, bool residual, const Last &last) {
+    if (lbg_small(n, m, sd, k, residual))
         return lbg_fit_small(ctx, d_x, n, ld, m, sd, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, d_codebooks,
                              h_iters_run, h_reseeds_used, pend_cb, pend_codes, last);
     hipStream_t st = ctx->stream;
@@ -1724,7 +1731,7 @@ int32_t vq_lbg_fit(vq_ctx *ctx, const float *d_x, int64_t n, int64_t ld, int32_t
                    const uint32_t *h_reseed_stream, int32_t n_reseed, float *d_codebooks,
                    int32_t *h_iters_run, int32_t *h_reseeds_used) {
     return lbg_fit_impl(ctx, d_x, n, ld, m, sd, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, d_codebooks,
-                        h_iters_run, h_reseeds_used, nullptr, nullptr);
+                        h_iters_run, h_reseeds_used, nullptr, nullptr, false);
 }
 
 int32_t vq_lbg_fit_residual(vq_ctx *ctx, float *d_res, int64_t n, int64_t ld, int32_t dim, int32_t k,
@@ -1751,10 +1758,10 @@ int32_t vq_lbg_fit_residual(vq_ctx *ctx, float *d_res, int64_t n, int64_t ld, in
     if (!fusable) {
         VQ_TRY(vq_residual_sub(ctx, d_res, n, ld, dim, k_prev, d_prev_codebook, d_prev_codes));
         return lbg_fit_impl(ctx, d_res, n, ld, 1, dim, k, max_iters, h_init_idx, h_reseed_stream, n_reseed,
-                            d_codebook, h_iters_run, h_reseeds_used, nullptr, nullptr);
+                            d_codebook, h_iters_run, h_reseeds_used, nullptr, nullptr, true);
     }
     return lbg_fit_impl(ctx, d_res, n, ld, 1, dim, k, max_iters, h_init_idx, h_reseed_stream, n_reseed, d_codebook,
-                        h_iters_run, h_reseeds_used, d_prev_codebook, d_prev_codes);
+                        h_iters_run, h_reseeds_used, d_prev_codebook, d_prev_codes, true);
 }
 
 int32_t vq_assign(vq_ctx *ctx, int32_t metric, const float *d_x, int64_t n, int64_t ld, int32_t m,
