@@ -119,7 +119,7 @@ __global__ void __launch_bounds__(256) k_decode_units(const CodeT *__restrict__ 
     }
 }
 
-// f16 rows of blocks of any width with the table of all blocks in LDS (up to 160 KB; one workgroup of 1024 threads per compute
+// f16 rows (16-byte aligned) of blocks of any width with the table of all blocks in LDS (up to 160 KB; one workgroup of 1024 threads per compute
 // unit, two up to 80 KB): a thread makes eight consecutive components per step whatever blocks they belong to, two steps in flight,
 // so a wave stores 1 KB of consecutive bytes.  FEW: eight components lie in two blocks at most, whose codes are read once.
 // The stores (4.0 TB/s at 372,160 x 315) or, in narrow blocks, the LDS reads and the codes bound it.
@@ -140,7 +140,6 @@ __global__ void __launch_bounds__(1024) k_decode_flat(const CodeT *__restrict__ 
     }
     for (uint32_t e = 4 * quads + threadIdx.x; e < entries; e += T) flat_tab[e] = (uint16_t)two(cb[e], 0.0f);
     __syncthreads();
-    const bool whole = (reinterpret_cast<uintptr_t>(out) & 15) == 0;  // uniform
     const int64_t blocks = n * m, total = blocks * sd;
     for (int64_t first = (int64_t)blockIdx.x * RUN; first < total; first += (int64_t)gridDim.x * RUN) {
         const int64_t b0 = total <= 0xFFFFFFFFll ? (uint32_t)first / (uint32_t)sd : first / sd;  // uniform
@@ -179,7 +178,7 @@ __global__ void __launch_bounds__(1024) k_decode_flat(const CodeT *__restrict__ 
                 }
             }
             const int64_t left = total - first - off;
-            if (left >= PER && whole) {
+            if (left >= PER) {
                 __builtin_nontemporal_store(u32x4_out{w[0], w[1], w[2], w[3]}, reinterpret_cast<u32x4_out *>(out + first + off));
             } else {
 #pragma unroll
@@ -191,11 +190,15 @@ __global__ void __launch_bounds__(1024) k_decode_flat(const CodeT *__restrict__ 
 }
 
 // Widths and alignments that k_decode_gather does not take, launched.  k: entries per block (of a tree: its nodes).
-// lds_set: the caller's, a bit per kernel whose LDS limit has been set.
+// lds_set: the caller's, a bit per kernel whose LDS limit has been set.  The table only for aligned outputs: with single stores of the
+// others 500,000 blocks of 5 take 3.1 us more than aligned ones, from memory 1.2 (200,000 x 10 of 10 42 us against 32 from memory).  Four
+// units in flight per thread against one: 20,000 x 20 of 9 19.1 us against 20.8, 20,000 x 40 of 10 20.6 against 22.8; of 12, whose units are four
+// components, 20,000 rows 20.7 against 20.1, 25,000 21.9 against 21.4, 1,000,000 x 4 of 4 23.5 against 24.3.
 template <bool F16, typename CodeT>
 hipError_t launch_decode_any(hipStream_t st, int compute_units, uint32_t &lds_set, const CodeT *codes, int64_t n, int m, int sd, int k,
                              const float *cb, void *out) {
-    const size_t lds = F16 && decode_flat_resident(n, m, sd, k) ? 2 * (size_t)m * k * sd : 0;
+    const bool whole = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    const size_t lds = F16 && whole && decode_flat_resident(n, m, sd, k) ? 2 * (size_t)m * k * sd : 0;
     const unsigned lds_groups = (unsigned)compute_units * (lds <= kDecodeFlatLds / 2 ? 2u : 1u);
     const uintptr_t at = reinterpret_cast<uintptr_t>(cb);
     const int64_t total = n * m * sd;
@@ -217,8 +220,9 @@ hipError_t launch_decode_any(hipStream_t st, int compute_units, uint32_t &lds_se
                 return hipSuccess;
             }
         }
-        auto kern = total < (1 << 21) * UNIT ? k_decode_units<F16, UNIT, 1, CodeT> : k_decode_units<F16, UNIT, 4, CodeT>;
-        const int64_t run = (total < (1 << 21) * UNIT ? 256 : 1024) * UNIT;
+        const bool one = total < (UNIT == 4 ? 3 << 22 : UNIT << 21);
+        auto kern = one ? k_decode_units<F16, UNIT, 1, CodeT> : k_decode_units<F16, UNIT, 4, CodeT>;
+        const int64_t run = (one ? 256 : 1024) * UNIT;
         hipLaunchKernelGGL(kern, dim3((unsigned)((total + run - 1) / run)), dim3(256), 0, st, codes, n, m, sd, k, cb, out);
         return hipSuccess;
     };
