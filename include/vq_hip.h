@@ -82,11 +82,12 @@ int32_t vq_ctx_set_assign_path(vq_ctx *ctx, int32_t path);
  * is 1; other descents do not look at this switch.  Both give the reference's results bit for bit; the switch exists for measurement and tests. */
 int32_t vq_ctx_set_few_path(vq_ctx *ctx, int32_t path);
 
-/* How vq_tsvq_build sums a node's squared deviations per dimension in row order (src/tsvq.rs:88-99)
- * when dim is a multiple of 8:
- *   0 (default)  groups of 32 squares as integer maps on the running sum, composed by a scan, with
- *                the groups in which the sum changes binade added one by one
- *   1            one chain of dependent adds per column
+/* How vq_tsvq_build sums a node's squared deviations per dimension in row order (src/tsvq.rs:88-99):
+ *   0 (default)  levels with a node above 8192 rows (16,384 from 89 columns on): groups of 32 squares as integer
+ *                maps on the running sum, composed by a scan, with the groups in which the sum changes binade
+ *                added one by one; the levels below by tiles of columns, without the host between them
+ *   1            one chain of dependent adds per column where dim is a multiple of 8 or the rows are padded to one,
+ *                else tiles of columns; the host between all levels
  * Both give the reference's sequential f32 sums bit for bit; the switch exists for measurement and
  * tests.  No counterpart in the reference. */
 int32_t vq_ctx_set_tsvq_variance_path(vq_ctx *ctx, int32_t path);

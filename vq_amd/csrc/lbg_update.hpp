@@ -809,7 +809,7 @@ static __global__ void __launch_bounds__(256) k_lbg_finalize(LbgState st, const 
 // brings in are those of a whole block of C / tiles clusters, but a stage holds 1024 or 512 members instead of 170 of 96 floats, and a
 // long cluster's are spread over several workgroups: what bounded it was one memory round trip per stage of the longest cluster.
 // An iteration of a residual fit of 6,264 x 96, k = 186 61 -> 49 us, 7,143 x 100, k = 214 87 -> 63; fits, three or four stages of six iterations, of
-// 8,000 x 256, k = 256 2356 -> 1647 us, 10,000 x 512 2729 -> 1830, 12,000 x 300, k = 100 3540 -> 2520.
+// 8,000 x 256, k = 256 2330 -> 1645 us, 10,000 x 512 2709 -> 1797, 12,000 x 300, k = 100 3536 -> 2273.
 // STAGED: sub_dim a multiple of 4 up to 512, a thread per component.  Else (wider blocks) a wave takes
 // one cluster and 64 components at a time and reads the rows themselves, 16 rows in flight.
 constexpr int kSmallList = 8192;    // listed rows held before the list is worked off: at least 16 per thread
